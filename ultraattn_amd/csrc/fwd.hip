@@ -74,6 +74,7 @@ __device__ __forceinline__ void half_tile(const unsigned char* sK, const unsigne
   }
   // element (mb, i) of this lane: key key0 + 32*mb + 8*(i/4) + 4*hi + i%4, query q_local
   if (mask) {
+    keep_branch_local(q_local);
 #pragma unroll
     for (int mb = 0; mb < 2; ++mb)
 #pragma unroll

@@ -30,13 +30,6 @@ __device__ __forceinline__ int lds_off_k(int r, int c) { return r * kRowBytes + 
 // transposing 64-bit read gathers land in 4 different bank groups.
 __device__ __forceinline__ int lds_off_v(int r, int c) { return r * kRowBytes + ((c ^ ((r & 3) << 2)) << 4); }
 
-// Universal layout: chunk index XOR (row mod 16 with its two 2-bit fields swapped).  Serves
-// both access patterns on one tile: 16 consecutive rows still hit 16 different slots, and 4
-// consecutive rows still hit 4 different 64-byte groups.
-__device__ __forceinline__ int lds_off_u(int r, int c) {
-  return r * kRowBytes + ((c ^ (((r & 3) << 2) | ((r >> 2) & 3))) << 4);
-}
-
 __device__ __forceinline__ bf16x8 lds_read_b128(const unsigned char* smem, int off) {
   return *reinterpret_cast<const bf16x8*>(smem + off);
 }
@@ -85,8 +78,10 @@ __device__ __forceinline__ bf16x8 lds_read_tr_frag(const unsigned char* smem, co
 }
 
 __device__ __forceinline__ void wait_vmem_all() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-// Keeps a wave-uniform branch a branch (the optimiser may not turn its body into selects).
-__device__ __forceinline__ void keep_branch() { asm volatile("" ::: "memory"); }
+// At the top of a rare wave-uniform branch: keeps it a branch (its body is not turned into selects), and what
+// the body computes from x stays in it.  Hoisted out of the walk, the comparisons of a masked tile take two
+// scalar registers each, and the attention kernels then spill a hundred of them into vector lanes.
+__device__ __forceinline__ void keep_branch_local(int& x) { asm volatile("" : "+v"(x) :: "memory"); }
 
 // Wave-uniform reads of the (read-only) tile-list arrays through the scalar cache.
 __device__ __forceinline__ int32_t sload(const int32_t* p, int i) {
