@@ -5,11 +5,12 @@
 // [batch, head, token] while the rows themselves are [batch, token, head, 128]; the workgroup
 // first handles the statistics with token-contiguous (coalesced) accesses and parks the row
 // weights in LDS, then streams the rows as 16-byte vectors (16 lanes per 256-byte row).
+#include <type_traits>
 #include "ua_common.h"
 
 namespace ua {
 
-constexpr int kTok = 16;          // tokens per workgroup (delta, single update)
+constexpr int kTok = 16;          // tokens per workgroup (single update)
 // The merge runs best with many small workgroups: with 2 tokens x 32 heads a workgroup issues
 // all of its row loads in one step (4 x 16 bytes per thread and partial) and retires; the
 // device then streams 4 reads : 1 write at the rate a bare copy kernel of the same shape reaches.
@@ -114,6 +115,7 @@ struct DeltaParams {
   Strides3 os, ds;
 };
 
+template <int kTok>
 __global__ __launch_bounds__(256) void delta_kernel(const DeltaParams p) {
   extern __shared__ float d_lds[];               // [n_heads][kTok]
   const int tid = threadIdx.x;
@@ -124,7 +126,7 @@ __global__ __launch_bounds__(256) void delta_kernel(const DeltaParams p) {
   const int rows = ntok * p.n_heads;
   const int sub = tid & 15;
   // 16 lanes per row; kRows rows per thread and step so that 2 * kRows 16-byte loads are in flight
-  constexpr int kRows = 4;
+  constexpr int kRows = 2;
   for (int row0 = tid >> 4; row0 < rows; row0 += 16 * kRows) {
     u32x4 a[kRows], g[kRows];
 #pragma unroll
@@ -293,15 +295,26 @@ extern "C" int ua_bsa_bwd_delta(const void* o, const void* dout, float* delta,
   if (!o || !dout || !delta || !o_strides || !do_strides) return UA_ERR_NULL;
   if (head_dim != kHeadDim) return UA_ERR_UNSUPPORTED;
   if (batch <= 0 || seqlen_q <= 0 || n_heads <= 0 || n_heads > kMaxHeadsLds) return UA_ERR_SHAPE;
-  if ((int64_t)batch * ((seqlen_q + kTok - 1) / kTok) > INT32_MAX) return UA_ERR_SHAPE;
+  if ((int64_t)batch * seqlen_q > INT32_MAX) return UA_ERR_SHAPE;
   if (!aligned16(o) || !aligned16(dout) || !strides_ok(o_strides) || !strides_ok(do_strides)) return UA_ERR_ALIGN;
   if (int rc = check_device()) return rc;
   DeltaParams p;
   p.o = (const bf16*)o; p.dout = (const bf16*)dout; p.delta = delta; p.seqlen = seqlen_q; p.n_heads = n_heads;
   p.os = {o_strides[0], o_strides[1], o_strides[2]};
   p.ds = {do_strides[0], do_strides[1], do_strides[2]};
-  hipLaunchKernelGGL(delta_kernel, dim3(batch * ((seqlen_q + kTok - 1) / kTok)), dim3(256),
-                     (size_t)kTok * n_heads * sizeof(float), (hipStream_t)stream, p);
+  hipStream_t st = (hipStream_t)stream;
+  // A workgroup takes 32 rows at most: they are read in one round of loads, and a short sequence of many heads still
+  // gives every CU work.  512 tokens x 32 heads: 17.2 us at 16 tokens per workgroup, 3.2 at one; 32768 x 32: equal
+  // (86.3, 86.9: 6.2 TB/s).  With few heads more tokens share a workgroup, up to a 64-byte run of the result.
+  auto go = [&](auto tok) {
+    constexpr int kT = decltype(tok)::value;
+    hipLaunchKernelGGL(delta_kernel<kT>, dim3((unsigned)(batch * (((int64_t)seqlen_q + kT - 1) / kT))), dim3(256), (size_t)kT * n_heads * sizeof(float), st, p);
+  };
+  if (n_heads <= 2)       go(std::integral_constant<int, 16>{});
+  else if (n_heads <= 4)  go(std::integral_constant<int, 8>{});
+  else if (n_heads <= 8)  go(std::integral_constant<int, 4>{});
+  else if (n_heads <= 16) go(std::integral_constant<int, 2>{});
+  else                    go(std::integral_constant<int, 1>{});
   return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH;
 }
 
