@@ -61,8 +61,8 @@ extern "C" {
 #define UA_NOALLOC_MAX_LINES 65532   /* most query tiles + key tiles of ua_tilelist_build_device_noalloc */
 
 /* 100 * major + minor.  102: `nnz` argument of the attention entry points, ua_merge_update, the
- * no-allocation builder, `work` of ua_tilelist_build_device grown to n_qtiles + n_ktiles + 7.  */
-#define UA_VERSION 103
+ * no-allocation builder, `work` of ua_tilelist_build_device grown to n_qtiles + n_ktiles + 7.  104: ua_bsa_bwd.  */
+#define UA_VERSION 104
 int ua_version(void);
 const char *ua_strerror(int rc);
 
@@ -165,6 +165,17 @@ int ua_bsa_bwd_dq(const void *q, const void *k, const void *v, const void *dout,
                   const int64_t *q_strides, const int64_t *k_strides, const int64_t *v_strides,
                   const int64_t *do_strides, const int64_t *dq_strides,
                   float softmax_scale, void *stream);
+
+/* ua_bsa_bwd_dkdv and ua_bsa_bwd_dq as one launch (same results): the two sides' workgroups share the
+ * device, so that neither leaves it partly empty at its end, and small masks need no second launch. */
+int ua_bsa_bwd(const void *q, const void *k, const void *v, const void *dout,
+               const float *lse, const float *delta, void *dq, void *dk, void *dv,
+               const int32_t *row_ptr, const int32_t *col_idx, const uint8_t *flag, const int32_t *q_order,
+               const int32_t *col_ptr, const int32_t *row_idx, const uint8_t *cflag, const int32_t *k_order,
+               int batch, int n_heads, int n_qtiles, int n_ktiles, int nnz, int head_dim,
+               const int64_t *q_strides, const int64_t *k_strides, const int64_t *v_strides,
+               const int64_t *do_strides, const int64_t *dq_strides, const int64_t *dk_strides,
+               const int64_t *dv_strides, float softmax_scale, void *stream);
 
 /* ---- dense rectangles: the reference's tile kernel itself ------------------------------------
  * One call = one `_flash_attn_forward(q, k, v, dropout_p=0, softmax_scale, causal, ..., out=)`

@@ -21,22 +21,29 @@
 
 namespace ua {
 
+// One side of the backward: the columns (dK, dV; walks the CSC) or the rows (dQ; walks the CSR).
+struct BwdSide {
+  const int32_t* ptr; const int32_t* idx; const uint8_t* flag; const int32_t* order;
+  bf16* out0; bf16* out1;                  // columns: dk, dv; rows: dq, unused
+  Strides3 o0s, o1s;
+  // The walk is cut into n_parts parts of part_len tiles; with out_f32 part i leaves an fp32 partial result at
+  // out + i * o_part (fp32 elements, contiguous [batch, tokens, heads, 128]) for a later sum.
+  int n_parts, part_len, out_f32;
+  int64_t o_part;
+};
 struct BwdParams {
   const bf16* q; const bf16* k; const bf16* v; const bf16* dout;
   const float* lse; const float* delta;
-  bf16* out0; bf16* out1;                  // dkdv: dk, dv; dq: dq, unused
-  const int32_t* ptr; const int32_t* idx; const uint8_t* flag; const int32_t* order;
   int batch, n_heads, n_qtiles, n_ktiles, nnz;
-  Strides3 qs, ks, vs, ds, o0s, o1s;
+  Strides3 qs, ks, vs, ds;
   float scale_log2, scale;
   int heads_per_xcd;
-  // Dense rectangle (no list arrays).  dq walks key tiles [0, n_ktiles) of a query tile, with
-  // dense_causal [0, qt + diag_off], the last one causal; dkdv walks query tiles [0, n_qtiles) of a
-  // key tile, with dense_causal [kt - diag_off, n_qtiles), the first one causal.  The walk is cut
-  // into n_parts parts of part_len tiles; with out_f32 part i leaves an fp32 partial result at
-  // out + i * o*_part (fp32 elements, contiguous [batch, tokens, heads, 128]) for a later sum.
-  int dense, dense_causal, diag_off, n_parts, part_len, out_f32;
-  int64_t o0_part, o1_part;
+  // Dense rectangle (no list arrays).  The rows walk key tiles [0, n_ktiles) of a query tile, with dense_causal
+  // [0, qt + diag_off], the last one causal; the columns walk query tiles [0, n_qtiles) of a key tile, with
+  // dense_causal [kt - diag_off, n_qtiles), the first one causal.
+  int dense, dense_causal, diag_off;
+  int n_col_blocks;                        // bwd_kernel: workgroups of the columns, those of the rows follow
+  BwdSide cols, rows;
 };
 
 __device__ __forceinline__ void store_acc_t(bf16* row_ptr, const f32x16 (&acc)[4], float mul, int hi) {
@@ -69,12 +76,12 @@ __device__ __forceinline__ ParamsLate params_late() {
   return p;
 }
 // Output row of a result tensor: the caller's strided bf16 tensor, or part `part` of the fp32 partials.
-__device__ __forceinline__ void store_result(ParamsLate p, bf16* out, int64_t os_b, int64_t os_s, int64_t os_h, int64_t part_stride,
-                                             int part, int b, int64_t row, int h, int64_t seq, const f32x16 (&acc)[4], float mul,
-                                             int hi) {
+__device__ __forceinline__ void store_result(const __attribute__((address_space(4))) BwdSide* p, bf16* out, int64_t os_b, int64_t os_s,
+                                             int64_t os_h, int n_heads, int part, int b, int64_t row, int h, int64_t seq,
+                                             const f32x16 (&acc)[4], float mul, int hi) {
   if (p->out_f32) {
-    float* base = reinterpret_cast<float*>(out) + part * part_stride;
-    store_acc_f32(base + (((int64_t)b * seq + row) * p->n_heads + h) * kHeadDim, acc, mul, hi);
+    float* base = reinterpret_cast<float*>(out) + part * p->o_part;
+    store_acc_f32(base + (((int64_t)b * seq + row) * n_heads + h) * kHeadDim, acc, mul, hi);
   } else {
     store_acc_t(out + b * os_b + row * os_s + h * os_h, acc, mul, hi);
   }
@@ -247,13 +254,11 @@ __device__ __forceinline__ void dkdv_block(const PairAddr& ad, uint32_t stat, co
   }
 }
 
-__global__ __launch_bounds__(256, 2) void dkdv_kernel(const BwdParams p) {
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[kDkdvLdsBytes];
-  const uint32_t lds_base = (uint32_t)(uintptr_t)(UA_LDS unsigned char*)smem;
+__device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_base, int block) {
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int pos, bh;
-  map_block(blockIdx.x, p.batch * p.n_heads, p.heads_per_xcd, p.n_ktiles * p.n_parts, pos, bh);
+  map_block(block, p.batch * p.n_heads, p.heads_per_xcd, p.n_ktiles * p.cols.n_parts, pos, bh);
   const int b = bh / p.n_heads, h = bh % p.n_heads;
   int kt, e0, e1, diag = -1, part = 0;
   if (p.dense) {
@@ -261,12 +266,12 @@ __global__ __launch_bounds__(256, 2) void dkdv_kernel(const BwdParams p) {
     kt = pos - part * p.n_ktiles;                          // column 0 is the longest of a causal rectangle
     if (p.dense_causal) diag = kt - p.diag_off;            // query tile on the diagonal (may lie outside)
     const int qbeg = p.dense_causal ? min(max(diag, 0), p.n_qtiles) : 0;
-    e0 = min(max(part * p.part_len, qbeg), p.n_qtiles);
-    e1 = max(min((part + 1) * p.part_len, p.n_qtiles), e0);
+    e0 = min(max(part * p.cols.part_len, qbeg), p.n_qtiles);
+    e1 = max(min((part + 1) * p.cols.part_len, p.n_qtiles), e0);
   } else {
-    kt = min(max(sload(p.order, pos), 0), p.n_ktiles - 1);
-    e0 = min(max(sload(p.ptr, kt), 0), p.nnz);
-    e1 = min(max(sload(p.ptr, kt + 1), e0), p.nnz);
+    kt = min(max(sload(p.cols.order, pos), 0), p.n_ktiles - 1);
+    e0 = min(max(sload(p.cols.ptr, kt), 0), p.nnz);
+    e1 = min(max(sload(p.cols.ptr, kt + 1), e0), p.nnz);
   }
   const int64_t seq_q = (int64_t)p.n_qtiles * kTile;
   const PairStream in(p.q + b * p.qs.b + h * p.qs.h, (int)p.qs.s, p.dout + b * p.ds.b + h * p.ds.h, (int)p.ds.s, lds_base, wave, lane);
@@ -278,7 +283,7 @@ __global__ __launch_bounds__(256, 2) void dkdv_kernel(const BwdParams p) {
     if (n_half == 0) return 0;        // an empty column owns no list entry (the arrays may be NULL)
     const int e = min(e0 + (i >> 1), e1 - 1);
     if (p.dense) return e | ((int)(e == diag) << 30);      // the entry is the query tile itself
-    return min(max(sload(p.idx, e), 0), p.n_qtiles - 1) | (sload(p.flag, e) << 30);
+    return min(max(sload(p.cols.idx, e), 0), p.n_qtiles - 1) | (sload(p.cols.flag, e) << 30);
   };
   // rows' statistics, staged in the form the accumulators start from: threads 0..63 carry
   // -lse/softmax_scale (lse = -inf, a row without keys, stays -inf so that P = 0), threads
@@ -363,8 +368,8 @@ __global__ __launch_bounds__(256, 2) void dkdv_kernel(const BwdParams p) {
   const ParamsLate pl = params_late();
   const int64_t seq_k = (int64_t)pl->n_ktiles * kTile;
   const int64_t krow_out = (int64_t)kt * kTile + wave * 32 + l32;
-  store_result(pl, pl->out0, pl->o0s.b, pl->o0s.s, pl->o0s.h, pl->o0_part, part, b, krow_out, h, seq_k, dk, pl->scale, hi);
-  store_result(pl, pl->out1, pl->o1s.b, pl->o1s.s, pl->o1s.h, pl->o1_part, part, b, krow_out, h, seq_k, dv, 1.f, hi);
+  store_result(&pl->cols, pl->cols.out0, pl->cols.o0s.b, pl->cols.o0s.s, pl->cols.o0s.h, pl->n_heads, part, b, krow_out, h, seq_k, dk, pl->scale, hi);
+  store_result(&pl->cols, pl->cols.out1, pl->cols.o1s.b, pl->cols.o1s.s, pl->cols.o1s.h, pl->n_heads, part, b, krow_out, h, seq_k, dv, 1.f, hi);
 }
 
 // ---- dQ -----------------------------------------------------------------------------------------
@@ -420,13 +425,11 @@ __device__ __forceinline__ void dq_block(const PairAddr& ad, const bf16x8 (&qf)[
   }
 }
 
-__global__ __launch_bounds__(256, 2) void dq_kernel(const BwdParams p) {
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[4 * kHalfPitch];
-  const uint32_t lds_base = (uint32_t)(uintptr_t)(UA_LDS unsigned char*)smem;
+__device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_base, int block) {
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int pos, bh;
-  map_block(blockIdx.x, p.batch * p.n_heads, p.heads_per_xcd, p.n_qtiles * p.n_parts, pos, bh);
+  map_block(block, p.batch * p.n_heads, p.heads_per_xcd, p.n_qtiles * p.rows.n_parts, pos, bh);
   const int b = bh / p.n_heads, h = bh % p.n_heads;
   const int64_t seq_q = (int64_t)p.n_qtiles * kTile;
   int qt, e0, e1, diag = -1, part = 0;
@@ -436,16 +439,16 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const BwdParams p) {
     qt = p.dense_causal ? p.n_qtiles - 1 - line : line;    // longest rows first
     if (p.dense_causal) diag = qt + p.diag_off;
     const int kend = p.dense_causal ? min(max(diag + 1, 0), p.n_ktiles) : p.n_ktiles;
-    e0 = min(part * p.part_len, kend);
-    e1 = min(e0 + p.part_len, kend);
+    e0 = min(part * p.rows.part_len, kend);
+    e1 = min(e0 + p.rows.part_len, kend);
   } else {
-    qt = min(max(sload(p.order, pos), 0), p.n_qtiles - 1);
-    e0 = min(max(sload(p.ptr, qt), 0), p.nnz);
-    e1 = min(max(sload(p.ptr, qt + 1), e0), p.nnz);
+    qt = min(max(sload(p.rows.order, pos), 0), p.n_qtiles - 1);
+    e0 = min(max(sload(p.rows.ptr, qt), 0), p.nnz);
+    e1 = min(max(sload(p.rows.ptr, qt + 1), e0), p.nnz);
   }
   const PairStream in(p.k + b * p.ks.b + h * p.ks.h, (int)p.ks.s, p.v + b * p.vs.b + h * p.vs.h, (int)p.vs.s, lds_base, wave, lane);
-  auto ktile = [&](int e) { return p.dense ? e : min(max(sload(p.idx, e), 0), p.n_ktiles - 1); };
-  auto is_causal = [&](int e) { return p.dense ? (int)(e == diag) : sload(p.flag, e); };
+  auto ktile = [&](int e) { return p.dense ? e : min(max(sload(p.rows.idx, e), 0), p.n_ktiles - 1); };
+  auto is_causal = [&](int e) { return p.dense ? (int)(e == diag) : sload(p.rows.flag, e); };
 
   int kt = e0 < e1 ? ktile(e0) : 0;
   if (e0 < e1) in.copy_in((int64_t)kt * kTile, 0);
@@ -496,20 +499,36 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const BwdParams p) {
   }
   const ParamsLate pl = params_late();
   const int64_t qrow_out = (int64_t)qt * kTile + wave * 32 + l32;
-  store_result(pl, pl->out0, pl->o0s.b, pl->o0s.s, pl->o0s.h, pl->o0_part, part, b, qrow_out, h, (int64_t)pl->n_qtiles * kTile, dq, pl->scale, hi);
+  store_result(&pl->rows, pl->rows.out0, pl->rows.o0s.b, pl->rows.o0s.s, pl->rows.o0s.h, pl->n_heads, part, b, qrow_out, h,
+               (int64_t)pl->n_qtiles * kTile, dq, pl->scale, hi);
+}
+
+// ---- kernels ------------------------------------------------------------------------------------
+__global__ __launch_bounds__(256, 2) void dkdv_kernel(const BwdParams p) {
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[kDkdvLdsBytes];
+  dkdv_walk(p, (uint32_t)(uintptr_t)(UA_LDS unsigned char*)smem, blockIdx.x);
+}
+__global__ __launch_bounds__(256, 2) void dq_kernel(const BwdParams p) {
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[4 * kHalfPitch];
+  dq_walk(p, (uint32_t)(uintptr_t)(UA_LDS unsigned char*)smem, blockIdx.x);
+}
+// Both sides in one launch.
+__global__ __launch_bounds__(256, 2) void bwd_kernel(const BwdParams p) {
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[kDkdvLdsBytes];
+  const uint32_t lds_base = (uint32_t)(uintptr_t)(UA_LDS unsigned char*)smem;
+  if ((int)blockIdx.x < p.n_col_blocks) dkdv_walk(p, lds_base, blockIdx.x);
+  else                                  dq_walk(p, lds_base, blockIdx.x - p.n_col_blocks);
 }
 
 static int fill_common(BwdParams& p, const void* q, const void* k, const void* v, const void* dout,
-                       const float* lse, const float* delta, const int32_t* idx, const uint8_t* flag,
+                       const float* lse, const float* delta,
                        int batch, int n_heads, int n_qtiles,
                        int n_ktiles, int nnz, int head_dim, const int64_t* qs, const int64_t* ks,
                        const int64_t* vs, const int64_t* ds, float softmax_scale) {
   if (!q || !k || !v || !dout || !lse || !delta || !qs || !ks || !vs || !ds) return UA_ERR_NULL;
   if (batch <= 0 || n_heads <= 0 || n_qtiles <= 0 || n_ktiles <= 0 || nnz < 0) return UA_ERR_SHAPE;
-  if (nnz > 0 && (!idx || !flag)) return UA_ERR_NULL;          // only an empty list may leave them out
-  if (flag && !aligned4(flag)) return UA_ERR_ALIGN;            // read one aligned 32-bit word at a time
-  if ((int64_t)batch * n_heads * n_qtiles * UA_MAX_PARTS > INT32_MAX ||
-      (int64_t)batch * n_heads * n_ktiles * UA_MAX_PARTS > INT32_MAX) return UA_ERR_SHAPE;
+  if ((int64_t)batch * n_heads * n_qtiles * UA_MAX_PARTS > INT32_MAX / 2 ||
+      (int64_t)batch * n_heads * n_ktiles * UA_MAX_PARTS > INT32_MAX / 2) return UA_ERR_SHAPE;
   if (head_dim != kHeadDim || !(softmax_scale > 0.f)) return UA_ERR_UNSUPPORTED;
   if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(dout)) return UA_ERR_ALIGN;
   if (!strides_ok(qs) || !strides_ok(ks) || !strides_ok(vs) || !strides_ok(ds)) return UA_ERR_ALIGN;
@@ -523,18 +542,67 @@ static int fill_common(BwdParams& p, const void* q, const void* k, const void* v
   p.scale = softmax_scale; p.scale_log2 = softmax_scale * kLog2e;
   const int nbh = batch * n_heads;
   p.heads_per_xcd = (nbh % 8 == 0) ? nbh / 8 : 0;
-  p.ptr = nullptr; p.idx = idx; p.flag = flag; p.order = nullptr;
-  p.dense = 0; p.dense_causal = 0; p.diag_off = 0; p.n_parts = 1; p.part_len = 0; p.out_f32 = 0; p.o0_part = 0; p.o1_part = 0;
-  return check_device();
+  p.dense = 0; p.dense_causal = 0; p.diag_off = 0; p.n_col_blocks = 0;
+  p.cols = BwdSide{}; p.rows = BwdSide{};
+  p.cols.n_parts = p.rows.n_parts = 1;
+  return UA_OK;
 }
 
-static int launch_dkdv(const BwdParams& p, hipStream_t st) {
-  hipLaunchKernelGGL(dkdv_kernel, dim3((unsigned)(p.batch * p.n_heads * p.n_ktiles * p.n_parts)), dim3(256), 0, st, p);
-  return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH;
+// List arrays and outputs of one side (out1 = NULL on the rows' side).
+static int fill_side(BwdSide& s, int nnz, const int32_t* ptr, const int32_t* idx, const uint8_t* flag, const int32_t* order, void* out0,
+                     const int64_t* o0s, void* out1, const int64_t* o1s, bool dense) {
+  if (nnz > 0 && (!idx || !flag)) return UA_ERR_NULL;          // only an empty list may leave them out
+  if (flag && !aligned4(flag)) return UA_ERR_ALIGN;            // read one aligned 32-bit word at a time
+  if (!out0 || !o0s || (o1s && !out1) || (!dense && (!ptr || !order))) return UA_ERR_NULL;
+  if (!aligned16(out0) || !strides_ok(o0s) || (o1s && (!aligned16(out1) || !strides_ok(o1s)))) return UA_ERR_ALIGN;
+  s.ptr = ptr; s.idx = idx; s.flag = flag; s.order = order;
+  s.out0 = (bf16*)out0; s.out1 = (bf16*)out1;
+  s.o0s = {o0s[0], o0s[1], o0s[2]};
+  if (o1s) s.o1s = {o1s[0], o1s[1], o1s[2]};
+  return UA_OK;
 }
-static int launch_dq(const BwdParams& p, hipStream_t st) {
-  hipLaunchKernelGGL(dq_kernel, dim3((unsigned)(p.batch * p.n_heads * p.n_qtiles * p.n_parts)), dim3(256), 0, st, p);
-  return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH;
+
+static int launched() { return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH; }
+static unsigned col_blocks(const BwdParams& p) { return (unsigned)(p.batch * p.n_heads * p.n_ktiles * p.cols.n_parts); }
+static unsigned row_blocks(const BwdParams& p) { return (unsigned)(p.batch * p.n_heads * p.n_qtiles * p.rows.n_parts); }
+static int launch_bwd(BwdParams& p, hipStream_t st) {
+  p.n_col_blocks = (int)col_blocks(p);
+  hipLaunchKernelGGL(bwd_kernel, dim3(col_blocks(p) + row_blocks(p)), dim3(256), 0, st, p);
+  return launched();
+}
+
+// How many parts the two sides of a dense backward are cut into, at most what the workspace holds.  A cut gives a
+// small rectangle enough workgroups for the device and costs the partials' way through memory and a
+// second launch; which wins is decided by an estimate of the launch's time in microseconds, fitted to 20 shapes of 1
+// to 32 heads and 512 to 8192 tokens (each within 8 % of its best cut):
+//  - 8.4 to start, load the resident rows, store the results and end;
+//  - a workgroup alone on its CU walks a tile in 3.4 (columns) or 2.4 (rows), two that share it in 6.6 and 4.3 each;
+//  - the sum takes 2.3, and the partials 1 per 3.7 MB.
+// 512 x 512, 32 heads: 40 us cut in two, 24 uncut; 1024 x 4096, one head: 84 uncut, 26 cut in 4 and 8.
+struct BwdCut { int cols, rows; };
+static BwdCut bwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int max_cols, int max_rows) {
+  if (max_cols <= 1 && max_rows <= 1) return {1, 1};
+  static constexpr int kParts[] = {1, 2, 3, 4, 6, 8, 12, 16};
+  const float density = causal ? 0.5f : 1.f, wk = (float)nbh * n_ktiles, wq = (float)nbh * n_qtiles;
+  BwdCut best = {1, 1};
+  float best_us = INFINITY;
+  for (int pc : kParts) {
+    if (pc > max_cols) break;
+    for (int pr : kParts) {
+      if (pr > max_rows) break;
+      const float groups = (wk * pc + wq * pr) * density;
+      const float shared = fminf(fmaxf((groups - 256.f) / 256.f, 0.f), 1.f);       // share of the workgroups with a neighbour
+      const float tc = 3.4f + 3.2f * shared, tr = 2.4f + 1.9f * shared;
+      const float longest = fmaxf((float)((n_qtiles + pc - 1) / pc) * tc, (float)((n_ktiles + pr - 1) / pr) * tr);
+      const float all = density * wk * n_qtiles * (6.6f + 4.3f) / 512.f;
+      float us = 8.4f + fmaxf(longest, all);
+      if (pc > 1 || pr > 1) us += 2.3f;
+      if (pc > 1) us += 2.f * pc * wk * (kTile * kHeadDim * 4) / 3.7e6f;
+      if (pr > 1) us += pr * wq * (kTile * kHeadDim * 4) / 3.7e6f;
+      if (us < best_us) { best_us = us; best = {pc, pr}; }
+    }
+  }
+  return best;
 }
 
 }  // namespace ua
@@ -549,15 +617,13 @@ extern "C" int ua_bsa_bwd_dkdv(const void* q, const void* k, const void* v, cons
                                float softmax_scale, void* stream) {
   using namespace ua;
   BwdParams p;
-  if (int rc = fill_common(p, q, k, v, dout, lse, delta, row_idx, cflag, batch, n_heads, n_qtiles, n_ktiles, nnz,
-                           head_dim, q_strides, k_strides, v_strides, do_strides, softmax_scale)) return rc;
-  if (!dk || !dv || !col_ptr || !k_order || !dk_strides || !dv_strides) return UA_ERR_NULL;
-  if (!aligned16(dk) || !aligned16(dv) || !strides_ok(dk_strides) || !strides_ok(dv_strides)) return UA_ERR_ALIGN;
-  p.out0 = (bf16*)dk; p.out1 = (bf16*)dv;
-  p.o0s = {dk_strides[0], dk_strides[1], dk_strides[2]};
-  p.o1s = {dv_strides[0], dv_strides[1], dv_strides[2]};
-  p.ptr = col_ptr; p.idx = row_idx; p.flag = cflag; p.order = k_order;
-  return launch_dkdv(p, (hipStream_t)stream);
+  if (int rc = fill_common(p, q, k, v, dout, lse, delta, batch, n_heads, n_qtiles, n_ktiles, nnz, head_dim, q_strides, k_strides,
+                           v_strides, do_strides, softmax_scale)) return rc;
+  if (!dv_strides) return UA_ERR_NULL;
+  if (int rc = fill_side(p.cols, nnz, col_ptr, row_idx, cflag, k_order, dk, dk_strides, dv, dv_strides, false)) return rc;
+  if (int rc = check_device()) return rc;
+  hipLaunchKernelGGL(dkdv_kernel, dim3(col_blocks(p)), dim3(256), 0, (hipStream_t)stream, p);
+  return launched();
 }
 
 extern "C" int ua_bsa_bwd_dq(const void* q, const void* k, const void* v, const void* dout,
@@ -570,15 +636,31 @@ extern "C" int ua_bsa_bwd_dq(const void* q, const void* k, const void* v, const 
                              float softmax_scale, void* stream) {
   using namespace ua;
   BwdParams p;
-  if (int rc = fill_common(p, q, k, v, dout, lse, delta, col_idx, flag, batch, n_heads, n_qtiles, n_ktiles, nnz,
-                           head_dim, q_strides, k_strides, v_strides, do_strides, softmax_scale)) return rc;
-  if (!dq || !row_ptr || !q_order || !dq_strides) return UA_ERR_NULL;
-  if (!aligned16(dq) || !strides_ok(dq_strides)) return UA_ERR_ALIGN;
-  p.out0 = (bf16*)dq; p.out1 = nullptr;
-  p.o0s = {dq_strides[0], dq_strides[1], dq_strides[2]};
-  p.o1s = p.o0s;
-  p.ptr = row_ptr; p.idx = col_idx; p.flag = flag; p.order = q_order;
-  return launch_dq(p, (hipStream_t)stream);
+  if (int rc = fill_common(p, q, k, v, dout, lse, delta, batch, n_heads, n_qtiles, n_ktiles, nnz, head_dim, q_strides, k_strides,
+                           v_strides, do_strides, softmax_scale)) return rc;
+  if (int rc = fill_side(p.rows, nnz, row_ptr, col_idx, flag, q_order, dq, dq_strides, nullptr, nullptr, false)) return rc;
+  if (int rc = check_device()) return rc;
+  hipLaunchKernelGGL(dq_kernel, dim3(row_blocks(p)), dim3(256), 0, (hipStream_t)stream, p);
+  return launched();
+}
+
+extern "C" int ua_bsa_bwd(const void* q, const void* k, const void* v, const void* dout,
+                          const float* lse, const float* delta, void* dq, void* dk, void* dv,
+                          const int32_t* row_ptr, const int32_t* col_idx, const uint8_t* flag, const int32_t* q_order,
+                          const int32_t* col_ptr, const int32_t* row_idx, const uint8_t* cflag, const int32_t* k_order,
+                          int batch, int n_heads, int n_qtiles, int n_ktiles, int nnz, int head_dim,
+                          const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides,
+                          const int64_t* do_strides, const int64_t* dq_strides, const int64_t* dk_strides,
+                          const int64_t* dv_strides, float softmax_scale, void* stream) {
+  using namespace ua;
+  BwdParams p;
+  if (int rc = fill_common(p, q, k, v, dout, lse, delta, batch, n_heads, n_qtiles, n_ktiles, nnz, head_dim, q_strides, k_strides,
+                           v_strides, do_strides, softmax_scale)) return rc;
+  if (!dv_strides) return UA_ERR_NULL;
+  if (int rc = fill_side(p.cols, nnz, col_ptr, row_idx, cflag, k_order, dk, dk_strides, dv, dv_strides, false)) return rc;
+  if (int rc = fill_side(p.rows, nnz, row_ptr, col_idx, flag, q_order, dq, dq_strides, nullptr, nullptr, false)) return rc;
+  if (int rc = check_device()) return rc;
+  return launch_bwd(p, (hipStream_t)stream);
 }
 
 extern "C" int ua_dense_bwd(const void* dout, const void* q, const void* k, const void* v,
@@ -591,62 +673,42 @@ extern "C" int ua_dense_bwd(const void* dout, const void* q, const void* k, cons
   using namespace ua;
   if (seqlen_q <= 0 || seqlen_k <= 0 || seqlen_q % kTile || seqlen_k % kTile) return UA_ERR_SHAPE;
   const int n_qtiles = seqlen_q / kTile, n_ktiles = seqlen_k / kTile;
-  if (!dq || !dk || !dv || !dq_strides || !dk_strides || !dv_strides) return UA_ERR_NULL;
-  if (!aligned16(dq) || !aligned16(dk) || !aligned16(dv) || !strides_ok(dq_strides) || !strides_ok(dk_strides) ||
-      !strides_ok(dv_strides)) return UA_ERR_ALIGN;
+  if (!dv_strides) return UA_ERR_NULL;
   BwdParams p;
-  if (int rc = fill_common(p, q, k, v, dout, lse, delta, nullptr, nullptr, batch, n_heads, n_qtiles, n_ktiles, 0,
-                           head_dim, q_strides, k_strides, v_strides, do_strides, softmax_scale)) return rc;
+  if (int rc = fill_common(p, q, k, v, dout, lse, delta, batch, n_heads, n_qtiles, n_ktiles, 0, head_dim, q_strides, k_strides,
+                           v_strides, do_strides, softmax_scale)) return rc;
+  if (int rc = fill_side(p.cols, 0, nullptr, nullptr, nullptr, nullptr, dk, dk_strides, dv, dv_strides, true)) return rc;
+  if (int rc = fill_side(p.rows, 0, nullptr, nullptr, nullptr, nullptr, dq, dq_strides, nullptr, nullptr, true)) return rc;
+  if (int rc = check_device()) return rc;
   hipStream_t st = (hipStream_t)stream;
   p.dense = 1; p.dense_causal = causal != 0; p.diag_off = n_ktiles - n_qtiles;
+  p.cols.part_len = n_qtiles; p.rows.part_len = n_ktiles;
   const DenseSplit d = dense_split(batch, n_heads, n_qtiles, n_ktiles);
   unsigned char* ws = static_cast<unsigned char*>(workspace);
   const bool ws_ok = workspace && aligned16(workspace) && workspace_bytes >= d.bwd_total;
-  const void* parts[UA_MAX_PARTS];
-
-  // dK, dV: one workgroup per (key tile, head) walks the query tiles; few key tiles -> parts of the query range
-  {
-    BwdParams c = p;
-    c.out0 = (bf16*)dk; c.out1 = (bf16*)dv;
-    c.o0s = {dk_strides[0], dk_strides[1], dk_strides[2]};
-    c.o1s = {dv_strides[0], dv_strides[1], dv_strides[2]};
-    c.part_len = n_qtiles;
-    if (d.dkdv_parts > 1 && ws_ok) {
-      const int len = (n_qtiles + d.dkdv_parts - 1) / d.dkdv_parts;
-      const int n = (n_qtiles + len - 1) / len;
-      float* base = reinterpret_cast<float*>(ws);
-      ws += (int64_t)d.dkdv_parts * d.dkdv_bytes;
-      c.n_parts = n; c.part_len = len; c.out_f32 = 1;
-      c.o0_part = c.o1_part = d.dkdv_bytes / 4;
-      c.out0 = reinterpret_cast<bf16*>(base);
-      c.out1 = reinterpret_cast<bf16*>(base + d.dkdv_bytes / 8);
-      if (int rc = launch_dkdv(c, st)) return rc;
-      for (int i = 0; i < n; ++i) parts[i] = base + i * c.o0_part;
-      if (int rc = launch_grad_sum(parts, n, true, dk, dk_strides, batch, seqlen_k, n_heads, 1.f, st)) return rc;
-      for (int i = 0; i < n; ++i) parts[i] = base + d.dkdv_bytes / 8 + i * c.o1_part;
-      if (int rc = launch_grad_sum(parts, n, true, dv, dv_strides, batch, seqlen_k, n_heads, 1.f, st)) return rc;
-    } else if (int rc = launch_dkdv(c, st)) {
-      return rc;
-    }
+  // Cut one side: parts of equal length, fp32 partials in the workspace.
+  auto cut = [&](BwdSide& s, int parts, int list_len, int64_t part_bytes) {
+    s.part_len = (list_len + parts - 1) / parts;
+    s.n_parts = (list_len + s.part_len - 1) / s.part_len;
+    s.out_f32 = 1;
+    s.o_part = part_bytes / 4;
+    s.out0 = reinterpret_cast<bf16*>(ws);
+    s.out1 = reinterpret_cast<bf16*>(ws + part_bytes / 2);       // columns: dV behind dK
+    ws += parts * part_bytes;
+  };
+  const BwdCut n = ws_ok ? bwd_cut((int64_t)batch * n_heads, n_qtiles, n_ktiles, p.dense_causal, d.dkdv_parts, d.dq_parts) : BwdCut{1, 1};
+  if (n.cols > 1) cut(p.cols, n.cols, n_qtiles, d.dkdv_bytes);
+  if (n.rows > 1) cut(p.rows, n.rows, n_ktiles, d.dq_bytes);
+  if (int rc = launch_bwd(p, st)) return rc;
+  PartialSum sums[3];
+  int n_sums = 0;
+  auto add_sum = [&](const BwdSide& s, const bf16* first, void* out, const int64_t* os, int seqlen) {
+    sums[n_sums++] = {reinterpret_cast<const float*>(first), (bf16*)out, s.o_part, s.n_parts, seqlen, {os[0], os[1], os[2]}};
+  };
+  if (p.cols.out_f32) {
+    add_sum(p.cols, p.cols.out0, dk, dk_strides, seqlen_k);
+    add_sum(p.cols, p.cols.out1, dv, dv_strides, seqlen_k);
   }
-  // dQ: one workgroup per (query tile, head) walks the key tiles; few query tiles -> parts of the key range
-  {
-    BwdParams c = p;
-    c.out0 = (bf16*)dq; c.out1 = nullptr;
-    c.o0s = {dq_strides[0], dq_strides[1], dq_strides[2]};
-    c.o1s = c.o0s;
-    c.part_len = n_ktiles;
-    if (d.dq_parts > 1 && ws_ok) {
-      const int len = (n_ktiles + d.dq_parts - 1) / d.dq_parts;
-      const int n = (n_ktiles + len - 1) / len;
-      float* base = reinterpret_cast<float*>(ws);
-      c.n_parts = n; c.part_len = len; c.out_f32 = 1;
-      c.o0_part = d.dq_bytes / 4;
-      c.out0 = reinterpret_cast<bf16*>(base);
-      if (int rc = launch_dq(c, st)) return rc;
-      for (int i = 0; i < n; ++i) parts[i] = base + i * c.o0_part;
-      return launch_grad_sum(parts, n, true, dq, dq_strides, batch, seqlen_q, n_heads, 1.f, st);
-    }
-    return launch_dq(c, st);
-  }
+  if (p.rows.out_f32) add_sum(p.rows, p.rows.out0, dq, dq_strides, seqlen_q);
+  return n_sums ? launch_partial_sums(sums, n_sums, batch, n_heads, st) : UA_OK;
 }

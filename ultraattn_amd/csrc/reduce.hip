@@ -109,19 +109,50 @@ __global__ __launch_bounds__(kRedThreads) void grad_sum_kernel(const SumParams p
   }
 }
 
-// Shared by ua_grad_sum and the split dense backward: the parts are contiguous [batch, seqlen,
-// n_heads, 128] arrays, the output takes (batch, token, head) element strides.
-int launch_grad_sum(const void* const* parts, int n_parts, bool parts_fp32, void* out, const int64_t* out_strides,
-                    int batch, int seqlen, int n_heads, float scale, hipStream_t st) {
-  SumParams p;
-  for (int i = 0; i < UA_MAX_PARTS; ++i) p.parts[i] = i < n_parts ? parts[i] : nullptr;
-  p.out = (bf16*)out; p.n_parts = n_parts; p.seqlen = seqlen; p.n_heads = n_heads;
-  p.os = {out_strides[0], out_strides[1], out_strides[2]};
-  p.scale = scale;
-  p.n_chunks = (int64_t)batch * seqlen * n_heads * 16;
-  const int blocks = (int)std::min<int64_t>((p.n_chunks + kRedThreads - 1) / kRedThreads, kRedBlocks);
-  if (parts_fp32) hipLaunchKernelGGL(grad_sum_kernel<true>, dim3(blocks), dim3(kRedThreads), 0, st, p);
-  else            hipLaunchKernelGGL(grad_sum_kernel<false>, dim3(blocks), dim3(kRedThreads), 0, st, p);
+// The partial results of one split backward, summed in one launch: the workgroups of sum j follow those of sum
+// j - 1.  The partials were just written and are read from L2; what bounds it at the sizes that split (a few
+// MB) is the latency of one launch and of one round of loads, so all loads of a chunk are issued together.
+struct PartialSumsParams {
+  PartialSum s[3];
+  int first_block[4];
+  int batch, n_heads;
+};
+__global__ __launch_bounds__(kRedThreads) void partial_sums_kernel(const PartialSumsParams p) {
+  const int j = (int)blockIdx.x >= p.first_block[2] ? 2 : ((int)blockIdx.x >= p.first_block[1] ? 1 : 0);
+  const PartialSum& s = p.s[j];
+  const int64_t c = (int64_t)(blockIdx.x - p.first_block[j]) * kRedThreads + threadIdx.x;
+  const int64_t row = c >> 4;
+  if (row >= (int64_t)p.batch * s.seqlen * p.n_heads) return;
+  const float* src = s.base + c * 8;
+  f32x4 x0{0}, x1{0};
+  for (int i0 = 0; i0 < s.n_parts; i0 += 4) {
+    f32x4 a[4], b[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (i0 + u < s.n_parts) {
+        a[u] = *reinterpret_cast<const f32x4*>(src + (i0 + u) * s.stride);
+        b[u] = *reinterpret_cast<const f32x4*>(src + (i0 + u) * s.stride + 4);
+      }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (i0 + u < s.n_parts) { x0 += a[u]; x1 += b[u]; }
+  }
+  const float x[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
+  const int h = (int)(row % p.n_heads);
+  const int64_t t = row / p.n_heads, tok = t % s.seqlen, b = t / s.seqlen;
+  *reinterpret_cast<bf16x8*>(s.out + b * s.os.b + tok * s.os.s + h * s.os.h + (c & 15) * 8) = pack8(x);
+}
+
+int launch_partial_sums(const PartialSum* sums, int n_sums, int batch, int n_heads, hipStream_t st) {
+  PartialSumsParams p{};
+  p.batch = batch; p.n_heads = n_heads;
+  for (int j = 0; j < 3; ++j) {
+    p.first_block[j + 1] = p.first_block[j];
+    if (j >= n_sums) continue;
+    p.s[j] = sums[j];
+    p.first_block[j + 1] += (int)(((int64_t)batch * sums[j].seqlen * n_heads * 16 + kRedThreads - 1) / kRedThreads);
+  }
+  hipLaunchKernelGGL(partial_sums_kernel, dim3(p.first_block[3]), dim3(kRedThreads), 0, st, p);
   return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH;
 }
 
@@ -155,5 +186,15 @@ extern "C" int ua_grad_sum(const void* const* parts, int n_parts, int parts_fp32
     if (!aligned16(parts[i])) return UA_ERR_ALIGN;
   }
   if (int rc = check_device()) return rc;
-  return launch_grad_sum(parts, n_parts, parts_fp32 != 0, out, out_strides, batch, seqlen, n_heads, scale, (hipStream_t)stream);
+  SumParams p;
+  for (int i = 0; i < UA_MAX_PARTS; ++i) p.parts[i] = i < n_parts ? parts[i] : nullptr;
+  p.out = (bf16*)out; p.n_parts = n_parts; p.seqlen = seqlen; p.n_heads = n_heads;
+  p.os = {out_strides[0], out_strides[1], out_strides[2]};
+  p.scale = scale;
+  p.n_chunks = (int64_t)batch * seqlen * n_heads * 16;
+  const int blocks = (int)std::min<int64_t>((p.n_chunks + kRedThreads - 1) / kRedThreads, kRedBlocks);
+  hipStream_t st = (hipStream_t)stream;
+  if (parts_fp32) hipLaunchKernelGGL(grad_sum_kernel<true>, dim3(blocks), dim3(kRedThreads), 0, st, p);
+  else            hipLaunchKernelGGL(grad_sum_kernel<false>, dim3(blocks), dim3(kRedThreads), 0, st, p);
+  return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH;
 }

@@ -201,7 +201,14 @@ inline DenseSplit dense_split(int batch, int n_heads, int n_qtiles, int n_ktiles
   d.bwd_total = (d.dq_parts > 1 ? d.dq_parts * d.dq_bytes : 0) + (d.dkdv_parts > 1 ? d.dkdv_parts * d.dkdv_bytes : 0);
   return d;
 }
-int launch_grad_sum(const void* const* parts, int n_parts, bool parts_fp32, void* out, const int64_t* out_strides,
-                    int batch, int seqlen, int n_heads, float scale, hipStream_t st);
+// One sum of fp32 partial results (contiguous [batch, seqlen, n_heads, 128], part i at base + i * stride floats)
+// into a strided bf16 tensor; up to three of them run in one launch.
+struct PartialSum {
+  const float* base; bf16* out;
+  int64_t stride;
+  int n_parts, seqlen;
+  Strides3 os;
+};
+int launch_partial_sums(const PartialSum* sums, int n_sums, int batch, int n_heads, hipStream_t st);
 
 }  // namespace ua

@@ -139,20 +139,13 @@ def bsa_bwd(dout, q, k, v, out, lse, tiles, softmax_scale: Optional[float] = Non
     lib = _lib.load()
     with torch.cuda.device(q.device):
         st = torch.cuda.current_stream().cuda_stream
-        rc = lib.ua_bsa_bwd_dkdv(q.data_ptr(), k.data_ptr(), v.data_ptr(), dout.data_ptr(), lse.data_ptr(),
-                                 softmax_d.data_ptr(), dk.data_ptr(), dv.data_ptr(),
-                                 d["col_ptr"].data_ptr(), d["row_idx"].data_ptr(), d["cflag"].data_ptr(),
-                                 d["k_order"].data_ptr(), B, Nh, tl.n_qtiles, tl.n_ktiles, tl.nnz, D,
-                                 _lib.strides3(q), _lib.strides3(k), _lib.strides3(v), _lib.strides3(dout),
-                                 _lib.strides3(dk), _lib.strides3(dv), float(softmax_scale), st)
-        _lib.check(rc, "ua_bsa_bwd_dkdv")
-        rc = lib.ua_bsa_bwd_dq(q.data_ptr(), k.data_ptr(), v.data_ptr(), dout.data_ptr(), lse.data_ptr(),
-                               softmax_d.data_ptr(), dq.data_ptr(),
-                               d["row_ptr"].data_ptr(), d["col_idx"].data_ptr(), d["flag"].data_ptr(),
-                               d["q_order"].data_ptr(), B, Nh, tl.n_qtiles, tl.n_ktiles, tl.nnz, D,
-                               _lib.strides3(q), _lib.strides3(k), _lib.strides3(v), _lib.strides3(dout),
-                               _lib.strides3(dq), float(softmax_scale), st)
-        _lib.check(rc, "ua_bsa_bwd_dq")
+        rc = lib.ua_bsa_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), dout.data_ptr(), lse.data_ptr(), softmax_d.data_ptr(),
+                            dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+                            *(d[n].data_ptr() for n in ("row_ptr", "col_idx", "flag", "q_order", "col_ptr", "row_idx", "cflag", "k_order")),
+                            B, Nh, tl.n_qtiles, tl.n_ktiles, tl.nnz, D,
+                            _lib.strides3(q), _lib.strides3(k), _lib.strides3(v), _lib.strides3(dout),
+                            _lib.strides3(dq), _lib.strides3(dk), _lib.strides3(dv), float(softmax_scale), st)
+        _lib.check(rc, "ua_bsa_bwd")
     return dq, dk, dv
 
 
