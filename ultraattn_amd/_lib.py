@@ -1,4 +1,5 @@
-"""ctypes binding of ``libultraattn_hip.so`` (the C ABI declared in ``include/ultraattn.h``).
+"""ctypes binding of ``libultraattn_hip.so`` (the C ABI declared in ``include/ultraattn.h``) and the
+loader of ``_native.so``, which calls the same ABI for the operators on torch tensors.
 
 There is no fallback: if the library has not been built, loading raises.
 """
@@ -6,7 +7,7 @@ import ctypes
 import os
 from ctypes import POINTER, c_char_p, c_float, c_int, c_int32, c_int64, c_uint8, c_void_p
 
-from .build import LIB_PATH
+from .build import LIB_PATH, NATIVE_PATH
 
 _i32p, _u8p, _i64p = POINTER(c_int32), POINTER(c_uint8), POINTER(c_int64)
 
@@ -53,6 +54,22 @@ def load() -> ctypes.CDLL:
             fn.restype, fn.argtypes = res, args
         _lib = lib
     return _lib
+
+
+_native = None
+
+
+def native():
+    """The native host side of the operators (``csrc/native.cpp``), loaded once behind the library."""
+    global _native
+    if _native is None:
+        load()
+        if not os.path.exists(NATIVE_PATH):
+            raise RuntimeError(f"{NATIVE_PATH} is missing: build it with `python -m ultraattn_amd.build`")
+        import torch  # noqa: F401  (its libraries hold the symbols that the module needs)
+        from . import _native as module
+        _native = module
+    return _native
 
 
 def check(rc: int, what: str) -> None:

@@ -1,5 +1,5 @@
 """Build step: compile the HIP sources in ``csrc/`` for gfx950 into ``libultraattn_hip.so``
-next to this file.  Run ``python -m ultraattn_amd.build`` (hipcc cross-compiles without a GPU).
+and the Python binding ``csrc/native.cpp`` into ``_native.so`` next to this file.  Run ``python -m ultraattn_amd.build`` (hipcc cross-compiles without a GPU).
 """
 import os
 import subprocess
@@ -9,6 +9,7 @@ PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_NAME = "libultraattn_hip.so"
 LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
+NATIVE_PATH = os.path.join(PKG_DIR, "_native.so")
 SOURCES = ["api.hip", "tilelist.hip", "merge.hip", "glue.hip", "reduce.hip", "fwd.hip", "bwd.hip"]
 # benchmark-only probes (register-only MFMA loop, streaming-mix ceiling): built beside bench.py,
 # never linked into the product library
@@ -26,8 +27,22 @@ def hipcc_path() -> str:
     return "hipcc"
 
 
+def _native_command():
+    """Host compiler line of the Python binding: it uses torch's C++ tensors and calls the shared library beside it."""
+    import sysconfig
+    import torch
+    root = os.path.dirname(torch.__file__)
+    lib = os.path.join(root, "lib")
+    return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
+            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            *(x for d in (os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+                          "/opt/rocm/include", sysconfig.get_paths()["include"]) for x in ("-isystem", d)),
+            os.path.join(CSRC, "native.cpp"), "-o", NATIVE_PATH, f"-L{PKG_DIR}", f"-l:{LIB_NAME}", "-Wl,-rpath,$ORIGIN",
+            f"-L{lib}", "-ltorch_python", "-ltorch_cpu", "-lc10_hip", "-lc10"]
+
+
 def build_library(verbose: bool = False, jobs: int = 4) -> str:
-    """Compile every source and link the shared library; returns its path."""
+    """Compile every source, link the shared library and the Python binding; returns the library's path."""
     objdir = os.path.join(PKG_DIR, "build")
     os.makedirs(objdir, exist_ok=True)
     procs = []
@@ -51,10 +66,13 @@ def build_library(verbose: bool = False, jobs: int = 4) -> str:
         if verbose and out.strip():
             print(out)
         objs.append(obj)
-    cmd = [hipcc_path(), "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", LIB_PATH]
-    r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
-    if r.returncode != 0:
-        raise RuntimeError(f"link failed:\n{r.stdout}")
+    link = [hipcc_path(), "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", LIB_PATH]
+    for cmd in (link, _native_command()):
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+        if r.returncode != 0:
+            raise RuntimeError(f"{cmd[0]} failed:\n{r.stdout}")
     return LIB_PATH
 
 

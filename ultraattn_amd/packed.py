@@ -13,6 +13,8 @@ from typing import Iterable, Optional, Tuple
 
 import torch
 
+from ._lib import native
+
 FULL_DTYPE = torch.float32          # orchestrated_attn/global_vars.py:4
 
 
@@ -184,24 +186,6 @@ class OutputColBwd(_Fp32Accumulated):
         self.dV = self.data[n:].view(k_shape)
 
 
-def _permute_cols(entry: str, src: torch.Tensor, n_chunks: int, k_shape, out: torch.Tensor = None) -> torch.Tensor:
-    from . import _lib
-    B, S, Nh, D = k_shape
-    inner = S * Nh * D
-    n = 2 * n_chunks * B * inner
-    if src.dim() != 1 or src.dtype != torch.bfloat16 or not src.is_cuda or src.numel() < n:
-        raise ValueError(f"the column buffer must be a flat bfloat16 CUDA tensor of at least {n} elements")
-    out = torch.empty(n, dtype=torch.bfloat16, device=src.device) if out is None else out
-    if out.dim() != 1 or out.dtype != torch.bfloat16 or out.device != src.device or out.numel() < n:
-        raise ValueError(f"out must be a flat bfloat16 tensor of at least {n} elements on the source's device")
-    lib = _lib.load()
-    with torch.cuda.device(src.device):
-        st = torch.cuda.current_stream().cuda_stream
-        rc = getattr(lib, entry)(src.data_ptr(), out.data_ptr(), n_chunks, B, inner, st)
-    _lib.check(rc, entry)
-    return out
-
-
 def gather_cols(buf: torch.Tensor, n_chunks: int, k_shape, out: torch.Tensor = None) -> InputColFwd:
     """Fused-rectangle column input: ``buf`` holds ``n_chunks`` received column chunks, each
     ``[K | V]`` of shape ``k_shape`` (B, Skv, Nh, D): ``[Y, 2, B, Skv, Nh, D]``.  Returns the
@@ -210,7 +194,7 @@ def gather_cols(buf: torch.Tensor, n_chunks: int, k_shape, out: torch.Tensor = N
     ``view(Y,2,B,Skv,Nh,D).transpose(0,1).transpose(1,2).flatten(2,3).contiguous()``
     (``orchestrated_attn/orchestrated_attn_impl.py:269, 512``)."""
     B, S, Nh, D = k_shape
-    data = _permute_cols("ua_cols_gather", buf, n_chunks, k_shape, out)
+    data = native().permute_cols(buf, out, n_chunks, B, S * Nh * D, True)
     return InputColFwd(data, (B, n_chunks * S, Nh, D))
 
 
@@ -220,7 +204,8 @@ def scatter_cols(col_out: OutputColBwd, n_chunks: int, k_shape, out: torch.Tenso
     of per-chunk ``[dK | dV]`` that the column reduce-scatter sends
     (``oc.view(2, Y, K_nelem).transpose(0,1).contiguous()``,
     ``orchestrated_attn/orchestrated_attn_impl.py:548``)."""
-    return _permute_cols("ua_cols_scatter", col_out.data, n_chunks, k_shape, out)
+    B, S, Nh, D = k_shape
+    return native().permute_cols(col_out.data, out, n_chunks, B, S * Nh * D, False)
 
 
 def _scaled(shape: Tuple[int, int, int, int], n_chunks: int) -> Tuple[int, int, int, int]:

@@ -50,7 +50,7 @@ class TileList:
     def on(self, device):
         """Device copies of all arrays as torch tensors (cached per device)."""
         import torch
-        key = str(torch.device(device))
+        key = torch.device(device)
         if key not in self._dev:
             if torch.cuda.is_current_stream_capturing():
                 # the staging buffers are released once the copies are done: a graph must not replay them
@@ -81,6 +81,14 @@ class TileList:
             else:                           # a later use on another stream orders itself behind the copies
                 torch.cuda.current_stream().wait_event(ready)
         return dev
+
+
+    def lists(self, device):
+        """The arrays of ``on(device)`` as one tuple in the order of the C ABI."""
+        dev = self.on(device)
+        if "_lists" not in dev:
+            dev["_lists"] = tuple(dev[n] for n in _HOST_FIELDS)
+        return dev["_lists"]
 
 
 def build_tile_list(block_mask, block: int = 512, tile: int = TILE, causal: bool = False,
