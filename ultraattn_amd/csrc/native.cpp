@@ -16,6 +16,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <cmath>
+#include <cstring>
 #include <mutex>
 #include <string>
 #include "../../include/ultraattn.h"
@@ -273,17 +274,27 @@ PyObject* dense_backward(PyObject* const* a) {
   return tuple_of(x.dq, x.dk, x.dv, x.delta);
 }
 
-// The device arrays of a tile list: tuple in the order of the C ABI (row_ptr, col_idx, flag, col_ptr, row_idx, cflag, q_order, k_order).
+// Tile lists in one device buffer of 32-bit words: row_ptr, col_ptr, q_order, k_order, col_idx, row_idx, flag, cflag (the
+// flags four to a word), so that a list travels in one copy.
 struct Lists {
-  const int32_t *row_ptr, *col_idx, *col_ptr, *row_idx, *q_order, *k_order;
+  int64_t at[9];             // first word of each array; at[8] = words in all
+  const int32_t *row_ptr, *col_ptr, *q_order, *k_order, *col_idx, *row_idx;
   const uint8_t *flag, *cflag;
-  explicit Lists(PyObject* t) {
-    if (!PyTuple_Check(t) || PyTuple_GET_SIZE(t) != 8) fail(PyExc_TypeError, "the tile list must be a tuple of 8 tensors");
-    const void* p[8];
-    for (int i = 0; i < 8; ++i) p[i] = tensor(PyTuple_GET_ITEM(t, i), "tile list").data_ptr();
-    row_ptr = (const int32_t*)p[0]; col_idx = (const int32_t*)p[1]; flag = (const uint8_t*)p[2];
-    col_ptr = (const int32_t*)p[3]; row_idx = (const int32_t*)p[4]; cflag = (const uint8_t*)p[5];
-    q_order = (const int32_t*)p[6]; k_order = (const int32_t*)p[7];
+  Lists(int64_t nqt, int64_t nkt, int64_t nnz) {
+    const int64_t words[8] = {nqt + 1, nkt + 1, nqt, nkt, nnz, nnz, (nnz + 3) / 4, (nnz + 3) / 4};
+    at[0] = 0;
+    for (int i = 0; i < 8; ++i) at[i + 1] = at[i] + words[i];
+  }
+  void point_into(const void* base) {
+    const int32_t* p = (const int32_t*)base;
+    row_ptr = p + at[0]; col_ptr = p + at[1]; q_order = p + at[2]; k_order = p + at[3]; col_idx = p + at[4]; row_idx = p + at[5];
+    flag = (const uint8_t*)(p + at[6]); cflag = (const uint8_t*)(p + at[7]);
+  }
+  Lists(PyObject* buf, int64_t nqt, int64_t nkt, int64_t nnz) : Lists(nqt, nkt, nnz) {
+    const at::Tensor& t = tensor(buf, "tile list");
+    if (nqt <= 0 || nkt <= 0 || nnz < 0 || !t.is_cuda() || t.scalar_type() != at::kInt || !t.is_contiguous() || t.numel() < at[8])
+      fail(PyExc_ValueError, "the tile list must be a contiguous int32 CUDA tensor that holds all of its arrays");
+    point_into(t.data_ptr());
   }
 };
 void check_grid(const at::Tensor& q, const at::Tensor& k, int64_t nqt, int64_t nkt) {
@@ -297,8 +308,8 @@ void check_grid(const at::Tensor& q, const at::Tensor& k, int64_t nqt, int64_t n
 PyObject* bsa_forward(PyObject* const* a) {
   const at::Tensor &q = tensor(a[0], "q"), &k = tensor(a[1], "k"), &v = tensor(a[2], "v");
   check_qkv(q, k, v);
-  const Lists l(a[3]);
   const int64_t nqt = integer(a[4]), nkt = integer(a[5]), nnz = integer(a[6]);
+  const Lists l(a[3], nqt, nkt, nnz);
   check_grid(q, k, nqt, nkt);
   const float scale = scale_of(a[7]);
   Slot out(a[8]), lse(a[9]);
@@ -322,8 +333,8 @@ PyObject* bsa_forward(PyObject* const* a) {
 
 // bsa_backward(dout, q, k, v, out, lse, dq, dk, dv, softmax_d, lists, n_qtiles, n_ktiles, nnz, softmax_scale) -> (dq, dk, dv)
 PyObject* bsa_backward(PyObject* const* a) {
-  const Lists l(a[10]);
   const int64_t nqt = integer(a[11]), nkt = integer(a[12]), nnz = integer(a[13]);
+  const Lists l(a[10], nqt, nkt, nnz);
   const float scale = scale_of(a[14]);
   BwdArgs x(a, "lse");
   check_grid(x.q, x.k, nqt, nkt);
@@ -337,6 +348,88 @@ PyObject* bsa_backward(PyObject* const* a) {
                       scale, on.stream);
   });
   return tuple_of(x.dq, x.dk, x.dv);
+}
+
+// ---- tile lists ---------------------------------------------------------------------------------------
+at::Tensor pinned(int64_t n, at::ScalarType dt) { return at::empty({n}, at::TensorOptions().dtype(dt).pinned_memory(true)); }
+at::Tensor to_device(const at::Tensor& host, int device) {      // asynchronous; torch keeps the pinned block until the copy is done
+  return host.to(at::Device(at::kCUDA, (c10::DeviceIndex)device), host.scalar_type(), /*non_blocking=*/true);
+}
+
+// lists_from_mask(mask, rows, columns, rate, device) -> (buffer, n_qtiles, n_ktiles, nnz): the lists of a mask that comes with the
+// call (mask: host bytes, row major).
+//
+// A short list is built here and copied over: the device then does nothing but the copy (2 us), while
+// the host still is far ahead of the kernel that will use it.  Host time grows with the list (44 us at 1000
+// tiles, 110 at 8000, 820 at 74000); from kHostTiles on the mask is copied instead and the device builds the
+// list in about 20 us.
+constexpr int64_t kHostTiles = 4096;
+PyObject* lists_from_mask(PyObject* const* a) {
+  const int64_t nqb = integer(a[1]), nkb = integer(a[2]), rate = integer(a[3]), device = integer(a[4]);
+  struct View {
+    Py_buffer b;
+    explicit View(PyObject* o) { if (PyObject_GetBuffer(o, &b, PyBUF_C_CONTIGUOUS)) throw PyError(); }
+    ~View() { PyBuffer_Release(&b); }
+  } mask(a[0]);
+  if (nqb <= 0 || nkb <= 0 || mask.b.len != nqb * nkb) fail(PyExc_ValueError, "the block mask must hold rows * columns bytes");
+  const uint8_t* bytes = (const uint8_t*)mask.b.buf;
+  int64_t nqt, nkt, nnz;
+  check_rc(ua_tilelist_size(bytes, (int)nqb, (int)nkb, (int)rate, &nqt, &nkt, &nnz), "ua_tilelist_size");
+  const int before = c10::hip::current_device();
+  struct Restore { int d; ~Restore() { if (c10::hip::current_device() != d) c10::hip::set_device(d); } } restore{before};
+  if (device != before) c10::hip::set_device((int)device);
+  if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None)
+    fail(PyExc_RuntimeError, "a tile list must be built before the stream is captured into a graph");
+  Lists l(nqt, nkt, nnz);
+  at::Tensor buf;
+  if (nnz <= kHostTiles) {
+    const at::Tensor host = pinned(l.at[8], at::kInt);
+    l.point_into(host.data_ptr());
+    call("ua_tilelist_build", [&] {
+      return ua_tilelist_build(bytes, (int)nqb, (int)nkb, (int)rate, (int32_t*)l.row_ptr, (int32_t*)l.col_idx, (uint8_t*)l.flag, (int32_t*)l.col_ptr,
+                               (int32_t*)l.row_idx, (uint8_t*)l.cflag, (int32_t*)l.q_order, (int32_t*)l.k_order);
+    });
+    buf = to_device(host, (int)device);
+  } else {
+    const at::Tensor host = pinned(nqb * nkb, at::kByte);
+    memcpy(host.data_ptr(), bytes, (size_t)(nqb * nkb));
+    const at::Tensor m = to_device(host, (int)device);
+    buf = at::empty({l.at[8]}, m.options().dtype(at::kInt));
+    const at::Tensor work = at::empty({nqt + nkt + 7}, buf.options());
+    l.point_into(buf.data_ptr());
+    const hipStream_t st = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream();
+    call("ua_tilelist_build_device", [&] {
+      return ua_tilelist_build_device((const uint8_t*)m.data_ptr(), (int)nqb, (int)nkb, (int)rate, (int32_t*)l.row_ptr, (int32_t*)l.col_idx,
+                                      (uint8_t*)l.flag, (int32_t*)l.col_ptr, (int32_t*)l.row_idx, (uint8_t*)l.cflag, (int32_t*)l.q_order,
+                                      (int32_t*)l.k_order, (int32_t*)work.data_ptr(), st);
+    });
+  }
+  return Py_BuildValue("(NLLL)", THPVariable_Wrap(buf), (long long)nqt, (long long)nkt, (long long)nnz);
+}
+
+// build_lists_device(mask, rate, nnz) -> (row_ptr, col_idx, flag, col_ptr, row_idx, cflag, q_order, k_order, work) of a device mask; nnz < 0:
+// sized for every tile active
+PyObject* build_lists_device(PyObject* const* a) {
+  const at::Tensor& m = tensor(a[0], "block_mask_dev");
+  const int64_t rate = integer(a[1]), given = integer(a[2]);
+  if (m.scalar_type() != at::kByte || m.dim() != 2 || !m.is_cuda() || !m.is_contiguous())
+    fail(PyExc_ValueError, "block_mask_dev must be a contiguous 2-D uint8 CUDA tensor");
+  const int64_t nqt = m.size(0) * rate, nkt = m.size(1) * rate, cap = given >= 0 ? given : nqt * nkt;
+  const int64_t room = ((cap > 1 ? cap : 1) + 3) / 4 * 4;         // not empty, whole 32-bit words of flags
+  const at::TensorOptions i32 = m.options().dtype(at::kInt), u8 = m.options();
+  at::Tensor t[9] = {at::empty({nqt + 1}, i32), at::empty({room}, i32), at::empty({room}, u8), at::empty({nkt + 1}, i32), at::empty({room}, i32),
+                     at::empty({room}, u8), at::empty({nqt}, i32), at::empty({nkt}, i32), at::empty({nqt + nkt + 7}, i32)};
+  const On on(m);
+  call("ua_tilelist_build_device", [&] {
+    return ua_tilelist_build_device((const uint8_t*)m.data_ptr(), (int)m.size(0), (int)m.size(1), (int)rate, (int32_t*)t[0].data_ptr(),
+                                    (int32_t*)t[1].data_ptr(), (uint8_t*)t[2].data_ptr(), (int32_t*)t[3].data_ptr(), (int32_t*)t[4].data_ptr(),
+                                    (uint8_t*)t[5].data_ptr(), (int32_t*)t[6].data_ptr(), (int32_t*)t[7].data_ptr(), (int32_t*)t[8].data_ptr(), on.stream);
+  });
+  if (room != cap)
+    for (int i : {1, 2, 4, 5}) t[i] = t[i].narrow(0, 0, cap);
+  PyObject* r = PyTuple_New(9);
+  for (int i = 0; i < 9; ++i) PyTuple_SET_ITEM(r, i, THPVariable_Wrap(t[i]));
+  return r;
 }
 
 // delta(out, dout, delta) -> delta
@@ -521,7 +614,8 @@ PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
 PyMethodDef methods[] = {
     UA_METHOD(dense_forward, 8), UA_METHOD(dense_backward, 14), UA_METHOD(bsa_forward, 10), UA_METHOD(bsa_backward, 15),
     UA_METHOD(delta, 3), UA_METHOD(grad_accumulate, 4), UA_METHOD(merge, 4), UA_METHOD(grad_sum, 3),
-    UA_METHOD(merge_update, 5), UA_METHOD(permute_cols, 6), {nullptr, nullptr, 0, nullptr}};
+    UA_METHOD(merge_update, 5), UA_METHOD(permute_cols, 6), UA_METHOD(lists_from_mask, 5),
+    UA_METHOD(build_lists_device, 3), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_native", "Native host side of the attention operators.", -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

@@ -18,7 +18,7 @@ static __device__ __align__(256) int32_t scratch[UA_NOALLOC_MAX_LINES + 8];
 namespace ua {
 
 // type of tile (qt, kt): 0 empty, 1 full, 2 causal
-__host__ __device__ __forceinline__ int tile_type(const uint8_t* mask, int nkb, int rate, int qt, int kt) {
+inline int tile_type(const uint8_t* mask, int nkb, int rate, int qt, int kt) {
   const int t = mask[(int64_t)(qt / rate) * nkb + kt / rate];
   if (t != 2) return t == 1 ? 1 : 0;
   const int a = qt % rate, b = kt % rate;
@@ -38,10 +38,10 @@ __host__ __device__ __forceinline__ int tile_type(const uint8_t* mask, int nkb, 
 //  4. Then lexicographic order of the index lists read from the anchor, a list that is a prefix
 //     (from_end: a suffix) of another sorting after it; ties by line number.  Lines that walk the
 //     same K/V (or Q/dO) tiles thus sit next to each other in the launch and share them in L2.
-__host__ __device__ __forceinline__ bool very_long(const int32_t* ptr, int n, int a) {
+inline bool very_long(const int32_t* ptr, int n, int a) {
   return (int64_t)(ptr[a + 1] - ptr[a]) * n > 2 * (int64_t)ptr[n];
 }
-__host__ __device__ __forceinline__ bool row_precedes(const int32_t* ptr, const int32_t* idx, int n, int rate, int longest_sub,
+inline bool row_precedes(const int32_t* ptr, const int32_t* idx, int n, int rate, int longest_sub,
                                                       bool from_end, int a, int b) {
   const int pa = ptr[a], pb = ptr[b];
   const int la = ptr[a + 1] - pa, lb = ptr[b + 1] - pb;
@@ -89,12 +89,19 @@ static int check_mask(const uint8_t* mask, int nqb, int nkb, int rate) {
 }
 
 // ---- device variant -----------------------------------------------------------------------
+// Three launches: count, fill, order.  At the benchmark's 256 x 256 blocks every one of them is a chain of a few
+// dependent loads, so what counts is how many launches there are and how long the longest chain is; eleven
+// launches (init, check, count, two scans, fill, three for the anchors, order) took 61 us.
+//
 // One wavefront per query tile (a "row" of the list) and per key tile (a "column"); lanes
 // stride over the blocks of that row or column of the block mask.  Number of active tiles
 // that block (qb, kb) gives to query tile qt = qb*rate + a: FULL rate, CAUSAL a + 1 (key
 // sub-tiles 0..a); to key tile kt = kb*rate + b: FULL rate, CAUSAL rate - b (query sub-tiles
 // b..rate-1).
 constexpr int kWavesPerGroup = 4;
+// A line's entry in the work array: its tile count, and whether its index is the first (last) index of
+// some line of the other side (set by the fill kernel for the order kernel's choice of anchor).
+constexpr int32_t kCountBits = 0x3fffffff, kIsFirst = 1 << 30, kIsLast = (int32_t)(1u << 31);
 
 struct Line {          // one row or one column of the tile grid, as seen by its wavefront
   bool is_row;
@@ -103,17 +110,18 @@ struct Line {          // one row or one column of the tile grid, as seen by its
   int sub;             // id % rate
   int64_t base, step;  // block (i) of the line sits at mask[base + i*step]
 };
+inline int line_groups(int n) { return (n + kWavesPerGroup - 1) / kWavesPerGroup; }
+// The first workgroups take the rows, the others the columns: a workgroup's lines belong to one side.
 __device__ __forceinline__ bool line_of_wave(int nqb, int nkb, int rate, Line& ln) {
-  const int w = blockIdx.x * kWavesPerGroup + (threadIdx.x >> 6);
   const int nqt = nqb * rate, nkt = nkb * rate;
-  if (w >= nqt + nkt) return false;
-  ln.is_row = w < nqt;
-  ln.id = ln.is_row ? w : w - nqt;
+  const int groups_q = (nqt + kWavesPerGroup - 1) / kWavesPerGroup;
+  ln.is_row = (int)blockIdx.x < groups_q;
+  ln.id = (blockIdx.x - (ln.is_row ? 0 : groups_q)) * kWavesPerGroup + (threadIdx.x >> 6);
   ln.n_blocks = ln.is_row ? nkb : nqb;
   ln.sub = ln.id % rate;
   ln.base = ln.is_row ? (int64_t)(ln.id / rate) * nkb : ln.id / rate;
   ln.step = ln.is_row ? 1 : nkb;
-  return true;
+  return ln.id < (ln.is_row ? nqt : nkt);
 }
 __device__ __forceinline__ int tiles_of_block(const Line& ln, int type, int rate) {
   return type == 1 ? rate : (type == 2 ? (ln.is_row ? ln.sub + 1 : rate - ln.sub) : 0);
@@ -124,73 +132,66 @@ __device__ __forceinline__ int wave_sum(int v) {
   return v;
 }
 
+// count: tiles per line.  The builder treats mask entries that are not a Block_Type (> 2) as EMPTY; how many
+// there are is left in q_order (one entry per row, still free here) and added up by the fill kernel, so that
+// the caller can detect them after the stream has been synchronised (the host builder returns UA_ERR_MASK).
 __global__ __launch_bounds__(64 * kWavesPerGroup) void tl_count_kernel(const uint8_t* mask, int nqb, int nkb, int rate,
-                                                                        int32_t* qcnt, int32_t* kcnt) {
+                                                                        int32_t* qcnt, int32_t* kcnt, int32_t* row_invalid) {
   Line ln;
   if (!line_of_wave(nqb, nkb, rate, ln)) return;
   const int lane = threadIdx.x & 63;
-  int n = 0;
-  for (int i = lane; i < ln.n_blocks; i += 64) n += tiles_of_block(ln, mask[ln.base + i * ln.step], rate);
+  int n = 0, bad = 0;
+  for (int i = lane; i < ln.n_blocks; i += 64) {
+    const int type = mask[ln.base + i * ln.step];
+    n += tiles_of_block(ln, type, rate);
+    bad += type > 2;
+  }
   n = wave_sum(n);
   if (lane == 0) (ln.is_row ? qcnt : kcnt)[ln.id] = n;
+  if (!ln.is_row) return;
+  bad = ln.sub == 0 ? wave_sum(bad) : 0;
+  if (lane == 0) row_invalid[ln.id] = bad;
 }
 
-// init: zeroes the counters that the later kernels of the stream accumulate into.
-__global__ void tl_init_kernel(int32_t* n_invalid, int32_t* anchor_cnt) {
-  if (threadIdx.x == 0) *n_invalid = 0;
-  if (threadIdx.x < 4) anchor_cnt[threadIdx.x] = 0;
-}
-
-// check: counts the mask entries that are not a Block_Type (> 2); the builder treats them as
-// EMPTY, and the count lets the caller detect them after the stream has been synchronised (the
-// host builder returns UA_ERR_MASK for the same input).  Grid-stride over the mask, one atomic per
-// workgroup.
-__global__ __launch_bounds__(1024) void tl_check_kernel(const uint8_t* mask, int64_t n, int32_t* n_invalid) {
-  __shared__ int32_t part[16];
-  int bad = 0;
-  for (int64_t i = (int64_t)blockIdx.x * 1024 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 1024) bad += mask[i] > 2;
-  bad = wave_sum(bad);
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = bad;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int s = 0;
-    for (int i = 0; i < 16; ++i) s += part[i];
-    if (s) atomicAdd(n_invalid, s);
-  }
-}
-
-// scan: a single workgroup turns counts into exclusive prefix sums.
-__global__ __launch_bounds__(1024) void tl_scan_kernel(const int32_t* cnt, int n, int32_t* ptr) {
-  __shared__ int32_t part[1024];
-  const int tid = threadIdx.x;
-  const int per = (n + 1023) / 1024;
-  const int lo = min(n, tid * per), hi = min(n, lo + per);
-  int s = 0;
-  for (int i = lo; i < hi; ++i) s += cnt[i];
-  part[tid] = s;
-  __syncthreads();
-  for (int off = 1; off < 1024; off <<= 1) {
-    const int v = tid >= off ? part[tid - off] : 0;
-    __syncthreads();
-    part[tid] += v;
-    __syncthreads();
-  }
-  int run = tid ? part[tid - 1] : 0;
-  for (int i = lo; i < hi; ++i) { ptr[i] = run; run += cnt[i]; }
-  if (tid == 1023) ptr[n] = part[1023];
-}
-
-// fill: the wavefront walks its line 64 blocks at a time; an exclusive scan of the per-block
-// tile counts gives every lane the slot where its block's tiles go, in ascending tile order.
-__global__ __launch_bounds__(64 * kWavesPerGroup) void tl_fill_kernel(const uint8_t* mask, int nqb, int nkb, int rate,
-                                                                       const int32_t* row_ptr, int32_t* col_idx, uint8_t* flag,
-                                                                       const int32_t* col_ptr, int32_t* row_idx, uint8_t* cflag) {
+// fill: a workgroup first adds up the counts of its side (those before its lines give its place in the list,
+// all of them the list's length), then each wavefront walks its line 64 blocks at a time; an exclusive
+// scan of the per-block tile counts gives every lane the slot where its block's tiles go, in ascending order.
+__global__ __launch_bounds__(64 * kWavesPerGroup) void tl_fill_kernel(const uint8_t* mask, int nqb, int nkb, int rate, int32_t* qcnt, int32_t* kcnt,
+                                                                       int32_t* row_ptr, int32_t* col_idx, uint8_t* flag,
+                                                                       int32_t* col_ptr, int32_t* row_idx, uint8_t* cflag,
+                                                                       const int32_t* row_invalid, int32_t* n_invalid) {
+  __shared__ int32_t part[kWavesPerGroup][3];
   Line ln;
-  if (!line_of_wave(nqb, nkb, rate, ln)) return;
-  const int lane = threadIdx.x & 63;
+  const bool live = line_of_wave(nqb, nkb, rate, ln);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int n = (ln.is_row ? nqb : nkb) * rate, first_line = ln.id - wave;
+  const int32_t* cnt = ln.is_row ? qcnt : kcnt;
+  int before = 0, all = 0, bad = 0;
+  for (int i = threadIdx.x; i < n; i += 64 * kWavesPerGroup) {
+    const int c = cnt[i] & kCountBits;
+    all += c;
+    if (i < first_line) before += c;
+    if (blockIdx.x == 0) bad += row_invalid[i];
+  }
+  before = wave_sum(before); all = wave_sum(all); bad = wave_sum(bad);
+  if (lane == 0) { part[wave][0] = before; part[wave][1] = all; part[wave][2] = bad; }
+  __syncthreads();
+  before = all = bad = 0;
+#pragma unroll
+  for (int w = 0; w < kWavesPerGroup; ++w) { before += part[w][0]; all += part[w][1]; bad += part[w][2]; }
+  if (blockIdx.x == 0 && threadIdx.x == 0) *n_invalid = bad;
+  if (!live) return;
+  int e = before;
+  for (int w = 0; w < wave; ++w) e += cnt[first_line + w] & kCountBits;
+  int32_t* ptr = ln.is_row ? row_ptr : col_ptr;
+  if (lane == 0) {
+    ptr[ln.id] = e;
+    if (ln.id == n - 1) ptr[n] = all;
+  }
+  const int begin = e;
   int32_t* idx = ln.is_row ? col_idx : row_idx;
   uint8_t* flg = ln.is_row ? flag : cflag;
-  int e = (ln.is_row ? row_ptr : col_ptr)[ln.id];
+  int first_idx = -1, last_idx = -1;
   for (int i0 = 0; i0 < ln.n_blocks; i0 += 64) {
     const int i = i0 + lane;
     const int type = i < ln.n_blocks ? mask[ln.base + i * ln.step] : 0;
@@ -211,77 +212,117 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void tl_fill_kernel(const uint
       flg[at] = type == 2 && s == ln.sub;
       ++at;
     }
+    const uint64_t some = __ballot(c > 0);
+    if (some) {
+      if (first_idx < 0) first_idx = __shfl(i * rate + first, __ffsll((unsigned long long)some) - 1);
+      last_idx = __shfl(i * rate + first + c - 1, 63 - __clzll((long long)some));
+    }
     e += __shfl(incl, 63);
   }
-}
-
-// anchor: number of distinct first and of distinct last indices over the lines of each side that are
-// neither empty nor very long -> anchor_cnt[0..1] for the rows, [2..3] for the columns.  Linear in
-// the number of lines: every line marks its two anchor values in a flag array indexed by tile id
-// (bit 0 = seen as a first index, bit 1 = as a last index), then the set bits are counted.  The flag
-// arrays are the launch-order outputs themselves, which are only written afterwards: a row's anchors
-// are key tiles (flags in k_order, n_ktiles entries), a column's are query tiles (flags in q_order).
-__global__ __launch_bounds__(256) void tl_anchor_clear_kernel(int32_t* q_order, int nq, int32_t* k_order, int nk) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < nq) q_order[i] = 0;
-  else if (i < nq + nk) k_order[i - nq] = 0;
-}
-__global__ __launch_bounds__(256) void tl_anchor_mark_kernel(const int32_t* qptr, const int32_t* qidx, int nq,
-                                                             const int32_t* kptr, const int32_t* kidx, int nk,
-                                                             int32_t* q_order, int32_t* k_order) {
-  const int t = blockIdx.x * 256 + threadIdx.x;
-  if (t >= nq + nk) return;
-  const bool is_row = t < nq;
-  const int32_t* ptr = is_row ? qptr : kptr;
-  const int32_t* idx = is_row ? qidx : kidx;
-  const int n = is_row ? nq : nk, i = is_row ? t : t - nq;
-  if (ptr[i + 1] == ptr[i] || very_long(ptr, n, i)) return;
-  int32_t* flags = is_row ? k_order : q_order;
-  const int limit = is_row ? nk : nq;
-  const int first = idx[ptr[i]], last = idx[ptr[i + 1] - 1];
-  if (first >= 0 && first < limit) atomicOr(&flags[first], 1);
-  if (last >= 0 && last < limit) atomicOr(&flags[last], 2);
-}
-__global__ __launch_bounds__(256) void tl_anchor_count_kernel(const int32_t* q_order, int nq, const int32_t* k_order, int nk,
-                                                              int32_t* anchor_cnt) {
-  const int t = blockIdx.x * 256 + threadIdx.x;
-  // flags in k_order belong to the rows (anchor_cnt[0..1]), flags in q_order to the columns ([2..3])
-  const int f = t < nq ? q_order[t] : (t < nq + nk ? k_order[t - nq] : 0);
-  const bool rows_side = t >= nq;
-  // a wavefront may straddle the boundary between the two arrays: its two sides are summed separately
-  const int r0 = wave_sum(rows_side ? (f & 1) : 0), r1 = wave_sum(rows_side ? ((f >> 1) & 1) : 0);
-  const int c0 = wave_sum(rows_side ? 0 : (f & 1)), c1 = wave_sum(rows_side ? 0 : ((f >> 1) & 1));
-  if ((threadIdx.x & 63) == 0) {
-    if (r0) atomicAdd(&anchor_cnt[0], r0);
-    if (r1) atomicAdd(&anchor_cnt[1], r1);
-    if (c0) atomicAdd(&anchor_cnt[2], c0);
-    if (c1) atomicAdd(&anchor_cnt[3], c1);
+  // anchors: lines that are neither empty nor very long (see very_long) mark their first and last index
+  if (lane == 0 && e > begin && (int64_t)(e - begin) * n <= 2 * (int64_t)all) {
+    int32_t* other = ln.is_row ? kcnt : qcnt;
+    atomicOr(&other[first_idx], kIsFirst);
+    atomicOr(&other[last_idx], kIsLast);
   }
 }
 
-// order: rank of a line = number of lines that precede it; one workgroup per line, its threads
-// share the comparisons.
-__global__ __launch_bounds__(256) void tl_order_kernel(const int32_t* qptr, const int32_t* qidx, int nq, int32_t* q_order,
-                                                       const int32_t* kptr, const int32_t* kidx, int nk, int32_t* k_order, int rate,
-                                                       const int32_t* anchor_cnt) {
-  __shared__ int rank_s;
-  const int t = blockIdx.x;
-  const int32_t* ptr = t < nq ? qptr : kptr;
-  const int32_t* idx = t < nq ? qidx : kidx;
-  const int n = t < nq ? nq : nk;
-  int32_t* order = t < nq ? q_order : k_order;
-  const int i = t < nq ? t : t - nq;
-  const int longest_sub = t < nq ? rate - 1 : 0;
-  const int32_t* cnt = anchor_cnt + (t < nq ? 0 : 2);
-  const bool from_end = cnt[1] < cnt[0];
-  if (threadIdx.x == 0) rank_s = 0;
+// order: rank of a line = number of lines that precede it by row_precedes.  A workgroup ranks kOrderLines lines:
+// every thread reads the keys (very long, anchor, block-line length) of one other line and compares them with those of
+// all kOrderLines; the few pairs that only the index lists decide are queued, and a wavefront compares 256
+// indices of both lists at once.  One line per workgroup and a thread per pair, list comparison included:
+// 32 us for 2 x 1024 lines, most of it the four rows of a block walking their common list one index at a time.
+constexpr int kOrderThreads = 1024, kOrderLines = 8;
+__global__ __launch_bounds__(kOrderThreads) void tl_order_kernel(const int32_t* qptr, const int32_t* qidx, int nq, int32_t* q_order,
+                                                                 const int32_t* kptr, const int32_t* kidx, int nk, int32_t* k_order, int rate,
+                                                                 const int32_t* qcnt, const int32_t* kcnt) {
+  struct Key { int32_t very, len, anchor, block_len; };
+  __shared__ Key own[kOrderLines];
+  __shared__ int32_t rank[kOrderLines], n_first, n_last, n_queued;
+  __shared__ uint32_t queue[kOrderThreads * kOrderLines];          // pairs of one round: line | slot << 28
+  const int groups_q = (nq + kOrderLines - 1) / kOrderLines;
+  const bool rows = (int)blockIdx.x < groups_q;
+  const int32_t *ptr = rows ? qptr : kptr, *idx = rows ? qidx : kidx, *marks = rows ? kcnt : qcnt;
+  const int n = rows ? nq : nk, n_marks = rows ? nk : nq, longest_sub = rows ? rate - 1 : 0;
+  const int line0 = (blockIdx.x - (rows ? 0 : groups_q)) * kOrderLines, n_own = min(kOrderLines, n - line0);
+  const int tid = threadIdx.x, lane = tid & 63;
+  if (tid < kOrderLines) rank[tid] = 0;
+  if (tid == 0) n_first = n_last = n_queued = 0;
   __syncthreads();
-  int rank = 0;
-  for (int j = threadIdx.x; j < n; j += 256) rank += (j != i) && row_precedes(ptr, idx, n, rate, longest_sub, from_end, j, i);
-  rank = wave_sum(rank);
-  if ((threadIdx.x & 63) == 0) atomicAdd(&rank_s, rank);
+  // which end anchors the lists: the one with fewer distinct values
+  int f = 0, l = 0;
+  for (int i = tid; i < n_marks; i += kOrderThreads) { const int32_t m = marks[i]; f += (m & kIsFirst) != 0; l += (m & kIsLast) != 0; }
+  f = wave_sum(f); l = wave_sum(l);
+  if (lane == 0 && (f | l)) { atomicAdd(&n_first, f); atomicAdd(&n_last, l); }
   __syncthreads();
-  if (threadIdx.x == 0) order[rank_s] = i;
+  const bool from_end = n_last < n_first;
+  const int64_t twice_all = 2 * (int64_t)ptr[n];
+  auto key_of = [&](int i) {
+    const int p = ptr[i], len = ptr[i + 1] - p, r = i / rate * rate + longest_sub;
+    return Key{(int64_t)len * n > twice_all, len, len ? idx[from_end ? p + len - 1 : p] : 0, ptr[r + 1] - ptr[r]};
+  };
+  if (tid < n_own) own[tid] = key_of(line0 + tid);
+  __syncthreads();
+  int before[kOrderLines] = {};
+  for (int j0 = 0; j0 < n; j0 += kOrderThreads) {
+    const int j = j0 + tid;
+    if (j < n) {
+      const Key a = key_of(j);
+#pragma unroll
+      for (int s = 0; s < kOrderLines; ++s) {
+        if (s >= n_own || j == line0 + s) continue;
+        const Key b = own[s];
+        bool less;
+        if (a.very != b.very) less = a.very > b.very;
+        else if (a.len == 0 || b.len == 0) less = a.len != b.len ? a.len > b.len : j < line0 + s;
+        else if (a.anchor == b.anchor && a.block_len == b.block_len) {
+          queue[atomicAdd(&n_queued, 1)] = (uint32_t)j | (uint32_t)s << 28;
+          less = false;
+        }
+        else if (a.very ? a.block_len != b.block_len : a.anchor == b.anchor) less = a.block_len > b.block_len;
+        else less = a.anchor < b.anchor;
+        before[s] += less;
+      }
+    }
+    __syncthreads();
+    const int queued = n_queued;
+    for (int e = tid >> 6; e < queued; e += kOrderThreads / 64) {
+      const int ja = queue[e] & 0xfffffff, slot = queue[e] >> 28, ib = line0 + slot;
+      const int pa = ptr[ja], pb = ptr[ib], la = ptr[ja + 1] - pa, lb = ptr[ib + 1] - pb, m = min(la, lb);
+      const int sa = from_end ? pa + la - 1 : pa, sb = from_end ? pb + lb - 1 : pb, step = from_end ? -1 : 1;
+      bool less = la != lb ? la > lb : ja < ib;                    // one list ends inside the other
+      for (int t0 = 1; t0 < m; t0 += 256) {
+        int ca[4], cb[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int t = min(t0 + 64 * u + lane, m - 1);
+          ca[u] = idx[sa + t * step];
+          cb[u] = idx[sb + t * step];
+        }
+        bool found = false;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const uint64_t differ = __ballot(ca[u] != cb[u]);
+          if (differ && !found) {
+            found = true;
+            less = __shfl((int)(ca[u] < cb[u]), __ffsll((unsigned long long)differ) - 1) != 0;
+          }
+        }
+        if (found) break;
+      }
+      if (lane == 0 && less) atomicAdd(&rank[slot], 1);
+    }
+    __syncthreads();
+    if (tid == 0) n_queued = 0;
+    __syncthreads();
+  }
+#pragma unroll
+  for (int s = 0; s < kOrderLines; ++s) {
+    const int c = wave_sum(before[s]);
+    if (lane == 0 && c) atomicAdd(&rank[s], c);
+  }
+  __syncthreads();
+  if (tid < n_own) (rows ? q_order : k_order)[rank[tid]] = line0 + tid;
 }
 
 }  // namespace ua
@@ -352,27 +393,13 @@ static int build_device_impl(const uint8_t* block_mask, int n_qblocks, int n_kbl
   const int nqt = n_qblocks * rate, nkt = n_kblocks * rate;
   int32_t* qcnt = work;
   int32_t* kcnt = work + nqt + 1;
-  int32_t* anchor_cnt = work + nqt + nkt + 3;
-  hipLaunchKernelGGL(tl_init_kernel, dim3(1), dim3(64), 0, st, n_invalid, anchor_cnt);
-  const int64_t n_mask = (int64_t)n_qblocks * n_kblocks;
-  hipLaunchKernelGGL(tl_check_kernel, dim3((unsigned)std::min<int64_t>((n_mask + 1023) / 1024, 2048)), dim3(1024), 0, st,
-                     block_mask, n_mask, n_invalid);
-  const int blocks = (nqt + nkt + kWavesPerGroup - 1) / kWavesPerGroup;
-  hipLaunchKernelGGL(tl_count_kernel, dim3(blocks), dim3(64 * kWavesPerGroup), 0, st, block_mask, n_qblocks, n_kblocks, rate, qcnt, kcnt);
-  hipLaunchKernelGGL(tl_scan_kernel, dim3(1), dim3(1024), 0, st, (const int32_t*)qcnt, nqt, row_ptr);
-  hipLaunchKernelGGL(tl_scan_kernel, dim3(1), dim3(1024), 0, st, (const int32_t*)kcnt, nkt, col_ptr);
-  hipLaunchKernelGGL(tl_fill_kernel, dim3(blocks), dim3(64 * kWavesPerGroup), 0, st, block_mask, n_qblocks, n_kblocks, rate,
-                     (const int32_t*)row_ptr, col_idx, flag, (const int32_t*)col_ptr, row_idx, cflag);
-  const int line_blocks = (nqt + nkt + 255) / 256;
-  hipLaunchKernelGGL(tl_anchor_clear_kernel, dim3(line_blocks), dim3(256), 0, st, q_order, nqt, k_order, nkt);
-  hipLaunchKernelGGL(tl_anchor_mark_kernel, dim3(line_blocks), dim3(256), 0, st,
-                     (const int32_t*)row_ptr, (const int32_t*)col_idx, nqt,
-                     (const int32_t*)col_ptr, (const int32_t*)row_idx, nkt, q_order, k_order);
-  hipLaunchKernelGGL(tl_anchor_count_kernel, dim3(line_blocks), dim3(256), 0, st,
-                     (const int32_t*)q_order, nqt, (const int32_t*)k_order, nkt, anchor_cnt);
-  hipLaunchKernelGGL(tl_order_kernel, dim3(nqt + nkt), dim3(256), 0, st,
-                     (const int32_t*)row_ptr, (const int32_t*)col_idx, nqt, q_order,
-                     (const int32_t*)col_ptr, (const int32_t*)row_idx, nkt, k_order, rate, (const int32_t*)anchor_cnt);
+  const dim3 lines((unsigned)(line_groups(nqt) + line_groups(nkt))), group(64 * kWavesPerGroup);
+  hipLaunchKernelGGL(tl_count_kernel, lines, group, 0, st, block_mask, n_qblocks, n_kblocks, rate, qcnt, kcnt, q_order);
+  hipLaunchKernelGGL(tl_fill_kernel, lines, group, 0, st, block_mask, n_qblocks, n_kblocks, rate, qcnt, kcnt, row_ptr, col_idx, flag,
+                     col_ptr, row_idx, cflag, (const int32_t*)q_order, n_invalid);
+  hipLaunchKernelGGL(tl_order_kernel, dim3((unsigned)((nqt + kOrderLines - 1) / kOrderLines + (nkt + kOrderLines - 1) / kOrderLines)),
+                     dim3(kOrderThreads), 0, st, (const int32_t*)row_ptr, (const int32_t*)col_idx, nqt, q_order,
+                     (const int32_t*)col_ptr, (const int32_t*)row_idx, nkt, k_order, rate, (const int32_t*)qcnt, (const int32_t*)kcnt);
   return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH;
 }
 

@@ -11,7 +11,7 @@ import numpy as np
 import torch
 
 from ._lib import native
-from .tilelist import TileList, build_tile_list
+from .tilelist import TILE, TileList, prepared_mask
 
 HEAD_DIM = 128
 
@@ -28,8 +28,9 @@ def _tiles_for(tiles: Union[TileList, np.ndarray, torch.Tensor], q, block, causa
             if q.shape[1] % m.shape[0] != 0:
                 raise ValueError("cannot infer block size: Sq is not a multiple of the mask's rows")
             block = q.shape[1] // m.shape[0]
-        tiles = build_tile_list(m, block=block, causal=causal, q_block_offset=q_block_offset)
-    return tiles.lists(q.device), tiles.n_qtiles, tiles.n_ktiles, tiles.nnz
+        m = prepared_mask(m, block, causal, q_block_offset)
+        return native().lists_from_mask(m, m.shape[0], m.shape[1], block // TILE, q.device.index)
+    return tiles.packed(q.device), tiles.n_qtiles, tiles.n_ktiles, tiles.nnz
 
 
 def bsa_fwd(q, k, v, tiles, softmax_scale: Optional[float] = None, causal: bool = False,

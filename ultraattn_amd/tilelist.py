@@ -13,6 +13,7 @@ from .masks import apply_causal_rule
 TILE = 128
 
 _HOST_FIELDS = ("row_ptr", "col_idx", "flag", "col_ptr", "row_idx", "cflag", "q_order", "k_order")
+_PACKED = ("row_ptr", "col_ptr", "q_order", "k_order", "col_idx", "row_idx", "flag", "cflag")    # order in the device buffer
 
 
 @dataclass
@@ -55,19 +56,22 @@ class TileList:
             if torch.cuda.is_current_stream_capturing():
                 # the staging buffers are released once the copies are done: a graph must not replay them
                 raise RuntimeError("TileList.on(device) must be called once before the stream is captured into a graph")
-            # staged through pinned host memory and copied on the current stream without a host
-            # synchronisation; the flag arrays are padded to a multiple of 4 bytes (the kernels read
-            # them one aligned 32-bit word at a time)
-            dev, pinned = {}, []
-            for n in _HOST_FIELDS:
-                a = np.ascontiguousarray(getattr(self, n))
-                size = -(-max(a.shape[0], 1) // 4) * 4
-                host = torch.zeros(size, dtype=torch.from_numpy(a).dtype, pin_memory=True)
-                host[:a.shape[0]].copy_(torch.from_numpy(a))
-                full = host.to(device, non_blocking=True)
-                dev[n] = full[:a.shape[0]] if a.shape[0] else full[:0]
-                pinned.append(host)
-            dev["_pinned"] = pinned         # kept alive: the copies may still be in flight
+            # one buffer (the layout that the native side expects) staged through pinned host memory and copied on
+            # the current stream without a host synchronisation
+            size = {n: getattr(self, n).shape[0] for n in _PACKED}
+            words = {n: -(-c // 4) if n in ("flag", "cflag") else c for n, c in size.items()}
+            host = torch.zeros(sum(words.values()), dtype=torch.int32, pin_memory=True)
+            flat, at, dev = host.numpy(), 0, {}
+            packed = torch.empty(host.shape, dtype=torch.int32, device=device)
+            for n in _PACKED:
+                part, on_dev = flat[at:at + words[n]], packed[at:at + words[n]]
+                if n in ("flag", "cflag"):
+                    part, on_dev = part.view(np.uint8), on_dev.view(torch.uint8)
+                part[:size[n]] = getattr(self, n)
+                dev[n] = on_dev[:size[n]]
+                at += words[n]
+            packed.copy_(host, non_blocking=True)
+            dev["_packed"], dev["_pinned"] = packed, host          # the host side is kept: the copy may still be in flight
             dev["_ready"] = torch.cuda.Event()
             dev["_ready"].record()
             self._dev[key] = dev
@@ -83,12 +87,19 @@ class TileList:
         return dev
 
 
-    def lists(self, device):
-        """The arrays of ``on(device)`` as one tuple in the order of the C ABI."""
-        dev = self.on(device)
-        if "_lists" not in dev:
-            dev["_lists"] = tuple(dev[n] for n in _HOST_FIELDS)
-        return dev["_lists"]
+    def packed(self, device):
+        """All arrays of ``on(device)`` as the one int32 tensor that they are views of."""
+        return self.on(device)["_packed"]
+
+
+def prepared_mask(block_mask, block: int, causal: bool, q_block_offset: int) -> np.ndarray:
+    """The contiguous uint8 form of a 2-D block mask, the diagonal rule applied."""
+    if block % TILE != 0 or block <= 0:
+        raise ValueError(f"block ({block}) must be a positive multiple of {TILE}")
+    m = np.asarray(block_mask)
+    if m.ndim != 2:
+        raise ValueError("block_mask must be 2-D [n_qblocks, n_kblocks]")
+    return apply_causal_rule(m.astype(np.uint8), causal, q_block_offset)
 
 
 def build_tile_list(block_mask, block: int = 512, tile: int = TILE, causal: bool = False,
@@ -103,12 +114,7 @@ def build_tile_list(block_mask, block: int = 512, tile: int = TILE, causal: bool
     the row-major order of ``search_algo/dependent_graph.py:235-240``."""
     if tile != TILE:
         raise ValueError(f"kernel tile is {TILE}, got {tile}")
-    if block % tile != 0 or block <= 0:
-        raise ValueError(f"block ({block}) must be a positive multiple of {tile}")
-    m = np.asarray(block_mask)
-    if m.ndim != 2:
-        raise ValueError("block_mask must be 2-D [n_qblocks, n_kblocks]")
-    m = apply_causal_rule(m.astype(np.uint8), causal, q_block_offset)
+    m = prepared_mask(block_mask, block, causal, q_block_offset)
     rate = block // tile
     lib = _lib.load()
     nqb, nkb = m.shape
@@ -131,30 +137,10 @@ def build_tile_list_device(block_mask_dev, block: int = 512, nnz: Optional[int] 
     same contents as ``build_tile_list(...).on(device)``.  ``nnz`` (from a host-side size
     query) trims the arrays; without it they are sized to the upper bound.  ``check`` reads back
     the builder's count of invalid mask entries (this synchronises) and raises if it is not 0."""
-    import torch
-    m = block_mask_dev
-    if m.dtype != torch.uint8 or m.dim() != 2 or not m.is_cuda or not m.is_contiguous():
-        raise ValueError("block_mask_dev must be a contiguous 2-D uint8 CUDA tensor")
     rate = block // TILE
-    nqb, nkb = m.shape
-    nqt, nkt = nqb * rate, nkb * rate
-    cap = nnz if nnz is not None else nqt * nkt
-    alloc = -(-max(cap, 1) // 4) * 4   # non-NULL for an empty list; flag arrays padded to whole 32-bit words
-    dev = m.device
-    i32 = dict(dtype=torch.int32, device=dev)
-    u8 = dict(dtype=torch.uint8, device=dev)
-    out = dict(row_ptr=torch.empty(nqt + 1, **i32), col_idx=torch.empty(alloc, **i32), flag=torch.empty(alloc, **u8),
-               col_ptr=torch.empty(nkt + 1, **i32), row_idx=torch.empty(alloc, **i32), cflag=torch.empty(alloc, **u8),
-               q_order=torch.empty(nqt, **i32), k_order=torch.empty(nkt, **i32))
-    work = torch.empty(nqt + nkt + 7, **i32)
-    lib = _lib.load()
-    with torch.cuda.device(dev):
-        st = torch.cuda.current_stream().cuda_stream
-        _lib.check(lib.ua_tilelist_build_device(m.data_ptr(), nqb, nkb, rate,
-                                                *[out[n].data_ptr() for n in _HOST_FIELDS],
-                                                work.data_ptr(), st), "ua_tilelist_build_device")
-    if check and int(work[nqt + nkt + 2].item()) != 0:
-        raise ValueError(f"block mask holds {int(work[nqt + nkt + 2].item())} entries other than 0 (EMPTY), 1 (FULL), 2 (CAUSAL)")
-    for n in ("col_idx", "flag", "row_idx", "cflag"):
-        out[n] = out[n][:cap]
-    return out
+    *lists, work = _lib.native().build_lists_device(block_mask_dev, rate, -1 if nnz is None else nnz)
+    if check:
+        bad = int(work[-5].item())              # behind the counts of both sides: n_qtiles + n_ktiles + 2
+        if bad != 0:
+            raise ValueError(f"block mask holds {bad} entries other than 0 (EMPTY), 1 (FULL), 2 (CAUSAL)")
+    return dict(zip(_HOST_FIELDS, lists))
