@@ -46,27 +46,6 @@ struct BwdParams {
   BwdSide cols, rows;
 };
 
-__device__ __forceinline__ void store_acc_t(bf16* row_ptr, const f32x16 (&acc)[4], float mul, int hi) {
-  // acc[mb][4g+j] holds column (32*mb + 8*g + 4*hi + j) of this lane's output row
-#pragma unroll
-  for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      bf16x4 w;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) w[j] = (bf16)(acc[mb][4 * g + j] * mul);
-      *reinterpret_cast<bf16x4*>(row_ptr + 32 * mb + 8 * g + 4 * hi) = w;
-    }
-}
-
-__device__ __forceinline__ void store_acc_f32(float* row_ptr, const f32x16 (&acc)[4], float mul, int hi) {
-#pragma unroll
-  for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-    for (int g = 0; g < 4; ++g)
-      *reinterpret_cast<f32x4*>(row_ptr + 32 * mb + 8 * g + 4 * hi) =
-          f32x4{acc[mb][4 * g] * mul, acc[mb][4 * g + 1] * mul, acc[mb][4 * g + 2] * mul, acc[mb][4 * g + 3] * mul};
-}
 // The kernel's parameters read again from the kernel-argument segment.  What only the epilogue needs is read
 // through this, so that it does not occupy scalar registers (or get spilled to vector lanes) during the walk.
 typedef const __attribute__((address_space(4))) BwdParams* ParamsLate;
@@ -75,15 +54,15 @@ __device__ __forceinline__ ParamsLate params_late() {
   asm volatile("" : "+s"(p));
   return p;
 }
-// Output row of a result tensor: the caller's strided bf16 tensor, or part `part` of the fp32 partials.
+// 32 output rows of a wave: in the caller's strided bf16 tensor, or in part `part` of the fp32 partials.
 __device__ __forceinline__ void store_result(const __attribute__((address_space(4))) BwdSide* p, bf16* out, int64_t os_b, int64_t os_s,
-                                             int64_t os_h, int n_heads, int part, int b, int64_t row, int h, int64_t seq,
-                                             const f32x16 (&acc)[4], float mul, int hi) {
+                                             int64_t os_h, int n_heads, int part, int b, int64_t row0, int h, int64_t seq,
+                                             const f32x16 (&acc)[4], float mul, uint32_t lds) {
   if (p->out_f32) {
     float* base = reinterpret_cast<float*>(out) + part * p->o_part;
-    store_acc_f32(base + (((int64_t)b * seq + row) * n_heads + h) * kHeadDim, acc, mul, hi);
+    store_rows_f32(base + (((int64_t)b * seq + row0) * n_heads + h) * kHeadDim, (int64_t)n_heads * kHeadDim, acc, mul, lds);
   } else {
-    store_acc_t(out + b * os_b + row * os_s + h * os_h, acc, mul, hi);
+    store_rows_bf16(out + b * os_b + row0 * os_s + h * os_h, os_s, acc, mul, lds);
   }
 }
 
@@ -311,14 +290,16 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_base,
   }
 
   // K and V rows as B operands: lane holds key row 32*wave + lane%32, d = 16*ks + 8*hi .. +7
-  const int krow = kt * kTile + wave * 32 + l32;
-  const bf16* kp = p.k + b * p.ks.b + (int64_t)krow * p.ks.s + h * p.ks.h + hi * 8;
-  const bf16* vp = p.v + b * p.vs.b + (int64_t)krow * p.vs.s + h * p.vs.h + hi * 8;
+  // (through the stage that the first step fills)
+  const int krow0 = kt * kTile + wave * 32;
   bf16x8 kf[8], vf[8];
-#pragma unroll
-  for (int ks = 0; ks < 8; ++ks) {
-    kf[ks] = *reinterpret_cast<const bf16x8*>(kp + ks * 16);
-    vf[ks] = *reinterpret_cast<const bf16x8*>(vp + ks * 16);
+  {
+    u32x4 kraw[8], vraw[8];
+    load_rows(kraw, p.k + b * p.ks.b + (int64_t)krow0 * p.ks.s + h * p.ks.h, p.ks.s);
+    load_rows(vraw, p.v + b * p.vs.b + (int64_t)krow0 * p.vs.s + h * p.vs.h, p.vs.s);
+    const uint32_t turn = lds_base + 2 * kHalfPitch + wave * kWaveRowsBytes;
+    rows_to_frags(kf, kraw, turn);
+    rows_to_frags(vf, vraw, turn);
   }
   f32x16 dk[4], dv[4];
 #pragma unroll
@@ -367,9 +348,10 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_base,
   }
   const ParamsLate pl = params_late();
   const int64_t seq_k = (int64_t)pl->n_ktiles * kTile;
-  const int64_t krow_out = (int64_t)kt * kTile + wave * 32 + l32;
-  store_result(&pl->cols, pl->cols.out0, pl->cols.o0s.b, pl->cols.o0s.s, pl->cols.o0s.h, pl->n_heads, part, b, krow_out, h, seq_k, dk, pl->scale, hi);
-  store_result(&pl->cols, pl->cols.out1, pl->cols.o1s.b, pl->cols.o1s.s, pl->cols.o1s.h, pl->n_heads, part, b, krow_out, h, seq_k, dv, 1.f, hi);
+  const int64_t krow_out = (int64_t)kt * kTile + wave * 32;
+  const uint32_t turn_out = lds_base + wave * kWaveRowsBytes;        // everyone is done with the stages
+  store_result(&pl->cols, pl->cols.out0, pl->cols.o0s.b, pl->cols.o0s.s, pl->cols.o0s.h, pl->n_heads, part, b, krow_out, h, seq_k, dk, pl->scale, turn_out);
+  store_result(&pl->cols, pl->cols.out1, pl->cols.o1s.b, pl->cols.o1s.s, pl->cols.o1s.h, pl->n_heads, part, b, krow_out, h, seq_k, dv, 1.f, turn_out);
 }
 
 // ---- dQ -----------------------------------------------------------------------------------------
@@ -453,17 +435,16 @@ __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_base, i
   int kt = e0 < e1 ? ktile(e0) : 0;
   if (e0 < e1) in.copy_in((int64_t)kt * kTile, 0);
 
-  const int qrow = qt * kTile + wave * 32 + l32;
-  const bf16* qp = p.q + b * p.qs.b + (int64_t)qrow * p.qs.s + h * p.qs.h + hi * 8;
-  const bf16* dop = p.dout + b * p.ds.b + (int64_t)qrow * p.ds.s + h * p.ds.h + hi * 8;
+  const int qrow0 = qt * kTile + wave * 32, qrow = qrow0 + l32;
   bf16x8 qf[8], dof[8];
-#pragma unroll
-  for (int ks = 0; ks < 8; ++ks) {
-    qf[ks] = *reinterpret_cast<const bf16x8*>(qp + ks * 16);
-    dof[ks] = *reinterpret_cast<const bf16x8*>(dop + ks * 16);
-  }
+  u32x4 qraw[8], doraw[8];
+  load_rows(qraw, p.q + b * p.qs.b + (int64_t)qrow0 * p.qs.s + h * p.qs.h, p.qs.s);
+  load_rows(doraw, p.dout + b * p.ds.b + (int64_t)qrow0 * p.ds.s + h * p.ds.h, p.ds.s);
   const float lse_raw = p.lse[((int64_t)b * p.n_heads + h) * seq_q + qrow];
   const float neg_delta = -p.delta[((int64_t)b * p.n_heads + h) * seq_q + qrow];
+  const uint32_t turn = lds_base + 2 * kHalfPitch + wave * kWaveRowsBytes;      // in the stage that the first step fills
+  rows_to_frags(qf, qraw, turn);
+  rows_to_frags(dof, doraw, turn);
   const float lse2 = (lse_raw == -INFINITY) ? INFINITY : lse_raw * kLog2e;
   f32x16 nd;
 #pragma unroll
@@ -498,9 +479,9 @@ __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_base, i
     kt = kt_next;
   }
   const ParamsLate pl = params_late();
-  const int64_t qrow_out = (int64_t)qt * kTile + wave * 32 + l32;
+  const int64_t qrow_out = (int64_t)qt * kTile + wave * 32;
   store_result(&pl->rows, pl->rows.out0, pl->rows.o0s.b, pl->rows.o0s.s, pl->rows.o0s.h, pl->n_heads, part, b, qrow_out, h,
-               (int64_t)pl->n_qtiles * kTile, dq, pl->scale, hi);
+               (int64_t)pl->n_qtiles * kTile, dq, pl->scale, lds_base + wave * kWaveRowsBytes);      // stage 0: everyone left it before the last step
 }
 
 // ---- kernels ------------------------------------------------------------------------------------

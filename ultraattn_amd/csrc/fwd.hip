@@ -191,12 +191,15 @@ __global__ __launch_bounds__(256, 2) void fwd_kernel(const FwdParams p) {
 
   // Q fragment (B operand of S^T): lane holds query row 32*wave + lane%32,
   // d = 16*ks + 8*(lane/32) .. +7 for ks = 0..7.
+  // (through the stage that the first step fills)
   const int q_local = wave * 32 + l32;
-  const int qrow = qt * kTile + q_local;
-  const bf16* qp = p.q + b * p.qs.b + (int64_t)qrow * p.qs.s + h * p.qs.h + hi * 8;
+  const int qrow0 = qt * kTile + wave * 32, qrow = qrow0 + l32;
   bf16x8 qf[8];
-#pragma unroll
-  for (int ks = 0; ks < 8; ++ks) qf[ks] = *reinterpret_cast<const bf16x8*>(qp + ks * 16);
+  {
+    u32x4 raw[8];
+    load_rows(raw, p.q + b * p.qs.b + (int64_t)qrow0 * p.qs.s + h * p.qs.h, p.qs.s);
+    rows_to_frags(qf, raw, (uint32_t)(uintptr_t)(lds_byte*)((wave < 2 ? sKB : sVB) + (wave & 1) * kWaveRowsBytes));
+  }
 
   f32x16 oacc[4];
 #pragma unroll
@@ -230,16 +233,8 @@ __global__ __launch_bounds__(256, 2) void fwd_kernel(const FwdParams p) {
   // ---- epilogue: normalise, write O (bf16) and LSE (natural log) -------------------------
   const float l_tot = xhalf_sum(st.l_run);
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-  bf16* op = p.o + part * p.o_part + b * p.os.b + (int64_t)qrow * p.os.s + h * p.os.h;
-#pragma unroll
-  for (int mbd = 0; mbd < 4; ++mbd)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      bf16x4 w;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) w[j] = (bf16)(oacc[mbd][4 * g + j] * inv);
-      *reinterpret_cast<bf16x4*>(op + 32 * mbd + 8 * g + 4 * hi) = w;
-    }
+  store_rows_bf16(p.o + part * p.o_part + b * p.os.b + (int64_t)qrow0 * p.os.s + h * p.os.h, p.os.s, oacc, inv,
+                  (uint32_t)(uintptr_t)(lds_byte*)((wave < 2 ? sKA : sVA) + (wave & 1) * kWaveRowsBytes));     // everyone left stage A before the last step
   if (hi == 0) {
     const float lse = l_tot > 0.f ? (st.m_run + __builtin_amdgcn_logf(l_tot)) * kLn2 : -INFINITY;
     p.lse[part * p.lse_part + ((int64_t)b * p.n_heads + h) * ((int64_t)p.n_qtiles * kTile) + qrow] = lse;
