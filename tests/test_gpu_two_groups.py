@@ -1,0 +1,61 @@
+"""Workgroups of two groups that share a tile line: walks of no tile, one tile and an odd number of them, rows whose
+causal tile is not the last one, and launches on both sides of every bound at which the two groups are chosen."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import attn_oracle as ao
+from tests.gpu_util import ATOL_O, RTOL_LSE, SCALE, lse_rel_err, max_abs
+from ultraattn_amd import ops
+from ultraattn_amd.flash_attn_interface import _flash_attn_backward, _flash_attn_forward
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _inputs(sq, sk, nh, seed=5):
+    g = torch.Generator().manual_seed(seed)
+    mk = lambda n: torch.randn(1, n, nh, 128, generator=g).to(torch.bfloat16)
+    return mk(sq), mk(sk), mk(sk), mk(sq)
+
+
+def _check(got, q, k, v, do, keep, heads):
+    o, lse, dq, dk, dv = got
+    for h in heads:
+        s = slice(h, h + 1)
+        cut = [t[:, :, s] for t in (q, k, v, do)]
+        ro, rl = ao.dense_fwd(*cut[:3], SCALE, keep)
+        rq, rk, rv = ao.dense_bwd_autograd(*cut, SCALE, keep)
+        assert max_abs(o[:, :, s], ro) <= ATOL_O and lse_rel_err(lse[:, s], rl) <= RTOL_LSE
+        for a, b in ((dq, rq), (dk, rk), (dv, rv)):
+            assert max_abs(a[:, :, s], b) <= 2e-2
+
+
+@pytest.mark.parametrize("mask", [
+    [[2]], [[0, 0], [1, 0]], [[2, 1, 1]], [[1, 2, 1], [2, 0, 0], [0, 0, 2]], [[1, 1, 1, 1, 1]],
+])
+def test_short_and_odd_walks(mask):
+    mask = np.array(mask, np.uint8)
+    q, k, v, do = _inputs(mask.shape[0] * 128, mask.shape[1] * 128, 3)
+    d = [t.to(DEV) for t in (q, k, v, do)]
+    o, lse = ops.bsa_fwd(*d[:3], mask, SCALE, block=128)
+    g = ops.bsa_bwd(d[3], *d[:3], o, lse, mask, SCALE, block=128)
+    _check((o, lse, *g), q, k, v, do, ao.element_mask(mask, 128), range(3))
+
+
+@pytest.mark.parametrize("sq,sk,nh,causal", [
+    (512, 128, 2, True),                                         # rows above the first key: empty walks
+    (128, 128, 128, False), (128, 128, 129, True),               # backward: 256 and 258 workgroups
+    (128, 256, 256, True), (384, 128, 86, False),                # forward: 256 and 258
+    (2048, 2048, 16, True), (2048, 2048, 17, True),              # causal, long walks: 512 and 544 in the backward
+    (2176, 1920, 9, True),                                       # 153 rows, 135 columns, bottom-right aligned
+])
+def test_around_the_bounds(sq, sk, nh, causal):
+    q, k, v, do = _inputs(sq, sk, nh)
+    d = [t.to(DEV) for t in (q, k, v, do)]
+    r = _flash_attn_forward(*d[:3], 0.0, SCALE, causal)
+    g = _flash_attn_backward(d[3], *d[:3], r[0], r[5], None, None, None, 0.0, SCALE, causal)
+    keep = torch.ones(sq, sk, dtype=torch.bool)
+    if causal:
+        keep = torch.arange(sk)[None, :] <= torch.arange(sq)[:, None] + (sk - sq)
+    _check((r[0], r[5], *g[:3]), q, k, v, do, keep, (0, nh - 1))

@@ -43,6 +43,7 @@ struct BwdParams {
   // dense_causal [kt - diag_off, n_qtiles), the first one causal.
   int dense, dense_causal, diag_off;
   int n_col_blocks;                        // bwd_kernel: workgroups of the columns, those of the rows follow
+  int cols_shortest_first;                 // dense causal: launch order of the columns (see launch_bwd)
   BwdSide cols, rows;
 };
 
@@ -171,6 +172,26 @@ struct PairStream {
   }
 };
 
+// A wave's accumulators handed to its partner in the other group: 16-byte pieces, 1 KiB per instruction.
+constexpr int kAccBytes = 64 * 64 * 4;
+__device__ __forceinline__ void put_acc(uint32_t lds, const f32x16 (&acc)[4]) {
+  lds += 16 * fresh_lane();
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const f32x16& a = acc[i >> 2];
+    lds_put(lds + 1024 * i, f32x4{a[4 * (i & 3)], a[4 * (i & 3) + 1], a[4 * (i & 3) + 2], a[4 * (i & 3) + 3]});
+  }
+}
+__device__ __forceinline__ void add_acc(uint32_t lds, f32x16 (&acc)[4]) {
+  lds += 16 * fresh_lane();
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const f32x4 x = lds_get<f32x4>(lds + 1024 * i);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i >> 2][4 * (i & 3) + j] += x[j];
+  }
+}
+
 // One block of 32 query rows for this wave's 32 keys.  kOff = LDS offset of the block's Q rows; dO lies one
 // half tile behind.
 template <int kOff, int kStatOff>
@@ -233,9 +254,16 @@ __device__ __forceinline__ void dkdv_block(const PairAddr& ad, uint32_t stat, co
   }
 }
 
-__device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_base, int block) {
-  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
+// kGroups = 2 (here and for dQ): two groups of four wavefronts share the workgroup's line, one takes the first half of every
+// tile, the other the second, each through stages of its own; the results are added through LDS.  Where the launch
+// gives a CU one workgroup at most, one wave per SIMD would leave the matrix pipe idle between its dependent steps (2.2 us
+// per half tile of dK/dV, 0.9 of them MFMAs); the second group fills the CU without partial results in memory.
+template <int kGroups>
+__device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block, int block) {
+  const int tid = threadIdx.x & 255, lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int group = kGroups == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  const uint32_t lds_base = lds_block + group * kDkdvLdsBytes;
   int pos, bh;
   map_block(block, p.batch * p.n_heads, p.heads_per_xcd, p.n_ktiles * p.cols.n_parts, pos, bh);
   const int b = bh / p.n_heads, h = bh % p.n_heads;
@@ -243,6 +271,7 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_base,
   if (p.dense) {
     part = pos / p.n_ktiles;
     kt = pos - part * p.n_ktiles;                          // column 0 is the longest of a causal rectangle
+    if (p.cols_shortest_first) kt = p.n_ktiles - 1 - kt;
     if (p.dense_causal) diag = kt - p.diag_off;            // query tile on the diagonal (may lie outside)
     const int qbeg = p.dense_causal ? min(max(diag, 0), p.n_qtiles) : 0;
     e0 = min(max(part * p.cols.part_len, qbeg), p.n_qtiles);
@@ -254,13 +283,14 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_base,
   }
   const int64_t seq_q = (int64_t)p.n_qtiles * kTile;
   const PairStream in(p.q + b * p.qs.b + h * p.qs.h, (int)p.qs.s, p.dout + b * p.ds.b + h * p.ds.h, (int)p.ds.s, lds_base, wave, lane);
-  const int n_half = 2 * (e1 - e0);
-  // half tile i = half (i & 1) of list entry e0 + i / 2.  The list entry (query tile, causal
-  // flag) of half tile i+1 is fetched one step before it is needed, so that no step starts by
-  // waiting for a scalar load.
+  const int n_half = (kGroups == 1 ? 2 : 1) * (e1 - e0);
+  // half tile i = half (i & 1) of list entry e0 + i / 2, with two groups half `group` of entry e0 + i.  The
+  // list entry (query tile, causal flag) of half tile i+1 is fetched one step before it is needed, so that
+  // no step starts by waiting for a scalar load.
+  auto half_of = [&](int i) { return kGroups == 1 ? i & 1 : group; };
   auto entry = [&](int i) {           // query tile | causal flag << 30
     if (n_half == 0) return 0;        // an empty column owns no list entry (the arrays may be NULL)
-    const int e = min(e0 + (i >> 1), e1 - 1);
+    const int e = min(e0 + (kGroups == 1 ? i >> 1 : i), e1 - 1);
     if (p.dense) return e | ((int)(e == diag) << 30);      // the entry is the query tile itself
     return min(max(sload(p.cols.idx, e), 0), p.n_qtiles - 1) | (sload(p.cols.flag, e) << 30);
   };
@@ -273,7 +303,7 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_base,
   const float* stat_src = (tid < kHalf ? p.lse : p.delta) + ((int64_t)b * p.n_heads + h) * seq_q + (tid & (kHalf - 1));
   auto load_stat = [&](int i, int qt) {
     float x = 0.f;
-    if (tid < 2 * kHalf) x = stat_src[qt * kTile + (i & 1) * kHalf];
+    if (tid < 2 * kHalf) x = stat_src[qt * kTile + half_of(i) * kHalf];
     return x;
   };
   auto put_stat = [&](int stage, float x) {
@@ -285,7 +315,7 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_base,
   int ent = entry(0), ent_next = entry(1);
   float st0 = 0.f;
   if (n_half > 0) {
-    in.copy_in((int64_t)(ent & 0x3fffffff) * kTile, 0);
+    in.copy_in((int64_t)(ent & 0x3fffffff) * kTile + half_of(0) * kHalf, 0);
     st0 = load_stat(0, ent & 0x3fffffff);
   }
 
@@ -329,10 +359,10 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_base,
     float stat = 0.f;
     if (more) {
       stat = load_stat(i + 1, cur_next & 0x3fffffff);
-      in.copy_in((int64_t)(cur_next & 0x3fffffff) * kTile + ((i + 1) & 1) * kHalf, kStage ^ 1);
+      in.copy_in((int64_t)(cur_next & 0x3fffffff) * kTile + half_of(i + 1) * kHalf, kStage ^ 1);
     }
     // causal tile: query block nb sees none of the wave's keys when nb < wave, some when nb == wave
-    const int nb = 2 * (i & 1);
+    const int nb = 2 * half_of(i);
     if (!causal || nb >= wave)
       dkdv_block<2 * kStage * kHalfPitch, kStage * kStatBytes>(ad, stat_addr, kf, vf, dk, dv, p.scale_log2, hi, l32, causal && nb == wave);
     if (!causal || nb + 1 >= wave)
@@ -346,12 +376,22 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_base,
     step(i, std::integral_constant<int, 0>{});
     step(i + 1, std::integral_constant<int, 1>{});
   }
+  uint32_t turn_out = lds_base + wave * kWaveRowsBytes;              // everyone is done with the stages
+  if constexpr (kGroups == 2) {
+    // the second group finishes dV, the first dK
+    const uint32_t mine = lds_block + (4 * group + wave) * kAccBytes, other = lds_block + (4 * (group ^ 1) + wave) * kAccBytes;
+    if (group) put_acc(mine, dk); else put_acc(mine, dv);
+    __syncthreads();
+    if (group) add_acc(other, dv); else add_acc(other, dk);
+    turn_out = other;
+  }
   const ParamsLate pl = params_late();
   const int64_t seq_k = (int64_t)pl->n_ktiles * kTile;
   const int64_t krow_out = (int64_t)kt * kTile + wave * 32;
-  const uint32_t turn_out = lds_base + wave * kWaveRowsBytes;        // everyone is done with the stages
-  store_result(&pl->cols, pl->cols.out0, pl->cols.o0s.b, pl->cols.o0s.s, pl->cols.o0s.h, pl->n_heads, part, b, krow_out, h, seq_k, dk, pl->scale, turn_out);
-  store_result(&pl->cols, pl->cols.out1, pl->cols.o1s.b, pl->cols.o1s.s, pl->cols.o1s.h, pl->n_heads, part, b, krow_out, h, seq_k, dv, 1.f, turn_out);
+  if (kGroups == 1 || group == 0)
+    store_result(&pl->cols, pl->cols.out0, pl->cols.o0s.b, pl->cols.o0s.s, pl->cols.o0s.h, pl->n_heads, part, b, krow_out, h, seq_k, dk, pl->scale, turn_out);
+  if (kGroups == 1 || group == 1)
+    store_result(&pl->cols, pl->cols.out1, pl->cols.o1s.b, pl->cols.o1s.s, pl->cols.o1s.h, pl->n_heads, part, b, krow_out, h, seq_k, dv, 1.f, turn_out);
 }
 
 // ---- dQ -----------------------------------------------------------------------------------------
@@ -407,9 +447,12 @@ __device__ __forceinline__ void dq_block(const PairAddr& ad, const bf16x8 (&qf)[
   }
 }
 
-__device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_base, int block) {
-  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
+template <int kGroups>
+__device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_block, int block) {
+  const int tid = threadIdx.x & 255, lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int group = kGroups == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  const uint32_t lds_base = lds_block + group * kDkdvLdsBytes;
   int pos, bh;
   map_block(block, p.batch * p.n_heads, p.heads_per_xcd, p.n_qtiles * p.rows.n_parts, pos, bh);
   const int b = bh / p.n_heads, h = bh % p.n_heads;
@@ -432,8 +475,9 @@ __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_base, i
   auto ktile = [&](int e) { return p.dense ? e : min(max(sload(p.rows.idx, e), 0), p.n_ktiles - 1); };
   auto is_causal = [&](int e) { return p.dense ? (int)(e == diag) : sload(p.rows.flag, e); };
 
+  const int n_steps = (kGroups == 1 ? 2 : 1) * (e1 - e0);          // half tiles, as in dK/dV's walk
   int kt = e0 < e1 ? ktile(e0) : 0;
-  if (e0 < e1) in.copy_in((int64_t)kt * kTile, 0);
+  if (e0 < e1) in.copy_in((int64_t)kt * kTile + group * kHalf, 0);
 
   const int qrow0 = qt * kTile + wave * 32, qrow = qrow0 + l32;
   bf16x8 qf[8], dof[8];
@@ -459,46 +503,62 @@ __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_base, i
 #pragma unroll
   for (int ks = 0; ks < 8; ++ks) asm volatile("" : "+v"(qf[ks]), "+v"(dof[ks]));
 
-  for (int e = e0; e < e1; ++e) {
-    const int causal = is_causal(e);
-    const int kt_next = e + 1 < e1 ? ktile(e + 1) : kt;
+  int causal = 0;
+  auto step = [&](int i, auto stage_tag) {
+    constexpr int kStage = decltype(stage_tag)::value;
+    if (i >= n_steps) return;   // workgroup-uniform
+    const int e = e0 + (kGroups == 1 ? i >> 1 : i), half = kGroups == 1 ? kStage : group;
+    if (kGroups == 2 || kStage == 0) causal = is_causal(e);
+    const bool more = i + 1 < n_steps;
+    const int kt_next = kGroups == 1 && kStage == 0 ? kt : (more ? ktile(e + 1) : kt);
     wait_vmem_all();
-    __syncthreads();            // stage 0 (keys 0..63) landed; everyone is done with stage 1
-    in.copy_in((int64_t)kt * kTile + kHalf, 1);
+    __syncthreads();            // this stage has landed; everyone is done with the other one
+    if (more) in.copy_in((int64_t)kt_next * kTile + (kGroups == 1 ? kStage ^ 1 : group) * kHalf, kStage ^ 1);
     // causal tile: key block nb is hidden from the wave's queries when nb > wave, in part when nb == wave
-    dq_block<0>(ad, qf, dof, nd, dq, p.scale_log2, lse2, hi, l32, causal && wave == 0);
-    if (!causal || wave >= 1)
-      dq_block<kBlockPitch>(ad, qf, dof, nd, dq, p.scale_log2, lse2, hi, l32, causal && wave == 1);
-    wait_vmem_all();
-    __syncthreads();            // stage 1 landed; everyone is done with stage 0
-    if (e + 1 < e1) in.copy_in((int64_t)kt_next * kTile, 0);
-    if (!causal || wave >= 2)
-      dq_block<2 * kHalfPitch>(ad, qf, dof, nd, dq, p.scale_log2, lse2, hi, l32, causal && wave == 2);
-    if (!causal || wave == 3)
-      dq_block<2 * kHalfPitch + kBlockPitch>(ad, qf, dof, nd, dq, p.scale_log2, lse2, hi, l32, causal);
+    const int nb = 2 * half;
+    if (!causal || wave >= nb)
+      dq_block<2 * kStage * kHalfPitch>(ad, qf, dof, nd, dq, p.scale_log2, lse2, hi, l32, causal && wave == nb);
+    if (!causal || wave >= nb + 1)
+      dq_block<2 * kStage * kHalfPitch + kBlockPitch>(ad, qf, dof, nd, dq, p.scale_log2, lse2, hi, l32, causal && wave == nb + 1);
     kt = kt_next;
+  };
+  for (int i = 0; i < n_steps; i += 2) {
+    step(i, std::integral_constant<int, 0>{});
+    step(i + 1, std::integral_constant<int, 1>{});
+  }
+  uint32_t turn_out = lds_base + wave * kWaveRowsBytes;              // stage 0: everyone left it before the last step
+  if constexpr (kGroups == 2) {
+    __syncthreads();
+    turn_out = lds_block + wave * kAccBytes;
+    if (group) put_acc(turn_out, dq);
+    __syncthreads();
+    if (group) return;
+    add_acc(turn_out, dq);
   }
   const ParamsLate pl = params_late();
   const int64_t qrow_out = (int64_t)qt * kTile + wave * 32;
   store_result(&pl->rows, pl->rows.out0, pl->rows.o0s.b, pl->rows.o0s.s, pl->rows.o0s.h, pl->n_heads, part, b, qrow_out, h,
-               (int64_t)pl->n_qtiles * kTile, dq, pl->scale, lds_base + wave * kWaveRowsBytes);      // stage 0: everyone left it before the last step
+               (int64_t)pl->n_qtiles * kTile, dq, pl->scale, turn_out);
 }
 
 // ---- kernels ------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256, 2) void dkdv_kernel(const BwdParams p) {
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[kDkdvLdsBytes];
-  dkdv_walk(p, (uint32_t)(uintptr_t)(UA_LDS unsigned char*)smem, blockIdx.x);
+template <int kGroups>
+__global__ __launch_bounds__(256 * kGroups, 2) void dkdv_kernel(const BwdParams p) {
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[kGroups * kDkdvLdsBytes];
+  dkdv_walk<kGroups>(p, (uint32_t)(uintptr_t)(UA_LDS unsigned char*)smem, blockIdx.x);
 }
-__global__ __launch_bounds__(256, 2) void dq_kernel(const BwdParams p) {
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[4 * kHalfPitch];
-  dq_walk(p, (uint32_t)(uintptr_t)(UA_LDS unsigned char*)smem, blockIdx.x);
+template <int kGroups>
+__global__ __launch_bounds__(256 * kGroups, 2) void dq_kernel(const BwdParams p) {
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[kGroups * kDkdvLdsBytes];
+  dq_walk<kGroups>(p, (uint32_t)(uintptr_t)(UA_LDS unsigned char*)smem, blockIdx.x);
 }
 // Both sides in one launch.
-__global__ __launch_bounds__(256, 2) void bwd_kernel(const BwdParams p) {
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[kDkdvLdsBytes];
+template <int kGroups>
+__global__ __launch_bounds__(256 * kGroups, 2) void bwd_kernel(const BwdParams p) {
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[kGroups * kDkdvLdsBytes];
   const uint32_t lds_base = (uint32_t)(uintptr_t)(UA_LDS unsigned char*)smem;
-  if ((int)blockIdx.x < p.n_col_blocks) dkdv_walk(p, lds_base, blockIdx.x);
-  else                                  dq_walk(p, lds_base, blockIdx.x - p.n_col_blocks);
+  if ((int)blockIdx.x < p.n_col_blocks) dkdv_walk<kGroups>(p, lds_base, blockIdx.x);
+  else                                  dq_walk<kGroups>(p, lds_base, blockIdx.x - p.n_col_blocks);
 }
 
 static int fill_common(BwdParams& p, const void* q, const void* k, const void* v, const void* dout,
@@ -523,7 +583,7 @@ static int fill_common(BwdParams& p, const void* q, const void* k, const void* v
   p.scale = softmax_scale; p.scale_log2 = softmax_scale * kLog2e;
   const int nbh = batch * n_heads;
   p.heads_per_xcd = (nbh % 8 == 0) ? nbh / 8 : 0;
-  p.dense = 0; p.dense_causal = 0; p.diag_off = 0; p.n_col_blocks = 0;
+  p.dense = 0; p.dense_causal = 0; p.diag_off = 0; p.n_col_blocks = 0; p.cols_shortest_first = 0;
   p.cols = BwdSide{}; p.rows = BwdSide{};
   p.cols.n_parts = p.rows.n_parts = 1;
   return UA_OK;
@@ -546,24 +606,46 @@ static int fill_side(BwdSide& s, int nnz, const int32_t* ptr, const int32_t* idx
 static int launched() { return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH; }
 static unsigned col_blocks(const BwdParams& p) { return (unsigned)(p.batch * p.n_heads * p.n_ktiles * p.cols.n_parts); }
 static unsigned row_blocks(const BwdParams& p) { return (unsigned)(p.batch * p.n_heads * p.n_qtiles * p.rows.n_parts); }
+// Two groups per workgroup where both sides together give a CU one workgroup at most and the walks are worth the handing
+// over at their end, from three tiles on; a launch of one side alone decides alike, so that its results are the
+// same bit for bit.  An uncut causal rectangle whose walks average 8 tiles is
+// better off with them up to two workgroups per CU: run in turn they balance its lines (8 heads of 4096: 135 us
+// resident at once, 118 in turn; shorter walks lose more to the second start: 32 heads of 1024 41, 50).
+static bool bwd_pairs(int64_t groups, int64_t both_walks, int n_parts, bool dense_causal, int n_qtiles, int n_ktiles) {
+  return both_walks >= 6 && (groups <= kCus || (groups <= 2 * kCus && dense_causal && n_parts == 2 && n_qtiles >= 16 && n_ktiles >= 16));
+}
+static unsigned both_blocks(const BwdParams& p) { return col_blocks(p) + row_blocks(p); }
+static bool pairs(const BwdParams& p) {
+  const int64_t walks = p.dense ? p.cols.part_len + p.rows.part_len : p.nnz / p.n_qtiles + p.nnz / p.n_ktiles;
+  return bwd_pairs(both_blocks(p), walks, p.cols.n_parts + p.rows.n_parts, p.dense_causal, p.n_qtiles, p.n_ktiles);
+}
 static int launch_bwd(BwdParams& p, hipStream_t st) {
   p.n_col_blocks = (int)col_blocks(p);
-  hipLaunchKernelGGL(bwd_kernel, dim3(col_blocks(p) + row_blocks(p)), dim3(256), 0, st, p);
+  if (pairs(p)) {
+    hipLaunchKernelGGL(bwd_kernel<2>, dim3(both_blocks(p)), dim3(512), 0, st, p);
+  } else {
+    // Up to two workgroups per CU the whole launch is resident at once, and the second 256 join the first in launch
+    // order.  Rows come longest first; of a causal rectangle the columns then come shortest first, so that the long
+    // ones of one side share a CU with the short ones of the other (32 heads of 1024: 43.6 -> 41.5 us).
+    p.cols_shortest_first = p.dense_causal && both_blocks(p) <= 2 * kCus;
+    hipLaunchKernelGGL(bwd_kernel<1>, dim3(both_blocks(p)), dim3(256), 0, st, p);
+  }
   return launched();
 }
 
 // How many parts the two sides of a dense backward are cut into, at most what the workspace holds.  A cut gives a
 // small rectangle enough workgroups for the device and costs the partials' way through memory and a
-// second launch; which wins is decided by an estimate of the launch's time in microseconds, fitted to 20 shapes of 1
-// to 32 heads and 512 to 8192 tokens (each within 8 % of its best cut):
-//  - 8.4 to start, load the resident rows, store the results and end;
-//  - a workgroup alone on its CU walks a tile in 3.4 (columns) or 2.4 (rows), two that share it in 6.6 and 4.3 each;
-//  - the sum takes 2.3, and the partials 1 per 3.7 MB.
-// 512 x 512, 32 heads: 40 us cut in two, 24 uncut; 1024 x 4096, one head: 84 uncut, 26 cut in 4 and 8.
+// second launch; which wins is decided by an estimate of the launch's time in microseconds, fitted to 47 shapes of 1
+// to 32 heads and 128 to 8192 tokens (the cut it takes is within 4 % of the best one on each):
+//  - 6.7 to start, load the resident rows, store the results and end, 8.4 with two groups per workgroup;
+//  - a tile takes 2.6 (columns) or 1.7 (rows) with two groups, else 3.2 and 2.2, and 4.4 and 4.9 where two workgroups
+//    share the CU;
+//  - the sum takes 2.7, and the partials 1 per 3.7 MB; a cut has to win by 6 %.
+// 512 x 512, 32 heads: 33 us cut in two, 22 uncut; 1024 x 4096, one head: 67 uncut, 25 cut in 4 and 8.
 struct BwdCut { int cols, rows; };
 static BwdCut bwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int max_cols, int max_rows) {
   if (max_cols <= 1 && max_rows <= 1) return {1, 1};
-  static constexpr int kParts[] = {1, 2, 3, 4, 6, 8, 12, 16};
+  static constexpr int kParts[] = {1, 2, 3, 4, 5, 6, 8, 12, 16};
   const float density = causal ? 0.5f : 1.f, wk = (float)nbh * n_ktiles, wq = (float)nbh * n_qtiles;
   BwdCut best = {1, 1};
   float best_us = INFINITY;
@@ -572,12 +654,15 @@ static BwdCut bwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int 
     for (int pr : kParts) {
       if (pr > max_rows) break;
       const float groups = (wk * pc + wq * pr) * density;
-      const float shared = fminf(fmaxf((groups - 256.f) / 256.f, 0.f), 1.f);       // share of the workgroups with a neighbour
-      const float tc = 3.4f + 3.2f * shared, tr = 2.4f + 1.9f * shared;
+      float us = 8.4f, tc = 2.6f, tr = 1.7f;
+      if (!bwd_pairs(nbh * ((int64_t)n_ktiles * pc + (int64_t)n_qtiles * pr), (n_qtiles + pc - 1) / pc + (n_ktiles + pr - 1) / pr, pc + pr, causal, n_qtiles, n_ktiles)) {
+        const float shared = fminf(fmaxf((groups - kCus) / kCus, 0.f), 1.f);       // share of the workgroups with a neighbour
+        us = 6.7f; tc = 3.2f + 1.2f * shared; tr = 2.2f + 2.7f * shared;
+      }
       const float longest = fmaxf((float)((n_qtiles + pc - 1) / pc) * tc, (float)((n_ktiles + pr - 1) / pr) * tr);
-      const float all = density * wk * n_qtiles * (6.6f + 4.3f) / 512.f;
-      float us = 8.4f + fmaxf(longest, all);
-      if (pc > 1 || pr > 1) us += 2.3f;
+      const float all = density * wk * n_qtiles * (4.4f + 4.9f) / (2 * kCus);
+      us += fmaxf(longest, all);
+      if (pc > 1 || pr > 1) us = (us + 2.7f) * 1.06f;
       if (pc > 1) us += 2.f * pc * wk * (kTile * kHeadDim * 4) / 3.7e6f;
       if (pr > 1) us += pr * wq * (kTile * kHeadDim * 4) / 3.7e6f;
       if (us < best_us) { best_us = us; best = {pc, pr}; }
@@ -603,7 +688,8 @@ extern "C" int ua_bsa_bwd_dkdv(const void* q, const void* k, const void* v, cons
   if (!dv_strides) return UA_ERR_NULL;
   if (int rc = fill_side(p.cols, nnz, col_ptr, row_idx, cflag, k_order, dk, dk_strides, dv, dv_strides, false)) return rc;
   if (int rc = check_device()) return rc;
-  hipLaunchKernelGGL(dkdv_kernel, dim3(col_blocks(p)), dim3(256), 0, (hipStream_t)stream, p);
+  if (pairs(p)) hipLaunchKernelGGL(dkdv_kernel<2>, dim3(col_blocks(p)), dim3(512), 0, (hipStream_t)stream, p);
+  else          hipLaunchKernelGGL(dkdv_kernel<1>, dim3(col_blocks(p)), dim3(256), 0, (hipStream_t)stream, p);
   return launched();
 }
 
@@ -621,7 +707,8 @@ extern "C" int ua_bsa_bwd_dq(const void* q, const void* k, const void* v, const 
                            v_strides, do_strides, softmax_scale)) return rc;
   if (int rc = fill_side(p.rows, nnz, row_ptr, col_idx, flag, q_order, dq, dq_strides, nullptr, nullptr, false)) return rc;
   if (int rc = check_device()) return rc;
-  hipLaunchKernelGGL(dq_kernel, dim3(row_blocks(p)), dim3(256), 0, (hipStream_t)stream, p);
+  if (pairs(p)) hipLaunchKernelGGL(dq_kernel<2>, dim3(row_blocks(p)), dim3(512), 0, (hipStream_t)stream, p);
+  else          hipLaunchKernelGGL(dq_kernel<1>, dim3(row_blocks(p)), dim3(256), 0, (hipStream_t)stream, p);
   return launched();
 }
 

@@ -11,6 +11,7 @@
 // lane (mirrored in lane ^ 32): the row max needs a single cross-half exchange, the rescale of
 // O^T is lane local, and S^T's accumulator registers are, after exp2 and bf16 packing, exactly
 // the B operand of the second product.
+#include <type_traits>
 #include "ua_common.h"
 
 namespace ua {
@@ -137,16 +138,24 @@ __device__ __forceinline__ void half_tile(const unsigned char* sK, const unsigne
   }
 }
 
-__global__ __launch_bounds__(256, 2) void fwd_kernel(const FwdParams p) {
-  // two pipeline stages, distinct arrays so that reads of one stage need not wait for the
+// kGroups = 2: two groups of four wavefronts share the query tile, one takes the first 64 keys of every tile, the
+// other the second; their results are combined through LDS.  A launch that gives a CU one workgroup at most runs it at
+// one wave per SIMD, where a half tile takes 1.2 us of which the matrix pipe is busy 0.4; with the second group the CU is
+// as full as with two workgroups, without partial results in memory.
+template <int kGroups>
+__global__ __launch_bounds__(256 * kGroups, 2) void fwd_kernel(const FwdParams p) {
+  // two pipeline stages per group, distinct arrays so that reads of one stage need not wait for the
   // copies in flight into the other
-  __shared__ __attribute__((aligned(1024))) unsigned char sKA[kHalfBytes];
-  __shared__ __attribute__((aligned(1024))) unsigned char sVA[kHalfBytes];
-  __shared__ __attribute__((aligned(1024))) unsigned char sKB[kHalfBytes];
-  __shared__ __attribute__((aligned(1024))) unsigned char sVB[kHalfBytes];
+  __shared__ __attribute__((aligned(1024))) unsigned char sKA[kGroups * kHalfBytes];
+  __shared__ __attribute__((aligned(1024))) unsigned char sVA[kGroups * kHalfBytes];
+  __shared__ __attribute__((aligned(1024))) unsigned char sKB[kGroups * kHalfBytes];
+  __shared__ __attribute__((aligned(1024))) unsigned char sVB[kGroups * kHalfBytes];
 
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave_in_block = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = kGroups == 1 ? wave_in_block : wave_in_block & 3, group = kGroups == 1 ? 0 : wave_in_block >> 2;
+  unsigned char *const kA = sKA + group * kHalfBytes, *const vA = sVA + group * kHalfBytes;
+  unsigned char *const kB = sKB + group * kHalfBytes, *const vB = sVB + group * kHalfBytes;
   const int l32 = lane & 31, hi = lane >> 5;
   int pos, bh;
   map_block(blockIdx.x, p.batch * p.n_heads, p.heads_per_xcd, p.n_qtiles * p.n_parts, pos, bh);
@@ -182,11 +191,15 @@ __global__ __launch_bounds__(256, 2) void fwd_kernel(const FwdParams p) {
   auto k_rsrc = [&](int kt) { return make_rsrc(kbase + (int64_t)kt * kTile * k_stride, k_extent); };
   auto v_rsrc = [&](int kt) { return make_rsrc(vbase + (int64_t)kt * kTile * v_stride, v_extent); };
 
-  // first half tile of the first entry goes in flight before anything else
-  int kt = e0 < e1 ? ktile(e0) : 0;
-  if (e0 < e1) {
-    dma_half_tile_buf<4>(sKA, k_rsrc(kt), koff, 0, wave);
-    dma_half_tile_buf<4>(sVA, v_rsrc(kt), voff, 0, wave);
+  // step i = one half tile of this group: half i % 2 of entry e0 + i / 2, with two groups half `group` of entry e0 + i
+  const int n_steps = (kGroups == 1 ? 2 : 1) * (e1 - e0);
+  auto entry_of = [&](int i) { return e0 + (kGroups == 1 ? i >> 1 : i); };
+  // the first half tile goes in flight before anything else
+  int kt = 0;
+  if (n_steps > 0) {
+    kt = ktile(e0);
+    dma_half_tile_buf<4>(kA, k_rsrc(kt), koff, group * k_half, wave);
+    dma_half_tile_buf<4>(vA, v_rsrc(kt), voff, group * v_half, wave);
   }
 
   // Q fragment (B operand of S^T): lane holds query row 32*wave + lane%32,
@@ -198,7 +211,7 @@ __global__ __launch_bounds__(256, 2) void fwd_kernel(const FwdParams p) {
   {
     u32x4 raw[8];
     load_rows(raw, p.q + b * p.qs.b + (int64_t)qrow0 * p.qs.s + h * p.qs.h, p.qs.s);
-    rows_to_frags(qf, raw, (uint32_t)(uintptr_t)(lds_byte*)((wave < 2 ? sKB : sVB) + (wave & 1) * kWaveRowsBytes));
+    rows_to_frags(qf, raw, (uint32_t)(uintptr_t)(lds_byte*)((wave < 2 ? kB : vB) + (wave & 1) * kWaveRowsBytes));
   }
 
   f32x16 oacc[4];
@@ -207,34 +220,67 @@ __global__ __launch_bounds__(256, 2) void fwd_kernel(const FwdParams p) {
   SoftmaxState st;
   const TrLane tr(lane);
 
-  for (int e = e0; e < e1; ++e) {
-    const int causal = is_causal(e);
-    const int kt_next = e + 1 < e1 ? ktile(e + 1) : kt;
-    // stage A (keys 0..63 of this tile) has landed; everyone is done with stage B
+  bool started = false;
+  int causal = 0;
+  auto step = [&](int i, auto stage_tag) {
+    constexpr int kStage = decltype(stage_tag)::value;
+    if (i >= n_steps) return;              // workgroup-uniform
+    const int e = entry_of(i), half = kGroups == 1 ? kStage : group;
+    if (kGroups == 2 || kStage == 0) causal = is_causal(e);
+    const bool more = i + 1 < n_steps;
+    const int kt_next = kGroups == 1 && kStage == 0 ? kt : (more ? ktile(e + 1) : kt);
+    // this stage has landed; everyone is done with the other one
     wait_vmem_all();
     __syncthreads();
-    dma_half_tile_buf<4>(sKB, k_rsrc(kt), koff, k_half, wave);
-    dma_half_tile_buf<4>(sVB, v_rsrc(kt), voff, v_half, wave);
-    // causal tile: queries 64..127 (waves 2, 3) see all of keys 0..63
-    half_tile(sKA, sVA, qf, oacc, st, tr, p.scale_log2, l32, hi, q_local, 0, causal && wave < 2, e == e0);
-    // stage B has landed; everyone is done with stage A
-    wait_vmem_all();
-    __syncthreads();
-    if (e + 1 < e1) {
-      dma_half_tile_buf<4>(sKA, k_rsrc(kt_next), koff, 0, wave);
-      dma_half_tile_buf<4>(sVA, v_rsrc(kt_next), voff, 0, wave);
+    if (more) {
+      const int half_next = kGroups == 1 ? kStage ^ 1 : group;
+      dma_half_tile_buf<4>(kStage ? kA : kB, k_rsrc(kt_next), koff, half_next * k_half, wave);
+      dma_half_tile_buf<4>(kStage ? vA : vB, v_rsrc(kt_next), voff, half_next * v_half, wave);
     }
-    // causal tile: queries 0..63 (waves 0, 1) see none of keys 64..127
-    if (!causal || wave >= 2)
-      half_tile(sKB, sVB, qf, oacc, st, tr, p.scale_log2, l32, hi, q_local, kHalf, causal, false);
+    // causal tile: queries 64..127 (waves 2, 3) see all of keys 0..63, queries 0..63 (waves 0, 1) none of keys 64..127
+    if (half == 0 || !causal || wave >= 2) {
+      half_tile(kStage ? kB : kA, kStage ? vB : vA, qf, oacc, st, tr, p.scale_log2, l32, hi, q_local, kHalf * half,
+                causal && (half == 0 ? wave < 2 : true), kGroups == 1 ? kStage == 0 && i == 0 : !started);
+      started = true;
+    }
     kt = kt_next;
+  };
+  for (int i = 0; i < n_steps; i += 2) {
+    step(i, std::integral_constant<int, 0>{});
+    step(i + 1, std::integral_constant<int, 1>{});
   }
 
   // ---- epilogue: normalise, write O (bf16) and LSE (natural log) -------------------------
-  const float l_tot = xhalf_sum(st.l_run);
+  float l_tot = xhalf_sum(st.l_run);
+  unsigned char* turn = (wave < 2 ? kA : vA) + (wave & 1) * kWaveRowsBytes;       // everyone left stage A before the last step
+  if constexpr (kGroups == 2) {
+    // the second group hands over its rows' max, sum and O: a 16-byte piece of a lane after the other, 1 KiB per instruction
+    __syncthreads();
+    turn = (wave < 2 ? sKA : sVA) + (wave & 1) * 2 * kWaveRowsBytes;
+    const uint32_t at = (uint32_t)(uintptr_t)(lds_byte*)turn + 16 * lane, at_stat = (uint32_t)(uintptr_t)(lds_byte*)sKB + wave * 512 + 4 * lane;
+    if (group == 1) {
+      lds_put(at_stat, st.m_run);
+      lds_put(at_stat + 256, l_tot);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) lds_put(at + 1024 * i, f32x4{oacc[i >> 2][4 * (i & 3)], oacc[i >> 2][4 * (i & 3) + 1], oacc[i >> 2][4 * (i & 3) + 2], oacc[i >> 2][4 * (i & 3) + 3]});
+    }
+    __syncthreads();
+    if (group == 1) return;
+    const float m1 = lds_get<float>(at_stat), l1 = lds_get<float>(at_stat + 256);
+    const float m = fmaxf(st.m_run, m1), ms = m == -INFINITY ? 0.f : m;
+    const float w0 = fast_exp2(st.m_run - ms), w1 = fast_exp2(m1 - ms);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const f32x4 x = lds_get<f32x4>(at + 1024 * i);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) oacc[i >> 2][4 * (i & 3) + j] = oacc[i >> 2][4 * (i & 3) + j] * w0 + x[j] * w1;
+    }
+    st.m_run = m;
+    l_tot = l_tot * w0 + l1 * w1;
+  }
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
   store_rows_bf16(p.o + part * p.o_part + b * p.os.b + (int64_t)qrow0 * p.os.s + h * p.os.h, p.os.s, oacc, inv,
-                  (uint32_t)(uintptr_t)(lds_byte*)((wave < 2 ? sKA : sVA) + (wave & 1) * kWaveRowsBytes));     // everyone left stage A before the last step
+                  (uint32_t)(uintptr_t)(lds_byte*)turn);
   if (hi == 0) {
     const float lse = l_tot > 0.f ? (st.m_run + __builtin_amdgcn_logf(l_tot)) * kLn2 : -INFINITY;
     p.lse[part * p.lse_part + ((int64_t)b * p.n_heads + h) * ((int64_t)p.n_qtiles * kTile) + qrow] = lse;
@@ -271,9 +317,47 @@ static int fwd_common(FwdParams& p, const void* q, const void* k, const void* v,
   return check_device();
 }
 
+// Two groups per workgroup where a CU gets one workgroup at most and the walk is worth the handing over at its end, from
+// three tiles on (two tiles: 8.1 us with one group, 8.5 with two).  An uncut causal rectangle is better off with
+// them up to two per CU: run one after the other, longest first, they balance its rows of different lengths, which
+// two workgroups resident from the start do not (16 heads of 4096: 91 us resident, 76 in turn; 8 of 8192: 156, 132); the
+// rows of a list are too much alike for that (strided 8k, 8 heads: 84 and 95).
+static bool fwd_pairs(int64_t groups, int64_t walk, int n_parts, bool dense_causal) {
+  return walk >= 3 && groups <= (dense_causal && n_parts == 1 ? 2 * kCus : kCus);
+}
 static int fwd_launch(const FwdParams& p, hipStream_t st) {
-  hipLaunchKernelGGL(fwd_kernel, dim3((unsigned)(p.batch * p.n_heads * p.n_qtiles * p.n_parts)), dim3(256), 0, st, p);
+  const unsigned groups = (unsigned)(p.batch * p.n_heads * p.n_qtiles * p.n_parts);
+  const int64_t walk = p.dense ? p.part_len : p.nnz / p.n_qtiles;
+  if (fwd_pairs(groups, walk, p.n_parts, p.dense_causal)) hipLaunchKernelGGL(fwd_kernel<2>, dim3(groups), dim3(512), 0, st, p);
+  else                                                    hipLaunchKernelGGL(fwd_kernel<1>, dim3(groups), dim3(256), 0, st, p);
   return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH;
+}
+
+// How many parts the walks of a dense forward are cut into, at most max_parts (what the workspace holds).  A cut
+// gives a small rectangle enough workgroups and costs the partials' way through memory and a merge; an estimate of the
+// launches' time in microseconds decides, fitted to 47 shapes of 1 to 32 heads and 128 to 8192 tokens (the cut it
+// takes is within 4 % of the best one on each):
+//  - 4.1 to start, load Q, store and end, 5.7 with two groups per workgroup;
+//  - a tile takes 1.5 with two groups, else 2.2, and 3.4 where two workgroups share the CU;
+//  - the merge takes 1.7 + 0.04 a part, and the partials 1 per 1.3 MB.
+// 512 x 512, 32 heads: 17 us cut in two, 12 uncut; 1024 x 4096, one head: 52 uncut, 14 cut in 16.
+static int fwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int max_parts) {
+  const float density = causal ? 0.5f : 1.f, lines = (float)nbh * n_qtiles;
+  int best = 1;
+  float best_us = INFINITY;
+  for (int parts = 1; parts <= max_parts; ++parts) {
+    const float groups = lines * parts, longest = (float)((n_ktiles + parts - 1) / parts);
+    float us = 4.1f;
+    if (fwd_pairs(nbh * n_qtiles * parts, (n_ktiles + parts - 1) / parts, parts, causal)) {
+      us += 1.6f + longest * 1.5f;
+    } else {
+      const float shared = fminf(fmaxf((groups * density - kCus) / kCus, 0.f), 1.f);      // share of the workgroups with a neighbour
+      us += fmaxf(longest * (2.2f + 1.2f * shared), density * lines * n_ktiles * 3.4f / (2 * kCus));
+    }
+    if (parts > 1) us += 1.7f + 0.04f * parts + groups * (kTile * kHeadDim * 2) / 1.3e6f;
+    if (us < best_us) { best_us = us; best = parts; }
+  }
+  return best;
 }
 
 static bool contiguous_bshd(const int64_t* st, int seqlen, int n_heads) {
@@ -322,10 +406,11 @@ extern "C" int ua_dense_fwd(const void* q, const void* k, const void* v, void* o
   hipStream_t st = (hipStream_t)stream;
   const DenseSplit d = dense_split(batch, n_heads, n_qtiles, n_ktiles);
   // the split path needs the caller's workspace and a contiguous output for the merge
-  const bool split = d.fwd_parts > 1 && workspace && aligned16(workspace) && workspace_bytes >= d.fwd_total &&
-                     contiguous_bshd(o_strides, seqlen_q, n_heads);
-  if (!split) return fwd_launch(p, st);
-  const int len = (n_ktiles + d.fwd_parts - 1) / d.fwd_parts;
+  const bool can_cut = d.fwd_parts > 1 && workspace && aligned16(workspace) && workspace_bytes >= d.fwd_total &&
+                       contiguous_bshd(o_strides, seqlen_q, n_heads);
+  const int cut = can_cut ? fwd_cut((int64_t)batch * n_heads, n_qtiles, n_ktiles, p.dense_causal, d.fwd_parts) : 1;
+  if (cut == 1) return fwd_launch(p, st);
+  const int len = (n_ktiles + cut - 1) / cut;
   const int parts = (n_ktiles + len - 1) / len;
   unsigned char* ws = static_cast<unsigned char*>(workspace);
   p.o = reinterpret_cast<bf16*>(ws);

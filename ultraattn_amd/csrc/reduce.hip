@@ -125,16 +125,16 @@ __global__ __launch_bounds__(kRedThreads) void partial_sums_kernel(const Partial
   if (row >= (int64_t)p.batch * s.seqlen * p.n_heads) return;
   const float* src = s.base + c * 8;
   f32x4 x0{0}, x1{0};
-  for (int i0 = 0; i0 < s.n_parts; i0 += 4) {
-    f32x4 a[4], b[4];
+  for (int i0 = 0; i0 < s.n_parts; i0 += 8) {
+    f32x4 a[8], b[8];
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int u = 0; u < 8; ++u)
       if (i0 + u < s.n_parts) {
         a[u] = *reinterpret_cast<const f32x4*>(src + (i0 + u) * s.stride);
         b[u] = *reinterpret_cast<const f32x4*>(src + (i0 + u) * s.stride + 4);
       }
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int u = 0; u < 8; ++u)
       if (i0 + u < s.n_parts) { x0 += a[u]; x1 += b[u]; }
   }
   const float x[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};

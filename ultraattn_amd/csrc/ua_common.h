@@ -13,6 +13,7 @@ typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 
+constexpr int kCus = 256;               // compute units of the device
 constexpr int kTile = UA_TILE;          // 128 x 128 kernel tile
 constexpr int kHeadDim = UA_HEAD_DIM;   // 128
 constexpr int kRowBytes = kHeadDim * 2; // one K/V/Q row of bf16 in LDS
