@@ -503,14 +503,17 @@ __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_block, 
 #pragma unroll
   for (int ks = 0; ks < 8; ++ks) asm volatile("" : "+v"(qf[ks]), "+v"(dof[ks]));
 
-  int causal = 0;
+  int causal = 0, kt_ahead = 0;
   auto step = [&](int i, auto stage_tag) {
     constexpr int kStage = decltype(stage_tag)::value;
-    if (i >= n_steps) return;   // workgroup-uniform
+    constexpr bool kSecond = kGroups == 1 && kStage == 1, kFirst = kGroups == 1 && kStage == 0;      // half of one tile
+    if (!kSecond && i >= n_steps) return;      // workgroup-uniform
     const int e = e0 + (kGroups == 1 ? i >> 1 : i), half = kGroups == 1 ? kStage : group;
-    if (kGroups == 2 || kStage == 0) causal = is_causal(e);
-    const bool more = i + 1 < n_steps;
-    const int kt_next = kGroups == 1 && kStage == 0 ? kt : (more ? ktile(e + 1) : kt);
+    if (!kSecond) causal = is_causal(e);
+    const bool more = kFirst || i + 1 < n_steps;
+    // the next tile's index: read a half tile before the copy that needs it
+    if (kFirst) kt_ahead = i + 2 < n_steps ? ktile(e + 1) : kt;
+    const int kt_next = kFirst ? kt : (kSecond ? kt_ahead : (more ? ktile(e + 1) : kt));
     wait_vmem_all();
     __syncthreads();            // this stage has landed; everyone is done with the other one
     if (more) in.copy_in((int64_t)kt_next * kTile + (kGroups == 1 ? kStage ^ 1 : group) * kHalf, kStage ^ 1);

@@ -221,14 +221,17 @@ __global__ __launch_bounds__(256 * kGroups, 2) void fwd_kernel(const FwdParams p
   const TrLane tr(lane);
 
   bool started = false;
-  int causal = 0;
+  int causal = 0, kt_ahead = 0;
   auto step = [&](int i, auto stage_tag) {
     constexpr int kStage = decltype(stage_tag)::value;
-    if (i >= n_steps) return;              // workgroup-uniform
+    constexpr bool kSecond = kGroups == 1 && kStage == 1, kFirst = kGroups == 1 && kStage == 0;      // half of one tile
+    if (!kSecond && i >= n_steps) return;  // workgroup-uniform
     const int e = entry_of(i), half = kGroups == 1 ? kStage : group;
-    if (kGroups == 2 || kStage == 0) causal = is_causal(e);
-    const bool more = i + 1 < n_steps;
-    const int kt_next = kGroups == 1 && kStage == 0 ? kt : (more ? ktile(e + 1) : kt);
+    if (!kSecond) causal = is_causal(e);
+    const bool more = kFirst || i + 1 < n_steps;
+    // the next tile's index: read a half tile before the copy that needs it
+    if (kFirst) kt_ahead = i + 2 < n_steps ? ktile(e + 1) : kt;
+    const int kt_next = kFirst ? kt : (kSecond ? kt_ahead : (more ? ktile(e + 1) : kt));
     // this stage has landed; everyone is done with the other one
     wait_vmem_all();
     __syncthreads();
