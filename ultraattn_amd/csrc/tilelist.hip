@@ -123,8 +123,16 @@ __device__ __forceinline__ bool line_of_wave(int nqb, int nkb, int rate, Line& l
   ln.step = ln.is_row ? 1 : nkb;
   return ln.id < (ln.is_row ? nqt : nkt);
 }
-__device__ __forceinline__ int tiles_of_block(const Line& ln, int type, int rate) {
-  return type == 1 ? rate : (type == 2 ? (ln.is_row ? ln.sub + 1 : rate - ln.sub) : 0);
+// Tiles that a CAUSAL block gives to the line; all of them give the same number, so sums over lanes are bit counts.
+__device__ __forceinline__ int causal_tiles(const Line& ln, int rate) { return ln.is_row ? ln.sub + 1 : rate - ln.sub; }
+// Types of 64 * kAhead blocks of the line, block i0 + 64 * u + lane in type[u], 0 beyond its end; all loads in flight at once.
+constexpr int kAhead = 4;
+__device__ __forceinline__ void load_types(const uint8_t* mask, const Line& ln, int i0, int (&type)[kAhead]) {
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u) {
+    const int i = i0 + 64 * u + (threadIdx.x & 63);
+    type[u] = i < ln.n_blocks ? mask[ln.base + i * ln.step] : 0;
+  }
 }
 __device__ __forceinline__ int wave_sum(int v) {
 #pragma unroll
@@ -141,16 +149,18 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void tl_count_kernel(const uin
   if (!line_of_wave(nqb, nkb, rate, ln)) return;
   const int lane = threadIdx.x & 63;
   int n = 0, bad = 0;
-  for (int i = lane; i < ln.n_blocks; i += 64) {
-    const int type = mask[ln.base + i * ln.step];
-    n += tiles_of_block(ln, type, rate);
-    bad += type > 2;
+  for (int i0 = 0; i0 < ln.n_blocks; i0 += 64 * kAhead) {
+    int type[kAhead];
+    load_types(mask, ln, i0, type);
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      n += rate * __popcll(__ballot(type[u] == 1)) + causal_tiles(ln, rate) * __popcll(__ballot(type[u] == 2));
+      bad += __popcll(__ballot(type[u] > 2));
+    }
   }
-  n = wave_sum(n);
-  if (lane == 0) (ln.is_row ? qcnt : kcnt)[ln.id] = n;
-  if (!ln.is_row) return;
-  bad = ln.sub == 0 ? wave_sum(bad) : 0;
-  if (lane == 0) row_invalid[ln.id] = bad;
+  if (lane != 0) return;
+  (ln.is_row ? qcnt : kcnt)[ln.id] = n;
+  if (ln.is_row) row_invalid[ln.id] = ln.sub == 0 ? bad : 0;
 }
 
 // fill: a workgroup first adds up the counts of its side (those before its lines give its place in the list,
@@ -166,14 +176,28 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void tl_fill_kernel(const uint
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int n = (ln.is_row ? nqb : nkb) * rate, first_line = ln.id - wave;
   const int32_t* cnt = ln.is_row ? qcnt : kcnt;
+  int type[kAhead];                   // the first blocks are on their way while the counts are added up
+  if (live) load_types(mask, ln, 0, type);
   int before = 0, all = 0, bad = 0;
-  for (int i = threadIdx.x; i < n; i += 64 * kWavesPerGroup) {
-    const int c = cnt[i] & kCountBits;
-    all += c;
-    if (i < first_line) before += c;
-    if (blockIdx.x == 0) bad += row_invalid[i];
+  for (int i0 = threadIdx.x; i0 < n; i0 += 64 * kWavesPerGroup * kAhead) {
+    int c[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int i = i0 + 64 * kWavesPerGroup * u;
+      c[u] = i < n ? cnt[i] & kCountBits : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      all += c[u];
+      if (i0 + 64 * kWavesPerGroup * u < first_line) before += c[u];
+    }
   }
-  before = wave_sum(before); all = wave_sum(all); bad = wave_sum(bad);
+  if (blockIdx.x == 0)
+    for (int i = threadIdx.x; i < n; i += 64 * kWavesPerGroup) bad += row_invalid[i];
+  int own = 0;                        // lines of the workgroup before this wavefront's
+  for (int w = 0; w < wave; ++w) own += first_line + w < n ? cnt[first_line + w] & kCountBits : 0;
+  before = wave_sum(before); all = wave_sum(all);
+  if (blockIdx.x == 0) bad = wave_sum(bad);
   if (lane == 0) { part[wave][0] = before; part[wave][1] = all; part[wave][2] = bad; }
   __syncthreads();
   before = all = bad = 0;
@@ -181,43 +205,39 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void tl_fill_kernel(const uint
   for (int w = 0; w < kWavesPerGroup; ++w) { before += part[w][0]; all += part[w][1]; bad += part[w][2]; }
   if (blockIdx.x == 0 && threadIdx.x == 0) *n_invalid = bad;
   if (!live) return;
-  int e = before;
-  for (int w = 0; w < wave; ++w) e += cnt[first_line + w] & kCountBits;
+  int e = before + own;
   int32_t* ptr = ln.is_row ? row_ptr : col_ptr;
   if (lane == 0) {
     ptr[ln.id] = e;
     if (ln.id == n - 1) ptr[n] = all;
   }
-  const int begin = e;
+  const int begin = e, n_causal = causal_tiles(ln, rate);
+  const uint64_t below = (1ull << lane) - 1;
   int32_t* idx = ln.is_row ? col_idx : row_idx;
   uint8_t* flg = ln.is_row ? flag : cflag;
   int first_idx = -1, last_idx = -1;
-  for (int i0 = 0; i0 < ln.n_blocks; i0 += 64) {
-    const int i = i0 + lane;
-    const int type = i < ln.n_blocks ? mask[ln.base + i * ln.step] : 0;
-    const int c = tiles_of_block(ln, type, rate);
-    int incl = c;
+  for (int i0 = 0; i0 < ln.n_blocks; i0 += 64 * kAhead) {
+    if (i0 > 0) load_types(mask, ln, i0, type);
 #pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int v = __shfl_up(incl, off);
-      if (lane >= off) incl += v;
-    }
-    int at = e + incl - c;
-    // sub-tiles along the line: a row takes key sub-tiles 0..sub of a causal block (the last one
-    // causal), a column takes query sub-tiles sub..rate-1 (the first one causal)
-    const int first = (type == 2 && !ln.is_row) ? ln.sub : 0;
-    for (int t = 0; t < c; ++t) {
-      const int s = first + t;
-      idx[at] = i * rate + s;
-      flg[at] = type == 2 && s == ln.sub;
-      ++at;
-    }
-    const uint64_t some = __ballot(c > 0);
-    if (some) {
+    for (int u = 0; u < kAhead; ++u) {
+      const int i = i0 + 64 * u + lane, ty = type[u];
+      const uint64_t full = __ballot(ty == 1), causal = __ballot(ty == 2), some = full | causal;
+      if (!some) continue;
+      const int c = ty == 1 ? rate : (ty == 2 ? n_causal : 0);
+      int at = e + rate * __popcll(full & below) + n_causal * __popcll(causal & below);
+      // sub-tiles along the line: a row takes key sub-tiles 0..sub of a causal block (the last one
+      // causal), a column takes query sub-tiles sub..rate-1 (the first one causal)
+      const int first = (ty == 2 && !ln.is_row) ? ln.sub : 0;
+      for (int t = 0; t < c; ++t) {
+        const int s = first + t;
+        idx[at] = i * rate + s;
+        flg[at] = ty == 2 && s == ln.sub;
+        ++at;
+      }
       if (first_idx < 0) first_idx = __shfl(i * rate + first, __ffsll((unsigned long long)some) - 1);
       last_idx = __shfl(i * rate + first + c - 1, 63 - __clzll((long long)some));
+      e += rate * __popcll(full) + n_causal * __popcll(causal);
     }
-    e += __shfl(incl, 63);
   }
   // anchors: lines that are neither empty nor very long (see very_long) mark their first and last index
   if (lane == 0 && e > begin && (int64_t)(e - begin) * n <= 2 * (int64_t)all) {
@@ -236,10 +256,11 @@ constexpr int kOrderThreads = 1024, kOrderLines = 8;
 __global__ __launch_bounds__(kOrderThreads) void tl_order_kernel(const int32_t* qptr, const int32_t* qidx, int nq, int32_t* q_order,
                                                                  const int32_t* kptr, const int32_t* kidx, int nk, int32_t* k_order, int rate,
                                                                  const int32_t* qcnt, const int32_t* kcnt) {
-  struct Key { int32_t very, len, anchor, block_len; };
+  struct Key { int32_t very, len, anchor, block_len, p; };
   __shared__ Key own[kOrderLines];
   __shared__ int32_t rank[kOrderLines], n_first, n_last, n_queued;
   __shared__ uint32_t queue[kOrderThreads * kOrderLines];          // pairs of one round: line | slot << 28
+  __shared__ int32_t list_at[kOrderThreads], list_len[kOrderThreads];
   const int groups_q = (nq + kOrderLines - 1) / kOrderLines;
   const bool rows = (int)blockIdx.x < groups_q;
   const int32_t *ptr = rows ? qptr : kptr, *idx = rows ? qidx : kidx, *marks = rows ? kcnt : qcnt;
@@ -248,26 +269,34 @@ __global__ __launch_bounds__(kOrderThreads) void tl_order_kernel(const int32_t* 
   const int tid = threadIdx.x, lane = tid & 63;
   if (tid < kOrderLines) rank[tid] = 0;
   if (tid == 0) n_first = n_last = n_queued = 0;
-  __syncthreads();
+  // Keys come with both ends of the list: everything this thread reads before the first barrier is on its way at once.
+  struct Raw { int32_t p, len, first, last, block_len; };
+  auto raw_of = [&](int i) {
+    const int p = ptr[i], len = ptr[i + 1] - p, r = i / rate * rate + longest_sub;
+    return Raw{p, len, len ? idx[p] : 0, len ? idx[p + len - 1] : 0, ptr[r + 1] - ptr[r]};
+  };
+  const int64_t twice_all = 2 * (int64_t)ptr[n];
+  Raw mine{}, own_raw{};
+  if (tid < n) mine = raw_of(tid);
+  if (tid < n_own) own_raw = raw_of(line0 + tid);
   // which end anchors the lists: the one with fewer distinct values
   int f = 0, l = 0;
   for (int i = tid; i < n_marks; i += kOrderThreads) { const int32_t m = marks[i]; f += (m & kIsFirst) != 0; l += (m & kIsLast) != 0; }
+  __syncthreads();
   f = wave_sum(f); l = wave_sum(l);
   if (lane == 0 && (f | l)) { atomicAdd(&n_first, f); atomicAdd(&n_last, l); }
   __syncthreads();
   const bool from_end = n_last < n_first;
-  const int64_t twice_all = 2 * (int64_t)ptr[n];
-  auto key_of = [&](int i) {
-    const int p = ptr[i], len = ptr[i + 1] - p, r = i / rate * rate + longest_sub;
-    return Key{(int64_t)len * n > twice_all, len, len ? idx[from_end ? p + len - 1 : p] : 0, ptr[r + 1] - ptr[r]};
-  };
-  if (tid < n_own) own[tid] = key_of(line0 + tid);
+  auto key_of = [&](const Raw& r) { return Key{(int64_t)r.len * n > twice_all, r.len, from_end ? r.last : r.first, r.block_len, r.p}; };
+  if (tid < n_own) own[tid] = key_of(own_raw);
   __syncthreads();
   int before[kOrderLines] = {};
   for (int j0 = 0; j0 < n; j0 += kOrderThreads) {
     const int j = j0 + tid;
     if (j < n) {
-      const Key a = key_of(j);
+      const Key a = key_of(j0 == 0 ? mine : raw_of(j));
+      list_at[tid] = a.p;
+      list_len[tid] = a.len;
 #pragma unroll
       for (int s = 0; s < kOrderLines; ++s) {
         if (s >= n_own || j == line0 + s) continue;
@@ -288,7 +317,7 @@ __global__ __launch_bounds__(kOrderThreads) void tl_order_kernel(const int32_t* 
     const int queued = n_queued;
     for (int e = tid >> 6; e < queued; e += kOrderThreads / 64) {
       const int ja = queue[e] & 0xfffffff, slot = queue[e] >> 28, ib = line0 + slot;
-      const int pa = ptr[ja], pb = ptr[ib], la = ptr[ja + 1] - pa, lb = ptr[ib + 1] - pb, m = min(la, lb);
+      const int pa = list_at[ja - j0], pb = own[slot].p, la = list_len[ja - j0], lb = own[slot].len, m = min(la, lb);
       const int sa = from_end ? pa + la - 1 : pa, sb = from_end ? pb + lb - 1 : pb, step = from_end ? -1 : 1;
       bool less = la != lb ? la > lb : ja < ib;                    // one list ends inside the other
       for (int t0 = 1; t0 < m; t0 += 256) {
