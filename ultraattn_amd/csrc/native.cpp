@@ -416,17 +416,28 @@ PyObject* build_lists_device(PyObject* const* a) {
     fail(PyExc_ValueError, "block_mask_dev must be a contiguous 2-D uint8 CUDA tensor");
   const int64_t nqt = m.size(0) * rate, nkt = m.size(1) * rate, cap = given >= 0 ? given : nqt * nkt;
   const int64_t room = ((cap > 1 ? cap : 1) + 3) / 4 * 4;         // not empty, whole 32-bit words of flags
-  const at::TensorOptions i32 = m.options().dtype(at::kInt), u8 = m.options();
-  at::Tensor t[9] = {at::empty({nqt + 1}, i32), at::empty({room}, i32), at::empty({room}, u8), at::empty({nkt + 1}, i32), at::empty({room}, i32),
-                     at::empty({room}, u8), at::empty({nqt}, i32), at::empty({nkt}, i32), at::empty({nqt + nkt + 7}, i32)};
+  // One allocation that the nine results are parts of, each on a 64-byte boundary: nine of them took a third of the call.
+  const int64_t bytes[9] = {4 * (nqt + 1), 4 * room, room, 4 * (nkt + 1), 4 * room, room, 4 * nqt, 4 * nkt, 4 * (nqt + nkt + 7)};
+  int64_t at_byte[10] = {0};
+  for (int i = 0; i < 9; ++i) at_byte[i + 1] = at_byte[i] + (bytes[i] + 63) / 64 * 64;
+  const at::Tensor all = at::empty({at_byte[9]}, m.options());
+  at::Tensor t[9];
+  for (int i = 0; i < 9; ++i) {
+    const bool flags = i == 2 || i == 5, list = flags || i == 1 || i == 4;
+    const int64_t size = flags ? 1 : 4;
+    auto impl = c10::make_intrusive<at::TensorImpl>(c10::Storage(all.storage()), all.key_set(), c10::scalarTypeToTypeMeta(flags ? at::kByte : at::kInt));
+    impl->set_storage_offset(at_byte[i] / size);
+    impl->set_sizes_contiguous({list ? cap : bytes[i] / size});
+    t[i] = at::Tensor(std::move(impl));
+  }
+  void* const base = all.data_ptr();
+  auto part = [&](int i) { return (void*)((char*)base + at_byte[i]); };
   const On on(m);
   call("ua_tilelist_build_device", [&] {
-    return ua_tilelist_build_device((const uint8_t*)m.data_ptr(), (int)m.size(0), (int)m.size(1), (int)rate, (int32_t*)t[0].data_ptr(),
-                                    (int32_t*)t[1].data_ptr(), (uint8_t*)t[2].data_ptr(), (int32_t*)t[3].data_ptr(), (int32_t*)t[4].data_ptr(),
-                                    (uint8_t*)t[5].data_ptr(), (int32_t*)t[6].data_ptr(), (int32_t*)t[7].data_ptr(), (int32_t*)t[8].data_ptr(), on.stream);
+    return ua_tilelist_build_device((const uint8_t*)m.data_ptr(), (int)m.size(0), (int)m.size(1), (int)rate, (int32_t*)part(0), (int32_t*)part(1),
+                                    (uint8_t*)part(2), (int32_t*)part(3), (int32_t*)part(4), (uint8_t*)part(5), (int32_t*)part(6), (int32_t*)part(7),
+                                    (int32_t*)part(8), on.stream);
   });
-  if (room != cap)
-    for (int i : {1, 2, 4, 5}) t[i] = t[i].narrow(0, 0, cap);
   PyObject* r = PyTuple_New(9);
   for (int i = 0; i < 9; ++i) PyTuple_SET_ITEM(r, i, THPVariable_Wrap(t[i]));
   return r;

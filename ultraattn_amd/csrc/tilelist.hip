@@ -91,7 +91,7 @@ static int check_mask(const uint8_t* mask, int nqb, int nkb, int rate) {
 // ---- device variant -----------------------------------------------------------------------
 // Three launches: count, fill, order.  At the benchmark's 256 x 256 blocks every one of them is a chain of a few
 // dependent loads, so what counts is how many launches there are and how long the longest chain is; eleven
-// launches (init, check, count, two scans, fill, three for the anchors, order) took 61 us.
+// launches (init, check, count, two scans, fill, three for the anchors, order) took 61 us a pass, these three 16.
 //
 // One wavefront per query tile (a "row" of the list) and per key tile (a "column"); lanes
 // stride over the blocks of that row or column of the block mask.  Number of active tiles
@@ -99,9 +99,6 @@ static int check_mask(const uint8_t* mask, int nqb, int nkb, int rate) {
 // sub-tiles 0..a); to key tile kt = kb*rate + b: FULL rate, CAUSAL rate - b (query sub-tiles
 // b..rate-1).
 constexpr int kWavesPerGroup = 4;
-// A line's entry in the work array: its tile count, and whether its index is the first (last) index of
-// some line of the other side (set by the fill kernel for the order kernel's choice of anchor).
-constexpr int32_t kCountBits = 0x3fffffff, kIsFirst = 1 << 30, kIsLast = (int32_t)(1u << 31);
 
 struct Line {          // one row or one column of the tile grid, as seen by its wavefront
   bool is_row;
@@ -134,10 +131,18 @@ __device__ __forceinline__ void load_types(const uint8_t* mask, const Line& ln, 
     type[u] = i < ln.n_blocks ? mask[ln.base + i * ln.step] : 0;
   }
 }
+// Sum over the wavefront by DPP additions (rows of 16, then across them; the total arrives in lane 63): through
+// LDS, as shuffles go, each of the six steps takes 60 ns.
+template <int kCtrl, int kRows>
+__device__ __forceinline__ int dpp_add(int v) { return v + __builtin_amdgcn_update_dpp(0, v, kCtrl, kRows, 0xf, false); }
 __device__ __forceinline__ int wave_sum(int v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-  return v;
+  v = dpp_add<0x111, 0xf>(v);      // row_shr 1, 2, 4, 8
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);      // row_bcast 15 into rows 1 and 3
+  v = dpp_add<0x143, 0xc>(v);      // row_bcast 31 into rows 2 and 3
+  return __builtin_amdgcn_readlane(v, 63);
 }
 
 // count: tiles per line.  The builder treats mask entries that are not a Block_Type (> 2) as EMPTY; how many
@@ -163,11 +168,13 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void tl_count_kernel(const uin
   if (ln.is_row) row_invalid[ln.id] = ln.sub == 0 ? bad : 0;
 }
 
+typedef __attribute__((ext_vector_type(4), aligned(4))) int32_t i32x4_any;       // at any element of a list
+typedef __attribute__((aligned(1))) uint32_t u32_any;
 // fill: a workgroup first adds up the counts of its side (those before its lines give its place in the list,
 // all of them the list's length), then each wavefront walks its line 64 blocks at a time; an exclusive
 // scan of the per-block tile counts gives every lane the slot where its block's tiles go, in ascending order.
-__global__ __launch_bounds__(64 * kWavesPerGroup) void tl_fill_kernel(const uint8_t* mask, int nqb, int nkb, int rate, int32_t* qcnt, int32_t* kcnt,
-                                                                       int32_t* row_ptr, int32_t* col_idx, uint8_t* flag,
+__global__ __launch_bounds__(64 * kWavesPerGroup) void tl_fill_kernel(const uint8_t* mask, int nqb, int nkb, int rate,
+                                                                       const int32_t* qcnt, const int32_t* kcnt, int32_t* row_ptr, int32_t* col_idx, uint8_t* flag,
                                                                        int32_t* col_ptr, int32_t* row_idx, uint8_t* cflag,
                                                                        const int32_t* row_invalid, int32_t* n_invalid) {
   __shared__ int32_t part[kWavesPerGroup][3];
@@ -184,7 +191,7 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void tl_fill_kernel(const uint
 #pragma unroll
     for (int u = 0; u < kAhead; ++u) {
       const int i = i0 + 64 * kWavesPerGroup * u;
-      c[u] = i < n ? cnt[i] & kCountBits : 0;
+      c[u] = i < n ? cnt[i] : 0;
     }
 #pragma unroll
     for (int u = 0; u < kAhead; ++u) {
@@ -195,7 +202,7 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void tl_fill_kernel(const uint
   if (blockIdx.x == 0)
     for (int i = threadIdx.x; i < n; i += 64 * kWavesPerGroup) bad += row_invalid[i];
   int own = 0;                        // lines of the workgroup before this wavefront's
-  for (int w = 0; w < wave; ++w) own += first_line + w < n ? cnt[first_line + w] & kCountBits : 0;
+  for (int w = 0; w < wave; ++w) own += first_line + w < n ? cnt[first_line + w] : 0;
   before = wave_sum(before); all = wave_sum(all);
   if (blockIdx.x == 0) bad = wave_sum(bad);
   if (lane == 0) { part[wave][0] = before; part[wave][1] = all; part[wave][2] = bad; }
@@ -211,66 +218,62 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void tl_fill_kernel(const uint
     ptr[ln.id] = e;
     if (ln.id == n - 1) ptr[n] = all;
   }
-  const int begin = e, n_causal = causal_tiles(ln, rate);
+  const int n_causal = causal_tiles(ln, rate);
   const uint64_t below = (1ull << lane) - 1;
   int32_t* idx = ln.is_row ? col_idx : row_idx;
   uint8_t* flg = ln.is_row ? flag : cflag;
-  int first_idx = -1, last_idx = -1;
   for (int i0 = 0; i0 < ln.n_blocks; i0 += 64 * kAhead) {
     if (i0 > 0) load_types(mask, ln, i0, type);
 #pragma unroll
     for (int u = 0; u < kAhead; ++u) {
       const int i = i0 + 64 * u + lane, ty = type[u];
-      const uint64_t full = __ballot(ty == 1), causal = __ballot(ty == 2), some = full | causal;
-      if (!some) continue;
+      const uint64_t full = __ballot(ty == 1), causal = __ballot(ty == 2);
+      if (!(full | causal)) continue;
       const int c = ty == 1 ? rate : (ty == 2 ? n_causal : 0);
       int at = e + rate * __popcll(full & below) + n_causal * __popcll(causal & below);
       // sub-tiles along the line: a row takes key sub-tiles 0..sub of a causal block (the last one
       // causal), a column takes query sub-tiles sub..rate-1 (the first one causal)
       const int first = (ty == 2 && !ln.is_row) ? ln.sub : 0;
-      for (int t = 0; t < c; ++t) {
-        const int s = first + t;
-        idx[at] = i * rate + s;
-        flg[at] = ty == 2 && s == ln.sub;
-        ++at;
+      // four tiles and their flags per store
+      int t = 0;
+      for (; t + 4 <= c; t += 4, at += 4) {
+        const int s = i * rate + first + t, mark = ln.sub - first - t;           // the causal one among them, if 0..3
+        *reinterpret_cast<i32x4_any*>(idx + at) = i32x4_any{s, s + 1, s + 2, s + 3};
+        *reinterpret_cast<u32_any*>(flg + at) = ty == 2 && (unsigned)mark < 4 ? 1u << (8 * mark) : 0;
       }
-      if (first_idx < 0) first_idx = __shfl(i * rate + first, __ffsll((unsigned long long)some) - 1);
-      last_idx = __shfl(i * rate + first + c - 1, 63 - __clzll((long long)some));
+      for (; t < c; ++t, ++at) {
+        idx[at] = i * rate + first + t;
+        flg[at] = ty == 2 && first + t == ln.sub;
+      }
       e += rate * __popcll(full) + n_causal * __popcll(causal);
     }
-  }
-  // anchors: lines that are neither empty nor very long (see very_long) mark their first and last index
-  if (lane == 0 && e > begin && (int64_t)(e - begin) * n <= 2 * (int64_t)all) {
-    int32_t* other = ln.is_row ? kcnt : qcnt;
-    atomicOr(&other[first_idx], kIsFirst);
-    atomicOr(&other[last_idx], kIsLast);
   }
 }
 
 // order: rank of a line = number of lines that precede it by row_precedes.  A workgroup ranks kOrderLines lines:
-// every thread reads the keys (very long, anchor, block-line length) of one other line and compares them with those of
-// all kOrderLines; the few pairs that only the index lists decide are queued, and a wavefront compares 256
-// indices of both lists at once.  One line per workgroup and a thread per pair, list comparison included:
-// 32 us for 2 x 1024 lines, most of it the four rows of a block walking their common list one index at a time.
-constexpr int kOrderThreads = 1024, kOrderLines = 8;
+// every thread packs what decides first about one other line (very long, anchor, block-line length) into one 64-bit key
+// and compares it with those of all kOrderLines; counts are ballots.  Pairs with equal keys are queued: lines of one block are decided by what refinement
+// makes of their common row of the mask, for the others 16 lanes compare 64 indices of both lists at once.  One line per workgroup and a thread per pair, list comparison included: 32 us for
+// 2 x 1024 lines, most of it the four rows of a block walking their common list one index at a time.
+constexpr int kOrderThreads = 1024, kOrderLines = 8, kSeen = 8192;
 __global__ __launch_bounds__(kOrderThreads) void tl_order_kernel(const int32_t* qptr, const int32_t* qidx, int nq, int32_t* q_order,
-                                                                 const int32_t* kptr, const int32_t* kidx, int nk, int32_t* k_order, int rate,
-                                                                 const int32_t* qcnt, const int32_t* kcnt) {
-  struct Key { int32_t very, len, anchor, block_len, p; };
-  __shared__ Key own[kOrderLines];
+                                                                 const int32_t* kptr, const int32_t* kidx, int nk, int32_t* k_order, int rate) {
+  struct ListOf { int32_t at, len, first; };
+  __shared__ uint64_t own_key[kOrderLines];
+  __shared__ ListOf own[kOrderLines], other[kOrderThreads];
   __shared__ int32_t rank[kOrderLines], n_first, n_last, n_queued;
+  __shared__ uint32_t seen_first[kSeen / 4], seen_last[kSeen / 4];             // a byte per value
   __shared__ uint32_t queue[kOrderThreads * kOrderLines];          // pairs of one round: line | slot << 28
-  __shared__ int32_t list_at[kOrderThreads], list_len[kOrderThreads];
   const int groups_q = (nq + kOrderLines - 1) / kOrderLines;
   const bool rows = (int)blockIdx.x < groups_q;
-  const int32_t *ptr = rows ? qptr : kptr, *idx = rows ? qidx : kidx, *marks = rows ? kcnt : qcnt;
+  const int32_t *ptr = rows ? qptr : kptr, *idx = rows ? qidx : kidx;
   const int n = rows ? nq : nk, n_marks = rows ? nk : nq, longest_sub = rows ? rate - 1 : 0;
   const int line0 = (blockIdx.x - (rows ? 0 : groups_q)) * kOrderLines, n_own = min(kOrderLines, n - line0);
   const int tid = threadIdx.x, lane = tid & 63;
   if (tid < kOrderLines) rank[tid] = 0;
   if (tid == 0) n_first = n_last = n_queued = 0;
-  // Keys come with both ends of the list: everything this thread reads before the first barrier is on its way at once.
-  struct Raw { int32_t p, len, first, last, block_len; };
+  // Both ends of the list are read, so that everything the first round needs is on its way before the first barrier.
+  struct Raw { int32_t at, len, first, last, block_len; };
   auto raw_of = [&](int i) {
     const int p = ptr[i], len = ptr[i + 1] - p, r = i / rate * rate + longest_sub;
     return Raw{p, len, len ? idx[p] : 0, len ? idx[p + len - 1] : 0, ptr[r + 1] - ptr[r]};
@@ -279,77 +282,107 @@ __global__ __launch_bounds__(kOrderThreads) void tl_order_kernel(const int32_t* 
   Raw mine{}, own_raw{};
   if (tid < n) mine = raw_of(tid);
   if (tid < n_own) own_raw = raw_of(line0 + tid);
-  // which end anchors the lists: the one with fewer distinct values
-  int f = 0, l = 0;
-  for (int i = tid; i < n_marks; i += kOrderThreads) { const int32_t m = marks[i]; f += (m & kIsFirst) != 0; l += (m & kIsLast) != 0; }
-  __syncthreads();
-  f = wave_sum(f); l = wave_sum(l);
-  if (lane == 0 && (f | l)) { atomicAdd(&n_first, f); atomicAdd(&n_last, l); }
-  __syncthreads();
+  // Which end anchors the lists: the one with fewer distinct values over the lines that are neither empty nor very
+  // long, counted kSeen values at a time.  (Marking them in memory, in the fill kernel, cost 5 us: lines share
+  // their anchors, and atomics of many XCDs on one word are served one by one.)
+  auto very_long = [&](int len) { return (int64_t)len * n > twice_all; };
+  for (int v0 = 0; v0 < n_marks; v0 += kSeen) {
+    const int words = (min(n_marks - v0, kSeen) + 3) / 4;
+    for (int i = tid; i < words; i += kOrderThreads) seen_first[i] = seen_last[i] = 0;
+    __syncthreads();
+    for (int i = tid; i < n; i += kOrderThreads) {
+      const Raw r = i == tid ? mine : raw_of(i);
+      const uint32_t f = r.first - v0, l = r.last - v0;
+      if (r.len == 0 || very_long(r.len)) continue;
+      if (f < kSeen) reinterpret_cast<uint8_t*>(seen_first)[f] = 1;
+      if (l < kSeen) reinterpret_cast<uint8_t*>(seen_last)[l] = 1;
+    }
+    __syncthreads();
+    int f = 0, l = 0;
+    for (int i = tid; i < words; i += kOrderThreads) { f += __popc(seen_first[i]); l += __popc(seen_last[i]); }
+    f = wave_sum(f); l = wave_sum(l);
+    if (lane == 0 && (f | l)) { atomicAdd(&n_first, f); atomicAdd(&n_last, l); }
+    __syncthreads();
+  }
   const bool from_end = n_last < n_first;
-  auto key_of = [&](const Raw& r) { return Key{(int64_t)r.len * n > twice_all, r.len, from_end ? r.last : r.first, r.block_len, r.p}; };
-  if (tid < n_own) own[tid] = key_of(own_raw);
+  // very long lines first, among them by block-line length before the anchor; empty ones last
+  auto key_of = [&](const Raw& r) {
+    const uint64_t anchor = from_end ? r.last : r.first, shorter = (1 << 30) - 1 - r.block_len;
+    if (r.len == 0) return ~0ull;
+    return very_long(r.len) ? shorter << 30 | anchor : 1ull << 62 | anchor << 30 | shorter;
+  };
+  if (tid < kOrderLines) {
+    own_key[tid] = tid < n_own ? key_of(own_raw) : 0;            // no line has a smaller key than 0, nor that one
+    own[tid] = {own_raw.at, own_raw.len, own_raw.first};
+  }
   __syncthreads();
-  int before[kOrderLines] = {};
+  int before[kOrderLines] = {};        // of this wavefront's lines, how many come first
   for (int j0 = 0; j0 < n; j0 += kOrderThreads) {
     const int j = j0 + tid;
-    if (j < n) {
-      const Key a = key_of(j0 == 0 ? mine : raw_of(j));
-      list_at[tid] = a.p;
-      list_len[tid] = a.len;
+    if (j0 > 0 && j < n) mine = raw_of(j);
+    const uint64_t key = j < n ? key_of(mine) : ~0ull;
+    other[tid] = {mine.at, mine.len, mine.first};
 #pragma unroll
-      for (int s = 0; s < kOrderLines; ++s) {
-        if (s >= n_own || j == line0 + s) continue;
-        const Key b = own[s];
-        bool less;
-        if (a.very != b.very) less = a.very > b.very;
-        else if (a.len == 0 || b.len == 0) less = a.len != b.len ? a.len > b.len : j < line0 + s;
-        else if (a.anchor == b.anchor && a.block_len == b.block_len) {
-          queue[atomicAdd(&n_queued, 1)] = (uint32_t)j | (uint32_t)s << 28;
-          less = false;
-        }
-        else if (a.very ? a.block_len != b.block_len : a.anchor == b.anchor) less = a.block_len > b.block_len;
-        else less = a.anchor < b.anchor;
-        before[s] += less;
+    for (int s = 0; s < kOrderLines; ++s) {
+      const uint64_t b = own_key[s];
+      before[s] += __popcll(__ballot(key < b));
+      if (__any(key == b)) {
+        if (key == b && j < n && j != line0 + s) queue[atomicAdd(&n_queued, 1)] = (uint32_t)j | (uint32_t)s << 28;
       }
     }
     __syncthreads();
     const int queued = n_queued;
-    for (int e = tid >> 6; e < queued; e += kOrderThreads / 64) {
-      const int ja = queue[e] & 0xfffffff, slot = queue[e] >> 28, ib = line0 + slot;
-      const int pa = list_at[ja - j0], pb = own[slot].p, la = list_len[ja - j0], lb = own[slot].len, m = min(la, lb);
-      const int sa = from_end ? pa + la - 1 : pa, sb = from_end ? pb + lb - 1 : pb, step = from_end ? -1 : 1;
-      bool less = la != lb ? la > lb : ja < ib;                    // one list ends inside the other
-      for (int t0 = 1; t0 < m; t0 += 256) {
-        int ca[4], cb[4];
+    for (int e0 = (tid >> 6) * 4; e0 < queued; e0 += kOrderThreads / 16) {
+      const int quarter = lane >> 4, sub = lane & 15;
+      const bool live = e0 + quarter < queued;
+      const uint32_t pair = queue[live ? e0 + quarter : e0];
+      const int ja = pair & 0xfffffff, slot = pair >> 28;
+      const ListOf a = other[ja - j0], b = own[slot];
+      const int m = min(a.len, b.len), step = from_end ? -1 : 1;
+      const int sa = from_end ? a.at + a.len - 1 : a.at, sb = from_end ? b.at + b.len - 1 : b.at;
+      const int d = ja - (line0 + slot), d_len = a.len - b.len;
+      bool less = d_len != 0 ? d_len > 0 : d < 0;                  // one list ends inside the other, or they are equal
+      bool open = live && m > 0;
+      // Lines of one block: their lists differ only where the block's line of the mask is CAUSAL, and by the number of
+      // such blocks in length (the same lists if there is none).
+      if (ja / rate == (line0 + slot) / rate) {
+        if (d_len == 0)                 open = false;
+        else if (rows)                { open = false; less = from_end ? d < 0 : d > 0; }      // keys 0..sub of the block: the longer list goes on in it
+        else if (!from_end)           { open = false; less = d < 0; }                         // queries sub..: the smaller sub's come first
+        else if (a.first == b.first)  { open = false; less = d > 0; }                         // read backwards, the larger sub leaves the block first
+        else if (abs(d_len) == abs(d)){ open = false; less = d < 0; }                         // and, this being the only one, ends there
+      }
+      for (int t0 = 1; __any(open && t0 < m); t0 += 64) {
+        int ca[4] = {}, cb[4] = {};
+        open &= t0 < m;
+        if (open) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int t = min(t0 + 64 * u + lane, m - 1);
-          ca[u] = idx[sa + t * step];
-          cb[u] = idx[sb + t * step];
-        }
-        bool found = false;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const uint64_t differ = __ballot(ca[u] != cb[u]);
-          if (differ && !found) {
-            found = true;
-            less = __shfl((int)(ca[u] < cb[u]), __ffsll((unsigned long long)differ) - 1) != 0;
+          for (int u = 0; u < 4; ++u) {
+            const int t = min(t0 + 16 * u + sub, m - 1);
+            ca[u] = idx[sa + t * step];
+            cb[u] = idx[sb + t * step];
           }
         }
-        if (found) break;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const uint32_t differ = (uint32_t)(__ballot(ca[u] != cb[u]) >> (16 * quarter)) & 0xffff;
+          const uint32_t smaller = (uint32_t)(__ballot(ca[u] < cb[u]) >> (16 * quarter));
+          if (open && differ) {
+            less = (smaller >> (__ffs(differ) - 1)) & 1;
+            open = false;
+          }
+        }
       }
-      if (lane == 0 && less) atomicAdd(&rank[slot], 1);
+      if (sub == 0 && live && less) atomicAdd(&rank[slot], 1);
     }
     __syncthreads();
     if (tid == 0) n_queued = 0;
     __syncthreads();
   }
+  int add = 0;
 #pragma unroll
-  for (int s = 0; s < kOrderLines; ++s) {
-    const int c = wave_sum(before[s]);
-    if (lane == 0 && c) atomicAdd(&rank[s], c);
-  }
+  for (int s = 0; s < kOrderLines; ++s) add = lane == s ? before[s] : add;
+  if (lane < n_own && add) atomicAdd(&rank[lane], add);
   __syncthreads();
   if (tid < n_own) (rows ? q_order : k_order)[rank[tid]] = line0 + tid;
 }
@@ -424,11 +457,11 @@ static int build_device_impl(const uint8_t* block_mask, int n_qblocks, int n_kbl
   int32_t* kcnt = work + nqt + 1;
   const dim3 lines((unsigned)(line_groups(nqt) + line_groups(nkt))), group(64 * kWavesPerGroup);
   hipLaunchKernelGGL(tl_count_kernel, lines, group, 0, st, block_mask, n_qblocks, n_kblocks, rate, qcnt, kcnt, q_order);
-  hipLaunchKernelGGL(tl_fill_kernel, lines, group, 0, st, block_mask, n_qblocks, n_kblocks, rate, qcnt, kcnt, row_ptr, col_idx, flag,
+  hipLaunchKernelGGL(tl_fill_kernel, lines, group, 0, st, block_mask, n_qblocks, n_kblocks, rate, (const int32_t*)qcnt, (const int32_t*)kcnt, row_ptr, col_idx, flag,
                      col_ptr, row_idx, cflag, (const int32_t*)q_order, n_invalid);
   hipLaunchKernelGGL(tl_order_kernel, dim3((unsigned)((nqt + kOrderLines - 1) / kOrderLines + (nkt + kOrderLines - 1) / kOrderLines)),
                      dim3(kOrderThreads), 0, st, (const int32_t*)row_ptr, (const int32_t*)col_idx, nqt, q_order,
-                     (const int32_t*)col_ptr, (const int32_t*)row_idx, nkt, k_order, rate, (const int32_t*)qcnt, (const int32_t*)kcnt);
+                     (const int32_t*)col_ptr, (const int32_t*)row_idx, nkt, k_order, rate);
   return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH;
 }
 
