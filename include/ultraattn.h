@@ -99,12 +99,12 @@ int ua_tilelist_build(const uint8_t *block_mask, int n_qblocks, int n_kblocks, i
  * The mask cannot be validated without a synchronisation: an entry that is not 0, 1 or 2 is
  * treated as EMPTY, and work[n_qtiles + n_ktiles + 2] receives the number of such entries (0 for
  * a valid mask; the host builder returns UA_ERR_MASK instead) for the caller to read later.
- * Cost: counting, filling and the anchor statistics are linear in the mask; the launch order ranks
- * every line against every other line of its side (comparisons stop at the first differing
+ * Cost: counting and filling are linear in the mask; the launch order compares every line with every
+ * other line of its side (lists only where their first keys agree, up to the first differing
  * index), i.e. it grows with the square of the number of lines.  Measured on MI355X, n_qtiles +
- * n_ktiles lines: 2 048 lines 0.1-0.3 ms, 8 192 lines 0.4-1.0 ms (dense causal: 0.4 ms),
- * 16 384 lines 1.1-2.7 ms, 32 768 lines 5-10 ms, 65 532 lines 34-45 ms (band and causal-band masks);
- * the benchmark masks have 2 048 to 4 608 lines (0.07-0.1 ms).                                */
+ * n_ktiles lines of band and causal masks: 2 048 lines 15 us, 8 192 lines 0.09 ms, 16 384 lines
+ * 0.32-0.36 ms, 32 768 lines 1.5 ms, 65 532 lines 9 ms; the benchmark masks have 2 048 to 4 608 lines:
+ * strided 15 us, streaming shard 0.09 ms, global+local, whose lines share long prefixes, 0.17 ms. */
 int ua_tilelist_build_device(const uint8_t *block_mask, int n_qblocks, int n_kblocks, int rate,
                              int32_t *row_ptr, int32_t *col_idx, uint8_t *flag,
                              int32_t *col_ptr, int32_t *row_idx, uint8_t *cflag,

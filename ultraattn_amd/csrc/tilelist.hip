@@ -305,14 +305,14 @@ __global__ __launch_bounds__(kOrderThreads) void tl_order_kernel(const int32_t* 
     __syncthreads();
   }
   const bool from_end = n_last < n_first;
-  // very long lines first, among them by block-line length before the anchor; empty ones last
-  auto key_of = [&](const Raw& r) {
+  // very long lines first, among them by block-line length before the anchor; empty ones last, by number
+  auto key_of = [&](const Raw& r, int i) {
     const uint64_t anchor = from_end ? r.last : r.first, shorter = (1 << 30) - 1 - r.block_len;
-    if (r.len == 0) return ~0ull;
+    if (r.len == 0) return 1ull << 63 | (uint64_t)i;
     return very_long(r.len) ? shorter << 30 | anchor : 1ull << 62 | anchor << 30 | shorter;
   };
   if (tid < kOrderLines) {
-    own_key[tid] = tid < n_own ? key_of(own_raw) : 0;            // no line has a smaller key than 0, nor that one
+    own_key[tid] = tid < n_own ? key_of(own_raw, line0 + tid) : 0;            // no line has a smaller key than 0, nor that one
     own[tid] = {own_raw.at, own_raw.len, own_raw.first};
   }
   __syncthreads();
@@ -320,7 +320,7 @@ __global__ __launch_bounds__(kOrderThreads) void tl_order_kernel(const int32_t* 
   for (int j0 = 0; j0 < n; j0 += kOrderThreads) {
     const int j = j0 + tid;
     if (j0 > 0 && j < n) mine = raw_of(j);
-    const uint64_t key = j < n ? key_of(mine) : ~0ull;
+    const uint64_t key = j < n ? key_of(mine, j) : ~0ull;
     other[tid] = {mine.at, mine.len, mine.first};
 #pragma unroll
     for (int s = 0; s < kOrderLines; ++s) {
@@ -342,7 +342,7 @@ __global__ __launch_bounds__(kOrderThreads) void tl_order_kernel(const int32_t* 
       const int sa = from_end ? a.at + a.len - 1 : a.at, sb = from_end ? b.at + b.len - 1 : b.at;
       const int d = ja - (line0 + slot), d_len = a.len - b.len;
       bool less = d_len != 0 ? d_len > 0 : d < 0;                  // one list ends inside the other, or they are equal
-      bool open = live && m > 0;
+      bool open = live;
       // Lines of one block: their lists differ only where the block's line of the mask is CAUSAL, and by the number of
       // such blocks in length (the same lists if there is none).
       if (ja / rate == (line0 + slot) / rate) {
