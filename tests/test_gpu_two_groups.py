@@ -1,5 +1,5 @@
-"""Workgroups of two groups that share a tile line: walks of no tile, one tile and an odd number of them, rows whose
-causal tile is not the last one, and launches on both sides of every bound at which the two groups are chosen."""
+"""Workgroups of two and four groups that share a tile line: walks of no tile, one tile and an odd number of them, rows whose
+causal tile is not the last one, and launches on both sides of every bound at which the groups are chosen."""
 import numpy as np
 import pytest
 import torch
@@ -45,7 +45,10 @@ def test_short_and_odd_walks(mask):
 
 @pytest.mark.parametrize("sq,sk,nh,causal", [
     (512, 128, 2, True),                                         # rows above the first key: empty walks
-    (128, 128, 128, False), (128, 128, 129, True),               # backward: 256 and 258 workgroups
+    (128, 128, 128, False), (128, 128, 129, True),               # backward: 256 and 258 lines
+    (256, 256, 32, False), (256, 384, 27, False),                # 128 and 135: four groups and two
+    (1024, 1024, 16, True), (2048, 2048, 8, True),               # causal, 256 in the backward, four groups
+    (256, 2048, 2, True),                                        # cut rows with four groups
     (128, 256, 256, True), (384, 128, 86, False),                # forward: 256 and 258
     (2048, 2048, 16, True), (2048, 2048, 17, True),              # causal, long walks: 512 and 544 in the backward
     (2176, 1920, 9, True),                                       # 153 rows, 135 columns, bottom-right aligned

@@ -67,8 +67,17 @@ __device__ __forceinline__ void store_result(const __attribute__((address_space(
   }
 }
 
-constexpr int kHalf = 64;
-constexpr int kHalfBytes = kHalf * kRowBytes;      // 16 KiB
+// The same for one block of 32 columns.
+__device__ __forceinline__ void store_block(const __attribute__((address_space(4))) BwdSide* p, bf16* out, int64_t os_b, int64_t os_s,
+                                            int64_t os_h, int n_heads, int part, int b, int64_t row0, int h, int64_t seq, int block,
+                                            const f32x16& acc, float mul, uint32_t lds) {
+  if (p->out_f32) {
+    float* base = reinterpret_cast<float*>(out) + part * p->o_part;
+    store_block_f32(base + (((int64_t)b * seq + row0) * n_heads + h) * kHeadDim + 32 * block, (int64_t)n_heads * kHeadDim, acc, mul, lds);
+  } else {
+    store_block_bf16(out + b * os_b + row0 * os_s + h * os_h + 32 * block, os_s, acc, mul, lds);
+  }
+}
 
 // ---- dK/dV ------------------------------------------------------------------------------------
 // Four wavefronts, wave w owns key rows 32w..32w+31 and keeps their K and V rows as B operands; the
@@ -91,12 +100,17 @@ constexpr int kHalfBytes = kHalf * kRowBytes;      // 16 KiB
 // address registers serve the 128-bit reads of both operands and four the transposing ones.
 #define UA_LDS __attribute__((address_space(3)))
 constexpr int kGroupPitch = 1040;                       // bytes between groups of 4 rows
-constexpr int kHalfPitch = (kHalf / 4) * kGroupPitch;   // one half tile
 constexpr int kBlockPitch = 8 * kGroupPitch;            // 32 rows
-constexpr int kStatBytes = 2 * kHalf * 4;               // -lse/scale and -delta of one half tile
-constexpr int kDkdvStat = 4 * kHalfPitch;               // stage s: Q at 2s, dO at 2s + 1; statistics behind them
-constexpr int kDkdvLdsBytes = kDkdvStat + 2 * kStatBytes;
-static_assert(3 * kHalfPitch + kBlockPitch + 6 * kGroupPitch < 65536, "operand offsets fit the instructions' offset field");
+// A group's LDS: stage s holds the first operand's rows at 2s * kPitch and the second's behind them; then the statistics
+// -lse/scale and -delta of either stage.
+template <int kGroups>
+struct Stages : Groups<kGroups> {
+  static constexpr int kPitch = Groups<kGroups>::kRows / 4 * kGroupPitch;
+  static constexpr int kStatBytes = 2 * Groups<kGroups>::kRows * 4;
+  static constexpr int kStat = 4 * kPitch;
+  static constexpr int kBytes = kStat + 2 * kStatBytes;
+};
+static_assert(3 * Stages<1>::kPitch + kBlockPitch + 6 * kGroupPitch < 65536, "operand offsets fit the instructions' offset field");
 
 __device__ __forceinline__ void keep_in_register(uint32_t& x) { asm volatile("" : "+v"(x)); }
 __device__ __forceinline__ bf16x8 lds_abs_b128(uint32_t a) { return *reinterpret_cast<const UA_LDS bf16x8*>(a); }
@@ -146,10 +160,12 @@ __device__ __forceinline__ bf16x8 pair_tr(const PairAddr& ad, int step16, int m)
   return lds_abs_tr_pair(ad.tr[m] + (kOff + 4 * kGroupPitch * step16), ad.tr[m] + (kOff + 4 * kGroupPitch * step16 + 2 * kGroupPitch));
 }
 
-// The walked pair of operands (Q and dO, or K and V): asynchronous copies of half tiles into an LDS stage.
-// 4 copies per wave and operand; copy j fills group 4*j + wave (rows 16*j + 4*wave ..), lane l the 16-byte
+// The walked pair of operands (Q and dO, or K and V): asynchronous copies of a group's rows into an LDS stage.
+// 4 copies per wave and operand; copy j fills group kWaves*j + wave (rows 4*kWaves*j + 4*wave ..), lane l the 16-byte
 // slot l%16 of row l/16 of the group, whose logical chunk is the slot XORed with 4 * (l/16).
+template <int kGroups>
 struct PairStream {
+  using S = Stages<kGroups>;
   const bf16 *x, *y;
   int xs, ys, xoff, yoff;
   uint32_t lds;
@@ -161,40 +177,20 @@ struct PairStream {
     lds = __builtin_amdgcn_readfirstlane(lds_base + wave * kGroupPitch);
   }
   __device__ __forceinline__ void copy_in(int64_t row0, int stage) const {
-    const u32x4 rx = make_rsrc_words(x + row0 * xs, (uint32_t)((kHalf - 1) * xs + kHeadDim) * 2);
-    const u32x4 ry = make_rsrc_words(y + row0 * ys, (uint32_t)((kHalf - 1) * ys + kHeadDim) * 2);
+    const u32x4 rx = make_rsrc_words(x + row0 * xs, (uint32_t)((S::kRows - 1) * xs + kHeadDim) * 2);
+    const u32x4 ry = make_rsrc_words(y + row0 * ys, (uint32_t)((S::kRows - 1) * ys + kHeadDim) * 2);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const uint32_t at = lds + 2 * stage * kHalfPitch + 4 * j * kGroupPitch;
-      dma16_abs(rx, at, xoff, j * 32 * xs);
-      dma16_abs(ry, at + kHalfPitch, yoff, j * 32 * ys);
+      const uint32_t at = lds + 2 * stage * S::kPitch + S::kWaves * j * kGroupPitch;
+      dma16_abs(rx, at, xoff, j * 8 * S::kWaves * xs);
+      dma16_abs(ry, at + S::kPitch, yoff, j * 8 * S::kWaves * ys);
     }
   }
 };
 
-// A wave's accumulators handed to its partner in the other group: 16-byte pieces, 1 KiB per instruction.
-constexpr int kAccBytes = 64 * 64 * 4;
-__device__ __forceinline__ void put_acc(uint32_t lds, const f32x16 (&acc)[4]) {
-  lds += 16 * fresh_lane();
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const f32x16& a = acc[i >> 2];
-    lds_put(lds + 1024 * i, f32x4{a[4 * (i & 3)], a[4 * (i & 3) + 1], a[4 * (i & 3) + 2], a[4 * (i & 3) + 3]});
-  }
-}
-__device__ __forceinline__ void add_acc(uint32_t lds, f32x16 (&acc)[4]) {
-  lds += 16 * fresh_lane();
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const f32x4 x = lds_get<f32x4>(lds + 1024 * i);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i >> 2][4 * (i & 3) + j] += x[j];
-  }
-}
-
-// One block of 32 query rows for this wave's 32 keys.  kOff = LDS offset of the block's Q rows; dO lies one
-// half tile behind.
-template <int kOff, int kStatOff>
+// One block of 32 query rows for this wave's 32 keys.  kOff = LDS offset of the block's Q rows; dO lies kPitch
+// behind, -delta kStatBytes / 2 behind -lse/scale.
+template <int kOff, int kPitch, int kStatOff, int kStatBytes>
 __device__ __forceinline__ void dkdv_block(const PairAddr& ad, uint32_t stat, const bf16x8 (&kf)[8], const bf16x8 (&vf)[8], f32x16 (&dk)[4],
                                            f32x16 (&dv)[4], float scale_log2, int hi, int key_b, bool mask) {
   f32x16 s, dp;
@@ -202,7 +198,7 @@ __device__ __forceinline__ void dkdv_block(const PairAddr& ad, uint32_t stat, co
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
     const f32x4 a = *reinterpret_cast<const UA_LDS f32x4*>(stat + (kStatOff + 32 * g));
-    const f32x4 c = *reinterpret_cast<const UA_LDS f32x4*>(stat + (kStatOff + kHalf * 4 + 32 * g));
+    const f32x4 c = *reinterpret_cast<const UA_LDS f32x4*>(stat + (kStatOff + kStatBytes / 2 + 32 * g));
 #pragma unroll
     for (int j = 0; j < 4; ++j) { s[4 * g + j] = a[j]; dp[4 * g + j] = c[j]; }
   }
@@ -210,7 +206,7 @@ __device__ __forceinline__ void dkdv_block(const PairAddr& ad, uint32_t stat, co
     // 16 row fragments, Q and dO alternating, fetched kAhead reads ahead of their MFMA
     constexpr int kAhead = 3;
     bf16x8 fr[16];
-    auto rd = [&](int i) { return (i & 1) ? pair_nat<kOff + kHalfPitch>(ad, i >> 1) : pair_nat<kOff>(ad, i >> 1); };
+    auto rd = [&](int i) { return (i & 1) ? pair_nat<kOff + kPitch>(ad, i >> 1) : pair_nat<kOff>(ad, i >> 1); };
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) fr[i] = rd(i);
     __builtin_amdgcn_sched_group_barrier(0x100, 8 + kAhead, 0);
@@ -225,7 +221,7 @@ __device__ __forceinline__ void dkdv_block(const PairAddr& ad, uint32_t stat, co
   }
   // transposed fragments i: dO for i even (dV), Q for i odd (dK); d-block (i/2)%4, 16-row step i/8
   auto rd_tr = [&](int i) {
-    return (i & 1) ? pair_tr<kOff>(ad, i >> 3, (i >> 1) & 3) : pair_tr<kOff + kHalfPitch>(ad, i >> 3, (i >> 1) & 3);
+    return (i & 1) ? pair_tr<kOff>(ad, i >> 3, (i >> 1) & 3) : pair_tr<kOff + kPitch>(ad, i >> 3, (i >> 1) & 3);
   };
   constexpr int kTAhead = 2;
   bf16x8 fr[16];
@@ -255,17 +251,21 @@ __device__ __forceinline__ void dkdv_block(const PairAddr& ad, uint32_t stat, co
 }
 
 // kGroups = 2 (here and for dQ): two groups of four wavefronts share the workgroup's line, one takes the first half of every
-// tile, the other the second, each through stages of its own; the results are added through LDS.  Where the launch
+// tile, the other the second, each through stages of its own; the results are added through LDS.  kGroups = 4: four groups
+// of two wavefronts share half a tile's rows, each takes a block of 32 of every tile.  Where the launch
 // gives a CU one workgroup at most, one wave per SIMD would leave the matrix pipe idle between its dependent steps (2.2 us
 // per half tile of dK/dV, 0.9 of them MFMAs); the second group fills the CU without partial results in memory.
 template <int kGroups>
 __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block, int block) {
-  const int tid = threadIdx.x & 255, lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
+  using S = Stages<kGroups>;
+  const int tid = threadIdx.x % (64 * S::kWaves), lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int group = kGroups == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
-  const uint32_t lds_base = lds_block + group * kDkdvLdsBytes;
+  const int group = kGroups == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * S::kWaves));
+  const uint32_t lds_base = lds_block + group * S::kBytes;
   int pos, bh;
-  map_block(block, p.batch * p.n_heads, p.heads_per_xcd, p.n_ktiles * p.cols.n_parts, pos, bh);
+  map_block(block, p.batch * p.n_heads, p.heads_per_xcd, p.n_ktiles * p.cols.n_parts * S::kLines, pos, bh);
+  const int sub = pos % S::kLines;         // which half of the tile's keys
+  pos /= S::kLines;
   const int b = bh / p.n_heads, h = bh % p.n_heads;
   int kt, e0, e1, diag = -1, part = 0;
   if (p.dense) {
@@ -282,10 +282,10 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block
     e1 = min(max(sload(p.cols.ptr, kt + 1), e0), p.nnz);
   }
   const int64_t seq_q = (int64_t)p.n_qtiles * kTile;
-  const PairStream in(p.q + b * p.qs.b + h * p.qs.h, (int)p.qs.s, p.dout + b * p.ds.b + h * p.ds.h, (int)p.ds.s, lds_base, wave, lane);
+  const PairStream<kGroups> in(p.q + b * p.qs.b + h * p.qs.h, (int)p.qs.s, p.dout + b * p.ds.b + h * p.ds.h, (int)p.ds.s, lds_base, wave, lane);
   const int n_half = (kGroups == 1 ? 2 : 1) * (e1 - e0);
-  // half tile i = half (i & 1) of list entry e0 + i / 2, with two groups half `group` of entry e0 + i.  The
-  // list entry (query tile, causal flag) of half tile i+1 is fetched one step before it is needed, so that
+  // step i = half (i & 1) of list entry e0 + i / 2, with more groups half or quarter `group` of entry e0 + i.  The
+  // list entry (query tile, causal flag) of step i+1 is fetched one step before it is needed, so that
   // no step starts by waiting for a scalar load.
   auto half_of = [&](int i) { return kGroups == 1 ? i & 1 : group; };
   auto entry = [&](int i) {           // query tile | causal flag << 30
@@ -294,40 +294,40 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block
     if (p.dense) return e | ((int)(e == diag) << 30);      // the entry is the query tile itself
     return min(max(sload(p.cols.idx, e), 0), p.n_qtiles - 1) | (sload(p.cols.flag, e) << 30);
   };
-  // rows' statistics, staged in the form the accumulators start from: threads 0..63 carry
-  // -lse/softmax_scale (lse = -inf, a row without keys, stays -inf so that P = 0), threads
-  // 64..127 carry -delta
+  // rows' statistics, staged in the form the accumulators start from: threads 0..kRows-1 carry
+  // -lse/softmax_scale (lse = -inf, a row without keys, stays -inf so that P = 0), the next
+  // kRows carry -delta
   // (the raw value is only touched when it is stored to LDS at the end of a step: no wait for
   // the global load may land between the copies' issue and the step's work)
   const float neg_inv_scale = -1.f / p.scale;
-  const float* stat_src = (tid < kHalf ? p.lse : p.delta) + ((int64_t)b * p.n_heads + h) * seq_q + (tid & (kHalf - 1));
+  const float* stat_src = (tid < S::kRows ? p.lse : p.delta) + ((int64_t)b * p.n_heads + h) * seq_q + (tid & (S::kRows - 1));
   auto load_stat = [&](int i, int qt) {
     float x = 0.f;
-    if (tid < 2 * kHalf) x = stat_src[qt * kTile + half_of(i) * kHalf];
+    if (tid < 2 * S::kRows) x = stat_src[qt * kTile + half_of(i) * S::kRows];
     return x;
   };
   auto put_stat = [&](int stage, float x) {
-    if (tid < 2 * kHalf) {
-      x = tid < kHalf ? ((x == -INFINITY) ? -INFINITY : x * neg_inv_scale) : -x;
-      *reinterpret_cast<UA_LDS float*>(lds_base + kDkdvStat + stage * kStatBytes + tid * 4) = x;
+    if (tid < 2 * S::kRows) {
+      x = tid < S::kRows ? ((x == -INFINITY) ? -INFINITY : x * neg_inv_scale) : -x;
+      *reinterpret_cast<UA_LDS float*>(lds_base + S::kStat + stage * S::kStatBytes + tid * 4) = x;
     }
   };
   int ent = entry(0), ent_next = entry(1);
   float st0 = 0.f;
   if (n_half > 0) {
-    in.copy_in((int64_t)(ent & 0x3fffffff) * kTile + half_of(0) * kHalf, 0);
+    in.copy_in((int64_t)(ent & 0x3fffffff) * kTile + half_of(0) * S::kRows, 0);
     st0 = load_stat(0, ent & 0x3fffffff);
   }
 
-  // K and V rows as B operands: lane holds key row 32*wave + lane%32, d = 16*ks + 8*hi .. +7
+  // K and V rows as B operands: lane holds key row 32*k_block + lane%32, d = 16*ks + 8*hi .. +7
   // (through the stage that the first step fills)
-  const int krow0 = kt * kTile + wave * 32;
+  const int k_block = S::kWaves * sub + wave, krow0 = kt * kTile + k_block * 32;
   bf16x8 kf[8], vf[8];
   {
     u32x4 kraw[8], vraw[8];
     load_rows(kraw, p.k + b * p.ks.b + (int64_t)krow0 * p.ks.s + h * p.ks.h, p.ks.s);
     load_rows(vraw, p.v + b * p.vs.b + (int64_t)krow0 * p.vs.s + h * p.vs.h, p.vs.s);
-    const uint32_t turn = lds_base + 2 * kHalfPitch + wave * kWaveRowsBytes;
+    const uint32_t turn = lds_base + 2 * S::kPitch + wave * kWaveRowsBytes;
     rows_to_frags(kf, kraw, turn);
     rows_to_frags(vf, vraw, turn);
   }
@@ -336,7 +336,7 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block
   for (int i = 0; i < 4; ++i) { dk[i] = f32x16{0}; dv[i] = f32x16{0}; }
 
   const PairAddr ad(lds_base, lane);
-  uint32_t stat_addr = lds_base + kDkdvStat + 16 * hi;     // this lane half's 4 consecutive row statistics
+  uint32_t stat_addr = lds_base + S::kStat + 16 * hi;     // this lane half's 4 consecutive row statistics
   keep_in_register(stat_addr);
   if (n_half > 0) put_stat(0, st0);
   // The compiler does not see the copies that the walk has in flight.  Were the K and V rows still
@@ -359,15 +359,18 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block
     float stat = 0.f;
     if (more) {
       stat = load_stat(i + 1, cur_next & 0x3fffffff);
-      in.copy_in((int64_t)(cur_next & 0x3fffffff) * kTile + half_of(i + 1) * kHalf, kStage ^ 1);
+      in.copy_in((int64_t)(cur_next & 0x3fffffff) * kTile + half_of(i + 1) * S::kRows, kStage ^ 1);
     }
-    // causal tile: query block nb sees none of the wave's keys when nb < wave, some when nb == wave
-    const int nb = 2 * half_of(i);
-    if (!causal || nb >= wave)
-      dkdv_block<2 * kStage * kHalfPitch, kStage * kStatBytes>(ad, stat_addr, kf, vf, dk, dv, p.scale_log2, hi, l32, causal && nb == wave);
-    if (!causal || nb + 1 >= wave)
-      dkdv_block<2 * kStage * kHalfPitch + kBlockPitch, kStage * kStatBytes + 128>(ad, stat_addr, kf, vf, dk, dv, p.scale_log2, hi, l32,
-                                                                                  causal && nb + 1 == wave);
+    // causal tile: query block nb sees none of the wave's keys when nb < k_block, some when nb == k_block
+    constexpr int kBlocks = S::kRows / 32, kOff = 2 * kStage * S::kPitch, kStatOff = kStage * S::kStatBytes;
+    const int nb = kBlocks * half_of(i);
+    if (!causal || nb >= k_block)
+      dkdv_block<kOff, S::kPitch, kStatOff, S::kStatBytes>(ad, stat_addr, kf, vf, dk, dv, p.scale_log2, hi, l32, causal && nb == k_block);
+    if constexpr (kBlocks == 2) {
+      if (!causal || nb + 1 >= k_block)
+        dkdv_block<kOff + kBlockPitch, S::kPitch, kStatOff + 128, S::kStatBytes>(ad, stat_addr, kf, vf, dk, dv, p.scale_log2, hi, l32,
+                                                                                 causal && nb + 1 == k_block);
+    }
     if (more) put_stat(kStage ^ 1, stat);
     wait_vmem_all();
     __syncthreads();     // the next stage has landed and everyone is done with this one
@@ -376,22 +379,43 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block
     step(i, std::integral_constant<int, 0>{});
     step(i + 1, std::integral_constant<int, 1>{});
   }
-  uint32_t turn_out = lds_base + wave * kWaveRowsBytes;              // everyone is done with the stages
+  // everyone is done with the stages
+  auto area = [&](int g) { return lds_block + (wave * kGroups + g) * kAccBytes; };       // of group g of this wave's rows
   if constexpr (kGroups == 2) {
     // the second group finishes dV, the first dK
-    const uint32_t mine = lds_block + (4 * group + wave) * kAccBytes, other = lds_block + (4 * (group ^ 1) + wave) * kAccBytes;
-    if (group) put_acc(mine, dk); else put_acc(mine, dv);
+    if (group) put_acc(area(1), dk); else put_acc(area(0), dv);
     __syncthreads();
-    if (group) add_acc(other, dv); else add_acc(other, dk);
-    turn_out = other;
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb)
+      if (group) add_block(area(0), mb, dv[mb]); else add_block(area(1), mb, dk[mb]);
+  }
+  f32x16 dk_sum{0}, dv_sum{0};             // four groups: each finishes a block of 32 columns of both
+  if constexpr (kGroups == 4) {
+    put_acc(area(group), dk);
+    __syncthreads();
+#pragma unroll
+    for (int g = 0; g < 4; ++g) add_block(area(g), group, dk_sum);
+    __syncthreads();
+    put_acc(area(group), dv);
+    __syncthreads();
+#pragma unroll
+    for (int g = 0; g < 4; ++g) add_block(area(g), group, dv_sum);
   }
   const ParamsLate pl = params_late();
   const int64_t seq_k = (int64_t)pl->n_ktiles * kTile;
-  const int64_t krow_out = (int64_t)kt * kTile + wave * 32;
-  if (kGroups == 1 || group == 0)
-    store_result(&pl->cols, pl->cols.out0, pl->cols.o0s.b, pl->cols.o0s.s, pl->cols.o0s.h, pl->n_heads, part, b, krow_out, h, seq_k, dk, pl->scale, turn_out);
-  if (kGroups == 1 || group == 1)
-    store_result(&pl->cols, pl->cols.out1, pl->cols.o1s.b, pl->cols.o1s.s, pl->cols.o1s.h, pl->n_heads, part, b, krow_out, h, seq_k, dv, 1.f, turn_out);
+  const int64_t krow_out = (int64_t)kt * kTile + k_block * 32;
+  if constexpr (kGroups == 4) {
+    // (this wave alone reads the block of its own area that it turns through)
+    const uint32_t turn = area(group) + 4096 * group;
+    store_block(&pl->cols, pl->cols.out0, pl->cols.o0s.b, pl->cols.o0s.s, pl->cols.o0s.h, pl->n_heads, part, b, krow_out, h, seq_k, group, dk_sum, pl->scale, turn);
+    store_block(&pl->cols, pl->cols.out1, pl->cols.o1s.b, pl->cols.o1s.s, pl->cols.o1s.h, pl->n_heads, part, b, krow_out, h, seq_k, group, dv_sum, 1.f, turn);
+  } else {
+    const uint32_t turn = kGroups == 1 ? lds_base + wave * kWaveRowsBytes : area(group ^ 1);
+    if (kGroups == 1 || group == 0)
+      store_result(&pl->cols, pl->cols.out0, pl->cols.o0s.b, pl->cols.o0s.s, pl->cols.o0s.h, pl->n_heads, part, b, krow_out, h, seq_k, dk, pl->scale, turn);
+    if (kGroups == 1 || group == 1)
+      store_result(&pl->cols, pl->cols.out1, pl->cols.o1s.b, pl->cols.o1s.s, pl->cols.o1s.h, pl->n_heads, part, b, krow_out, h, seq_k, dv, 1.f, turn);
+  }
 }
 
 // ---- dQ -----------------------------------------------------------------------------------------
@@ -399,7 +423,7 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block
 // streamed like dK/dV's operands.  Per block of 32 keys: S^T = K Q^T and dP'^T = V dO^T - delta (16 MFMAs),
 // dS^T in the lanes, dQ^T += K^T dS^T (8 MFMAs).  A lane holds one query column, so -delta is one value per
 // lane: it is kept in 16 registers that dP's first MFMA takes as its addend, which spares 16 moves per block.
-template <int kOff>
+template <int kOff, int kPitch>
 __device__ __forceinline__ void dq_block(const PairAddr& ad, const bf16x8 (&qf)[8], const bf16x8 (&dof)[8], const f32x16& neg_delta,
                                          f32x16 (&dq)[4], float scale_log2, float lse2, int hi, int q_b, bool mask) {
   f32x16 s, dp;
@@ -407,7 +431,7 @@ __device__ __forceinline__ void dq_block(const PairAddr& ad, const bf16x8 (&qf)[
     // 16 row fragments, K and V alternating, fetched kAhead reads ahead of their MFMA
     constexpr int kAhead = 4;
     bf16x8 fr[16];
-    auto rd = [&](int i) { return (i & 1) ? pair_nat<kOff + kHalfPitch>(ad, i >> 1) : pair_nat<kOff>(ad, i >> 1); };
+    auto rd = [&](int i) { return (i & 1) ? pair_nat<kOff + kPitch>(ad, i >> 1) : pair_nat<kOff>(ad, i >> 1); };
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) fr[i] = rd(i);
     __builtin_amdgcn_sched_group_barrier(0x100, kAhead, 0);
@@ -449,12 +473,15 @@ __device__ __forceinline__ void dq_block(const PairAddr& ad, const bf16x8 (&qf)[
 
 template <int kGroups>
 __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_block, int block) {
-  const int tid = threadIdx.x & 255, lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
+  using S = Stages<kGroups>;
+  const int tid = threadIdx.x % (64 * S::kWaves), lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int group = kGroups == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
-  const uint32_t lds_base = lds_block + group * kDkdvLdsBytes;
+  const int group = kGroups == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * S::kWaves));
+  const uint32_t lds_base = lds_block + group * S::kBytes;
   int pos, bh;
-  map_block(block, p.batch * p.n_heads, p.heads_per_xcd, p.n_qtiles * p.rows.n_parts, pos, bh);
+  map_block(block, p.batch * p.n_heads, p.heads_per_xcd, p.n_qtiles * p.rows.n_parts * S::kLines, pos, bh);
+  const int sub = pos % S::kLines;         // which half of the tile's queries
+  pos /= S::kLines;
   const int b = bh / p.n_heads, h = bh % p.n_heads;
   const int64_t seq_q = (int64_t)p.n_qtiles * kTile;
   int qt, e0, e1, diag = -1, part = 0;
@@ -471,22 +498,22 @@ __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_block, 
     e0 = min(max(sload(p.rows.ptr, qt), 0), p.nnz);
     e1 = min(max(sload(p.rows.ptr, qt + 1), e0), p.nnz);
   }
-  const PairStream in(p.k + b * p.ks.b + h * p.ks.h, (int)p.ks.s, p.v + b * p.vs.b + h * p.vs.h, (int)p.vs.s, lds_base, wave, lane);
+  const PairStream<kGroups> in(p.k + b * p.ks.b + h * p.ks.h, (int)p.ks.s, p.v + b * p.vs.b + h * p.vs.h, (int)p.vs.s, lds_base, wave, lane);
   auto ktile = [&](int e) { return p.dense ? e : min(max(sload(p.rows.idx, e), 0), p.n_ktiles - 1); };
   auto is_causal = [&](int e) { return p.dense ? (int)(e == diag) : sload(p.rows.flag, e); };
 
   const int n_steps = (kGroups == 1 ? 2 : 1) * (e1 - e0);          // half tiles, as in dK/dV's walk
   int kt = e0 < e1 ? ktile(e0) : 0;
-  if (e0 < e1) in.copy_in((int64_t)kt * kTile + group * kHalf, 0);
+  if (e0 < e1) in.copy_in((int64_t)kt * kTile + group * S::kRows, 0);
 
-  const int qrow0 = qt * kTile + wave * 32, qrow = qrow0 + l32;
+  const int q_block = S::kWaves * sub + wave, qrow0 = qt * kTile + q_block * 32, qrow = qrow0 + l32;
   bf16x8 qf[8], dof[8];
   u32x4 qraw[8], doraw[8];
   load_rows(qraw, p.q + b * p.qs.b + (int64_t)qrow0 * p.qs.s + h * p.qs.h, p.qs.s);
   load_rows(doraw, p.dout + b * p.ds.b + (int64_t)qrow0 * p.ds.s + h * p.ds.h, p.ds.s);
   const float lse_raw = p.lse[((int64_t)b * p.n_heads + h) * seq_q + qrow];
   const float neg_delta = -p.delta[((int64_t)b * p.n_heads + h) * seq_q + qrow];
-  const uint32_t turn = lds_base + 2 * kHalfPitch + wave * kWaveRowsBytes;      // in the stage that the first step fills
+  const uint32_t turn = lds_base + 2 * S::kPitch + wave * kWaveRowsBytes;      // in the stage that the first step fills
   rows_to_frags(qf, qraw, turn);
   rows_to_frags(dof, doraw, turn);
   const float lse2 = (lse_raw == -INFINITY) ? INFINITY : lse_raw * kLog2e;
@@ -516,49 +543,65 @@ __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_block, 
     const int kt_next = kFirst ? kt : (kSecond ? kt_ahead : (more ? ktile(e + 1) : kt));
     wait_vmem_all();
     __syncthreads();            // this stage has landed; everyone is done with the other one
-    if (more) in.copy_in((int64_t)kt_next * kTile + (kGroups == 1 ? kStage ^ 1 : group) * kHalf, kStage ^ 1);
-    // causal tile: key block nb is hidden from the wave's queries when nb > wave, in part when nb == wave
-    const int nb = 2 * half;
-    if (!causal || wave >= nb)
-      dq_block<2 * kStage * kHalfPitch>(ad, qf, dof, nd, dq, p.scale_log2, lse2, hi, l32, causal && wave == nb);
-    if (!causal || wave >= nb + 1)
-      dq_block<2 * kStage * kHalfPitch + kBlockPitch>(ad, qf, dof, nd, dq, p.scale_log2, lse2, hi, l32, causal && wave == nb + 1);
+    if (more) in.copy_in((int64_t)kt_next * kTile + (kGroups == 1 ? kStage ^ 1 : group) * S::kRows, kStage ^ 1);
+    // causal tile: key block nb is hidden from the wave's queries when nb > q_block, in part when nb == q_block
+    constexpr int kBlocks = S::kRows / 32, kOff = 2 * kStage * S::kPitch;
+    const int nb = kBlocks * half;
+    if (!causal || q_block >= nb)
+      dq_block<kOff, S::kPitch>(ad, qf, dof, nd, dq, p.scale_log2, lse2, hi, l32, causal && q_block == nb);
+    if constexpr (kBlocks == 2) {
+      if (!causal || q_block >= nb + 1)
+        dq_block<kOff + kBlockPitch, S::kPitch>(ad, qf, dof, nd, dq, p.scale_log2, lse2, hi, l32, causal && q_block == nb + 1);
+    }
     kt = kt_next;
   };
   for (int i = 0; i < n_steps; i += 2) {
     step(i, std::integral_constant<int, 0>{});
     step(i + 1, std::integral_constant<int, 1>{});
   }
-  uint32_t turn_out = lds_base + wave * kWaveRowsBytes;              // stage 0: everyone left it before the last step
-  if constexpr (kGroups == 2) {
-    __syncthreads();
-    turn_out = lds_block + wave * kAccBytes;
-    if (group) put_acc(turn_out, dq);
-    __syncthreads();
-    if (group) return;
-    add_acc(turn_out, dq);
-  }
   const ParamsLate pl = params_late();
-  const int64_t qrow_out = (int64_t)qt * kTile + wave * 32;
-  store_result(&pl->rows, pl->rows.out0, pl->rows.o0s.b, pl->rows.o0s.s, pl->rows.o0s.h, pl->n_heads, part, b, qrow_out, h,
-               (int64_t)pl->n_qtiles * kTile, dq, pl->scale, turn_out);
+  const int64_t qrow_out = (int64_t)qt * kTile + q_block * 32, seq_out = (int64_t)pl->n_qtiles * kTile;
+  auto area = [&](int g) { return lds_block + (wave * kGroups + g) * kAccBytes; };       // of group g of this wave's rows
+  if constexpr (kGroups == 4) {
+    __syncthreads();
+    put_acc(area(group), dq);
+    __syncthreads();
+    f32x16 sum{0};
+#pragma unroll
+    for (int g = 0; g < 4; ++g) add_block(area(g), group, sum);
+    store_block(&pl->rows, pl->rows.out0, pl->rows.o0s.b, pl->rows.o0s.s, pl->rows.o0s.h, pl->n_heads, part, b, qrow_out, h, seq_out, group, sum,
+                pl->scale, area(group) + 4096 * group);
+  } else {
+    uint32_t turn = lds_base + wave * kWaveRowsBytes;                // stage 0: everyone left it before the last step
+    if constexpr (kGroups == 2) {
+      __syncthreads();
+      turn = area(1);
+      if (group) put_acc(turn, dq);
+      __syncthreads();
+      if (group) return;
+#pragma unroll
+      for (int mb = 0; mb < 4; ++mb) add_block(turn, mb, dq[mb]);
+    }
+    store_result(&pl->rows, pl->rows.out0, pl->rows.o0s.b, pl->rows.o0s.s, pl->rows.o0s.h, pl->n_heads, part, b, qrow_out, h, seq_out, dq, pl->scale,
+                 turn);
+  }
 }
 
 // ---- kernels ------------------------------------------------------------------------------------
 template <int kGroups>
-__global__ __launch_bounds__(256 * kGroups, 2) void dkdv_kernel(const BwdParams p) {
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[kGroups * kDkdvLdsBytes];
+__global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void dkdv_kernel(const BwdParams p) {
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[kGroups * Stages<kGroups>::kBytes];
   dkdv_walk<kGroups>(p, (uint32_t)(uintptr_t)(UA_LDS unsigned char*)smem, blockIdx.x);
 }
 template <int kGroups>
-__global__ __launch_bounds__(256 * kGroups, 2) void dq_kernel(const BwdParams p) {
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[kGroups * kDkdvLdsBytes];
+__global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void dq_kernel(const BwdParams p) {
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[kGroups * Stages<kGroups>::kBytes];
   dq_walk<kGroups>(p, (uint32_t)(uintptr_t)(UA_LDS unsigned char*)smem, blockIdx.x);
 }
 // Both sides in one launch.
 template <int kGroups>
-__global__ __launch_bounds__(256 * kGroups, 2) void bwd_kernel(const BwdParams p) {
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[kGroups * kDkdvLdsBytes];
+__global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void bwd_kernel(const BwdParams p) {
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[kGroups * Stages<kGroups>::kBytes];
   const uint32_t lds_base = (uint32_t)(uintptr_t)(UA_LDS unsigned char*)smem;
   if ((int)blockIdx.x < p.n_col_blocks) dkdv_walk<kGroups>(p, lds_base, blockIdx.x);
   else                                  dq_walk<kGroups>(p, lds_base, blockIdx.x - p.n_col_blocks);
@@ -609,30 +652,38 @@ static int fill_side(BwdSide& s, int nnz, const int32_t* ptr, const int32_t* idx
 static int launched() { return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH; }
 static unsigned col_blocks(const BwdParams& p) { return (unsigned)(p.batch * p.n_heads * p.n_ktiles * p.cols.n_parts); }
 static unsigned row_blocks(const BwdParams& p) { return (unsigned)(p.batch * p.n_heads * p.n_qtiles * p.rows.n_parts); }
-// Two groups per workgroup where both sides together give a CU one workgroup at most and the walks are worth the handing
-// over at their end, from three tiles on; a launch of one side alone decides alike, so that its results are the
-// same bit for bit.  An uncut causal rectangle whose walks average 8 tiles is
-// better off with them up to two workgroups per CU: run in turn they balance its lines (8 heads of 4096: 135 us
-// resident at once, 118 in turn; shorter walks lose more to the second start: 32 heads of 1024 41, 50).
-static bool bwd_pairs(int64_t groups, int64_t both_walks, int n_parts, bool dense_causal, int n_qtiles, int n_ktiles) {
-  return both_walks >= 6 && (groups <= kCus || (groups <= 2 * kCus && dense_causal && n_parts == 2 && n_qtiles >= 16 && n_ktiles >= 16));
+// Groups per workgroup for n lines of 128 rows on both sides together (parts counted), as in the forward: four while half
+// lines leave a CU one workgroup at most (8 heads of 1024: 34 us with one group, 31 with two, 24 with four), two up to one
+// per CU and from three tiles a walk on.  Of an uncut causal rectangle, whose lines differ in length, four up to 256
+// lines that average four tiles (8 heads of 2048: 54 us with two, 44 with four) and two up to 512 that average eight (8 of
+// 4096: 140 us with one, 132 with two; 32 of 1024: 42, 54).  A launch of one side alone decides by both sides too,
+// so that its results are the same bit for bit.
+static int bwd_groups(int64_t n, int64_t both_walks, int n_parts, bool dense_causal, int n_qtiles, int n_ktiles) {
+  const bool uneven = dense_causal && n_parts == 2;
+  if (both_walks >= 3 && (2 * n <= kCus || (uneven && n <= kCus && both_walks >= 16))) return 4;
+  if (both_walks < 6) return 1;
+  return n <= kCus || (uneven && n <= 2 * kCus && n_qtiles >= 16 && n_ktiles >= 16) ? 2 : 1;
 }
 static unsigned both_blocks(const BwdParams& p) { return col_blocks(p) + row_blocks(p); }
-static bool pairs(const BwdParams& p) {
+// Launches kernel<groups> for n workgroups of one line each.
+#define UA_LAUNCH_GROUPS(KERNEL, N, P, ST)                                                          \
+  switch (groups_of(P)) {                                                                           \
+    case 4: hipLaunchKernelGGL(KERNEL<4>, dim3(2 * (N)), dim3(512), 0, ST, P); break;               \
+    case 2: hipLaunchKernelGGL(KERNEL<2>, dim3(N), dim3(512), 0, ST, P); break;                     \
+    default: hipLaunchKernelGGL(KERNEL<1>, dim3(N), dim3(256), 0, ST, P);                           \
+  }
+static int groups_of(const BwdParams& p) {
   const int64_t walks = p.dense ? p.cols.part_len + p.rows.part_len : p.nnz / p.n_qtiles + p.nnz / p.n_ktiles;
-  return bwd_pairs(both_blocks(p), walks, p.cols.n_parts + p.rows.n_parts, p.dense_causal, p.n_qtiles, p.n_ktiles);
+  return bwd_groups(both_blocks(p), walks, p.cols.n_parts + p.rows.n_parts, p.dense_causal, p.n_qtiles, p.n_ktiles);
 }
 static int launch_bwd(BwdParams& p, hipStream_t st) {
-  p.n_col_blocks = (int)col_blocks(p);
-  if (pairs(p)) {
-    hipLaunchKernelGGL(bwd_kernel<2>, dim3(both_blocks(p)), dim3(512), 0, st, p);
-  } else {
-    // Up to two workgroups per CU the whole launch is resident at once, and the second 256 join the first in launch
-    // order.  Rows come longest first; of a causal rectangle the columns then come shortest first, so that the long
-    // ones of one side share a CU with the short ones of the other (32 heads of 1024: 43.6 -> 41.5 us).
-    p.cols_shortest_first = p.dense_causal && both_blocks(p) <= 2 * kCus;
-    hipLaunchKernelGGL(bwd_kernel<1>, dim3(both_blocks(p)), dim3(256), 0, st, p);
-  }
+  const int groups = groups_of(p);
+  p.n_col_blocks = (int)col_blocks(p) * (groups == 4 ? 2 : 1);
+  // Up to two workgroups per CU the whole launch is resident at once, and the second 256 join the first in launch
+  // order.  Rows come longest first; of a causal rectangle the columns then come shortest first, so that the long
+  // ones of one side share a CU with the short ones of the other (32 heads of 1024: 43.6 -> 41.5 us).
+  p.cols_shortest_first = groups == 1 && p.dense_causal && both_blocks(p) <= 2 * kCus;
+  UA_LAUNCH_GROUPS(bwd_kernel, both_blocks(p), p, st)
   return launched();
 }
 
@@ -640,11 +691,11 @@ static int launch_bwd(BwdParams& p, hipStream_t st) {
 // small rectangle enough workgroups for the device and costs the partials' way through memory and a
 // second launch; which wins is decided by an estimate of the launch's time in microseconds, fitted to 47 shapes of 1
 // to 32 heads and 128 to 8192 tokens (the cut it takes is within 4 % of the best one on each):
-//  - 6.7 to start, load the resident rows, store the results and end, 8.4 with two groups per workgroup;
-//  - a tile takes 2.6 (columns) or 1.7 (rows) with two groups, else 3.2 and 2.2, and 4.4 and 4.9 where two workgroups
-//    share the CU;
-//  - the sum takes 2.7, and the partials 1 per 3.7 MB; a cut has to win by 6 %.
-// 512 x 512, 32 heads: 33 us cut in two, 22 uncut; 1024 x 4096, one head: 67 uncut, 25 cut in 4 and 8.
+//  - 6.5 to start, load the resident rows, store the results and end, 9.8 with two groups per workgroup, 7.1 with four;
+//  - a tile takes 1.9 (columns) or 1 (rows) with four groups, 2.6 and 1.7 with two, else 3.5 and 2.1, and 4.9 and 5.5
+//    where two workgroups share the CU;
+//  - the sum takes 2.4, and the partials 1 per 3.7 MB; a cut has to win by 6 %.
+// 1024 x 4096, one head: 42 us uncut, 24 cut in 2 and 5.
 struct BwdCut { int cols, rows; };
 static BwdCut bwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int max_cols, int max_rows) {
   if (max_cols <= 1 && max_rows <= 1) return {1, 1};
@@ -657,15 +708,20 @@ static BwdCut bwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int 
     for (int pr : kParts) {
       if (pr > max_rows) break;
       const float groups = (wk * pc + wq * pr) * density;
-      float us = 8.4f, tc = 2.6f, tr = 1.7f;
-      if (!bwd_pairs(nbh * ((int64_t)n_ktiles * pc + (int64_t)n_qtiles * pr), (n_qtiles + pc - 1) / pc + (n_ktiles + pr - 1) / pr, pc + pr, causal, n_qtiles, n_ktiles)) {
-        const float shared = fminf(fmaxf((groups - kCus) / kCus, 0.f), 1.f);       // share of the workgroups with a neighbour
-        us = 6.7f; tc = 3.2f + 1.2f * shared; tr = 2.2f + 2.7f * shared;
+      float us, tc, tr;
+      switch (bwd_groups(nbh * ((int64_t)n_ktiles * pc + (int64_t)n_qtiles * pr), (n_qtiles + pc - 1) / pc + (n_ktiles + pr - 1) / pr, pc + pr, causal,
+                         n_qtiles, n_ktiles)) {
+        case 4: us = 7.1f; tc = 1.86f; tr = 0.96f; break;
+        case 2: us = 9.8f; tc = 2.6f; tr = 1.7f; break;
+        default: {
+          const float shared = fminf(fmaxf((groups - kCus) / kCus, 0.f), 1.f);       // share of the workgroups with a neighbour
+          us = 6.5f; tc = 3.5f + 1.4f * shared; tr = 2.1f + 3.4f * shared;
+        }
       }
       const float longest = fmaxf((float)((n_qtiles + pc - 1) / pc) * tc, (float)((n_ktiles + pr - 1) / pr) * tr);
-      const float all = density * wk * n_qtiles * (4.4f + 4.9f) / (2 * kCus);
+      const float all = density * wk * n_qtiles * (4.9f + 5.5f) / (2 * kCus);
       us += fmaxf(longest, all);
-      if (pc > 1 || pr > 1) us = (us + 2.7f) * 1.06f;
+      if (pc > 1 || pr > 1) us = (us + 2.4f) * 1.06f;
       if (pc > 1) us += 2.f * pc * wk * (kTile * kHeadDim * 4) / 3.7e6f;
       if (pr > 1) us += pr * wq * (kTile * kHeadDim * 4) / 3.7e6f;
       if (us < best_us) { best_us = us; best = {pc, pr}; }
@@ -691,8 +747,7 @@ extern "C" int ua_bsa_bwd_dkdv(const void* q, const void* k, const void* v, cons
   if (!dv_strides) return UA_ERR_NULL;
   if (int rc = fill_side(p.cols, nnz, col_ptr, row_idx, cflag, k_order, dk, dk_strides, dv, dv_strides, false)) return rc;
   if (int rc = check_device()) return rc;
-  if (pairs(p)) hipLaunchKernelGGL(dkdv_kernel<2>, dim3(col_blocks(p)), dim3(512), 0, (hipStream_t)stream, p);
-  else          hipLaunchKernelGGL(dkdv_kernel<1>, dim3(col_blocks(p)), dim3(256), 0, (hipStream_t)stream, p);
+  UA_LAUNCH_GROUPS(dkdv_kernel, col_blocks(p), p, (hipStream_t)stream)
   return launched();
 }
 
@@ -710,8 +765,7 @@ extern "C" int ua_bsa_bwd_dq(const void* q, const void* k, const void* v, const 
                            v_strides, do_strides, softmax_scale)) return rc;
   if (int rc = fill_side(p.rows, nnz, row_ptr, col_idx, flag, q_order, dq, dq_strides, nullptr, nullptr, false)) return rc;
   if (int rc = check_device()) return rc;
-  if (pairs(p)) hipLaunchKernelGGL(dq_kernel<2>, dim3(row_blocks(p)), dim3(512), 0, (hipStream_t)stream, p);
-  else          hipLaunchKernelGGL(dq_kernel<1>, dim3(row_blocks(p)), dim3(256), 0, (hipStream_t)stream, p);
+  UA_LAUNCH_GROUPS(dq_kernel, row_blocks(p), p, (hipStream_t)stream)
   return launched();
 }
 

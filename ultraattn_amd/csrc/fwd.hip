@@ -31,8 +31,6 @@ struct FwdParams {
   int64_t o_part, lse_part;
 };
 
-constexpr int kHalf = 64;                          // keys per pipeline stage
-constexpr int kHalfBytes = kHalf * kRowBytes;      // 16 KiB
 // P is computed against the row's current reference max without looking at the new scores'
 // max; only when a block's row sum shows that some score exceeded the reference by more than
 // ~2^kRaiseLog2 is the reference raised (and O, l rescaled, P recomputed).  O/l stay exact
@@ -45,30 +43,31 @@ struct SoftmaxState {
   float l_run = 0.f;         // this half-wave's partial row sum
 };
 
-// One 64-key half tile for this wave's 32 query rows.  With `mask` (wave-uniform) keys beyond
-// the query's own tile-local index are hidden; `key0` = tile-local index of the half's first key.
-__device__ __forceinline__ void half_tile(const unsigned char* sK, const unsigned char* sV, const bf16x8 (&qf)[8],
+// kB blocks of 32 keys for this wave's 32 query rows.  With `mask` (wave-uniform) keys beyond
+// the query's own tile-local index are hidden; `key0` = tile-local index of the first key.
+template <int kB>
+__device__ __forceinline__ void key_blocks(const unsigned char* sK, const unsigned char* sV, const bf16x8 (&qf)[8],
                                           f32x16 (&oacc)[4], SoftmaxState& st, const TrLane& tr, float scale_log2,
                                           int l32, int hi, int q_local, int key0, bool mask, bool first) {
-  // ---- S^T = K Q^T : 2 blocks of 32 keys x 32 queries ------------------------------------
-  // The 16 K fragments are fetched kAhead reads ahead of the MFMA that consumes them, so the
+  // ---- S^T = K Q^T : kB blocks of 32 keys x 32 queries -----------------------------------
+  // The 8 * kB K fragments are fetched kAhead reads ahead of the MFMA that consumes them, so the
   // LDS latency is covered by the preceding MFMAs instead of being paid before each one.
-  f32x16 s[2];
-  s[0] = f32x16{0};
-  s[1] = f32x16{0};
+  f32x16 s[kB];
+#pragma unroll
+  for (int mb = 0; mb < kB; ++mb) s[mb] = f32x16{0};
   {
     constexpr int kAhead = 4;
-    bf16x8 kfr[16];
+    bf16x8 kfr[8 * kB];
 #pragma unroll
-    for (int i = 0; i < kAhead; ++i) kfr[i] = lds_read_b128(sK, lds_off_k(32 * (i & 1) + l32, 2 * (i >> 1) + hi));
+    for (int i = 0; i < kAhead; ++i) kfr[i] = lds_read_b128(sK, lds_off_k(32 * (i % kB) + l32, 2 * (i / kB) + hi));
     __builtin_amdgcn_sched_group_barrier(0x100, kAhead, 0);   // kAhead LDS reads up front
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      if (i + kAhead < 16) {
+    for (int i = 0; i < 8 * kB; ++i) {
+      if (i + kAhead < 8 * kB) {
         const int j = i + kAhead;
-        kfr[j] = lds_read_b128(sK, lds_off_k(32 * (j & 1) + l32, 2 * (j >> 1) + hi));
+        kfr[j] = lds_read_b128(sK, lds_off_k(32 * (j % kB) + l32, 2 * (j / kB) + hi));
       }
-      s[i & 1] = mfma32(kfr[i], qf[i >> 1], s[i & 1]);
+      s[i % kB] = mfma32(kfr[i], qf[i / kB], s[i % kB]);
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // then 1 MFMA, 1 LDS read, ...
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
     }
@@ -77,7 +76,7 @@ __device__ __forceinline__ void half_tile(const unsigned char* sK, const unsigne
   if (mask) {
     keep_branch_local(q_local);
 #pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
+    for (int mb = 0; mb < kB; ++mb)
 #pragma unroll
       for (int i = 0; i < 16; ++i)
         if (key0 + 32 * mb + 8 * (i >> 2) + 4 * hi + (i & 3) > q_local) s[mb][i] = -INFINITY;
@@ -89,11 +88,11 @@ __device__ __forceinline__ void half_tile(const unsigned char* sK, const unsigne
   for (int i = 0; i < kVAhead; ++i) vfr[i] = lds_read_tr_frag<lds_off_v>(sV, tr, 16 * (i >> 2), i & 3);
   // ---- online softmax (fp32, log2 domain) ---------------------------------------------------
   float rs = 0.f;
-  bf16x8 pf[4];
+  bf16x8 pf[2 * kB];
   bool raise = first;
   if (!first) {
 #pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
+    for (int mb = 0; mb < kB; ++mb)
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const float pv = fast_exp2(fmaf(s[mb][i], scale_log2, -st.m_use));
@@ -103,9 +102,11 @@ __device__ __forceinline__ void half_tile(const unsigned char* sK, const unsigne
     raise = __builtin_amdgcn_ballot_w64(!(rs < kRaiseSum)) != 0;       // wave-uniform, rare
   }
   if (raise) {
-    float mx = fmaxf(s[0][0], s[1][0]);
+    float mx = -INFINITY;
 #pragma unroll
-    for (int i = 1; i < 16; ++i) mx = fmaxf(mx, fmaxf(s[0][i], s[1][i]));
+    for (int i = 0; i < 16; ++i)
+#pragma unroll
+      for (int mb = 0; mb < kB; ++mb) mx = fmaxf(mx, s[mb][i]);
     mx = xhalf_max(mx) * scale_log2;
     const float m_new = fmaxf(st.m_run, mx);
     const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
@@ -119,7 +120,7 @@ __device__ __forceinline__ void half_tile(const unsigned char* sK, const unsigne
       for (int i = 0; i < 16; ++i) oacc[mbd][i] *= alpha;
     rs = 0.f;
 #pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
+    for (int mb = 0; mb < kB; ++mb)
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const float pv = fast_exp2(fmaf(s[mb][i], scale_log2, -m_use));
@@ -128,10 +129,10 @@ __device__ __forceinline__ void half_tile(const unsigned char* sK, const unsigne
       }
   }
   st.l_run += rs;
-  // ---- O^T += V^T P^T : 4 blocks of 32 d x 32 queries, 4 steps of 16 keys -------------------
+  // ---- O^T += V^T P^T : 4 blocks of 32 d x 32 queries, 2 * kB steps of 16 keys -------------------
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    if (i + kVAhead < 16) vfr[(i + kVAhead) & 3] = lds_read_tr_frag<lds_off_v>(sV, tr, 16 * ((i + kVAhead) >> 2), (i + kVAhead) & 3);
+  for (int i = 0; i < 8 * kB; ++i) {
+    if (i + kVAhead < 8 * kB) vfr[(i + kVAhead) & 3] = lds_read_tr_frag<lds_off_v>(sV, tr, 16 * ((i + kVAhead) >> 2), (i + kVAhead) & 3);
     oacc[i & 3] = mfma32(vfr[i & 3], pf[i >> 2], oacc[i & 3]);
     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // 1 MFMA
     __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);   // 2 LDS reads (one fragment)
@@ -139,26 +140,31 @@ __device__ __forceinline__ void half_tile(const unsigned char* sK, const unsigne
 }
 
 // kGroups = 2: two groups of four wavefronts share the query tile, one takes the first 64 keys of every tile, the
-// other the second; their results are combined through LDS.  A launch that gives a CU one workgroup at most runs it at
+// other the second; their results are combined through LDS.  kGroups = 4: four groups of two wavefronts share half
+// a query tile, each takes 32 keys of every tile.  A launch that gives a CU one workgroup at most runs it at
 // one wave per SIMD, where a half tile takes 1.2 us of which the matrix pipe is busy 0.4; with the second group the CU is
 // as full as with two workgroups, without partial results in memory.
 template <int kGroups>
-__global__ __launch_bounds__(256 * kGroups, 2) void fwd_kernel(const FwdParams p) {
+__global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void fwd_kernel(const FwdParams p) {
+  constexpr int kWaves = Groups<kGroups>::kWaves, kRows = Groups<kGroups>::kRows, kLines = Groups<kGroups>::kLines;
+  constexpr int kStageBytes = kRows * kRowBytes;
   // two pipeline stages per group, distinct arrays so that reads of one stage need not wait for the
   // copies in flight into the other
-  __shared__ __attribute__((aligned(1024))) unsigned char sKA[kGroups * kHalfBytes];
-  __shared__ __attribute__((aligned(1024))) unsigned char sVA[kGroups * kHalfBytes];
-  __shared__ __attribute__((aligned(1024))) unsigned char sKB[kGroups * kHalfBytes];
-  __shared__ __attribute__((aligned(1024))) unsigned char sVB[kGroups * kHalfBytes];
+  __shared__ __attribute__((aligned(1024))) unsigned char sKA[kGroups * kStageBytes];
+  __shared__ __attribute__((aligned(1024))) unsigned char sVA[kGroups * kStageBytes];
+  __shared__ __attribute__((aligned(1024))) unsigned char sKB[kGroups * kStageBytes];
+  __shared__ __attribute__((aligned(1024))) unsigned char sVB[kGroups * kStageBytes];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave_in_block = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wave = kGroups == 1 ? wave_in_block : wave_in_block & 3, group = kGroups == 1 ? 0 : wave_in_block >> 2;
-  unsigned char *const kA = sKA + group * kHalfBytes, *const vA = sVA + group * kHalfBytes;
-  unsigned char *const kB = sKB + group * kHalfBytes, *const vB = sVB + group * kHalfBytes;
+  const int wave = wave_in_block % kWaves, group = wave_in_block / kWaves;
+  unsigned char *const kA = sKA + group * kStageBytes, *const vA = sVA + group * kStageBytes;
+  unsigned char *const kB = sKB + group * kStageBytes, *const vB = sVB + group * kStageBytes;
   const int l32 = lane & 31, hi = lane >> 5;
   int pos, bh;
-  map_block(blockIdx.x, p.batch * p.n_heads, p.heads_per_xcd, p.n_qtiles * p.n_parts, pos, bh);
+  map_block(blockIdx.x, p.batch * p.n_heads, p.heads_per_xcd, p.n_qtiles * p.n_parts * kLines, pos, bh);
+  const int sub = pos % kLines;            // which half of the tile's rows
+  pos /= kLines;
   const int b = bh / p.n_heads, h = bh % p.n_heads;
   int qt, e0, e1, diag = -1, part = 0;
   if (p.dense) {
@@ -183,35 +189,36 @@ __global__ __launch_bounds__(256 * kGroups, 2) void fwd_kernel(const FwdParams p
   const bf16* vbase = p.v + b * p.vs.b + h * p.vs.h;
   const int k_stride = (int)p.ks.s, v_stride = (int)p.vs.s;
   int koff[4], voff[4];
-  dma_voffsets<lds_off_k, 4>(koff, k_stride, wave, lane);
-  dma_voffsets<lds_off_v, 4>(voff, v_stride, wave, lane);
-  const int k_half = kHalf * k_stride * 2, v_half = kHalf * v_stride * 2;                 // bytes
+  dma_voffsets<lds_off_k, kWaves>(koff, k_stride, wave, lane);
+  dma_voffsets<lds_off_v, kWaves>(voff, v_stride, wave, lane);
+  const int k_half = kRows * k_stride * 2, v_half = kRows * v_stride * 2;                 // bytes of one stage in memory
   const uint32_t k_extent = (uint32_t)((kTile - 1) * k_stride + kHeadDim) * 2;            // bytes of one tile
   const uint32_t v_extent = (uint32_t)((kTile - 1) * v_stride + kHeadDim) * 2;
   auto k_rsrc = [&](int kt) { return make_rsrc(kbase + (int64_t)kt * kTile * k_stride, k_extent); };
   auto v_rsrc = [&](int kt) { return make_rsrc(vbase + (int64_t)kt * kTile * v_stride, v_extent); };
 
-  // step i = one half tile of this group: half i % 2 of entry e0 + i / 2, with two groups half `group` of entry e0 + i
+  // step i = one stage of this group: half i % 2 of entry e0 + i / 2, else half or quarter `group` of entry e0 + i
   const int n_steps = (kGroups == 1 ? 2 : 1) * (e1 - e0);
   auto entry_of = [&](int i) { return e0 + (kGroups == 1 ? i >> 1 : i); };
-  // the first half tile goes in flight before anything else
+  // the first stage goes in flight before anything else
   int kt = 0;
   if (n_steps > 0) {
     kt = ktile(e0);
-    dma_half_tile_buf<4>(kA, k_rsrc(kt), koff, group * k_half, wave);
-    dma_half_tile_buf<4>(vA, v_rsrc(kt), voff, group * v_half, wave);
+    dma_rows_buf<kWaves>(kA, k_rsrc(kt), koff, group * k_half, wave);
+    dma_rows_buf<kWaves>(vA, v_rsrc(kt), voff, group * v_half, wave);
   }
 
-  // Q fragment (B operand of S^T): lane holds query row 32*wave + lane%32,
+  // Q fragment (B operand of S^T): lane holds query row 32*q_block + lane%32,
   // d = 16*ks + 8*(lane/32) .. +7 for ks = 0..7.
   // (through the stage that the first step fills)
-  const int q_local = wave * 32 + l32;
-  const int qrow0 = qt * kTile + wave * 32, qrow = qrow0 + l32;
+  const int q_block = kWaves * sub + wave;
+  const int q_local = q_block * 32 + l32;
+  const int qrow0 = qt * kTile + q_block * 32, qrow = qrow0 + l32;
   bf16x8 qf[8];
   {
     u32x4 raw[8];
     load_rows(raw, p.q + b * p.qs.b + (int64_t)qrow0 * p.qs.s + h * p.qs.h, p.qs.s);
-    rows_to_frags(qf, raw, (uint32_t)(uintptr_t)(lds_byte*)((wave < 2 ? kB : vB) + (wave & 1) * kWaveRowsBytes));
+    rows_to_frags(qf, raw, (uint32_t)(uintptr_t)(lds_byte*)((wave < kWaves / 2 ? kB : vB) + wave % (kWaves / 2) * kWaveRowsBytes));
   }
 
   f32x16 oacc[4];
@@ -237,13 +244,14 @@ __global__ __launch_bounds__(256 * kGroups, 2) void fwd_kernel(const FwdParams p
     __syncthreads();
     if (more) {
       const int half_next = kGroups == 1 ? kStage ^ 1 : group;
-      dma_half_tile_buf<4>(kStage ? kA : kB, k_rsrc(kt_next), koff, half_next * k_half, wave);
-      dma_half_tile_buf<4>(kStage ? vA : vB, v_rsrc(kt_next), voff, half_next * v_half, wave);
+      dma_rows_buf<kWaves>(kStage ? kA : kB, k_rsrc(kt_next), koff, half_next * k_half, wave);
+      dma_rows_buf<kWaves>(kStage ? vA : vB, v_rsrc(kt_next), voff, half_next * v_half, wave);
     }
-    // causal tile: queries 64..127 (waves 2, 3) see all of keys 0..63, queries 0..63 (waves 0, 1) none of keys 64..127
-    if (half == 0 || !causal || wave >= 2) {
-      half_tile(kStage ? kB : kA, kStage ? vB : vA, qf, oacc, st, tr, p.scale_log2, l32, hi, q_local, kHalf * half,
-                causal && (half == 0 ? wave < 2 : true), kGroups == 1 ? kStage == 0 && i == 0 : !started);
+    // causal tile: blocks of keys beyond the wave's block of queries are hidden, that block itself in part
+    constexpr int kBlocks = kRows / 32;
+    if (!causal || kBlocks * half <= q_block) {
+      key_blocks<kBlocks>(kStage ? kB : kA, kStage ? vB : vA, qf, oacc, st, tr, p.scale_log2, l32, hi, q_local, kRows * half,
+                     causal && q_block < kBlocks * half + kBlocks, kGroups == 1 ? kStage == 0 && i == 0 : !started);
       started = true;
     }
     kt = kt_next;
@@ -255,36 +263,47 @@ __global__ __launch_bounds__(256 * kGroups, 2) void fwd_kernel(const FwdParams p
 
   // ---- epilogue: normalise, write O (bf16) and LSE (natural log) -------------------------
   float l_tot = xhalf_sum(st.l_run);
-  unsigned char* turn = (wave < 2 ? kA : vA) + (wave & 1) * kWaveRowsBytes;       // everyone left stage A before the last step
-  if constexpr (kGroups == 2) {
-    // the second group hands over its rows' max, sum and O: a 16-byte piece of a lane after the other, 1 KiB per instruction
+  bf16* const orow = p.o + part * p.o_part + b * p.os.b + (int64_t)qrow0 * p.os.s + h * p.os.h;
+  auto lds_at = [](unsigned char* x) { return (uint32_t)(uintptr_t)(lds_byte*)x; };
+  if constexpr (kGroups == 1) {
+    const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+    store_rows_bf16(orow, p.os.s, oacc, inv, lds_at((wave < 2 ? kA : vA) + (wave & 1) * kWaveRowsBytes));   // everyone left stage A before the last step
+  } else {
+    // the groups exchange their rows' max, sum and O.  Area x of the stages' LDS belongs to group x % kGroups of wave x / kGroups.
+    __shared__ float stat[8][2][64];
+    auto area = [&](int x) { return lds_at(x < 2 ? sKA : x < 4 ? sVA : x < 6 ? sKB : sVB) + (x & 1) * kAccBytes; };
+    const int own = wave * kGroups + group;
+    constexpr bool kAll = kGroups == 2;        // the first group finishes whole rows; with four groups each a block of 32 columns
     __syncthreads();
-    turn = (wave < 2 ? sKA : sVA) + (wave & 1) * 2 * kWaveRowsBytes;
-    const uint32_t at = (uint32_t)(uintptr_t)(lds_byte*)turn + 16 * lane, at_stat = (uint32_t)(uintptr_t)(lds_byte*)sKB + wave * 512 + 4 * lane;
-    if (group == 1) {
-      lds_put(at_stat, st.m_run);
-      lds_put(at_stat + 256, l_tot);
-#pragma unroll
-      for (int i = 0; i < 16; ++i) lds_put(at + 1024 * i, f32x4{oacc[i >> 2][4 * (i & 3)], oacc[i >> 2][4 * (i & 3) + 1], oacc[i >> 2][4 * (i & 3) + 2], oacc[i >> 2][4 * (i & 3) + 3]});
-    }
+    stat[own][0][lane] = st.m_run;
+    stat[own][1][lane] = l_tot;
+    if (!kAll || group == 1) put_acc(area(own), oacc);
     __syncthreads();
-    if (group == 1) return;
-    const float m1 = lds_get<float>(at_stat), l1 = lds_get<float>(at_stat + 256);
-    const float m = fmaxf(st.m_run, m1), ms = m == -INFINITY ? 0.f : m;
-    const float w0 = fast_exp2(st.m_run - ms), w1 = fast_exp2(m1 - ms);
+    if (kAll && group == 1) return;
+    float m = -INFINITY, w[kGroups];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const f32x4 x = lds_get<f32x4>(at + 1024 * i);
+    for (int g = 0; g < kGroups; ++g) m = fmaxf(m, stat[wave * kGroups + g][0][lane]);
+    const float ms = m == -INFINITY ? 0.f : m;
+    l_tot = 0.f;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) oacc[i >> 2][4 * (i & 3) + j] = oacc[i >> 2][4 * (i & 3) + j] * w0 + x[j] * w1;
+    for (int g = 0; g < kGroups; ++g) {
+      w[g] = fast_exp2(stat[wave * kGroups + g][0][lane] - ms);
+      l_tot += stat[wave * kGroups + g][1][lane] * w[g];
     }
     st.m_run = m;
-    l_tot = l_tot * w0 + l1 * w1;
+    const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+    if constexpr (kAll) {
+#pragma unroll
+      for (int mb = 0; mb < 4; ++mb) add_block(area(own + 1), mb, oacc[mb], w[0], w[1]);
+      store_rows_bf16(orow, p.os.s, oacc, inv, area(own + 1));
+    } else {
+      f32x16 o{0};
+#pragma unroll
+      for (int g = 0; g < kGroups; ++g) add_block(area(wave * kGroups + g), group, o, 1.f, w[g]);
+      store_block_bf16(orow + 32 * group, p.os.s, o, inv, area(own) + 4096 * group);
+    }
   }
-  const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-  store_rows_bf16(p.o + part * p.o_part + b * p.os.b + (int64_t)qrow0 * p.os.s + h * p.os.h, p.os.s, oacc, inv,
-                  (uint32_t)(uintptr_t)(lds_byte*)turn);
-  if (hi == 0) {
+  if (hi == 0 && group == 0) {
     const float lse = l_tot > 0.f ? (st.m_run + __builtin_amdgcn_logf(l_tot)) * kLn2 : -INFINITY;
     p.lse[part * p.lse_part + ((int64_t)b * p.n_heads + h) * ((int64_t)p.n_qtiles * kTile) + qrow] = lse;
   }
@@ -320,44 +339,53 @@ static int fwd_common(FwdParams& p, const void* q, const void* k, const void* v,
   return check_device();
 }
 
-// Two groups per workgroup where a CU gets one workgroup at most and the walk is worth the handing over at its end, from
-// three tiles on (two tiles: 8.1 us with one group, 8.5 with two).  An uncut causal rectangle is better off with
-// them up to two per CU: run one after the other, longest first, they balance its rows of different lengths, which
-// two workgroups resident from the start do not (16 heads of 4096: 91 us resident, 76 in turn; 8 of 8192: 156, 132); the
-// rows of a list are too much alike for that (strided 8k, 8 heads: 84 and 95).
-static bool fwd_pairs(int64_t groups, int64_t walk, int n_parts, bool dense_causal) {
-  return walk >= 3 && groups <= (dense_causal && n_parts == 1 ? 2 * kCus : kCus);
+// Groups per workgroup for n lines of 128 rows (parts counted):
+//  - four, on half lines, while those leave a CU one workgroup at most (8 heads of 1024: 17.2 us with two groups, 13.8
+//    with four; 2048: 29.9, 24.3).  A walk of one tile is not worth the handing over at its end (6.1 us, one group 5.7).
+//  - two, on whole lines, up to one workgroup per CU and from three tiles on (32 heads of 1024: 25 us with one, 22 with two).
+//  - The rows of an uncut causal rectangle differ in length.  Run one after the other, longest first, they are
+//    balanced, which workgroups resident side by side from the start do not achieve: four groups up to 256 lines of 16
+//    tiles (8 heads of 4096: 57 us with two, 48 with four), two up to 512 lines (16 heads of 4096: 89 us with one, 77 with
+//    two).  The rows of a list are too much alike for that (strided 8k, 8 heads: 84 us with one, 95 with two).
+static int fwd_groups(int64_t n, int64_t walk, int n_parts, bool dense_causal) {
+  const bool uneven = dense_causal && n_parts == 1;
+  if (walk >= 2 && (2 * n <= kCus || (uneven && n <= kCus && walk >= 16))) return 4;
+  return walk >= 3 && n <= (uneven ? 2 * kCus : kCus) ? 2 : 1;
 }
 static int fwd_launch(const FwdParams& p, hipStream_t st) {
-  const unsigned groups = (unsigned)(p.batch * p.n_heads * p.n_qtiles * p.n_parts);
-  const int64_t walk = p.dense ? p.part_len : p.nnz / p.n_qtiles;
-  if (fwd_pairs(groups, walk, p.n_parts, p.dense_causal)) hipLaunchKernelGGL(fwd_kernel<2>, dim3(groups), dim3(512), 0, st, p);
-  else                                                    hipLaunchKernelGGL(fwd_kernel<1>, dim3(groups), dim3(256), 0, st, p);
+  const unsigned n = (unsigned)(p.batch * p.n_heads * p.n_qtiles * p.n_parts);
+  switch (fwd_groups(n, p.dense ? p.part_len : p.nnz / p.n_qtiles, p.n_parts, p.dense_causal)) {
+    case 4: hipLaunchKernelGGL(fwd_kernel<4>, dim3(2 * n), dim3(512), 0, st, p); break;
+    case 2: hipLaunchKernelGGL(fwd_kernel<2>, dim3(n), dim3(512), 0, st, p); break;
+    default: hipLaunchKernelGGL(fwd_kernel<1>, dim3(n), dim3(256), 0, st, p);
+  }
   return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH;
 }
 
 // How many parts the walks of a dense forward are cut into, at most max_parts (what the workspace holds).  A cut
 // gives a small rectangle enough workgroups and costs the partials' way through memory and a merge; an estimate of the
 // launches' time in microseconds decides, fitted to 47 shapes of 1 to 32 heads and 128 to 8192 tokens (the cut it
-// takes is within 4 % of the best one on each):
-//  - 4.1 to start, load Q, store and end, 5.7 with two groups per workgroup;
-//  - a tile takes 1.5 with two groups, else 2.2, and 3.4 where two workgroups share the CU;
-//  - the merge takes 1.7 + 0.04 a part, and the partials 1 per 1.3 MB.
-// 512 x 512, 32 heads: 17 us cut in two, 12 uncut; 1024 x 4096, one head: 52 uncut, 14 cut in 16.
+// takes is within 3 % of the best one on each):
+//  - 3.8 to start, load Q, store and end, 4.3 with two groups per workgroup, 5.1 with four;
+//  - a tile takes 1.1 with four groups, 1.8 with two, else 2.2, and 3.7 where two workgroups share the CU;
+//  - the merge takes 2.4, and the partials 1 per 1.5 MB.
+// 1024 x 4096, one head: 41 us uncut, 13 cut in 16.
 static int fwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int max_parts) {
   const float density = causal ? 0.5f : 1.f, lines = (float)nbh * n_qtiles;
   int best = 1;
   float best_us = INFINITY;
   for (int parts = 1; parts <= max_parts; ++parts) {
     const float groups = lines * parts, longest = (float)((n_ktiles + parts - 1) / parts);
-    float us = 4.1f;
-    if (fwd_pairs(nbh * n_qtiles * parts, (n_ktiles + parts - 1) / parts, parts, causal)) {
-      us += 1.6f + longest * 1.5f;
-    } else {
-      const float shared = fminf(fmaxf((groups * density - kCus) / kCus, 0.f), 1.f);      // share of the workgroups with a neighbour
-      us += fmaxf(longest * (2.2f + 1.2f * shared), density * lines * n_ktiles * 3.4f / (2 * kCus));
+    float us;
+    switch (fwd_groups(nbh * n_qtiles * parts, (n_ktiles + parts - 1) / parts, parts, causal)) {
+      case 4: us = 5.1f + longest * 1.1f; break;
+      case 2: us = 4.3f + longest * 1.8f; break;
+      default: {
+        const float shared = fminf(fmaxf((groups * density - kCus) / kCus, 0.f), 1.f);      // share of the workgroups with a neighbour
+        us = 3.8f + fmaxf(longest * (2.2f + 1.5f * shared), density * lines * n_ktiles * 3.7f / (2 * kCus));
+      }
     }
-    if (parts > 1) us += 1.7f + 0.04f * parts + groups * (kTile * kHeadDim * 2) / 1.3e6f;
+    if (parts > 1) us += 2.4f + 0.03f * parts + groups * (kTile * kHeadDim * 2) / 1.5e6f;
     if (us < best_us) { best_us = us; best = parts; }
   }
   return best;

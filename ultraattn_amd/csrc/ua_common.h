@@ -147,6 +147,66 @@ __device__ __forceinline__ void store_rows_f32(float* rows, int64_t row_stride, 
   }
 }
 
+// One block of 32 columns of the same rows (a wave's share after a sum over groups): acc[4g + j] = column
+// 8 * g + 4 * (lane / 32) + j of row lane % 32, `rows` already at the block; through 2 or 4 KiB of LDS.
+__device__ __forceinline__ void store_block_bf16(bf16* rows, int64_t row_stride, const f32x16& acc, float mul, uint32_t lds) {
+  const int lane = fresh_lane(), r = lane & 31;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    bf16x4 w;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[j] = (bf16)(acc[4 * g + j] * mul);
+    lds_put(lds + r * 64 + ((g ^ (r >> 2 & 3)) << 4) + 8 * (lane >> 5), w);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int row = 16 * i + (lane >> 2), c = lane & 3;
+    *reinterpret_cast<u32x4*>(rows + row * row_stride + 8 * c) = lds_get<u32x4>(lds + row * 64 + ((c ^ (row >> 2 & 3)) << 4));
+  }
+}
+__device__ __forceinline__ void store_block_f32(float* rows, int64_t row_stride, const f32x16& acc, float mul, uint32_t lds) {
+  const int lane = fresh_lane(), r = lane & 31;
+#pragma unroll
+  for (int g = 0; g < 4; ++g)
+    lds_put(lds + r * 128 + (((2 * g + (lane >> 5)) ^ (r >> 1 & 7)) << 4),
+            f32x4{acc[4 * g] * mul, acc[4 * g + 1] * mul, acc[4 * g + 2] * mul, acc[4 * g + 3] * mul});
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = 8 * i + (lane >> 3), c = lane & 7;
+    *reinterpret_cast<f32x4*>(rows + row * row_stride + 4 * c) = lds_get<f32x4>(lds + row * 128 + ((c ^ (row >> 1 & 7)) << 4));
+  }
+}
+// A wave's accumulators in LDS for the waves of the other groups: 16-byte pieces, 1 KiB per instruction; block mb of 32
+// columns is the 4 KiB at 4096 * mb.
+constexpr int kAccBytes = 64 * 64 * 4;
+__device__ __forceinline__ void put_acc(uint32_t lds, const f32x16 (&acc)[4]) {
+  lds += 16 * fresh_lane();
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const f32x16& a = acc[i >> 2];
+    lds_put(lds + 1024 * i, f32x4{a[4 * (i & 3)], a[4 * (i & 3) + 1], a[4 * (i & 3) + 2], a[4 * (i & 3) + 3]});
+  }
+}
+// acc = acc * wa + (block mb) * wb
+__device__ __forceinline__ void add_block(uint32_t lds, int mb, f32x16& acc, float wa = 1.f, float wb = 1.f) {
+  lds += 16 * fresh_lane() + 4096 * mb;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const f32x4 x = lds_get<f32x4>(lds + 1024 * i);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[4 * i + j] = acc[4 * i + j] * wa + x[j] * wb;
+  }
+}
+// What the attention kernels' groups share: with 1 or 2 groups a group is four waves, its line the 128 rows of a tile and its
+// stage a half tile of the other side; with 4 groups two waves, half a tile's rows (64) and a block of 32.
+template <int kGroups>
+struct Groups {
+  static constexpr int kWaves = kGroups == 4 ? 2 : 4;
+  static constexpr int kRows = kGroups == 4 ? 32 : 64;         // rows per stage
+  static constexpr int kLines = kGroups == 4 ? 2 : 1;          // lines per tile
+  static constexpr int kThreads = kGroups == 1 ? 256 : 512;
+};
+
 __device__ __forceinline__ void wait_vmem_all() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 // At the top of a rare wave-uniform branch: keeps it a branch (its body is not turned into selects), and what
 // the body computes from x stays in it.  Hoisted out of the walk, the comparisons of a masked tile take two
@@ -176,24 +236,24 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, ui
 __device__ __forceinline__ void dma16_buf(__amdgpu_buffer_rsrc_t r, unsigned char* lds_dst, int voff, int soff) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds_dst, 16, voff, soff, 0, 0);
 }
-// Per-thread byte offsets for staging a [64][128] bf16 half tile (16 KiB) with NW waves: each
-// thread issues 16/NW copies; copy i of wave w fills LDS rows 4*(NW*i + w) .. +3; lane l lands in
+// Per-thread byte offsets for staging 16 * NW rows of 128 bf16 with NW waves: each thread issues 4
+// copies; copy i of wave w fills LDS rows 4*(NW*i + w) .. +3; lane l lands in
 // that group's row l/16, physical 16-byte slot l%16, so it must fetch the logical chunk that the
 // XOR layout `OFF` maps to that slot.
 template <int (*OFF)(int, int), int NW>
-__device__ __forceinline__ void dma_voffsets(int (&off)[16 / NW], int row_stride, int wave, int lane) {
+__device__ __forceinline__ void dma_voffsets(int (&off)[4], int row_stride, int wave, int lane) {
 #pragma unroll
-  for (int i = 0; i < 16 / NW; ++i) {
+  for (int i = 0; i < 4; ++i) {
     const int r = 4 * (NW * i + wave) + (lane >> 4);
     const int c = ((OFF(r, 0) - r * kRowBytes) >> 4) ^ (lane & 15);
     off[i] = (r * row_stride + c * 8) * 2;
   }
 }
 template <int NW>
-__device__ __forceinline__ void dma_half_tile_buf(unsigned char* lds, __amdgpu_buffer_rsrc_t r, const int (&voff)[16 / NW],
+__device__ __forceinline__ void dma_rows_buf(unsigned char* lds, __amdgpu_buffer_rsrc_t r, const int (&voff)[4],
                                                   int soff, int wave) {
 #pragma unroll
-  for (int i = 0; i < 16 / NW; ++i) dma16_buf(r, lds + (NW * i + wave) * 1024, voff[i], soff);
+  for (int i = 0; i < 4; ++i) dma16_buf(r, lds + (NW * i + wave) * 1024, voff[i], soff);
 }
 
 // blockIdx -> (position in the launch order, batch*head).  Consecutive workgroups go to
