@@ -43,7 +43,7 @@ struct BwdParams {
   // dense_causal [kt - diag_off, n_qtiles), the first one causal.
   int dense, dense_causal, diag_off;
   int n_col_blocks;                        // bwd_kernel: workgroups of the columns, those of the rows follow
-  int cols_shortest_first;                 // dense causal: launch order of the columns (see launch_bwd)
+  int cols_reversed;                       // launch order of the columns (see launch_bwd)
   BwdSide cols, rows;
 };
 
@@ -271,13 +271,13 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block
   if (p.dense) {
     part = pos / p.n_ktiles;
     kt = pos - part * p.n_ktiles;                          // column 0 is the longest of a causal rectangle
-    if (p.cols_shortest_first) kt = p.n_ktiles - 1 - kt;
+    if (p.cols_reversed) kt = p.n_ktiles - 1 - kt;
     if (p.dense_causal) diag = kt - p.diag_off;            // query tile on the diagonal (may lie outside)
     const int qbeg = p.dense_causal ? min(max(diag, 0), p.n_qtiles) : 0;
     e0 = min(max(part * p.cols.part_len, qbeg), p.n_qtiles);
     e1 = max(min((part + 1) * p.cols.part_len, p.n_qtiles), e0);
   } else {
-    kt = min(max(sload(p.cols.order, pos), 0), p.n_ktiles - 1);
+    kt = min(max(sload(p.cols.order, p.cols_reversed ? p.n_ktiles - 1 - pos : pos), 0), p.n_ktiles - 1);
     e0 = min(max(sload(p.cols.ptr, kt), 0), p.nnz);
     e1 = min(max(sload(p.cols.ptr, kt + 1), e0), p.nnz);
   }
@@ -629,7 +629,7 @@ static int fill_common(BwdParams& p, const void* q, const void* k, const void* v
   p.scale = softmax_scale; p.scale_log2 = softmax_scale * kLog2e;
   const int nbh = batch * n_heads;
   p.heads_per_xcd = (nbh % 8 == 0) ? nbh / 8 : 0;
-  p.dense = 0; p.dense_causal = 0; p.diag_off = 0; p.n_col_blocks = 0; p.cols_shortest_first = 0;
+  p.dense = 0; p.dense_causal = 0; p.diag_off = 0; p.n_col_blocks = 0; p.cols_reversed = 0;
   p.cols = BwdSide{}; p.rows = BwdSide{};
   p.cols.n_parts = p.rows.n_parts = 1;
   return UA_OK;
@@ -680,9 +680,9 @@ static int launch_bwd(BwdParams& p, hipStream_t st) {
   const int groups = groups_of(p);
   p.n_col_blocks = (int)col_blocks(p) * (groups == 4 ? 2 : 1);
   // Up to two workgroups per CU the whole launch is resident at once, and the second 256 join the first in launch
-  // order.  Rows come longest first; of a causal rectangle the columns then come shortest first, so that the long
-  // ones of one side share a CU with the short ones of the other (32 heads of 1024: 43.6 -> 41.5 us).
-  p.cols_shortest_first = groups == 1 && p.dense_causal && both_blocks(p) <= 2 * kCus;
+  // order.  Both sides come longest first (lists roughly); the columns are then taken in reverse, so that the long ones
+  // of one side share a CU with the short ones of the other (32 causal heads of 1024: 43.6 -> 41.5 us).
+  p.cols_reversed = groups == 1 && (p.dense_causal || !p.dense) && both_blocks(p) > kCus && both_blocks(p) <= 2 * kCus;
   UA_LAUNCH_GROUPS(bwd_kernel, both_blocks(p), p, st)
   return launched();
 }
@@ -715,16 +715,16 @@ static BwdCut bwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int 
         case 2: us = 9.8f; tc = 2.6f; tr = 1.7f; break;
         default: {
           const float shared = fminf(fmaxf((groups - kCus) / kCus, 0.f), 1.f);       // share of the workgroups with a neighbour
-          us = 6.5f; tc = 3.5f + 1.4f * shared; tr = 2.1f + 3.4f * shared;
+          us = 6.5f; tc = 3.5f + 1.44f * shared; tr = 2.1f + 3.37f * shared;
         }
       }
       const float longest = fmaxf((float)((n_qtiles + pc - 1) / pc) * tc, (float)((n_ktiles + pr - 1) / pr) * tr);
-      const float all = density * wk * n_qtiles * (4.9f + 5.5f) / (2 * kCus);
+      const float all = density * wk * n_qtiles * (4.94f + 5.47f) / (2 * kCus);
       us += fmaxf(longest, all);
       if (pc > 1 || pr > 1) us = (us + 2.4f) * 1.06f;
       if (pc > 1) us += 2.f * pc * wk * (kTile * kHeadDim * 4) / 3.7e6f;
       if (pr > 1) us += pr * wq * (kTile * kHeadDim * 4) / 3.7e6f;
-      if (us < best_us) { best_us = us; best = {pc, pr}; }
+      if (us < 0.99f * best_us) { best_us = us; best = {pc, pr}; }        // more parts for a gain, not for a tie
     }
   }
   return best;

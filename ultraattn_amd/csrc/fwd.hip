@@ -20,6 +20,7 @@ struct FwdParams {
   const bf16* q; const bf16* k; const bf16* v; bf16* o; float* lse;
   const int32_t* row_ptr; const int32_t* col_idx; const uint8_t* flag; const int32_t* q_order;
   int batch, n_heads, n_qtiles, n_ktiles, nnz;
+  int n_first;           // positions of the launch order that are taken in reverse (see fwd_launch)
   Strides3 qs, ks, vs, os;
   float scale_log2;      // softmax_scale * log2(e)
   int heads_per_xcd;     // batch*n_heads / 8 when divisible, else 0
@@ -165,6 +166,7 @@ __global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void fwd_kernel(const
   map_block(blockIdx.x, p.batch * p.n_heads, p.heads_per_xcd, p.n_qtiles * p.n_parts * kLines, pos, bh);
   const int sub = pos % kLines;            // which half of the tile's rows
   pos /= kLines;
+  if (pos < p.n_first) pos = p.n_first - 1 - pos;
   const int b = bh / p.n_heads, h = bh % p.n_heads;
   int qt, e0, e1, diag = -1, part = 0;
   if (p.dense) {
@@ -327,7 +329,7 @@ static int fwd_common(FwdParams& p, const void* q, const void* k, const void* v,
   if (k_strides[1] > (INT32_MAX >> 9) || v_strides[1] > (INT32_MAX >> 9)) return UA_ERR_SHAPE;
   p.q = (const bf16*)q; p.k = (const bf16*)k; p.v = (const bf16*)v; p.o = (bf16*)o; p.lse = lse;
   p.row_ptr = nullptr; p.col_idx = nullptr; p.flag = nullptr; p.q_order = nullptr;
-  p.batch = batch; p.n_heads = n_heads; p.n_qtiles = n_qtiles; p.n_ktiles = n_ktiles; p.nnz = 0;
+  p.batch = batch; p.n_heads = n_heads; p.n_qtiles = n_qtiles; p.n_ktiles = n_ktiles; p.nnz = 0; p.n_first = 0;
   p.qs = {q_strides[0], q_strides[1], q_strides[2]};
   p.ks = {k_strides[0], k_strides[1], k_strides[2]};
   p.vs = {v_strides[0], v_strides[1], v_strides[2]};
@@ -352,12 +354,17 @@ static int fwd_groups(int64_t n, int64_t walk, int n_parts, bool dense_causal) {
   if (walk >= 2 && (2 * n <= kCus || (uneven && n <= kCus && walk >= 16))) return 4;
   return walk >= 3 && n <= (uneven ? 2 * kCus : kCus) ? 2 : 1;
 }
-static int fwd_launch(const FwdParams& p, hipStream_t st) {
+static int fwd_launch(FwdParams& p, hipStream_t st) {
   const unsigned n = (unsigned)(p.batch * p.n_heads * p.n_qtiles * p.n_parts);
   switch (fwd_groups(n, p.dense ? p.part_len : p.nnz / p.n_qtiles, p.n_parts, p.dense_causal)) {
     case 4: hipLaunchKernelGGL(fwd_kernel<4>, dim3(2 * n), dim3(512), 0, st, p); break;
     case 2: hipLaunchKernelGGL(fwd_kernel<2>, dim3(n), dim3(512), 0, st, p); break;
-    default: hipLaunchKernelGGL(fwd_kernel<1>, dim3(n), dim3(256), 0, st, p);
+    default:
+      // Up to two workgroups per CU the whole launch is resident at once, and those after the first 256 join them in
+      // launch order.  Lists come roughly by falling length, so the first ones are taken in reverse: long and
+      // short lists then share a CU (strided 8k, 8 heads: the longest sum on a CU 40 -> 37 tiles, causal 96 -> 65).
+      if (!p.dense && n > kCus && n <= 2 * kCus) p.n_first = kCus * p.n_qtiles / (int)n;
+      hipLaunchKernelGGL(fwd_kernel<1>, dim3(n), dim3(256), 0, st, p);
   }
   return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH;
 }
@@ -386,7 +393,7 @@ static int fwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int max
       }
     }
     if (parts > 1) us += 2.4f + 0.03f * parts + groups * (kTile * kHeadDim * 2) / 1.5e6f;
-    if (us < best_us) { best_us = us; best = parts; }
+    if (us < 0.99f * best_us) { best_us = us; best = parts; }            // more parts for a gain, not for a tie
   }
   return best;
 }
