@@ -25,10 +25,12 @@ struct FwdParams {
   float scale_log2;      // softmax_scale * log2(e)
   int heads_per_xcd;     // batch*n_heads / 8 when divisible, else 0
   // Dense rectangle (no list arrays): query tile qt walks key tiles [0, n_ktiles), or with
-  // dense_causal [0, qt + diag_off] with the last one causal.  The key range is cut into n_parts
-  // parts of part_len tiles; part i writes its partial (O, LSE) at o + i * o_part, lse + i * lse_part
-  // (elements).  Longest rows are launched first.
-  int dense, dense_causal, diag_off, n_parts, part_len;
+  // dense_causal [0, qt + diag_off] with the last one causal; longest rows first.  The first n_whole query tiles (all
+  // if nothing is cut) are walked whole; the key range of the others is cut into n_parts parts of part_len tiles, and
+  // part i leaves its partial (O, LSE), contiguous over those n_qtiles - n_whole tiles, at part_o + i * o_part and
+  // part_lse + i * lse_part (elements).
+  int dense, dense_causal, diag_off, n_whole, n_parts, part_len;
+  bf16* part_o; float* part_lse;
   int64_t o_part, lse_part;
 };
 
@@ -163,20 +165,24 @@ __global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void fwd_kernel(const
   unsigned char *const kB = sKB + group * kStageBytes, *const vB = sVB + group * kStageBytes;
   const int l32 = lane & 31, hi = lane >> 5;
   int pos, bh;
-  map_block(blockIdx.x, p.batch * p.n_heads, p.heads_per_xcd, p.n_qtiles * p.n_parts * kLines, pos, bh);
+  map_block(blockIdx.x, p.batch * p.n_heads, p.heads_per_xcd, (p.n_whole + (p.n_qtiles - p.n_whole) * p.n_parts) * kLines, pos, bh);
   const int sub = pos % kLines;            // which half of the tile's rows
   pos /= kLines;
   if (pos < p.n_first) pos = p.n_first - 1 - pos;
   const int b = bh / p.n_heads, h = bh % p.n_heads;
-  int qt, e0, e1, diag = -1, part = 0;
+  int qt, e0, e1, diag = -1, part = -1;
   if (p.dense) {
-    part = pos / p.n_qtiles;
-    const int line = pos - part * p.n_qtiles;
+    int line = pos;
+    if (pos >= p.n_whole) {
+      const int n_cut = p.n_qtiles - p.n_whole;
+      part = (pos - p.n_whole) / n_cut;
+      line = pos - part * n_cut;
+    }
     qt = p.dense_causal ? p.n_qtiles - 1 - line : line;
     if (p.dense_causal) diag = qt + p.diag_off;          // key tile on the diagonal (may lie outside the rectangle)
     const int kend = p.dense_causal ? min(max(diag + 1, 0), p.n_ktiles) : p.n_ktiles;
-    e0 = min(part * p.part_len, kend);
-    e1 = min(e0 + p.part_len, kend);
+    e0 = part < 0 ? 0 : min(part * p.part_len, kend);
+    e1 = part < 0 ? kend : min(e0 + p.part_len, kend);
   } else {
     qt = min(max(sload(p.q_order, pos), 0), p.n_qtiles - 1);
     // list bounds are clamped to the arrays' extent: an inconsistent row_ptr cannot read beyond them
@@ -265,11 +271,19 @@ __global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void fwd_kernel(const
 
   // ---- epilogue: normalise, write O (bf16) and LSE (natural log) -------------------------
   float l_tot = xhalf_sum(st.l_run);
-  bf16* const orow = p.o + part * p.o_part + b * p.os.b + (int64_t)qrow0 * p.os.s + h * p.os.h;
+  bf16* orow = p.o + b * p.os.b + (int64_t)qrow0 * p.os.s + h * p.os.h;
+  float* lrow = p.lse + ((int64_t)b * p.n_heads + h) * ((int64_t)p.n_qtiles * kTile) + qrow0;
+  int64_t o_stride = p.os.s;
+  if (part >= 0) {
+    const int64_t seq = (int64_t)(p.n_qtiles - p.n_whole) * kTile, row = qrow0 - (int64_t)p.n_whole * kTile;
+    orow = p.part_o + part * p.o_part + ((b * seq + row) * p.n_heads + h) * kHeadDim;
+    lrow = p.part_lse + part * p.lse_part + ((int64_t)b * p.n_heads + h) * seq + row;
+    o_stride = (int64_t)p.n_heads * kHeadDim;
+  }
   auto lds_at = [](unsigned char* x) { return (uint32_t)(uintptr_t)(lds_byte*)x; };
   if constexpr (kGroups == 1) {
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-    store_rows_bf16(orow, p.os.s, oacc, inv, lds_at((wave < 2 ? kA : vA) + (wave & 1) * kWaveRowsBytes));   // everyone left stage A before the last step
+    store_rows_bf16(orow, o_stride, oacc, inv, lds_at((wave < 2 ? kA : vA) + (wave & 1) * kWaveRowsBytes));   // everyone left stage A before the last step
   } else {
     // the groups exchange their rows' max, sum and O.  Area x of the stages' LDS belongs to group x % kGroups of wave x / kGroups.
     __shared__ float stat[8][2][64];
@@ -297,17 +311,17 @@ __global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void fwd_kernel(const
     if constexpr (kAll) {
 #pragma unroll
       for (int mb = 0; mb < 4; ++mb) add_block(area(own + 1), mb, oacc[mb], w[0], w[1]);
-      store_rows_bf16(orow, p.os.s, oacc, inv, area(own + 1));
+      store_rows_bf16(orow, o_stride, oacc, inv, area(own + 1));
     } else {
       f32x16 o{0};
 #pragma unroll
       for (int g = 0; g < kGroups; ++g) add_block(area(wave * kGroups + g), group, o, 1.f, w[g]);
-      store_block_bf16(orow + 32 * group, p.os.s, o, inv, area(own) + 4096 * group);
+      store_block_bf16(orow + 32 * group, o_stride, o, inv, area(own) + 4096 * group);
     }
   }
   if (hi == 0 && group == 0) {
     const float lse = l_tot > 0.f ? (st.m_run + __builtin_amdgcn_logf(l_tot)) * kLn2 : -INFINITY;
-    p.lse[part * p.lse_part + ((int64_t)b * p.n_heads + h) * ((int64_t)p.n_qtiles * kTile) + qrow] = lse;
+    lrow[l32] = lse;
   }
 }
 
@@ -337,7 +351,8 @@ static int fwd_common(FwdParams& p, const void* q, const void* k, const void* v,
   p.scale_log2 = softmax_scale * kLog2e;
   const int nbh = batch * n_heads;
   p.heads_per_xcd = (nbh % 8 == 0) ? nbh / 8 : 0;
-  p.dense = 0; p.dense_causal = 0; p.diag_off = 0; p.n_parts = 1; p.part_len = n_ktiles; p.o_part = 0; p.lse_part = 0;
+  p.dense = 0; p.dense_causal = 0; p.diag_off = 0; p.n_whole = n_qtiles; p.n_parts = 1; p.part_len = n_ktiles;
+  p.part_o = nullptr; p.part_lse = nullptr; p.o_part = 0; p.lse_part = 0;
   return check_device();
 }
 
@@ -355,7 +370,7 @@ static int fwd_groups(int64_t n, int64_t walk, int n_parts, bool dense_causal) {
   return walk >= 3 && n <= (uneven ? 2 * kCus : kCus) ? 2 : 1;
 }
 static int fwd_launch(FwdParams& p, hipStream_t st) {
-  const unsigned n = (unsigned)(p.batch * p.n_heads * p.n_qtiles * p.n_parts);
+  const unsigned n = (unsigned)(p.batch * p.n_heads * (p.n_whole + (p.n_qtiles - p.n_whole) * p.n_parts));
   switch (fwd_groups(n, p.dense ? p.part_len : p.nnz / p.n_qtiles, p.n_parts, p.dense_causal)) {
     case 4: hipLaunchKernelGGL(fwd_kernel<4>, dim3(2 * n), dim3(512), 0, st, p); break;
     case 2: hipLaunchKernelGGL(fwd_kernel<2>, dim3(n), dim3(512), 0, st, p); break;
@@ -422,11 +437,43 @@ extern "C" int ua_bsa_fwd(const void* q, const void* k, const void* v, void* o, 
   return fwd_launch(p, (hipStream_t)stream);
 }
 
+namespace ua {
+
+// The last wave of a large rectangle.  Its lines run two to a CU, 512 at a time; up to 256 lines left over would hold
+// the launch open for a whole walk with most of the device idle (2304 x 3456, 32 heads: 576 lines of 27 tiles, 154 us, of
+// which 50 for the last 64 lines).  The left-over query tiles at the end of every sequence are then cut into parts
+// that fill the device, if the estimate of that and of their merge is shorter.  Causal rows balance themselves.
+struct Tail { int tiles, parts; };
+static Tail fwd_tail(int64_t nbh, int n_qtiles, int n_ktiles) {
+  constexpr int kRound = 2 * kCus;
+  const int64_t lines = nbh * n_qtiles, rounds = lines / kRound;
+  if (rounds == 0 || lines % kRound == 0 || lines % kRound > kCus) return {0, 1};
+  const int tail = n_qtiles - (int)(rounds * kRound / nbh);
+  const int64_t cut = nbh * tail;
+  const int64_t most = n_ktiles / 2 < UA_MAX_PARTS ? n_ktiles / 2 : UA_MAX_PARTS, parts = kRound / cut < most ? kRound / cut : most;
+  if (tail >= n_qtiles || parts < 2) return {0, 1};
+  const float us = 3.7f * cut * n_ktiles / kRound + 4.f + 2.4f + cut * parts * (kTile * kHeadDim * 2) / 1.5e6f;
+  return us < 2.2f * n_ktiles ? Tail{tail, (int)parts} : Tail{0, 1};
+}
+// Query tiles at the end that are cut, and into how many parts.
+static Tail dense_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int max_parts) {
+  if (max_parts == 1) return causal ? Tail{0, 1} : fwd_tail(nbh, n_qtiles, n_ktiles);
+  const int parts = fwd_cut(nbh, n_qtiles, n_ktiles, causal, max_parts);
+  return {parts > 1 ? n_qtiles : 0, parts};
+}
+
+}  // namespace ua
+
 extern "C" int64_t ua_dense_workspace_bytes(int batch, int n_heads, int seqlen_q, int seqlen_k, int backward) {
   using namespace ua;
   if (batch <= 0 || n_heads <= 0 || seqlen_q <= 0 || seqlen_k <= 0 || seqlen_q % kTile || seqlen_k % kTile) return 0;
-  const DenseSplit d = dense_split(batch, n_heads, seqlen_q / kTile, seqlen_k / kTile);
-  return backward ? d.bwd_total : d.fwd_total;
+  const int n_qtiles = seqlen_q / kTile, n_ktiles = seqlen_k / kTile;
+  const DenseSplit d = dense_split(batch, n_heads, n_qtiles, n_ktiles);
+  if (backward) return d.bwd_total;
+  if (d.fwd_parts > 1) return d.fwd_total;
+  const Tail t = fwd_tail((int64_t)batch * n_heads, n_qtiles, n_ktiles);
+  const DenseSplit dt = dense_split(batch, n_heads, t.tiles, n_ktiles);
+  return t.tiles ? t.parts * (dt.fwd_o_bytes + dt.fwd_lse_bytes) : 0;
 }
 
 extern "C" int ua_dense_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
@@ -442,23 +489,23 @@ extern "C" int ua_dense_fwd(const void* q, const void* k, const void* v, void* o
                           v_strides, o_strides, softmax_scale)) return rc;
   p.dense = 1; p.dense_causal = causal != 0; p.diag_off = n_ktiles - n_qtiles;
   hipStream_t st = (hipStream_t)stream;
-  const DenseSplit d = dense_split(batch, n_heads, n_qtiles, n_ktiles);
-  // the split path needs the caller's workspace and a contiguous output for the merge
-  const bool can_cut = d.fwd_parts > 1 && workspace && aligned16(workspace) && workspace_bytes >= d.fwd_total &&
-                       contiguous_bshd(o_strides, seqlen_q, n_heads);
-  const int cut = can_cut ? fwd_cut((int64_t)batch * n_heads, n_qtiles, n_ktiles, p.dense_causal, d.fwd_parts) : 1;
-  if (cut == 1) return fwd_launch(p, st);
-  const int len = (n_ktiles + cut - 1) / cut;
-  const int parts = (n_ktiles + len - 1) / len;
-  unsigned char* ws = static_cast<unsigned char*>(workspace);
-  p.o = reinterpret_cast<bf16*>(ws);
-  p.lse = reinterpret_cast<float*>(ws + (int64_t)parts * d.fwd_o_bytes);
+  const int max_parts = dense_split(batch, n_heads, n_qtiles, n_ktiles).fwd_parts;
+  const Tail cut = dense_cut((int64_t)batch * n_heads, n_qtiles, n_ktiles, p.dense_causal, max_parts);
+  if (cut.tiles == 0) return fwd_launch(p, st);
+  // cutting needs the caller's workspace and a contiguous output for the merge
+  const DenseSplit d = dense_split(batch, n_heads, cut.tiles, n_ktiles);             // sizes of one part
+  const int64_t need = cut.parts * (d.fwd_o_bytes + d.fwd_lse_bytes);
+  if (!workspace || !aligned16(workspace) || workspace_bytes < need || !contiguous_bshd(o_strides, seqlen_q, n_heads)) return fwd_launch(p, st);
+  p.n_whole = n_qtiles - cut.tiles;
+  p.part_len = (n_ktiles + cut.parts - 1) / cut.parts;
+  p.n_parts = (n_ktiles + p.part_len - 1) / p.part_len;
+  p.part_o = static_cast<bf16*>(workspace);
+  p.part_lse = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + p.n_parts * d.fwd_o_bytes);
   p.o_part = d.fwd_o_bytes / 2; p.lse_part = d.fwd_lse_bytes / 4;
-  p.os = {(int64_t)seqlen_q * n_heads * kHeadDim, (int64_t)n_heads * kHeadDim, kHeadDim};
-  p.n_parts = parts; p.part_len = len;
   if (int rc = fwd_launch(p, st)) return rc;
   const void* op[UA_MAX_PARTS];
   const float* lp[UA_MAX_PARTS];
-  for (int i = 0; i < parts; ++i) { op[i] = p.o + i * p.o_part; lp[i] = p.lse + i * p.lse_part; }
-  return ua_merge(op, lp, parts, o, lse, batch, seqlen_q, n_heads, head_dim, stream);
+  for (int i = 0; i < p.n_parts; ++i) { op[i] = p.part_o + i * p.o_part; lp[i] = p.part_lse + i * p.lse_part; }
+  const int64_t first = (int64_t)p.n_whole * kTile;
+  return merge_rows(op, lp, p.n_parts, p.o + first * n_heads * kHeadDim, lse + first, seqlen_q, batch, cut.tiles * kTile, n_heads, head_dim, stream);
 }

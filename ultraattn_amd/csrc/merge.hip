@@ -26,6 +26,7 @@ struct MergeParams {
   const float* lse_parts[UA_MAX_PARTS];
   bf16* o; float* lse;
   int n_parts, seqlen, n_heads, tok;           // tok: tokens per workgroup
+  int out_seq;                                 // tokens of o and lse, of which the partials' are the first seqlen
 };
 
 template <int P>
@@ -42,6 +43,7 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
   // thread per step, and the loads of step n+1 are issued before step n is combined, so that
   // P * kUnroll (..2x) 16-byte loads per thread are always in flight.
   const int64_t base = ((int64_t)b * p.seqlen + s0) * p.n_heads * kHeadDim;
+  const int64_t out_base = ((int64_t)b * p.out_seq + s0) * p.n_heads * kHeadDim;
   const int n_chunks = rows * 16;
   constexpr int kUnroll = P <= 4 ? 4 : (P <= 8 ? 2 : 1);
   constexpr int kStep = 256 * kUnroll;
@@ -76,7 +78,7 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
     const int row = sl * p.n_heads + h;
 #pragma unroll
     for (int i = 0; i < P; ++i) w_lds[i * rows + row] = l[i] * inv;
-    p.lse[li] = den > 0.f ? ms + __builtin_amdgcn_logf(den) * kLn2 : -INFINITY;
+    p.lse[((int64_t)b * p.n_heads + h) * p.out_seq + s0 + sl] = den > 0.f ? ms + __builtin_amdgcn_logf(den) * kLn2 : -INFINITY;
   }
   __syncthreads();
 
@@ -108,7 +110,7 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
       bf16x8 out;
 #pragma unroll
       for (int j = 0; j < 8; ++j) out[j] = (bf16)acc[j];
-      __builtin_nontemporal_store(out, reinterpret_cast<bf16x8*>(p.o + base) + c);
+      __builtin_nontemporal_store(out, reinterpret_cast<bf16x8*>(p.o + out_base) + c);
     }
   }
 }
@@ -252,11 +254,8 @@ static int launch_merge(const MergeParams& p, int blocks, size_t lds, hipStream_
   return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH;
 }
 
-}  // namespace ua
-
-extern "C" int ua_merge(const void* const* o_parts, const float* const* lse_parts, int n_parts,
-                        void* o, float* lse, int batch, int seqlen, int n_heads, int head_dim, void* stream) {
-  using namespace ua;
+int merge_rows(const void* const* o_parts, const float* const* lse_parts, int n_parts, void* o, float* lse, int out_seq, int batch, int seqlen,
+               int n_heads, int head_dim, void* stream) {
   if (!o_parts || !lse_parts || !o || !lse) return UA_ERR_NULL;
   if (n_parts < 1 || n_parts > UA_MAX_PARTS) return UA_ERR_UNSUPPORTED;
   if (head_dim != kHeadDim) return UA_ERR_UNSUPPORTED;
@@ -272,7 +271,7 @@ extern "C" int ua_merge(const void* const* o_parts, const float* const* lse_part
     p.lse_parts[i] = lse_parts[i];
   }
   for (int i = n_parts; i < UA_MAX_PARTS; ++i) { p.o_parts[i] = nullptr; p.lse_parts[i] = nullptr; }
-  p.o = (bf16*)o; p.lse = lse; p.n_parts = n_parts; p.seqlen = seqlen; p.n_heads = n_heads; p.tok = tok;
+  p.o = (bf16*)o; p.lse = lse; p.n_parts = n_parts; p.seqlen = seqlen; p.n_heads = n_heads; p.tok = tok; p.out_seq = out_seq;
   if (int rc = check_device()) return rc;
   const int blocks = batch * ((seqlen + tok - 1) / tok);
   const size_t lds = (size_t)n_parts * tok * n_heads * sizeof(float);
@@ -285,6 +284,13 @@ extern "C" int ua_merge(const void* const* o_parts, const float* const* lse_part
 #undef UA_CASE
   }
   return UA_ERR_UNSUPPORTED;
+}
+
+}  // namespace ua
+
+extern "C" int ua_merge(const void* const* o_parts, const float* const* lse_parts, int n_parts,
+                        void* o, float* lse, int batch, int seqlen, int n_heads, int head_dim, void* stream) {
+  return ua::merge_rows(o_parts, lse_parts, n_parts, o, lse, seqlen, batch, seqlen, n_heads, head_dim, stream);
 }
 
 extern "C" int ua_bsa_bwd_delta(const void* o, const void* dout, float* delta,

@@ -339,6 +339,9 @@ struct PartialSum {
   int n_parts, seqlen;
   Strides3 os;
 };
+// ua_merge into the first `seqlen` of `out_seq` tokens of o and lse (which may point into larger tensors).
+int merge_rows(const void* const* o_parts, const float* const* lse_parts, int n_parts, void* o, float* lse, int out_seq, int batch, int seqlen,
+               int n_heads, int head_dim, void* stream);
 int launch_partial_sums(const PartialSum* sums, int n_sums, int batch, int n_heads, hipStream_t st);
 
 }  // namespace ua
