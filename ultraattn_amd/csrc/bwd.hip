@@ -119,23 +119,6 @@ __device__ __forceinline__ bf16x8 lds_abs_tr_pair(uint32_t a_lo, uint32_t a_hi) 
   const bf16x4 y = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(reinterpret_cast<UA_LDS bf16x4*>(a_hi));
   return __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7);
 }
-// buffer_load_dwordx4 ... lds with the LDS destination (wave-uniform) in M0; see dma16_buf.
-// M0 is declared clobbered; "memory" is left out on purpose so that LDS reads of the other
-// stage may be scheduled across the copy (completion is awaited explicitly at the step's end).
-__device__ __forceinline__ void dma16_abs(u32x4 rsrc, uint32_t lds_addr, int voff, int soff) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               :: "s"(lds_addr), "v"(voff), "s"(rsrc), "s"(soff) : "m0");
-}
-__device__ __forceinline__ u32x4 make_rsrc_words(const void* base, uint32_t bytes) {
-  const uint64_t a = reinterpret_cast<uint64_t>(base);
-  u32x4 r;
-  r[0] = __builtin_amdgcn_readfirstlane((uint32_t)a);
-  r[1] = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffffu);
-  r[2] = __builtin_amdgcn_readfirstlane(bytes);
-  r[3] = 0x00020000u;
-  return r;
-}
-
 // Per-lane absolute LDS addresses within the first operand's half tile of stage 0; the second operand, later
 // rows and stage 1 are compile-time offsets.
 struct PairAddr {
@@ -323,13 +306,22 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block
   // (through the stage that the first step fills)
   const int k_block = S::kWaves * sub + wave, krow0 = kt * kTile + k_block * 32;
   bf16x8 kf[8], vf[8];
-  {
+  if constexpr (kGroups == 1) {
     u32x4 kraw[8], vraw[8];
     load_rows(kraw, p.k + b * p.ks.b + (int64_t)krow0 * p.ks.s + h * p.ks.h, p.ks.s);
     load_rows(vraw, p.v + b * p.vs.b + (int64_t)krow0 * p.vs.s + h * p.vs.h, p.vs.s);
     const uint32_t turn = lds_base + 2 * S::kPitch + wave * kWaveRowsBytes;
     rows_to_frags(kf, kraw, turn);
     rows_to_frags(vf, vraw, turn);
+  } else {
+    const int64_t line0 = (int64_t)kt * kTile + sub * 32 * S::kWaves;
+    const uint32_t k_lds = lds_block + 2 * S::kPitch, v_lds = k_lds + S::kBytes;           // stage 1 of groups 0 and 1
+    copy_shared_rows<32 * S::kWaves>(p.k + b * p.ks.b + line0 * p.ks.s + h * p.ks.h, (int)p.ks.s, k_lds);
+    copy_shared_rows<32 * S::kWaves>(p.v + b * p.vs.b + line0 * p.vs.s + h * p.vs.h, (int)p.vs.s, v_lds);
+    wait_vmem_all();
+    __syncthreads();
+    shared_rows_to_frags(kf, k_lds, wave);
+    shared_rows_to_frags(vf, v_lds, wave);
   }
   f32x16 dk[4], dv[4];
 #pragma unroll
@@ -509,13 +501,27 @@ __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_block, 
   const int q_block = S::kWaves * sub + wave, qrow0 = qt * kTile + q_block * 32, qrow = qrow0 + l32;
   bf16x8 qf[8], dof[8];
   u32x4 qraw[8], doraw[8];
-  load_rows(qraw, p.q + b * p.qs.b + (int64_t)qrow0 * p.qs.s + h * p.qs.h, p.qs.s);
-  load_rows(doraw, p.dout + b * p.ds.b + (int64_t)qrow0 * p.ds.s + h * p.ds.h, p.ds.s);
+  const uint32_t q_lds = lds_block + 2 * S::kPitch, do_lds = q_lds + S::kBytes;            // stage 1 of groups 0 and 1
+  if constexpr (kGroups == 1) {
+    load_rows(qraw, p.q + b * p.qs.b + (int64_t)qrow0 * p.qs.s + h * p.qs.h, p.qs.s);
+    load_rows(doraw, p.dout + b * p.ds.b + (int64_t)qrow0 * p.ds.s + h * p.ds.h, p.ds.s);
+  } else {
+    const int64_t line0 = (int64_t)qt * kTile + sub * 32 * S::kWaves;
+    copy_shared_rows<32 * S::kWaves>(p.q + b * p.qs.b + line0 * p.qs.s + h * p.qs.h, (int)p.qs.s, q_lds);
+    copy_shared_rows<32 * S::kWaves>(p.dout + b * p.ds.b + line0 * p.ds.s + h * p.ds.h, (int)p.ds.s, do_lds);
+  }
   const float lse_raw = p.lse[((int64_t)b * p.n_heads + h) * seq_q + qrow];
   const float neg_delta = -p.delta[((int64_t)b * p.n_heads + h) * seq_q + qrow];
-  const uint32_t turn = lds_base + 2 * S::kPitch + wave * kWaveRowsBytes;      // in the stage that the first step fills
-  rows_to_frags(qf, qraw, turn);
-  rows_to_frags(dof, doraw, turn);
+  if constexpr (kGroups == 1) {
+    const uint32_t turn = lds_base + 2 * S::kPitch + wave * kWaveRowsBytes;      // in the stage that the first step fills
+    rows_to_frags(qf, qraw, turn);
+    rows_to_frags(dof, doraw, turn);
+  } else {
+    wait_vmem_all();
+    __syncthreads();
+    shared_rows_to_frags(qf, q_lds, wave);
+    shared_rows_to_frags(dof, do_lds, wave);
+  }
   const float lse2 = (lse_raw == -INFINITY) ? INFINITY : lse_raw * kLog2e;
   f32x16 nd;
 #pragma unroll

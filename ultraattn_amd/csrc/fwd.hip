@@ -223,10 +223,18 @@ __global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void fwd_kernel(const
   const int q_local = q_block * 32 + l32;
   const int qrow0 = qt * kTile + q_block * 32, qrow = qrow0 + l32;
   bf16x8 qf[8];
-  {
+  if constexpr (kGroups == 1) {
     u32x4 raw[8];
     load_rows(raw, p.q + b * p.qs.b + (int64_t)qrow0 * p.qs.s + h * p.qs.h, p.qs.s);
-    rows_to_frags(qf, raw, (uint32_t)(uintptr_t)(lds_byte*)((wave < kWaves / 2 ? kB : vB) + wave % (kWaves / 2) * kWaveRowsBytes));
+    rows_to_frags(qf, raw, (uint32_t)(uintptr_t)(lds_byte*)((wave < 2 ? kB : vB) + (wave & 1) * kWaveRowsBytes));
+  } else {
+    const uint32_t q_lds = (uint32_t)(uintptr_t)(lds_byte*)sKB;
+    copy_shared_rows<32 * kWaves>(p.q + b * p.qs.b + ((int64_t)qt * kTile + sub * 32 * kWaves) * p.qs.s + h * p.qs.h, (int)p.qs.s, q_lds);
+    wait_vmem_all();
+    __syncthreads();
+    shared_rows_to_frags(qf, q_lds, wave);
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) asm volatile("" : "+v"(qf[ks]));      // read before the first step's barrier
   }
 
   f32x16 oacc[4];
@@ -371,7 +379,8 @@ static int fwd_groups(int64_t n, int64_t walk, int n_parts, bool dense_causal) {
 }
 static int fwd_launch(FwdParams& p, hipStream_t st) {
   const unsigned n = (unsigned)(p.batch * p.n_heads * (p.n_whole + (p.n_qtiles - p.n_whole) * p.n_parts));
-  switch (fwd_groups(n, p.dense ? p.part_len : p.nnz / p.n_qtiles, p.n_parts, p.dense_causal)) {
+  // (several groups copy Q through a buffer descriptor, whose offsets have 32 bits)
+  switch (p.qs.s > (INT32_MAX >> 9) ? 1 : fwd_groups(n, p.dense ? p.part_len : p.nnz / p.n_qtiles, p.n_parts, p.dense_causal)) {
     case 4: hipLaunchKernelGGL(fwd_kernel<4>, dim3(2 * n), dim3(512), 0, st, p); break;
     case 2: hipLaunchKernelGGL(fwd_kernel<2>, dim3(n), dim3(512), 0, st, p); break;
     default:

@@ -111,6 +111,43 @@ __device__ __forceinline__ void rows_to_frags(bf16x8 (&f)[8], const u32x4 (&raw)
 #pragma unroll
   for (int ks = 0; ks < 8; ++ks) f[ks] = lds_get<bf16x8>(lds + row_slot(lane & 31, 2 * ks + (lane >> 5)));
 }
+// buffer_load_dwordx4 ... lds with the LDS destination (wave-uniform) in M0; see dma16_buf.
+// M0 is declared clobbered; "memory" is left out on purpose so that LDS reads of the other
+// stage may be scheduled across the copy (completion is awaited explicitly at the step's end).
+__device__ __forceinline__ void dma16_abs(u32x4 rsrc, uint32_t lds_addr, int voff, int soff) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :: "s"(lds_addr), "v"(voff), "s"(rsrc), "s"(soff) : "m0");
+}
+__device__ __forceinline__ u32x4 make_rsrc_words(const void* base, uint32_t bytes) {
+  const uint64_t a = reinterpret_cast<uint64_t>(base);
+  u32x4 r;
+  r[0] = __builtin_amdgcn_readfirstlane((uint32_t)a);
+  r[1] = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffffu);
+  r[2] = __builtin_amdgcn_readfirstlane(bytes);
+  r[3] = 0x00020000u;
+  return r;
+}
+
+// Rows that all groups of a workgroup of 512 threads hold as B operands: copied once, straight into LDS in the same layout,
+// with wave w taking the fours of rows j with j % 4 == w % 4, whose source chunks then are one offset.  Every wave loading
+// its own, 128 KiB a workgroup, made the first loads of dK/dV last 3.4 us.
+template <int kRows>
+__device__ __forceinline__ void copy_shared_rows(const bf16* rows, int row_stride, uint32_t lds) {
+  const int lane = fresh_lane(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = 4 * (w & 3) + (lane >> 4);                  // row within 16
+  const int voff = (r * row_stride + ((lane & 15) ^ r) * 8) * 2;
+  const u32x4 rsrc = make_rsrc_words(rows, (uint32_t)((kRows - 1) * row_stride + kHeadDim) * 2);
+#pragma unroll
+  for (int i = 0; i < kRows / 32; ++i) {
+    const int sixteen = 2 * i + (w >> 2);
+    dma16_abs(rsrc, lds + (4 * sixteen + (w & 3)) * 1024, voff, sixteen * 32 * row_stride);
+  }
+}
+__device__ __forceinline__ void shared_rows_to_frags(bf16x8 (&f)[8], uint32_t lds, int block) {
+  const int lane = fresh_lane();
+#pragma unroll
+  for (int ks = 0; ks < 8; ++ks) f[ks] = lds_get<bf16x8>(lds + row_slot(32 * block + (lane & 31), 2 * ks + (lane >> 5)));
+}
 // acc[mb][4g + j] holds column 32 * mb + 8 * g + 4 * (lane / 32) + j of row lane % 32; written times `mul` as bf16.
 __device__ __forceinline__ void store_rows_bf16(bf16* rows, int64_t row_stride, const f32x16 (&acc)[4], float mul, uint32_t lds) {
   const int lane = fresh_lane();
