@@ -15,6 +15,7 @@
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -389,6 +390,13 @@ PyObject* lists_from_mask(PyObject* const* a) {
       return ua_tilelist_build(bytes, (int)nqb, (int)nkb, (int)rate, (int32_t*)l.row_ptr, (int32_t*)l.col_idx, (uint8_t*)l.flag, (int32_t*)l.col_ptr,
                                (int32_t*)l.row_idx, (uint8_t*)l.cflag, (int32_t*)l.q_order, (int32_t*)l.k_order);
     });
+    // Lists this short stay in the caches whatever the order, and few workgroups a CU make the longest sum of their
+    // walks count: longest first, which the kernels pair with the shortest where all of them are resident at once.
+    auto longest_first = [](const int32_t* ptr, const int32_t* order, int64_t n) {
+      std::stable_sort((int32_t*)order, (int32_t*)order + n, [ptr](int32_t i, int32_t j) { return ptr[i + 1] - ptr[i] > ptr[j + 1] - ptr[j]; });
+    };
+    longest_first(l.row_ptr, l.q_order, nqt);
+    longest_first(l.col_ptr, l.k_order, nkt);
     buf = to_device(host, (int)device);
   } else {
     const at::Tensor host = pinned(nqb * nkb, at::kByte);
