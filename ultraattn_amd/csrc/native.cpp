@@ -276,26 +276,36 @@ PyObject* dense_backward(PyObject* const* a) {
 }
 
 // Tile lists in one device buffer of 32-bit words: row_ptr, col_ptr, q_order, k_order, col_idx, row_idx, flag, cflag (the
-// flags four to a word), so that a list travels in one copy.
+// flags four to a word), so that a list travels in one copy.  Behind them may lie a second pair of launch orders, the
+// longest lines first, for launches of up to kShortLaunch lines: their operands stay in the caches in any order, and how
+// evenly the walks end decides.  Strided 8k, 16 heads: forward 135 -> 122 us; 32k, 8 heads: 452 -> 422; 64k: 1367 -> 1318
+// (4096 lines); from 8192 lines on the shared tiles of the first order win (32k, 32 heads: 1772, 1847).
+constexpr int64_t kShortLaunch = 4096;
 struct Lists {
-  int64_t at[9];             // first word of each array; at[8] = words in all
+  int64_t at[11];            // first word of each array; at[8] = words without, at[10] with the second orders
   const int32_t *row_ptr, *col_ptr, *q_order, *k_order, *col_idx, *row_idx;
   const uint8_t *flag, *cflag;
   Lists(int64_t nqt, int64_t nkt, int64_t nnz) {
     const int64_t words[8] = {nqt + 1, nkt + 1, nqt, nkt, nnz, nnz, (nnz + 3) / 4, (nnz + 3) / 4};
     at[0] = 0;
     for (int i = 0; i < 8; ++i) at[i + 1] = at[i] + words[i];
+    at[9] = at[8] + nqt;
+    at[10] = at[9] + nkt;
   }
   void point_into(const void* base) {
     const int32_t* p = (const int32_t*)base;
     row_ptr = p + at[0]; col_ptr = p + at[1]; q_order = p + at[2]; k_order = p + at[3]; col_idx = p + at[4]; row_idx = p + at[5];
     flag = (const uint8_t*)(p + at[6]); cflag = (const uint8_t*)(p + at[7]);
   }
-  Lists(PyObject* buf, int64_t nqt, int64_t nkt, int64_t nnz) : Lists(nqt, nkt, nnz) {
+  Lists(PyObject* buf, int64_t nqt, int64_t nkt, int64_t nnz, int64_t heads) : Lists(nqt, nkt, nnz) {
     const at::Tensor& t = tensor(buf, "tile list");
     if (nqt <= 0 || nkt <= 0 || nnz < 0 || !t.is_cuda() || t.scalar_type() != at::kInt || !t.is_contiguous() || t.numel() < at[8])
       fail(PyExc_ValueError, "the tile list must be a contiguous int32 CUDA tensor that holds all of its arrays");
     point_into(t.data_ptr());
+    if (t.numel() >= at[10]) {
+      if (heads * nqt <= kShortLaunch) q_order = (const int32_t*)t.data_ptr() + at[8];
+      if (heads * nkt <= kShortLaunch) k_order = (const int32_t*)t.data_ptr() + at[9];
+    }
   }
 };
 void check_grid(const at::Tensor& q, const at::Tensor& k, int64_t nqt, int64_t nkt) {
@@ -310,7 +320,7 @@ PyObject* bsa_forward(PyObject* const* a) {
   const at::Tensor &q = tensor(a[0], "q"), &k = tensor(a[1], "k"), &v = tensor(a[2], "v");
   check_qkv(q, k, v);
   const int64_t nqt = integer(a[4]), nkt = integer(a[5]), nnz = integer(a[6]);
-  const Lists l(a[3], nqt, nkt, nnz);
+  const Lists l(a[3], nqt, nkt, nnz, q.size(0) * q.size(2));
   check_grid(q, k, nqt, nkt);
   const float scale = scale_of(a[7]);
   Slot out(a[8]), lse(a[9]);
@@ -335,9 +345,9 @@ PyObject* bsa_forward(PyObject* const* a) {
 // bsa_backward(dout, q, k, v, out, lse, dq, dk, dv, softmax_d, lists, n_qtiles, n_ktiles, nnz, softmax_scale) -> (dq, dk, dv)
 PyObject* bsa_backward(PyObject* const* a) {
   const int64_t nqt = integer(a[11]), nkt = integer(a[12]), nnz = integer(a[13]);
-  const Lists l(a[10], nqt, nkt, nnz);
   const float scale = scale_of(a[14]);
   BwdArgs x(a, "lse");
+  const Lists l(a[10], nqt, nkt, nnz, x.q.size(0) * x.q.size(2));
   check_grid(x.q, x.k, nqt, nkt);
   x.allocate(a[4]);
   const On on(x.q);
@@ -384,19 +394,19 @@ PyObject* lists_from_mask(PyObject* const* a) {
   Lists l(nqt, nkt, nnz);
   at::Tensor buf;
   if (nnz <= kHostTiles) {
-    const at::Tensor host = pinned(l.at[8], at::kInt);
+    const at::Tensor host = pinned(l.at[10], at::kInt);
     l.point_into(host.data_ptr());
     call("ua_tilelist_build", [&] {
       return ua_tilelist_build(bytes, (int)nqb, (int)nkb, (int)rate, (int32_t*)l.row_ptr, (int32_t*)l.col_idx, (uint8_t*)l.flag, (int32_t*)l.col_ptr,
                                (int32_t*)l.row_idx, (uint8_t*)l.cflag, (int32_t*)l.q_order, (int32_t*)l.k_order);
     });
-    // Lists this short stay in the caches whatever the order, and few workgroups a CU make the longest sum of their
-    // walks count: longest first, which the kernels pair with the shortest where all of them are resident at once.
-    auto longest_first = [](const int32_t* ptr, const int32_t* order, int64_t n) {
-      std::stable_sort((int32_t*)order, (int32_t*)order + n, [ptr](int32_t i, int32_t j) { return ptr[i + 1] - ptr[i] > ptr[j + 1] - ptr[j]; });
+    auto longest_first = [&](const int32_t* ptr, int64_t to, int64_t n) {
+      int32_t* order = (int32_t*)host.data_ptr() + to;
+      for (int64_t i = 0; i < n; ++i) order[i] = (int32_t)i;
+      std::stable_sort(order, order + n, [ptr](int32_t i, int32_t j) { return ptr[i + 1] - ptr[i] > ptr[j + 1] - ptr[j]; });
     };
-    longest_first(l.row_ptr, l.q_order, nqt);
-    longest_first(l.col_ptr, l.k_order, nkt);
+    longest_first(l.row_ptr, l.at[8], nqt);
+    longest_first(l.col_ptr, l.at[9], nkt);
     buf = to_device(host, (int)device);
   } else {
     const at::Tensor host = pinned(nqb * nkb, at::kByte);

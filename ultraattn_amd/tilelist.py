@@ -58,17 +58,19 @@ class TileList:
                 raise RuntimeError("TileList.on(device) must be called once before the stream is captured into a graph")
             # one buffer (the layout that the native side expects) staged through pinned host memory and copied on
             # the current stream without a host synchronisation
-            size = {n: getattr(self, n).shape[0] for n in _PACKED}
-            words = {n: -(-c // 4) if n in ("flag", "cflag") else c for n, c in size.items()}
+            arrays = {n: getattr(self, n) for n in _PACKED}
+            for n, ptr in (("_q_long", self.row_ptr), ("_k_long", self.col_ptr)):      # second launch orders: longest lines first
+                arrays[n] = np.argsort(-np.diff(ptr), kind="stable").astype(np.int32)
+            words = {n: -(-a.shape[0] // 4) if n in ("flag", "cflag") else a.shape[0] for n, a in arrays.items()}
             host = torch.zeros(sum(words.values()), dtype=torch.int32, pin_memory=True)
             flat, at, dev = host.numpy(), 0, {}
             packed = torch.empty(host.shape, dtype=torch.int32, device=device)
-            for n in _PACKED:
+            for n, a in arrays.items():
                 part, on_dev = flat[at:at + words[n]], packed[at:at + words[n]]
                 if n in ("flag", "cflag"):
                     part, on_dev = part.view(np.uint8), on_dev.view(torch.uint8)
-                part[:size[n]] = getattr(self, n)
-                dev[n] = on_dev[:size[n]]
+                part[:a.shape[0]] = a
+                dev[n] = on_dev[:a.shape[0]]
                 at += words[n]
             packed.copy_(host, non_blocking=True)
             dev["_packed"], dev["_pinned"] = packed, host          # the host side is kept: the copy may still be in flight
@@ -85,7 +87,6 @@ class TileList:
             else:                           # a later use on another stream orders itself behind the copies
                 torch.cuda.current_stream().wait_event(ready)
         return dev
-
 
     def packed(self, device):
         """All arrays of ``on(device)`` as the one int32 tensor that they are views of."""
