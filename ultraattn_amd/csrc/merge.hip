@@ -308,18 +308,21 @@ extern "C" int ua_bsa_bwd_delta(const void* o, const void* dout, float* delta,
   p.os = {o_strides[0], o_strides[1], o_strides[2]};
   p.ds = {do_strides[0], do_strides[1], do_strides[2]};
   hipStream_t st = (hipStream_t)stream;
-  // A workgroup takes 32 rows at most: they are read in one round of loads, and a short sequence of many heads still
-  // gives every CU work.  512 tokens x 32 heads: 17.2 us at 16 tokens per workgroup, 3.2 at one; 32768 x 32: equal
-  // (86.3, 86.9: 6.2 TB/s).  With few heads more tokens share a workgroup, up to a 64-byte run of the result.
+  // Tokens per workgroup: four workgroups per CU as long as there are enough, so that a short sequence of many heads still
+  // gives every CU work (512 tokens x 32 heads: 19 us at 16 tokens, 3.4 at one), and from there on longer runs of the
+  // result, whose single values cost a memory transaction each (131072 x 32: 388 us at one token, 355 at 32; 32768 x 32:
+  // 87.5, 82.0 = 6.6 TB/s).  With few heads at least 32 rows, one round of loads.
   auto go = [&](auto tok) {
     constexpr int kT = decltype(tok)::value;
     hipLaunchKernelGGL(delta_kernel<kT>, dim3((unsigned)(batch * (((int64_t)seqlen_q + kT - 1) / kT))), dim3(256), (size_t)kT * n_heads * sizeof(float), st, p);
   };
-  if (n_heads <= 2)       go(std::integral_constant<int, 16>{});
-  else if (n_heads <= 4)  go(std::integral_constant<int, 8>{});
-  else if (n_heads <= 8)  go(std::integral_constant<int, 4>{});
-  else if (n_heads <= 16) go(std::integral_constant<int, 2>{});
-  else                    go(std::integral_constant<int, 1>{});
+  int tok = n_heads <= 2 ? 16 : (n_heads <= 4 ? 8 : (n_heads <= 8 ? 4 : (n_heads <= 16 ? 2 : 1)));
+  while (tok < 32 && (int64_t)batch * seqlen_q >= 2 * tok * (int64_t)(4 * kCus)) tok *= 2;
+  switch (tok) {
+#define UA_CASE(N) case N: go(std::integral_constant<int, N>{}); break;
+    UA_CASE(1) UA_CASE(2) UA_CASE(4) UA_CASE(8) UA_CASE(16) UA_CASE(32)
+#undef UA_CASE
+  }
   return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH;
 }
 
