@@ -28,9 +28,10 @@ struct FwdParams {
   // dense_causal [0, qt + diag_off] with the last one causal; longest rows first.  The first n_whole query tiles (all
   // if nothing is cut) are walked whole; the key range of the others is cut into n_parts parts of part_len tiles, and
   // part i leaves its partial (O, LSE), contiguous over those n_qtiles - n_whole tiles, at part_o + i * o_part and
-  // part_lse + i * lse_part (elements).
+  // part_lse + i * lse_part (elements).  Beside whole tiles the partial O is fp32, so that every row of a result is
+  // rounded to bf16 once; where everything is cut it is bf16.
   int dense, dense_causal, diag_off, n_whole, n_parts, part_len;
-  bf16* part_o; float* part_lse;
+  void* part_o; float* part_lse;
   int64_t o_part, lse_part;
 };
 
@@ -283,16 +284,20 @@ __global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void fwd_kernel(const
   bf16* orow = p.o + b * p.os.b + (int64_t)qrow0 * p.os.s + h * p.os.h;
   float* lrow = p.lse + ((int64_t)b * p.n_heads + h) * ((int64_t)p.n_qtiles * kTile) + qrow0;
   int64_t o_stride = p.os.s;
+  int64_t part_at = 0;                     // element of the partial O
   if (part >= 0) {
     const int64_t seq = (int64_t)(p.n_qtiles - p.n_whole) * kTile, row = qrow0 - (int64_t)p.n_whole * kTile;
-    orow = p.part_o + part * p.o_part + ((b * seq + row) * p.n_heads + h) * kHeadDim;
+    part_at = part * p.o_part + ((b * seq + row) * p.n_heads + h) * kHeadDim;
+    orow = static_cast<bf16*>(p.part_o) + part_at;
     lrow = p.part_lse + part * p.lse_part + ((int64_t)b * p.n_heads + h) * seq + row;
     o_stride = (int64_t)p.n_heads * kHeadDim;
   }
   auto lds_at = [](unsigned char* x) { return (uint32_t)(uintptr_t)(lds_byte*)x; };
   if constexpr (kGroups == 1) {
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-    store_rows_bf16(orow, o_stride, oacc, inv, lds_at((wave < 2 ? kA : vA) + (wave & 1) * kWaveRowsBytes));   // everyone left stage A before the last step
+    const uint32_t turn = lds_at((wave < 2 ? kA : vA) + (wave & 1) * kWaveRowsBytes);   // everyone left stage A before the last step
+    if (part >= 0 && p.n_whole > 0) store_rows_f32(static_cast<float*>(p.part_o) + part_at, o_stride, oacc, inv, turn);
+    else                            store_rows_bf16(orow, o_stride, oacc, inv, turn);
   } else {
     // the groups exchange their rows' max, sum and O.  Area x of the stages' LDS belongs to group x % kGroups of wave x / kGroups.
     __shared__ float stat[8][2][64];
@@ -450,9 +455,12 @@ extern "C" int ua_bsa_fwd(const void* q, const void* k, const void* v, void* o, 
 namespace ua {
 
 // The last wave of a large rectangle.  Its lines run two to a CU, 512 at a time; up to 256 lines left over would hold
-// the launch open for a whole walk with most of the device idle (2304 x 3456, 32 heads: 576 lines of 27 tiles, 154 us, of
-// which 50 for the last 64 lines).  The left-over query tiles at the end of every sequence are then cut into parts
-// that fill the device, if the estimate of that and of their merge is shorter.  Causal rows balance themselves.
+// the launch open for a whole walk with most of the device idle (2304 x 3456, 32 heads: 576 lines of 27 tiles, 149 us, of
+// which 50 for the last 64 lines; cut 129).  The left-over query tiles at the end of every sequence are then cut into parts
+// that fill the device, if the estimate of that and of their merge is shorter: the fp32 partials take 1 us per 2.5 MB
+// (2560 x 2048, 32 heads, 128 lines over: 91.2 us, cut 89.1; 3072 x 2048, 256 over: 97, cut in two 103, not done).  bf16
+// partials took up to 3 us less at the first shape and gave the rows of the last wave a second rounding, an error 20 % larger
+// than their neighbours'.  Causal rows balance themselves.
 struct Tail { int tiles, parts; };
 static Tail fwd_tail(int64_t nbh, int n_qtiles, int n_ktiles) {
   constexpr int kRound = 2 * kCus;
@@ -462,8 +470,17 @@ static Tail fwd_tail(int64_t nbh, int n_qtiles, int n_ktiles) {
   const int64_t cut = nbh * tail;
   const int64_t most = n_ktiles / 2 < UA_MAX_PARTS ? n_ktiles / 2 : UA_MAX_PARTS, parts = kRound / cut < most ? kRound / cut : most;
   if (tail >= n_qtiles || parts < 2) return {0, 1};
-  const float us = 3.7f * cut * n_ktiles / kRound + 4.f + 2.4f + cut * parts * (kTile * kHeadDim * 2) / 1.5e6f;
+  const float us = 3.7f * cut * n_ktiles / kRound + 4.f + 2.4f + cut * parts * (kTile * kHeadDim * 4) / 2.5e6f;
   return us < 2.2f * n_ktiles ? Tail{tail, (int)parts} : Tail{0, 1};
+}
+// One part's share of the workspace for n_tiles cut query tiles.
+struct PartBytes {
+  int64_t o, lse;
+  int64_t total() const { return o + lse; }
+};
+static PartBytes part_bytes(int batch, int n_heads, int n_tiles, bool f32) {
+  const int64_t rows = (int64_t)batch * n_heads * n_tiles * kTile;
+  return {align256(rows * kHeadDim * (f32 ? 4 : 2)), align256(rows * 4)};
 }
 // Query tiles at the end that are cut, and into how many parts.
 static Tail dense_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int max_parts) {
@@ -482,8 +499,7 @@ extern "C" int64_t ua_dense_workspace_bytes(int batch, int n_heads, int seqlen_q
   if (backward) return d.bwd_total;
   if (d.fwd_parts > 1) return d.fwd_total;
   const Tail t = fwd_tail((int64_t)batch * n_heads, n_qtiles, n_ktiles);
-  const DenseSplit dt = dense_split(batch, n_heads, t.tiles, n_ktiles);
-  return t.tiles ? t.parts * (dt.fwd_o_bytes + dt.fwd_lse_bytes) : 0;
+  return t.tiles ? t.parts * part_bytes(batch, n_heads, t.tiles, true).total() : 0;
 }
 
 extern "C" int ua_dense_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
@@ -503,19 +519,24 @@ extern "C" int ua_dense_fwd(const void* q, const void* k, const void* v, void* o
   const Tail cut = dense_cut((int64_t)batch * n_heads, n_qtiles, n_ktiles, p.dense_causal, max_parts);
   if (cut.tiles == 0) return fwd_launch(p, st);
   // cutting needs the caller's workspace and a contiguous output for the merge
-  const DenseSplit d = dense_split(batch, n_heads, cut.tiles, n_ktiles);             // sizes of one part
-  const int64_t need = cut.parts * (d.fwd_o_bytes + d.fwd_lse_bytes);
+  const bool beside_whole = cut.tiles < n_qtiles;
+  const PartBytes d = part_bytes(batch, n_heads, cut.tiles, beside_whole);
+  const int64_t need = cut.parts * d.total();
   if (!workspace || !aligned16(workspace) || workspace_bytes < need || !contiguous_bshd(o_strides, seqlen_q, n_heads)) return fwd_launch(p, st);
   p.n_whole = n_qtiles - cut.tiles;
   p.part_len = (n_ktiles + cut.parts - 1) / cut.parts;
   p.n_parts = (n_ktiles + p.part_len - 1) / p.part_len;
-  p.part_o = static_cast<bf16*>(workspace);
-  p.part_lse = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + p.n_parts * d.fwd_o_bytes);
-  p.o_part = d.fwd_o_bytes / 2; p.lse_part = d.fwd_lse_bytes / 4;
+  p.part_o = workspace;
+  p.part_lse = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + p.n_parts * d.o);
+  p.o_part = d.o / (beside_whole ? 4 : 2); p.lse_part = d.lse / 4;
   if (int rc = fwd_launch(p, st)) return rc;
+  if (beside_whole) {
+    const int64_t first = (int64_t)p.n_whole * kTile;
+    return merge_f32_rows((const float*)p.part_o, p.o_part, p.part_lse, p.lse_part, p.n_parts, p.o + first * n_heads * kHeadDim, lse + first, seqlen_q,
+                          batch, cut.tiles * kTile, n_heads, st);
+  }
   const void* op[UA_MAX_PARTS];
   const float* lp[UA_MAX_PARTS];
-  for (int i = 0; i < p.n_parts; ++i) { op[i] = p.part_o + i * p.o_part; lp[i] = p.part_lse + i * p.lse_part; }
-  const int64_t first = (int64_t)p.n_whole * kTile;
-  return merge_rows(op, lp, p.n_parts, p.o + first * n_heads * kHeadDim, lse + first, seqlen_q, batch, cut.tiles * kTile, n_heads, head_dim, stream);
+  for (int i = 0; i < p.n_parts; ++i) { op[i] = (const bf16*)p.part_o + i * p.o_part; lp[i] = p.part_lse + i * p.lse_part; }
+  return ua_merge(op, lp, p.n_parts, p.o, lse, batch, seqlen_q, n_heads, head_dim, stream);
 }

@@ -26,7 +26,6 @@ struct MergeParams {
   const float* lse_parts[UA_MAX_PARTS];
   bf16* o; float* lse;
   int n_parts, seqlen, n_heads, tok;           // tok: tokens per workgroup
-  int out_seq;                                 // tokens of o and lse, of which the partials' are the first seqlen
 };
 
 template <int P>
@@ -43,7 +42,6 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
   // thread per step, and the loads of step n+1 are issued before step n is combined, so that
   // P * kUnroll (..2x) 16-byte loads per thread are always in flight.
   const int64_t base = ((int64_t)b * p.seqlen + s0) * p.n_heads * kHeadDim;
-  const int64_t out_base = ((int64_t)b * p.out_seq + s0) * p.n_heads * kHeadDim;
   const int n_chunks = rows * 16;
   constexpr int kUnroll = P <= 4 ? 4 : (P <= 8 ? 2 : 1);
   constexpr int kStep = 256 * kUnroll;
@@ -78,7 +76,7 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
     const int row = sl * p.n_heads + h;
 #pragma unroll
     for (int i = 0; i < P; ++i) w_lds[i * rows + row] = l[i] * inv;
-    p.lse[((int64_t)b * p.n_heads + h) * p.out_seq + s0 + sl] = den > 0.f ? ms + __builtin_amdgcn_logf(den) * kLn2 : -INFINITY;
+    p.lse[li] = den > 0.f ? ms + __builtin_amdgcn_logf(den) * kLn2 : -INFINITY;
   }
   __syncthreads();
 
@@ -110,9 +108,53 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
       bf16x8 out;
 #pragma unroll
       for (int j = 0; j < 8; ++j) out[j] = (bf16)acc[j];
-      __builtin_nontemporal_store(out, reinterpret_cast<bf16x8*>(p.o + out_base) + c);
+      __builtin_nontemporal_store(out, reinterpret_cast<bf16x8*>(p.o + base) + c);
     }
   }
+}
+
+// fp32 partials of the last `seqlen` query rows of every sequence (what the last wave of a large dense forward leaves), into
+// rows of a bf16 tensor and statistics of out_seq tokens.  They were just written and come from the memory-side cache; with
+// 16 lanes per row and every load issued first (beyond n_parts the last part again, weight 0), a workgroup waits once.
+struct MergeF32Params {
+  const float* o_parts; const float* lse_parts;
+  int64_t o_part, lse_part;                    // elements from part to part
+  bf16* o; float* lse;
+  int n_parts, seqlen, n_heads, out_seq, rows;
+};
+template <int P>
+__global__ __launch_bounds__(256) void merge_f32_kernel(const MergeF32Params p) {
+  const int row = blockIdx.x * 16 + (threadIdx.x >> 4), sub = threadIdx.x & 15;
+  if (row >= p.rows) return;
+  const int h = row % p.n_heads, t = row / p.n_heads, s = t % p.seqlen, b = t / p.seqlen;
+  const float* src = p.o_parts + (int64_t)row * kHeadDim + sub * 8;
+  const float* stat = p.lse_parts + ((int64_t)b * p.n_heads + h) * p.seqlen + s;
+  float l[P], m = -INFINITY, den = 0.f;
+  f32x4 x[P][2];
+#pragma unroll
+  for (int i = 0; i < P; ++i) l[i] = stat[min(i, p.n_parts - 1) * p.lse_part];
+#pragma unroll
+  for (int i = 0; i < P; ++i)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) x[i][u] = *reinterpret_cast<const f32x4*>(src + min(i, p.n_parts - 1) * p.o_part + 4 * u);
+#pragma unroll
+  for (int i = 0; i < P; ++i) m = fmaxf(m, l[i]);
+  const float ms = (m == -INFINITY) ? 0.f : m;
+  f32x4 sum[2] = {f32x4{0}, f32x4{0}};
+#pragma unroll
+  for (int i = 0; i < P; ++i) {
+    const float w = i < p.n_parts ? fast_exp2((l[i] - ms) * kLog2e) : 0.f;
+    den += w;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) sum[u] += x[i][u] * w;
+  }
+  const float inv = den > 0.f ? 1.f / den : 0.f;
+  const int64_t out_row = ((int64_t)b * p.out_seq + s) * p.n_heads + h;
+  bf16x8 w;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) w[j] = (bf16)(sum[j >> 2][j & 3] * inv);
+  *reinterpret_cast<bf16x8*>(p.o + out_row * kHeadDim + sub * 8) = w;
+  if (sub == 0) p.lse[((int64_t)b * p.n_heads + h) * p.out_seq + s] = den > 0.f ? ms + __builtin_amdgcn_logf(den) * kLn2 : -INFINITY;
 }
 
 struct DeltaParams {
@@ -254,8 +296,21 @@ static int launch_merge(const MergeParams& p, int blocks, size_t lds, hipStream_
   return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH;
 }
 
-int merge_rows(const void* const* o_parts, const float* const* lse_parts, int n_parts, void* o, float* lse, int out_seq, int batch, int seqlen,
-               int n_heads, int head_dim, void* stream) {
+int merge_f32_rows(const float* o_parts, int64_t o_part, const float* lse_parts, int64_t lse_part, int n_parts, bf16* o, float* lse, int out_seq,
+                   int batch, int seqlen, int n_heads, hipStream_t st) {
+  const MergeF32Params p = {o_parts, lse_parts, o_part, lse_part, o, lse, n_parts, seqlen, n_heads, out_seq, batch * seqlen * n_heads};
+  const dim3 grid((p.rows + 15) / 16);
+  if (n_parts <= 4)      hipLaunchKernelGGL(merge_f32_kernel<4>, grid, dim3(256), 0, st, p);
+  else if (n_parts <= 8) hipLaunchKernelGGL(merge_f32_kernel<8>, grid, dim3(256), 0, st, p);
+  else                   hipLaunchKernelGGL(merge_f32_kernel<UA_MAX_PARTS>, grid, dim3(256), 0, st, p);
+  return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH;
+}
+
+}  // namespace ua
+
+extern "C" int ua_merge(const void* const* o_parts, const float* const* lse_parts, int n_parts,
+                        void* o, float* lse, int batch, int seqlen, int n_heads, int head_dim, void* stream) {
+  using namespace ua;
   if (!o_parts || !lse_parts || !o || !lse) return UA_ERR_NULL;
   if (n_parts < 1 || n_parts > UA_MAX_PARTS) return UA_ERR_UNSUPPORTED;
   if (head_dim != kHeadDim) return UA_ERR_UNSUPPORTED;
@@ -271,7 +326,7 @@ int merge_rows(const void* const* o_parts, const float* const* lse_parts, int n_
     p.lse_parts[i] = lse_parts[i];
   }
   for (int i = n_parts; i < UA_MAX_PARTS; ++i) { p.o_parts[i] = nullptr; p.lse_parts[i] = nullptr; }
-  p.o = (bf16*)o; p.lse = lse; p.n_parts = n_parts; p.seqlen = seqlen; p.n_heads = n_heads; p.tok = tok; p.out_seq = out_seq;
+  p.o = (bf16*)o; p.lse = lse; p.n_parts = n_parts; p.seqlen = seqlen; p.n_heads = n_heads; p.tok = tok;
   if (int rc = check_device()) return rc;
   const int blocks = batch * ((seqlen + tok - 1) / tok);
   const size_t lds = (size_t)n_parts * tok * n_heads * sizeof(float);
@@ -284,13 +339,6 @@ int merge_rows(const void* const* o_parts, const float* const* lse_parts, int n_
 #undef UA_CASE
   }
   return UA_ERR_UNSUPPORTED;
-}
-
-}  // namespace ua
-
-extern "C" int ua_merge(const void* const* o_parts, const float* const* lse_parts, int n_parts,
-                        void* o, float* lse, int batch, int seqlen, int n_heads, int head_dim, void* stream) {
-  return ua::merge_rows(o_parts, lse_parts, n_parts, o, lse, seqlen, batch, seqlen, n_heads, head_dim, stream);
 }
 
 extern "C" int ua_bsa_bwd_delta(const void* o, const void* dout, float* delta,

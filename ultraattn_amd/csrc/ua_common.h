@@ -376,9 +376,10 @@ struct PartialSum {
   int n_parts, seqlen;
   Strides3 os;
 };
-// ua_merge into the first `seqlen` of `out_seq` tokens of o and lse (which may point into larger tensors).
-int merge_rows(const void* const* o_parts, const float* const* lse_parts, int n_parts, void* o, float* lse, int out_seq, int batch, int seqlen,
-               int n_heads, int head_dim, void* stream);
+// Merge of fp32 partials, part i at o_parts + i * o_part and lse_parts + i * lse_part (contiguous [batch, seqlen, n_heads, 128] and
+// [batch, n_heads, seqlen]), into the first `seqlen` of `out_seq` tokens of o and lse, which may point into larger tensors.
+int merge_f32_rows(const float* o_parts, int64_t o_part, const float* lse_parts, int64_t lse_part, int n_parts, bf16* o, float* lse, int out_seq,
+                   int batch, int seqlen, int n_heads, hipStream_t st);
 int launch_partial_sums(const PartialSum* sums, int n_sums, int batch, int n_heads, hipStream_t st);
 
 }  // namespace ua
