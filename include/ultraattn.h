@@ -129,7 +129,8 @@ int ua_tilelist_build_device_noalloc(const uint8_t *block_mask, int n_qblocks, i
  * out=)` launches of fwd_comp_func (orchestrated_attn/orchestrated_attn_impl.py:320-338; same
  * call hierarchy_attn/hierarchy_attn_impl.py:40-53) by one launch over the tile list.
  * Writes o (bf16) and lse (fp32) for every query row; rows without an active tile get o = 0,
- * lse = -inf.                                                                               */
+ * lse = -inf.  A row's result depends on its list alone: a launch over some of the heads or some of
+ * the rows gives bit for bit what the whole gives (so do dq, dk and dv below).                 */
 int ua_bsa_fwd(const void *q, const void *k, const void *v, void *o, float *lse,
                const int32_t *row_ptr, const int32_t *col_idx, const uint8_t *flag,
                const int32_t *q_order,
@@ -185,15 +186,20 @@ int ua_bsa_bwd(const void *q, const void *k, const void *v, const void *dout,
  * with no tile list: the kernels enumerate the tiles themselves.  causal != 0 aligns the diagonal
  * to the bottom-right corner as flash-attn >= 2.1 does (query i sees key j iff
  * j <= i + seqlen_k - seqlen_q; rows that see no key get o = 0, lse = -inf, zero gradients).
- * Rectangles with few tile lines (B * Nh * seqlen / 128 well below two workgroups per CU) and long
- * walks are cut into up to UA_MAX_PARTS parts that run as workgroups of their own: the forward
- * leaves partial (O, LSE) and finishes with ua_merge's kernel, the backward leaves fp32 partial
- * dQ (parts of the key range) and dK, dV (parts of the query range) and sums them in one pass.
+ * Rectangles with few tile lines (B * Nh * seqlen / 128 well below two workgroups per CU) run with
+ * several groups of wavefronts per line, and where their walks are long they are cut into up to
+ * UA_MAX_PARTS parts that run as workgroups of their own: the forward leaves partial (O, LSE) and
+ * finishes with ua_merge's kernel, the backward leaves fp32 partial dQ (parts of the key range) and
+ * dK, dV (parts of the query range) and sums them in one pass.  Of a large forward that is not
+ * causal only the last query tiles are cut, those left over after the last full wave of workgroups;
+ * their partial O is fp32.
  * The partials live in `workspace` (device memory, 16-byte aligned, caller-owned, overwritten by
- * every call: calls that share it must not overlap); ua_dense_workspace_bytes() gives the size
- * that lets a shape split (0 = it never splits).  With workspace == NULL or too small, or a
- * forward output that is not contiguous, the call runs unsplit: same results, one workgroup per
- * line.                                                                                       */
+ * every call: calls that share it must not overlap); ua_dense_workspace_bytes() gives a size
+ * that lets a shape split, causal or not (0 = it never splits).  With a workspace that is too small
+ * (any pointer with workspace_bytes = 0 included) or a forward output that is not contiguous nothing
+ * is cut.  The last bits of a row then depend on the launch, i.e. on how many rows and heads run
+ * with it.  With workspace == NULL every line is walked whole by one group: the results are those
+ * of ua_bsa_fwd / ua_bsa_bwd over the rectangle's tile list, bit for bit.                        */
 int64_t ua_dense_workspace_bytes(int batch, int n_heads, int seqlen_q, int seqlen_k, int backward);
 int ua_dense_fwd(const void *q, const void *k, const void *v, void *o, float *lse,
                  int batch, int n_heads, int seqlen_q, int seqlen_k, int head_dim,

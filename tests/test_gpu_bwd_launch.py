@@ -1,6 +1,7 @@
 """The backward's two sides in one launch (ua_bsa_bwd) equal the two separate launches bit for bit: the
 same walks, whatever shares a CU with them.  Masks with one tile, empty lines, more columns than rows and
-causal tiles; head counts on both sides of the XCD mapping."""
+causal tiles; head counts on both sides of the XCD mapping; up to 256 lines on both sides together, up to 512 (where the
+one launch takes the columns in reverse) and beyond."""
 import numpy as np
 import pytest
 import torch
@@ -18,6 +19,10 @@ DEV = "cuda:0"
     (np.zeros((2, 3), np.uint8), 3, 1),
     (masks.config_strided(9, 2, 4), 5, 2),
     (masks.config_streaming_shard(3, 11, 2), 8, 1),
+    (masks.config_strided(16, 2, 4), 8, 1),                      # 256 lines
+    (masks.config_causal(17), 8, 1),                             # 272
+    (masks.config_global_local(16), 16, 1),                      # 512
+    (masks.config_strided(17, 2, 4), 8, 2),                      # 544
 ])
 def test_one_launch_equals_two(lib, mask, nh, batch):
     g = torch.Generator(device=DEV).manual_seed(nh)

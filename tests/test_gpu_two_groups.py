@@ -1,5 +1,6 @@
-"""Workgroups of two and four groups that share a tile line: walks of no tile, one tile and an odd number of them, rows whose
-causal tile is not the last one, and launches on both sides of every bound at which the groups are chosen."""
+"""Workgroups of one, two and four groups per tile line: walks of no tile, one tile and an odd number of them, rows whose
+causal tile is not the last one (tile lists, one group), and dense launches on both sides of every bound at which the
+groups are chosen."""
 import numpy as np
 import pytest
 import torch
@@ -52,6 +53,9 @@ def test_short_and_odd_walks(mask):
     (128, 256, 256, True), (384, 128, 86, False),                # forward: 256 and 258
     (2048, 2048, 16, True), (2048, 2048, 17, True),              # causal, long walks: 512 and 544 in the backward
     (2176, 1920, 9, True),                                       # 153 rows, 135 columns, bottom-right aligned
+    (128, 384, 100, False), (128, 384, 150, False),              # walks of three: four groups and two
+    (640, 384, 20, True),                                        # four groups, walks of none to three
+    (1920, 1920, 17, True),                                      # two groups, walks of one to fifteen
 ])
 def test_around_the_bounds(sq, sk, nh, causal):
     q, k, v, do = _inputs(sq, sk, nh)

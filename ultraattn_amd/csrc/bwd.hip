@@ -233,7 +233,7 @@ __device__ __forceinline__ void dkdv_block(const PairAddr& ad, uint32_t stat, co
   }
 }
 
-// kGroups = 2 (here and for dQ): two groups of four wavefronts share the workgroup's line, one takes the first half of every
+// kGroups = 2 (here and for dQ; dense rectangles only, as 4): two groups of four wavefronts share the workgroup's line, one takes the first half of every
 // tile, the other the second, each through stages of its own; the results are added through LDS.  kGroups = 4: four groups
 // of two wavefronts share half a tile's rows, each takes a block of 32 of every tile.  Where the launch
 // gives a CU one workgroup at most, one wave per SIMD would leave the matrix pipe idle between its dependent steps (2.2 us
@@ -250,8 +250,9 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block
   const int sub = pos % S::kLines;         // which half of the tile's keys
   pos /= S::kLines;
   const int b = bh / p.n_heads, h = bh % p.n_heads;
+  const bool dense = kGroups > 1 || p.dense;
   int kt, e0, e1, diag = -1, part = 0;
-  if (p.dense) {
+  if (dense) {
     part = pos / p.n_ktiles;
     kt = pos - part * p.n_ktiles;                          // column 0 is the longest of a causal rectangle
     if (p.cols_reversed) kt = p.n_ktiles - 1 - kt;
@@ -274,7 +275,7 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block
   auto entry = [&](int i) {           // query tile | causal flag << 30
     if (n_half == 0) return 0;        // an empty column owns no list entry (the arrays may be NULL)
     const int e = min(e0 + (kGroups == 1 ? i >> 1 : i), e1 - 1);
-    if (p.dense) return e | ((int)(e == diag) << 30);      // the entry is the query tile itself
+    if (dense) return e | ((int)(e == diag) << 30);      // the entry is the query tile itself
     return min(max(sload(p.cols.idx, e), 0), p.n_qtiles - 1) | (sload(p.cols.flag, e) << 30);
   };
   // rows' statistics, staged in the form the accumulators start from: threads 0..kRows-1 carry
@@ -476,8 +477,9 @@ __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_block, 
   pos /= S::kLines;
   const int b = bh / p.n_heads, h = bh % p.n_heads;
   const int64_t seq_q = (int64_t)p.n_qtiles * kTile;
+  const bool dense = kGroups > 1 || p.dense;
   int qt, e0, e1, diag = -1, part = 0;
-  if (p.dense) {
+  if (dense) {
     part = pos / p.n_qtiles;
     const int line = pos - part * p.n_qtiles;
     qt = p.dense_causal ? p.n_qtiles - 1 - line : line;    // longest rows first
@@ -491,8 +493,8 @@ __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_block, 
     e1 = min(max(sload(p.rows.ptr, qt + 1), e0), p.nnz);
   }
   const PairStream<kGroups> in(p.k + b * p.ks.b + h * p.ks.h, (int)p.ks.s, p.v + b * p.vs.b + h * p.vs.h, (int)p.vs.s, lds_base, wave, lane);
-  auto ktile = [&](int e) { return p.dense ? e : min(max(sload(p.rows.idx, e), 0), p.n_ktiles - 1); };
-  auto is_causal = [&](int e) { return p.dense ? (int)(e == diag) : sload(p.rows.flag, e); };
+  auto ktile = [&](int e) { return dense ? e : min(max(sload(p.rows.idx, e), 0), p.n_ktiles - 1); };
+  auto is_causal = [&](int e) { return dense ? (int)(e == diag) : sload(p.rows.flag, e); };
 
   const int n_steps = (kGroups == 1 ? 2 : 1) * (e1 - e0);          // half tiles, as in dK/dV's walk
   int kt = e0 < e1 ? ktile(e0) : 0;
@@ -594,15 +596,13 @@ __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_block, 
 }
 
 // ---- kernels ------------------------------------------------------------------------------------
-template <int kGroups>
-__global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void dkdv_kernel(const BwdParams p) {
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[kGroups * Stages<kGroups>::kBytes];
-  dkdv_walk<kGroups>(p, (uint32_t)(uintptr_t)(UA_LDS unsigned char*)smem, blockIdx.x);
+__global__ __launch_bounds__(Groups<1>::kThreads, 2) void dkdv_kernel(const BwdParams p) {
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[Stages<1>::kBytes];
+  dkdv_walk<1>(p, (uint32_t)(uintptr_t)(UA_LDS unsigned char*)smem, blockIdx.x);
 }
-template <int kGroups>
-__global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void dq_kernel(const BwdParams p) {
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[kGroups * Stages<kGroups>::kBytes];
-  dq_walk<kGroups>(p, (uint32_t)(uintptr_t)(UA_LDS unsigned char*)smem, blockIdx.x);
+__global__ __launch_bounds__(Groups<1>::kThreads, 2) void dq_kernel(const BwdParams p) {
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[Stages<1>::kBytes];
+  dq_walk<1>(p, (uint32_t)(uintptr_t)(UA_LDS unsigned char*)smem, blockIdx.x);
 }
 // Both sides in one launch.
 template <int kGroups>
@@ -658,38 +658,31 @@ static int fill_side(BwdSide& s, int nnz, const int32_t* ptr, const int32_t* idx
 static int launched() { return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH; }
 static unsigned col_blocks(const BwdParams& p) { return (unsigned)(p.batch * p.n_heads * p.n_ktiles * p.cols.n_parts); }
 static unsigned row_blocks(const BwdParams& p) { return (unsigned)(p.batch * p.n_heads * p.n_qtiles * p.rows.n_parts); }
-// Groups per workgroup for n lines of 128 rows on both sides together (parts counted), as in the forward: four while half
-// lines leave a CU one workgroup at most (8 heads of 1024: 34 us with one group, 31 with two, 24 with four), two up to one
-// per CU and from three tiles a walk on.  Of an uncut causal rectangle, whose lines differ in length, four up to 256
-// lines that average four tiles (8 heads of 2048: 54 us with two, 44 with four) and two up to 512 that average eight (8 of
-// 4096: 140 us with one, 132 with two; 32 of 1024: 42, 54).  A launch of one side alone decides by both sides too,
-// so that its results are the same bit for bit.
+// Groups per workgroup for n lines of 128 rows on both sides of a dense rectangle together (parts counted), as in the
+// forward: four while half lines leave a CU one workgroup at most (8 heads of 1024: 34 us with one group, 31 with two, 24
+// with four), two up to one per CU and from three tiles a walk on.  Of an uncut causal rectangle, whose lines differ in
+// length, four up to 256 lines that average four tiles (8 heads of 2048: 54 us with two, 44 with four) and two up to 512 that
+// average eight (8 of 4096: 140 us with one, 132 with two; 32 of 1024: 42, 54).  Tile lists run with one, as in the forward.
 static int bwd_groups(int64_t n, int64_t both_walks, int n_parts, bool dense_causal, int n_qtiles, int n_ktiles) {
   const bool uneven = dense_causal && n_parts == 2;
   if (both_walks >= 3 && (2 * n <= kCus || (uneven && n <= kCus && both_walks >= 16))) return 4;
   if (both_walks < 6) return 1;
   return n <= kCus || (uneven && n <= 2 * kCus && n_qtiles >= 16 && n_ktiles >= 16) ? 2 : 1;
 }
-static unsigned both_blocks(const BwdParams& p) { return col_blocks(p) + row_blocks(p); }
-// Launches kernel<groups> for n workgroups of one line each.
-#define UA_LAUNCH_GROUPS(KERNEL, N, P, ST)                                                          \
-  switch (groups_of(P)) {                                                                           \
-    case 4: hipLaunchKernelGGL(KERNEL<4>, dim3(2 * (N)), dim3(512), 0, ST, P); break;               \
-    case 2: hipLaunchKernelGGL(KERNEL<2>, dim3(N), dim3(512), 0, ST, P); break;                     \
-    default: hipLaunchKernelGGL(KERNEL<1>, dim3(N), dim3(256), 0, ST, P);                           \
-  }
-static int groups_of(const BwdParams& p) {
-  const int64_t walks = p.dense ? p.cols.part_len + p.rows.part_len : p.nnz / p.n_qtiles + p.nnz / p.n_ktiles;
-  return bwd_groups(both_blocks(p), walks, p.cols.n_parts + p.rows.n_parts, p.dense_causal, p.n_qtiles, p.n_ktiles);
-}
-static int launch_bwd(BwdParams& p, hipStream_t st) {
-  const int groups = groups_of(p);
+// `plain`: one group per workgroup.
+static int launch_bwd(BwdParams& p, bool plain, hipStream_t st) {
+  const unsigned n = col_blocks(p) + row_blocks(p);
+  const int groups = plain ? 1 : bwd_groups(n, p.cols.part_len + p.rows.part_len, p.cols.n_parts + p.rows.n_parts, p.dense_causal, p.n_qtiles, p.n_ktiles);
   p.n_col_blocks = (int)col_blocks(p) * (groups == 4 ? 2 : 1);
   // Up to two workgroups per CU the whole launch is resident at once, and the second 256 join the first in launch
   // order.  Both sides come longest first (lists roughly); the columns are then taken in reverse, so that the long ones
   // of one side share a CU with the short ones of the other (32 causal heads of 1024: 43.6 -> 41.5 us).
-  p.cols_reversed = groups == 1 && (p.dense_causal || !p.dense) && both_blocks(p) > kCus && both_blocks(p) <= 2 * kCus;
-  UA_LAUNCH_GROUPS(bwd_kernel, both_blocks(p), p, st)
+  p.cols_reversed = groups == 1 && (p.dense_causal || !p.dense) && n > kCus && n <= 2 * kCus;
+  switch (groups) {
+    case 4: hipLaunchKernelGGL(bwd_kernel<4>, dim3(2 * n), dim3(512), 0, st, p); break;
+    case 2: hipLaunchKernelGGL(bwd_kernel<2>, dim3(n), dim3(512), 0, st, p); break;
+    default: hipLaunchKernelGGL(bwd_kernel<1>, dim3(n), dim3(256), 0, st, p);
+  }
   return launched();
 }
 
@@ -753,7 +746,7 @@ extern "C" int ua_bsa_bwd_dkdv(const void* q, const void* k, const void* v, cons
   if (!dv_strides) return UA_ERR_NULL;
   if (int rc = fill_side(p.cols, nnz, col_ptr, row_idx, cflag, k_order, dk, dk_strides, dv, dv_strides, false)) return rc;
   if (int rc = check_device()) return rc;
-  UA_LAUNCH_GROUPS(dkdv_kernel, col_blocks(p), p, (hipStream_t)stream)
+  hipLaunchKernelGGL(dkdv_kernel, dim3(col_blocks(p)), dim3(256), 0, (hipStream_t)stream, p);
   return launched();
 }
 
@@ -771,7 +764,7 @@ extern "C" int ua_bsa_bwd_dq(const void* q, const void* k, const void* v, const 
                            v_strides, do_strides, softmax_scale)) return rc;
   if (int rc = fill_side(p.rows, nnz, row_ptr, col_idx, flag, q_order, dq, dq_strides, nullptr, nullptr, false)) return rc;
   if (int rc = check_device()) return rc;
-  UA_LAUNCH_GROUPS(dq_kernel, row_blocks(p), p, (hipStream_t)stream)
+  hipLaunchKernelGGL(dq_kernel, dim3(row_blocks(p)), dim3(256), 0, (hipStream_t)stream, p);
   return launched();
 }
 
@@ -791,7 +784,7 @@ extern "C" int ua_bsa_bwd(const void* q, const void* k, const void* v, const voi
   if (int rc = fill_side(p.cols, nnz, col_ptr, row_idx, cflag, k_order, dk, dk_strides, dv, dv_strides, false)) return rc;
   if (int rc = fill_side(p.rows, nnz, row_ptr, col_idx, flag, q_order, dq, dq_strides, nullptr, nullptr, false)) return rc;
   if (int rc = check_device()) return rc;
-  return launch_bwd(p, (hipStream_t)stream);
+  return launch_bwd(p, true, (hipStream_t)stream);
 }
 
 extern "C" int ua_dense_bwd(const void* dout, const void* q, const void* k, const void* v,
@@ -830,7 +823,7 @@ extern "C" int ua_dense_bwd(const void* dout, const void* q, const void* k, cons
   const BwdCut n = ws_ok ? bwd_cut((int64_t)batch * n_heads, n_qtiles, n_ktiles, p.dense_causal, d.dkdv_parts, d.dq_parts) : BwdCut{1, 1};
   if (n.cols > 1) cut(p.cols, n.cols, n_qtiles, d.dkdv_bytes);
   if (n.rows > 1) cut(p.rows, n.rows, n_ktiles, d.dq_bytes);
-  if (int rc = launch_bwd(p, st)) return rc;
+  if (int rc = launch_bwd(p, !workspace, st)) return rc;
   PartialSum sums[3];
   int n_sums = 0;
   auto add_sum = [&](const BwdSide& s, const bf16* first, void* out, const int64_t* os, int seqlen) {

@@ -143,7 +143,7 @@ __device__ __forceinline__ void key_blocks(const unsigned char* sK, const unsign
   }
 }
 
-// kGroups = 2: two groups of four wavefronts share the query tile, one takes the first 64 keys of every tile, the
+// kGroups = 2 (dense rectangles only, as 4): two groups of four wavefronts share the query tile, one takes the first 64 keys of every tile, the
 // other the second; their results are combined through LDS.  kGroups = 4: four groups of two wavefronts share half
 // a query tile, each takes 32 keys of every tile.  A launch that gives a CU one workgroup at most runs it at
 // one wave per SIMD, where a half tile takes 1.2 us of which the matrix pipe is busy 0.4; with the second group the CU is
@@ -172,8 +172,9 @@ __global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void fwd_kernel(const
   pos /= kLines;
   if (pos < p.n_first) pos = p.n_first - 1 - pos;
   const int b = bh / p.n_heads, h = bh % p.n_heads;
+  const bool dense = kGroups > 1 || p.dense;
   int qt, e0, e1, diag = -1, part = -1;
-  if (p.dense) {
+  if (dense) {
     int line = pos;
     if (pos >= p.n_whole) {
       const int n_cut = p.n_qtiles - p.n_whole;
@@ -192,8 +193,8 @@ __global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void fwd_kernel(const
     e1 = min(max(sload(p.row_ptr, qt + 1), e0), p.nnz);
   }
   // entry e of the walk: its key tile, and whether it is a causal tile
-  auto ktile = [&](int e) { return p.dense ? e : min(max(sload(p.col_idx, e), 0), p.n_ktiles - 1); };
-  auto is_causal = [&](int e) { return p.dense ? (int)(e == diag) : sload(p.flag, e); };
+  auto ktile = [&](int e) { return dense ? e : min(max(sload(p.col_idx, e), 0), p.n_ktiles - 1); };
+  auto is_causal = [&](int e) { return dense ? (int)(e == diag) : sload(p.flag, e); };
 
   const bf16* kbase = p.k + b * p.ks.b + h * p.ks.h;
   const bf16* vbase = p.v + b * p.vs.b + h * p.vs.h;
@@ -370,23 +371,28 @@ static int fwd_common(FwdParams& p, const void* q, const void* k, const void* v,
   return check_device();
 }
 
-// Groups per workgroup for n lines of 128 rows (parts counted):
+// Groups per workgroup for n lines of 128 rows (parts counted) of a dense rectangle:
 //  - four, on half lines, while those leave a CU one workgroup at most (8 heads of 1024: 17.2 us with two groups, 13.8
 //    with four; 2048: 29.9, 24.3).  A walk of one tile is not worth the handing over at its end (6.1 us, one group 5.7).
 //  - two, on whole lines, up to one workgroup per CU and from three tiles on (32 heads of 1024: 25 us with one, 22 with two).
 //  - The rows of an uncut causal rectangle differ in length.  Run one after the other, longest first, they are
 //    balanced, which workgroups resident side by side from the start do not achieve: four groups up to 256 lines of 16
 //    tiles (8 heads of 4096: 57 us with two, 48 with four), two up to 512 lines (16 heads of 4096: 89 us with one, 77 with
-//    two).  The rows of a list are too much alike for that (strided 8k, 8 heads: 84 us with one, 95 with two).
+//    two).
+// Groups sum in another order, so that the last bits of a row depend on how many lines the launch has.  Tile lists, whose
+// launches are shards of the rows and heads of one mask, therefore run with one group whatever their size: a row's result is
+// the same bit for bit in every launch that holds its list.  Lists of up to 128 lines pay for that with half-empty CUs (one
+// head, causal 4096: forward 41 us with four groups, 67 with one, backward 61 and 117; from 512 lines on nothing changes).
 static int fwd_groups(int64_t n, int64_t walk, int n_parts, bool dense_causal) {
   const bool uneven = dense_causal && n_parts == 1;
   if (walk >= 2 && (2 * n <= kCus || (uneven && n <= kCus && walk >= 16))) return 4;
   return walk >= 3 && n <= (uneven ? 2 * kCus : kCus) ? 2 : 1;
 }
-static int fwd_launch(FwdParams& p, hipStream_t st) {
+// `plain`: one group per workgroup.
+static int fwd_launch(FwdParams& p, bool plain, hipStream_t st) {
   const unsigned n = (unsigned)(p.batch * p.n_heads * (p.n_whole + (p.n_qtiles - p.n_whole) * p.n_parts));
   // (several groups copy Q through a buffer descriptor, whose offsets have 32 bits)
-  switch (p.qs.s > (INT32_MAX >> 9) ? 1 : fwd_groups(n, p.dense ? p.part_len : p.nnz / p.n_qtiles, p.n_parts, p.dense_causal)) {
+  switch (plain || p.qs.s > (INT32_MAX >> 9) ? 1 : fwd_groups(n, p.part_len, p.n_parts, p.dense_causal)) {
     case 4: hipLaunchKernelGGL(fwd_kernel<4>, dim3(2 * n), dim3(512), 0, st, p); break;
     case 2: hipLaunchKernelGGL(fwd_kernel<2>, dim3(n), dim3(512), 0, st, p); break;
     default:
@@ -449,7 +455,7 @@ extern "C" int ua_bsa_fwd(const void* q, const void* k, const void* v, void* o, 
   if (int rc = fwd_common(p, q, k, v, o, lse, batch, n_heads, n_qtiles, n_ktiles, head_dim, q_strides, k_strides,
                           v_strides, o_strides, softmax_scale)) return rc;
   p.row_ptr = row_ptr; p.col_idx = col_idx; p.flag = flag; p.q_order = q_order; p.nnz = nnz;
-  return fwd_launch(p, (hipStream_t)stream);
+  return fwd_launch(p, true, (hipStream_t)stream);
 }
 
 namespace ua {
@@ -515,21 +521,22 @@ extern "C" int ua_dense_fwd(const void* q, const void* k, const void* v, void* o
                           v_strides, o_strides, softmax_scale)) return rc;
   p.dense = 1; p.dense_causal = causal != 0; p.diag_off = n_ktiles - n_qtiles;
   hipStream_t st = (hipStream_t)stream;
+  if (!workspace) return fwd_launch(p, true, st);
   const int max_parts = dense_split(batch, n_heads, n_qtiles, n_ktiles).fwd_parts;
   const Tail cut = dense_cut((int64_t)batch * n_heads, n_qtiles, n_ktiles, p.dense_causal, max_parts);
-  if (cut.tiles == 0) return fwd_launch(p, st);
+  if (cut.tiles == 0) return fwd_launch(p, false, st);
   // cutting needs the caller's workspace and a contiguous output for the merge
   const bool beside_whole = cut.tiles < n_qtiles;
   const PartBytes d = part_bytes(batch, n_heads, cut.tiles, beside_whole);
   const int64_t need = cut.parts * d.total();
-  if (!workspace || !aligned16(workspace) || workspace_bytes < need || !contiguous_bshd(o_strides, seqlen_q, n_heads)) return fwd_launch(p, st);
+  if (!aligned16(workspace) || workspace_bytes < need || !contiguous_bshd(o_strides, seqlen_q, n_heads)) return fwd_launch(p, false, st);
   p.n_whole = n_qtiles - cut.tiles;
   p.part_len = (n_ktiles + cut.parts - 1) / cut.parts;
   p.n_parts = (n_ktiles + p.part_len - 1) / p.part_len;
   p.part_o = workspace;
   p.part_lse = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + p.n_parts * d.o);
   p.o_part = d.o / (beside_whole ? 4 : 2); p.lse_part = d.lse / 4;
-  if (int rc = fwd_launch(p, st)) return rc;
+  if (int rc = fwd_launch(p, false, st)) return rc;
   if (beside_whole) {
     const int64_t first = (int64_t)p.n_whole * kTile;
     return merge_f32_rows((const float*)p.part_o, p.o_part, p.part_lse, p.lse_part, p.n_parts, p.o + first * n_heads * kHeadDim, lse + first, seqlen_q,

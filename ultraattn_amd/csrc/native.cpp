@@ -220,7 +220,7 @@ PyObject* dense_forward(PyObject* const* a) {
     if (ws.defined()) lock.lock();
     return ua_dense_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.t.data_ptr(), (float*)lse.t.data_ptr(), (int)q.size(0), (int)q.size(2),
                         (int)q.size(1), (int)k.size(1), (int)kDim, Strides(q), Strides(k), Strides(v), Strides(out.t), scale, causal,
-                        ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? ws.numel() : 0, on.stream);
+                        ws.defined() ? ws.data_ptr() : q.data_ptr(), ws.defined() ? ws.numel() : 0, on.stream);    // (NULL would rule out several groups)
   });
   return tuple_of(out, lse);
 }
@@ -270,7 +270,7 @@ PyObject* dense_backward(PyObject* const* a) {
     return ua_dense_bwd(x.dout.data_ptr(), x.q.data_ptr(), x.k.data_ptr(), x.v.data_ptr(), (const float*)x.lse.data_ptr(),
                         (const float*)x.delta.t.data_ptr(), x.dq.t.data_ptr(), x.dk.t.data_ptr(), x.dv.t.data_ptr(), (int)x.q.size(0), (int)x.q.size(2),
                         (int)x.q.size(1), (int)x.k.size(1), (int)kDim, Strides(x.q), Strides(x.k), Strides(x.v), Strides(x.dout), Strides(x.dq.t),
-                        Strides(x.dk.t), Strides(x.dv.t), scale, causal, ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? ws.numel() : 0, on.stream);
+                        Strides(x.dk.t), Strides(x.dv.t), scale, causal, ws.defined() ? ws.data_ptr() : x.q.data_ptr(), ws.defined() ? ws.numel() : 0, on.stream);
   });
   return tuple_of(x.dq, x.dk, x.dv, x.delta);
 }
