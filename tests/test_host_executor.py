@@ -9,8 +9,9 @@ import pytest
 import torch
 
 from oracle import tilelist_oracle as to
-from ultraattn_amd import packed
+from ultraattn_amd import executor, packed
 from ultraattn_amd.executor import comp_kernels_from_schedule, mask_from_comp_kernels
+from ultraattn_amd.tilelist import build_tile_list
 
 
 def test_causal_rule_over_all_keys():
@@ -171,3 +172,40 @@ def test_create_buf_dict_fused_graph_matches_the_reference_formulas():
         packed.create_buf_dict(qs, ks, 1, buf[:1000], fused_xy=(X, Y))
     with pytest.raises(ValueError):
         packed.create_buf_dict(qs, ks, 2, buf)
+
+
+@pytest.mark.parametrize("kind,shape,n,heads", [
+    ("dense", (64, 1024), 4, {15: False, 16: True, 32: True}),
+    ("dense", (63, 1024), 4, {16: False, 17: True}),           # 1008 and 1071 long lines
+    ("dense", (32, 1024), 8, {16: False, 32: True}),
+    ("dense", (64, 1023), 4, {32: False}),                     # rows too short
+    ("dense", (64, 1028), 4, {32: False}),                     # ranges of 257 tiles
+    ("dense", (64, 1024), 1, {32: False}),
+    ("mixed", (64, 1024), 4, {32: True}),                      # every other row has 8 tiles
+    ("few", (64, 1024), 4, {32: False}),                       # half the work in rows of 512
+    ("none", (64, 1024), 4, {32: False}),
+])
+def test_kernel_tiles_are_launched_for_many_long_rows_only(monkeypatch, kind, shape, n, heads):
+    """The executor's rule, the lists it builds for it, and the launches that follow from it."""
+    m = np.ones(shape, np.uint8)
+    if kind == "mixed":
+        m[1::2, 8:] = 0
+    elif kind == "few":
+        m[::3, 512:] = 0
+        m[1::3, 512:] = 0
+    elif kind == "none":
+        m[:] = 0
+    ex = executor.BlockSparseExecutor(m, 128, kernel_tiles=n)
+    built = []
+    monkeypatch.setattr(executor, "build_tile_list", lambda *a, **kw: built.append(1) or build_tile_list(*a, **kw))
+    walked = []
+    monkeypatch.setattr(executor, "bsa_fwd", lambda q, k, v, tiles, scale, out=None, lse=None: walked.append(tiles) or (out, lse))
+    monkeypatch.setattr(executor, "merge_partials", lambda outs, lses, out=None, lse=None: walked.append(len(outs)) or (out, lse))
+    for nh, launched in heads.items():
+        walked.clear()
+        q = torch.empty(1, 128, nh, 128, dtype=torch.bfloat16)
+        ex.forward(q, None, None)
+        assert ex.launches_kernel_tiles(q) == launched
+        assert len(built) == (n if launched else 0)               # no list that is not walked
+        assert walked == ([*ex.kernel_tiles, n] if launched else [ex.tiles])
+    assert len(ex.kernel_tiles) == (0 if n == 1 else n if m.any() else 1) and sum(t.nnz for t in ex.kernel_tiles) == (ex.tiles.nnz if n > 1 else 0)

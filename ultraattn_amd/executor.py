@@ -72,15 +72,22 @@ class BlockSparseExecutor:
 
     ``block_mask``: uint8 [row chunks, column chunks] of 0 EMPTY / 1 FULL / 2 CAUSAL for the
     chunks this device computes; ``chunk`` = tokens per chunk (``S_per_partition``).
-    ``kernel_tiles`` > 1 splits the key range into that many kernel tiles.  Rows of many tiles are then
-    computed kernel tile by kernel tile into partial (O, LSE) that are merged; shorter ones
-    walk their kernel tiles one after the other in one launch, whose running softmax is that merge."""
+    ``kernel_tiles`` > 1 splits the key range into that many kernel tiles, a hint for long rows: where
+    it pays the forward computes kernel tile by kernel tile into partial (O, LSE) that are merged, else
+    it walks the kernel tiles one after the other in one launch, whose running softmax is that merge (and
+    whose O is rounded once).  ``launches_kernel_tiles(q)`` says which; the attribute
+    ``kernel_tiles`` holds the tile lists of the kernel tiles, built when they are first asked for or
+    launched."""
 
-    # Key ranges keep the K/V that many rows walk at the same time in the caches and in few DRAM pages, which pays
-    # for the partials' way through memory from about 512 tiles (64k keys) a row on: dense rows, 32 heads, 4 key ranges
-    # against one launch: 256 tiles 15.3 ms against 15.0, 512 30.0 / 31.6, 1024 60.3 / 65.0, 4096 131 / 143.
-    # Streaming rows of 66 tiles: 8.66 against 7.92, of 10 tiles 2.35 against 1.51.
-    _LONG_ROW = 384
+    # What launches of their own buy: the K/V that many rows walk at the same time stay in the caches and in few DRAM
+    # pages.  What they cost: the partials' way through memory and a prologue per row and kernel tile.  One launch against n,
+    # MI355X, dense rows of 128-token tiles (n launches' time relative to one; 32, 64 and 128 rows):
+    #   rows of 1024, heads 32: 4 of 256 tiles -1.6 -2.4 -4.2 %, 8 of 128 -2.5 -3.7 -5.9 %, 2 of 512 -0.7 +0.6 -1.3 %
+    #   rows of 1024, heads 16: 4 of 256 +0.8 -2.7 -2.0 %; heads 24: -0.4 +0.5 -0.8 %; heads 8: +1.3 -0.9 -0.7 %; heads 1 to 4: 0 to +5 %
+    #   rows of 2048, 8 of 256: heads 32 -2.3 -5.2 -6.7 %, 16 -0.5 -2.2 -5.0 %, 8 +0.5 +0.9 -1.8 %
+    #   rows of 512, 4 of 128: heads 32 -0.6 to -2.3 %, 16 -1.7 to +0.4 %, 24 +1.3 %, fewer +1.5 to +3.6 %
+    #   rows of 64 to 256: always slower, up to 30 %; a few long rows among short ones: up to 22 % slower
+    _LONG_ROW, _RANGE, _HEADS, _LINES = 1024, 256, 16, 1024
 
     def __init__(self, block_mask: np.ndarray, chunk: int, softmax_scale: Optional[float] = None,
                  kernel_tiles: int = 1):
@@ -88,17 +95,30 @@ class BlockSparseExecutor:
         self.chunk = int(chunk)
         self.softmax_scale = softmax_scale
         self.tiles: TileList = build_tile_list(self.mask, block=self.chunk)
-        self.kernel_tiles: List[TileList] = []
+        self._kernel_tiles: Optional[List[TileList]] = None
         self._parts, self._part_key = None, None
-        # average row, empty rows left out
-        rows = int(np.count_nonzero(np.diff(self.tiles.row_ptr)))
-        self._by_kernel_tile = kernel_tiles > 1 and self.tiles.nnz >= self._LONG_ROW * max(rows, 1)
-        if kernel_tiles > 1:
-            cols = np.nonzero(self.mask.any(0))[0]
-            for part in np.array_split(cols, min(kernel_tiles, max(1, len(cols)))):
+        cols = np.nonzero(self.mask.any(0))[0]
+        self._ranges = np.array_split(cols, min(kernel_tiles, max(1, len(cols)))) if kernel_tiles > 1 else []
+        # rows that are long; most of the work must be theirs, in ranges that are not long themselves
+        length = np.diff(self.tiles.row_ptr)
+        length = length[length >= self._LONG_ROW]
+        work = int(length.sum())
+        self._long_rows = len(length) if 4 * work >= 3 * self.tiles.nnz and work <= self._RANGE * len(length) * len(self._ranges) else 0
+
+    @property
+    def kernel_tiles(self) -> List[TileList]:
+        if self._kernel_tiles is None:
+            self._kernel_tiles = []
+            for part in self._ranges:
                 sub = np.zeros_like(self.mask)
                 sub[:, part] = self.mask[:, part]
-                self.kernel_tiles.append(build_tile_list(sub, block=self.chunk))
+                self._kernel_tiles.append(build_tile_list(sub, block=self.chunk))
+        return self._kernel_tiles
+
+    def launches_kernel_tiles(self, q) -> bool:
+        """Whether ``forward`` runs its kernel tiles as launches of their own for this q."""
+        heads = q.shape[0] * q.shape[2]
+        return self._long_rows > 0 and heads >= self._HEADS and heads * self._long_rows >= self._LINES
 
     @classmethod
     def from_comp_kernels(cls, keys: Iterable[CompKey], n_row_chunks: int, n_col_chunks: int, chunk: int,
@@ -126,10 +146,10 @@ class BlockSparseExecutor:
         return self._parts
 
     def forward(self, q, k, v, out=None, lse=None):
-        """-> (out, lse); one launch, or for long rows ``kernel_tiles`` launches into partial buffers that
-        the executor keeps + one merge.  The partials are overwritten by the next call with kernel
-        tiles, so calls on different streams must not overlap."""
-        if not self._by_kernel_tile:
+        """-> (out, lse); one launch, or where ``launches_kernel_tiles(q)`` one per kernel tile into partial
+        buffers that the executor keeps + one merge.  The partials are overwritten by the next call with
+        kernel tiles, so calls on different streams must not overlap."""
+        if not self.launches_kernel_tiles(q):
             return bsa_fwd(q, k, v, self.tiles, self.softmax_scale, out=out, lse=lse)
         parts = [bsa_fwd(q, k, v, t, self.softmax_scale, out=po, lse=pl)
                  for t, (po, pl) in zip(self.kernel_tiles, self._partials(q))]
