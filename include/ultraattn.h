@@ -194,12 +194,14 @@ int ua_bsa_bwd(const void *q, const void *k, const void *v, const void *dout,
  * causal only the last query tiles are cut, those left over after the last full wave of workgroups;
  * their partial O is fp32.
  * The partials live in `workspace` (device memory, 16-byte aligned, caller-owned, overwritten by
- * every call: calls that share it must not overlap); ua_dense_workspace_bytes() gives a size
- * that lets a shape split, causal or not (0 = it never splits).  With a workspace that is too small
+ * every call: calls that share it must not overlap).  ua_dense_workspace_used() gives what a call
+ * of this shape cuts with (0 = it is not cut), ua_dense_workspace_bytes() an upper bound of it that
+ * does not depend on `causal`.  With a workspace that is too small
  * (any pointer with workspace_bytes = 0 included) or a forward output that is not contiguous nothing
  * is cut.  The last bits of a row then depend on the launch, i.e. on how many rows and heads run
  * with it.  With workspace == NULL every line is walked whole by one group: the results are those
  * of ua_bsa_fwd / ua_bsa_bwd over the rectangle's tile list, bit for bit.                        */
+int64_t ua_dense_workspace_used(int batch, int n_heads, int seqlen_q, int seqlen_k, int causal, int backward);
 int64_t ua_dense_workspace_bytes(int batch, int n_heads, int seqlen_q, int seqlen_k, int backward);
 int ua_dense_fwd(const void *q, const void *k, const void *v, void *o, float *lse,
                  int batch, int n_heads, int seqlen_q, int seqlen_k, int head_dim,

@@ -143,6 +143,28 @@ def test_dense_entry_points_without_gpu(lib):
     assert ws(1, 32, 2048, 4096, 0) == 0                                               # 512 workgroups: full launch
 
 
+def test_dense_workspace_used_without_gpu(lib):
+    """What a call cuts with: nothing where it is not cut, never more than the bound that does not know `causal`."""
+    used, bound = lib.ua_dense_workspace_used, lib.ua_dense_workspace_bytes
+    for shape in ((1, 32, 512, 512), (1, 8, 1024, 1024)):                             # few lines, but short walks: not cut
+        assert bound(*shape, 0) > 0 and bound(*shape, 1) > 0
+        assert all(used(*shape, causal, backward) == 0 for causal in (0, 1) for backward in (0, 1))
+    assert used(1, 32, 2304, 3456, 0, 0) == bound(1, 32, 2304, 3456, 0) > 0           # the last wave is cut ...
+    assert used(1, 32, 2304, 3456, 1, 0) == 0                                        # ... unless the call is causal
+    assert used(1, 1, 1000, 4096, 0, 0) == used(0, 1, 1024, 4096, 0, 1) == 0          # nothing to size
+    sizes = [1, 2, 3, 5, 8, 11, 16, 21, 27, 32, 64, 75, 171]
+    cut = 0
+    for nh in (1, 2, 3, 5, 8, 12, 32, 64):
+        for q in sizes:
+            for k in sizes:
+                for backward in (0, 1):
+                    most = bound(1, nh, 128 * q, 128 * k, backward)
+                    got = [used(1, nh, 128 * q, 128 * k, causal, backward) for causal in (0, 1)]
+                    assert 0 <= min(got) and max(got) <= most, (nh, q, k, backward)
+                    cut += sum(x > 0 for x in got)
+    assert cut > 100
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "_lib", None)
     monkeypatch.setattr(_lib, "LIB_PATH", str(tmp_path / "nope.so"))

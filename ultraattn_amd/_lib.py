@@ -26,6 +26,7 @@ SIGNATURES = {
     "ua_bsa_bwd_dq": (c_int, [c_void_p] * 11 + [c_int] * 6 + [_i64p] * 5 + [c_float, c_void_p]),
     "ua_bsa_bwd": (c_int, [c_void_p] * 17 + [c_int] * 6 + [_i64p] * 7 + [c_float, c_void_p]),
     "ua_dense_workspace_bytes": (c_int64, [c_int] * 5),
+    "ua_dense_workspace_used": (c_int64, [c_int] * 6),
     "ua_dense_fwd": (c_int, [c_void_p] * 5 + [c_int] * 5 + [_i64p] * 4 + [c_float, c_int, c_void_p, c_int64, c_void_p]),
     "ua_dense_bwd": (c_int, [c_void_p] * 9 + [c_int] * 5 + [_i64p] * 7 + [c_float, c_int, c_void_p, c_int64, c_void_p]),
     "ua_merge": (c_int, [POINTER(c_void_p), POINTER(c_void_p), c_int, c_void_p, c_void_p,

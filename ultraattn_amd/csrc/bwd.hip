@@ -700,16 +700,20 @@ static BwdCut bwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int 
   if (max_cols <= 1 && max_rows <= 1) return {1, 1};
   static constexpr int kParts[] = {1, 2, 3, 4, 5, 6, 8, 12, 16};
   const float density = causal ? 0.5f : 1.f, wk = (float)nbh * n_ktiles, wq = (float)nbh * n_qtiles;
+  const float all = density * wk * n_qtiles * (4.94f + 5.47f) / (2 * kCus);
+  int row_len[sizeof(kParts) / sizeof(int)], n_rows = 0;
+  for (int pr : kParts)
+    if (pr <= max_rows) row_len[n_rows++] = (n_ktiles + pr - 1) / pr;
   BwdCut best = {1, 1};
   float best_us = INFINITY;
   for (int pc : kParts) {
     if (pc > max_cols) break;
-    for (int pr : kParts) {
-      if (pr > max_rows) break;
+    const int clen = (n_qtiles + pc - 1) / pc;
+    for (int i = 0; i < n_rows; ++i) {
+      const int pr = kParts[i], rlen = row_len[i];
       const float groups = (wk * pc + wq * pr) * density;
       float us, tc, tr;
-      switch (bwd_groups(nbh * ((int64_t)n_ktiles * pc + (int64_t)n_qtiles * pr), (n_qtiles + pc - 1) / pc + (n_ktiles + pr - 1) / pr, pc + pr, causal,
-                         n_qtiles, n_ktiles)) {
+      switch (bwd_groups(nbh * ((int64_t)n_ktiles * pc + (int64_t)n_qtiles * pr), clen + rlen, pc + pr, causal, n_qtiles, n_ktiles)) {
         case 4: us = 7.1f; tc = 1.86f; tr = 0.96f; break;
         case 2: us = 9.8f; tc = 2.6f; tr = 1.7f; break;
         default: {
@@ -717,9 +721,7 @@ static BwdCut bwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int 
           us = 6.5f; tc = 3.5f + 1.44f * shared; tr = 2.1f + 3.37f * shared;
         }
       }
-      const float longest = fmaxf((float)((n_qtiles + pc - 1) / pc) * tc, (float)((n_ktiles + pr - 1) / pr) * tr);
-      const float all = density * wk * n_qtiles * (4.94f + 5.47f) / (2 * kCus);
-      us += fmaxf(longest, all);
+      us += fmaxf(fmaxf(clen * tc, rlen * tr), all);
       if (pc > 1 || pr > 1) us = (us + 2.4f) * 1.06f;
       if (pc > 1) us += 2.f * pc * wk * (kTile * kHeadDim * 4) / 3.7e6f;
       if (pr > 1) us += pr * wq * (kTile * kHeadDim * 4) / 3.7e6f;
@@ -727,6 +729,11 @@ static BwdCut bwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int 
     }
   }
   return best;
+}
+int64_t bwd_workspace_used(int batch, int n_heads, int n_qtiles, int n_ktiles, bool causal) {
+  const DenseSplit d = dense_split(batch, n_heads, n_qtiles, n_ktiles);
+  const BwdCut n = bwd_cut((int64_t)batch * n_heads, n_qtiles, n_ktiles, causal, d.dkdv_parts, d.dq_parts);
+  return (n.cols > 1 ? n.cols * d.dkdv_bytes : 0) + (n.rows > 1 ? n.rows * d.dq_bytes : 0);
 }
 
 }  // namespace ua
@@ -809,7 +816,6 @@ extern "C" int ua_dense_bwd(const void* dout, const void* q, const void* k, cons
   p.cols.part_len = n_qtiles; p.rows.part_len = n_ktiles;
   const DenseSplit d = dense_split(batch, n_heads, n_qtiles, n_ktiles);
   unsigned char* ws = static_cast<unsigned char*>(workspace);
-  const bool ws_ok = workspace && aligned16(workspace) && workspace_bytes >= d.bwd_total;
   // Cut one side: parts of equal length, fp32 partials in the workspace.
   auto cut = [&](BwdSide& s, int parts, int list_len, int64_t part_bytes) {
     s.part_len = (list_len + parts - 1) / parts;
@@ -820,7 +826,11 @@ extern "C" int ua_dense_bwd(const void* dout, const void* q, const void* k, cons
     s.out1 = reinterpret_cast<bf16*>(ws + part_bytes / 2);       // columns: dV behind dK
     ws += parts * part_bytes;
   };
-  const BwdCut n = ws_ok ? bwd_cut((int64_t)batch * n_heads, n_qtiles, n_ktiles, p.dense_causal, d.dkdv_parts, d.dq_parts) : BwdCut{1, 1};
+  BwdCut n = {1, 1};
+  if (workspace && aligned16(workspace) && workspace_bytes > 0) {
+    n = bwd_cut((int64_t)batch * n_heads, n_qtiles, n_ktiles, p.dense_causal, d.dkdv_parts, d.dq_parts);
+    if (workspace_bytes < (n.cols > 1 ? n.cols * d.dkdv_bytes : 0) + (n.rows > 1 ? n.rows * d.dq_bytes : 0)) n = {1, 1};
+  }
   if (n.cols > 1) cut(p.cols, n.cols, n_qtiles, d.dkdv_bytes);
   if (n.rows > 1) cut(p.rows, n.rows, n_ktiles, d.dq_bytes);
   if (int rc = launch_bwd(p, !workspace, st)) return rc;

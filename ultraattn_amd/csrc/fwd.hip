@@ -495,7 +495,19 @@ static Tail dense_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int 
   return {parts > 1 ? n_qtiles : 0, parts};
 }
 
+static int64_t fwd_workspace_used(int batch, int n_heads, int n_qtiles, int n_ktiles, bool causal) {
+  const int max_parts = dense_split(batch, n_heads, n_qtiles, n_ktiles).fwd_parts;
+  const Tail cut = dense_cut((int64_t)batch * n_heads, n_qtiles, n_ktiles, causal, max_parts);
+  return cut.tiles ? cut.parts * part_bytes(batch, n_heads, cut.tiles, cut.tiles < n_qtiles).total() : 0;
+}
+
 }  // namespace ua
+
+extern "C" int64_t ua_dense_workspace_used(int batch, int n_heads, int seqlen_q, int seqlen_k, int causal, int backward) {
+  using namespace ua;
+  if (batch <= 0 || n_heads <= 0 || seqlen_q <= 0 || seqlen_k <= 0 || seqlen_q % kTile || seqlen_k % kTile) return 0;
+  return (backward ? bwd_workspace_used : fwd_workspace_used)(batch, n_heads, seqlen_q / kTile, seqlen_k / kTile, causal != 0);
+}
 
 extern "C" int64_t ua_dense_workspace_bytes(int batch, int n_heads, int seqlen_q, int seqlen_k, int backward) {
   using namespace ua;

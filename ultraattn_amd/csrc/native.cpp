@@ -135,15 +135,20 @@ template <class F> void call(const char* what, F&& f) {
   check_rc(rc, what);
 }
 
-// ---- workspaces of split dense calls --------------------------------------------------------------
+// ---- workspaces of cut dense calls ----------------------------------------------------------------
 // `cache`: dict (device index, stream handle) -> uint8 tensor.  Calls on one stream run in order, so they can
 // share it; it only ever grows.  At most kMaxWorkspaces are kept, the least recently used goes first (stream
 // handles come and go).  `captured` (list) keeps those that a captured graph may replay into.
 constexpr Py_ssize_t kMaxWorkspaces = 16;
-std::mutex workspace_use;        // a split call's launches stay together when threads share a stream
+// The launches of a cut call stay together when threads share its stream and so its workspace: each workspace has a mutex
+// (one of 64 by its address; calls on different workspaces hardly ever meet).
+std::mutex workspace_use[64];
+std::unique_lock<std::mutex> hold(const at::Tensor& ws) {
+  return ws.defined() ? std::unique_lock<std::mutex>(workspace_use[(reinterpret_cast<uintptr_t>(ws.data_ptr()) >> 9) % 64]) : std::unique_lock<std::mutex>();
+}
 
-at::Tensor workspace(PyObject* cache, PyObject* captured, const On& on, const at::Tensor& q, const at::Tensor& k, bool backward) {
-  const int64_t need = ua_dense_workspace_bytes((int)q.size(0), (int)q.size(2), (int)q.size(1), (int)k.size(1), backward);
+at::Tensor workspace(PyObject* cache, PyObject* captured, const On& on, const at::Tensor& q, const at::Tensor& k, bool causal, bool backward) {
+  const int64_t need = ua_dense_workspace_used((int)q.size(0), (int)q.size(2), (int)q.size(1), (int)k.size(1), causal, backward);
   if (need <= 0) return at::Tensor();
   PyObject* key = Py_BuildValue("(iK)", on.device, (unsigned long long)(uintptr_t)on.stream);
   if (!key) throw PyError();
@@ -214,10 +219,10 @@ PyObject* dense_forward(PyObject* const* a) {
   lse.t = stat_of(q);
   const On on(q);
   init_device(on.device);
-  const at::Tensor ws = workspace(a[6], a[7], on, q, k, false);
+  // (an output that is not contiguous is not cut)
+  const at::Tensor ws = out.t.is_contiguous() ? workspace(a[6], a[7], on, q, k, causal, false) : at::Tensor();
   call("ua_dense_fwd", [&] {
-    std::unique_lock<std::mutex> lock(workspace_use, std::defer_lock);
-    if (ws.defined()) lock.lock();
+    const auto held = hold(ws);
     return ua_dense_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.t.data_ptr(), (float*)lse.t.data_ptr(), (int)q.size(0), (int)q.size(2),
                         (int)q.size(1), (int)k.size(1), (int)kDim, Strides(q), Strides(k), Strides(v), Strides(out.t), scale, causal,
                         ws.defined() ? ws.data_ptr() : q.data_ptr(), ws.defined() ? ws.numel() : 0, on.stream);    // (NULL would rule out several groups)
@@ -263,10 +268,9 @@ PyObject* dense_backward(PyObject* const* a) {
   x.allocate(a[4]);
   const On on(x.q);
   init_device(on.device);
-  const at::Tensor ws = workspace(a[12], a[13], on, x.q, x.k, true);
+  const at::Tensor ws = workspace(a[12], a[13], on, x.q, x.k, causal, true);
   call("ua_dense_bwd", [&] {
-    std::unique_lock<std::mutex> lock(workspace_use, std::defer_lock);
-    if (ws.defined()) lock.lock();
+    const auto held = hold(ws);
     return ua_dense_bwd(x.dout.data_ptr(), x.q.data_ptr(), x.k.data_ptr(), x.v.data_ptr(), (const float*)x.lse.data_ptr(),
                         (const float*)x.delta.t.data_ptr(), x.dq.t.data_ptr(), x.dk.t.data_ptr(), x.dv.t.data_ptr(), (int)x.q.size(0), (int)x.q.size(2),
                         (int)x.q.size(1), (int)x.k.size(1), (int)kDim, Strides(x.q), Strides(x.k), Strides(x.v), Strides(x.dout), Strides(x.dq.t),

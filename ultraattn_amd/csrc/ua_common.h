@@ -368,6 +368,8 @@ inline DenseSplit dense_split(int batch, int n_heads, int n_qtiles, int n_ktiles
   d.bwd_total = (d.dq_parts > 1 ? d.dq_parts * d.dq_bytes : 0) + (d.dkdv_parts > 1 ? d.dkdv_parts * d.dkdv_bytes : 0);
   return d;
 }
+// Bytes of workspace that a dense backward of this shape uses (0: it is not cut).
+int64_t bwd_workspace_used(int batch, int n_heads, int n_qtiles, int n_ktiles, bool causal);
 // One sum of fp32 partial results (contiguous [batch, seqlen, n_heads, 128], part i at base + i * stride floats)
 // into a strided bf16 tensor; up to three of them run in one launch.
 struct PartialSum {
