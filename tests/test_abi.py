@@ -152,6 +152,7 @@ def test_dense_workspace_used_without_gpu(lib):
     assert used(1, 32, 2304, 3456, 0, 0) == bound(1, 32, 2304, 3456, 0) > 0           # the last wave is cut ...
     assert used(1, 32, 2304, 3456, 1, 0) == 0                                        # ... unless the call is causal
     assert used(1, 1, 1000, 4096, 0, 0) == used(0, 1, 1024, 4096, 0, 1) == 0          # nothing to size
+    assert used(1, 257, 128, 8192, 0, 0) == 0                                         # more heads than the merge takes
     sizes = [1, 2, 3, 5, 8, 11, 16, 21, 27, 32, 64, 75, 171]
     cut = 0
     for nh in (1, 2, 3, 5, 8, 12, 32, 64):

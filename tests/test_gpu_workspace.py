@@ -5,7 +5,7 @@ import threading
 import pytest
 import torch
 
-from tests.gpu_util import SCALE
+from tests.gpu_util import ATOL_O, SCALE
 from ultraattn_amd import flash_attn_interface as fai
 from ultraattn_amd.flash_attn_interface import _flash_attn_backward, _flash_attn_forward
 
@@ -61,3 +61,15 @@ def test_threads(n_threads, own_streams):
     for t in threads:
         t.join()
     assert not wrong, wrong
+
+
+@pytest.mark.parametrize("nh", [255, 256, 257])
+def test_heads_beyond_the_merge(nh):
+    """A forward of few lines and many heads with a long walk: the merge of a cut takes 256 heads, more run uncut."""
+    sq, sk = 128, 8192
+    q, k, v, _ = _inputs(sq, sk, nh, 1)
+    r = _flash_attn_forward(q, k, v, 0.0, SCALE, False)
+    for h in (0, nh - 1):
+        s = (q[0, :, h].float() @ k[0, :, h].float().T) * SCALE
+        assert (r[0][0, :, h].float() - torch.softmax(s, -1) @ v[0, :, h].float()).abs().max().item() <= ATOL_O
+        assert (r[5][0, h] - torch.logsumexp(s, -1)).abs().max().item() <= 1e-4

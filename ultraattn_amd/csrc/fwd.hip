@@ -489,15 +489,16 @@ static PartBytes part_bytes(int batch, int n_heads, int n_tiles, bool f32) {
   return {align256(rows * kHeadDim * (f32 ? 4 : 2)), align256(rows * 4)};
 }
 // Query tiles at the end that are cut, and into how many parts.
-static Tail dense_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int max_parts) {
+static Tail dense_cut(int batch, int n_heads, int n_qtiles, int n_ktiles, bool causal) {
+  const int64_t nbh = (int64_t)batch * n_heads;
+  const int max_parts = dense_split(batch, n_heads, n_qtiles, n_ktiles).fwd_parts;
   if (max_parts == 1) return causal ? Tail{0, 1} : fwd_tail(nbh, n_qtiles, n_ktiles);
-  const int parts = fwd_cut(nbh, n_qtiles, n_ktiles, causal, max_parts);
+  const int parts = n_heads > kMaxHeadsLds ? 1 : fwd_cut(nbh, n_qtiles, n_ktiles, causal, max_parts);       // (more heads: not merged)
   return {parts > 1 ? n_qtiles : 0, parts};
 }
 
 static int64_t fwd_workspace_used(int batch, int n_heads, int n_qtiles, int n_ktiles, bool causal) {
-  const int max_parts = dense_split(batch, n_heads, n_qtiles, n_ktiles).fwd_parts;
-  const Tail cut = dense_cut((int64_t)batch * n_heads, n_qtiles, n_ktiles, causal, max_parts);
+  const Tail cut = dense_cut(batch, n_heads, n_qtiles, n_ktiles, causal);
   return cut.tiles ? cut.parts * part_bytes(batch, n_heads, cut.tiles, cut.tiles < n_qtiles).total() : 0;
 }
 
@@ -534,8 +535,7 @@ extern "C" int ua_dense_fwd(const void* q, const void* k, const void* v, void* o
   p.dense = 1; p.dense_causal = causal != 0; p.diag_off = n_ktiles - n_qtiles;
   hipStream_t st = (hipStream_t)stream;
   if (!workspace) return fwd_launch(p, true, st);
-  const int max_parts = dense_split(batch, n_heads, n_qtiles, n_ktiles).fwd_parts;
-  const Tail cut = dense_cut((int64_t)batch * n_heads, n_qtiles, n_ktiles, p.dense_causal, max_parts);
+  const Tail cut = dense_cut(batch, n_heads, n_qtiles, n_ktiles, p.dense_causal);
   if (cut.tiles == 0) return fwd_launch(p, false, st);
   // cutting needs the caller's workspace and a contiguous output for the merge
   const bool beside_whole = cut.tiles < n_qtiles;

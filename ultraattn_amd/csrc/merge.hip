@@ -19,7 +19,6 @@ inline int merge_tokens(int64_t tokens, int n_heads) {
   while (tok * 2 * n_heads <= 64 && tokens / (tok * 2) >= 2 * kCus) tok *= 2;
   return tok;
 }
-constexpr int kMaxHeadsLds = 256;
 
 struct MergeParams {
   const bf16* o_parts[UA_MAX_PARTS];

@@ -18,6 +18,7 @@ constexpr int kTile = UA_TILE;          // 128 x 128 kernel tile
 constexpr int kHeadDim = UA_HEAD_DIM;   // 128
 constexpr int kRowBytes = kHeadDim * 2; // one K/V/Q row of bf16 in LDS
 constexpr int kTileBytes = kTile * kRowBytes;  // 32 KiB
+constexpr int kMaxHeadsLds = 256;       // heads whose statistics the merge, update and delta kernels take
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 
