@@ -87,7 +87,7 @@ __device__ __forceinline__ void store_block(const __attribute__((address_space(4
 //   dV^T += dO^T P,  dK^T += Q^T dS                     16 MFMAs, Q and dO read through the transposing path
 // P and dS never leave the wave.  The accumulators of S and dP' start from the rows' statistics.
 //
-// Bound: matrix pipe at the clock the socket's power allows (68 % busy at 1.73 GHz).  192 of a wave's 256 registers
+// Bound: matrix pipe at the clock the socket's power allows (70 % busy at 1.68 GHz).  192 of a wave's 256 registers
 // hold K, V, dK and dV; two independent workgroups share a CU, so that one's exp2 and barriers hide behind
 // the other's MFMAs.  Against one workgroup of eight waves in two roles (S/dV and dP/dK, P handed over
 // through LDS): strided 128k, 32 heads 37.8 -> 33.5 ms, causal 32k 15.8 -> 13.7 ms (1.25-1.3 PFLOP/s of the four
@@ -694,7 +694,7 @@ static int launch_bwd(BwdParams& p, bool plain, hipStream_t st) {
 //  - a tile takes 1.9 (columns) or 1 (rows) with four groups, 2.6 and 1.7 with two, else 3.5 and 2.1, and 4.9 and 5.5
 //    where two workgroups share the CU;
 //  - the sum takes 2.4, and the partials 1 per 3.7 MB; a cut has to win by 6 %.
-// 1024 x 4096, one head: 42 us uncut, 24 cut in 2 and 5.
+// 1024 x 4096, one head: 42 us uncut, 24 cut in 2 and 4.
 struct BwdCut { int cols, rows; };
 static BwdCut bwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int max_cols, int max_rows) {
   if (max_cols <= 1 && max_rows <= 1) return {1, 1};

@@ -412,7 +412,7 @@ static int fwd_launch(FwdParams& p, bool plain, hipStream_t st) {
 //  - 3.8 to start, load Q, store and end, 4.3 with two groups per workgroup, 5.1 with four;
 //  - a tile takes 1.1 with four groups, 1.8 with two, else 2.2, and 3.7 where two workgroups share the CU;
 //  - the merge takes 2.4, and the partials 1 per 1.5 MB.
-// 1024 x 4096, one head: 41 us uncut, 13 cut in 16.
+// 1024 x 4096, one head: 41 us uncut, 13 cut in 11.
 static int fwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int max_parts) {
   const float density = causal ? 0.5f : 1.f, lines = (float)nbh * n_qtiles;
   int best = 1;

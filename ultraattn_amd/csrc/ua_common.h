@@ -333,13 +333,13 @@ inline bool strides_ok(const int64_t* s) { return s && s[0] % 8 == 0 && s[1] % 8
 
 int check_device();   // UA_OK when the current device is gfx950
 
-// ---- dense rectangles: how many parts a walk is cut into -------------------------------------
+// ---- dense rectangles: how many parts a walk may be cut into ----------------------------------
 // A dense rectangle launches one workgroup per (tile line, head); with few lines and heads the
-// device (256 CUs, two resident workgroups each for the row walks) stays empty while every
-// workgroup walks a long list.  The walk is then cut into parts that run as workgroups of their
-// own and leave partial results, combined by a second, HBM-bound kernel.  No split when the launch
-// fills the device anyway or the list is short; else enough parts for ~2 workgroups per CU, at
-// least two tiles each, at most UA_MAX_PARTS.
+// device (256 CUs, two resident workgroups each) stays empty while every workgroup walks a long
+// list.  The walk may then be cut into parts that run as workgroups of their own and leave partial
+// results, combined by a second kernel.  No cut when the launch fills the device anyway or the list
+// is short; else at most as many parts as make ~2 workgroups per CU, of at least two tiles each, and
+// at most UA_MAX_PARTS.  How many are made is for the estimates of fwd_cut and bwd_cut to choose.
 constexpr int kDenseFullLaunch = 384, kDenseTargetGroups = 512;
 inline int dense_parts(int64_t n_workgroups, int list_len) {
   if (n_workgroups >= kDenseFullLaunch || list_len < 4) return 1;
@@ -359,7 +359,10 @@ inline DenseSplit dense_split(int batch, int n_heads, int n_qtiles, int n_ktiles
   DenseSplit d;
   const int64_t nbh = (int64_t)batch * n_heads;
   d.fwd_parts = d.dq_parts = dense_parts(nbh * n_qtiles, n_ktiles);
-  d.dkdv_parts = dense_parts(nbh * n_ktiles * 2, n_qtiles);      // one dK/dV workgroup fills a CU
+  // Columns count twice: dQ's rows are in the same launch, and from 192 columns on the estimate would take cuts that do not pay
+  // (4096 causal queries x 2048 keys, 23 heads, 368 columns: 92 us, cut 117; 16384 x 8192, 3 heads, 192 columns: 610, 642; in
+  // 22 other shapes of 192 to 368 columns it takes none and the time is the same).
+  d.dkdv_parts = dense_parts(nbh * n_ktiles * 2, n_qtiles);
   const int64_t q_elems = nbh * n_qtiles * kTile * kHeadDim, k_elems = nbh * n_ktiles * kTile * kHeadDim;
   d.fwd_o_bytes = align256(q_elems * 2);
   d.fwd_lse_bytes = align256(nbh * n_qtiles * kTile * 4);
