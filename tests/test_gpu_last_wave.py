@@ -48,3 +48,18 @@ def test_tail_equals_the_single_launch(lib, B, nh, sq, sk):
         err, err_cut = _rel(res[0][b, :128 * whole, h], want[:128 * whole]), _rel(res[0][b, cut, h], want[cut])
         assert err <= 5e-3 and err_cut <= 1.05 * err, (err, err_cut)
         assert lse_rel_err(res[5][b, h, cut], torch.logsumexp(s, -1)[cut].float().cpu()) <= 1e-5
+
+
+@pytest.mark.parametrize("key", [0, 3455])
+def test_infinities_stay_where_they_belong(lib, key):
+    """An infinite value of the first or the last part (seven here) reaches the outputs it belongs to, cut lines and whole ones
+    alike, and turns none into NaN."""
+    nh, sq, sk = 32, 2304, 3456
+    g = torch.Generator(device=DEV).manual_seed(key)
+    mk = lambda n: torch.randn(1, n, nh, 128, device=DEV, generator=g).to(torch.bfloat16)
+    q, k, v = mk(sq), mk(sk), mk(sk)
+    v[0, key, :, 5] = float("inf")
+    v[0, key, :, 6] = float("-inf")
+    o = _flash_attn_forward(q, k, v, 0.0, SCALE, False)[0].float()
+    assert (o[..., 5] == float("inf")).all() and (o[..., 6] == float("-inf")).all()
+    assert torch.isfinite(o[..., :5]).all() and torch.isfinite(o[..., 7:]).all()

@@ -114,7 +114,7 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
 
 // fp32 partials of the last `seqlen` query rows of every sequence (what the last wave of a large dense forward leaves), into
 // rows of a bf16 tensor and statistics of out_seq tokens.  They were just written and come from the memory-side cache; with
-// 16 lanes per row and every load issued first (beyond n_parts the last part again, weight 0), a workgroup waits once.
+// 16 lanes per row and every load issued first (beyond n_parts the last part again, left out of the sum), a workgroup waits once.
 struct MergeF32Params {
   const float* o_parts; const float* lse_parts;
   int64_t o_part, lse_part;                    // elements from part to part
@@ -142,7 +142,8 @@ __global__ __launch_bounds__(256) void merge_f32_kernel(const MergeF32Params p) 
   f32x4 sum[2] = {f32x4{0}, f32x4{0}};
 #pragma unroll
   for (int i = 0; i < P; ++i) {
-    const float w = i < p.n_parts ? fast_exp2((l[i] - ms) * kLog2e) : 0.f;
+    if (i >= p.n_parts) break;                 // (the last part again: not even times 0, which would make NaN of an infinity)
+    const float w = fast_exp2((l[i] - ms) * kLog2e);
     den += w;
 #pragma unroll
     for (int u = 0; u < 2; ++u) sum[u] += x[i][u] * w;
