@@ -102,13 +102,14 @@ __device__ __forceinline__ void store_block(const __attribute__((address_space(4
 constexpr int kGroupPitch = 1040;                       // bytes between groups of 4 rows
 constexpr int kBlockPitch = 8 * kGroupPitch;            // 32 rows
 // A group's LDS: stage s holds the first operand's rows at 2s * kPitch and the second's behind them; then the statistics
-// -lse/scale and -delta of either stage.
+// -lse/scale and -delta of either stage and the waves' list entries.
 template <int kGroups>
 struct Stages : Groups<kGroups> {
   static constexpr int kPitch = Groups<kGroups>::kRows / 4 * kGroupPitch;
   static constexpr int kStatBytes = 2 * Groups<kGroups>::kRows * 4;
   static constexpr int kStat = 4 * kPitch;
-  static constexpr int kBytes = kStat + 2 * kStatBytes;
+  static constexpr int kEntries = kStat + 2 * kStatBytes;
+  static constexpr int kBytes = kEntries + 4 * Walk<kGroups, false>::kBytes;
 };
 static_assert(3 * Stages<1>::kPitch + kBlockPitch + 6 * kGroupPitch < 65536, "operand offsets fit the instructions' offset field");
 
@@ -134,6 +135,10 @@ struct PairAddr {
       keep_in_register(tr[j]);
     }
   }
+  __device__ __forceinline__ void shift(int bytes) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) { nat[j] += bytes; tr[j] += bytes; }
+  }
 };
 // Fragment reads at a compile-time offset: k-step ks of 32 rows, and 16 rows x d-block m transposed.
 template <int kOff>
@@ -149,9 +154,11 @@ __device__ __forceinline__ bf16x8 pair_tr(const PairAddr& ad, int step16, int m)
 template <int kGroups>
 struct PairStream {
   using S = Stages<kGroups>;
+  static constexpr int kCopies = 8;        // per stage and wave, the operands in turn
   const bf16 *x, *y;
   int xs, ys, xoff, yoff;
   uint32_t lds;
+  u32x4 rx, ry;                            // the tile that copies read
   __device__ __forceinline__ PairStream(const bf16* x_, int xs_, const bf16* y_, int ys_, uint32_t lds_base, int wave, int lane)
       : x(x_), y(y_), xs(xs_), ys(ys_) {
     const int row = 4 * wave + (lane >> 4), chunk = (lane & 15) ^ ((lane >> 4) << 2);
@@ -159,24 +166,28 @@ struct PairStream {
     yoff = (row * ys + chunk * 8) * 2;
     lds = __builtin_amdgcn_readfirstlane(lds_base + wave * kGroupPitch);
   }
-  __device__ __forceinline__ void copy_in(int64_t row0, int stage) const {
-    const u32x4 rx = make_rsrc_words(x + row0 * xs, (uint32_t)((S::kRows - 1) * xs + kHeadDim) * 2);
-    const u32x4 ry = make_rsrc_words(y + row0 * ys, (uint32_t)((S::kRows - 1) * ys + kHeadDim) * 2);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t at = lds + 2 * stage * S::kPitch + S::kWaves * j * kGroupPitch;
-      dma16_abs(rx, at, xoff, j * 8 * S::kWaves * xs);
-      dma16_abs(ry, at + S::kPitch, yoff, j * 8 * S::kWaves * ys);
-    }
+  // Without `more` the copies that follow read nothing and fill with zeros a stage that no step reads: no branch at each of them.
+  __device__ __forceinline__ void tile(int t, bool more) {
+    const int64_t row0 = (int64_t)t * kTile;
+    rx = make_rsrc_words(x + row0 * xs, more ? (uint32_t)((kTile - 1) * xs + kHeadDim) * 2 : 0);
+    ry = make_rsrc_words(y + row0 * ys, more ? (uint32_t)((kTile - 1) * ys + kHeadDim) * 2 : 0);
+  }
+  // copy n of kCopies into stage kStage, rows from 64 or 32 * part of the tile on
+  template <int kStage>
+  __device__ __forceinline__ void copy(int n, int part) const {
+    const int j = n >> 1, at = 2 * kStage * S::kPitch + S::kWaves * j * kGroupPitch, row = part * S::kRows + 4 * S::kWaves * j;
+    if (n & 1) dma16_abs(ry, lds + at + S::kPitch, yoff, row * ys * 2);
+    else       dma16_abs(rx, lds + at, xoff, row * xs * 2);
   }
 };
 
 // One block of 32 query rows for this wave's 32 keys.  kOff = LDS offset of the block's Q rows; dO lies kPitch
-// behind, -delta kStatBytes / 2 behind -lse/scale.
-template <int kOff, int kPitch, int kStatOff, int kStatBytes>
-__device__ __forceinline__ void dkdv_block(const PairAddr& ad, uint32_t stat, const bf16x8 (&kf)[8], const bf16x8 (&vf)[8], f32x16 (&dk)[4],
-                                           f32x16 (&dv)[4], float scale_log2, int hi, int key_b, bool mask) {
+// behind, -delta kStatBytes / 2 behind -lse/scale.  `copy(n)`, n = 0 .. kCopies - 1, is called between the first MFMAs.
+template <int kOff, int kPitch, int kStatOff, int kStatBytes, int kCopies, class Copy>
+__device__ __forceinline__ void dkdv_block(const PairAddr& ad, uint32_t stat_base, const bf16x8 (&kf)[8], const bf16x8 (&vf)[8], f32x16 (&dk)[4],
+                                           f32x16 (&dv)[4], float scale_log2, bool mask, Copy copy) {
   f32x16 s, dp;
+  const uint32_t stat = stat_base + 16 * (fresh_lane() >> 5);           // this lane half's 4 consecutive row statistics
   // element i of a block: query row 8*(i/4) + 4*hi + i%4, key column lane%32
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
@@ -187,7 +198,7 @@ __device__ __forceinline__ void dkdv_block(const PairAddr& ad, uint32_t stat, co
   }
   {
     // 16 row fragments, Q and dO alternating, fetched kAhead reads ahead of their MFMA
-    constexpr int kAhead = 3;
+    constexpr int kAhead = 2;
     bf16x8 fr[16];
     auto rd = [&](int i) { return (i & 1) ? pair_nat<kOff + kPitch>(ad, i >> 1) : pair_nat<kOff>(ad, i >> 1); };
 #pragma unroll
@@ -200,6 +211,7 @@ __device__ __forceinline__ void dkdv_block(const PairAddr& ad, uint32_t stat, co
       else       s = mfma32(fr[i], kf[i >> 1], s);
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      if ((i + 1) * kCopies / 16 != i * kCopies / 16) copy(i * kCopies / 16);
     }
   }
   // transposed fragments i: dO for i even (dV), Q for i odd (dK); d-block (i/2)%4, 16-row step i/8
@@ -211,10 +223,10 @@ __device__ __forceinline__ void dkdv_block(const PairAddr& ad, uint32_t stat, co
 #pragma unroll
   for (int i = 0; i < kTAhead; ++i) fr[i] = rd_tr(i);
   if (mask) {
-    keep_branch_local(key_b);
+    const int lane = fresh_lane(), key_b = lane & 31, hi4 = 4 * (lane >> 5);
 #pragma unroll
     for (int i = 0; i < 16; ++i)
-      if (key_b > 8 * (i >> 2) + 4 * hi + (i & 3)) s[i] = -INFINITY;
+      if (key_b > 8 * (i >> 2) + hi4 + (i & 3)) s[i] = -INFINITY;
   }
   bf16x8 pb[2], dsb[2];
 #pragma unroll
@@ -241,7 +253,7 @@ __device__ __forceinline__ void dkdv_block(const PairAddr& ad, uint32_t stat, co
 template <int kGroups>
 __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block, int block) {
   using S = Stages<kGroups>;
-  const int tid = threadIdx.x % (64 * S::kWaves), lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
+  const int tid = threadIdx.x % (64 * S::kWaves), lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int group = kGroups == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * S::kWaves));
   const uint32_t lds_base = lds_block + group * S::kBytes;
@@ -266,41 +278,38 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block
     e1 = min(max(sload(p.cols.ptr, kt + 1), e0), p.nnz);
   }
   const int64_t seq_q = (int64_t)p.n_qtiles * kTile;
-  const PairStream<kGroups> in(p.q + b * p.qs.b + h * p.qs.h, (int)p.qs.s, p.dout + b * p.ds.b + h * p.ds.h, (int)p.ds.s, lds_base, wave, lane);
-  const int n_half = (kGroups == 1 ? 2 : 1) * (e1 - e0);
-  // step i = half (i & 1) of list entry e0 + i / 2, with more groups half or quarter `group` of entry e0 + i.  The
-  // list entry (query tile, causal flag) of step i+1 is fetched one step before it is needed, so that
-  // no step starts by waiting for a scalar load.
-  auto half_of = [&](int i) { return kGroups == 1 ? i & 1 : group; };
-  auto entry = [&](int i) {           // query tile | causal flag << 30
-    if (n_half == 0) return 0;        // an empty column owns no list entry (the arrays may be NULL)
-    const int e = min(e0 + (kGroups == 1 ? i >> 1 : i), e1 - 1);
-    if (dense) return e | ((int)(e == diag) << 30);      // the entry is the query tile itself
-    return min(max(sload(p.cols.idx, e), 0), p.n_qtiles - 1) | (sload(p.cols.flag, e) << 30);
+  PairStream<kGroups> in(p.q + b * p.qs.b + h * p.qs.h, (int)p.qs.s, p.dout + b * p.ds.b + h * p.ds.h, (int)p.ds.s, lds_base, wave, lane);
+  // A step is one half of a tile, in order; with more groups half or quarter `group` of a tile.
+  Walk<kGroups, false> walk(e0, e1, diag, lds_base + S::kEntries + wave * Walk<kGroups, false>::kBytes);
+  auto fetch = [&](int e) { walk.fetch(e, dense, p.cols.idx, p.cols.flag, p.n_qtiles); };
+  // The rows' statistics of a step: its rows' -lse/softmax_scale (lse = -inf, a row without keys, stays -inf so that P = 0) and
+  // -delta, which the accumulators of S and dP' start from.  Every wave brings 16 rows of both: lanes 0..15 (and
+  // 32..47, which do the same) lse, the others delta.  They are loaded two steps before their use, turned and put into LDS a step
+  // before it: by then everything loaded has arrived at the end of a step, and nothing waits.  (Two of the waves bringing all of
+  // it, with their addresses in scratch memory, kept the other two waiting for a tenth of every step.)
+  const int64_t stat_row = ((int64_t)b * p.n_heads + h) * seq_q + 16 * wave;
+  const float *const lse_rows = p.lse + stat_row, *const delta_rows = p.delta + stat_row;
+  auto load_stat = [&](int entry, int part) {
+    const int l = fresh_lane();
+    return (l & 16 ? delta_rows : lse_rows)[walk.tile(entry) * kTile + part * S::kRows + (l & 15)];
   };
-  // rows' statistics, staged in the form the accumulators start from: threads 0..kRows-1 carry
-  // -lse/softmax_scale (lse = -inf, a row without keys, stays -inf so that P = 0), the next
-  // kRows carry -delta
-  // (the raw value is only touched when it is stored to LDS at the end of a step: no wait for
-  // the global load may land between the copies' issue and the step's work)
   const float neg_inv_scale = -1.f / p.scale;
-  const float* stat_src = (tid < S::kRows ? p.lse : p.delta) + ((int64_t)b * p.n_heads + h) * seq_q + (tid & (S::kRows - 1));
-  auto load_stat = [&](int i, int qt) {
-    float x = 0.f;
-    if (tid < 2 * S::kRows) x = stat_src[qt * kTile + half_of(i) * S::kRows];
-    return x;
-  };
   auto put_stat = [&](int stage, float x) {
-    if (tid < 2 * S::kRows) {
-      x = tid < S::kRows ? ((x == -INFINITY) ? -INFINITY : x * neg_inv_scale) : -x;
-      *reinterpret_cast<UA_LDS float*>(lds_base + S::kStat + stage * S::kStatBytes + tid * 4) = x;
-    }
+    const int l = fresh_lane();
+    const float y = x * (l & 16 ? -1.f : neg_inv_scale);
+    lds_put(lds_base + S::kStat + stage * S::kStatBytes + (16 * wave + (l & 15) + (l & 16 ? S::kRows : 0)) * 4, !(l & 16) && x == -INFINITY ? x : y);
   };
-  int ent = entry(0), ent_next = entry(1);
-  float st0 = 0.f;
-  if (n_half > 0) {
-    in.copy_in((int64_t)(ent & 0x3fffffff) * kTile + half_of(0) * S::kRows, 0);
-    st0 = load_stat(0, ent & 0x3fffffff);
+  int ent = 0, ent_next = 0;
+  float st0 = 0.f, stat = 0.f;
+  const int part0 = kGroups == 1 ? 0 : group;
+  if (e0 < e1) {
+    fetch(e0);
+    ent = walk.at(e0);
+    in.tile(walk.tile(ent), true);
+#pragma unroll
+    for (int n = 0; n < in.kCopies; ++n) in.template copy<0>(n, part0);
+    st0 = load_stat(ent, part0);
+    stat = kGroups == 1 ? load_stat(ent, 1) : load_stat(walk.at(min(e0 + 1, e1 - 1)), group);
   }
 
   // K and V rows as B operands: lane holds key row 32*k_block + lane%32, d = 16*ks + 8*hi .. +7
@@ -328,10 +337,8 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block
 #pragma unroll
   for (int i = 0; i < 4; ++i) { dk[i] = f32x16{0}; dv[i] = f32x16{0}; }
 
-  const PairAddr ad(lds_base, lane);
-  uint32_t stat_addr = lds_base + S::kStat + 16 * hi;     // this lane half's 4 consecutive row statistics
-  keep_in_register(stat_addr);
-  if (n_half > 0) put_stat(0, st0);
+  PairAddr ad(lds_base, lane);
+  if (e0 < e1) put_stat(0, st0);
   // The compiler does not see the copies that the walk has in flight.  Were the K and V rows still
   // outstanding for it there, it would wait for them by count inside the loop, i.e. for the copies: they are
   // made to arrive here.
@@ -340,37 +347,55 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block
   wait_vmem_all();
   __syncthreads();
 
-  // One step on stage i % 2: the copies of half tile i+1 go in flight into the other stage, which everyone
-  // has left at the barrier that ended step i-1.
-  auto step = [&](int i, auto stage_tag) {
+  // One step on stage kStage: the copies of the next step's rows go in flight into the other stage, which everyone has left at the
+  // barrier that ended the last step, between the MFMAs: all of them at the step's start kept a wave from its first product for
+  // 500 to 1100 of 3900 to 6900 cycles (64 bytes a cycle and CU is what the copies' path takes).
+  auto step = [&](int e, auto stage_tag) {
     constexpr int kStage = decltype(stage_tag)::value;
-    if (i >= n_half) return;           // workgroup-uniform: the column is done
-    const bool more = i + 1 < n_half, causal = (ent >> 30) != 0;
-    const int cur_next = ent_next;
-    ent = ent_next;
-    ent_next = entry(i + 2);
-    float stat = 0.f;
-    if (more) {
-      stat = load_stat(i + 1, cur_next & 0x3fffffff);
-      in.copy_in((int64_t)(cur_next & 0x3fffffff) * kTile + half_of(i + 1) * S::kRows, kStage ^ 1);
+    constexpr bool kFirst = kGroups == 1 && kStage == 0;          // the tile's second half follows
+    if (kGroups > 1 && e >= e1) return;                           // workgroup-uniform
+    if (kGroups > 1 || kFirst) {
+      if (!walk.has(e + 1)) fetch(e + 1);
+      ent_next = walk.at(min(e + 1, e1 - 1));
     }
+    put_stat(kStage ^ 1, stat);
+    stat = kGroups == 1 ? load_stat(ent_next, kStage) : load_stat(walk.at(min(e + 2, e1 - 1)), group);
+    if (!kFirst) in.tile(walk.tile(ent_next), e + 1 < e1);
+    const bool causal = (ent >> 30) != 0;
     // causal tile: query block nb sees none of the wave's keys when nb < k_block, some when nb == k_block
-    constexpr int kBlocks = S::kRows / 32, kOff = 2 * kStage * S::kPitch, kStatOff = kStage * S::kStatBytes;
-    const int nb = kBlocks * half_of(i);
-    if (!causal || nb >= k_block)
-      dkdv_block<kOff, S::kPitch, kStatOff, S::kStatBytes>(ad, stat_addr, kf, vf, dk, dv, p.scale_log2, hi, l32, causal && nb == k_block);
-    if constexpr (kBlocks == 2) {
-      if (!causal || nb + 1 >= k_block)
-        dkdv_block<kOff + kBlockPitch, S::kPitch, kStatOff + 128, S::kStatBytes>(ad, stat_addr, kf, vf, dk, dv, p.scale_log2, hi, l32,
-                                                                                 causal && nb + 1 == k_block);
+    constexpr int kBlocks = S::kRows / 32, kCopies = in.kCopies / kBlocks, kOff = 2 * kStage * S::kPitch, kStatOff = kStage * S::kStatBytes;
+    const int nb = kBlocks * (kGroups == 1 ? kStage : group), part_next = kGroups == 1 ? kStage ^ 1 : group;
+    if (!causal) {
+      auto block = [&](auto mb_tag) {
+        constexpr int kMb = decltype(mb_tag)::value;
+        dkdv_block<kOff + kMb * kBlockPitch, S::kPitch, kStatOff + kMb * 128, S::kStatBytes, kCopies>(
+            ad, lds_base + S::kStat, kf, vf, dk, dv, p.scale_log2, false, [&](int n) { in.template copy<kStage ^ 1>(kMb * kCopies + n, part_next); });
+      };
+      block(std::integral_constant<int, 0>{});
+      if constexpr (kBlocks == 2) block(std::integral_constant<int, 1>{});
     }
-    if (more) put_stat(kStage ^ 1, stat);
+    // (Not the other side of one branch, where the products do not stay in the same registers: 400 to 700 are spilled.)
+    int is_causal = __builtin_amdgcn_readfirstlane((int)causal);
+    asm volatile("" : "+s"(is_causal));
+    if (is_causal) {
+      // Rare: one block after the other from the first that sees some of the wave's keys, after the copies.
+#pragma unroll
+      for (int n = 0; n < in.kCopies; ++n) in.template copy<kStage ^ 1>(n, part_next);
+#pragma unroll 1
+      for (int mb = max(k_block - nb, 0); mb < kBlocks; ++mb) {
+        ad.shift(mb * kBlockPitch);
+        dkdv_block<kOff, S::kPitch, kStatOff, S::kStatBytes, 0>(ad, lds_base + S::kStat + mb * 128, kf, vf, dk, dv, p.scale_log2, nb + mb == k_block,
+                                                                [](int) {});
+        ad.shift(-mb * kBlockPitch);
+      }
+    }
+    if (!kFirst) ent = ent_next;
     wait_vmem_all();
     __syncthreads();     // the next stage has landed and everyone is done with this one
   };
-  for (int i = 0; i < n_half; i += 2) {
-    step(i, std::integral_constant<int, 0>{});
-    step(i + 1, std::integral_constant<int, 1>{});
+  for (int e = e0; e < e1; e += kGroups == 1 ? 1 : 2) {
+    step(e, std::integral_constant<int, 0>{});
+    step(kGroups == 1 ? e : e + 1, std::integral_constant<int, 1>{});
   }
   // everyone is done with the stages
   auto area = [&](int g) { return lds_block + (wave * kGroups + g) * kAccBytes; };       // of group g of this wave's rows
@@ -416,9 +441,9 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block
 // streamed like dK/dV's operands.  Per block of 32 keys: S^T = K Q^T and dP'^T = V dO^T - delta (16 MFMAs),
 // dS^T in the lanes, dQ^T += K^T dS^T (8 MFMAs).  A lane holds one query column, so -delta is one value per
 // lane: it is kept in 16 registers that dP's first MFMA takes as its addend, which spares 16 moves per block.
-template <int kOff, int kPitch>
+template <int kOff, int kPitch, int kCopies, class Copy, class Side>
 __device__ __forceinline__ void dq_block(const PairAddr& ad, const bf16x8 (&qf)[8], const bf16x8 (&dof)[8], const f32x16& neg_delta,
-                                         f32x16 (&dq)[4], float scale_log2, float lse2, int hi, int q_b, bool mask) {
+                                         f32x16 (&dq)[4], float scale_log2, float lse2, bool mask, Copy copy, Side side) {
   f32x16 s, dp;
   {
     // 16 row fragments, K and V alternating, fetched kAhead reads ahead of their MFMA
@@ -435,6 +460,7 @@ __device__ __forceinline__ void dq_block(const PairAddr& ad, const bf16x8 (&qf)[
       else       s = mfma32(fr[i], qf[i >> 1], i == 0 ? f32x16{0} : s);
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      if ((i + 1) * kCopies / 16 != i * kCopies / 16) copy(i * kCopies / 16);
     }
   }
   // the first K^T fragments of the dQ product are fetched now, behind the pointwise work
@@ -444,11 +470,12 @@ __device__ __forceinline__ void dq_block(const PairAddr& ad, const bf16x8 (&qf)[
   for (int i = 0; i < kTAhead; ++i) tfr[i] = pair_tr<kOff>(ad, i >> 2, i & 3);
   // element i: key 8*(i/4) + 4*hi + i%4 of the block, query column lane%32
   if (mask) {
-    keep_branch_local(q_b);
+    const int lane = fresh_lane(), q_b = lane & 31, hi4 = 4 * (lane >> 5);
 #pragma unroll
     for (int i = 0; i < 16; ++i)
-      if (8 * (i >> 2) + 4 * hi + (i & 3) > q_b) s[i] = -INFINITY;
+      if (8 * (i >> 2) + hi4 + (i & 3) > q_b) s[i] = -INFINITY;
   }
+  side();
   bf16x8 dsb[2];
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
@@ -467,7 +494,7 @@ __device__ __forceinline__ void dq_block(const PairAddr& ad, const bf16x8 (&qf)[
 template <int kGroups>
 __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_block, int block) {
   using S = Stages<kGroups>;
-  const int tid = threadIdx.x % (64 * S::kWaves), lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
+  const int tid = threadIdx.x % (64 * S::kWaves), lane = tid & 63, l32 = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int group = kGroups == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * S::kWaves));
   const uint32_t lds_base = lds_block + group * S::kBytes;
@@ -492,13 +519,17 @@ __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_block, 
     e0 = min(max(sload(p.rows.ptr, qt), 0), p.nnz);
     e1 = min(max(sload(p.rows.ptr, qt + 1), e0), p.nnz);
   }
-  const PairStream<kGroups> in(p.k + b * p.ks.b + h * p.ks.h, (int)p.ks.s, p.v + b * p.vs.b + h * p.vs.h, (int)p.vs.s, lds_base, wave, lane);
-  auto ktile = [&](int e) { return dense ? e : min(max(sload(p.rows.idx, e), 0), p.n_ktiles - 1); };
-  auto is_causal = [&](int e) { return dense ? (int)(e == diag) : sload(p.rows.flag, e); };
-
-  const int n_steps = (kGroups == 1 ? 2 : 1) * (e1 - e0);          // half tiles, as in dK/dV's walk
-  int kt = e0 < e1 ? ktile(e0) : 0;
-  if (e0 < e1) in.copy_in((int64_t)kt * kTile + group * S::kRows, 0);
+  PairStream<kGroups> in(p.k + b * p.ks.b + h * p.ks.h, (int)p.ks.s, p.v + b * p.vs.b + h * p.vs.h, (int)p.vs.s, lds_base, wave, lane);
+  Walk<kGroups, true> walk(e0, e1, diag);      // steps as in dK/dV's walk
+  auto fetch = [&](int e) { walk.fetch(e, dense, p.rows.idx, p.rows.flag, p.n_ktiles); };
+  int ent = 0, ent_next = 0;
+  if (e0 < e1) {
+    fetch(e0);
+    ent = walk.at(e0);
+    in.tile(walk.tile(ent), true);
+#pragma unroll
+    for (int n = 0; n < in.kCopies; ++n) in.template copy<0>(n, kGroups == 1 ? 0 : group);
+  }
 
   const int q_block = S::kWaves * sub + wave, qrow0 = qt * kTile + q_block * 32, qrow = qrow0 + l32;
   bf16x8 qf[8], dof[8];
@@ -538,40 +569,50 @@ __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_block, 
 #pragma unroll
   for (int ks = 0; ks < 8; ++ks) asm volatile("" : "+v"(qf[ks]), "+v"(dof[ks]));
 
-  int causal = 0, kt_ahead = 0;
-  auto step = [&](int i, auto stage_tag) {
+  auto step = [&](int e, auto stage_tag) {
     constexpr int kStage = decltype(stage_tag)::value;
-    constexpr bool kSecond = kGroups == 1 && kStage == 1, kFirst = kGroups == 1 && kStage == 0;      // half of one tile
-    if (!kSecond && i >= n_steps) return;      // workgroup-uniform
-    const int e = e0 + (kGroups == 1 ? i >> 1 : i), half = kGroups == 1 ? kStage : group;
-    if (!kSecond) causal = is_causal(e);
-    const bool more = kFirst || i + 1 < n_steps;
-    // the next tile's index: read a half tile before the copy that needs it
-    if (kFirst) kt_ahead = i + 2 < n_steps ? ktile(e + 1) : kt;
-    const int kt_next = kFirst ? kt : (kSecond ? kt_ahead : (more ? ktile(e + 1) : kt));
+    constexpr bool kFirst = kGroups == 1 && kStage == 0;          // the tile's second half follows
+    if (kGroups > 1 && e >= e1) return;                           // workgroup-uniform
+    auto look_ahead = [&]() {                                     // the next tile's entry
+      if (kGroups == 1 && !kFirst) return;
+      if (!walk.has(e + 1)) fetch(e + 1);
+      ent_next = walk.at(min(e + 1, e1 - 1));
+    };
+    if (kGroups > 1) look_ahead();
+    if (!kFirst) in.tile(walk.tile(ent_next), e + 1 < e1);
     wait_vmem_all();
-    __syncthreads();            // this stage has landed; everyone is done with the other one
-    if (more) in.copy_in((int64_t)kt_next * kTile + (kGroups == 1 ? kStage ^ 1 : group) * S::kRows, kStage ^ 1);
+    __syncthreads();            // this stage has landed; everyone is done with the other one, which the copies now fill
+    const bool causal = (ent >> 30) != 0;
     // causal tile: key block nb is hidden from the wave's queries when nb > q_block, in part when nb == q_block
-    constexpr int kBlocks = S::kRows / 32, kOff = 2 * kStage * S::kPitch;
-    const int nb = kBlocks * half;
-    if (!causal || q_block >= nb)
-      dq_block<kOff, S::kPitch>(ad, qf, dof, nd, dq, p.scale_log2, lse2, hi, l32, causal && q_block == nb);
-    if constexpr (kBlocks == 2) {
-      if (!causal || q_block >= nb + 1)
-        dq_block<kOff + kBlockPitch, S::kPitch>(ad, qf, dof, nd, dq, p.scale_log2, lse2, hi, l32, causal && q_block == nb + 1);
+    constexpr int kBlocks = S::kRows / 32, kCopies = in.kCopies / kBlocks, kOff = 2 * kStage * S::kPitch;
+    const int nb = kBlocks * (kGroups == 1 ? kStage : group), part_next = kGroups == 1 ? kStage ^ 1 : group;
+    auto block = [&](auto mb_tag) {
+      constexpr int kMb = decltype(mb_tag)::value;
+      if (!causal || q_block >= nb + kMb)
+        dq_block<kOff + kMb * kBlockPitch, S::kPitch, kCopies>(ad, qf, dof, nd, dq, p.scale_log2, lse2, causal && q_block == nb + kMb,
+                                                               [&](int n) { in.template copy<kStage ^ 1>(kMb * kCopies + n, part_next); },
+                                                               [&]() { if (kFirst && kMb == 0) look_ahead(); });
+    };
+    if (causal) {                                  // rare: the copies of the blocks that are left out
+      for (int mb = 0; mb < kBlocks; ++mb)
+        if (q_block < nb + mb)
+#pragma unroll
+          for (int n = 0; n < kCopies; ++n) in.template copy<kStage ^ 1>(mb * kCopies + n, part_next);
     }
-    kt = kt_next;
+    block(std::integral_constant<int, 0>{});
+    if constexpr (kBlocks == 2) block(std::integral_constant<int, 1>{});
+    if (!kFirst) ent = ent_next;
   };
-  for (int i = 0; i < n_steps; i += 2) {
-    step(i, std::integral_constant<int, 0>{});
-    step(i + 1, std::integral_constant<int, 1>{});
+  for (int e = e0; e < e1; e += kGroups == 1 ? 1 : 2) {
+    step(e, std::integral_constant<int, 0>{});
+    step(kGroups == 1 ? e : e + 1, std::integral_constant<int, 1>{});
   }
+  wait_vmem_all();              // the last step's copies filled with zeros a stage that is used for the results now
+  __syncthreads();
   const ParamsLate pl = params_late();
   const int64_t qrow_out = (int64_t)qt * kTile + q_block * 32, seq_out = (int64_t)pl->n_qtiles * kTile;
   auto area = [&](int g) { return lds_block + (wave * kGroups + g) * kAccBytes; };       // of group g of this wave's rows
   if constexpr (kGroups == 4) {
-    __syncthreads();
     put_acc(area(group), dq);
     __syncthreads();
     f32x16 sum{0};
@@ -582,7 +623,6 @@ __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_block, 
   } else {
     uint32_t turn = lds_base + wave * kWaveRowsBytes;                // stage 0: everyone left it before the last step
     if constexpr (kGroups == 2) {
-      __syncthreads();
       turn = area(1);
       if (group) put_acc(turn, dq);
       __syncthreads();

@@ -49,10 +49,11 @@ struct SoftmaxState {
 
 // kB blocks of 32 keys for this wave's 32 query rows.  With `mask` (wave-uniform) keys beyond
 // the query's own tile-local index are hidden; `key0` = tile-local index of the first key.
-template <int kB>
+// kCopies: `copy(n)`, n = 0 .. 7, is called between the MFMAs of S; `side()` beside the softmax.
+template <int kB, bool kCopies, class Copy, class Side>
 __device__ __forceinline__ void key_blocks(const unsigned char* sK, const unsigned char* sV, const bf16x8 (&qf)[8],
                                           f32x16 (&oacc)[4], SoftmaxState& st, const TrLane& tr, float scale_log2,
-                                          int l32, int hi, int q_local, int key0, bool mask, bool first) {
+                                          int l32, int hi, int q_block, int key0, bool mask, bool first, Copy copy, Side side) {
   // ---- S^T = K Q^T : kB blocks of 32 keys x 32 queries -----------------------------------
   // The 8 * kB K fragments are fetched kAhead reads ahead of the MFMA that consumes them, so the
   // LDS latency is covered by the preceding MFMAs instead of being paid before each one.
@@ -74,22 +75,24 @@ __device__ __forceinline__ void key_blocks(const unsigned char* sK, const unsign
       s[i % kB] = mfma32(kfr[i], qf[i / kB], s[i % kB]);
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // then 1 MFMA, 1 LDS read, ...
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      if (kCopies && (i + 1) % kB == 0) copy(i / kB);
     }
   }
-  // element (mb, i) of this lane: key key0 + 32*mb + 8*(i/4) + 4*hi + i%4, query q_local
+  // element (mb, i) of this lane: key key0 + 32*mb + 8*(i/4) + 4*hi + i%4, query 32 * q_block + lane%32 of the tile
   if (mask) {
-    keep_branch_local(q_local);
+    const int lane = fresh_lane(), q_local = 32 * q_block + (lane & 31), hi4 = 4 * (lane >> 5);
 #pragma unroll
     for (int mb = 0; mb < kB; ++mb)
 #pragma unroll
       for (int i = 0; i < 16; ++i)
-        if (key0 + 32 * mb + 8 * (i >> 2) + 4 * hi + (i & 3) > q_local) s[mb][i] = -INFINITY;
+        if (key0 + 32 * mb + 8 * (i >> 2) + hi4 + (i & 3) > q_local) s[mb][i] = -INFINITY;
   }
   // the first V^T fragments are fetched now: their latency hides behind the softmax
   constexpr int kVAhead = 3;
   bf16x8 vfr[4];
 #pragma unroll
   for (int i = 0; i < kVAhead; ++i) vfr[i] = lds_read_tr_frag<lds_off_v>(sV, tr, 16 * (i >> 2), i & 3);
+  side();
   // ---- online softmax (fp32, log2 domain) ---------------------------------------------------
   float rs = 0.f;
   bf16x8 pf[2 * kB];
@@ -192,10 +195,6 @@ __global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void fwd_kernel(const
     e0 = min(max(sload(p.row_ptr, qt), 0), p.nnz);
     e1 = min(max(sload(p.row_ptr, qt + 1), e0), p.nnz);
   }
-  // entry e of the walk: its key tile, and whether it is a causal tile
-  auto ktile = [&](int e) { return dense ? e : min(max(sload(p.col_idx, e), 0), p.n_ktiles - 1); };
-  auto is_causal = [&](int e) { return dense ? (int)(e == diag) : sload(p.flag, e); };
-
   const bf16* kbase = p.k + b * p.ks.b + h * p.ks.h;
   const bf16* vbase = p.v + b * p.vs.b + h * p.vs.h;
   const int k_stride = (int)p.ks.s, v_stride = (int)p.vs.s;
@@ -205,26 +204,47 @@ __global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void fwd_kernel(const
   const int k_half = kRows * k_stride * 2, v_half = kRows * v_stride * 2;                 // bytes of one stage in memory
   const uint32_t k_extent = (uint32_t)((kTile - 1) * k_stride + kHeadDim) * 2;            // bytes of one tile
   const uint32_t v_extent = (uint32_t)((kTile - 1) * v_stride + kHeadDim) * 2;
-  auto k_rsrc = [&](int kt) { return make_rsrc(kbase + (int64_t)kt * kTile * k_stride, k_extent); };
-  auto v_rsrc = [&](int kt) { return make_rsrc(vbase + (int64_t)kt * kTile * v_stride, v_extent); };
+  auto lds_at = [](unsigned char* x) { return (uint32_t)(uintptr_t)(lds_byte*)x; };
+  // One group copies the next stage between the MFMAs of S (pieces 0..7 in turn; at the step's start, 8 at once held a wave's first
+  // product up), several groups all of it at the start: of 64 copies per CU and step, late ones are what the next step waits for
+  // (2 x 5 heads, causal 1408 x 2688: 27.9 us, between the MFMAs 28.4 to 30.1).
+  u32x4 k_rsrc, v_rsrc;                    // the tile that copies read; without `more` they fill with zeros a stage that no step reads
+  auto tile = [&](int t, bool more) {
+    k_rsrc = make_rsrc_words(kbase + (int64_t)t * kTile * k_stride, more ? k_extent : 0);
+    v_rsrc = make_rsrc_words(vbase + (int64_t)t * kTile * v_stride, more ? v_extent : 0);
+  };
+  auto copy_piece = [&](int n, unsigned char* k_stage, unsigned char* v_stage, int part) {
+    const int j = n >> 1;                  // (the offsets of pieces 16 rows apart differ by that alone: one register each for K and V)
+    if (n & 1) dma16_abs(v_rsrc, lds_at(v_stage) + (4 * j + wave) * 1024, voff[0], part * v_half + j * 32 * v_stride);
+    else       dma16_abs(k_rsrc, lds_at(k_stage) + (4 * j + wave) * 1024, koff[0], part * k_half + j * 32 * k_stride);
+  };
+  auto copy_stage = [&](int t, unsigned char* k_stage, unsigned char* v_stage, int part) {
+    dma_rows_buf<kWaves>(k_stage, make_rsrc(kbase + (int64_t)t * kTile * k_stride, k_extent), koff, part * k_half, wave);
+    dma_rows_buf<kWaves>(v_stage, make_rsrc(vbase + (int64_t)t * kTile * v_stride, v_extent), voff, part * v_half, wave);
+  };
 
-  // step i = one stage of this group: half i % 2 of entry e0 + i / 2, else half or quarter `group` of entry e0 + i
-  const int n_steps = (kGroups == 1 ? 2 : 1) * (e1 - e0);
-  auto entry_of = [&](int i) { return e0 + (kGroups == 1 ? i >> 1 : i); };
+  // A step is one half of a tile, in order; with more groups half or quarter `group` of a tile.
+  Walk<kGroups, true> walk(e0, e1, diag);
+  auto fetch = [&](int e) { walk.fetch(e, dense, p.col_idx, p.flag, p.n_ktiles); };
   // the first stage goes in flight before anything else
-  int kt = 0;
-  if (n_steps > 0) {
-    kt = ktile(e0);
-    dma_rows_buf<kWaves>(kA, k_rsrc(kt), koff, group * k_half, wave);
-    dma_rows_buf<kWaves>(vA, v_rsrc(kt), voff, group * v_half, wave);
+  int ent = 0, ent_next = 0;
+  if (e0 < e1) {
+    fetch(e0);
+    ent = walk.at(e0);
+    if constexpr (kGroups == 1) {
+      tile(walk.tile(ent), true);
+#pragma unroll
+      for (int n = 0; n < 8; ++n) copy_piece(n, kA, vA, 0);
+    } else {
+      copy_stage(walk.tile(ent), kA, vA, group);
+    }
   }
 
   // Q fragment (B operand of S^T): lane holds query row 32*q_block + lane%32,
   // d = 16*ks + 8*(lane/32) .. +7 for ks = 0..7.
   // (through the stage that the first step fills)
   const int q_block = kWaves * sub + wave;
-  const int q_local = q_block * 32 + l32;
-  const int qrow0 = qt * kTile + q_block * 32, qrow = qrow0 + l32;
+  const int qrow0 = qt * kTile + q_block * 32;
   bf16x8 qf[8];
   if constexpr (kGroups == 1) {
     u32x4 raw[8];
@@ -236,9 +256,9 @@ __global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void fwd_kernel(const
     wait_vmem_all();
     __syncthreads();
     shared_rows_to_frags(qf, q_lds, wave);
-#pragma unroll
-    for (int ks = 0; ks < 8; ++ks) asm volatile("" : "+v"(qf[ks]));      // read before the first step's barrier
   }
+#pragma unroll
+  for (int ks = 0; ks < 8; ++ks) asm volatile("" : "+v"(qf[ks]));      // read before the first step's barrier
 
   f32x16 oacc[4];
 #pragma unroll
@@ -247,37 +267,49 @@ __global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void fwd_kernel(const
   const TrLane tr(lane);
 
   bool started = false;
-  int causal = 0, kt_ahead = 0;
-  auto step = [&](int i, auto stage_tag) {
-    constexpr int kStage = decltype(stage_tag)::value;
-    constexpr bool kSecond = kGroups == 1 && kStage == 1, kFirst = kGroups == 1 && kStage == 0;      // half of one tile
-    if (!kSecond && i >= n_steps) return;  // workgroup-uniform
-    const int e = entry_of(i), half = kGroups == 1 ? kStage : group;
-    if (!kSecond) causal = is_causal(e);
-    const bool more = kFirst || i + 1 < n_steps;
-    // the next tile's index: read a half tile before the copy that needs it
-    if (kFirst) kt_ahead = i + 2 < n_steps ? ktile(e + 1) : kt;
-    const int kt_next = kFirst ? kt : (kSecond ? kt_ahead : (more ? ktile(e + 1) : kt));
+  auto step = [&](int e, auto stage_tag) {
+    constexpr int kStage = decltype(stage_tag)::value, kBlocks = kRows / 32;
+    constexpr bool kFirst = kGroups == 1 && kStage == 0;          // the tile's second half follows
+    if (kGroups > 1 && e >= e1) return;                           // workgroup-uniform
+    auto look_ahead = [&]() {                                     // the next tile's entry
+      if (kGroups == 1 && !kFirst) return;
+      if (!walk.has(e + 1)) fetch(e + 1);
+      ent_next = walk.at(min(e + 1, e1 - 1));
+    };
+    if (kGroups > 1) look_ahead();
+    if (kGroups == 1 && !kFirst) tile(walk.tile(ent_next), e + 1 < e1);
     // this stage has landed; everyone is done with the other one
     wait_vmem_all();
     __syncthreads();
-    if (more) {
-      const int half_next = kGroups == 1 ? kStage ^ 1 : group;
-      dma_rows_buf<kWaves>(kStage ? kA : kB, k_rsrc(kt_next), koff, half_next * k_half, wave);
-      dma_rows_buf<kWaves>(kStage ? vA : vB, v_rsrc(kt_next), voff, half_next * v_half, wave);
-    }
+    unsigned char *const k_other = kStage ? kA : kB, *const v_other = kStage ? vA : vB;
+    if (kGroups > 1 && e + 1 < e1) copy_stage(walk.tile(ent_next), k_other, v_other, group);
+    auto copy = [&](int n) { copy_piece(n, k_other, v_other, kStage ^ 1); };
     // causal tile: blocks of keys beyond the wave's block of queries are hidden, that block itself in part
-    constexpr int kBlocks = kRows / 32;
+    const int half = kGroups == 1 ? kStage : group;
+    const bool causal = (ent >> 30) != 0;
     if (!causal || kBlocks * half <= q_block) {
-      key_blocks<kBlocks>(kStage ? kB : kA, kStage ? vB : vA, qf, oacc, st, tr, p.scale_log2, l32, hi, q_local, kRows * half,
-                     causal && q_block < kBlocks * half + kBlocks, kGroups == 1 ? kStage == 0 && i == 0 : !started);
+      key_blocks<kBlocks, kGroups == 1>(kStage ? kB : kA, kStage ? vB : vA, qf, oacc, st, tr, p.scale_log2, l32, hi, q_block, kRows * half,
+                                        causal && q_block < kBlocks * half + kBlocks, kGroups == 1 ? kStage == 0 && e == e0 : !started, copy,
+                                        [&]() { if (kFirst) look_ahead(); });
       started = true;
     }
-    kt = kt_next;
+    if (kGroups == 1 && kStage == 1) {
+      // the copies of a hidden half (not the other side of one branch, where the products do not stay in the same registers)
+      int hidden = (ent >> 30) * max(kBlocks * half - q_block, 0);
+      asm volatile("" : "+s"(hidden));
+      if (hidden)
+#pragma unroll
+        for (int n = 0; n < 8; ++n) copy(n);
+    }
+    if (!kFirst) ent = ent_next;
   };
-  for (int i = 0; i < n_steps; i += 2) {
-    step(i, std::integral_constant<int, 0>{});
-    step(i + 1, std::integral_constant<int, 1>{});
+  for (int e = e0; e < e1; e += kGroups == 1 ? 1 : 2) {
+    step(e, std::integral_constant<int, 0>{});
+    step(kGroups == 1 ? e : e + 1, std::integral_constant<int, 1>{});
+  }
+  if constexpr (kGroups == 1) {
+    wait_vmem_all();            // the last step's copies filled with zeros a stage that is used for the results now
+    __syncthreads();
   }
 
   // ---- epilogue: normalise, write O (bf16) and LSE (natural log) -------------------------
@@ -293,10 +325,9 @@ __global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void fwd_kernel(const
     lrow = p.part_lse + part * p.lse_part + ((int64_t)b * p.n_heads + h) * seq + row;
     o_stride = (int64_t)p.n_heads * kHeadDim;
   }
-  auto lds_at = [](unsigned char* x) { return (uint32_t)(uintptr_t)(lds_byte*)x; };
   if constexpr (kGroups == 1) {
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-    const uint32_t turn = lds_at((wave < 2 ? kA : vA) + (wave & 1) * kWaveRowsBytes);   // everyone left stage A before the last step
+    const uint32_t turn = lds_at((wave < 2 ? kA : vA) + (wave & 1) * kWaveRowsBytes);
     if (part >= 0 && p.n_whole > 0) store_rows_f32(static_cast<float*>(p.part_o) + part_at, o_stride, oacc, inv, turn);
     else                            store_rows_bf16(orow, o_stride, oacc, inv, turn);
   } else {
@@ -334,9 +365,10 @@ __global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void fwd_kernel(const
       store_block_bf16(orow + 32 * group, o_stride, o, inv, area(own) + 4096 * group);
     }
   }
-  if (hi == 0 && group == 0) {
+  const int out_lane = fresh_lane();
+  if (out_lane < 32 && group == 0) {
     const float lse = l_tot > 0.f ? (st.m_run + __builtin_amdgcn_logf(l_tot)) * kLn2 : -INFINITY;
-    lrow[l32] = lse;
+    lrow[out_lane] = lse;
   }
 }
 
