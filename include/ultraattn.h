@@ -61,8 +61,9 @@ extern "C" {
 #define UA_NOALLOC_MAX_LINES 65532   /* most query tiles + key tiles of ua_tilelist_build_device_noalloc */
 
 /* 100 * major + minor.  102: `nnz` argument of the attention entry points, ua_merge_update, the
- * no-allocation builder, `work` of ua_tilelist_build_device grown to n_qtiles + n_ktiles + 7.  104: ua_bsa_bwd.  */
-#define UA_VERSION 104
+ * no-allocation builder, `work` of ua_tilelist_build_device grown to n_qtiles + n_ktiles + 7.  104: ua_bsa_bwd.
+ * 105: ua_tilelist_build_device_scratch.  */
+#define UA_VERSION 105
 int ua_version(void);
 const char *ua_strerror(int rc);
 
@@ -109,6 +110,17 @@ int ua_tilelist_build_device(const uint8_t *block_mask, int n_qblocks, int n_kbl
                              int32_t *row_ptr, int32_t *col_idx, uint8_t *flag,
                              int32_t *col_ptr, int32_t *row_idx, uint8_t *cflag,
                              int32_t *q_order, int32_t *k_order, int32_t *work, void *stream);
+
+/* The same with a device scratch (16-byte aligned) of ua_tilelist_scratch_bytes(): masks of up to 256 x 256 blocks of up to 64 tiles
+ * are then built in two launches instead of three, and lines that share long prefixes are told apart by bits: 2 048 lines 10.5 us,
+ * global+local too (a pass through Python, host bound).  Where that is 0 (larger masks), or the scratch NULL, misaligned or too
+ * small, it is ua_tilelist_build_device.  Same arrays, same meaning of `work`.  Calls that overlap in time need a scratch each. */
+int64_t ua_tilelist_scratch_bytes(int n_qblocks, int n_kblocks, int rate);
+int ua_tilelist_build_device_scratch(const uint8_t *block_mask, int n_qblocks, int n_kblocks, int rate,
+                                     int32_t *row_ptr, int32_t *col_idx, uint8_t *flag,
+                                     int32_t *col_ptr, int32_t *row_idx, uint8_t *cflag,
+                                     int32_t *q_order, int32_t *k_order, int32_t *work,
+                                     void *scratch, int64_t scratch_bytes, void *stream);
 
 /* No counterpart in the reference.  For callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid it): the same builder as

@@ -417,13 +417,14 @@ PyObject* lists_from_mask(PyObject* const* a) {
     memcpy(host.data_ptr(), bytes, (size_t)(nqb * nkb));
     const at::Tensor m = to_device(host, (int)device);
     buf = at::empty({l.at[8]}, m.options().dtype(at::kInt));
-    const at::Tensor work = at::empty({nqt + nkt + 7}, buf.options());
+    const int64_t scratch = ua_tilelist_scratch_bytes((int)nqb, (int)nkb, (int)rate), work_words = (nqt + nkt + 7 + 3) / 4 * 4;      // (the scratch on a 16-byte boundary)
+    const at::Tensor work = at::empty({work_words + scratch / 4}, buf.options());
     l.point_into(buf.data_ptr());
     const hipStream_t st = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream();
     call("ua_tilelist_build_device", [&] {
-      return ua_tilelist_build_device((const uint8_t*)m.data_ptr(), (int)nqb, (int)nkb, (int)rate, (int32_t*)l.row_ptr, (int32_t*)l.col_idx,
-                                      (uint8_t*)l.flag, (int32_t*)l.col_ptr, (int32_t*)l.row_idx, (uint8_t*)l.cflag, (int32_t*)l.q_order,
-                                      (int32_t*)l.k_order, (int32_t*)work.data_ptr(), st);
+      return ua_tilelist_build_device_scratch((const uint8_t*)m.data_ptr(), (int)nqb, (int)nkb, (int)rate, (int32_t*)l.row_ptr, (int32_t*)l.col_idx,
+                                              (uint8_t*)l.flag, (int32_t*)l.col_ptr, (int32_t*)l.row_idx, (uint8_t*)l.cflag, (int32_t*)l.q_order,
+                                              (int32_t*)l.k_order, (int32_t*)work.data_ptr(), (int32_t*)work.data_ptr() + work_words, scratch, st);
     });
   }
   return Py_BuildValue("(NLLL)", THPVariable_Wrap(buf), (long long)nqt, (long long)nkt, (long long)nnz);
@@ -438,11 +439,12 @@ PyObject* build_lists_device(PyObject* const* a) {
     fail(PyExc_ValueError, "block_mask_dev must be a contiguous 2-D uint8 CUDA tensor");
   const int64_t nqt = m.size(0) * rate, nkt = m.size(1) * rate, cap = given >= 0 ? given : nqt * nkt;
   const int64_t room = ((cap > 1 ? cap : 1) + 3) / 4 * 4;         // not empty, whole 32-bit words of flags
-  // One allocation that the nine results are parts of, each on a 64-byte boundary: nine of them took a third of the call.
-  const int64_t bytes[9] = {4 * (nqt + 1), 4 * room, room, 4 * (nkt + 1), 4 * room, room, 4 * nqt, 4 * nkt, 4 * (nqt + nkt + 7)};
-  int64_t at_byte[10] = {0};
-  for (int i = 0; i < 9; ++i) at_byte[i + 1] = at_byte[i] + (bytes[i] + 63) / 64 * 64;
-  const at::Tensor all = at::empty({at_byte[9]}, m.options());
+  // One allocation that the nine results and the scratch are parts of, each on a 64-byte boundary: nine of them took a third of the call.
+  const int64_t scratch = ua_tilelist_scratch_bytes((int)m.size(0), (int)m.size(1), (int)rate);
+  const int64_t bytes[10] = {4 * (nqt + 1), 4 * room, room, 4 * (nkt + 1), 4 * room, room, 4 * nqt, 4 * nkt, 4 * (nqt + nkt + 7), scratch};
+  int64_t at_byte[11] = {0};
+  for (int i = 0; i < 10; ++i) at_byte[i + 1] = at_byte[i] + (bytes[i] + 63) / 64 * 64;
+  const at::Tensor all = at::empty({at_byte[10]}, m.options());
   at::Tensor t[9];
   for (int i = 0; i < 9; ++i) {
     const bool flags = i == 2 || i == 5, list = flags || i == 1 || i == 4;
@@ -456,9 +458,9 @@ PyObject* build_lists_device(PyObject* const* a) {
   auto part = [&](int i) { return (void*)((char*)base + at_byte[i]); };
   const On on(m);
   call("ua_tilelist_build_device", [&] {
-    return ua_tilelist_build_device((const uint8_t*)m.data_ptr(), (int)m.size(0), (int)m.size(1), (int)rate, (int32_t*)part(0), (int32_t*)part(1),
-                                    (uint8_t*)part(2), (int32_t*)part(3), (int32_t*)part(4), (uint8_t*)part(5), (int32_t*)part(6), (int32_t*)part(7),
-                                    (int32_t*)part(8), on.stream);
+    return ua_tilelist_build_device_scratch((const uint8_t*)m.data_ptr(), (int)m.size(0), (int)m.size(1), (int)rate, (int32_t*)part(0), (int32_t*)part(1),
+                                            (uint8_t*)part(2), (int32_t*)part(3), (int32_t*)part(4), (uint8_t*)part(5), (int32_t*)part(6),
+                                            (int32_t*)part(7), (int32_t*)part(8), part(9), scratch, on.stream);
   });
   PyObject* r = PyTuple_New(9);
   for (int i = 0; i < 9; ++i) PyTuple_SET_ITEM(r, i, THPVariable_Wrap(t[i]));

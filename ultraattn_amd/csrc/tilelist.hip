@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <atomic>
 #include <numeric>
+#include <type_traits>
 #include <vector>
 #include "ua_common.h"
 
@@ -170,9 +171,33 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void tl_count_kernel(const uin
 
 typedef __attribute__((ext_vector_type(4), aligned(4))) int32_t i32x4_any;       // at any element of a list
 typedef __attribute__((aligned(1))) uint32_t u32_any;
+// The tiles that 64 blocks of a line, of which `full` and `causal` tell the types, give it, from slot e on; returns the slot behind
+// them.  An exclusive scan of the per-block tile counts gives every lane the slot where its block's tiles go, in ascending order.
+__device__ __forceinline__ int fill_blocks(bool is_row, int sub, int rate, int i0, uint64_t full, uint64_t causal, int e, int32_t* idx, uint8_t* flg) {
+  if (!(full | causal)) return e;
+  const int lane = threadIdx.x & 63, n_causal = is_row ? sub + 1 : rate - sub, i = i0 + lane;
+  const uint64_t below = (1ull << lane) - 1;
+  const int ty = (full >> lane & 1) ? 1 : ((causal >> lane & 1) ? 2 : 0);
+  const int c = ty == 1 ? rate : (ty == 2 ? n_causal : 0);
+  int at = e + rate * __popcll(full & below) + n_causal * __popcll(causal & below);
+  // sub-tiles along the line: a row takes key sub-tiles 0..sub of a causal block (the last one
+  // causal), a column takes query sub-tiles sub..rate-1 (the first one causal)
+  const int first = (ty == 2 && !is_row) ? sub : 0;
+  // four tiles and their flags per store
+  int t = 0;
+  for (; t + 4 <= c; t += 4, at += 4) {
+    const int s = i * rate + first + t, mark = sub - first - t;           // the causal one among them, if 0..3
+    *reinterpret_cast<i32x4_any*>(idx + at) = i32x4_any{s, s + 1, s + 2, s + 3};
+    *reinterpret_cast<u32_any*>(flg + at) = ty == 2 && (unsigned)mark < 4 ? 1u << (8 * mark) : 0;
+  }
+  for (; t < c; ++t, ++at) {
+    idx[at] = i * rate + first + t;
+    flg[at] = ty == 2 && first + t == sub;
+  }
+  return e + rate * __popcll(full) + n_causal * __popcll(causal);
+}
 // fill: a workgroup first adds up the counts of its side (those before its lines give its place in the list,
-// all of them the list's length), then each wavefront walks its line 64 blocks at a time; an exclusive
-// scan of the per-block tile counts gives every lane the slot where its block's tiles go, in ascending order.
+// all of them the list's length), then each wavefront walks its line 64 blocks at a time.
 __global__ __launch_bounds__(64 * kWavesPerGroup) void tl_fill_kernel(const uint8_t* mask, int nqb, int nkb, int rate,
                                                                        const int32_t* qcnt, const int32_t* kcnt, int32_t* row_ptr, int32_t* col_idx, uint8_t* flag,
                                                                        int32_t* col_ptr, int32_t* row_idx, uint8_t* cflag,
@@ -218,35 +243,13 @@ __global__ __launch_bounds__(64 * kWavesPerGroup) void tl_fill_kernel(const uint
     ptr[ln.id] = e;
     if (ln.id == n - 1) ptr[n] = all;
   }
-  const int n_causal = causal_tiles(ln, rate);
-  const uint64_t below = (1ull << lane) - 1;
   int32_t* idx = ln.is_row ? col_idx : row_idx;
   uint8_t* flg = ln.is_row ? flag : cflag;
   for (int i0 = 0; i0 < ln.n_blocks; i0 += 64 * kAhead) {
     if (i0 > 0) load_types(mask, ln, i0, type);
 #pragma unroll
-    for (int u = 0; u < kAhead; ++u) {
-      const int i = i0 + 64 * u + lane, ty = type[u];
-      const uint64_t full = __ballot(ty == 1), causal = __ballot(ty == 2);
-      if (!(full | causal)) continue;
-      const int c = ty == 1 ? rate : (ty == 2 ? n_causal : 0);
-      int at = e + rate * __popcll(full & below) + n_causal * __popcll(causal & below);
-      // sub-tiles along the line: a row takes key sub-tiles 0..sub of a causal block (the last one
-      // causal), a column takes query sub-tiles sub..rate-1 (the first one causal)
-      const int first = (ty == 2 && !ln.is_row) ? ln.sub : 0;
-      // four tiles and their flags per store
-      int t = 0;
-      for (; t + 4 <= c; t += 4, at += 4) {
-        const int s = i * rate + first + t, mark = ln.sub - first - t;           // the causal one among them, if 0..3
-        *reinterpret_cast<i32x4_any*>(idx + at) = i32x4_any{s, s + 1, s + 2, s + 3};
-        *reinterpret_cast<u32_any*>(flg + at) = ty == 2 && (unsigned)mark < 4 ? 1u << (8 * mark) : 0;
-      }
-      for (; t < c; ++t, ++at) {
-        idx[at] = i * rate + first + t;
-        flg[at] = ty == 2 && first + t == ln.sub;
-      }
-      e += rate * __popcll(full) + n_causal * __popcll(causal);
-    }
+    for (int u = 0; u < kAhead; ++u)
+      e = fill_blocks(ln.is_row, ln.sub, rate, i0 + 64 * u, __ballot(type[u] == 1), __ballot(type[u] == 2), e, idx, flg);
   }
 }
 
@@ -387,6 +390,274 @@ __global__ __launch_bounds__(kOrderThreads) void tl_order_kernel(const int32_t* 
   if (tid < n_own) (rows ? q_order : k_order)[rank[tid]] = line0 + tid;
 }
 
+// ---- the same in two launches, for masks of up to kScanBlocks blocks a side and a caller that has scratch for them ---------------
+// The lists' places, ends and order all follow from the block lines.  The first launch leaves each of them as bits (FULL blocks,
+// CAUSAL blocks) and as what is asked of it most; the second reads that, fills the lists and ranks them, in workgroups of their own
+// that do not wait for each other.  In three launches the ranks wait for the lists, and lines with equal keys are told apart by
+// walking both.  Two dependent launches that do nothing take 5 us.  A pass of 256 x 256 blocks of 512: strided 15.8 -> 10.5 us, causal 17.0 ->
+// 10.8, global+local, whose rows all begin with the same blocks, 67.8 -> 10.3; 8 x 8 blocks of 128: 11.3 -> 8.7.
+constexpr int kScanBlocks = 256, kScanWords = kScanBlocks / 64, kListThreads = 256;
+struct BlockLine {
+  uint64_t full[kScanWords], causal[kScanWords];
+};
+struct BlockStat {
+  uint16_t n, n_causal;                    // blocks that are not EMPTY, CAUSAL ones
+  uint8_t first, last;                     // of those that are not EMPTY
+  uint8_t ends;                            // bit 0: the first is CAUSAL, 1: the last is, 2: the line holds an entry that is no Block_Type
+  uint8_t unused;
+};
+static_assert(sizeof(BlockLine) == 64 && sizeof(BlockStat) == 8, "read 16 and 8 bytes at a time");
+struct ListSide {
+  BlockLine* lines;
+  BlockStat* stats;
+  int32_t *ptr, *idx, *order;
+  uint8_t* flag;
+  int n_blocks, n_other;                   // block lines, blocks along each
+};
+// Tiles of line `sub` of a block line, and of all of its lines.
+__device__ __forceinline__ int line_tiles(const BlockStat& b, bool rows, int sub, int rate) {
+  return rate * (b.n - b.n_causal) + b.n_causal * (rows ? sub + 1 : rate - sub);
+}
+__device__ __forceinline__ int block_tiles(const BlockStat& b, int rate) { return rate * rate * (b.n - b.n_causal) + b.n_causal * (rate * (rate + 1) / 2); }
+
+__global__ __launch_bounds__(64 * kWavesPerGroup) void tl_scan_kernel(const uint8_t* mask, int nqb, int nkb, ListSide q, ListSide k) {
+  Line ln;
+  if (!line_of_wave(nqb, nkb, 1, ln)) return;
+  static_assert(kAhead == kScanWords, "a line's blocks are loaded in one go");
+  int type[kAhead];
+  load_types(mask, ln, 0, type);
+  BlockLine bits;
+  BlockStat st = {};
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u) {
+    const uint64_t full = __ballot(type[u] == 1), causal = __ballot(type[u] == 2), any = full | causal;
+    bits.full[u] = full; bits.causal[u] = causal;
+    if (__any(type[u] > 2)) st.ends |= 4;
+    if (!any) continue;
+    const int lo = __builtin_ctzll(any), hi = 63 - __builtin_clzll(any);
+    if (st.n == 0) { st.first = 64 * u + lo; st.ends |= (uint8_t)(causal >> lo & 1); }
+    st.last = 64 * u + hi;
+    st.ends = (st.ends & 5) | (uint8_t)(causal >> hi & 1) << 1;
+    st.n += __popcll(any);
+    st.n_causal += __popcll(causal);
+  }
+  if ((threadIdx.x & 63) != 0) return;
+  const ListSide& s = ln.is_row ? q : k;
+  s.lines[ln.id] = bits;
+  s.stats[ln.id] = st;
+}
+
+// One wavefront fills one line: its place is what the block lines before it hold.
+__device__ __forceinline__ void fill_line(const ListSide& s, bool rows, int rate, int id) {
+  const int lane = threadIdx.x & 63, own = id / rate, sub = id % rate;
+  BlockStat x[kScanWords];
+#pragma unroll
+  for (int u = 0; u < kScanWords; ++u) x[u] = 64 * u + lane < own ? s.stats[64 * u + lane] : BlockStat{};
+  const BlockStat me = s.stats[own];
+  const BlockLine bits = s.lines[own];
+  int e = 0;
+#pragma unroll
+  for (int u = 0; u < kScanWords; ++u) e += block_tiles(x[u], rate);
+  e = wave_sum(e) + sub * rate * (me.n - me.n_causal) + me.n_causal * (rows ? sub * (sub + 1) / 2 : sub * rate - sub * (sub - 1) / 2);
+  if (lane == 0) {
+    s.ptr[id] = e;
+    if (id == s.n_blocks * rate - 1) s.ptr[id + 1] = e + line_tiles(me, rows, sub, rate);
+  }
+#pragma unroll
+  for (int u = 0; u < kScanWords; ++u) e = fill_blocks(rows, sub, rate, 64 * u, bits.full[u], bits.causal[u], e, s.idx, s.flag);
+}
+
+// Where two block lines part, read from the anchor (distance 0 = that end of the line, kNever = nowhere): the first block that
+// only one of them holds, the first that is FULL in a and CAUSAL in b, the other way round, and CAUSAL in both.
+constexpr int kNever = 512;
+struct Parting {
+  int one, full_causal, causal_full, both_causal;
+  bool one_is_a;
+};
+__device__ __forceinline__ Parting part_lines(const BlockLine& a, const BlockLine& b, bool from_end) {
+  int d[4] = {kNever, kNever, kNever, kNever};
+  uint32_t one_is_a = 0;
+  auto words = [](const uint64_t (&x)[kScanWords], int w) { return (uint32_t)(x[w >> 1] >> (32 * (w & 1))); };
+  auto part = [&](auto towards_end) {
+    constexpr bool kEnd = decltype(towards_end)::value;
+#pragma unroll
+    for (int v = 0; v < 2 * kScanWords; ++v) {             // from the far end: the last one found is the first one met
+      const int w = kEnd ? v : 2 * kScanWords - 1 - v, base = 32 * (2 * kScanWords - 1 - v);
+      const uint32_t fa = words(a.full, w), ca = words(a.causal, w), fb = words(b.full, w), cb = words(b.causal, w);
+      const uint32_t m[4] = {(fa | ca) ^ (fb | cb), fa & cb, ca & fb, ca & cb};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int at = kEnd ? __builtin_clz(m[i] | 1) : __builtin_ctz(m[i] | 1u << 31);
+        d[i] = m[i] ? base + at : d[i];
+        if (i == 0) one_is_a = m[0] ? (fa | ca) >> (kEnd ? 31 - at : at) & 1 : one_is_a;
+      }
+    }
+  };
+  if (from_end) part(std::true_type{}); else part(std::false_type{});
+  return {d[0], d[1], d[2], d[3], one_is_a != 0};
+}
+
+// Rank of kRankLines lines among all of their side, in the order of row_precedes.  Thread t has block line t: what decides first about
+// each of its lines (very long, anchor, block-line length) is packed into one key and compared with those of the workgroup's
+// lines, and where keys are equal the block lines' bits tell which list goes on how.
+// (Keys of 32 bits, counts added up per thread, no branch in part_lines: with 64-bit keys, a ballot per comparison and a branch around every
+// word that has nothing to tell, comparing took 6 of 11 us.)
+constexpr int kRankLines = 4;          // lines of a workgroup
+constexpr int kSubs = 4;               // lines of its block that a thread compares at a time
+constexpr int kScanRate = 64;          // an index and a block line's length have 15 bits each in a key
+__device__ __forceinline__ void rank_lines(const ListSide& s, bool rows, int rate, int line0) {
+  __shared__ BlockLine own_bits[kRankLines];
+  __shared__ BlockStat own_stat[kRankLines];
+  __shared__ int32_t rank[kRankLines], sums[3][kListThreads / 64];
+  __shared__ uint32_t seen_first[kScanBlocks * kScanRate / 4], seen_last[kScanBlocks * kScanRate / 4];             // a byte per tile
+  static_assert(kListThreads == kScanBlocks, "a thread has one block line");
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = s.n_blocks * rate, n_own = min(kRankLines, n - line0), n_words = (s.n_other * rate + 3) / 4;
+  const int own0 = line0 / rate;                             // block line of the first of the workgroup's lines
+  const bool held = tid < s.n_blocks;
+  BlockStat st = {};
+  BlockLine bits = {};
+  if (held) { st = s.stats[tid]; bits = s.lines[tid]; }
+  if (tid < kRankLines) rank[tid] = 0;
+  for (int i = tid; i < n_words; i += kListThreads) seen_first[i] = seen_last[i] = 0;
+  if (tid >= own0 && tid < own0 + kRankLines) { own_bits[tid - own0] = bits; own_stat[tid - own0] = st; }
+  const int tiles = wave_sum(block_tiles(st, rate));
+  if (lane == 0) sums[0][wave] = tiles;
+  __syncthreads();
+  auto total = [&](int which) {
+    int x = 0;
+#pragma unroll
+    for (int w = 0; w < kListThreads / 64; ++w) x += sums[which][w];
+    return x;
+  };
+  const int64_t twice_all = 2 * (int64_t)total(0);
+  auto very_long = [&](int len) { return (int64_t)len * n > twice_all; };
+  auto first_tile = [&](const BlockStat& x, int sub) { return x.first * rate + (!rows && (x.ends & 1) ? sub : 0); };
+  auto last_tile = [&](const BlockStat& x, int sub) { return x.last * rate + (rows && (x.ends & 2) ? sub : rate - 1); };
+  // Which end anchors the lists: the one with fewer distinct values over the lines that are neither empty nor very long.
+  if (st.n > 0)
+    for (int sub = 0; sub < rate; ++sub)
+      if (!very_long(line_tiles(st, rows, sub, rate))) {
+        reinterpret_cast<uint8_t*>(seen_first)[first_tile(st, sub)] = 1;
+        reinterpret_cast<uint8_t*>(seen_last)[last_tile(st, sub)] = 1;
+      }
+  __syncthreads();
+  int n_first = 0, n_last = 0;
+  for (int i = tid; i < n_words; i += kListThreads) { n_first += __popc(seen_first[i]); n_last += __popc(seen_last[i]); }
+  n_first = wave_sum(n_first); n_last = wave_sum(n_last);
+  if (lane == 0) { sums[1][wave] = n_first; sums[2][wave] = n_last; }
+  __syncthreads();
+  const bool from_end = total(2) < total(1);
+  // very long lines first, among them by block-line length before the anchor; empty ones last, by number
+  auto key_of = [&](const BlockStat& x, int sub, int line) {
+    const int len = line_tiles(x, rows, sub, rate);
+    const uint32_t anchor = from_end ? last_tile(x, sub) : first_tile(x, sub), shorter = (1 << 15) - 1 - rate * x.n;
+    if (len == 0) return 1u << 31 | (uint32_t)line;
+    return very_long(len) ? shorter << 15 | anchor : 1u << 30 | anchor << 15 | shorter;
+  };
+  // lane t: line t of the workgroup
+  const int own_line = line0 + min(lane, n_own - 1), own_block = own_line / rate, own_sub = own_line - own_block * rate;
+  const uint32_t own_key = key_of(own_stat[own_block - own0], own_sub, own_line);
+  int before = 0;                      // lane t: how many of this wavefront's lines come before line t
+  if (wave == 0 && lane < n_own) {
+    // Lines of one block: their lists differ only where the block's line of the mask is CAUSAL, and by the number of such blocks in
+    // length (the same lists if there is none).  The smaller sub's comes first, or else the larger's: rows hold keys 0..sub of a CAUSAL
+    // block, so read forwards the longer list goes on in it, and read backwards the smaller sub's index there is smaller; columns hold
+    // queries sub.., so read forwards the smaller sub's index is smaller, and read backwards the larger sub leaves the last such block
+    // first, unless the list's first block is the only one, where it ends.
+    const BlockStat x = own_stat[own_block - own0];
+    const bool larger_first = x.n_causal > 0 && (rows ? !from_end : from_end && !((x.ends & 1) && x.n_causal == 1));
+    for (int sub = 0; sub < rate; ++sub) {
+      const uint32_t key = key_of(x, sub, own_block * rate + sub);
+      before += key < own_key || (key == own_key && (larger_first ? sub > own_sub : sub < own_sub));
+    }
+  }
+  for (int sub0 = 0; sub0 < rate; sub0 += kSubs) {
+    uint32_t key[kSubs];
+#pragma unroll
+    for (int u = 0; u < kSubs; ++u) key[u] = held && sub0 + u < rate ? key_of(st, sub0 + u, tid * rate + sub0 + u) : ~0u;
+    int count[kRankLines];             // of this thread's lines, how many come before line t by their keys
+    uint32_t ask = 0;                  // lines whose key a line of another block has
+#pragma unroll
+    for (int t = 0; t < kRankLines; ++t) {
+      const uint32_t key_b = __builtin_amdgcn_readlane(own_key, t);
+      const bool other = tid != __builtin_amdgcn_readlane(own_block, t);
+      uint32_t apart = ~0u;
+      count[t] = 0;
+#pragma unroll
+      for (int u = 0; u < kSubs; ++u) {
+        count[t] += key[u] < key_b;
+        apart = min(apart, key[u] ^ key_b);
+      }
+      count[t] = other ? count[t] : 0;
+      ask |= __any(apart == 0 && other) ? 1u << t : 0;
+    }
+    for (ask &= (1u << n_own) - 1; ask;) {
+      // all lines of one block: how this thread's block line and that one part
+      const int t0 = __builtin_ctz(ask), block_b = __builtin_amdgcn_readlane(own_block, t0), first_b = own_stat[block_b - own0].first;
+      const Parting p = part_lines(bits, own_bits[block_b - own0], from_end);
+      // Does line a come first, that holds more (`a_more`) tiles of the block `at` where they part?  Read forwards, the tile that only one of
+      // them holds comes next in its list.  Read backwards, the one with more tiles there holds the larger index, and comes first only
+      // if the other's list has ended.  Equal lists: by number.
+      auto comes_first = [&](int at, bool a_more) {
+        const bool ended = (a_more ? first_b : (int)st.first) >= kScanBlocks - 1 - at && (at == p.one || !rows);
+        return at == kNever ? tid < block_b : (!from_end || ended ? a_more : !a_more);
+      };
+      const bool plain = comes_first(p.one, p.one_is_a);
+#pragma unroll
+      for (int t = 0; t < kRankLines; ++t) {
+        if (!(ask >> t & 1) || __builtin_amdgcn_readlane(own_block, t) != block_b) continue;
+        ask &= ~(1u << t);
+        const uint32_t key_b = __builtin_amdgcn_readlane(own_key, t);
+        const int sub_b = __builtin_amdgcn_readlane(own_sub, t), causal_b = rows ? sub_b + 1 : rate - sub_b;
+        const int fc = causal_b < rate ? p.full_causal : kNever;
+#pragma unroll
+        for (int u = 0; u < kSubs; ++u) {
+          const int causal_a = rows ? sub0 + u + 1 : rate - sub0 - u;
+          const int cf = causal_a < rate ? p.causal_full : kNever, cc = causal_a != causal_b ? p.both_causal : kNever, at = min(fc, min(cf, cc));
+          const bool comes = at < p.one ? comes_first(at, at == fc || (at == cc && causal_a > causal_b)) : plain;
+          count[t] += key[u] == key_b && tid != block_b && comes;
+        }
+      }
+    }
+    static_assert(kRankLines == 4 && kSubs * 64 < 65536, "two lines' counts in one sum");
+    const int sum01 = wave_sum(count[0] | count[1] << 16), sum23 = wave_sum(count[2] | count[3] << 16);
+    const int sum = lane & 2 ? sum23 : sum01;
+    before += lane < kRankLines ? (lane & 1 ? sum >> 16 : sum & 0xffff) : 0;
+  }
+  if (lane < n_own && before) atomicAdd(&rank[lane], before);
+  __syncthreads();
+  if (tid < n_own) s.order[rank[tid]] = line0 + tid;
+}
+
+// Workgroups: ranks of the rows and of the columns, lines of both, and one that counts the invalid entries of the rows that hold some.
+__global__ __launch_bounds__(kListThreads) void tl_lists_kernel(const uint8_t* mask, int rate, ListSide q, ListSide k, int32_t* n_invalid) {
+  constexpr int kWaves = kListThreads / 64;
+  const int nq = q.n_blocks * rate, nk = k.n_blocks * rate, rank_q = (nq + kRankLines - 1) / kRankLines, rank_k = (nk + kRankLines - 1) / kRankLines;
+  const int fill_q = (nq + kWaves - 1) / kWaves, fill_k = (nk + kWaves - 1) / kWaves;
+  int g = blockIdx.x;
+  if (g < rank_q + rank_k) {
+    const bool rows = g < rank_q;
+    rank_lines(rows ? q : k, rows, rate, (rows ? g : g - rank_q) * kRankLines);
+    return;
+  }
+  g -= rank_q + rank_k;
+  if (g < fill_q + fill_k) {
+    const bool rows = g < fill_q;
+    const int id = __builtin_amdgcn_readfirstlane((rows ? g : g - fill_q) * kWaves + (threadIdx.x >> 6));
+    if (id < (rows ? nq : nk)) fill_line(rows ? q : k, rows, rate, id);
+    return;
+  }
+  __shared__ int32_t bad;
+  if (threadIdx.x == 0) bad = 0;
+  __syncthreads();
+  int here = 0;
+  if ((int)threadIdx.x < q.n_blocks && (q.stats[threadIdx.x].ends & 4))
+    for (int i = 0; i < q.n_other; ++i) here += mask[(int64_t)threadIdx.x * q.n_other + i] > 2;
+  if (here) atomicAdd(&bad, here);
+  __syncthreads();
+  if (threadIdx.x == 0) *n_invalid = bad;
+}
+
 }  // namespace ua
 
 extern "C" int ua_tilelist_size(const uint8_t* block_mask, int n_qblocks, int n_kblocks, int rate,
@@ -448,11 +719,28 @@ extern "C" int ua_tilelist_build(const uint8_t* block_mask, int n_qblocks, int n
 
 namespace ua {
 
+// Bytes of scratch that the two-launch build works in; 0: larger masks go through the lists.
+static int64_t scan_bytes(int n_qblocks, int n_kblocks, int rate) {
+  if (n_qblocks > kScanBlocks || n_kblocks > kScanBlocks || rate > kScanRate) return 0;
+  return (int64_t)(n_qblocks + n_kblocks) * (sizeof(BlockLine) + sizeof(BlockStat));
+}
 static int build_device_impl(const uint8_t* block_mask, int n_qblocks, int n_kblocks, int rate,
                              int32_t* row_ptr, int32_t* col_idx, uint8_t* flag,
                              int32_t* col_ptr, int32_t* row_idx, uint8_t* cflag,
-                             int32_t* q_order, int32_t* k_order, int32_t* work, int32_t* n_invalid, hipStream_t st) {
+                             int32_t* q_order, int32_t* k_order, int32_t* work, int32_t* n_invalid, void* scratch, int64_t scratch_bytes, hipStream_t st) {
   const int nqt = n_qblocks * rate, nkt = n_kblocks * rate;
+  const int64_t wanted = scan_bytes(n_qblocks, n_kblocks, rate);
+  if (scratch && wanted > 0 && scratch_bytes >= wanted && aligned16(scratch)) {
+    BlockLine* lines = static_cast<BlockLine*>(scratch);
+    BlockStat* stats = reinterpret_cast<BlockStat*>(lines + n_qblocks + n_kblocks);
+    const ListSide q = {lines, stats, row_ptr, col_idx, q_order, flag, n_qblocks, n_kblocks};
+    const ListSide k = {lines + n_qblocks, stats + n_qblocks, col_ptr, row_idx, k_order, cflag, n_kblocks, n_qblocks};
+    auto groups = [](int n, int per) { return (unsigned)((n + per - 1) / per); };
+    hipLaunchKernelGGL(tl_scan_kernel, dim3(line_groups(n_qblocks) + line_groups(n_kblocks)), dim3(64 * kWavesPerGroup), 0, st, block_mask, n_qblocks, n_kblocks, q, k);
+    hipLaunchKernelGGL(tl_lists_kernel, dim3(groups(nqt, kRankLines) + groups(nkt, kRankLines) + groups(nqt, kListThreads / 64) + groups(nkt, kListThreads / 64) + 1),
+                       dim3(kListThreads), 0, st, block_mask, rate, q, k, n_invalid);
+    return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH;
+  }
   int32_t* qcnt = work;
   int32_t* kcnt = work + nqt + 1;
   const dim3 lines((unsigned)(line_groups(nqt) + line_groups(nkt))), group(64 * kWavesPerGroup);
@@ -477,10 +765,15 @@ static int check_device_builder_args(const uint8_t* block_mask, int n_qblocks, i
 
 }  // namespace ua
 
-extern "C" int ua_tilelist_build_device(const uint8_t* block_mask, int n_qblocks, int n_kblocks, int rate,
-                                        int32_t* row_ptr, int32_t* col_idx, uint8_t* flag,
-                                        int32_t* col_ptr, int32_t* row_idx, uint8_t* cflag,
-                                        int32_t* q_order, int32_t* k_order, int32_t* work, void* stream) {
+extern "C" int64_t ua_tilelist_scratch_bytes(int n_qblocks, int n_kblocks, int rate) {
+  return n_qblocks > 0 && n_kblocks > 0 && rate > 0 ? ua::scan_bytes(n_qblocks, n_kblocks, rate) : 0;
+}
+
+extern "C" int ua_tilelist_build_device_scratch(const uint8_t* block_mask, int n_qblocks, int n_kblocks, int rate,
+                                                int32_t* row_ptr, int32_t* col_idx, uint8_t* flag,
+                                                int32_t* col_ptr, int32_t* row_idx, uint8_t* cflag,
+                                                int32_t* q_order, int32_t* k_order, int32_t* work,
+                                                void* scratch, int64_t scratch_bytes, void* stream) {
   using namespace ua;
   if (!work) return UA_ERR_NULL;
   if (int rc = check_device_builder_args(block_mask, n_qblocks, n_kblocks, rate, row_ptr, col_idx, flag, col_ptr,
@@ -488,7 +781,15 @@ extern "C" int ua_tilelist_build_device(const uint8_t* block_mask, int n_qblocks
   if (int rc = check_device()) return rc;
   const int nqt = n_qblocks * rate, nkt = n_kblocks * rate;
   return build_device_impl(block_mask, n_qblocks, n_kblocks, rate, row_ptr, col_idx, flag, col_ptr, row_idx, cflag,
-                           q_order, k_order, work, work + nqt + nkt + 2, (hipStream_t)stream);
+                           q_order, k_order, work, work + nqt + nkt + 2, scratch, scratch_bytes, (hipStream_t)stream);
+}
+
+extern "C" int ua_tilelist_build_device(const uint8_t* block_mask, int n_qblocks, int n_kblocks, int rate,
+                                        int32_t* row_ptr, int32_t* col_idx, uint8_t* flag,
+                                        int32_t* col_ptr, int32_t* row_idx, uint8_t* cflag,
+                                        int32_t* q_order, int32_t* k_order, int32_t* work, void* stream) {
+  return ua_tilelist_build_device_scratch(block_mask, n_qblocks, n_kblocks, rate, row_ptr, col_idx, flag, col_ptr, row_idx, cflag, q_order, k_order, work,
+                                          nullptr, 0, stream);
 }
 
 // The device address of `scratch`, looked up once per device with that device current.  In host
@@ -527,8 +828,10 @@ extern "C" int ua_tilelist_build_device_noalloc(const uint8_t* block_mask, int n
   if (int rc = check_device()) return rc;
   int32_t* work = nullptr;
   if (int rc = scratch_of_current_device(&work)) return rc;
-  // the counts are written before they are read and the invalid-entry count is stored, not
-  // accumulated: nothing in the scratch has to start at zero
+  // What is read is written before, and the invalid-entry count is stored, not accumulated: nothing in the scratch has to start at zero.
+  // Masks that the two-launch build takes have at most 32768 lines, which leaves it its room behind them.
+  static_assert(2 * kScanBlocks * kScanRate + 12 + 2 * kScanBlocks * (int)(sizeof(BlockLine) + sizeof(BlockStat)) / 4 <= UA_NOALLOC_MAX_LINES + 8, "fits the scratch");
+  const int64_t room = (lines + 8 + 3) / 4 * 4;
   return build_device_impl(block_mask, n_qblocks, n_kblocks, rate, row_ptr, col_idx, flag, col_ptr, row_idx, cflag,
-                           q_order, k_order, work, n_invalid ? n_invalid : work + lines + 2, (hipStream_t)stream);
+                           q_order, k_order, work, n_invalid ? n_invalid : work + lines + 2, work + room, (UA_NOALLOC_MAX_LINES + 8 - room) * 4, (hipStream_t)stream);
 }
