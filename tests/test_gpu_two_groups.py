@@ -66,3 +66,17 @@ def test_around_the_bounds(sq, sk, nh, causal):
     if causal:
         keep = torch.arange(sk)[None, :] <= torch.arange(sq)[:, None] + (sk - sq)
     _check((r[0], r[5], *g[:3]), q, k, v, do, keep, (0, nh - 1))
+
+
+@pytest.mark.parametrize("sq,sk,nh,causal", [
+    (128, 128, 65, False), (128, 128, 128, True),                # half lines: 130 and 256 lines of one tile
+    (512, 512, 32, True), (128, 256, 85, True),                  # 256 and 255 lines
+    (1024, 1024, 12, True), (1024, 1024, 13, True),              # 192 and 208 uneven ones: four groups, half lines
+    (1536, 1536, 10, True),                                      # 240 that average six tiles: four groups
+    (512, 512, 40, True), (512, 512, 41, True),                  # 320 and 328
+    (128, 128, 130, True), (256, 256, 70, True),                 # 260 of one tile, 280 of one or two
+    (512, 128, 50, True), (128, 640, 42, False),                 # empty walks on half lines; odd walks of one and five
+    (2048, 256, 6, False), (640, 1408, 5, False),                # cut columns and cut rows on half lines
+])
+def test_half_lines(sq, sk, nh, causal):
+    test_around_the_bounds(sq, sk, nh, causal)

@@ -103,13 +103,13 @@ constexpr int kGroupPitch = 1040;                       // bytes between groups 
 constexpr int kBlockPitch = 8 * kGroupPitch;            // 32 rows
 // A group's LDS: stage s holds the first operand's rows at 2s * kPitch and the second's behind them; then the statistics
 // -lse/scale and -delta of either stage and the waves' list entries.
-template <int kGroups>
-struct Stages : Groups<kGroups> {
-  static constexpr int kPitch = Groups<kGroups>::kRows / 4 * kGroupPitch;
-  static constexpr int kStatBytes = 2 * Groups<kGroups>::kRows * 4;
+template <int kForm>
+struct Stages : Groups<kForm> {
+  static constexpr int kPitch = Groups<kForm>::kRows / 4 * kGroupPitch;
+  static constexpr int kStatBytes = 2 * Groups<kForm>::kRows * 4;
   static constexpr int kStat = 4 * kPitch;
   static constexpr int kEntries = kStat + 2 * kStatBytes;
-  static constexpr int kBytes = kEntries + 4 * Walk<kGroups, false>::kBytes;
+  static constexpr int kBytes = kEntries + 4 * Walk<kForm, false>::kBytes;
 };
 static_assert(3 * Stages<1>::kPitch + kBlockPitch + 6 * kGroupPitch < 65536, "operand offsets fit the instructions' offset field");
 
@@ -151,9 +151,9 @@ __device__ __forceinline__ bf16x8 pair_tr(const PairAddr& ad, int step16, int m)
 // The walked pair of operands (Q and dO, or K and V): asynchronous copies of a group's rows into an LDS stage.
 // 4 copies per wave and operand; copy j fills group kWaves*j + wave (rows 4*kWaves*j + 4*wave ..), lane l the 16-byte
 // slot l%16 of row l/16 of the group, whose logical chunk is the slot XORed with 4 * (l/16).
-template <int kGroups>
+template <int kForm>
 struct PairStream {
-  using S = Stages<kGroups>;
+  using S = Stages<kForm>;
   static constexpr int kCopies = 8;        // per stage and wave, the operands in turn
   const bf16 *x, *y;
   int xs, ys, xoff, yoff;
@@ -245,24 +245,23 @@ __device__ __forceinline__ void dkdv_block(const PairAddr& ad, uint32_t stat_bas
   }
 }
 
-// kGroups = 2 (here and for dQ; dense rectangles only, as 4): two groups of four wavefronts share the workgroup's line, one takes the first half of every
-// tile, the other the second, each through stages of its own; the results are added through LDS.  kGroups = 4: four groups
-// of two wavefronts share half a tile's rows, each takes a block of 32 of every tile.  Where the launch
-// gives a CU one workgroup at most, one wave per SIMD would leave the matrix pipe idle between its dependent steps (2.2 us
-// per half tile of dK/dV, 0.9 of them MFMAs); the second group fills the CU without partial results in memory.
-template <int kGroups>
+// kForm (here and for dQ; other than 1 for dense rectangles only): how the workgroup's waves share the line, see Groups.  Each group walks
+// its share of every tile through stages of its own, and the results are added through LDS.  Where the launch gives a CU one workgroup of
+// four waves at most, one wave per SIMD would leave the matrix pipe idle between its dependent steps (2.2 us
+// per half tile of dK/dV, 0.9 of them MFMAs); the other groups fill the CU without partial results in memory.
+template <int kForm>
 __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block, int block) {
-  using S = Stages<kGroups>;
+  using S = Stages<kForm>;
   const int tid = threadIdx.x % (64 * S::kWaves), lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int group = kGroups == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * S::kWaves));
+  const int group = S::kCount == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * S::kWaves));
   const uint32_t lds_base = lds_block + group * S::kBytes;
   int pos, bh;
   map_block(block, p.batch * p.n_heads, p.heads_per_xcd, p.n_ktiles * p.cols.n_parts * S::kLines, pos, bh);
   const int sub = pos % S::kLines;         // which half of the tile's keys
   pos /= S::kLines;
   const int b = bh / p.n_heads, h = bh % p.n_heads;
-  const bool dense = kGroups > 1 || p.dense;
+  const bool dense = kForm > 1 || p.dense;
   int kt, e0, e1, diag = -1, part = 0;
   if (dense) {
     part = pos / p.n_ktiles;
@@ -278,9 +277,9 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block
     e1 = min(max(sload(p.cols.ptr, kt + 1), e0), p.nnz);
   }
   const int64_t seq_q = (int64_t)p.n_qtiles * kTile;
-  PairStream<kGroups> in(p.q + b * p.qs.b + h * p.qs.h, (int)p.qs.s, p.dout + b * p.ds.b + h * p.ds.h, (int)p.ds.s, lds_base, wave, lane);
+  PairStream<kForm> in(p.q + b * p.qs.b + h * p.qs.h, (int)p.qs.s, p.dout + b * p.ds.b + h * p.ds.h, (int)p.ds.s, lds_base, wave, lane);
   // A step is one half of a tile, in order; with more groups half or quarter `group` of a tile.
-  Walk<kGroups, false> walk(e0, e1, diag, lds_base + S::kEntries + wave * Walk<kGroups, false>::kBytes);
+  Walk<kForm, false> walk(e0, e1, diag, lds_base + S::kEntries + wave * Walk<kForm, false>::kBytes);
   auto fetch = [&](int e) { walk.fetch(e, dense, p.cols.idx, p.cols.flag, p.n_qtiles); };
   // The rows' statistics of a step: its rows' -lse/softmax_scale (lse = -inf, a row without keys, stays -inf so that P = 0) and
   // -delta, which the accumulators of S and dP' start from.  Every wave brings 16 rows of both: lanes 0..15 (and
@@ -301,22 +300,22 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block
   };
   int ent = 0, ent_next = 0;
   float st0 = 0.f, stat = 0.f;
-  const int part0 = kGroups == 1 ? 0 : group;
+  auto part_of = [&](int stage) { return S::kSteps * group + (S::kSteps == 2 ? stage : 0); };      // half or quarter of the tile
   if (e0 < e1) {
     fetch(e0);
     ent = walk.at(e0);
     in.tile(walk.tile(ent), true);
 #pragma unroll
-    for (int n = 0; n < in.kCopies; ++n) in.template copy<0>(n, part0);
-    st0 = load_stat(ent, part0);
-    stat = kGroups == 1 ? load_stat(ent, 1) : load_stat(walk.at(min(e0 + 1, e1 - 1)), group);
+    for (int n = 0; n < in.kCopies; ++n) in.template copy<0>(n, part_of(0));
+    st0 = load_stat(ent, part_of(0));
+    stat = S::kSteps == 2 ? load_stat(ent, part_of(1)) : load_stat(walk.at(min(e0 + 1, e1 - 1)), group);
   }
 
   // K and V rows as B operands: lane holds key row 32*k_block + lane%32, d = 16*ks + 8*hi .. +7
   // (through the stage that the first step fills)
   const int k_block = S::kWaves * sub + wave, krow0 = kt * kTile + k_block * 32;
   bf16x8 kf[8], vf[8];
-  if constexpr (kGroups == 1) {
+  if constexpr (kForm == 1) {
     u32x4 kraw[8], vraw[8];
     load_rows(kraw, p.k + b * p.ks.b + (int64_t)krow0 * p.ks.s + h * p.ks.h, p.ks.s);
     load_rows(vraw, p.v + b * p.vs.b + (int64_t)krow0 * p.vs.s + h * p.vs.h, p.vs.s);
@@ -326,8 +325,8 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block
   } else {
     const int64_t line0 = (int64_t)kt * kTile + sub * 32 * S::kWaves;
     const uint32_t k_lds = lds_block + 2 * S::kPitch, v_lds = k_lds + S::kBytes;           // stage 1 of groups 0 and 1
-    copy_shared_rows<32 * S::kWaves>(p.k + b * p.ks.b + line0 * p.ks.s + h * p.ks.h, (int)p.ks.s, k_lds);
-    copy_shared_rows<32 * S::kWaves>(p.v + b * p.vs.b + line0 * p.vs.s + h * p.vs.h, (int)p.vs.s, v_lds);
+    copy_shared_rows<32 * S::kWaves, S::kThreads>(p.k + b * p.ks.b + line0 * p.ks.s + h * p.ks.h, (int)p.ks.s, k_lds);
+    copy_shared_rows<32 * S::kWaves, S::kThreads>(p.v + b * p.vs.b + line0 * p.vs.s + h * p.vs.h, (int)p.vs.s, v_lds);
     wait_vmem_all();
     __syncthreads();
     shared_rows_to_frags(kf, k_lds, wave);
@@ -352,19 +351,19 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block
   // 500 to 1100 of 3900 to 6900 cycles (64 bytes a cycle and CU is what the copies' path takes).
   auto step = [&](int e, auto stage_tag) {
     constexpr int kStage = decltype(stage_tag)::value;
-    constexpr bool kFirst = kGroups == 1 && kStage == 0;          // the tile's second half follows
-    if (kGroups > 1 && e >= e1) return;                           // workgroup-uniform
-    if (kGroups > 1 || kFirst) {
+    constexpr bool kFirst = S::kSteps == 2 && kStage == 0;        // the tile's second half follows
+    if (S::kSteps == 1 && e >= e1) return;                        // workgroup-uniform
+    if (S::kSteps == 1 || kFirst) {
       if (!walk.has(e + 1)) fetch(e + 1);
       ent_next = walk.at(min(e + 1, e1 - 1));
     }
     put_stat(kStage ^ 1, stat);
-    stat = kGroups == 1 ? load_stat(ent_next, kStage) : load_stat(walk.at(min(e + 2, e1 - 1)), group);
+    stat = S::kSteps == 2 ? load_stat(ent_next, part_of(kStage)) : load_stat(walk.at(min(e + 2, e1 - 1)), group);
     if (!kFirst) in.tile(walk.tile(ent_next), e + 1 < e1);
     const bool causal = (ent >> 30) != 0;
     // causal tile: query block nb sees none of the wave's keys when nb < k_block, some when nb == k_block
     constexpr int kBlocks = S::kRows / 32, kCopies = in.kCopies / kBlocks, kOff = 2 * kStage * S::kPitch, kStatOff = kStage * S::kStatBytes;
-    const int nb = kBlocks * (kGroups == 1 ? kStage : group), part_next = kGroups == 1 ? kStage ^ 1 : group;
+    const int nb = kBlocks * part_of(kStage), part_next = part_of(kStage ^ 1);
     if (!causal) {
       auto block = [&](auto mb_tag) {
         constexpr int kMb = decltype(mb_tag)::value;
@@ -393,13 +392,13 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block
     wait_vmem_all();
     __syncthreads();     // the next stage has landed and everyone is done with this one
   };
-  for (int e = e0; e < e1; e += kGroups == 1 ? 1 : 2) {
+  for (int e = e0; e < e1; e += S::kSteps == 2 ? 1 : 2) {
     step(e, std::integral_constant<int, 0>{});
-    step(kGroups == 1 ? e : e + 1, std::integral_constant<int, 1>{});
+    step(S::kSteps == 2 ? e : e + 1, std::integral_constant<int, 1>{});
   }
   // everyone is done with the stages
-  auto area = [&](int g) { return lds_block + (wave * kGroups + g) * kAccBytes; };       // of group g of this wave's rows
-  if constexpr (kGroups == 2) {
+  auto area = [&](int g) { return lds_block + (wave * S::kCount + g) * kAccBytes; };       // of group g of this wave's rows
+  if constexpr (S::kCount == 2) {
     // the second group finishes dV, the first dK
     if (group) put_acc(area(1), dk); else put_acc(area(0), dv);
     __syncthreads();
@@ -408,7 +407,7 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block
       if (group) add_block(area(0), mb, dv[mb]); else add_block(area(1), mb, dk[mb]);
   }
   f32x16 dk_sum{0}, dv_sum{0};             // four groups: each finishes a block of 32 columns of both
-  if constexpr (kGroups == 4) {
+  if constexpr (kForm == 4) {
     put_acc(area(group), dk);
     __syncthreads();
 #pragma unroll
@@ -422,16 +421,16 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block
   const ParamsLate pl = params_late();
   const int64_t seq_k = (int64_t)pl->n_ktiles * kTile;
   const int64_t krow_out = (int64_t)kt * kTile + k_block * 32;
-  if constexpr (kGroups == 4) {
+  if constexpr (kForm == 4) {
     // (this wave alone reads the block of its own area that it turns through)
     const uint32_t turn = area(group) + 4096 * group;
     store_block(&pl->cols, pl->cols.out0, pl->cols.o0s.b, pl->cols.o0s.s, pl->cols.o0s.h, pl->n_heads, part, b, krow_out, h, seq_k, group, dk_sum, pl->scale, turn);
     store_block(&pl->cols, pl->cols.out1, pl->cols.o1s.b, pl->cols.o1s.s, pl->cols.o1s.h, pl->n_heads, part, b, krow_out, h, seq_k, group, dv_sum, 1.f, turn);
   } else {
-    const uint32_t turn = kGroups == 1 ? lds_base + wave * kWaveRowsBytes : area(group ^ 1);
-    if (kGroups == 1 || group == 0)
+    const uint32_t turn = kForm == 1 ? lds_base + wave * kWaveRowsBytes : area(group ^ 1);
+    if (kForm == 1 || group == 0)
       store_result(&pl->cols, pl->cols.out0, pl->cols.o0s.b, pl->cols.o0s.s, pl->cols.o0s.h, pl->n_heads, part, b, krow_out, h, seq_k, dk, pl->scale, turn);
-    if (kGroups == 1 || group == 1)
+    if (kForm == 1 || group == 1)
       store_result(&pl->cols, pl->cols.out1, pl->cols.o1s.b, pl->cols.o1s.s, pl->cols.o1s.h, pl->n_heads, part, b, krow_out, h, seq_k, dv, 1.f, turn);
   }
 }
@@ -491,12 +490,12 @@ __device__ __forceinline__ void dq_block(const PairAddr& ad, const bf16x8 (&qf)[
   }
 }
 
-template <int kGroups>
+template <int kForm>
 __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_block, int block) {
-  using S = Stages<kGroups>;
+  using S = Stages<kForm>;
   const int tid = threadIdx.x % (64 * S::kWaves), lane = tid & 63, l32 = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int group = kGroups == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * S::kWaves));
+  const int group = S::kCount == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * S::kWaves));
   const uint32_t lds_base = lds_block + group * S::kBytes;
   int pos, bh;
   map_block(block, p.batch * p.n_heads, p.heads_per_xcd, p.n_qtiles * p.rows.n_parts * S::kLines, pos, bh);
@@ -504,7 +503,7 @@ __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_block, 
   pos /= S::kLines;
   const int b = bh / p.n_heads, h = bh % p.n_heads;
   const int64_t seq_q = (int64_t)p.n_qtiles * kTile;
-  const bool dense = kGroups > 1 || p.dense;
+  const bool dense = kForm > 1 || p.dense;
   int qt, e0, e1, diag = -1, part = 0;
   if (dense) {
     part = pos / p.n_qtiles;
@@ -519,33 +518,34 @@ __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_block, 
     e0 = min(max(sload(p.rows.ptr, qt), 0), p.nnz);
     e1 = min(max(sload(p.rows.ptr, qt + 1), e0), p.nnz);
   }
-  PairStream<kGroups> in(p.k + b * p.ks.b + h * p.ks.h, (int)p.ks.s, p.v + b * p.vs.b + h * p.vs.h, (int)p.vs.s, lds_base, wave, lane);
-  Walk<kGroups, true> walk(e0, e1, diag);      // steps as in dK/dV's walk
+  PairStream<kForm> in(p.k + b * p.ks.b + h * p.ks.h, (int)p.ks.s, p.v + b * p.vs.b + h * p.vs.h, (int)p.vs.s, lds_base, wave, lane);
+  Walk<kForm, true> walk(e0, e1, diag);      // steps as in dK/dV's walk
   auto fetch = [&](int e) { walk.fetch(e, dense, p.rows.idx, p.rows.flag, p.n_ktiles); };
+  auto part_of = [&](int stage) { return S::kSteps * group + (S::kSteps == 2 ? stage : 0); };      // half or quarter of the tile
   int ent = 0, ent_next = 0;
   if (e0 < e1) {
     fetch(e0);
     ent = walk.at(e0);
     in.tile(walk.tile(ent), true);
 #pragma unroll
-    for (int n = 0; n < in.kCopies; ++n) in.template copy<0>(n, kGroups == 1 ? 0 : group);
+    for (int n = 0; n < in.kCopies; ++n) in.template copy<0>(n, part_of(0));
   }
 
   const int q_block = S::kWaves * sub + wave, qrow0 = qt * kTile + q_block * 32, qrow = qrow0 + l32;
   bf16x8 qf[8], dof[8];
   u32x4 qraw[8], doraw[8];
   const uint32_t q_lds = lds_block + 2 * S::kPitch, do_lds = q_lds + S::kBytes;            // stage 1 of groups 0 and 1
-  if constexpr (kGroups == 1) {
+  if constexpr (kForm == 1) {
     load_rows(qraw, p.q + b * p.qs.b + (int64_t)qrow0 * p.qs.s + h * p.qs.h, p.qs.s);
     load_rows(doraw, p.dout + b * p.ds.b + (int64_t)qrow0 * p.ds.s + h * p.ds.h, p.ds.s);
   } else {
     const int64_t line0 = (int64_t)qt * kTile + sub * 32 * S::kWaves;
-    copy_shared_rows<32 * S::kWaves>(p.q + b * p.qs.b + line0 * p.qs.s + h * p.qs.h, (int)p.qs.s, q_lds);
-    copy_shared_rows<32 * S::kWaves>(p.dout + b * p.ds.b + line0 * p.ds.s + h * p.ds.h, (int)p.ds.s, do_lds);
+    copy_shared_rows<32 * S::kWaves, S::kThreads>(p.q + b * p.qs.b + line0 * p.qs.s + h * p.qs.h, (int)p.qs.s, q_lds);
+    copy_shared_rows<32 * S::kWaves, S::kThreads>(p.dout + b * p.ds.b + line0 * p.ds.s + h * p.ds.h, (int)p.ds.s, do_lds);
   }
   const float lse_raw = p.lse[((int64_t)b * p.n_heads + h) * seq_q + qrow];
   const float neg_delta = -p.delta[((int64_t)b * p.n_heads + h) * seq_q + qrow];
-  if constexpr (kGroups == 1) {
+  if constexpr (kForm == 1) {
     const uint32_t turn = lds_base + 2 * S::kPitch + wave * kWaveRowsBytes;      // in the stage that the first step fills
     rows_to_frags(qf, qraw, turn);
     rows_to_frags(dof, doraw, turn);
@@ -571,21 +571,21 @@ __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_block, 
 
   auto step = [&](int e, auto stage_tag) {
     constexpr int kStage = decltype(stage_tag)::value;
-    constexpr bool kFirst = kGroups == 1 && kStage == 0;          // the tile's second half follows
-    if (kGroups > 1 && e >= e1) return;                           // workgroup-uniform
+    constexpr bool kFirst = S::kSteps == 2 && kStage == 0;        // the tile's second half follows
+    if (S::kSteps == 1 && e >= e1) return;                        // workgroup-uniform
     auto look_ahead = [&]() {                                     // the next tile's entry
-      if (kGroups == 1 && !kFirst) return;
+      if (S::kSteps == 2 && !kFirst) return;
       if (!walk.has(e + 1)) fetch(e + 1);
       ent_next = walk.at(min(e + 1, e1 - 1));
     };
-    if (kGroups > 1) look_ahead();
+    if (S::kSteps == 1) look_ahead();
     if (!kFirst) in.tile(walk.tile(ent_next), e + 1 < e1);
     wait_vmem_all();
     __syncthreads();            // this stage has landed; everyone is done with the other one, which the copies now fill
     const bool causal = (ent >> 30) != 0;
     // causal tile: key block nb is hidden from the wave's queries when nb > q_block, in part when nb == q_block
     constexpr int kBlocks = S::kRows / 32, kCopies = in.kCopies / kBlocks, kOff = 2 * kStage * S::kPitch;
-    const int nb = kBlocks * (kGroups == 1 ? kStage : group), part_next = kGroups == 1 ? kStage ^ 1 : group;
+    const int nb = kBlocks * part_of(kStage), part_next = part_of(kStage ^ 1);
     auto block = [&](auto mb_tag) {
       constexpr int kMb = decltype(mb_tag)::value;
       if (!causal || q_block >= nb + kMb)
@@ -603,16 +603,16 @@ __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_block, 
     if constexpr (kBlocks == 2) block(std::integral_constant<int, 1>{});
     if (!kFirst) ent = ent_next;
   };
-  for (int e = e0; e < e1; e += kGroups == 1 ? 1 : 2) {
+  for (int e = e0; e < e1; e += S::kSteps == 2 ? 1 : 2) {
     step(e, std::integral_constant<int, 0>{});
-    step(kGroups == 1 ? e : e + 1, std::integral_constant<int, 1>{});
+    step(S::kSteps == 2 ? e : e + 1, std::integral_constant<int, 1>{});
   }
   wait_vmem_all();              // the last step's copies filled with zeros a stage that is used for the results now
   __syncthreads();
   const ParamsLate pl = params_late();
   const int64_t qrow_out = (int64_t)qt * kTile + q_block * 32, seq_out = (int64_t)pl->n_qtiles * kTile;
-  auto area = [&](int g) { return lds_block + (wave * kGroups + g) * kAccBytes; };       // of group g of this wave's rows
-  if constexpr (kGroups == 4) {
+  auto area = [&](int g) { return lds_block + (wave * S::kCount + g) * kAccBytes; };       // of group g of this wave's rows
+  if constexpr (kForm == 4) {
     put_acc(area(group), dq);
     __syncthreads();
     f32x16 sum{0};
@@ -622,7 +622,7 @@ __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_block, 
                 pl->scale, area(group) + 4096 * group);
   } else {
     uint32_t turn = lds_base + wave * kWaveRowsBytes;                // stage 0: everyone left it before the last step
-    if constexpr (kGroups == 2) {
+    if constexpr (S::kCount == 2) {
       turn = area(1);
       if (group) put_acc(turn, dq);
       __syncthreads();
@@ -645,12 +645,12 @@ __global__ __launch_bounds__(Groups<1>::kThreads, 2) void dq_kernel(const BwdPar
   dq_walk<1>(p, (uint32_t)(uintptr_t)(UA_LDS unsigned char*)smem, blockIdx.x);
 }
 // Both sides in one launch.
-template <int kGroups>
-__global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void bwd_kernel(const BwdParams p) {
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[kGroups * Stages<kGroups>::kBytes];
+template <int kForm>
+__global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void bwd_kernel(const BwdParams p) {
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[Stages<kForm>::kCount * Stages<kForm>::kBytes];
   const uint32_t lds_base = (uint32_t)(uintptr_t)(UA_LDS unsigned char*)smem;
-  if ((int)blockIdx.x < p.n_col_blocks) dkdv_walk<kGroups>(p, lds_base, blockIdx.x);
-  else                                  dq_walk<kGroups>(p, lds_base, blockIdx.x - p.n_col_blocks);
+  if ((int)blockIdx.x < p.n_col_blocks) dkdv_walk<kForm>(p, lds_base, blockIdx.x);
+  else                                  dq_walk<kForm>(p, lds_base, blockIdx.x - p.n_col_blocks);
 }
 
 static int fill_common(BwdParams& p, const void* q, const void* k, const void* v, const void* dout,
@@ -698,29 +698,38 @@ static int fill_side(BwdSide& s, int nnz, const int32_t* ptr, const int32_t* idx
 static int launched() { return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH; }
 static unsigned col_blocks(const BwdParams& p) { return (unsigned)(p.batch * p.n_heads * p.n_ktiles * p.cols.n_parts); }
 static unsigned row_blocks(const BwdParams& p) { return (unsigned)(p.batch * p.n_heads * p.n_qtiles * p.rows.n_parts); }
-// Groups per workgroup for n lines of 128 rows on both sides of a dense rectangle together (parts counted), as in the
-// forward: four while half lines leave a CU one workgroup at most (8 heads of 1024: 34 us with one group, 31 with two, 24
-// with four), two up to one per CU and from three tiles a walk on.  Of an uncut causal rectangle, whose lines differ in
-// length, four up to 256 lines that average four tiles (8 heads of 2048: 54 us with two, 44 with four) and two up to 512 that
-// average eight (8 of 4096: 140 us with one, 132 with two; 32 of 1024: 42, 54).  Tile lists run with one, as in the forward.
-static int bwd_groups(int64_t n, int64_t both_walks, int n_parts, bool dense_causal, int n_qtiles, int n_ktiles) {
+// The form (see Groups) for n lines of 128 rows on both sides of a dense rectangle together (parts counted), as in the forward:
+//  - four groups while half lines leave a CU one workgroup at most (8 heads of 1024: 34 us with one group, 31 with two, 24
+//    with four).  Of an uncut causal rectangle, whose lines differ in length, up to 256 lines that average four tiles (8
+//    heads of 2048: 54 us with two, 44 with four), beyond 192 that average six (16 of 1024: 25.2, in halves 23.8).
+//  - half lines of two groups up to 256 lines, and up to 320 of an uncut causal rectangle: the columns' half lines, which take longer,
+//    share the CUs with the rows', and the two workgroups of a CU are in different phases of their steps.  Against two groups
+//    on whole lines, which fill a CU with one workgroup each: 32 heads of 512 21.1 -> 19.5 us, causal 18.1 -> 15.6; 40 of 256
+//    14.5 -> 11.5; 16 of 1024 32.4 -> 30.4; causal 20 of 1024, 320 lines, 37.2 -> 29.0 against one group.  Beyond, and where lines
+//    average one tile (causal 150 of 128: 14.1, in halves 17.5), whole lines of one group fill the device as well and copy half as
+//    much (40 heads of 512: 25.2, in halves 28.7).
+//  - two groups for an uncut causal rectangle of up to 512 lines that average eight tiles (8 of 4096: 140 us with one, 132 with two).
+// Tile lists run with one, as in the forward.
+static int bwd_form(int64_t n, int64_t both_walks, int n_parts, bool dense_causal, int n_qtiles, int n_ktiles) {
   const bool uneven = dense_causal && n_parts == 2;
-  if (both_walks >= 3 && (2 * n <= kCus || (uneven && n <= kCus && both_walks >= 16))) return 4;
-  if (both_walks < 6) return 1;
-  return n <= kCus || (uneven && n <= 2 * kCus && n_qtiles >= 16 && n_ktiles >= 16) ? 2 : 1;
+  if (both_walks >= 3 && 2 * n <= kCus) return 4;
+  if (uneven && n <= kCus && both_walks >= (4 * n <= 3 * kCus ? 16 : 24)) return 4;
+  if (2 * n > kCus && (n <= kCus || (uneven && 4 * n <= 5 * kCus && both_walks >= 4))) return kHalves;
+  return uneven && n <= 2 * kCus && n_qtiles >= 16 && n_ktiles >= 16 ? 2 : 1;
 }
-// `plain`: one group per workgroup.
+// `plain`: form 1.
 static int launch_bwd(BwdParams& p, bool plain, hipStream_t st) {
   const unsigned n = col_blocks(p) + row_blocks(p);
-  const int groups = plain ? 1 : bwd_groups(n, p.cols.part_len + p.rows.part_len, p.cols.n_parts + p.rows.n_parts, p.dense_causal, p.n_qtiles, p.n_ktiles);
-  p.n_col_blocks = (int)col_blocks(p) * (groups == 4 ? 2 : 1);
+  const int form = plain ? 1 : bwd_form(n, p.cols.part_len + p.rows.part_len, p.cols.n_parts + p.rows.n_parts, p.dense_causal, p.n_qtiles, p.n_ktiles);
+  p.n_col_blocks = (int)col_blocks(p) * (form > 2 ? 2 : 1);
   // Up to two workgroups per CU the whole launch is resident at once, and the second 256 join the first in launch
   // order.  Both sides come longest first (lists roughly); the columns are then taken in reverse, so that the long ones
   // of one side share a CU with the short ones of the other (32 causal heads of 1024: 43.6 -> 41.5 us).
-  p.cols_reversed = groups == 1 && (p.dense_causal || !p.dense) && n > kCus && n <= 2 * kCus;
-  switch (groups) {
+  p.cols_reversed = form == kHalves ? p.dense_causal : form == 1 && (p.dense_causal || !p.dense) && n > kCus && n <= 2 * kCus;
+  switch (form) {
     case 4: hipLaunchKernelGGL(bwd_kernel<4>, dim3(2 * n), dim3(512), 0, st, p); break;
     case 2: hipLaunchKernelGGL(bwd_kernel<2>, dim3(n), dim3(512), 0, st, p); break;
+    case kHalves: hipLaunchKernelGGL(bwd_kernel<kHalves>, dim3(2 * n), dim3(Groups<kHalves>::kThreads), 0, st, p); break;
     default: hipLaunchKernelGGL(bwd_kernel<1>, dim3(n), dim3(256), 0, st, p);
   }
   return launched();
@@ -730,9 +739,9 @@ static int launch_bwd(BwdParams& p, bool plain, hipStream_t st) {
 // small rectangle enough workgroups for the device and costs the partials' way through memory and a
 // second launch; which wins is decided by an estimate of the launch's time in microseconds, fitted to 47 shapes of 1
 // to 32 heads and 128 to 8192 tokens (the cut it takes is within 4 % of the best one on each):
-//  - 6.5 to start, load the resident rows, store the results and end, 9.8 with two groups per workgroup, 7.1 with four;
-//  - a tile takes 1.9 (columns) or 1 (rows) with four groups, 2.6 and 1.7 with two, else 3.5 and 2.1, and 4.9 and 5.5
-//    where two workgroups share the CU;
+//  - 6.5 to start, load the resident rows, store the results and end, 9.8 in form 2, 7.1 in form 4, 6.3 in halves;
+//  - a tile takes 1.9 (columns) or 1 (rows) in form 4, 2.6 and 1.7 in form 2, 2.4 and 1.8 in halves (5.6 together on a full device), else
+//    3.5 and 2.1, and 4.9 and 5.5 where two workgroups share the CU;
 //  - the sum takes 2.4, and the partials 1 per 3.7 MB; a cut has to win by 6 %.
 // 1024 x 4096, one head: 42 us uncut, 24 cut in 2 and 4.
 struct BwdCut { int cols, rows; };
@@ -752,16 +761,17 @@ static BwdCut bwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int 
     for (int i = 0; i < n_rows; ++i) {
       const int pr = kParts[i], rlen = row_len[i];
       const float groups = (wk * pc + wq * pr) * density;
-      float us, tc, tr;
-      switch (bwd_groups(nbh * ((int64_t)n_ktiles * pc + (int64_t)n_qtiles * pr), clen + rlen, pc + pr, causal, n_qtiles, n_ktiles)) {
+      float us, tc, tr, least = all;                                       // the work of a CU, however long the walks
+      switch (bwd_form(nbh * ((int64_t)n_ktiles * pc + (int64_t)n_qtiles * pr), clen + rlen, pc + pr, causal, n_qtiles, n_ktiles)) {
         case 4: us = 7.1f; tc = 1.86f; tr = 0.96f; break;
         case 2: us = 9.8f; tc = 2.6f; tr = 1.7f; break;
+        case kHalves: us = 6.3f; tc = 2.4f; tr = 1.8f; least = density * wk * n_qtiles * 5.6f / kCus; break;
         default: {
           const float shared = fminf(fmaxf((groups - kCus) / kCus, 0.f), 1.f);       // share of the workgroups with a neighbour
           us = 6.5f; tc = 3.5f + 1.44f * shared; tr = 2.1f + 3.37f * shared;
         }
       }
-      us += fmaxf(fmaxf(clen * tc, rlen * tr), all);
+      us += fmaxf(fmaxf(clen * tc, rlen * tr), least);
       if (pc > 1 || pr > 1) us = (us + 2.4f) * 1.06f;
       if (pc > 1) us += 2.f * pc * wk * (kTile * kHeadDim * 4) / 3.7e6f;
       if (pr > 1) us += pr * wq * (kTile * kHeadDim * 4) / 3.7e6f;

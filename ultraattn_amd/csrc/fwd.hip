@@ -146,26 +146,25 @@ __device__ __forceinline__ void key_blocks(const unsigned char* sK, const unsign
   }
 }
 
-// kGroups = 2 (dense rectangles only, as 4): two groups of four wavefronts share the query tile, one takes the first 64 keys of every tile, the
-// other the second; their results are combined through LDS.  kGroups = 4: four groups of two wavefronts share half
-// a query tile, each takes 32 keys of every tile.  A launch that gives a CU one workgroup at most runs it at
-// one wave per SIMD, where a half tile takes 1.2 us of which the matrix pipe is busy 0.4; with the second group the CU is
+// kForm (1, 2 or 4; other than 1 for dense rectangles only): how the workgroup's waves share the query tile, see Groups; the groups' results
+// are combined through LDS.  A launch that gives a CU one workgroup of four waves at most runs it at
+// one wave per SIMD, where a half tile takes 1.2 us of which the matrix pipe is busy 0.4; with more groups the CU is
 // as full as with two workgroups, without partial results in memory.
-template <int kGroups>
-__global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void fwd_kernel(const FwdParams p) {
-  constexpr int kWaves = Groups<kGroups>::kWaves, kRows = Groups<kGroups>::kRows, kLines = Groups<kGroups>::kLines;
+template <int kForm>
+__global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void fwd_kernel(const FwdParams p) {
+  constexpr int kWaves = Groups<kForm>::kWaves, kRows = Groups<kForm>::kRows, kLines = Groups<kForm>::kLines;
   constexpr int kStageBytes = kRows * kRowBytes;
   // two pipeline stages per group, distinct arrays so that reads of one stage need not wait for the
   // copies in flight into the other
-  __shared__ __attribute__((aligned(1024))) unsigned char sKA[kGroups * kStageBytes];
-  __shared__ __attribute__((aligned(1024))) unsigned char sVA[kGroups * kStageBytes];
-  __shared__ __attribute__((aligned(1024))) unsigned char sKB[kGroups * kStageBytes];
-  __shared__ __attribute__((aligned(1024))) unsigned char sVB[kGroups * kStageBytes];
+  __shared__ __attribute__((aligned(1024))) unsigned char sKA[kForm * kStageBytes];
+  __shared__ __attribute__((aligned(1024))) unsigned char sVA[kForm * kStageBytes];
+  __shared__ __attribute__((aligned(1024))) unsigned char sKB[kForm * kStageBytes];
+  __shared__ __attribute__((aligned(1024))) unsigned char sVB[kForm * kStageBytes];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave_in_block = __builtin_amdgcn_readfirstlane(tid >> 6);
   // (group a constant for one group: the stages' addresses then are constants too, ten additions fewer per tile)
-  const int wave = kGroups == 1 ? wave_in_block : wave_in_block % kWaves, group = kGroups == 1 ? 0 : wave_in_block / kWaves;
+  const int wave = kForm == 1 ? wave_in_block : wave_in_block % kWaves, group = kForm == 1 ? 0 : wave_in_block / kWaves;
   unsigned char *const kA = sKA + group * kStageBytes, *const vA = sVA + group * kStageBytes;
   unsigned char *const kB = sKB + group * kStageBytes, *const vB = sVB + group * kStageBytes;
   const int l32 = lane & 31, hi = lane >> 5;
@@ -175,7 +174,7 @@ __global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void fwd_kernel(const
   pos /= kLines;
   if (pos < p.n_first) pos = p.n_first - 1 - pos;
   const int b = bh / p.n_heads, h = bh % p.n_heads;
-  const bool dense = kGroups > 1 || p.dense;
+  const bool dense = kForm > 1 || p.dense;
   int qt, e0, e1, diag = -1, part = -1;
   if (dense) {
     int line = pos;
@@ -224,14 +223,14 @@ __global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void fwd_kernel(const
   };
 
   // A step is one half of a tile, in order; with more groups half or quarter `group` of a tile.
-  Walk<kGroups, true> walk(e0, e1, diag);
+  Walk<kForm, true> walk(e0, e1, diag);
   auto fetch = [&](int e) { walk.fetch(e, dense, p.col_idx, p.flag, p.n_ktiles); };
   // the first stage goes in flight before anything else
   int ent = 0, ent_next = 0;
   if (e0 < e1) {
     fetch(e0);
     ent = walk.at(e0);
-    if constexpr (kGroups == 1) {
+    if constexpr (kForm == 1) {
       tile(walk.tile(ent), true);
 #pragma unroll
       for (int n = 0; n < 8; ++n) copy_piece(n, kA, vA, 0);
@@ -246,7 +245,7 @@ __global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void fwd_kernel(const
   const int q_block = kWaves * sub + wave;
   const int qrow0 = qt * kTile + q_block * 32;
   bf16x8 qf[8];
-  if constexpr (kGroups == 1) {
+  if constexpr (kForm == 1) {
     u32x4 raw[8];
     load_rows(raw, p.q + b * p.qs.b + (int64_t)qrow0 * p.qs.s + h * p.qs.h, p.qs.s);
     rows_to_frags(qf, raw, (uint32_t)(uintptr_t)(lds_byte*)((wave < 2 ? kB : vB) + (wave & 1) * kWaveRowsBytes));
@@ -269,31 +268,31 @@ __global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void fwd_kernel(const
   bool started = false;
   auto step = [&](int e, auto stage_tag) {
     constexpr int kStage = decltype(stage_tag)::value, kBlocks = kRows / 32;
-    constexpr bool kFirst = kGroups == 1 && kStage == 0;          // the tile's second half follows
-    if (kGroups > 1 && e >= e1) return;                           // workgroup-uniform
+    constexpr bool kFirst = kForm == 1 && kStage == 0;          // the tile's second half follows
+    if (kForm > 1 && e >= e1) return;                           // workgroup-uniform
     auto look_ahead = [&]() {                                     // the next tile's entry
-      if (kGroups == 1 && !kFirst) return;
+      if (kForm == 1 && !kFirst) return;
       if (!walk.has(e + 1)) fetch(e + 1);
       ent_next = walk.at(min(e + 1, e1 - 1));
     };
-    if (kGroups > 1) look_ahead();
-    if (kGroups == 1 && !kFirst) tile(walk.tile(ent_next), e + 1 < e1);
+    if (kForm > 1) look_ahead();
+    if (kForm == 1 && !kFirst) tile(walk.tile(ent_next), e + 1 < e1);
     // this stage has landed; everyone is done with the other one
     wait_vmem_all();
     __syncthreads();
     unsigned char *const k_other = kStage ? kA : kB, *const v_other = kStage ? vA : vB;
-    if (kGroups > 1 && e + 1 < e1) copy_stage(walk.tile(ent_next), k_other, v_other, group);
+    if (kForm > 1 && e + 1 < e1) copy_stage(walk.tile(ent_next), k_other, v_other, group);
     auto copy = [&](int n) { copy_piece(n, k_other, v_other, kStage ^ 1); };
     // causal tile: blocks of keys beyond the wave's block of queries are hidden, that block itself in part
-    const int half = kGroups == 1 ? kStage : group;
+    const int half = kForm == 1 ? kStage : group;
     const bool causal = (ent >> 30) != 0;
     if (!causal || kBlocks * half <= q_block) {
-      key_blocks<kBlocks, kGroups == 1>(kStage ? kB : kA, kStage ? vB : vA, qf, oacc, st, tr, p.scale_log2, l32, hi, q_block, kRows * half,
-                                        causal && q_block < kBlocks * half + kBlocks, kGroups == 1 ? kStage == 0 && e == e0 : !started, copy,
+      key_blocks<kBlocks, kForm == 1>(kStage ? kB : kA, kStage ? vB : vA, qf, oacc, st, tr, p.scale_log2, l32, hi, q_block, kRows * half,
+                                        causal && q_block < kBlocks * half + kBlocks, kForm == 1 ? kStage == 0 && e == e0 : !started, copy,
                                         [&]() { if (kFirst) look_ahead(); });
       started = true;
     }
-    if (kGroups == 1 && kStage == 1) {
+    if (kForm == 1 && kStage == 1) {
       // the copies of a hidden half (not the other side of one branch, where the products do not stay in the same registers)
       int hidden = (ent >> 30) * max(kBlocks * half - q_block, 0);
       asm volatile("" : "+s"(hidden));
@@ -303,11 +302,11 @@ __global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void fwd_kernel(const
     }
     if (!kFirst) ent = ent_next;
   };
-  for (int e = e0; e < e1; e += kGroups == 1 ? 1 : 2) {
+  for (int e = e0; e < e1; e += kForm == 1 ? 1 : 2) {
     step(e, std::integral_constant<int, 0>{});
-    step(kGroups == 1 ? e : e + 1, std::integral_constant<int, 1>{});
+    step(kForm == 1 ? e : e + 1, std::integral_constant<int, 1>{});
   }
-  if constexpr (kGroups == 1) {
+  if constexpr (kForm == 1) {
     wait_vmem_all();            // the last step's copies filled with zeros a stage that is used for the results now
     __syncthreads();
   }
@@ -325,32 +324,32 @@ __global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void fwd_kernel(const
     lrow = p.part_lse + part * p.lse_part + ((int64_t)b * p.n_heads + h) * seq + row;
     o_stride = (int64_t)p.n_heads * kHeadDim;
   }
-  if constexpr (kGroups == 1) {
+  if constexpr (kForm == 1) {
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
     const uint32_t turn = lds_at((wave < 2 ? kA : vA) + (wave & 1) * kWaveRowsBytes);
     if (part >= 0 && p.n_whole > 0) store_rows_f32(static_cast<float*>(p.part_o) + part_at, o_stride, oacc, inv, turn);
     else                            store_rows_bf16(orow, o_stride, oacc, inv, turn);
   } else {
-    // the groups exchange their rows' max, sum and O.  Area x of the stages' LDS belongs to group x % kGroups of wave x / kGroups.
+    // the groups exchange their rows' max, sum and O.  Area x of the stages' LDS belongs to group x % kForm of wave x / kForm.
     __shared__ float stat[8][2][64];
     auto area = [&](int x) { return lds_at(x < 2 ? sKA : x < 4 ? sVA : x < 6 ? sKB : sVB) + (x & 1) * kAccBytes; };
-    const int own = wave * kGroups + group;
-    constexpr bool kAll = kGroups == 2;        // the first group finishes whole rows; with four groups each a block of 32 columns
+    const int own = wave * kForm + group;
+    constexpr bool kAll = kForm == 2;        // the first group finishes whole rows; with four groups each a block of 32 columns
     __syncthreads();
     stat[own][0][lane] = st.m_run;
     stat[own][1][lane] = l_tot;
     if (!kAll || group == 1) put_acc(area(own), oacc);
     __syncthreads();
     if (kAll && group == 1) return;
-    float m = -INFINITY, w[kGroups];
+    float m = -INFINITY, w[kForm];
 #pragma unroll
-    for (int g = 0; g < kGroups; ++g) m = fmaxf(m, stat[wave * kGroups + g][0][lane]);
+    for (int g = 0; g < kForm; ++g) m = fmaxf(m, stat[wave * kForm + g][0][lane]);
     const float ms = m == -INFINITY ? 0.f : m;
     l_tot = 0.f;
 #pragma unroll
-    for (int g = 0; g < kGroups; ++g) {
-      w[g] = fast_exp2(stat[wave * kGroups + g][0][lane] - ms);
-      l_tot += stat[wave * kGroups + g][1][lane] * w[g];
+    for (int g = 0; g < kForm; ++g) {
+      w[g] = fast_exp2(stat[wave * kForm + g][0][lane] - ms);
+      l_tot += stat[wave * kForm + g][1][lane] * w[g];
     }
     st.m_run = m;
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
@@ -361,7 +360,7 @@ __global__ __launch_bounds__(Groups<kGroups>::kThreads, 2) void fwd_kernel(const
     } else {
       f32x16 o{0};
 #pragma unroll
-      for (int g = 0; g < kGroups; ++g) add_block(area(wave * kGroups + g), group, o, 1.f, w[g]);
+      for (int g = 0; g < kForm; ++g) add_block(area(wave * kForm + g), group, o, 1.f, w[g]);
       store_block_bf16(orow + 32 * group, o_stride, o, inv, area(own) + 4096 * group);
     }
   }

@@ -129,18 +129,18 @@ __device__ __forceinline__ u32x4 make_rsrc_words(const void* base, uint32_t byte
   return r;
 }
 
-// Rows that all groups of a workgroup of 512 threads hold as B operands: copied once, straight into LDS in the same layout,
+// Rows that all groups of a workgroup hold as B operands: copied once, straight into LDS in the same layout,
 // with wave w taking the fours of rows j with j % 4 == w % 4, whose source chunks then are one offset.  Every wave loading
 // its own, 128 KiB a workgroup, made the first loads of dK/dV last 3.4 us.
-template <int kRows>
+template <int kRows, int kThreads = 512>
 __device__ __forceinline__ void copy_shared_rows(const bf16* rows, int row_stride, uint32_t lds) {
   const int lane = fresh_lane(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = 4 * (w & 3) + (lane >> 4);                  // row within 16
   const int voff = (r * row_stride + ((lane & 15) ^ r) * 8) * 2;
   const u32x4 rsrc = make_rsrc_words(rows, (uint32_t)((kRows - 1) * row_stride + kHeadDim) * 2);
 #pragma unroll
-  for (int i = 0; i < kRows / 32; ++i) {
-    const int sixteen = 2 * i + (w >> 2);
+  for (int i = 0; i < kRows * 256 / (16 * kThreads); ++i) {
+    const int sixteen = kThreads / 256 * i + (w >> 2);
     dma16_abs(rsrc, lds + (4 * sixteen + (w & 3)) * 1024, voff, sixteen * 32 * row_stride);
   }
 }
@@ -235,38 +235,45 @@ __device__ __forceinline__ void add_block(uint32_t lds, int mb, f32x16& acc, flo
     for (int j = 0; j < 4; ++j) acc[4 * i + j] = acc[4 * i + j] * wa + x[j] * wb;
   }
 }
-// What the attention kernels' groups share: with 1 or 2 groups a group is four waves, its line the 128 rows of a tile and its
-// stage a half tile of the other side; with 4 groups two waves, half a tile's rows (64) and a block of 32.
-template <int kGroups>
+// How a workgroup's waves share a line, by kForm:
+//   1       one group of four waves, the 128 rows of a tile, both halves of every tile of the other side one after the other;
+//   2       two groups of four waves on those rows, each takes a half of every tile;
+//   4       four groups of two waves on half a tile's rows (64), each takes a quarter of every tile;
+//   kHalves two groups of two waves on half a tile's rows, each takes two quarters one after the other.
+// Forms 2 and 4 fill a CU with one workgroup, 1 and kHalves with two.
+constexpr int kHalves = 3;
+template <int kForm>
 struct Groups {
-  static constexpr int kWaves = kGroups == 4 ? 2 : 4;
-  static constexpr int kRows = kGroups == 4 ? 32 : 64;         // rows per stage
-  static constexpr int kLines = kGroups == 4 ? 2 : 1;          // lines per tile
-  static constexpr int kThreads = kGroups == 1 ? 256 : 512;
+  static constexpr int kCount = kForm == kHalves ? 2 : kForm;  // groups
+  static constexpr int kLines = kForm > 2 ? 2 : 1;             // lines per tile
+  static constexpr int kWaves = 4 / kLines;                    // of a group
+  static constexpr int kRows = 64 / kLines;                    // rows per stage
+  static constexpr int kSteps = 2 * kLines / kCount;           // of a group per tile
+  static constexpr int kThreads = 64 * kWaves * kCount;
 };
 
 // The entries e0 .. e1 - 1 of a workgroup's line: tile | causal flag << 30.  With one group every wave holds 64 of them, in a register
 // or, where none is left, in kBytes of LDS of its own: read one by one through the scalar cache they cost the walks two
 // dependent loads per tile (strided 128k, 32 heads, with the copies between the MFMAs: forward 18.3 -> 17.9 ms, dQ 25.6 -> 24.5).
 // With more groups (dense rectangles) entry e is tile e itself.
-template <int kGroups, bool kInRegister>
+template <int kForm, bool kInRegister>
 struct Walk {
-  static constexpr int kBytes = kGroups == 1 && !kInRegister ? 256 : 0;
+  static constexpr int kBytes = kForm == 1 && !kInRegister ? 256 : 0;
   int e0, e1, diag, window;
   uint32_t lds;
   __device__ __forceinline__ Walk(int e0_, int e1_, int diag_, uint32_t lds_ = 0) : e0(e0_), e1(e1_), diag(diag_), window(0), lds(lds_) {}
   // Brings entries e .. e + 63 (e < e1); a dense walk's tiles are e itself.
   __device__ __forceinline__ void fetch(int e, bool dense, const int32_t* idx, const uint8_t* flag, int n_tiles) {
-    if constexpr (kGroups == 1) {
+    if constexpr (kForm == 1) {
       const int lane = fresh_lane(), i = min(e + lane, e1 - 1);
       window = dense ? i | ((int)(i == diag) << 30) : min(max(idx[i], 0), n_tiles - 1) | ((int)(flag[i] != 0) << 30);
       if constexpr (!kInRegister) lds_put(lds + 4 * lane, window);
     }
   }
   // The first of every 64 entries has to be fetched before it is asked for.
-  __device__ __forceinline__ bool has(int e) const { return kGroups > 1 || ((e - e0) & 63) != 0 || e >= e1; }
+  __device__ __forceinline__ bool has(int e) const { return kForm > 1 || ((e - e0) & 63) != 0 || e >= e1; }
   __device__ __forceinline__ int at(int e) const {
-    if constexpr (kGroups > 1) return e | ((int)(e == diag) << 30);
+    if constexpr (kForm > 1) return e | ((int)(e == diag) << 30);
     if constexpr (kInRegister) return __builtin_amdgcn_readlane(window, (e - e0) & 63);
     return __builtin_amdgcn_readfirstlane(lds_get<int>(lds + 4 * ((e - e0) & 63)));
   }
