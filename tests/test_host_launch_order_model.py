@@ -1,6 +1,7 @@
 """Quality of the launch orders (q_order, k_order) under a model of one XCD: 64 resident workgroups
-that take rows in the kernels' dispatch order (two heads at a time, teams of four positions, heads
-alternating team by team), every workgroup one tile per step, and an LRU cache of 64 K/V (or Q/dO)
+that take rows two heads at a time, in teams of four positions, heads alternating team by team (the
+kernels alternate position by position, which is the same or faster on the device but lets whole causal
+rows fall off this strict cache), every workgroup one tile per step, and an LRU cache of 64 K/V (or Q/dO)
 tiles = the 4 MiB L2 of an XCD.  The model reproduced the measured effect of the order on the device
 (strided 128k forward: 80 -> 22 GB fetched per launch, +6 %); here it guards the rule against
 regressions on the benchmark masks.  No GPU."""

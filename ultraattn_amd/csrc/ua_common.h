@@ -333,29 +333,19 @@ __device__ __forceinline__ void dma_rows_buf(unsigned char* lds, __amdgpu_buffer
 // consecutive XCDs.  Each XCD gets its own heads (heads_per_xcd = batch*n_heads/8 when
 // divisible, else 0 = plain mapping) and works on them kHeadGroup at a time, so that the
 // workgroups resident on an XCD belong to few heads and share K/V (or Q/dO) tiles in its L2.
-// Within a head group the dispatch order goes team by team: a team is kTeam consecutive
-// positions of the launch order (rows with the same or nearly the same tile lists); its
-// members are dispatched back to back, start together and walk their lists in step.
+// Within a head group the heads take turns, position by position: adjacent positions of the launch order (rows with the same
+// or nearly the same tile lists) start together and walk their lists in step.  Each head taking four positions at a turn was
+// 0.5 to 2 % slower where L2 is short (strided mask: 32k, 16 heads, dK/dV 1633 -> 1598 us; 128k, 32 heads, 33.5 -> 33.2 ms; causal
+// 8192, 32 heads, backward 1567 -> 1553 us, 4096 434 -> 421) and the same elsewhere; so are one head at a time 2 to 4 % and four 1 to 2 %.
 constexpr int kHeadGroup = 2;
-constexpr int kTeam = 4;
 __device__ __forceinline__ void map_block(int bid, int nbh, int heads_per_xcd, int n_pos, int& pos, int& bh) {
   if (heads_per_xcd > 0) {
     const int xcd = bid & 7, idx = bid >> 3;
     const int g = (heads_per_xcd % kHeadGroup == 0) ? kHeadGroup : 1;
     const int per_group = n_pos * g;
     const int hg = idx / per_group, r = idx % per_group;
-    const int full = (n_pos / kTeam) * kTeam;        // positions in complete teams
-    int hs;
-    if (r < full * g) {
-      const int team = r / (kTeam * g), rr = r % (kTeam * g);
-      hs = rr / kTeam;
-      pos = team * kTeam + rr % kTeam;
-    } else {                                         // the last, shorter team
-      const int t = n_pos - full, rr = r - full * g;
-      hs = rr / t;
-      pos = full + rr % t;
-    }
-    bh = xcd * heads_per_xcd + hg * g + hs;
+    pos = r / g;
+    bh = xcd * heads_per_xcd + hg * g + r % g;
   } else {
     pos = bid / nbh;
     bh = bid % nbh;
