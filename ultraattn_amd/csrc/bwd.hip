@@ -406,17 +406,16 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block
     for (int mb = 0; mb < 4; ++mb)
       if (group) add_block(area(0), mb, dv[mb]); else add_block(area(1), mb, dk[mb]);
   }
-  f32x16 dk_sum{0}, dv_sum{0};             // four groups: each finishes a block of 32 columns of both
+  f32x16 dk_sum, dv_sum;             // four groups: each finishes a block of 32 columns of both
   if constexpr (kForm == 4) {
-    put_acc(area(group), dk);
+    constexpr float kOnes[4] = {1.f, 1.f, 1.f, 1.f};
+    put_acc(area(group), dk, group);
     __syncthreads();
-#pragma unroll
-    for (int g = 0; g < 4; ++g) add_block(area(g), group, dk_sum);
+    sum_blocks(dk_sum, dk, group, area, kOnes);
     __syncthreads();
-    put_acc(area(group), dv);
+    put_acc(area(group), dv, group);
     __syncthreads();
-#pragma unroll
-    for (int g = 0; g < 4; ++g) add_block(area(g), group, dv_sum);
+    sum_blocks(dv_sum, dv, group, area, kOnes);
   }
   const ParamsLate pl = params_late();
   const int64_t seq_k = (int64_t)pl->n_ktiles * kTile;
@@ -613,11 +612,11 @@ __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_block, 
   const int64_t qrow_out = (int64_t)qt * kTile + q_block * 32, seq_out = (int64_t)pl->n_qtiles * kTile;
   auto area = [&](int g) { return lds_block + (wave * S::kCount + g) * kAccBytes; };       // of group g of this wave's rows
   if constexpr (kForm == 4) {
-    put_acc(area(group), dq);
+    put_acc(area(group), dq, group);
     __syncthreads();
-    f32x16 sum{0};
-#pragma unroll
-    for (int g = 0; g < 4; ++g) add_block(area(g), group, sum);
+    constexpr float kOnes[4] = {1.f, 1.f, 1.f, 1.f};
+    f32x16 sum;
+    sum_blocks(sum, dq, group, area, kOnes);
     store_block(&pl->rows, pl->rows.out0, pl->rows.o0s.b, pl->rows.o0s.s, pl->rows.o0s.h, pl->n_heads, part, b, qrow_out, h, seq_out, group, sum,
                 pl->scale, area(group) + 4096 * group);
   } else {

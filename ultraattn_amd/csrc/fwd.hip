@@ -160,6 +160,10 @@ __global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void fwd_kernel(const F
   __shared__ __attribute__((aligned(1024))) unsigned char sVA[kForm * kStageBytes];
   __shared__ __attribute__((aligned(1024))) unsigned char sKB[kForm * kStageBytes];
   __shared__ __attribute__((aligned(1024))) unsigned char sVB[kForm * kStageBytes];
+  // With four groups the query rows have room of their own: the first step's copies need not wait for everyone's reads of them
+  // (with the step's barrier at its end: two causal tiles 6.4 -> 6.25 us, 8 heads of 1024 12.75 -> 12.5).
+  constexpr bool kOwnQ = kForm == 4;
+  __shared__ __attribute__((aligned(1024))) unsigned char sQ[kOwnQ ? 32 * kWaves * kRowBytes : 1];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave_in_block = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -250,14 +254,15 @@ __global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void fwd_kernel(const F
     load_rows(raw, p.q + b * p.qs.b + (int64_t)qrow0 * p.qs.s + h * p.qs.h, p.qs.s);
     rows_to_frags(qf, raw, (uint32_t)(uintptr_t)(lds_byte*)((wave < 2 ? kB : vB) + (wave & 1) * kWaveRowsBytes));
   } else {
-    const uint32_t q_lds = (uint32_t)(uintptr_t)(lds_byte*)sKB;
+    const uint32_t q_lds = lds_at(kOwnQ ? sQ : sKB);
     copy_shared_rows<32 * kWaves>(p.q + b * p.qs.b + ((int64_t)qt * kTile + sub * 32 * kWaves) * p.qs.s + h * p.qs.h, (int)p.qs.s, q_lds);
     wait_vmem_all();
     __syncthreads();
     shared_rows_to_frags(qf, q_lds, wave);
+    if (!kOwnQ) __syncthreads();
   }
 #pragma unroll
-  for (int ks = 0; ks < 8; ++ks) asm volatile("" : "+v"(qf[ks]));      // read before the first step's barrier
+  for (int ks = 0; ks < 8; ++ks) asm volatile("" : "+v"(qf[ks]));      // read before the walk
 
   f32x16 oacc[4];
 #pragma unroll
@@ -277,9 +282,11 @@ __global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void fwd_kernel(const F
     };
     if (kForm > 1) look_ahead();
     if (kForm == 1 && !kFirst) tile(walk.tile(ent_next), e + 1 < e1);
-    // this stage has landed; everyone is done with the other one
-    wait_vmem_all();
-    __syncthreads();
+    auto landed = [&]() {        // the next stage has landed; everyone is done with this one
+      wait_vmem_all();
+      __syncthreads();
+    };
+    if (kForm == 1) landed();
     unsigned char *const k_other = kStage ? kA : kB, *const v_other = kStage ? vA : vB;
     if (kForm > 1 && e + 1 < e1) copy_stage(walk.tile(ent_next), k_other, v_other, group);
     auto copy = [&](int n) { copy_piece(n, k_other, v_other, kStage ^ 1); };
@@ -301,6 +308,7 @@ __global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void fwd_kernel(const F
         for (int n = 0; n < 8; ++n) copy(n);
     }
     if (!kFirst) ent = ent_next;
+    if (kForm > 1) landed();
   };
   for (int e = e0; e < e1; e += kForm == 1 ? 1 : 2) {
     step(e, std::integral_constant<int, 0>{});
@@ -335,10 +343,9 @@ __global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void fwd_kernel(const F
     auto area = [&](int x) { return lds_at(x < 2 ? sKA : x < 4 ? sVA : x < 6 ? sKB : sVB) + (x & 1) * kAccBytes; };
     const int own = wave * kForm + group;
     constexpr bool kAll = kForm == 2;        // the first group finishes whole rows; with four groups each a block of 32 columns
-    __syncthreads();
     stat[own][0][lane] = st.m_run;
     stat[own][1][lane] = l_tot;
-    if (!kAll || group == 1) put_acc(area(own), oacc);
+    if (!kAll || group == 1) put_acc(area(own), oacc, kAll ? -1 : group);
     __syncthreads();
     if (kAll && group == 1) return;
     float m = -INFINITY, w[kForm];
@@ -358,9 +365,8 @@ __global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void fwd_kernel(const F
       for (int mb = 0; mb < 4; ++mb) add_block(area(own + 1), mb, oacc[mb], w[0], w[1]);
       store_rows_bf16(orow, o_stride, oacc, inv, area(own + 1));
     } else {
-      f32x16 o{0};
-#pragma unroll
-      for (int g = 0; g < kForm; ++g) add_block(area(wave * kForm + g), group, o, 1.f, w[g]);
+      f32x16 o;
+      sum_blocks(o, oacc, group, [&](int g) { return area(wave * kForm + g); }, w);
       store_block_bf16(orow + 32 * group, o_stride, o, inv, area(own) + 4096 * group);
     }
   }

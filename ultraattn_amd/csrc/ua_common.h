@@ -215,14 +215,15 @@ __device__ __forceinline__ void store_block_f32(float* rows, int64_t row_stride,
   }
 }
 // A wave's accumulators in LDS for the waves of the other groups: 16-byte pieces, 1 KiB per instruction; block mb of 32
-// columns is the 4 KiB at 4096 * mb.
+// columns is the 4 KiB at 4096 * mb.  Block `own` (wave-uniform), which the wave finishes itself, is left out.
 constexpr int kAccBytes = 64 * 64 * 4;
-__device__ __forceinline__ void put_acc(uint32_t lds, const f32x16 (&acc)[4]) {
+__device__ __forceinline__ void put_acc(uint32_t lds, const f32x16 (&acc)[4], int own = -1) {
   lds += 16 * fresh_lane();
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const f32x16& a = acc[i >> 2];
-    lds_put(lds + 1024 * i, f32x4{a[4 * (i & 3)], a[4 * (i & 3) + 1], a[4 * (i & 3) + 2], a[4 * (i & 3) + 3]});
+  for (int mb = 0; mb < 4; ++mb) {
+    if (mb == own) continue;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) lds_put(lds + 4096 * mb + 1024 * g, f32x4{acc[mb][4 * g], acc[mb][4 * g + 1], acc[mb][4 * g + 2], acc[mb][4 * g + 3]});
   }
 }
 // acc = acc * wa + (block mb) * wb
@@ -233,6 +234,21 @@ __device__ __forceinline__ void add_block(uint32_t lds, int mb, f32x16& acc, flo
     const f32x4 x = lds_get<f32x4>(lds + 1024 * i);
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[4 * i + j] = acc[4 * i + j] * wa + x[j] * wb;
+  }
+}
+// sum = the groups' blocks `own` in order, times w: this wave's from its accumulators, the other groups' from at(g).
+// (Its own block through LDS as well was a fourth of what the four groups' end moves there: 8 heads of 1024, forward
+// 12.85 -> 12.75 us, backward 19.8 -> 19.4; 32 of 512, forward 10.2 -> 9.9.)
+template <class At>
+__device__ __forceinline__ void sum_blocks(f32x16& sum, const f32x16 (&acc)[4], int own, At at, const float (&w)[4]) {
+  sum = f32x16{0};
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    if (g != own) add_block(at(g), own, sum, 1.f, w[g]);
+    if (g == own) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sum[i] = sum[i] * 1.f + acc[g][i] * w[g];
+    }
   }
 }
 // How a workgroup's waves share a line, by kForm:
