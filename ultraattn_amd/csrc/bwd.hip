@@ -30,6 +30,8 @@ struct BwdSide {
   // out + i * o_part (fp32 elements, contiguous [batch, tokens, heads, 128]) for a later sum.
   int n_parts, part_len, out_f32;
   int64_t o_part;
+  BlockMap map;
+  Div by_lines;                            // tiles of this side
 };
 struct BwdParams {
   const bf16* q; const bf16* k; const bf16* v; const bf16* dout;
@@ -37,7 +39,7 @@ struct BwdParams {
   int batch, n_heads, n_qtiles, n_ktiles, nnz;
   Strides3 qs, ks, vs, ds;
   float scale_log2, scale;
-  int heads_per_xcd;
+  Div by_heads;
   // Dense rectangle (no list arrays).  The rows walk key tiles [0, n_ktiles) of a query tile, with dense_causal
   // [0, qt + diag_off], the last one causal; the columns walk query tiles [0, n_qtiles) of a key tile, with
   // dense_causal [kt - diag_off, n_qtiles), the first one causal.
@@ -257,14 +259,14 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block
   const int group = S::kCount == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * S::kWaves));
   const uint32_t lds_base = lds_block + group * S::kBytes;
   int pos, bh;
-  map_block(block, p.batch * p.n_heads, p.heads_per_xcd, p.n_ktiles * p.cols.n_parts * S::kLines, pos, bh);
-  const int sub = pos % S::kLines;         // which half of the tile's keys
-  pos /= S::kLines;
-  const int b = bh / p.n_heads, h = bh % p.n_heads;
+  map_block(block, p.cols.map, pos, bh);
+  const int sub = pos & (S::kLines - 1);         // which half of the tile's keys
+  pos >>= S::kLines - 1;
+  const int b = quotient(bh, p.by_heads), h = bh - b * p.n_heads;
   const bool dense = kForm > 1 || p.dense;
   int kt, e0, e1, diag = -1, part = 0;
   if (dense) {
-    part = pos / p.n_ktiles;
+    part = quotient(pos, p.cols.by_lines);
     kt = pos - part * p.n_ktiles;                          // column 0 is the longest of a causal rectangle
     if (p.cols_reversed) kt = p.n_ktiles - 1 - kt;
     if (p.dense_causal) diag = kt - p.diag_off;            // query tile on the diagonal (may lie outside)
@@ -497,15 +499,15 @@ __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_block, 
   const int group = S::kCount == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * S::kWaves));
   const uint32_t lds_base = lds_block + group * S::kBytes;
   int pos, bh;
-  map_block(block, p.batch * p.n_heads, p.heads_per_xcd, p.n_qtiles * p.rows.n_parts * S::kLines, pos, bh);
-  const int sub = pos % S::kLines;         // which half of the tile's queries
-  pos /= S::kLines;
-  const int b = bh / p.n_heads, h = bh % p.n_heads;
+  map_block(block, p.rows.map, pos, bh);
+  const int sub = pos & (S::kLines - 1);         // which half of the tile's queries
+  pos >>= S::kLines - 1;
+  const int b = quotient(bh, p.by_heads), h = bh - b * p.n_heads;
   const int64_t seq_q = (int64_t)p.n_qtiles * kTile;
   const bool dense = kForm > 1 || p.dense;
   int qt, e0, e1, diag = -1, part = 0;
   if (dense) {
-    part = pos / p.n_qtiles;
+    part = quotient(pos, p.rows.by_lines);
     const int line = pos - part * p.n_qtiles;
     qt = p.dense_causal ? p.n_qtiles - 1 - line : line;    // longest rows first
     if (p.dense_causal) diag = qt + p.diag_off;
@@ -672,8 +674,6 @@ static int fill_common(BwdParams& p, const void* q, const void* k, const void* v
   p.qs = {qs[0], qs[1], qs[2]}; p.ks = {ks[0], ks[1], ks[2]};
   p.vs = {vs[0], vs[1], vs[2]}; p.ds = {ds[0], ds[1], ds[2]};
   p.scale = softmax_scale; p.scale_log2 = softmax_scale * kLog2e;
-  const int nbh = batch * n_heads;
-  p.heads_per_xcd = (nbh % 8 == 0) ? nbh / 8 : 0;
   p.dense = 0; p.dense_causal = 0; p.diag_off = 0; p.n_col_blocks = 0; p.cols_reversed = 0;
   p.cols = BwdSide{}; p.rows = BwdSide{};
   p.cols.n_parts = p.rows.n_parts = 1;
@@ -696,6 +696,14 @@ static int fill_side(BwdSide& s, int nnz, const int32_t* ptr, const int32_t* idx
 
 static int launched() { return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH; }
 static unsigned col_blocks(const BwdParams& p) { return (unsigned)(p.batch * p.n_heads * p.n_ktiles * p.cols.n_parts); }
+// Where the workgroups of both sides are, for `lines` of them per tile.
+static void place(BwdParams& p, int lines) {
+  p.by_heads = make_div(p.n_heads);
+  p.cols.map = block_map(p.batch * p.n_heads, p.n_ktiles * p.cols.n_parts * lines);
+  p.rows.map = block_map(p.batch * p.n_heads, p.n_qtiles * p.rows.n_parts * lines);
+  p.cols.by_lines = make_div(p.n_ktiles);
+  p.rows.by_lines = make_div(p.n_qtiles);
+}
 static unsigned row_blocks(const BwdParams& p) { return (unsigned)(p.batch * p.n_heads * p.n_qtiles * p.rows.n_parts); }
 // The form (see Groups) for n lines of 128 rows on both sides of a dense rectangle together (parts counted), as in the forward:
 //  - four groups while half lines leave a CU one workgroup at most (8 heads of 1024: 34 us with one group, 31 with two, 24
@@ -720,7 +728,9 @@ static int bwd_form(int64_t n, int64_t both_walks, int n_parts, bool dense_causa
 static int launch_bwd(BwdParams& p, bool plain, hipStream_t st) {
   const unsigned n = col_blocks(p) + row_blocks(p);
   const int form = plain ? 1 : bwd_form(n, p.cols.part_len + p.rows.part_len, p.cols.n_parts + p.rows.n_parts, p.dense_causal, p.n_qtiles, p.n_ktiles);
-  p.n_col_blocks = (int)col_blocks(p) * (form > 2 ? 2 : 1);
+  const int lines = form > 2 ? 2 : 1;
+  p.n_col_blocks = (int)col_blocks(p) * lines;
+  place(p, lines);
   // Up to two workgroups per CU the whole launch is resident at once, and the second 256 join the first in launch
   // order.  Both sides come longest first (lists roughly); the columns are then taken in reverse, so that the long ones
   // of one side share a CU with the short ones of the other (32 causal heads of 1024: 43.6 -> 41.5 us).
@@ -802,6 +812,7 @@ extern "C" int ua_bsa_bwd_dkdv(const void* q, const void* k, const void* v, cons
   if (!dv_strides) return UA_ERR_NULL;
   if (int rc = fill_side(p.cols, nnz, col_ptr, row_idx, cflag, k_order, dk, dk_strides, dv, dv_strides, false)) return rc;
   if (int rc = check_device()) return rc;
+  place(p, 1);
   hipLaunchKernelGGL(dkdv_kernel, dim3(col_blocks(p)), dim3(256), 0, (hipStream_t)stream, p);
   return launched();
 }
@@ -820,6 +831,7 @@ extern "C" int ua_bsa_bwd_dq(const void* q, const void* k, const void* v, const 
                            v_strides, do_strides, softmax_scale)) return rc;
   if (int rc = fill_side(p.rows, nnz, row_ptr, col_idx, flag, q_order, dq, dq_strides, nullptr, nullptr, false)) return rc;
   if (int rc = check_device()) return rc;
+  place(p, 1);
   hipLaunchKernelGGL(dq_kernel, dim3(row_blocks(p)), dim3(256), 0, (hipStream_t)stream, p);
   return launched();
 }

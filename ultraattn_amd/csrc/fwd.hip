@@ -23,7 +23,8 @@ struct FwdParams {
   int n_first;           // positions of the launch order that are taken in reverse (see fwd_launch)
   Strides3 qs, ks, vs, os;
   float scale_log2;      // softmax_scale * log2(e)
-  int heads_per_xcd;     // batch*n_heads / 8 when divisible, else 0
+  BlockMap map;
+  Div by_heads, by_cut;  // n_heads; query tiles that are cut (1 if none)
   // Dense rectangle (no list arrays): query tile qt walks key tiles [0, n_ktiles), or with
   // dense_causal [0, qt + diag_off] with the last one causal; longest rows first.  The first n_whole query tiles (all
   // if nothing is cut) are walked whole; the key range of the others is cut into n_parts parts of part_len tiles, and
@@ -173,19 +174,18 @@ __global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void fwd_kernel(const F
   unsigned char *const kB = sKB + group * kStageBytes, *const vB = sVB + group * kStageBytes;
   const int l32 = lane & 31, hi = lane >> 5;
   int pos, bh;
-  map_block(blockIdx.x, p.batch * p.n_heads, p.heads_per_xcd, (p.n_whole + (p.n_qtiles - p.n_whole) * p.n_parts) * kLines, pos, bh);
-  const int sub = pos % kLines;            // which half of the tile's rows
-  pos /= kLines;
+  map_block(blockIdx.x, p.map, pos, bh);
+  const int sub = pos & (kLines - 1);      // which half of the tile's rows
+  pos >>= kLines - 1;
   if (pos < p.n_first) pos = p.n_first - 1 - pos;
-  const int b = bh / p.n_heads, h = bh % p.n_heads;
+  const int b = quotient(bh, p.by_heads), h = bh - b * p.n_heads;
   const bool dense = kForm > 1 || p.dense;
   int qt, e0, e1, diag = -1, part = -1;
   if (dense) {
     int line = pos;
     if (pos >= p.n_whole) {
-      const int n_cut = p.n_qtiles - p.n_whole;
-      part = (pos - p.n_whole) / n_cut;
-      line = pos - part * n_cut;
+      part = quotient(pos - p.n_whole, p.by_cut);
+      line = pos - part * p.by_cut.d;
     }
     qt = p.dense_causal ? p.n_qtiles - 1 - line : line;
     if (p.dense_causal) diag = qt + p.diag_off;          // key tile on the diagonal (may lie outside the rectangle)
@@ -401,8 +401,6 @@ static int fwd_common(FwdParams& p, const void* q, const void* k, const void* v,
   p.vs = {v_strides[0], v_strides[1], v_strides[2]};
   p.os = {o_strides[0], o_strides[1], o_strides[2]};
   p.scale_log2 = softmax_scale * kLog2e;
-  const int nbh = batch * n_heads;
-  p.heads_per_xcd = (nbh % 8 == 0) ? nbh / 8 : 0;
   p.dense = 0; p.dense_causal = 0; p.diag_off = 0; p.n_whole = n_qtiles; p.n_parts = 1; p.part_len = n_ktiles;
   p.part_o = nullptr; p.part_lse = nullptr; p.o_part = 0; p.lse_part = 0;
   return check_device();
@@ -429,7 +427,12 @@ static int fwd_groups(int64_t n, int64_t walk, int n_parts, bool dense_causal) {
 static int fwd_launch(FwdParams& p, bool plain, hipStream_t st) {
   const unsigned n = (unsigned)(p.batch * p.n_heads * (p.n_whole + (p.n_qtiles - p.n_whole) * p.n_parts));
   // (several groups copy Q through a buffer descriptor, whose offsets have 32 bits)
-  switch (plain || p.qs.s > (INT32_MAX >> 9) ? 1 : fwd_groups(n, p.part_len, p.n_parts, p.dense_causal)) {
+  const int form = plain || p.qs.s > (INT32_MAX >> 9) ? 1 : fwd_groups(n, p.part_len, p.n_parts, p.dense_causal);
+  const int n_cut = p.n_qtiles - p.n_whole;
+  p.map = block_map(p.batch * p.n_heads, (p.n_whole + n_cut * p.n_parts) * (form == 4 ? 2 : 1));
+  p.by_heads = make_div(p.n_heads);
+  p.by_cut = make_div(n_cut ? n_cut : 1);
+  switch (form) {
     case 4: hipLaunchKernelGGL(fwd_kernel<4>, dim3(2 * n), dim3(512), 0, st, p); break;
     case 2: hipLaunchKernelGGL(fwd_kernel<2>, dim3(n), dim3(512), 0, st, p); break;
     default:

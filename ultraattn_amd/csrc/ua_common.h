@@ -247,7 +247,7 @@ __device__ __forceinline__ void sum_blocks(f32x16& sum, const f32x16 (&acc)[4], 
     if (g != own) add_block(at(g), own, sum, 1.f, w[g]);
     if (g == own) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) sum[i] = sum[i] * 1.f + acc[g][i] * w[g];
+      for (int i = 0; i < 16; ++i) sum[i] += acc[g][i] * w[g];
     }
   }
 }
@@ -345,6 +345,18 @@ __device__ __forceinline__ void dma_rows_buf(unsigned char* lds, __amdgpu_buffer
   for (int i = 0; i < 4; ++i) dma16_buf(r, lds + (NW * i + wave) * 1024, voff[i], soff);
 }
 
+// n / d for 0 <= n < 2^31 as one multiplication: mul = ceil(2^shift / d), shift = 31 + ceil(log2 d), is off by less than d, so that
+// n * mul is off by less than 2^shift.  (A workgroup's place takes three to five divisions in a row before its first copy; with
+// the divisors' reciprocals formed there, 30 dependent instructions each, it came 0.4 us later: 8 heads of 1024, forward 12.54 -> 12.39 us,
+// backward 19.3 -> 19.1; one head of 256 6.24 -> 6.18.)
+struct Div { int d; uint32_t mul, shift; };
+inline Div make_div(uint32_t d) {
+  uint32_t log = 0;
+  while ((1u << log) < d) ++log;
+  return {(int)d, (uint32_t)(((1ull << (31 + log)) + d - 1) / d), 31 + log};
+}
+__device__ __forceinline__ int quotient(int n, const Div& by) { return (int)(((uint64_t)(uint32_t)n * by.mul) >> by.shift); }
+
 // blockIdx -> (position in the launch order, batch*head).  Consecutive workgroups go to
 // consecutive XCDs.  Each XCD gets its own heads (heads_per_xcd = batch*n_heads/8 when
 // divisible, else 0 = plain mapping) and works on them kHeadGroup at a time, so that the
@@ -354,18 +366,21 @@ __device__ __forceinline__ void dma_rows_buf(unsigned char* lds, __amdgpu_buffer
 // 0.5 to 2 % slower where L2 is short (strided mask: 32k, 16 heads, dK/dV 1633 -> 1598 us; 128k, 32 heads, 33.5 -> 33.2 ms; causal
 // 8192, 32 heads, backward 1567 -> 1553 us, 4096 434 -> 421) and the same elsewhere; so are one head at a time 2 to 4 % and four 1 to 2 %.
 constexpr int kHeadGroup = 2;
-__device__ __forceinline__ void map_block(int bid, int nbh, int heads_per_xcd, int n_pos, int& pos, int& bh) {
-  if (heads_per_xcd > 0) {
-    const int xcd = bid & 7, idx = bid >> 3;
-    const int g = (heads_per_xcd % kHeadGroup == 0) ? kHeadGroup : 1;
-    const int per_group = n_pos * g;
-    const int hg = idx / per_group, r = idx % per_group;
-    pos = r / g;
-    bh = xcd * heads_per_xcd + hg * g + r % g;
-  } else {
-    pos = bid / nbh;
-    bh = bid % nbh;
-  }
+struct BlockMap {
+  int own_heads, heads_per_xcd, bid_shift, group_shift;      // own_heads: -1 with whole heads per XCD, else 0 (and so the others)
+  Div by;                                                    // workgroups of a head group, or (batch, head) pairs
+};
+inline BlockMap block_map(int nbh, int n_pos) {
+  if (nbh % 8) return {0, 0, 0, 0, make_div(nbh)};
+  const int heads = nbh / 8, shift = heads % kHeadGroup == 0 ? 1 : 0;
+  return {-1, heads, 3, shift, make_div((uint32_t)n_pos << shift)};
+}
+__device__ __forceinline__ void map_block(int bid, const BlockMap& m, int& pos, int& bh) {
+  const int idx = bid >> m.bid_shift, q = quotient(idx, m.by), r = idx - q * m.by.d;
+  const int own_bh = (bid & 7) * m.heads_per_xcd + (q << m.group_shift) + (r & ((1 << m.group_shift) - 1));
+  // (without branches, so that all parameters are read at once)
+  pos = q ^ ((q ^ (r >> m.group_shift)) & m.own_heads);
+  bh = r ^ ((r ^ own_bh) & m.own_heads);
 }
 
 inline bool aligned4(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 3) == 0; }
