@@ -102,3 +102,16 @@ def test_grad_accumulate_argument_checks():
         ops.grad_accumulate(x, x.float())
     with pytest.raises(RuntimeError):
         ops.grad_accumulate(x[:12], x[16:28])          # not a multiple of 8 elements
+
+
+@pytest.mark.parametrize("n", [8, 2040, 2056, 4194304, 4194312])           # around a workgroup, and the largest small sum
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_grad_accumulate_sizes(n, mode):
+    g = torch.Generator().manual_seed(n + mode)
+    mk = lambda dt: torch.randn(n, generator=g).to(dt).to(DEV)
+    acc, part, out = mk(torch.float32), mk(torch.bfloat16), mk(torch.bfloat16)
+    want = (acc if mode == 0 else out.float()) + part.float()
+    ops.grad_accumulate(part, out, None if mode == 2 else acc, mode == 1)
+    if mode != 2:
+        assert torch.equal(acc, want)
+    assert torch.equal(out, want.to(torch.bfloat16))

@@ -25,15 +25,15 @@ struct MergeParams {
   const float* lse_parts[UA_MAX_PARTS];
   bf16* o; float* lse;
   int n_parts, seqlen, n_heads, tok;           // tok: tokens per workgroup
+  Div by_tiles, by_tok;                        // workgroups of a sequence; tok
 };
 
 template <int P>
 __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
   extern __shared__ float w_lds[];              // [P][rows], rows = p.tok * n_heads
   const int tid = threadIdx.x;
-  const int tiles_per_batch = (p.seqlen + p.tok - 1) / p.tok;
-  const int b = blockIdx.x / tiles_per_batch;
-  const int s0 = (blockIdx.x % tiles_per_batch) * p.tok;
+  const int b = quotient(blockIdx.x, p.by_tiles);
+  const int s0 = (blockIdx.x - b * p.by_tiles.d) * p.tok;
   const int ntok = min(p.tok, p.seqlen - s0);       // the last workgroup of a batch may be ragged
   const int rows = ntok * p.n_heads;
 
@@ -60,7 +60,7 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeParams p) {
 
   // phase 1: one thread per (head, token): statistics, coalesced along the token axis
   for (int t = tid; t < p.tok * p.n_heads; t += 256) {
-    const int h = t / p.tok, sl = t % p.tok;
+    const int h = quotient(t, p.by_tok), sl = t - h * p.tok;
     if (sl >= ntok) continue;
     const int64_t li = ((int64_t)b * p.n_heads + h) * p.seqlen + s0 + sl;
     float l[P];
@@ -120,12 +120,13 @@ struct MergeF32Params {
   int64_t o_part, lse_part;                    // elements from part to part
   bf16* o; float* lse;
   int n_parts, seqlen, n_heads, out_seq, rows;
+  Div by_heads, by_seq;
 };
 template <int P>
 __global__ __launch_bounds__(256) void merge_f32_kernel(const MergeF32Params p) {
   const int row = blockIdx.x * 16 + (threadIdx.x >> 4), sub = threadIdx.x & 15;
   if (row >= p.rows) return;
-  const int h = row % p.n_heads, t = row / p.n_heads, s = t % p.seqlen, b = t / p.seqlen;
+  const int t = quotient(row, p.by_heads), h = row - t * p.n_heads, b = quotient(t, p.by_seq), s = t - b * p.seqlen;
   const float* src = p.o_parts + (int64_t)row * kHeadDim + sub * 8;
   const float* stat = p.lse_parts + ((int64_t)b * p.n_heads + h) * p.seqlen + s;
   float l[P], m = -INFINITY, den = 0.f;
@@ -157,19 +158,21 @@ __global__ __launch_bounds__(256) void merge_f32_kernel(const MergeF32Params p) 
   if (sub == 0) p.lse[((int64_t)b * p.n_heads + h) * p.out_seq + s] = den > 0.f ? ms + __builtin_amdgcn_logf(den) * kLn2 : -INFINITY;
 }
 
+// (8 heads of 1024, 32 of 512: 2.65 and 2.95 us with divisions by n_heads, 2.45 and 2.75 with multiplications; likewise the update
+// below, 3.2 -> 3.05.)
 struct DeltaParams {
   const bf16* o; const bf16* dout; float* delta;
   int seqlen, n_heads;
   Strides3 os, ds;
+  Div by_tiles, by_heads;      // workgroups of a sequence; n_heads
 };
 
 template <int kTok>
 __global__ __launch_bounds__(256) void delta_kernel(const DeltaParams p) {
   extern __shared__ float d_lds[];               // [n_heads][kTok]
   const int tid = threadIdx.x;
-  const int tiles_per_batch = (p.seqlen + kTok - 1) / kTok;
-  const int b = blockIdx.x / tiles_per_batch;
-  const int s0 = (blockIdx.x % tiles_per_batch) * kTok;
+  const int b = quotient(blockIdx.x, p.by_tiles);
+  const int s0 = (blockIdx.x - b * p.by_tiles.d) * kTok;
   const int ntok = min(kTok, p.seqlen - s0);
   const int rows = ntok * p.n_heads;
   const int sub = tid & 15;
@@ -181,7 +184,7 @@ __global__ __launch_bounds__(256) void delta_kernel(const DeltaParams p) {
     for (int u = 0; u < kRows; ++u) {
       const int row = row0 + 16 * u;
       if (row < rows) {
-        const int sl = row / p.n_heads, h = row % p.n_heads;
+        const int sl = quotient(row, p.by_heads), h = row - sl * p.n_heads;
         const int64_t s = s0 + sl;
         a[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p.o + b * p.os.b + s * p.os.s + h * p.os.h + sub * 8));
         g[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p.dout + b * p.ds.b + s * p.ds.s + h * p.ds.h + sub * 8));
@@ -191,7 +194,7 @@ __global__ __launch_bounds__(256) void delta_kernel(const DeltaParams p) {
     for (int u = 0; u < kRows; ++u) {
       const int row = row0 + 16 * u;
       if (row >= rows) break;
-      const int sl = row / p.n_heads, h = row % p.n_heads;
+      const int sl = quotient(row, p.by_heads), h = row - sl * p.n_heads;
       float acc = 0.f;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -222,6 +225,7 @@ struct UpdateParams {
   void* new_out; float* new_lse;
   int n_rows, n_heads;
   Strides3 os, ls, bs, bls, ns, nls;
+  Div by_groups, by_heads;     // workgroups of a sequence; n_heads
 };
 
 template <bool kF32>
@@ -258,13 +262,13 @@ constexpr int kUpdRows = 2;       // rows per 16 lanes, every load of both issue
 constexpr int kUpdGroup = 16 * kUpdRows;
 template <bool kOutF32, bool kBlkF32, bool kNewF32>
 __global__ __launch_bounds__(256) void merge_update_kernel(const UpdateParams p) {
-  const int rows = p.n_rows * p.n_heads, groups = (rows + kUpdGroup - 1) / kUpdGroup;
-  const int sub = threadIdx.x & 15, b = blockIdx.x / groups, row0 = (blockIdx.x % groups) * kUpdGroup + (threadIdx.x >> 4);
+  const int rows = p.n_rows * p.n_heads, b = quotient(blockIdx.x, p.by_groups);
+  const int sub = threadIdx.x & 15, row0 = (blockIdx.x - b * p.by_groups.d) * kUpdGroup + (threadIdx.x >> 4);
   float x[kUpdRows][8], y[kUpdRows][8], a[kUpdRows], c[kUpdRows];
 #pragma unroll
   for (int u = 0; u < kUpdRows; ++u) {
     const int row = min(row0 + 16 * u, rows - 1);
-    const int64_t s = row / p.n_heads, h = row % p.n_heads;
+    const int64_t s = quotient(row, p.by_heads), h = row - (int)s * p.n_heads;
     a[u] = p.lse[b * p.ls.b + s * p.ls.s + h * p.ls.h];
     c[u] = p.blk_lse[b * p.bls.b + s * p.bls.s + h * p.bls.h];
     load8<kOutF32>(p.out, b * p.os.b + s * p.os.s + h * p.os.h + sub * 8, x[u]);
@@ -274,7 +278,7 @@ __global__ __launch_bounds__(256) void merge_update_kernel(const UpdateParams p)
   for (int u = 0; u < kUpdRows; ++u) {
     const int row = row0 + 16 * u;
     if (row >= rows) break;
-    const int64_t s = row / p.n_heads, h = row % p.n_heads;
+    const int64_t s = quotient(row, p.by_heads), h = row - (int)s * p.n_heads;
     const float m = fmaxf(a[u], c[u]);
     const float ms = (m == -INFINITY) ? 0.f : m;
     const float ea = fast_exp2((a[u] - ms) * kLog2e), ec = fast_exp2((c[u] - ms) * kLog2e);
@@ -298,7 +302,8 @@ static int launch_merge(const MergeParams& p, int blocks, size_t lds, hipStream_
 
 int merge_f32_rows(const float* o_parts, int64_t o_part, const float* lse_parts, int64_t lse_part, int n_parts, bf16* o, float* lse, int out_seq,
                    int batch, int seqlen, int n_heads, hipStream_t st) {
-  const MergeF32Params p = {o_parts, lse_parts, o_part, lse_part, o, lse, n_parts, seqlen, n_heads, out_seq, batch * seqlen * n_heads};
+  const MergeF32Params p = {o_parts, lse_parts, o_part, lse_part, o, lse, n_parts, seqlen, n_heads, out_seq, batch * seqlen * n_heads,
+                           make_div(n_heads), make_div(seqlen)};
   const dim3 grid((p.rows + 15) / 16);
   if (n_parts <= 4)      hipLaunchKernelGGL(merge_f32_kernel<4>, grid, dim3(256), 0, st, p);
   else if (n_parts <= 8) hipLaunchKernelGGL(merge_f32_kernel<8>, grid, dim3(256), 0, st, p);
@@ -328,7 +333,8 @@ extern "C" int ua_merge(const void* const* o_parts, const float* const* lse_part
   for (int i = n_parts; i < UA_MAX_PARTS; ++i) { p.o_parts[i] = nullptr; p.lse_parts[i] = nullptr; }
   p.o = (bf16*)o; p.lse = lse; p.n_parts = n_parts; p.seqlen = seqlen; p.n_heads = n_heads; p.tok = tok;
   if (int rc = check_device()) return rc;
-  const int blocks = batch * ((seqlen + tok - 1) / tok);
+  p.by_tiles = make_div((seqlen + tok - 1) / tok); p.by_tok = make_div(tok);
+  const int blocks = batch * p.by_tiles.d;
   const size_t lds = (size_t)n_parts * tok * n_heads * sizeof(float);
   if (lds > 65536) return UA_ERR_SHAPE;   // n_parts * n_heads <= 1024
   hipStream_t st = (hipStream_t)stream;
@@ -362,7 +368,9 @@ extern "C" int ua_bsa_bwd_delta(const void* o, const void* dout, float* delta,
   // 87.5, 82.0 = 6.6 TB/s).  With few heads at least 32 rows, one round of loads.
   auto go = [&](auto tok) {
     constexpr int kT = decltype(tok)::value;
-    hipLaunchKernelGGL(delta_kernel<kT>, dim3((unsigned)(batch * (((int64_t)seqlen_q + kT - 1) / kT))), dim3(256), (size_t)kT * n_heads * sizeof(float), st, p);
+    p.by_tiles = make_div((uint32_t)(((int64_t)seqlen_q + kT - 1) / kT));
+    p.by_heads = make_div(n_heads);
+    hipLaunchKernelGGL(delta_kernel<kT>, dim3((unsigned)(batch * p.by_tiles.d)), dim3(256), (size_t)kT * n_heads * sizeof(float), st, p);
   };
   int tok = n_heads <= 2 ? 16 : (n_heads <= 4 ? 8 : (n_heads <= 8 ? 4 : (n_heads <= 16 ? 2 : 1)));
   while (tok < 32 && (int64_t)batch * seqlen_q >= 2 * tok * (int64_t)(4 * kCus)) tok *= 2;
@@ -403,6 +411,7 @@ extern "C" int ua_merge_update(const void* out, const float* lse, const void* bl
   UpdateParams p;
   p.out = out; p.lse = lse; p.blk = block_out; p.blk_lse = block_lse; p.new_out = new_out; p.new_lse = new_lse;
   p.n_rows = n_rows; p.n_heads = n_heads;
+  p.by_groups = make_div((uint32_t)groups); p.by_heads = make_div(n_heads);
   auto s3 = [](const int64_t* st) { return Strides3{st[0], st[1], st[2]}; };
   p.os = s3(out_strides); p.ls = s3(lse_strides); p.bs = s3(block_out_strides); p.bls = s3(block_lse_strides);
   p.ns = s3(new_out_strides); p.nls = s3(new_lse_strides);
