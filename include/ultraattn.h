@@ -62,8 +62,8 @@ extern "C" {
 
 /* 100 * major + minor.  102: `nnz` argument of the attention entry points, ua_merge_update, the
  * no-allocation builder, `work` of ua_tilelist_build_device grown to n_qtiles + n_ktiles + 7.  104: ua_bsa_bwd.
- * 105: ua_tilelist_build_device_scratch.  */
-#define UA_VERSION 105
+ * 105: ua_tilelist_build_device_scratch.  106: ua_copy_in.  */
+#define UA_VERSION 106
 int ua_version(void);
 const char *ua_strerror(int rc);
 
@@ -292,6 +292,11 @@ int ua_grad_sum(const void *const *parts, int n_parts, int parts_fp32, void *out
  * aligned, and must not overlap; 2*n_chunks*batch <= 65535.                                      */
 int ua_cols_gather(const void *src, void *dst, int n_chunks, int batch, int64_t inner_elems, void *stream);
 int ua_cols_scatter(const void *src, void *dst, int n_chunks, int batch, int64_t inner_elems, void *stream);
+
+/* No counterpart in the reference.  Copies `bytes` (a multiple of 16, at most 16 MiB) from page-locked host memory that the
+ * device can address, or from device memory, to the device, by a kernel on `stream`; both 16-byte aligned.  For what
+ * is made on the host for one call: a tile list, a block mask.  The host memory has to stay until the kernel is through. */
+int ua_copy_in(void *dst, const void *src, int64_t bytes, void *stream);
 
 #ifdef __cplusplus
 }

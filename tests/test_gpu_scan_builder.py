@@ -73,3 +73,24 @@ def test_scratch_that_does_not_fit_leaves_the_lists_the_same(lib):
         for f in FIELDS:
             w = getattr(want, f)
             assert np.array_equal(out[f].cpu().numpy()[:w.shape[0]], w), (scratch, size, f)
+
+
+@pytest.mark.parametrize("rows,cols,rate", [(1, 1, 1), (3, 5, 2), (16, 16, 4), (33, 31, 4), (257, 255, 1), (1031, 1031, 1)])
+def test_lists_of_a_mask_on_the_host(rows, cols, rate):
+    """Copied over as lists or as a mask, of sizes that are no multiple of 16 bytes, the largest beyond 1 MiB."""
+    from ultraattn_amd._lib import native
+    m = np.random.RandomState(rows).randint(0, 3, size=(rows, cols)).astype(np.uint8)
+    if rows > 1000:
+        m *= np.random.RandomState(1).rand(rows, cols) < 0.05
+    want = build_tile_list(m, 128 * rate)
+    buf, nqt, nkt, nnz = native().lists_from_mask(m, rows, cols, rate, 0)
+    assert (nqt, nkt, nnz) == (rows * rate, cols * rate, want.nnz)
+    got, at = buf.cpu().numpy(), 0
+    for f in ("row_ptr", "col_ptr", "q_order", "k_order", "col_idx", "row_idx"):
+        w = getattr(want, f)
+        assert np.array_equal(got[at:at + len(w)], w), f
+        at += len(w)
+    for f in ("flag", "cflag"):
+        w = getattr(want, f)
+        assert np.array_equal(got[at:at + (nnz + 3) // 4].view(np.uint8)[:nnz], w[:nnz]), f
+        at += (nnz + 3) // 4

@@ -38,6 +38,7 @@ SIGNATURES = {
     "ua_grad_sum": (c_int, [POINTER(c_void_p), c_int, c_int, c_void_p, c_int, c_int, c_int, c_int, _i64p, c_float, c_void_p]),
     "ua_cols_gather": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int64, c_void_p]),
     "ua_cols_scatter": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int64, c_void_p]),
+    "ua_copy_in": (c_int, [c_void_p, c_void_p, c_int64, c_void_p]),
 }
 
 _lib = None

@@ -67,6 +67,13 @@ static int launch_permute(const void* src, void* dst, int n_chunks, int batch, i
   return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH;
 }
 
+// A few KiB from pinned host memory, one 16-byte vector per thread: a launch and one round trip over the host link.  The runtime's copy
+// takes the same path with a signal to the host behind it, which the next kernel waits for: mask per call, strided 8k, 8 heads, 73.6 -> 71.9 us.
+__global__ __launch_bounds__(64) void copy_in_kernel(u32x4* dst, const u32x4* src, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * 64 + threadIdx.x;
+  if (i < n) dst[i] = src[i];
+}
+
 }  // namespace ua
 
 extern "C" int ua_cols_gather(const void* src, void* dst, int n_chunks, int batch, int64_t inner_elems, void* stream) {
@@ -75,4 +82,15 @@ extern "C" int ua_cols_gather(const void* src, void* dst, int n_chunks, int batc
 
 extern "C" int ua_cols_scatter(const void* src, void* dst, int n_chunks, int batch, int64_t inner_elems, void* stream) {
   return ua::launch_permute(src, dst, n_chunks, batch, inner_elems, 0, stream);
+}
+
+extern "C" int ua_copy_in(void* dst, const void* src, int64_t bytes, void* stream) {
+  using namespace ua;
+  if (!dst || !src) return UA_ERR_NULL;
+  if (bytes <= 0 || bytes > (1 << 24)) return UA_ERR_SHAPE;
+  if (bytes % 16 != 0 || !aligned16(dst) || !aligned16(src)) return UA_ERR_ALIGN;
+  if (int rc = check_device()) return rc;
+  const int64_t n = bytes / 16;
+  hipLaunchKernelGGL(copy_in_kernel, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, (hipStream_t)stream, (u32x4*)dst, (const u32x4*)src, n);
+  return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH;
 }
