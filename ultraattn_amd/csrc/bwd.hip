@@ -746,47 +746,57 @@ static int launch_bwd(BwdParams& p, bool plain, hipStream_t st) {
 
 // How many parts the two sides of a dense backward are cut into, at most what the workspace holds.  A cut gives a
 // small rectangle enough workgroups for the device and costs the partials' way through memory and a
-// second launch; which wins is decided by an estimate of the launch's time in microseconds, fitted to 47 shapes of 1
-// to 32 heads and 128 to 8192 tokens (the cut it takes is within 4 % of the best one on each):
-//  - 6.5 to start, load the resident rows, store the results and end, 9.8 in form 2, 7.1 in form 4, 6.3 in halves;
-//  - a tile takes 1.9 (columns) or 1 (rows) in form 4, 2.6 and 1.7 in form 2, 2.4 and 1.8 in halves (5.6 together on a full device), else
-//    3.5 and 2.1, and 4.9 and 5.5 where two workgroups share the CU;
-//  - the sum takes 2.4, and the partials 1 per 3.7 MB; a cut has to win by 6 %.
-// 1024 x 4096, one head: 42 us uncut, 24 cut in 2 and 4.
+// second launch; which wins is decided by an estimate of the time in microseconds, fitted to 108 rectangles of 1
+// to 20 heads and 256 to 16384 tokens (the cut it takes is within 1 % of the best one on average, 6 at most; with the forms' times
+// before their ends got shorter, and half of every causal rectangle taken for hidden, 5 and 58):
+//  - 6.7 to start, load the resident rows, store the results and end, 9.8 in form 2, 7.3 in halves, 5.9 in form 4 and up to 2.8 as the
+//    workgroups fill the device;
+//  - a tile takes 1.4 (columns) or 0.85 (rows) in form 4, 2.6 and 1.7 in form 2, 2.3 and 1.5 in halves (5.7 together on a full device), else
+//    3.8 and 1.6, and 5 and 3.5 where two workgroups share the CU;
+//  - the sum takes 3, the columns' partials 0.5 and 1 per 4.2 MB, the rows' 1 per 3.7 MB; a cut has to win by 3 %.
+// 1024 x 4096, one head: 34 us uncut, 21 cut in 2 and 5; 4 heads of 1024 19.9 cut in 2 and 1, 18.1 uncut; causal 8192 x 512 17.4 and 11.9.
 struct BwdCut { int cols, rows; };
 static BwdCut bwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int max_cols, int max_rows) {
   if (max_cols <= 1 && max_rows <= 1) return {1, 1};
   static constexpr int kParts[] = {1, 2, 3, 4, 5, 6, 8, 12, 16};
-  const float density = causal ? 0.5f : 1.f, wk = (float)nbh * n_ktiles, wq = (float)nbh * n_qtiles;
-  const float all = density * wk * n_qtiles * (4.94f + 5.47f) / (2 * kCus);
-  int row_len[sizeof(kParts) / sizeof(int)], n_rows = 0;
-  for (int pr : kParts)
-    if (pr <= max_rows) row_len[n_rows++] = (n_ktiles + pr - 1) / pr;
+  struct Side { int parts, n, len; };                                      // asked for, made, tiles of each
+  auto sides = [](Side (&s)[9], int most, int list_len) {
+    int n = 0;
+    for (int parts : kParts)
+      if (parts <= most) {
+        const int len = (list_len + parts - 1) / parts;
+        s[n++] = {parts, (list_len + len - 1) / len, len};
+      }
+    return n;
+  };
+  Side cols[9], rows[9];
+  const int n_cols = sides(cols, max_cols, n_qtiles), n_rows = sides(rows, max_rows, n_ktiles);
+  const float density = visible_share(n_qtiles, n_ktiles, causal), wk = (float)nbh * n_ktiles, wq = (float)nbh * n_qtiles;
+  const float tiles = density * wk * n_qtiles, part_us = kTile * kHeadDim * 4 / 1e6f;
+  const int seen = causal && n_ktiles < n_qtiles ? n_ktiles : n_qtiles;    // the longest column
   BwdCut best = {1, 1};
   float best_us = INFINITY;
-  for (int pc : kParts) {
-    if (pc > max_cols) break;
-    const int clen = (n_qtiles + pc - 1) / pc;
-    for (int i = 0; i < n_rows; ++i) {
-      const int pr = kParts[i], rlen = row_len[i];
-      const float groups = (wk * pc + wq * pr) * density;
-      float us, tc, tr, least = all;                                       // the work of a CU, however long the walks
-      switch (bwd_form(nbh * ((int64_t)n_ktiles * pc + (int64_t)n_qtiles * pr), clen + rlen, pc + pr, causal, n_qtiles, n_ktiles)) {
-        case 4: us = 7.1f; tc = 1.86f; tr = 0.96f; break;
+  for (int i = 0; i < n_cols; ++i)
+    for (int j = 0; j < n_rows; ++j) {
+      const Side &c = cols[i], &r = rows[j];
+      const float groups = (wk * c.n + wq * r.n) * density;
+      const int64_t lines = nbh * ((int64_t)n_ktiles * c.n + (int64_t)n_qtiles * r.n);
+      float us, tc, tr, least = tiles * 11.3f / (2 * kCus);                // the work of a CU, however long the walks
+      switch (bwd_form(lines, c.len + r.len, c.n + r.n, causal, n_qtiles, n_ktiles)) {
+        case 4: us = 5.9f + 2.8f * (lines / 128.f) * (lines / 128.f); tc = 1.42f; tr = 0.84f; break;
         case 2: us = 9.8f; tc = 2.6f; tr = 1.7f; break;
-        case kHalves: us = 6.3f; tc = 2.4f; tr = 1.8f; least = density * wk * n_qtiles * 5.6f / kCus; break;
+        case kHalves: us = 7.3f; tc = 2.26f; tr = 1.54f; least = tiles * 5.7f / kCus; break;
         default: {
           const float shared = fminf(fmaxf((groups - kCus) / kCus, 0.f), 1.f);       // share of the workgroups with a neighbour
-          us = 6.5f; tc = 3.5f + 1.44f * shared; tr = 2.1f + 3.37f * shared;
+          us = 6.7f; tc = 3.83f + 1.2f * shared; tr = 1.58f + 1.92f * shared;
         }
       }
-      us += fmaxf(fmaxf(clen * tc, rlen * tr), least);
-      if (pc > 1 || pr > 1) us = (us + 2.4f) * 1.06f;
-      if (pc > 1) us += 2.f * pc * wk * (kTile * kHeadDim * 4) / 3.7e6f;
-      if (pr > 1) us += pr * wq * (kTile * kHeadDim * 4) / 3.7e6f;
-      if (us < 0.99f * best_us) { best_us = us; best = {pc, pr}; }        // more parts for a gain, not for a tie
+      us += fmaxf(fmaxf((c.len < seen ? c.len : seen) * tc, r.len * tr), least);
+      if (c.n > 1 || r.n > 1) us = (us + 3.f) * 1.03f;
+      if (c.n > 1) us += 0.5f + 2.f * c.n * wk * part_us / 4.2f;
+      if (r.n > 1) us += r.n * wq * part_us / 3.7f;
+      if (us < 0.99f * best_us) { best_us = us; best = {c.parts, r.parts}; }         // more parts for a gain, not for a tie
     }
-  }
   return best;
 }
 int64_t bwd_workspace_used(int batch, int n_heads, int n_qtiles, int n_ktiles, bool causal) {

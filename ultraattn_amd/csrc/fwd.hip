@@ -447,28 +447,29 @@ static int fwd_launch(FwdParams& p, bool plain, hipStream_t st) {
 
 // How many parts the walks of a dense forward are cut into, at most max_parts (what the workspace holds).  A cut
 // gives a small rectangle enough workgroups and costs the partials' way through memory and a merge; an estimate of the
-// launches' time in microseconds decides, fitted to 47 shapes of 1 to 32 heads and 128 to 8192 tokens (the cut it
-// takes is within 3 % of the best one on each):
-//  - 3.8 to start, load Q, store and end, 4.3 with two groups per workgroup, 5.1 with four;
-//  - a tile takes 1.1 with four groups, 1.8 with two, else 2.2, and 3.7 where two workgroups share the CU;
-//  - the merge takes 2.4, and the partials 1 per 1.5 MB.
-// 1024 x 4096, one head: 41 us uncut, 13 cut in 11.
+// launches' time in microseconds decides, fitted to 108 rectangles of 1 to 20 heads and 256 to 16384 tokens (the cut it
+// takes is within 0.3 % of the best one on average, 7 at most):
+//  - 3.7 to start, load Q, store and end, 4.9 with two groups per workgroup, 4.2 with four and 0.5 as they fill the device;
+//  - a tile takes 1.05 with four groups, 1.6 with two, else 2.3, and 3.7 where two workgroups share the CU;
+//  - the merge takes 3.3, and the partials 1 per 1.6 MB.
+// 1024 x 4096, one head: 34 us uncut, 12 cut in 11.
 static int fwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int max_parts) {
-  const float density = causal ? 0.5f : 1.f, lines = (float)nbh * n_qtiles;
+  const float density = visible_share(n_qtiles, n_ktiles, causal), lines = (float)nbh * n_qtiles;
   int best = 1;
   float best_us = INFINITY;
   for (int parts = 1; parts <= max_parts; ++parts) {
-    const float groups = lines * parts, longest = (float)((n_ktiles + parts - 1) / parts);
+    const int len = (n_ktiles + parts - 1) / parts, made = (n_ktiles + len - 1) / len;
+    const float groups = lines * made;
     float us;
-    switch (fwd_groups(nbh * n_qtiles * parts, (n_ktiles + parts - 1) / parts, parts, causal)) {
-      case 4: us = 5.1f + longest * 1.1f; break;
-      case 2: us = 4.3f + longest * 1.8f; break;
+    switch (fwd_groups(nbh * n_qtiles * made, len, made, causal)) {
+      case 4: us = 4.2f + 0.5f * (groups / 128) * (groups / 128) + len * 1.05f; break;
+      case 2: us = 4.9f + len * 1.6f; break;
       default: {
         const float shared = fminf(fmaxf((groups * density - kCus) / kCus, 0.f), 1.f);      // share of the workgroups with a neighbour
-        us = 3.8f + fmaxf(longest * (2.2f + 1.5f * shared), density * lines * n_ktiles * 3.7f / (2 * kCus));
+        us = 3.7f + fmaxf(len * (2.3f + 1.4f * shared), density * lines * n_ktiles * 3.7f / (2 * kCus));
       }
     }
-    if (parts > 1) us += 2.4f + 0.03f * parts + groups * (kTile * kHeadDim * 2) / 1.5e6f;
+    if (made > 1) us += 3.3f + 0.034f * made + groups * (kTile * kHeadDim * 2) / 1.64e6f;
     if (us < 0.99f * best_us) { best_us = us; best = parts; }            // more parts for a gain, not for a tie
   }
   return best;

@@ -404,6 +404,12 @@ inline int dense_parts(int64_t n_workgroups, int list_len) {
   if (want > list_len / 2) want = list_len / 2;
   return want >= 2 ? (int)want : 1;
 }
+// Share of a rectangle's tiles that is visible; causal ones are aligned at the bottom right.
+inline float visible_share(int n_qtiles, int n_ktiles, bool causal) {
+  if (!causal) return 1.f;
+  const float q = (float)n_qtiles, k = (float)n_ktiles;
+  return q >= k ? (k + 1) / (2 * q) : (k - q + 0.5f * (q + 1)) / k;
+}
 inline int64_t align256(int64_t x) { return (x + 255) / 256 * 256; }
 struct DenseSplit {     // parts and workspace layout of one dense call (bytes, 256-byte aligned blocks)
   int fwd_parts, dq_parts, dkdv_parts;
