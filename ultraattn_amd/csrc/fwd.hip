@@ -447,11 +447,12 @@ static int fwd_launch(FwdParams& p, bool plain, hipStream_t st) {
 
 // How many parts the walks of a dense forward are cut into, at most max_parts (what the workspace holds).  A cut
 // gives a small rectangle enough workgroups and costs the partials' way through memory and a merge; an estimate of the
-// launches' time in microseconds decides, fitted to 108 rectangles of 1 to 20 heads and 256 to 16384 tokens (the cut it
-// takes is within 0.3 % of the best one on average, 7 at most):
-//  - 3.7 to start, load Q, store and end, 4.9 with two groups per workgroup, 4.2 with four and 0.5 as they fill the device;
-//  - a tile takes 1.05 with four groups, 1.6 with two, else 2.3, and 3.7 where two workgroups share the CU;
-//  - the merge takes 3.3, and the partials 1 per 1.6 MB.
+// launches' time in microseconds decides, fitted to 140 rectangles of 1 to 20 heads and 256 to 16384 tokens (the cut it
+// takes is 0.6 % slower than the best one on average, 7 at most but for one of 16; with half of every causal rectangle taken for
+// hidden, 1.6 and 18):
+//  - 3.35 to start, load Q, store and end, 4.9 with two groups per workgroup, 4.3 with four and 0.5 as they fill the device;
+//  - a tile takes 1.04 with four groups, 1.55 with two, else 2.4, and 3.55 where two workgroups share the CU;
+//  - the merge takes 3.3, and the partials 1 per 1.7 MB.
 // 1024 x 4096, one head: 34 us uncut, 12 cut in 11.
 static int fwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int max_parts) {
   const float density = visible_share(n_qtiles, n_ktiles, causal), lines = (float)nbh * n_qtiles;
@@ -462,14 +463,14 @@ static int fwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int max
     const float groups = lines * made;
     float us;
     switch (fwd_groups(nbh * n_qtiles * made, len, made, causal)) {
-      case 4: us = 4.2f + 0.5f * (groups / 128) * (groups / 128) + len * 1.05f; break;
-      case 2: us = 4.9f + len * 1.6f; break;
+      case 4: us = 4.3f + 0.5f * (groups / 128) * (groups / 128) + len * 1.04f; break;
+      case 2: us = 4.9f + len * 1.55f; break;
       default: {
         const float shared = fminf(fmaxf((groups * density - kCus) / kCus, 0.f), 1.f);      // share of the workgroups with a neighbour
-        us = 3.7f + fmaxf(len * (2.3f + 1.4f * shared), density * lines * n_ktiles * 3.7f / (2 * kCus));
+        us = 3.35f + fmaxf(len * (2.4f + 1.15f * shared), density * lines * n_ktiles * 3.66f / (2 * kCus));
       }
     }
-    if (made > 1) us += 3.3f + 0.034f * made + groups * (kTile * kHeadDim * 2) / 1.64e6f;
+    if (made > 1) us += 3.3f + 0.034f * made + groups * (kTile * kHeadDim * 2) / 1.72e6f;
     if (us < 0.99f * best_us) { best_us = us; best = parts; }            // more parts for a gain, not for a tie
   }
   return best;
