@@ -749,12 +749,12 @@ static int launch_bwd(BwdParams& p, bool plain, hipStream_t st) {
 // second launch; which wins is decided by an estimate of the time in microseconds, fitted to 140 rectangles of 1
 // to 20 heads and 256 to 16384 tokens (the cut it takes is 1 % slower than the best one on average, and up to 8 but for one causal
 // rectangle of 12288; with half of every causal rectangle taken for hidden and the forms' times of before, 7 and 58):
-//  - 6.75 to start, load the resident rows, store the results and end, 9.8 in form 2, 6.4 in halves, 5.9 in form 4 and up to 2.7 as the
-//    workgroups fill the device;
-//  - a tile takes 1.4 (columns) or 0.85 (rows) in form 4, 2.6 and 1.7 in form 2, 1.9 and 1.3 in halves, 2.4 and 1.7 where two of those
-//    share a CU (5.9 together on a full device), else 3.8 and 2, and 5.1 and 3.6 where two workgroups share the CU;
-//  - the sum takes 3.2, the columns' partials 0.5, and all of them 1 per 3.7 MB; a cut has to win by 1 %.
-// 1024 x 4096, one head: 34 us uncut, 21 cut in 2 and 5; 4 heads of 1024 19.9 cut in 2 and 1, 18.1 uncut; causal 8192 x 512 17.4 and 11.9.
+//  - 6.7 to start, load the resident rows, store the results and end, 9.8 in form 2, 5.9 in halves and in form 4, there up to 2.7 more as
+//    the workgroups fill the device;
+//  - a tile takes 1.4 (columns) or 0.9 (rows) in form 4, 2.6 and 1.7 in form 2, 1.9 and 1.3 in halves, 2.4 and 1.7 where two of those
+//    share a CU (5.9 together on a full device), else 3.75 and 2, and 5.3 and 3.6 where two workgroups share the CU;
+//  - the sum takes 2.7, 0.5 more for columns, the partials 1 per 4.4 MB and 0.7 at 8 MB, 2.6 from 16 on; a cut has to win by 2 %.
+// 1024 x 4096, one head: 34 us uncut, 21.4 cut in 2 and 5, 20.5 in 1 and 3; 4 heads of 1024 19.9 cut in 2 and 1, 18.1 uncut; causal 8192 x 512 17.4 and 11.9.
 struct BwdCut { int cols, rows; };
 static BwdCut bwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int max_cols, int max_rows) {
   if (max_cols <= 1 && max_rows <= 1) return {1, 1};
@@ -772,7 +772,7 @@ static BwdCut bwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int 
   Side cols[9], rows[9];
   const int n_cols = sides(cols, max_cols, n_qtiles), n_rows = sides(rows, max_rows, n_ktiles);
   const float density = visible_share(n_qtiles, n_ktiles, causal), wk = (float)nbh * n_ktiles, wq = (float)nbh * n_qtiles;
-  const float tiles = density * wk * n_qtiles, part_us = kTile * kHeadDim * 4 / 1e6f;
+  const float tiles = density * wk * n_qtiles;
   const int seen = causal && n_ktiles < n_qtiles ? n_ktiles : n_qtiles;    // the longest column
   BwdCut best = {1, 1};
   float best_us = INFINITY;
@@ -783,22 +783,21 @@ static BwdCut bwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int 
       const int64_t lines = nbh * ((int64_t)n_ktiles * c.n + (int64_t)n_qtiles * r.n);
       float us, tc, tr, least = tiles * 10.5f / (2 * kCus);                // the work of a CU, however long the walks
       switch (bwd_form(lines, c.len + r.len, c.n + r.n, causal, n_qtiles, n_ktiles)) {
-        case 4: us = 5.9f + 2.7f * (lines / 128.f) * (lines / 128.f); tc = 1.42f; tr = 0.84f; break;
+        case 4: us = 5.9f + 2.7f * (lines / 128.f) * (lines / 128.f); tc = 1.42f; tr = 0.88f; break;
         case 2: us = 9.8f; tc = 2.6f; tr = 1.7f; break;
         case kHalves: {
           const float shared = fminf((lines - 128) * (3.f / 128), 1.f);              // lines > 128
-          us = 6.4f; tc = 1.87f + 0.55f * shared; tr = 1.34f + 0.37f * shared; least = tiles * 5.9f / kCus;
+          us = 5.9f; tc = 1.87f + 0.55f * shared; tr = 1.3f + 0.36f * shared; least = tiles * 5.9f / kCus;
           break;
         }
         default: {
           const float shared = fminf(fmaxf((groups - kCus) / kCus, 0.f), 1.f);       // share of the workgroups with a neighbour
-          us = 6.75f; tc = 3.8f + 1.32f * shared; tr = 2.05f + 1.6f * shared;
+          us = 6.7f; tc = 3.75f + 1.58f * shared; tr = 2.f + 1.6f * shared;
         }
       }
       us += fmaxf(fmaxf((c.len < seen ? c.len : seen) * tc, r.len * tr), least);
-      if (c.n > 1 || r.n > 1) us = (us + 3.2f) * 1.01f;
-      if (c.n > 1) us += 0.5f + 2.f * c.n * wk * part_us / 3.7f;
-      if (r.n > 1) us += r.n * wq * part_us / 3.7f;
+      const float mb = ((c.n > 1 ? 2.f * c.n * wk : 0.f) + (r.n > 1 ? r.n * wq : 0.f)) * (kTile * kHeadDim * 4 / 1e6f), full = fminf(mb / 8, 2.f);
+      if (mb > 0.f) us = (us + 2.7f) * 1.02f + (c.n > 1 ? 0.5f : 0.f) + mb / 4.4f + 0.66f * full * full;
       if (us < 0.99f * best_us) { best_us = us; best = {c.parts, r.parts}; }         // more parts for a gain, not for a tie
     }
   return best;
