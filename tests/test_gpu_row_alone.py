@@ -8,6 +8,7 @@ import torch
 from tests.gpu_util import SCALE
 from tests.test_gpu_dense import dense_unsplit
 from ultraattn_amd import masks, ops
+from ultraattn_amd.tilelist import build_tile_list
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -65,3 +66,16 @@ def test_dense_without_workspace_equals_the_tile_list(lib, nq, nk, nh, causal):
     got = dense_unsplit(lib, q, k, v, do, causal)
     for a, b in zip((o, lse, delta, *ops.bsa_bwd(do, q, k, v, None, lse, mask, SCALE, block=128, softmax_d=delta)), got):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("heads", [128, 132])                # 32768 and 33792 lines: both sides of a backward in one launch and in two
+def test_backward_in_one_launch_and_in_two(heads):
+    tiles = build_tile_list(masks.config_strided(16), block=512)
+    q, k, v, do = _inputs(8192, 8192, heads, batch=2)
+    o, lse = ops.bsa_fwd(q, k, v, tiles, SCALE)
+    grads = ops.bsa_bwd(do, q, k, v, o, lse, tiles, SCALE)
+    for b, h in ((0, 0), (1, heads - 1)):
+        at = (slice(b, b + 1), slice(None), slice(h, h + 1))
+        alone = ops.bsa_bwd(*(t[at].contiguous() for t in (do, q, k, v, o)), lse[b:b + 1, h:h + 1].contiguous(), tiles, SCALE)
+        for whole, one in zip(grads, alone):
+            assert torch.equal(whole[at], one)
