@@ -446,34 +446,47 @@ static int fwd_launch(FwdParams& p, bool plain, hipStream_t st) {
 }
 
 // How many parts the walks of a dense forward are cut into, at most max_parts (what the workspace holds).  A cut
-// gives a small rectangle enough workgroups and costs the partials' way through memory and a merge; an estimate of the
-// launches' time in microseconds decides, fitted to 140 rectangles of 1 to 20 heads and 256 to 16384 tokens (the cut it
-// takes is 0.6 % slower than the best one on average, 7 at most but for one of 16; with half of every causal rectangle taken for
-// hidden, 1.6 and 18):
-//  - 3.35 to start, load Q, store and end, 4.9 with two groups per workgroup, 4.3 with four and 0.5 as they fill the device;
-//  - a tile takes 1.04 with four groups, 1.55 with two, else 2.4, and 3.55 where two workgroups share the CU;
-//  - the merge takes 3.3, and the partials 1 per 1.7 MB.
+// gives a small rectangle enough workgroups and costs the partials' way through memory, a merge, and a second rounding of
+// every row: the partial O is bf16, as the workspace's size has it (error against fp64 2.33e-3 whole and 2.85e-3 cut at 8 heads of 4480, and
+// as much in 11 parts as in two).  Two estimates of the launches' time in microseconds therefore have to agree on a cut:
+//  - the first, fitted to 47 shapes of 1 to 32 heads and 128 to 8192 tokens, says which rectangles have enough to gain (5 heads of 8192,
+//    200 us whole and 179 cut in two, do not);
+//  - the second, fitted to 140 rectangles of 1 to 20 heads and 256 to 16384 tokens, counts what a causal rectangle shows and gives the number
+//    of parts, or none: 16 heads, causal 640 x 1920, 21.6 us cut in three, 19.5 whole; 2 x 3 causal 6784 94.9 and 89.8.
+// Terms: start, loading Q, storing and the end; a tile, and one where two workgroups share the CU; the merge, and the partials' bytes.
 // 1024 x 4096, one head: 34 us uncut, 12 cut in 11.
 static int fwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int max_parts) {
-  const float density = visible_share(n_qtiles, n_ktiles, causal), lines = (float)nbh * n_qtiles;
-  int best = 1;
-  float best_us = INFINITY;
-  for (int parts = 1; parts <= max_parts; ++parts) {
-    const int len = (n_ktiles + parts - 1) / parts, made = (n_ktiles + len - 1) / len;
-    const float groups = lines * made;
-    float us;
-    switch (fwd_groups(nbh * n_qtiles * made, len, made, causal)) {
-      case 4: us = 4.3f + 0.5f * (groups / 128) * (groups / 128) + len * 1.04f; break;
-      case 2: us = 4.9f + len * 1.55f; break;
-      default: {
-        const float shared = fminf(fmaxf((groups * density - kCus) / kCus, 0.f), 1.f);      // share of the workgroups with a neighbour
-        us = 3.35f + fmaxf(len * (2.4f + 1.15f * shared), density * lines * n_ktiles * 3.66f / (2 * kCus));
-      }
+  const float lines = (float)nbh * n_qtiles;
+  auto share = [](float groups) { return fminf(fmaxf((groups - kCus) / kCus, 0.f), 1.f); };        // of the workgroups with a neighbour
+  auto first = [&](int parts) {
+    const int len = (n_ktiles + parts - 1) / parts;
+    const float density = causal ? 0.5f : 1.f, groups = lines * parts, merge = parts > 1 ? 2.4f + 0.03f * parts + groups * (kTile * kHeadDim * 2) / 1.5e6f : 0.f;
+    switch (fwd_groups(nbh * n_qtiles * parts, len, parts, causal)) {
+      case 4: return merge + 5.1f + len * 1.1f;
+      case 2: return merge + 4.3f + len * 1.8f;
+      default: return merge + 3.8f + fmaxf(len * (2.2f + 1.5f * share(groups * density)), density * lines * n_ktiles * 3.7f / (2 * kCus));
     }
-    if (made > 1) us += 3.3f + 0.034f * made + groups * (kTile * kHeadDim * 2) / 1.72e6f;
-    if (us < 0.99f * best_us) { best_us = us; best = parts; }            // more parts for a gain, not for a tie
-  }
-  return best;
+  };
+  auto second = [&](int parts) {
+    const int len = (n_ktiles + parts - 1) / parts, made = (n_ktiles + len - 1) / len;
+    const float density = visible_share(n_qtiles, n_ktiles, causal), groups = lines * made;
+    const float merge = made > 1 ? 3.3f + 0.034f * made + groups * (kTile * kHeadDim * 2) / 1.72e6f : 0.f;
+    switch (fwd_groups(nbh * n_qtiles * made, len, made, causal)) {
+      case 4: return merge + 4.3f + 0.5f * (groups / 128) * (groups / 128) + len * 1.04f;
+      case 2: return merge + 4.9f + len * 1.55f;
+      default: return merge + 3.35f + fmaxf(len * (2.4f + 1.15f * share(groups * density)), density * lines * n_ktiles * 3.66f / (2 * kCus));
+    }
+  };
+  auto least = [&](auto us_of) {
+    int best = 1;
+    float best_us = INFINITY;
+    for (int parts = 1; parts <= max_parts; ++parts) {
+      const float us = us_of(parts);
+      if (us < 0.99f * best_us) { best_us = us; best = parts; }          // more parts for a gain, not for a tie
+    }
+    return best;
+  };
+  return least(first) > 1 ? least(second) : 1;
 }
 
 static bool contiguous_bshd(const int64_t* st, int seqlen, int n_heads) {
