@@ -57,6 +57,11 @@ __device__ __forceinline__ ParamsLate params_late() {
   asm volatile("" : "+s"(p));
   return p;
 }
+// With one group what a walk needs is read behind the branch that leads to it: read before, the parameters of both sides at once ask for more
+// scalar registers than there are, and up to 61 of them live in vector lanes (causal 32 heads of 2048, backward 131.9 -> 121.6 us with
+// the two kinds of walk in kernels of their own).  The short walks of more groups start 2 % earlier with all parameters in flight before the branch.
+template <int kForm>
+__device__ __forceinline__ const BwdParams& params_of_walk(const BwdParams& given) { return kForm == 1 ? *(const BwdParams*)params_late() : given; }
 // 32 output rows of a wave: in the caller's strided bf16 tensor, or in part `part` of the fp32 partials.
 __device__ __forceinline__ void store_result(const __attribute__((address_space(4))) BwdSide* p, bf16* out, int64_t os_b, int64_t os_s,
                                              int64_t os_h, int n_heads, int part, int b, int64_t row0, int h, int64_t seq,
@@ -111,7 +116,7 @@ struct Stages : Groups<kForm> {
   static constexpr int kStatBytes = 2 * Groups<kForm>::kRows * 4;
   static constexpr int kStat = 4 * kPitch;
   static constexpr int kEntries = kStat + 2 * kStatBytes;
-  static constexpr int kBytes = kEntries + 4 * Walk<kForm, false>::kBytes;
+  static constexpr int kBytes = kEntries + (kForm == 1 ? 4 * Walk<false, false>::kBytes : 0);
 };
 static_assert(3 * Stages<1>::kPitch + kBlockPitch + 6 * kGroupPitch < 65536, "operand offsets fit the instructions' offset field");
 
@@ -251,8 +256,9 @@ __device__ __forceinline__ void dkdv_block(const PairAddr& ad, uint32_t stat_bas
 // its share of every tile through stages of its own, and the results are added through LDS.  Where the launch gives a CU one workgroup of
 // four waves at most, one wave per SIMD would leave the matrix pipe idle between its dependent steps (2.2 us
 // per half tile of dK/dV, 0.9 of them MFMAs); the other groups fill the CU without partial results in memory.
-template <int kForm>
-__device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block, int block) {
+template <int kForm, bool kDense>
+__device__ __forceinline__ void dkdv_walk(const BwdParams& given, uint32_t lds_block, int block) {
+  const BwdParams& p = params_of_walk<kForm>(given);
   using S = Stages<kForm>;
   const int tid = threadIdx.x % (64 * S::kWaves), lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -263,9 +269,8 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block
   const int sub = pos & (S::kLines - 1);         // which half of the tile's keys
   pos >>= S::kLines - 1;
   const int b = quotient(bh, p.by_heads), h = bh - b * p.n_heads;
-  const bool dense = kForm > 1 || p.dense;
   int kt, e0, e1, diag = -1, part = 0;
-  if (dense) {
+  if constexpr (kDense) {
     part = quotient(pos, p.cols.by_lines);
     kt = pos - part * p.n_ktiles;                          // column 0 is the longest of a causal rectangle
     if (p.cols_reversed) kt = p.n_ktiles - 1 - kt;
@@ -281,8 +286,9 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& p, uint32_t lds_block
   const int64_t seq_q = (int64_t)p.n_qtiles * kTile;
   PairStream<kForm> in(p.q + b * p.qs.b + h * p.qs.h, (int)p.qs.s, p.dout + b * p.ds.b + h * p.ds.h, (int)p.ds.s, lds_base, wave, lane);
   // A step is one half of a tile, in order; with more groups half or quarter `group` of a tile.
-  Walk<kForm, false> walk(e0, e1, diag, lds_base + S::kEntries + wave * Walk<kForm, false>::kBytes);
-  auto fetch = [&](int e) { walk.fetch(e, dense, p.cols.idx, p.cols.flag, p.n_qtiles); };
+  using W = Walk<kDense, false>;
+  W walk(e0, e1, diag, lds_base + S::kEntries + wave * W::kBytes);
+  auto fetch = [&](int e) { walk.fetch(e, p.cols.idx, p.cols.flag, p.n_qtiles); };
   // The rows' statistics of a step: its rows' -lse/softmax_scale (lse = -inf, a row without keys, stays -inf so that P = 0) and
   // -delta, which the accumulators of S and dP' start from.  Every wave brings 16 rows of both: lanes 0..15 (and
   // 32..47, which do the same) lse, the others delta.  They are loaded two steps before their use, turned and put into LDS a step
@@ -491,8 +497,9 @@ __device__ __forceinline__ void dq_block(const PairAddr& ad, const bf16x8 (&qf)[
   }
 }
 
-template <int kForm>
-__device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_block, int block) {
+template <int kForm, bool kDense>
+__device__ __forceinline__ void dq_walk(const BwdParams& given, uint32_t lds_block, int block) {
+  const BwdParams& p = params_of_walk<kForm>(given);
   using S = Stages<kForm>;
   const int tid = threadIdx.x % (64 * S::kWaves), lane = tid & 63, l32 = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -504,9 +511,8 @@ __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_block, 
   pos >>= S::kLines - 1;
   const int b = quotient(bh, p.by_heads), h = bh - b * p.n_heads;
   const int64_t seq_q = (int64_t)p.n_qtiles * kTile;
-  const bool dense = kForm > 1 || p.dense;
   int qt, e0, e1, diag = -1, part = 0;
-  if (dense) {
+  if constexpr (kDense) {
     part = quotient(pos, p.rows.by_lines);
     const int line = pos - part * p.n_qtiles;
     qt = p.dense_causal ? p.n_qtiles - 1 - line : line;    // longest rows first
@@ -520,8 +526,8 @@ __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_block, 
     e1 = min(max(sload(p.rows.ptr, qt + 1), e0), p.nnz);
   }
   PairStream<kForm> in(p.k + b * p.ks.b + h * p.ks.h, (int)p.ks.s, p.v + b * p.vs.b + h * p.vs.h, (int)p.vs.s, lds_base, wave, lane);
-  Walk<kForm, true> walk(e0, e1, diag);      // steps as in dK/dV's walk
-  auto fetch = [&](int e) { walk.fetch(e, dense, p.rows.idx, p.rows.flag, p.n_ktiles); };
+  Walk<kDense, true> walk(e0, e1, diag);      // steps as in dK/dV's walk
+  auto fetch = [&](int e) { walk.fetch(e, p.rows.idx, p.rows.flag, p.n_ktiles); };
   auto part_of = [&](int stage) { return S::kSteps * group + (S::kSteps == 2 ? stage : 0); };      // half or quarter of the tile
   int ent = 0, ent_next = 0;
   if (e0 < e1) {
@@ -639,19 +645,19 @@ __device__ __forceinline__ void dq_walk(const BwdParams& p, uint32_t lds_block, 
 // ---- kernels ------------------------------------------------------------------------------------
 __global__ __launch_bounds__(Groups<1>::kThreads, 2) void dkdv_kernel(const BwdParams p) {
   __shared__ __attribute__((aligned(1024))) unsigned char smem[Stages<1>::kBytes];
-  dkdv_walk<1>(p, (uint32_t)(uintptr_t)(UA_LDS unsigned char*)smem, blockIdx.x);
+  dkdv_walk<1, false>(p, (uint32_t)(uintptr_t)(UA_LDS unsigned char*)smem, blockIdx.x);
 }
 __global__ __launch_bounds__(Groups<1>::kThreads, 2) void dq_kernel(const BwdParams p) {
   __shared__ __attribute__((aligned(1024))) unsigned char smem[Stages<1>::kBytes];
-  dq_walk<1>(p, (uint32_t)(uintptr_t)(UA_LDS unsigned char*)smem, blockIdx.x);
+  dq_walk<1, false>(p, (uint32_t)(uintptr_t)(UA_LDS unsigned char*)smem, blockIdx.x);
 }
 // Both sides in one launch.
-template <int kForm>
+template <int kForm, bool kDense>
 __global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void bwd_kernel(const BwdParams p) {
   __shared__ __attribute__((aligned(1024))) unsigned char smem[Stages<kForm>::kCount * Stages<kForm>::kBytes];
   const uint32_t lds_base = (uint32_t)(uintptr_t)(UA_LDS unsigned char*)smem;
-  if ((int)blockIdx.x < p.n_col_blocks) dkdv_walk<kForm>(p, lds_base, blockIdx.x);
-  else                                  dq_walk<kForm>(p, lds_base, blockIdx.x - p.n_col_blocks);
+  if ((int)blockIdx.x < p.n_col_blocks) dkdv_walk<kForm, kDense>(p, lds_base, blockIdx.x);
+  else                                  dq_walk<kForm, kDense>(p, lds_base, blockIdx.x - p.n_col_blocks);
 }
 
 static int fill_common(BwdParams& p, const void* q, const void* k, const void* v, const void* dout,
@@ -736,9 +742,9 @@ static int launch_bwd(BwdParams& p, bool plain, hipStream_t st) {
   // of one side share a CU with the short ones of the other (32 causal heads of 1024: 43.6 -> 41.5 us).
   p.cols_reversed = form == kHalves ? p.dense_causal : form == 1 && (p.dense_causal || !p.dense) && n > kCus && n <= 2 * kCus;
   switch (form) {
-    case 4: hipLaunchKernelGGL(bwd_kernel<4>, dim3(2 * n), dim3(512), 0, st, p); break;
-    case 2: hipLaunchKernelGGL(bwd_kernel<2>, dim3(n), dim3(512), 0, st, p); break;
-    case kHalves: hipLaunchKernelGGL(bwd_kernel<kHalves>, dim3(2 * n), dim3(Groups<kHalves>::kThreads), 0, st, p); break;
+    case 4: hipLaunchKernelGGL((bwd_kernel<4, true>), dim3(2 * n), dim3(512), 0, st, p); break;
+    case 2: hipLaunchKernelGGL((bwd_kernel<2, true>), dim3(n), dim3(512), 0, st, p); break;
+    case kHalves: hipLaunchKernelGGL((bwd_kernel<kHalves, true>), dim3(2 * n), dim3(Groups<kHalves>::kThreads), 0, st, p); break;
     default:
       // Of the longest launches over tile lists each side runs as its own: the last workgroups of the columns and the first of the
       // rows have little to share there, and the kernel of both keeps more of its scalars in vector lanes (32 heads of 128k, 65536
@@ -749,7 +755,8 @@ static int launch_bwd(BwdParams& p, bool plain, hipStream_t st) {
         hipLaunchKernelGGL(dq_kernel, dim3(row_blocks(p)), dim3(256), 0, st, p);
         break;
       }
-      hipLaunchKernelGGL(bwd_kernel<1>, dim3(n), dim3(256), 0, st, p);
+      if (p.dense) hipLaunchKernelGGL((bwd_kernel<1, true>), dim3(n), dim3(256), 0, st, p);
+      else         hipLaunchKernelGGL((bwd_kernel<1, false>), dim3(n), dim3(256), 0, st, p);
   }
   return launched();
 }

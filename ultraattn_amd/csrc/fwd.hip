@@ -151,7 +151,7 @@ __device__ __forceinline__ void key_blocks(const unsigned char* sK, const unsign
 // are combined through LDS.  A launch that gives a CU one workgroup of four waves at most runs it at
 // one wave per SIMD, where a half tile takes 1.2 us of which the matrix pipe is busy 0.4; with more groups the CU is
 // as full as with two workgroups, without partial results in memory.
-template <int kForm>
+template <int kForm, bool kDense>
 __global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void fwd_kernel(const FwdParams p) {
   constexpr int kWaves = Groups<kForm>::kWaves, kRows = Groups<kForm>::kRows, kLines = Groups<kForm>::kLines;
   constexpr int kStageBytes = kRows * kRowBytes;
@@ -179,9 +179,8 @@ __global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void fwd_kernel(const F
   pos >>= kLines - 1;
   if (pos < p.n_first) pos = p.n_first - 1 - pos;
   const int b = quotient(bh, p.by_heads), h = bh - b * p.n_heads;
-  const bool dense = kForm > 1 || p.dense;
   int qt, e0, e1, diag = -1, part = -1;
-  if (dense) {
+  if constexpr (kDense) {
     int line = pos;
     if (pos >= p.n_whole) {
       part = quotient(pos - p.n_whole, p.by_cut);
@@ -227,8 +226,8 @@ __global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void fwd_kernel(const F
   };
 
   // A step is one half of a tile, in order; with more groups half or quarter `group` of a tile.
-  Walk<kForm, true> walk(e0, e1, diag);
-  auto fetch = [&](int e) { walk.fetch(e, dense, p.col_idx, p.flag, p.n_ktiles); };
+  Walk<kDense, true> walk(e0, e1, diag);
+  auto fetch = [&](int e) { walk.fetch(e, p.col_idx, p.flag, p.n_ktiles); };
   // the first stage goes in flight before anything else
   int ent = 0, ent_next = 0;
   if (e0 < e1) {
@@ -433,14 +432,15 @@ static int fwd_launch(FwdParams& p, bool plain, hipStream_t st) {
   p.by_heads = make_div(p.n_heads);
   p.by_cut = make_div(n_cut ? n_cut : 1);
   switch (form) {
-    case 4: hipLaunchKernelGGL(fwd_kernel<4>, dim3(2 * n), dim3(512), 0, st, p); break;
-    case 2: hipLaunchKernelGGL(fwd_kernel<2>, dim3(n), dim3(512), 0, st, p); break;
+    case 4: hipLaunchKernelGGL((fwd_kernel<4, true>), dim3(2 * n), dim3(512), 0, st, p); break;
+    case 2: hipLaunchKernelGGL((fwd_kernel<2, true>), dim3(n), dim3(512), 0, st, p); break;
     default:
       // Up to two workgroups per CU the whole launch is resident at once, and those after the first 256 join them in
       // launch order.  Lists come roughly by falling length, so the first ones are taken in reverse: long and
       // short lists then share a CU (strided 8k, 8 heads: the longest sum on a CU 40 -> 37 tiles, causal 96 -> 65).
       if (!p.dense && n > kCus && n <= 2 * kCus) p.n_first = kCus * p.n_qtiles / (int)n;
-      hipLaunchKernelGGL(fwd_kernel<1>, dim3(n), dim3(256), 0, st, p);
+      if (p.dense) hipLaunchKernelGGL((fwd_kernel<1, true>), dim3(n), dim3(256), 0, st, p);
+      else         hipLaunchKernelGGL((fwd_kernel<1, false>), dim3(n), dim3(256), 0, st, p);
   }
   return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH;
 }

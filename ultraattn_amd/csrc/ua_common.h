@@ -268,28 +268,28 @@ struct Groups {
   static constexpr int kThreads = 64 * kWaves * kCount;
 };
 
-// The entries e0 .. e1 - 1 of a workgroup's line: tile | causal flag << 30.  With one group every wave holds 64 of them, in a register
+// The entries e0 .. e1 - 1 of a workgroup's line: tile | causal flag << 30.  Of a list every wave holds 64 of them, in a register
 // or, where none is left, in kBytes of LDS of its own: read one by one through the scalar cache they cost the walks two
 // dependent loads per tile (strided 128k, 32 heads, with the copies between the MFMAs: forward 18.3 -> 17.9 ms, dQ 25.6 -> 24.5).
-// With more groups (dense rectangles) entry e is tile e itself.
-template <int kForm, bool kInRegister>
+// Entry e of a dense rectangle is tile e itself.
+template <bool kDense, bool kInRegister>
 struct Walk {
-  static constexpr int kBytes = kForm == 1 && !kInRegister ? 256 : 0;
+  static constexpr int kBytes = kDense || kInRegister ? 0 : 256;
   int e0, e1, diag, window;
   uint32_t lds;
   __device__ __forceinline__ Walk(int e0_, int e1_, int diag_, uint32_t lds_ = 0) : e0(e0_), e1(e1_), diag(diag_), window(0), lds(lds_) {}
-  // Brings entries e .. e + 63 (e < e1); a dense walk's tiles are e itself.
-  __device__ __forceinline__ void fetch(int e, bool dense, const int32_t* idx, const uint8_t* flag, int n_tiles) {
-    if constexpr (kForm == 1) {
+  // Brings entries e .. e + 63 (e < e1).
+  __device__ __forceinline__ void fetch(int e, const int32_t* idx, const uint8_t* flag, int n_tiles) {
+    if constexpr (!kDense) {
       const int lane = fresh_lane(), i = min(e + lane, e1 - 1);
-      window = dense ? i | ((int)(i == diag) << 30) : min(max(idx[i], 0), n_tiles - 1) | ((int)(flag[i] != 0) << 30);
+      window = min(max(idx[i], 0), n_tiles - 1) | ((int)(flag[i] != 0) << 30);
       if constexpr (!kInRegister) lds_put(lds + 4 * lane, window);
     }
   }
   // The first of every 64 entries has to be fetched before it is asked for.
-  __device__ __forceinline__ bool has(int e) const { return kForm > 1 || ((e - e0) & 63) != 0 || e >= e1; }
+  __device__ __forceinline__ bool has(int e) const { return kDense || ((e - e0) & 63) != 0 || e >= e1; }
   __device__ __forceinline__ int at(int e) const {
-    if constexpr (kForm > 1) return e | ((int)(e == diag) << 30);
+    if constexpr (kDense) return e | ((int)(e == diag) << 30);
     if constexpr (kInRegister) return __builtin_amdgcn_readlane(window, (e - e0) & 63);
     return __builtin_amdgcn_readfirstlane(lds_get<int>(lds + 4 * ((e - e0) & 63)));
   }
