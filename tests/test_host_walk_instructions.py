@@ -61,3 +61,8 @@ def test_no_scalars_in_vector_lanes(assembly, backward_assembly):
     spills = {**_spills(assembly, "sgpr"), **_spills(backward_assembly, "sgpr")}
     form_1 = {k: n for k, n in spills.items() if "kernelILi" not in k or "kernelILi1E" in k}
     assert len(form_1) == 6 and all(n <= 2 for n in form_1.values()), form_1
+
+
+def test_no_vector_registers_spilled_in_the_backward(backward_assembly):
+    spills = _spills(backward_assembly, "vgpr")
+    assert len(spills) == 7 and not any(spills.values()), spills

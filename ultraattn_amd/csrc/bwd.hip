@@ -38,7 +38,7 @@ struct BwdParams {
   const float* lse; const float* delta;
   int batch, n_heads, n_qtiles, n_ktiles, nnz;
   Strides3 qs, ks, vs, ds;
-  float scale_log2, scale;
+  float scale_log2, scale, neg_inv_scale;
   Div by_heads;
   // Dense rectangle (no list arrays).  The rows walk key tiles [0, n_ktiles) of a query tile, with dense_causal
   // [0, qt + diag_off], the last one causal; the columns walk query tiles [0, n_qtiles) of a key tile, with
@@ -98,7 +98,8 @@ __device__ __forceinline__ void store_block(const __attribute__((address_space(4
 // hold K, V, dK and dV; two independent workgroups share a CU, so that one's exp2 and barriers hide behind
 // the other's MFMAs.  Against one workgroup of eight waves in two roles (S/dV and dP/dK, P handed over
 // through LDS): strided 128k, 32 heads 37.8 -> 33.5 ms, causal 32k 15.8 -> 13.7 ms (1.25-1.3 PFLOP/s of the four
-// products).  More fragments ahead or a P computed during dP's MFMAs spill registers: 3-15 % slower.
+// products).  Row fragments are fetched two MFMAs ahead (three: the same within 0.5 %); a P computed during dP's MFMAs spills
+// registers: 3-15 % slower.
 //
 // LDS: four consecutive rows (1 KiB, one copy instruction of one wave) lie at a pitch of 1040 bytes and a
 // row's 16-byte chunks are XORed with 4 * (row % 4).  16 consecutive rows then hit 16 different slots
@@ -121,6 +122,11 @@ struct Stages : Groups<kForm> {
 static_assert(3 * Stages<1>::kPitch + kBlockPitch + 6 * kGroupPitch < 65536, "operand offsets fit the instructions' offset field");
 
 __device__ __forceinline__ void keep_in_register(uint32_t& x) { asm volatile("" : "+v"(x)); }
+__device__ __forceinline__ float in_scalar(float x) {            // a wave-uniform value in a scalar register
+  int bits = __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x));
+  asm volatile("" : "+s"(bits));
+  return __builtin_bit_cast(float, bits);
+}
 __device__ __forceinline__ bf16x8 lds_abs_b128(uint32_t a) { return *reinterpret_cast<const UA_LDS bf16x8*>(a); }
 __device__ __forceinline__ bf16x8 lds_abs_tr_pair(uint32_t a_lo, uint32_t a_hi) {
   const bf16x4 x = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(reinterpret_cast<UA_LDS bf16x4*>(a_lo));
@@ -194,7 +200,8 @@ template <int kOff, int kPitch, int kStatOff, int kStatBytes, int kCopies, class
 __device__ __forceinline__ void dkdv_block(const PairAddr& ad, uint32_t stat_base, const bf16x8 (&kf)[8], const bf16x8 (&vf)[8], f32x16 (&dk)[4],
                                            f32x16 (&dv)[4], float scale_log2, bool mask, Copy copy) {
   f32x16 s, dp;
-  const uint32_t stat = stat_base + 16 * (fresh_lane() >> 5);           // this lane half's 4 consecutive row statistics
+  uint32_t stat = stat_base + 16 * (fresh_lane() >> 5);           // this lane half's 4 consecutive row statistics
+  keep_in_register(stat);                // (the reads' offsets then are constants: a lone workgroup 2 % faster)
   // element i of a block: query row 8*(i/4) + 4*hi + i%4, key column lane%32
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
@@ -203,6 +210,7 @@ __device__ __forceinline__ void dkdv_block(const PairAddr& ad, uint32_t stat_bas
 #pragma unroll
     for (int j = 0; j < 4; ++j) { s[4 * g + j] = a[j]; dp[4 * g + j] = c[j]; }
   }
+  __builtin_amdgcn_sched_barrier(0);       // the reads below, mixed with what came before them, spill registers
   {
     // 16 row fragments, Q and dO alternating, fetched kAhead reads ahead of their MFMA
     constexpr int kAhead = 2;
@@ -290,21 +298,21 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& given, uint32_t lds_b
   W walk(e0, e1, diag, lds_base + S::kEntries + wave * W::kBytes);
   auto fetch = [&](int e) { walk.fetch(e, p.cols.idx, p.cols.flag, p.n_qtiles); };
   // The rows' statistics of a step: its rows' -lse/softmax_scale (lse = -inf, a row without keys, stays -inf so that P = 0) and
-  // -delta, which the accumulators of S and dP' start from.  Every wave brings 16 rows of both: lanes 0..15 (and
-  // 32..47, which do the same) lse, the others delta.  They are loaded two steps before their use, turned and put into LDS a step
-  // before it: by then everything loaded has arrived at the end of a step, and nothing waits.  (Two of the waves bringing all of
-  // it, with their addresses in scratch memory, kept the other two waiting for a tenth of every step.)
-  const int64_t stat_row = ((int64_t)b * p.n_heads + h) * seq_q + 16 * wave;
-  const float *const lse_rows = p.lse + stat_row, *const delta_rows = p.delta + stat_row;
+  // -delta, which the accumulators of S and dP' start from.  Every wave brings 32 of them (lanes 32..63 do the same), the first half
+  // of the waves lse, the others delta: which of the two, and where, are scalars.  They are loaded two steps before their use, turned and
+  // put into LDS a step before it: by then everything loaded has arrived at the end of a step, and nothing waits.  (Half of every wave's lanes
+  // bringing lse and half delta took 42 more vector instructions a half tile, and a lone workgroup 5 % more time: causal 4096, one head,
+  // dK/dV 122.5 -> 116.0 us; causal 8 heads of 6144, backward 275 -> 263; strided 32k, 16 heads, dK/dV 1643 -> 1634.)
+  const float scale_log2 = in_scalar(p.scale_log2);        // (else read from memory at every block)
+  const bool of_delta = wave >= S::kWaves / 2;
+  const float* const stat_rows = (of_delta ? p.delta : p.lse) + ((int64_t)b * p.n_heads + h) * seq_q + 32 * (wave & (S::kWaves / 2 - 1));
+  const float factor = in_scalar(of_delta ? -1.f : p.neg_inv_scale), kept = in_scalar(of_delta ? __builtin_nanf("") : -INFINITY);
   auto load_stat = [&](int entry, int part) {
-    const int l = fresh_lane();
-    return (l & 16 ? delta_rows : lse_rows)[walk.tile(entry) * kTile + part * S::kRows + (l & 15)];
+    const float* const rows = stat_rows + (int64_t)walk.tile(entry) * kTile + part * S::kRows;
+    return rows[(uint32_t)(fresh_lane() & 31)];
   };
-  const float neg_inv_scale = -1.f / p.scale;
   auto put_stat = [&](int stage, float x) {
-    const int l = fresh_lane();
-    const float y = x * (l & 16 ? -1.f : neg_inv_scale);
-    lds_put(lds_base + S::kStat + stage * S::kStatBytes + (16 * wave + (l & 15) + (l & 16 ? S::kRows : 0)) * 4, !(l & 16) && x == -INFINITY ? x : y);
+    lds_put(lds_base + S::kStat + stage * S::kStatBytes + 128 * wave + 4 * (fresh_lane() & 31), x == kept ? x : x * factor);
   };
   int ent = 0, ent_next = 0;
   float st0 = 0.f, stat = 0.f;
@@ -376,7 +384,7 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& given, uint32_t lds_b
       auto block = [&](auto mb_tag) {
         constexpr int kMb = decltype(mb_tag)::value;
         dkdv_block<kOff + kMb * kBlockPitch, S::kPitch, kStatOff + kMb * 128, S::kStatBytes, kCopies>(
-            ad, lds_base + S::kStat, kf, vf, dk, dv, p.scale_log2, false, [&](int n) { in.template copy<kStage ^ 1>(kMb * kCopies + n, part_next); });
+            ad, lds_base + S::kStat, kf, vf, dk, dv, scale_log2, false, [&](int n) { in.template copy<kStage ^ 1>(kMb * kCopies + n, part_next); });
       };
       block(std::integral_constant<int, 0>{});
       if constexpr (kBlocks == 2) block(std::integral_constant<int, 1>{});
@@ -391,7 +399,7 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& given, uint32_t lds_b
 #pragma unroll 1
       for (int mb = max(k_block - nb, 0); mb < kBlocks; ++mb) {
         ad.shift(mb * kBlockPitch);
-        dkdv_block<kOff, S::kPitch, kStatOff, S::kStatBytes, 0>(ad, lds_base + S::kStat + mb * 128, kf, vf, dk, dv, p.scale_log2, nb + mb == k_block,
+        dkdv_block<kOff, S::kPitch, kStatOff, S::kStatBytes, 0>(ad, lds_base + S::kStat + mb * 128, kf, vf, dk, dv, scale_log2, nb + mb == k_block,
                                                                 [](int) {});
         ad.shift(-mb * kBlockPitch);
       }
@@ -679,7 +687,7 @@ static int fill_common(BwdParams& p, const void* q, const void* k, const void* v
   p.batch = batch; p.n_heads = n_heads; p.n_qtiles = n_qtiles; p.n_ktiles = n_ktiles; p.nnz = nnz;
   p.qs = {qs[0], qs[1], qs[2]}; p.ks = {ks[0], ks[1], ks[2]};
   p.vs = {vs[0], vs[1], vs[2]}; p.ds = {ds[0], ds[1], ds[2]};
-  p.scale = softmax_scale; p.scale_log2 = softmax_scale * kLog2e;
+  p.scale = softmax_scale; p.scale_log2 = softmax_scale * kLog2e; p.neg_inv_scale = -1.f / softmax_scale;
   p.dense = 0; p.dense_causal = 0; p.diag_off = 0; p.n_col_blocks = 0; p.cols_reversed = 0;
   p.cols = BwdSide{}; p.rows = BwdSide{};
   p.cols.n_parts = p.rows.n_parts = 1;
