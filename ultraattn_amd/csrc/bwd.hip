@@ -273,7 +273,7 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& given, uint32_t lds_b
   const int group = S::kCount == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * S::kWaves));
   const uint32_t lds_base = lds_block + group * S::kBytes;
   int pos, bh;
-  map_block(block, p.cols.map, pos, bh);
+  map_block<kForm == kHalves>(block, p.cols.map, pos, bh);
   const int sub = pos & (S::kLines - 1);         // which half of the tile's keys
   pos >>= S::kLines - 1;
   const int b = quotient(bh, p.by_heads), h = bh - b * p.n_heads;
@@ -514,7 +514,7 @@ __device__ __forceinline__ void dq_walk(const BwdParams& given, uint32_t lds_blo
   const int group = S::kCount == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * S::kWaves));
   const uint32_t lds_base = lds_block + group * S::kBytes;
   int pos, bh;
-  map_block(block, p.rows.map, pos, bh);
+  map_block<kForm == kHalves>(block, p.rows.map, pos, bh);
   const int sub = pos & (S::kLines - 1);         // which half of the tile's queries
   pos >>= S::kLines - 1;
   const int b = quotient(bh, p.by_heads), h = bh - b * p.n_heads;
