@@ -82,3 +82,9 @@ def test_around_the_bounds(sq, sk, nh, causal):
 ])
 def test_half_lines(sq, sk, nh, causal):
     test_around_the_bounds(sq, sk, nh, causal)
+
+
+@pytest.mark.parametrize("sq,sk,nh", [(512, 512, 64), (512, 512, 65), (384, 640, 96), (512, 384, 90), (128, 128, 256)])
+def test_two_to_three_workgroups_per_cu(sq, sk, nh):
+    """512 and 520 lines, 768 with longer rows, 630 with longer columns, 512 of one tile: where the rows' wavefronts go first and where not."""
+    test_around_the_bounds(sq, sk, nh, False)

@@ -46,6 +46,7 @@ struct BwdParams {
   int dense, dense_causal, diag_off;
   int n_col_blocks;                        // bwd_kernel: workgroups of the columns, those of the rows follow
   int cols_reversed;                       // launch order of the columns (see launch_bwd)
+  int rows_ahead;                          // the rows' wavefronts go first on a CU (see launch_bwd)
   BwdSide cols, rows;
 };
 
@@ -508,6 +509,7 @@ __device__ __forceinline__ void dq_block(const PairAddr& ad, const bf16x8 (&qf)[
 template <int kForm, bool kDense>
 __device__ __forceinline__ void dq_walk(const BwdParams& given, uint32_t lds_block, int block) {
   const BwdParams& p = params_of_walk<kForm>(given);
+  if (kForm == 1 && kDense && p.rows_ahead) __builtin_amdgcn_s_setprio(1);
   using S = Stages<kForm>;
   const int tid = threadIdx.x % (64 * S::kWaves), lane = tid & 63, l32 = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -688,7 +690,7 @@ static int fill_common(BwdParams& p, const void* q, const void* k, const void* v
   p.qs = {qs[0], qs[1], qs[2]}; p.ks = {ks[0], ks[1], ks[2]};
   p.vs = {vs[0], vs[1], vs[2]}; p.ds = {ds[0], ds[1], ds[2]};
   p.scale = softmax_scale; p.scale_log2 = softmax_scale * kLog2e; p.neg_inv_scale = -1.f / softmax_scale;
-  p.dense = 0; p.dense_causal = 0; p.diag_off = 0; p.n_col_blocks = 0; p.cols_reversed = 0;
+  p.dense = 0; p.dense_causal = 0; p.diag_off = 0; p.n_col_blocks = 0; p.cols_reversed = 0; p.rows_ahead = 0;
   p.cols = BwdSide{}; p.rows = BwdSide{};
   p.cols.n_parts = p.rows.n_parts = 1;
   return UA_OK;
@@ -749,6 +751,11 @@ static int launch_bwd(BwdParams& p, bool plain, hipStream_t st) {
   // order.  Both sides come longest first (lists roughly); the columns are then taken in reverse, so that the long ones
   // of one side share a CU with the short ones of the other (32 causal heads of 1024: 43.6 -> 41.5 us).
   p.cols_reversed = form == kHalves ? p.dense_causal : form == 1 && (p.dense_causal || !p.dense) && n > kCus && n <= 2 * kCus;
+  // Of up to three workgroups per CU the third one starts when a row of the first 512 is through, and the launch ends with rows that began
+  // second: the rows' wavefronts go first where a CU has a column's as well (16 heads of 2304: 158 us, without 143; 64 of 640: 56.1, 48.9; 9 x 27
+  // tiles, 16 heads cut, 113.5, 111.9).  Not where the columns are the longer ones (32 heads of 1536 x 768: 67.6, 75.6), and
+  // beyond 768 lines it goes either way (8 x 8 tiles, 896 lines 104.4 and 106.9, 1200 148.5 and 141.4, 1504 175.4 and 189.2).
+  p.rows_ahead = form == 1 && p.dense && !p.dense_causal && n > 2 * kCus && n <= 3 * kCus && p.rows.part_len >= p.cols.part_len;
   switch (form) {
     case 4: hipLaunchKernelGGL((bwd_kernel<4, true>), dim3(2 * n), dim3(512), 0, st, p); break;
     case 2: hipLaunchKernelGGL((bwd_kernel<2, true>), dim3(n), dim3(512), 0, st, p); break;
