@@ -78,7 +78,8 @@ def test_around_the_bounds(sq, sk, nh, causal):
     (512, 128, 50, True), (128, 640, 42, False),                 # empty walks on half lines; odd walks of one and five
     (128, 256, 43, False), (256, 128, 44, True),                 # 86 and 43, 44 and 88 lines a side: the last 8 of a side not full
     (384, 384, 23, False), (256, 256, 33, True), (128, 384, 33, True),      # halves of 69, of 66, of 33 and 99
-    (2048, 256, 6, False), (640, 1408, 5, False),                # cut columns and cut rows on half lines
+    (2048, 256, 6, False), (640, 1408, 5, False),                # cut columns on half lines; odd walks of five and eleven
+    (384, 2560, 4, False), (256, 2816, 4, True),                 # cut rows on half lines
 ])
 def test_half_lines(sq, sk, nh, causal):
     test_around_the_bounds(sq, sk, nh, causal)

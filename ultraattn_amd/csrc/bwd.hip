@@ -778,15 +778,20 @@ static int launch_bwd(BwdParams& p, bool plain, hipStream_t st) {
 
 // How many parts the two sides of a dense backward are cut into, at most what the workspace holds.  A cut gives a
 // small rectangle enough workgroups for the device and costs the partials' way through memory and a
-// second launch; which wins is decided by an estimate of the time in microseconds, fitted to 140 rectangles of 1
-// to 20 heads and 256 to 16384 tokens (the cut it takes is 1 % slower than the best one on average, and up to 8 but for one causal
-// rectangle of 12288; with half of every causal rectangle taken for hidden and the forms' times of before, 7 and 58):
-//  - 6.7 to start, load the resident rows, store the results and end, 9.8 in form 2, 5.9 in halves and in form 4, there up to 2.7 more as
-//    the workgroups fill the device;
-//  - a tile takes 1.4 (columns) or 0.9 (rows) in form 4, 2.6 and 1.7 in form 2, 1.9 and 1.3 in halves, 2.4 and 1.7 where two of those
-//    share a CU (5.9 together on a full device), else 3.75 and 2, and 5.3 and 3.6 where two workgroups share the CU;
-//  - the sum takes 2.7, 0.5 more for columns, the partials 1 per 4.4 MB and 0.7 at 8 MB, 2.6 from 16 on; a cut has to win by 2 %.
-// 1024 x 4096, one head: 34 us uncut, 21.4 cut in 2 and 5, 20.5 in 1 and 3; 4 heads of 1024 19.9 cut in 2 and 1, 18.1 uncut; causal 8192 x 512 17.4 and 11.9.
+// second launch; which wins is decided by an estimate of the time in microseconds, fitted to all cuts of 1427 rectangles of 1
+// to 130 heads and 256 to 24000 tokens.  The cut it takes is 0.9 % slower than the best one on average, 72 times by more than 5 %, 22 % at
+// most; without what is said of launches beyond 256 and 512 lines 2.4 %, 255 times and 39 % (2 heads of 11136: 472 us cut
+// in 2 and 1, 409 whole, 389 in 2 and 2):
+//  - a start and end (loading the resident rows, storing the results), longer as half lines fill the device, and the longest walks;
+//  - with one group per workgroup a tile takes 3.6 (column) or 2.3 (row), 4.1 or 3.6 where two workgroups share the CU.  The second
+//    workgroups of 257 to 512 even lines are the last of the rows, beside a column;
+//  - beyond 512 the last rows begin when something else is through: a row beside a column if those are few and shorter, else a row or
+//    column, or a round of columns; sooner where the rows' wavefronts go first (see launch_bwd), and where a causal
+//    rectangle's short walks make room;
+//  - no less than all tiles and workgroups take on a full device;
+//  - the sum takes 2, 0.7 more for columns, 1.3 for columns and rows, the partials 1 per 4.3 MB and 0.3 at 8 MB, 1.2 from 16 on; a cut
+//    has to win by 3.5 %.
+// 1024 x 4096, one head: 34 us uncut, 20.7 cut in 1 and 3; 4 heads of 1024 19.9 cut in 2 and 1, 18.1 uncut; causal 8192 x 512 17.4 and 11.9.
 struct BwdCut { int cols, rows; };
 static BwdCut bwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int max_cols, int max_rows) {
   if (max_cols <= 1 && max_rows <= 1) return {1, 1};
@@ -804,33 +809,51 @@ static BwdCut bwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int 
   Side cols[9], rows[9];
   const int n_cols = sides(cols, max_cols, n_qtiles), n_rows = sides(rows, max_rows, n_ktiles);
   const float density = visible_share(n_qtiles, n_ktiles, causal), wk = (float)nbh * n_ktiles, wq = (float)nbh * n_qtiles;
-  const float tiles = density * wk * n_qtiles;
+  const float tiles = density * wk * n_qtiles, kFull = 2 * kCus;
   const int seen = causal && n_ktiles < n_qtiles ? n_ktiles : n_qtiles;    // the longest column
+  constexpr float kCol = 3.56f, kCol2 = 4.09f, kRow = 2.31f, kRow2 = 3.62f;
   BwdCut best = {1, 1};
   float best_us = INFINITY;
   for (int i = 0; i < n_cols; ++i)
     for (int j = 0; j < n_rows; ++j) {
       const Side &c = cols[i], &r = rows[j];
-      const float groups = (wk * c.n + wq * r.n) * density;
-      const int64_t lines = nbh * ((int64_t)n_ktiles * c.n + (int64_t)n_qtiles * r.n);
-      float us, tc, tr, least = tiles * 10.5f / (2 * kCus);                // the work of a CU, however long the walks
-      switch (bwd_form(lines, c.len + r.len, c.n + r.n, causal, n_qtiles, n_ktiles)) {
-        case 4: us = 5.9f + 2.7f * (lines / 128.f) * (lines / 128.f); tc = 1.42f; tr = 0.88f; break;
-        case 2: us = 9.8f; tc = 2.6f; tr = 1.7f; break;
+      const float n_col_lines = wk * c.n, lines = n_col_lines + wq * r.n;
+      const float col = c.len < seen ? c.len : seen, row = r.len;                          // the longest walks
+      float us, walks, least = (tiles * 9.31f + lines * 3.34f) / kFull;    // the work of a CU, however long the walks
+      switch (bwd_form((int64_t)lines, c.len + r.len, c.n + r.n, causal, n_qtiles, n_ktiles)) {
+        case 4: us = 7.06f + 1.95f * (lines / 128) * (lines / 128); walks = fmaxf(col * 1.23f, row * 0.715f); break;
+        case 2: us = 10.f; walks = fmaxf(col * 2.7f, row * 2.f); break;
         case kHalves: {
           const float shared = fminf((lines - 128) * (3.f / 128), 1.f);              // lines > 128
-          us = 5.9f; tc = 1.87f + 0.55f * shared; tr = 1.3f + 0.36f * shared; least = tiles * 5.9f / kCus;
+          us = 8.67f; walks = fmaxf(col * (1.64f + 0.094f * shared), row * (1.18f + 0.355f * shared)); least = 0.f;
           break;
         }
         default: {
-          const float shared = fminf(fmaxf((groups - kCus) / kCus, 0.f), 1.f);       // share of the workgroups with a neighbour
-          us = 6.7f; tc = 3.75f + 1.58f * shared; tr = 2.f + 1.6f * shared;
+          us = 6.7f;
+          if (!causal && lines <= kFull) {
+            const float a = col * kCol2, b = row * kRow2;
+            walks = lines <= kCus ? fmaxf(col * kCol, row * kRow) : b > a ? a + (row - a / kRow2) * kRow : b + (col - b / kCol2) * kCol;
+            if (n_col_lines > kCus) walks = fmaxf(walks, a);
+            break;
+          }
+          const float shared = fmaxf((lines * density - kCus) / kCus, 0.f);          // share of the workgroups with a neighbour
+          const float tc = shared > 0.f ? kCol2 : kCol, tr = kRow + (kRow2 - kRow) * fminf(1.49f * shared, 1.f);
+          const float a = col * tc, b = row * tr, over = lines - kFull, first_rows = kFull - n_col_lines;
+          walks = fmaxf(a, b);
+          if (over <= 0) break;
+          float from;                                                        // where the last rows begin
+          if (first_rows <= 0)                  from = (0.6f * ceilf(over / kFull) + 0.4f * over / kFull) * (c.len * density * tc + 12.2f);
+          else if (over <= first_rows && b < a) from = 0.69f * b + 12.2f;
+          else                                  from = over <= fmaxf(n_col_lines, first_rows) ? 0.8f * fminf(a, b) + 12.2f : walks + 12.2f;
+          if (!causal && lines <= 3 * kCus && r.len >= c.len) from *= 0.48f;
+          if (causal && first_rows > 0) from *= fminf(0.03f + 4.f * over / kFull, 1.f);
+          walks = fmaxf(walks, from + kRow2 * (causal ? fmaxf(row - 0.16f * n_qtiles, 0.15f * row) : row));
         }
       }
-      us += fmaxf(fmaxf((c.len < seen ? c.len : seen) * tc, r.len * tr), least);
+      us += fmaxf(walks, least);
       const float mb = ((c.n > 1 ? 2.f * c.n * wk : 0.f) + (r.n > 1 ? r.n * wq : 0.f)) * (kTile * kHeadDim * 4 / 1e6f), full = fminf(mb / 8, 2.f);
-      if (mb > 0.f) us = (us + 2.7f) * 1.02f + (c.n > 1 ? 0.5f : 0.f) + mb / 4.4f + 0.66f * full * full;
-      if (us < 0.99f * best_us) { best_us = us; best = {c.parts, r.parts}; }         // more parts for a gain, not for a tie
+      if (mb > 0.f) us = (us + 1.96f) * 1.035f + (c.n > 1 ? 0.7f : 0.f) + (c.n > 1 && r.n > 1 ? 0.58f : 0.f) + mb / 4.34f + 0.31f * full * full;
+      if (us < 0.995f * best_us) { best_us = us; best = {c.parts, r.parts}; }         // more parts for a gain, not for a tie
     }
   return best;
 }
