@@ -74,6 +74,10 @@ def test_around_the_bounds(sq, sk, nh, causal):
     (1024, 1024, 12, True), (1024, 1024, 13, True),              # 192 and 208 uneven ones: four groups, half lines
     (1536, 1536, 10, True),                                      # 240 that average six tiles: four groups
     (512, 512, 40, True), (512, 512, 41, True),                  # 320 and 328
+    (512, 512, 48, True), (512, 512, 49, True),                  # 384 and 392 that average four tiles
+    (640, 640, 51, True), (640, 640, 52, True),                  # 510 and 520 that average five
+    (512, 640, 35, True), (512, 640, 36, True),                  # 315 and 324 with more keys than queries
+    (384, 384, 50, True), (256, 256, 65, True),                  # 300 of three tiles at most; 260 of two: one group
     (128, 128, 130, True), (256, 256, 70, True),                 # 260 of one tile, 280 of one or two
     (512, 128, 50, True), (128, 640, 42, False),                 # empty walks on half lines; odd walks of one and five
     (128, 256, 43, False), (256, 128, 44, True),                 # 86 and 43, 44 and 88 lines a side: the last 8 of a side not full

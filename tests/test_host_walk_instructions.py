@@ -65,4 +65,4 @@ def test_no_scalars_in_vector_lanes(assembly, backward_assembly):
 
 def test_no_vector_registers_spilled_in_the_backward(backward_assembly):
     spills = _spills(backward_assembly, "vgpr")
-    assert len(spills) == 7 and not any(spills.values()), spills
+    assert len(spills) == 6 and not any(spills.values()), spills

@@ -274,7 +274,7 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& given, uint32_t lds_b
   const int group = S::kCount == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * S::kWaves));
   const uint32_t lds_base = lds_block + group * S::kBytes;
   int pos, bh;
-  map_block<kForm == kHalves>(block, p.cols.map, pos, bh);
+  map_block<S::kLines == 2>(block, p.cols.map, pos, bh);
   const int sub = pos & (S::kLines - 1);         // which half of the tile's keys
   pos >>= S::kLines - 1;
   const int b = quotient(bh, p.by_heads), h = bh - b * p.n_heads;
@@ -516,7 +516,7 @@ __device__ __forceinline__ void dq_walk(const BwdParams& given, uint32_t lds_blo
   const int group = S::kCount == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * S::kWaves));
   const uint32_t lds_base = lds_block + group * S::kBytes;
   int pos, bh;
-  map_block<kForm == kHalves>(block, p.rows.map, pos, bh);
+  map_block<S::kLines == 2>(block, p.rows.map, pos, bh);
   const int sub = pos & (S::kLines - 1);         // which half of the tile's queries
   pos >>= S::kLines - 1;
   const int b = quotient(bh, p.by_heads), h = bh - b * p.n_heads;
@@ -721,24 +721,28 @@ static void place(BwdParams& p, int lines) {
   p.rows.by_lines = make_div(p.n_qtiles);
 }
 static unsigned row_blocks(const BwdParams& p) { return (unsigned)(p.batch * p.n_heads * p.n_qtiles * p.rows.n_parts); }
-// The form (see Groups) for n lines of 128 rows on both sides of a dense rectangle together (parts counted), as in the forward:
-//  - four groups while half lines leave a CU one workgroup at most (8 heads of 1024: 34 us with one group, 31 with two, 24
-//    with four).  Of an uncut causal rectangle, whose lines differ in length, up to 256 lines that average four tiles (8
-//    heads of 2048: 54 us with two, 44 with four), beyond 192 that average six (16 of 1024: 25.2, in halves 23.8).
-//  - half lines of two groups up to 256 lines, and up to 320 of an uncut causal rectangle: the columns' half lines, which take longer,
-//    share the CUs with the rows', and the two workgroups of a CU are in different phases of their steps.  Against two groups
-//    on whole lines, which fill a CU with one workgroup each: 32 heads of 512 21.1 -> 19.5 us, causal 18.1 -> 15.6; 40 of 256
-//    14.5 -> 11.5; 16 of 1024 32.4 -> 30.4; causal 20 of 1024, 320 lines, 37.2 -> 29.0 against one group.  Beyond, and where lines
-//    average one tile (causal 150 of 128: 14.1, in halves 17.5), whole lines of one group fill the device as well and copy half as
-//    much (40 heads of 512: 25.2, in halves 28.7).
-//  - two groups for an uncut causal rectangle of up to 512 lines that average eight tiles (8 of 4096: 140 us with one, 132 with two).
-// Tile lists run with one, as in the forward.
+// The form (see Groups) for n lines of 128 rows on both sides of a dense rectangle together (parts counted):
+//  - four groups while half lines leave a CU one workgroup at most (8 heads of 1024: 34 us with one group, 24
+//    with four).  Of an uncut causal rectangle, whose lines differ in length, up to 192 lines that average four tiles (8
+//    heads of 2048: 54 us with one, 44 with four) and up to 256 that average six (16 of 1024: 25.2, in halves 23.8).
+//  - half lines of two groups up to 256 lines: the columns' half lines, which take longer, share the CUs with the rows', and the two
+//    workgroups of a CU are in different phases of their steps (32 heads of 512 23.1 us with one group, in halves 19.8; 42 of 384 21.0 and
+//    18.9).  Beyond, whole lines of one group fill the device as well and copy half as much (44 heads of 384, 264 lines: 21.1, in halves
+//    23.2; 22 of 768 34.3 and 35.7).
+//  - half lines of uncut causal rectangles, where they also even out the lines: up to 512 of them where no key lies beyond the first query and they average
+//    five tiles (30 heads of 1024, 480 lines: 42.3 and 37.4; 8 of 4096, 512: 137 and 112), up to 384 where they average three (36 of 512,
+//    288 lines: 21.5 and 18.4; 64 of 384 the same; 56 of 512, 448 lines, 23.5 and 24.9), up to 320 with more keys than
+//    queries, whose lines differ less (9 of 1280 x 2560, 270 lines, 19 % faster; 40 of 640 x 1280, 420, 5 % slower).  Lines of one or two tiles
+//    have nothing to even out (150 of 128: 14.0 and 15.4).
+// Tile lists run with one group, as in the forward.
 static int bwd_form(int64_t n, int64_t both_walks, int n_parts, bool dense_causal, int n_qtiles, int n_ktiles) {
   const bool uneven = dense_causal && n_parts == 2;
   if (both_walks >= 3 && 2 * n <= kCus) return 4;
   if (uneven && n <= kCus && both_walks >= (4 * n <= 3 * kCus ? 16 : 24)) return 4;
-  if (2 * n > kCus && (n <= kCus || (uneven && 4 * n <= 5 * kCus && both_walks >= 4))) return kHalves;
-  return uneven && n <= 2 * kCus && n_qtiles >= 16 && n_ktiles >= 16 ? 2 : 1;
+  if (2 * n > kCus && n <= kCus) return kHalves;
+  if (!uneven || both_walks < 6) return 1;
+  const int most = n_qtiles < n_ktiles ? 5 * kCus / 4 : both_walks < 10 ? 3 * kCus / 2 : 2 * kCus;
+  return n <= most ? kHalves : 1;
 }
 // `plain`: form 1.
 static int launch_bwd(BwdParams& p, bool plain, hipStream_t st) {
@@ -758,7 +762,6 @@ static int launch_bwd(BwdParams& p, bool plain, hipStream_t st) {
   p.rows_ahead = form == 1 && p.dense && !p.dense_causal && n > 2 * kCus && n <= 3 * kCus && p.rows.part_len >= p.cols.part_len;
   switch (form) {
     case 4: hipLaunchKernelGGL((bwd_kernel<4, true>), dim3(2 * n), dim3(512), 0, st, p); break;
-    case 2: hipLaunchKernelGGL((bwd_kernel<2, true>), dim3(n), dim3(512), 0, st, p); break;
     case kHalves: hipLaunchKernelGGL((bwd_kernel<kHalves, true>), dim3(2 * n), dim3(Groups<kHalves>::kThreads), 0, st, p); break;
     default:
       // Of the longest launches over tile lists each side runs as its own: the last workgroups of the columns and the first of the
@@ -822,7 +825,6 @@ static BwdCut bwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int 
       float us, walks, least = (tiles * 9.31f + lines * 3.34f) / kFull;    // the work of a CU, however long the walks
       switch (bwd_form((int64_t)lines, c.len + r.len, c.n + r.n, causal, n_qtiles, n_ktiles)) {
         case 4: us = 7.06f + 1.95f * (lines / 128) * (lines / 128); walks = fmaxf(col * 1.23f, row * 0.715f); break;
-        case 2: us = 10.f; walks = fmaxf(col * 2.7f, row * 2.f); break;
         case kHalves: {
           const float shared = fminf((lines - 128) * (3.f / 128), 1.f);              // lines > 128
           us = 8.67f; walks = fmaxf(col * (1.64f + 0.094f * shared), row * (1.18f + 0.355f * shared)); least = 0.f;

@@ -253,9 +253,9 @@ __device__ __forceinline__ void sum_blocks(f32x16& sum, const f32x16 (&acc)[4], 
 }
 // How a workgroup's waves share a line, by kForm:
 //   1       one group of four waves, the 128 rows of a tile, both halves of every tile of the other side one after the other;
-//   2       two groups of four waves on those rows, each takes a half of every tile;
+//   2       two groups of four waves on those rows, each takes a half of every tile (forward);
 //   4       four groups of two waves on half a tile's rows (64), each takes a quarter of every tile;
-//   kHalves two groups of two waves on half a tile's rows, each takes two quarters one after the other.
+//   kHalves two groups of two waves on half a tile's rows, each takes two quarters one after the other (backward).
 // Forms 2 and 4 fill a CU with one workgroup, 1 and kHalves with two.
 constexpr int kHalves = 3;
 template <int kForm>
