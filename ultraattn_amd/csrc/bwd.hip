@@ -63,6 +63,17 @@ __device__ __forceinline__ ParamsLate params_late() {
 // the two kinds of walk in kernels of their own).  The short walks of more groups start 2 % earlier with all parameters in flight before the branch.
 template <int kForm>
 __device__ __forceinline__ const BwdParams& params_of_walk(const BwdParams& given) { return kForm == 1 ? *(const BwdParams*)params_late() : given; }
+// Brings all parameters into the scalar cache while the first ones are on their way, for a walk that reads them behind a branch (short
+// walks of one group: 171 heads of 128, causal, 15.5 -> 14.9 us, 92 of 128 x 256 15.0 -> 14.3, 32 of 1024 53.2 -> 52.5).
+__device__ __forceinline__ void touch_params() {
+  constexpr int kLines = 9, kWords = sizeof(BwdParams) / 4;
+  static_assert(16 * (kLines - 1) < kWords && kWords <= 16 * kLines, "one word of every 64 bytes");
+  const auto* p = (const __attribute__((address_space(4))) int*)__builtin_amdgcn_kernarg_segment_ptr();
+  int x[kLines];
+#pragma unroll
+  for (int i = 0; i < kLines; ++i) x[i] = p[16 * i];
+  asm volatile("" :: "s"(x[0]), "s"(x[1]), "s"(x[2]), "s"(x[3]), "s"(x[4]), "s"(x[5]), "s"(x[6]), "s"(x[7]), "s"(x[8]));
+}
 // 32 output rows of a wave: in the caller's strided bf16 tensor, or in part `part` of the fp32 partials.
 __device__ __forceinline__ void store_result(const __attribute__((address_space(4))) BwdSide* p, bf16* out, int64_t os_b, int64_t os_s,
                                              int64_t os_h, int n_heads, int part, int b, int64_t row0, int h, int64_t seq,
@@ -666,6 +677,7 @@ template <int kForm, bool kDense>
 __global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void bwd_kernel(const BwdParams p) {
   __shared__ __attribute__((aligned(1024))) unsigned char smem[Stages<kForm>::kCount * Stages<kForm>::kBytes];
   const uint32_t lds_base = (uint32_t)(uintptr_t)(UA_LDS unsigned char*)smem;
+  if (kForm == 1) touch_params();
   if ((int)blockIdx.x < p.n_col_blocks) dkdv_walk<kForm, kDense>(p, lds_base, blockIdx.x);
   else                                  dq_walk<kForm, kDense>(p, lds_base, blockIdx.x - p.n_col_blocks);
 }
