@@ -520,6 +520,7 @@ __device__ __forceinline__ void dq_block(const PairAddr& ad, const bf16x8 (&qf)[
 template <int kForm, bool kDense>
 __device__ __forceinline__ void dq_walk(const BwdParams& given, uint32_t lds_block, int block) {
   const BwdParams& p = params_of_walk<kForm>(given);
+  static_assert(kDense || kForm == 1, "lists run with one group");
   if (kForm == 1 && kDense && p.rows_ahead) __builtin_amdgcn_s_setprio(1);
   using S = Stages<kForm>;
   const int tid = threadIdx.x % (64 * S::kWaves), lane = tid & 63, l32 = lane & 31;
@@ -606,7 +607,8 @@ __device__ __forceinline__ void dq_walk(const BwdParams& given, uint32_t lds_blo
       if (!walk.has(e + 1)) fetch(e + 1);
       ent_next = walk.at(min(e + 1, e1 - 1));
     };
-    if (S::kSteps == 1) look_ahead();
+    // (of a list beside the first block, which one group always sees; a group of several may see none of its blocks)
+    if (kDense) look_ahead();
     if (!kFirst) in.tile(walk.tile(ent_next), e + 1 < e1);
     wait_vmem_all();
     __syncthreads();            // this stage has landed; everyone is done with the other one, which the copies now fill
@@ -619,7 +621,7 @@ __device__ __forceinline__ void dq_walk(const BwdParams& given, uint32_t lds_blo
       if (!causal || q_block >= nb + kMb)
         dq_block<kOff + kMb * kBlockPitch, S::kPitch, kCopies>(ad, qf, dof, nd, dq, p.scale_log2, lse2, causal && q_block == nb + kMb,
                                                                [&](int n) { in.template copy<kStage ^ 1>(kMb * kCopies + n, part_next); },
-                                                               [&]() { if (kFirst && kMb == 0) look_ahead(); });
+                                                               [&]() { if (!kDense && kFirst && kMb == 0) look_ahead(); });
     };
     if (causal) {                                  // rare: the copies of the blocks that are left out
       for (int mb = 0; mb < kBlocks; ++mb)
