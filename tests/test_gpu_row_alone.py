@@ -68,8 +68,8 @@ def test_dense_without_workspace_equals_the_tile_list(lib, nq, nk, nh, causal):
         assert torch.equal(a, b)
 
 
-@pytest.mark.parametrize("heads", [128, 132])                # 32768 and 33792 lines: both sides of a backward in one launch and in two
-def test_backward_in_one_launch_and_in_two(heads):
+@pytest.mark.parametrize("heads", [128, 132])                # 32768 and 33792 lines
+def test_backward_of_32768_lines_and_more(heads):
     tiles = build_tile_list(masks.config_strided(16), block=512)
     q, k, v, do = _inputs(8192, 8192, heads, batch=2)
     o, lse = ops.bsa_fwd(q, k, v, tiles, SCALE)

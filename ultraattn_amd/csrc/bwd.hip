@@ -778,15 +778,8 @@ static int launch_bwd(BwdParams& p, bool plain, hipStream_t st) {
     case 4: hipLaunchKernelGGL((bwd_kernel<4, true>), dim3(2 * n), dim3(512), 0, st, p); break;
     case kHalves: hipLaunchKernelGGL((bwd_kernel<kHalves, true>), dim3(2 * n), dim3(Groups<kHalves>::kThreads), 0, st, p); break;
     default:
-      // Of the longest launches over tile lists each side runs as its own: the last workgroups of the columns and the first of the
-      // rows have little to share there, and the kernel of both keeps more of its scalars in vector lanes (32 heads of 128k, 65536
-      // lines, both in one launch and in two: strided mask 60.3 and 58.2 ms, global and local 57.0 and 55.7; 16384 lines of
-      // five masks within 1 % either way; strided 8k, 1024 lines, 214 and 232 us; dense, 4096 lines, 1 % faster in one).
-      if (!p.dense && n > 128 * kCus) {
-        hipLaunchKernelGGL(dkdv_kernel, dim3(col_blocks(p)), dim3(256), 0, st, p);
-        hipLaunchKernelGGL(dq_kernel, dim3(row_blocks(p)), dim3(256), 0, st, p);
-        break;
-      }
+      // (both sides in one launch at every length: against a launch for each 1-2 % faster at 4096 lines, above that within
+      // 1 % either way, strided mask of 128k, 65536 lines, 57.9 and 58.1 ms, of 64k, 32768 lines, 17.10 and 16.99)
       if (p.dense) hipLaunchKernelGGL((bwd_kernel<1, true>), dim3(n), dim3(256), 0, st, p);
       else         hipLaunchKernelGGL((bwd_kernel<1, false>), dim3(n), dim3(256), 0, st, p);
   }
