@@ -25,9 +25,9 @@
  *    rows sharing K/V tiles run together.
  *    `nnz` is the number of entries of col_idx/flag (row_idx/cflag): the kernels clamp every
  *    list bound to it, and only an empty list (nnz = 0) may pass NULL for those arrays.
- *    flag / cflag are read one aligned 32-bit word at a time: they must start on a 4-byte boundary
- *    (else UA_ERR_ALIGN) and be readable up to the next multiple of 4 bytes after entry nnz-1, i.e.
- *    allocate (nnz + 3) / 4 * 4 bytes; the padding bytes are never interpreted.
+ *    flag / cflag must start on a 4-byte boundary (else UA_ERR_ALIGN) and be readable up to the next
+ *    multiple of 4 bytes after entry nnz-1, i.e. allocate (nnz + 3) / 4 * 4 bytes; the padding bytes
+ *    are never interpreted (the kernels here read single bytes; the rule leaves them free to read words).
  *  - Every function returns 0 (UA_OK) or a negative UA_ERR_* code; ua_strerror() names it.
  *    No exceptions cross this boundary and nothing aborts.
  *  - Functions may be called from several host threads on different streams.  The only state

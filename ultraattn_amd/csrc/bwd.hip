@@ -714,7 +714,7 @@ static int fill_common(BwdParams& p, const void* q, const void* k, const void* v
 static int fill_side(BwdSide& s, int nnz, const int32_t* ptr, const int32_t* idx, const uint8_t* flag, const int32_t* order, void* out0,
                      const int64_t* o0s, void* out1, const int64_t* o1s, bool dense) {
   if (nnz > 0 && (!idx || !flag)) return UA_ERR_NULL;          // only an empty list may leave them out
-  if (flag && !aligned4(flag)) return UA_ERR_ALIGN;            // read one aligned 32-bit word at a time
+  if (flag && !aligned4(flag)) return UA_ERR_ALIGN;            // (a rule of the interface: whole words, so that a reader may take four at once)
   if (!out0 || !o0s || (o1s && !out1) || (!dense && (!ptr || !order))) return UA_ERR_NULL;
   if (!aligned16(out0) || !strides_ok(o0s) || (o1s && (!aligned16(out1) || !strides_ok(o1s)))) return UA_ERR_ALIGN;
   s.ptr = ptr; s.idx = idx; s.flag = flag; s.order = order;

@@ -505,7 +505,7 @@ extern "C" int ua_bsa_fwd(const void* q, const void* k, const void* v, void* o, 
   if (!row_ptr || !q_order) return UA_ERR_NULL;
   if (nnz < 0) return UA_ERR_SHAPE;
   if (nnz > 0 && (!col_idx || !flag)) return UA_ERR_NULL;      // only an empty list may leave them out
-  if (flag && !aligned4(flag)) return UA_ERR_ALIGN;            // read one aligned 32-bit word at a time
+  if (flag && !aligned4(flag)) return UA_ERR_ALIGN;            // (a rule of the interface: whole words, so that a reader may take four at once)
   FwdParams p;
   if (int rc = fwd_common(p, q, k, v, o, lse, batch, n_heads, n_qtiles, n_ktiles, head_dim, q_strides, k_strides,
                           v_strides, o_strides, softmax_scale)) return rc;

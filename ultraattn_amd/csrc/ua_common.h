@@ -297,21 +297,10 @@ struct Walk {
 };
 
 __device__ __forceinline__ void wait_vmem_all() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-// At the top of a rare wave-uniform branch: keeps it a branch (its body is not turned into selects), and what
-// the body computes from x stays in it.  Hoisted out of the walk, the comparisons of a masked tile take two
-// scalar registers each, and the attention kernels then spill a hundred of them into vector lanes.
-__device__ __forceinline__ void keep_branch_local(int& x) { asm volatile("" : "+v"(x) :: "memory"); }
 
 // Wave-uniform reads of the (read-only) tile-list arrays through the scalar cache.
 __device__ __forceinline__ int32_t sload(const int32_t* p, int i) {
   return ((const __attribute__((address_space(4))) int32_t*)p)[i];
-}
-__device__ __forceinline__ int sload(const uint8_t* p, int i) {
-  // the scalar unit loads dwords: fetch the aligned word that holds byte i (the entry points
-  // require p on a 4-byte boundary and the array padded to a multiple of 4 bytes)
-  const uintptr_t a = reinterpret_cast<uintptr_t>(p) + (uintptr_t)i;
-  const uint32_t w = *reinterpret_cast<const __attribute__((address_space(4))) uint32_t*>(a & ~(uintptr_t)3);
-  return (w >> (8 * (a & 3))) & 0xff;
 }
 
 // Asynchronous global -> LDS copy (buffer_load_dwordx4 ... lds), 16 bytes per lane: the wave's
