@@ -29,3 +29,28 @@ def test_rectangles_that_stay_whole(lib):
     for nh, seqs in ((8, range(4224, 4993, 128)), (5, range(7808, 9473, 128)), (3, (4480, 5248))):
         for s in seqs:
             assert lib.ua_dense_workspace_used(1, nh, s, s, 0, 0) == 0, (nh, s)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nh,sq,sk", [(10, 1664, 6656), (24, 768, 2944), (48, 768, 2944), (43, 384, 2048), (65, 256, 2048), (9, 2432, 4608)])
+def test_causal_rectangles_in_two_rounds_are_cut_and_rounded_once(lib, nh, sq, sk):
+    """129 to 383 long causal lines: 130 and 144 of four groups in two rounds, 288 of two; then 129 and 130 short ones; 171 whose last
+    part the first rows do not reach."""
+    g = torch.Generator(device=DEV).manual_seed(sk)
+    q, k, v = (torch.randn(1, n, nh, 128, device=DEV, generator=g).to(torch.bfloat16) for n in (sq, sk, sk))
+    rows = nh * sq
+    assert lib.ua_dense_workspace_used(1, nh, sq, sk, 1, 0) >= 2 * rows * (128 * 4 + 4)          # two parts or more, fp32
+    assert lib.ua_dense_workspace_bytes(1, nh, sq, sk, 0) >= lib.ua_dense_workspace_used(1, nh, sq, sk, 1, 0)
+    got = _flash_attn_forward(q, k, v, 0.0, SCALE, True)
+    whole = dense_unsplit(lib, q, k, v, q, True)
+    hidden = torch.ones(sq, sk, dtype=torch.bool, device=DEV).triu(sk - sq + 1)
+    for h in (0, nh - 1):
+        s = ((q[0, :, h].double() @ k[0, :, h].double().T) * SCALE).masked_fill(hidden, -torch.inf)
+        want, lse = torch.softmax(s, -1) @ v[0, :, h].double(), torch.logsumexp(s, -1)
+        err, err_whole = ((x[0][0, :, h].double() - want).norm().item() for x in (got, whole))
+        assert err <= 1.02 * err_whole, (h, err / err_whole)
+        assert ((lse_of(got)[0, h] - lse).abs() / lse.abs()).max().item() <= 1e-5
+
+
+def lse_of(result):
+    return next(x for x in result if torch.is_tensor(x) and x.dtype == torch.float32 and x.dim() == 3)

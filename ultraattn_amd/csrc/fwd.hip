@@ -11,6 +11,7 @@
 // lane (mirrored in lane ^ 32): the row max needs a single cross-half exchange, the rescale of
 // O^T is lane local, and S^T's accumulator registers are, after exp2 and bf16 packing, exactly
 // the B operand of the second product.
+#include <algorithm>
 #include <type_traits>
 #include "ua_common.h"
 
@@ -29,9 +30,9 @@ struct FwdParams {
   // dense_causal [0, qt + diag_off] with the last one causal; longest rows first.  The first n_whole query tiles (all
   // if nothing is cut) are walked whole; the key range of the others is cut into n_parts parts of part_len tiles, and
   // part i leaves its partial (O, LSE), contiguous over those n_qtiles - n_whole tiles, at part_o + i * o_part and
-  // part_lse + i * lse_part (elements).  Beside whole tiles the partial O is fp32, so that every row of a result is
-  // rounded to bf16 once; where everything is cut it is bf16.
-  int dense, dense_causal, diag_off, n_whole, n_parts, part_len;
+  // part_lse + i * lse_part (elements).  The partial O is fp32 (part_f32) beside whole tiles, so that every row of a result is
+  // rounded to bf16 once; where everything is cut it is bf16 or fp32, see fwd_cut.
+  int dense, dense_causal, diag_off, n_whole, n_parts, part_len, part_f32;
   void* part_o; float* part_lse;
   int64_t o_part, lse_part;
 };
@@ -334,7 +335,7 @@ __global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void fwd_kernel(const F
   if constexpr (kForm == 1) {
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
     const uint32_t turn = lds_at((wave < 2 ? kA : vA) + (wave & 1) * kWaveRowsBytes);
-    if (part >= 0 && p.n_whole > 0) store_rows_f32(static_cast<float*>(p.part_o) + part_at, o_stride, oacc, inv, turn);
+    if (part >= 0 && p.part_f32)    store_rows_f32(static_cast<float*>(p.part_o) + part_at, o_stride, oacc, inv, turn);
     else                            store_rows_bf16(orow, o_stride, oacc, inv, turn);
   } else {
     // the groups exchange their rows' max, sum and O.  Area x of the stages' LDS belongs to group x % kForm of wave x / kForm.
@@ -401,7 +402,7 @@ static int fwd_common(FwdParams& p, const void* q, const void* k, const void* v,
   p.os = {o_strides[0], o_strides[1], o_strides[2]};
   p.scale_log2 = softmax_scale * kLog2e;
   p.dense = 0; p.dense_causal = 0; p.diag_off = 0; p.n_whole = n_qtiles; p.n_parts = 1; p.part_len = n_ktiles;
-  p.part_o = nullptr; p.part_lse = nullptr; p.o_part = 0; p.lse_part = 0;
+  p.part_o = nullptr; p.part_lse = nullptr; p.o_part = 0; p.lse_part = 0; p.part_f32 = 0;
   return check_device();
 }
 
@@ -447,7 +448,7 @@ static int fwd_launch(FwdParams& p, bool plain, hipStream_t st) {
 
 // How many parts the walks of a dense forward are cut into, at most max_parts (what the workspace holds).  A cut
 // gives a small rectangle enough workgroups and costs the partials' way through memory, a merge, and a second rounding of
-// every row: the partial O is bf16, as the workspace's size has it (error against fp64 2.33e-3 whole and 2.85e-3 cut at 8 heads of 4480, and
+// every row: the partial O is bf16 (error against fp64 2.33e-3 whole and 2.85e-3 cut at 8 heads of 4480, and
 // as much in 11 parts as in two).  Two estimates of the launches' time in microseconds therefore have to agree on a cut:
 //  - the first, fitted to 47 shapes of 1 to 32 heads and 128 to 8192 tokens, says which rectangles have enough to gain (5 heads of 8192,
 //    200 us whole and 179 cut in two, do not);
@@ -455,7 +456,16 @@ static int fwd_launch(FwdParams& p, bool plain, hipStream_t st) {
 //    of parts, or none: 16 heads, causal 640 x 1920, 21.6 us cut in three, 19.5 whole; 2 x 3 causal 6784 94.9 and 89.8.
 // Terms: start, loading Q, storing and the end; a tile, and one where two workgroups share the CU; the merge, and the partials' bytes.
 // 1024 x 4096, one head: 34 us uncut, 12 cut in 11.
-static int fwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int max_parts) {
+//
+// Causal rectangles of more keys than queries whose whole walks run in a second round (more than 128 lines in four groups, more than 256 in
+// two) are cut by an estimate of their own: the second round begins when the shortest rows of the first are through, and all rows
+// are long.  Their partial O is fp32, so that every row is rounded once (bf16 partials take 2 to 4 us less).  Fitted to 270 rectangles of
+// 129 to 383 lines; over 410 others 9 % less time than whole: 10 heads of 1664 x 6144 87.8 -> 56.4 us, 3 of 7296 x 29440 430 -> 282.
+struct FwdCut {
+  int parts;
+  bool f32;
+};
+static FwdCut fwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int max_parts) {
   const float lines = (float)nbh * n_qtiles;
   auto share = [](float groups) { return fminf(fmaxf((groups - kCus) / kCus, 0.f), 1.f); };        // of the workgroups with a neighbour
   auto first = [&](int parts) {
@@ -486,7 +496,19 @@ static int fwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int max
     }
     return best;
   };
-  return least(first) > 1 ? least(second) : 1;
+  if (const int parts = least(first) > 1 ? least(second) : 1; parts > 1) return {parts, false};
+  const int whole = fwd_groups(nbh * n_qtiles, n_ktiles, 1, causal), round = whole == 4 ? kCus / 2 : kCus;
+  if (!causal || n_ktiles <= n_qtiles || whole == 1 || lines <= round) return {1, false};
+  const float shortest = n_ktiles - n_qtiles * round / lines;                  // row of the first round
+  auto rounded_once = [&](int parts) {
+    if (parts == 1) return 0.95f * (5.f + (whole == 4 ? fmaxf(1.25f * n_ktiles, 2.5f * shortest) : fmaxf(1.65f * n_ktiles, 3.6f * shortest)));
+    const int len = (n_ktiles + parts - 1) / parts, made = (n_ktiles + len - 1) / len;
+    if (fwd_groups(nbh * n_qtiles * made, len, made, causal) != 1) return INFINITY;          // (several groups leave bf16)
+    const float density = visible_share(n_qtiles, n_ktiles, causal), groups = lines * made;
+    return 6.65f + groups * (kTile * kHeadDim * 4) / 2.5e6f + fmaxf(len * (2.4f + 1.15f * share(groups * density)), density * lines * n_ktiles * 3.66f / (2 * kCus));
+  };
+  const int parts = least(rounded_once);
+  return {parts, parts > 1};
 }
 
 static bool contiguous_bshd(const int64_t* st, int seqlen, int n_heads) {
@@ -522,17 +544,20 @@ namespace ua {
 // (2560 x 2048, 32 heads, 128 lines over: 91.2 us, cut 89.1; 3072 x 2048, 256 over: 97, cut in two 103, not done).  bf16
 // partials took up to 3 us less at the first shape and gave the rows of the last wave a second rounding, an error 20 % larger
 // than their neighbours'.  Causal rows balance themselves.
-struct Tail { int tiles, parts; };
-static Tail fwd_tail(int64_t nbh, int n_qtiles, int n_ktiles) {
+struct Cut {
+  int tiles, parts;
+  bool f32;                                // partial O
+};
+static Cut fwd_tail(int64_t nbh, int n_qtiles, int n_ktiles) {
   constexpr int kRound = 2 * kCus;
   const int64_t lines = nbh * n_qtiles, rounds = lines / kRound;
-  if (rounds == 0 || lines % kRound == 0 || lines % kRound > kCus) return {0, 1};
+  if (rounds == 0 || lines % kRound == 0 || lines % kRound > kCus) return {0, 1, false};
   const int tail = n_qtiles - (int)(rounds * kRound / nbh);
   const int64_t cut = nbh * tail;
   const int64_t most = n_ktiles / 2 < UA_MAX_PARTS ? n_ktiles / 2 : UA_MAX_PARTS, parts = kRound / cut < most ? kRound / cut : most;
-  if (tail >= n_qtiles || parts < 2) return {0, 1};
+  if (tail >= n_qtiles || parts < 2) return {0, 1, false};
   const float us = 3.7f * cut * n_ktiles / kRound + 4.f + 2.4f + cut * parts * (kTile * kHeadDim * 4) / 2.5e6f;
-  return us < 2.2f * n_ktiles ? Tail{tail, (int)parts} : Tail{0, 1};
+  return us < 2.2f * n_ktiles ? Cut{tail, (int)parts, true} : Cut{0, 1, false};
 }
 // One part's share of the workspace for n_tiles cut query tiles.
 struct PartBytes {
@@ -544,17 +569,17 @@ static PartBytes part_bytes(int batch, int n_heads, int n_tiles, bool f32) {
   return {align256(rows * kHeadDim * (f32 ? 4 : 2)), align256(rows * 4)};
 }
 // Query tiles at the end that are cut, and into how many parts.
-static Tail dense_cut(int batch, int n_heads, int n_qtiles, int n_ktiles, bool causal) {
+static Cut dense_cut(int batch, int n_heads, int n_qtiles, int n_ktiles, bool causal) {
   const int64_t nbh = (int64_t)batch * n_heads;
   const int max_parts = dense_split(batch, n_heads, n_qtiles, n_ktiles).fwd_parts;
-  if (max_parts == 1) return causal ? Tail{0, 1} : fwd_tail(nbh, n_qtiles, n_ktiles);
-  const int parts = n_heads > kMaxHeadsLds ? 1 : fwd_cut(nbh, n_qtiles, n_ktiles, causal, max_parts);       // (more heads: not merged)
-  return {parts > 1 ? n_qtiles : 0, parts};
+  if (max_parts == 1) return causal ? Cut{0, 1, false} : fwd_tail(nbh, n_qtiles, n_ktiles);
+  const FwdCut cut = n_heads > kMaxHeadsLds ? FwdCut{1, false} : fwd_cut(nbh, n_qtiles, n_ktiles, causal, max_parts);       // (more heads: not merged)
+  return {cut.parts > 1 ? n_qtiles : 0, cut.parts, cut.f32};
 }
 
 static int64_t fwd_workspace_used(int batch, int n_heads, int n_qtiles, int n_ktiles, bool causal) {
-  const Tail cut = dense_cut(batch, n_heads, n_qtiles, n_ktiles, causal);
-  return cut.tiles ? cut.parts * part_bytes(batch, n_heads, cut.tiles, cut.tiles < n_qtiles).total() : 0;
+  const Cut cut = dense_cut(batch, n_heads, n_qtiles, n_ktiles, causal);
+  return cut.tiles ? cut.parts * part_bytes(batch, n_heads, cut.tiles, cut.f32).total() : 0;
 }
 
 }  // namespace ua
@@ -571,8 +596,8 @@ extern "C" int64_t ua_dense_workspace_bytes(int batch, int n_heads, int seqlen_q
   const int n_qtiles = seqlen_q / kTile, n_ktiles = seqlen_k / kTile;
   const DenseSplit d = dense_split(batch, n_heads, n_qtiles, n_ktiles);
   if (backward) return d.bwd_total;
-  if (d.fwd_parts > 1) return d.fwd_total;
-  const Tail t = fwd_tail((int64_t)batch * n_heads, n_qtiles, n_ktiles);
+  if (d.fwd_parts > 1) return std::max(d.fwd_total, fwd_workspace_used(batch, n_heads, n_qtiles, n_ktiles, true));       // (causal ones may leave fp32)
+  const Cut t = fwd_tail((int64_t)batch * n_heads, n_qtiles, n_ktiles);
   return t.tiles ? t.parts * part_bytes(batch, n_heads, t.tiles, true).total() : 0;
 }
 
@@ -590,11 +615,10 @@ extern "C" int ua_dense_fwd(const void* q, const void* k, const void* v, void* o
   p.dense = 1; p.dense_causal = causal != 0; p.diag_off = n_ktiles - n_qtiles;
   hipStream_t st = (hipStream_t)stream;
   if (!workspace) return fwd_launch(p, true, st);
-  const Tail cut = dense_cut(batch, n_heads, n_qtiles, n_ktiles, p.dense_causal);
+  const Cut cut = dense_cut(batch, n_heads, n_qtiles, n_ktiles, p.dense_causal);
   if (cut.tiles == 0) return fwd_launch(p, false, st);
   // cutting needs the caller's workspace and a contiguous output for the merge
-  const bool beside_whole = cut.tiles < n_qtiles;
-  const PartBytes d = part_bytes(batch, n_heads, cut.tiles, beside_whole);
+  const PartBytes d = part_bytes(batch, n_heads, cut.tiles, cut.f32);
   const int64_t need = cut.parts * d.total();
   if (!aligned16(workspace) || workspace_bytes < need || !contiguous_bshd(o_strides, seqlen_q, n_heads)) return fwd_launch(p, false, st);
   p.n_whole = n_qtiles - cut.tiles;
@@ -602,9 +626,9 @@ extern "C" int ua_dense_fwd(const void* q, const void* k, const void* v, void* o
   p.n_parts = (n_ktiles + p.part_len - 1) / p.part_len;
   p.part_o = workspace;
   p.part_lse = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + p.n_parts * d.o);
-  p.o_part = d.o / (beside_whole ? 4 : 2); p.lse_part = d.lse / 4;
+  p.o_part = d.o / (cut.f32 ? 4 : 2); p.lse_part = d.lse / 4; p.part_f32 = cut.f32;
   if (int rc = fwd_launch(p, false, st)) return rc;
-  if (beside_whole) {
+  if (cut.f32) {
     const int64_t first = (int64_t)p.n_whole * kTile;
     return merge_f32_rows((const float*)p.part_o, p.o_part, p.part_lse, p.lse_part, p.n_parts, p.o + first * n_heads * kHeadDim, lse + first, seqlen_q,
                           batch, cut.tiles * kTile, n_heads, st);
