@@ -93,3 +93,15 @@ def test_half_lines(sq, sk, nh, causal):
 def test_two_to_three_workgroups_per_cu(sq, sk, nh):
     """512 and 520 lines, 768 with longer rows, 630 with longer columns, 512 of one tile: where the rows' wavefronts go first and where not."""
     test_around_the_bounds(sq, sk, nh, False)
+
+
+@pytest.mark.parametrize("sq,sk,nh", [
+    (896, 512, 12), (768, 640, 1), (896, 768, 1), (896, 896, 1),         # four groups of 132 lines; cuts of both sides in halves, of columns and of both in four
+    (128, 768, 1), (128, 1536, 20), (128, 1536, 40),                     # rows cut in halves: 7, 260 and 520 lines
+    (128, 2048, 6), (128, 2688, 24), (256, 2688, 32),                    # rows cut, one group: 102, 528 and 736
+    (1536, 128, 20), (128, 1280, 48), (512, 128, 48),                    # whole lines: 260 and 528 in halves, 240 short ones of one group
+    (640, 256, 109), (640, 256, 110), (512, 2048, 40),                   # 763 and 770, on both sides of the last bound; 800 with cut rows
+])
+def test_causal_plans(sq, sk, nh):
+    """Every form with every kind of cut that a causal backward takes."""
+    test_around_the_bounds(sq, sk, nh, True)

@@ -16,6 +16,7 @@
 //                Here a lane holds one query column, so lse and delta are per-lane scalars.
 //  P = exp2(scale*log2e*S - lse*log2e);  dS = P * (dP - delta);  dQ, dK are scaled by
 //  softmax_scale on output.
+#include <algorithm>
 #include <type_traits>
 #include "ua_common.h"
 
@@ -106,7 +107,7 @@ __device__ __forceinline__ void store_block(const __attribute__((address_space(4
 //   dV^T += dO^T P,  dK^T += Q^T dS                     16 MFMAs, Q and dO read through the transposing path
 // P and dS never leave the wave.  The accumulators of S and dP' start from the rows' statistics.
 //
-// Bound: matrix pipe at the clock the socket's power allows (70 % busy at 1.68 GHz).  192 of a wave's 256 registers
+// Bound: matrix pipe at the clock the socket's power allows (71 % busy at 1.68 GHz).  192 of a wave's 256 registers
 // hold K, V, dK and dV; two independent workgroups share a CU, so that one's exp2 and barriers hide behind
 // the other's MFMAs.  Against one workgroup of eight waves in two roles (S/dV and dP/dK, P handed over
 // through LDS): strided 128k, 32 heads 37.8 -> 33.5 ms, causal 32k 15.8 -> 13.7 ms (1.25-1.3 PFLOP/s of the four
@@ -735,33 +736,19 @@ static void place(BwdParams& p, int lines) {
   p.rows.by_lines = make_div(p.n_qtiles);
 }
 static unsigned row_blocks(const BwdParams& p) { return (unsigned)(p.batch * p.n_heads * p.n_qtiles * p.rows.n_parts); }
-// The form (see Groups) for n lines of 128 rows on both sides of a dense rectangle together (parts counted):
-//  - four groups while half lines leave a CU one workgroup at most (8 heads of 1024: 34 us with one group, 24
-//    with four).  Of an uncut causal rectangle, whose lines differ in length, up to 192 lines that average four tiles (8
-//    heads of 2048: 54 us with one, 44 with four) and up to 256 that average six (16 of 1024: 25.2, in halves 23.8).
+// The form (see Groups) for n lines of 128 rows on both sides of a rectangle that is not causal together (parts counted):
+//  - four groups while half lines leave a CU one workgroup at most (8 heads of 1024: 34 us with one group, 24 with four).
 //  - half lines of two groups up to 256 lines: the columns' half lines, which take longer, share the CUs with the rows', and the two
 //    workgroups of a CU are in different phases of their steps (32 heads of 512 23.1 us with one group, in halves 19.8; 42 of 384 21.0 and
 //    18.9).  Beyond, whole lines of one group fill the device as well and copy half as much (44 heads of 384, 264 lines: 21.1, in halves
 //    23.2; 22 of 768 34.3 and 35.7).
-//  - half lines of uncut causal rectangles, where they also even out the lines: up to 512 of them where no key lies beyond the first query and they average
-//    five tiles (30 heads of 1024, 480 lines: 42.3 and 37.4; 8 of 4096, 512: 137 and 112), up to 384 where they average three (36 of 512,
-//    288 lines: 21.5 and 18.4; 64 of 384 the same; 56 of 512, 448 lines, 23.5 and 24.9), up to 320 with more keys than
-//    queries, whose lines differ less (9 of 1280 x 2560, 270 lines, 19 % faster; 40 of 640 x 1280, 420, 5 % slower).  Lines of one or two tiles
-//    have nothing to even out (150 of 128: 14.0 and 15.4).
-// Tile lists run with one group, as in the forward.
-static int bwd_form(int64_t n, int64_t both_walks, int n_parts, bool dense_causal, int n_qtiles, int n_ktiles) {
-  const bool uneven = dense_causal && n_parts == 2;
+// A causal one's form is chosen with its cut, see bwd_plan.  Tile lists run with one group, as in the forward.
+static int bwd_form(int64_t n, int64_t both_walks) {
   if (both_walks >= 3 && 2 * n <= kCus) return 4;
-  if (uneven && n <= kCus && both_walks >= (4 * n <= 3 * kCus ? 16 : 24)) return 4;
-  if (2 * n > kCus && n <= kCus) return kHalves;
-  if (!uneven || both_walks < 6) return 1;
-  const int most = n_qtiles < n_ktiles ? 5 * kCus / 4 : both_walks < 10 ? 3 * kCus / 2 : 2 * kCus;
-  return n <= most ? kHalves : 1;
+  return 2 * n > kCus && n <= kCus ? kHalves : 1;
 }
-// `plain`: form 1.
-static int launch_bwd(BwdParams& p, bool plain, hipStream_t st) {
+static int launch_bwd(BwdParams& p, int form, hipStream_t st) {
   const unsigned n = col_blocks(p) + row_blocks(p);
-  const int form = plain ? 1 : bwd_form(n, p.cols.part_len + p.rows.part_len, p.cols.n_parts + p.rows.n_parts, p.dense_causal, p.n_qtiles, p.n_ktiles);
   const int lines = form > 2 ? 2 : 1;
   p.n_col_blocks = (int)col_blocks(p) * lines;
   place(p, lines);
@@ -786,89 +773,112 @@ static int launch_bwd(BwdParams& p, bool plain, hipStream_t st) {
   return launched();
 }
 
-// How many parts the two sides of a dense backward are cut into, at most what the workspace holds.  A cut gives a
-// small rectangle enough workgroups for the device and costs the partials' way through memory and a
-// second launch; which wins is decided by an estimate of the time in microseconds, fitted to all cuts of 1427 rectangles of 1
-// to 130 heads and 256 to 24000 tokens.  The cut it takes is 0.9 % slower than the best one on average, 72 times by more than 5 %, 22 % at
-// most; without what is said of launches beyond 256 and 512 lines 2.4 %, 255 times and 39 % (2 heads of 11136: 472 us cut
-// in 2 and 1, 409 whole, 389 in 2 and 2):
+// How many parts the two sides of a dense backward are cut into, at most what the workspace holds, and its form.  A cut gives a
+// small rectangle enough workgroups for the device and costs the partials' way through memory and a second launch; which wins is decided
+// by an estimate of the time in microseconds.
+// The sum of the partials takes 2, 0.7 more for columns, 1.3 for columns and rows, the partials 1 per 4.3 MB and 0.3 at 8 MB, 1.2 from 16 on.
+//
+// Not causal: fitted to all cuts of 1427 rectangles of 1 to 130 heads and 256 to 24000 tokens, causal ones among them:
 //  - a start and end (loading the resident rows, storing the results), longer as half lines fill the device, and the longest walks;
 //  - with one group per workgroup a tile takes 3.6 (column) or 2.3 (row), 4.1 or 3.6 where two workgroups share the CU.  The second
-//    workgroups of 257 to 512 even lines are the last of the rows, beside a column;
+//    workgroups of 257 to 512 lines are the last of the rows, beside a column;
 //  - beyond 512 the last rows begin when something else is through: a row beside a column if those are few and shorter, else a row or
-//    column, or a round of columns; sooner where the rows' wavefronts go first (see launch_bwd), and where a causal
-//    rectangle's short walks make room;
-//  - no less than all tiles and workgroups take on a full device;
-//  - the sum takes 2, 0.7 more for columns, 1.3 for columns and rows, the partials 1 per 4.3 MB and 0.3 at 8 MB, 1.2 from 16 on; a cut
-//    has to win by 3.5 %.
-// 1024 x 4096, one head: 34 us uncut, 20.7 cut in 1 and 3; 4 heads of 1024 19.9 cut in 2 and 1, 18.1 uncut; causal 8192 x 512 17.4 and 11.9.
-struct BwdCut { int cols, rows; };
-static BwdCut bwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int max_cols, int max_rows) {
-  if (max_cols <= 1 && max_rows <= 1) return {1, 1};
+//    column, or a round of columns; sooner where the rows' wavefronts go first (see launch_bwd);
+//  - no less than all tiles and workgroups take on a full device; a cut has to win by 3.5 %.
+// (2 heads of 11136: 472 us cut in 2 and 1, 409 whole, 389 in 2 and 2; 1024 x 4096, one head: 34 us uncut, 20.7 cut in 1 and 3; 4 heads of
+// 1024 19.9 cut in 2 and 1, 18.1 uncut.)
+//
+// Causal: lines differ in length and even out beyond one round of workgroups, less the more keys there are before the first query.  Every form is
+// estimated with every cut up to 768 lines, fitted to 5300 rectangles of 1 to 64 heads and 128 to 24000 tokens; of those kept apart from
+// the fit the plan taken is 1.5 % slower than the best one on average, 3 % of them by more than 10, 18 at most.  (One estimate for
+// both kinds and bounds of lines for the forms: 5.4 % on average, and half lines or four groups, whose second round it did not see, up
+// to 50 % slower than a cut where all lines are long: one head, 4992 x 19968, 222 us, cut 158; 5 of 1024 x 4096 57 and 44.)
+//  - a start and end, and the longest walk, whose tiles take longer the fuller the device is;
+//  - beyond one round all tiles and workgroups of a CU, and a share of the rows' mean length and of the longest beyond it at the end.
+struct BwdPlan { int cols, rows, form; };
+struct BwdWalk { int parts, n, len; };                                     // parts asked for and made, tiles of each
+struct BwdRates {
+  int form, slots;                           // workgroups that the device holds
+  float start, col, col_full, row, row_full, fullest, work, work_even, each, mean, mean_even, beyond;
+};
+static constexpr BwdRates kCausalRates[3] = {
+  {1, 2 * kCus, 5.52f, 3.344f, 0.288f, 2.055f, 0.132f, 2.f, 2.193f, -0.485f, 1.578f, -0.401f, 1.035f, 0.722f},
+  {kHalves, 2 * kCus, 5.46f, 1.785f, 0.187f, 1.128f, 0.077f, 2.f, 1.898f, -0.202f, 1.101f, -0.179f, 0.748f, 0.607f},
+  {4, kCus, 6.62f, 1.385f, 0.067f, 0.758f, 0.237f, 1.5f, 1.282f, -0.088f, 2.65f, -0.018f, 0.539f, 0.205f},
+};
+static float bwd_causal_us(const BwdRates& f, float nbh, int n_qtiles, int n_ktiles, float tiles, const BwdWalk& c, const BwdWalk& r) {
+  const float lines = nbh * (n_ktiles * c.n + n_qtiles * r.n), groups = (f.form == 1 ? 1 : 2) * lines, full = groups / kCus;
+  const float even = n_ktiles > n_qtiles ? (float)(n_ktiles - n_qtiles) / n_ktiles : 0.f;
+  const float col = f.col + f.col_full * fminf(full, f.fullest), row = f.row + f.row_full * fminf(full, f.fullest);
+  const float walk = fmaxf(std::min(c.len, n_ktiles) * col, r.len * row);                  // (the longest column has n_ktiles queries at most)
+  if (full <= 1.f) return f.start + walk;
+  const float mean = tiles / (nbh * n_qtiles * r.n);
+  const float work = (f.form == 1 ? 1 : 2) * tiles * (col + row) * (f.work + f.work_even * even) / f.slots + f.each * full +
+                     ((f.mean + f.mean_even * even) * mean + f.beyond * (r.len - mean)) * row;
+  const float longer = fmaxf(walk, work), ratio = fminf(walk, fmaxf(work, 0.f)) / longer, r2 = ratio * ratio, r4 = r2 * r2, r8 = r4 * r4;
+  return f.start + longer * sqrtf(sqrtf(sqrtf(sqrtf(1.f + r8 * r8))));
+}
+static float bwd_us(int form, float nbh, int n_qtiles, int n_ktiles, const BwdWalk& c, const BwdWalk& r) {
+  const float wk = nbh * n_ktiles, wq = nbh * n_qtiles, tiles = wk * n_qtiles, n_col_lines = wk * c.n, lines = n_col_lines + wq * r.n;
+  const float col = c.len, row = r.len, kFull = 2 * kCus, least = (tiles * 9.31f + lines * 3.34f) / kFull;         // the work of a CU
+  constexpr float kCol = 3.56f, kCol2 = 4.09f, kRow = 2.31f, kRow2 = 3.62f;
+  if (form == 4) return 7.06f + 1.95f * (lines / 128) * (lines / 128) + fmaxf(fmaxf(col * 1.23f, row * 0.715f), least);
+  if (form == kHalves) {
+    const float shared = fminf((lines - 128) * (3.f / 128), 1.f);                    // lines > 128
+    return 8.67f + fmaxf(col * (1.64f + 0.094f * shared), row * (1.18f + 0.355f * shared));
+  }
+  float walks;
+  const float a = col * kCol2, b = row * kRow2;
+  if (lines <= kFull) {
+    walks = lines <= kCus ? fmaxf(col * kCol, row * kRow) : b > a ? a + (row - a / kRow2) * kRow : b + (col - b / kCol2) * kCol;
+    if (n_col_lines > kCus) walks = fmaxf(walks, a);
+  } else {
+    const float over = lines - kFull, first_rows = kFull - n_col_lines;
+    float from;                                                              // where the last rows begin
+    if (first_rows <= 0)                  from = (0.6f * ceilf(over / kFull) + 0.4f * over / kFull) * (a + 12.2f);
+    else if (over <= first_rows && b < a) from = 0.69f * b + 12.2f;
+    else                                  from = over <= fmaxf(n_col_lines, first_rows) ? 0.8f * fminf(a, b) + 12.2f : fmaxf(a, b) + 12.2f;
+    if (lines <= 3 * kCus && r.len >= c.len) from *= 0.48f;
+    walks = fmaxf(fmaxf(a, b), from + b);
+  }
+  return 6.7f + fmaxf(walks, least);
+}
+static BwdPlan bwd_plan(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int max_cols, int max_rows) {
   static constexpr int kParts[] = {1, 2, 3, 4, 5, 6, 8, 12, 16};
-  struct Side { int parts, n, len; };                                      // asked for, made, tiles of each
-  auto sides = [](Side (&s)[9], int most, int list_len) {
+  auto sides = [](BwdWalk (&s)[9], int most, int list_len) {
     int n = 0;
     for (int parts : kParts)
-      if (parts <= most) {
+      if (parts <= most || parts == 1) {
         const int len = (list_len + parts - 1) / parts;
         s[n++] = {parts, (list_len + len - 1) / len, len};
       }
     return n;
   };
-  Side cols[9], rows[9];
+  BwdWalk cols[9], rows[9];
   const int n_cols = sides(cols, max_cols, n_qtiles), n_rows = sides(rows, max_rows, n_ktiles);
-  const float density = visible_share(n_qtiles, n_ktiles, causal), wk = (float)nbh * n_ktiles, wq = (float)nbh * n_qtiles;
-  const float tiles = density * wk * n_qtiles, kFull = 2 * kCus;
-  const int seen = causal && n_ktiles < n_qtiles ? n_ktiles : n_qtiles;    // the longest column
-  constexpr float kCol = 3.56f, kCol2 = 4.09f, kRow = 2.31f, kRow2 = 3.62f;
-  BwdCut best = {1, 1};
+  const int n_forms = causal && nbh * (n_ktiles + n_qtiles) <= 3 * kCus ? 3 : 1;
+  if (n_cols * n_rows * n_forms == 1) return {1, 1, causal ? 1 : bwd_form(nbh * ((int64_t)n_ktiles + n_qtiles), (int64_t)n_qtiles + n_ktiles)};
+  const float wk = (float)nbh * n_ktiles, wq = (float)nbh * n_qtiles, tiles = visible_share(n_qtiles, n_ktiles, causal) * wk * n_qtiles;
+  BwdPlan best = {1, 1, 1};
   float best_us = INFINITY;
   for (int i = 0; i < n_cols; ++i)
     for (int j = 0; j < n_rows; ++j) {
-      const Side &c = cols[i], &r = rows[j];
-      const float n_col_lines = wk * c.n, lines = n_col_lines + wq * r.n;
-      const float col = c.len < seen ? c.len : seen, row = r.len;                          // the longest walks
-      float us, walks, least = (tiles * 9.31f + lines * 3.34f) / kFull;    // the work of a CU, however long the walks
-      switch (bwd_form((int64_t)lines, c.len + r.len, c.n + r.n, causal, n_qtiles, n_ktiles)) {
-        case 4: us = 7.06f + 1.95f * (lines / 128) * (lines / 128); walks = fmaxf(col * 1.23f, row * 0.715f); break;
-        case kHalves: {
-          const float shared = fminf((lines - 128) * (3.f / 128), 1.f);              // lines > 128
-          us = 8.67f; walks = fmaxf(col * (1.64f + 0.094f * shared), row * (1.18f + 0.355f * shared)); least = 0.f;
-          break;
-        }
-        default: {
-          us = 6.7f;
-          if (!causal && lines <= kFull) {
-            const float a = col * kCol2, b = row * kRow2;
-            walks = lines <= kCus ? fmaxf(col * kCol, row * kRow) : b > a ? a + (row - a / kRow2) * kRow : b + (col - b / kCol2) * kCol;
-            if (n_col_lines > kCus) walks = fmaxf(walks, a);
-            break;
-          }
-          const float shared = fmaxf((lines * density - kCus) / kCus, 0.f);          // share of the workgroups with a neighbour
-          const float tc = shared > 0.f ? kCol2 : kCol, tr = kRow + (kRow2 - kRow) * fminf(1.49f * shared, 1.f);
-          const float a = col * tc, b = row * tr, over = lines - kFull, first_rows = kFull - n_col_lines;
-          walks = fmaxf(a, b);
-          if (over <= 0) break;
-          float from;                                                        // where the last rows begin
-          if (first_rows <= 0)                  from = (0.6f * ceilf(over / kFull) + 0.4f * over / kFull) * (c.len * density * tc + 12.2f);
-          else if (over <= first_rows && b < a) from = 0.69f * b + 12.2f;
-          else                                  from = over <= fmaxf(n_col_lines, first_rows) ? 0.8f * fminf(a, b) + 12.2f : walks + 12.2f;
-          if (!causal && lines <= 3 * kCus && r.len >= c.len) from *= 0.48f;
-          if (causal && first_rows > 0) from *= fminf(0.03f + 4.f * over / kFull, 1.f);
-          walks = fmaxf(walks, from + kRow2 * (causal ? fmaxf(row - 0.16f * n_qtiles, 0.15f * row) : row));
-        }
-      }
-      us += fmaxf(walks, least);
+      const BwdWalk &c = cols[i], &r = rows[j];
       const float mb = ((c.n > 1 ? 2.f * c.n * wk : 0.f) + (r.n > 1 ? r.n * wq : 0.f)) * (kTile * kHeadDim * 4 / 1e6f), full = fminf(mb / 8, 2.f);
-      if (mb > 0.f) us = (us + 1.96f) * 1.035f + (c.n > 1 ? 0.7f : 0.f) + (c.n > 1 && r.n > 1 ? 0.58f : 0.f) + mb / 4.34f + 0.31f * full * full;
-      if (us < 0.995f * best_us) { best_us = us; best = {c.parts, r.parts}; }         // more parts for a gain, not for a tie
+      const float sum = mb > 0.f ? 1.96f + (c.n > 1 ? 0.7f : 0.f) + (c.n > 1 && r.n > 1 ? 0.58f : 0.f) + mb / 4.34f + 0.31f * full * full : 0.f;
+      for (int f = 0; f < n_forms; ++f) {
+        const int form = causal ? kCausalRates[f].form : bwd_form(nbh * ((int64_t)n_ktiles * c.n + (int64_t)n_qtiles * r.n), (int64_t)c.len + r.len);
+        float us = causal ? bwd_causal_us(kCausalRates[f], (float)nbh, n_qtiles, n_ktiles, tiles, c, r)
+                          : bwd_us(form, (float)nbh, n_qtiles, n_ktiles, c, r) * (mb > 0.f ? 1.035f : 1.f);
+        us += sum;
+        if (us < 0.995f * best_us) { best_us = us; best = {c.parts, r.parts, form}; }      // more parts for a gain, not for a tie
+      }
     }
   return best;
 }
 int64_t bwd_workspace_used(int batch, int n_heads, int n_qtiles, int n_ktiles, bool causal) {
   const DenseSplit d = dense_split(batch, n_heads, n_qtiles, n_ktiles);
-  const BwdCut n = bwd_cut((int64_t)batch * n_heads, n_qtiles, n_ktiles, causal, d.dkdv_parts, d.dq_parts);
+  const BwdPlan n = bwd_plan((int64_t)batch * n_heads, n_qtiles, n_ktiles, causal, d.dkdv_parts, d.dq_parts);
   return (n.cols > 1 ? n.cols * d.dkdv_bytes : 0) + (n.rows > 1 ? n.rows * d.dq_bytes : 0);
 }
 
@@ -929,7 +939,7 @@ extern "C" int ua_bsa_bwd(const void* q, const void* k, const void* v, const voi
   if (int rc = fill_side(p.cols, nnz, col_ptr, row_idx, cflag, k_order, dk, dk_strides, dv, dv_strides, false)) return rc;
   if (int rc = fill_side(p.rows, nnz, row_ptr, col_idx, flag, q_order, dq, dq_strides, nullptr, nullptr, false)) return rc;
   if (int rc = check_device()) return rc;
-  return launch_bwd(p, true, (hipStream_t)stream);
+  return launch_bwd(p, 1, (hipStream_t)stream);
 }
 
 extern "C" int ua_dense_bwd(const void* dout, const void* q, const void* k, const void* v,
@@ -964,14 +974,17 @@ extern "C" int ua_dense_bwd(const void* dout, const void* q, const void* k, cons
     s.out1 = reinterpret_cast<bf16*>(ws + part_bytes / 2);       // columns: dV behind dK
     ws += parts * part_bytes;
   };
-  BwdCut n = {1, 1};
-  if (workspace && aligned16(workspace) && workspace_bytes > 0) {
-    n = bwd_cut((int64_t)batch * n_heads, n_qtiles, n_ktiles, p.dense_causal, d.dkdv_parts, d.dq_parts);
-    if (workspace_bytes < (n.cols > 1 ? n.cols * d.dkdv_bytes : 0) + (n.rows > 1 ? n.rows * d.dq_bytes : 0)) n = {1, 1};
+  // (without a workspace lines are walked whole by one group; one that is too small or misaligned only keeps them from being cut)
+  BwdPlan n = {1, 1, 1};
+  if (workspace) {
+    auto plan = [&](int max_cols, int max_rows) { return bwd_plan((int64_t)batch * n_heads, n_qtiles, n_ktiles, p.dense_causal, max_cols, max_rows); };
+    n = plan(d.dkdv_parts, d.dq_parts);
+    const int64_t need = (n.cols > 1 ? n.cols * d.dkdv_bytes : 0) + (n.rows > 1 ? n.rows * d.dq_bytes : 0);
+    if (need > 0 && (workspace_bytes < need || !aligned16(workspace))) n = plan(1, 1);
   }
   if (n.cols > 1) cut(p.cols, n.cols, n_qtiles, d.dkdv_bytes);
   if (n.rows > 1) cut(p.rows, n.rows, n_ktiles, d.dq_bytes);
-  if (int rc = launch_bwd(p, !workspace, st)) return rc;
+  if (int rc = launch_bwd(p, n.form, st)) return rc;
   PartialSum sums[3];
   int n_sums = 0;
   auto add_sum = [&](const BwdSide& s, const bf16* first, void* out, const int64_t* os, int seqlen) {

@@ -397,7 +397,7 @@ int check_device();   // UA_OK when the current device is gfx950
 // list.  The walk may then be cut into parts that run as workgroups of their own and leave partial
 // results, combined by a second kernel.  No cut when the launch fills the device anyway or the list
 // is short; else at most as many parts as make ~2 workgroups per CU, of at least two tiles each, and
-// at most UA_MAX_PARTS.  How many are made is for the estimates of fwd_cut and bwd_cut to choose.
+// at most UA_MAX_PARTS.  How many are made is for the estimates of fwd_cut and bwd_plan to choose.
 constexpr int kDenseFullLaunch = 384, kDenseTargetGroups = 512;
 inline int dense_parts(int64_t n_workgroups, int list_len) {
   if (n_workgroups >= kDenseFullLaunch || list_len < 4) return 1;
