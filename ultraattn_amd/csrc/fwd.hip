@@ -417,7 +417,7 @@ static int fwd_common(FwdParams& p, const void* q, const void* k, const void* v,
 // Groups sum in another order, so that the last bits of a row depend on how many lines the launch has.  Tile lists, whose
 // launches are shards of the rows and heads of one mask, therefore run with one group whatever their size: a row's result is
 // the same bit for bit in every launch that holds its list.  Lists of up to 128 lines pay for that with half-empty CUs (one
-// head, causal 4096: forward 41 us with four groups, 67 with one, backward 61 and 117; from 512 lines on nothing changes).
+// head, causal 4096: forward 35 us with four groups, 58 with one, backward 51 and 119; from 512 lines on little changes).
 static int fwd_groups(int64_t n, int64_t walk, int n_parts, bool dense_causal) {
   const bool uneven = dense_causal && n_parts == 1;
   if (walk >= 2 && (2 * n <= kCus || (uneven && n <= kCus && walk >= 16))) return 4;
@@ -459,8 +459,9 @@ static int fwd_launch(FwdParams& p, bool plain, hipStream_t st) {
 //
 // Causal rectangles of more keys than queries whose whole walks run in a second round (more than 128 lines in four groups, more than 256 in
 // two) are cut by an estimate of their own: the second round begins when the shortest rows of the first are through, and all rows
-// are long.  Their partial O is fp32, so that every row is rounded once (bf16 partials take 2 to 4 us less).  Fitted to 270 rectangles of
-// 129 to 383 lines; over 410 others 9 % less time than whole: 10 heads of 1664 x 6144 87.8 -> 56.4 us, 3 of 7296 x 29440 430 -> 282.
+// are long.  Their partial O is fp32, so that every row is rounded once (bf16 partials take 2 to 4 us less).  10 heads of 1664 x 6144 87.8 -> 56.4
+// us, 3 of 7296 x 29440 430 -> 282; over 5400 causal rectangles of 129 to 511 lines 8 % less time than whole, three of them
+// more than 6 % slower, 9 at most.  (256 lines, the most of four groups, stay whole: what callers are told to bring there is two parts in bf16.)
 struct FwdCut {
   int parts;
   bool f32;
@@ -498,10 +499,11 @@ static FwdCut fwd_cut(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, int 
   };
   if (const int parts = least(first) > 1 ? least(second) : 1; parts > 1) return {parts, false};
   const int whole = fwd_groups(nbh * n_qtiles, n_ktiles, 1, causal), round = whole == 4 ? kCus / 2 : kCus;
-  if (!causal || n_ktiles <= n_qtiles || whole == 1 || lines <= round) return {1, false};
+  if (!causal || n_ktiles <= n_qtiles || whole == 1 || lines <= round || (whole == 4 && max_parts <= 2)) return {1, false};
   const float shortest = n_ktiles - n_qtiles * round / lines;                  // row of the first round
   auto rounded_once = [&](int parts) {
-    if (parts == 1) return 0.95f * (5.f + (whole == 4 ? fmaxf(1.25f * n_ktiles, 2.5f * shortest) : fmaxf(1.65f * n_ktiles, 3.6f * shortest)));
+    // (a workgroup of the second round starts anew; a cut has to win by 3 %)
+    if (parts == 1) return 0.97f * (whole == 4 ? fmaxf(5.f + 1.08f * n_ktiles, 9.f + 2.4f * shortest) : fmaxf(5.f + 1.6f * n_ktiles, 14.f + 3.5f * shortest));
     const int len = (n_ktiles + parts - 1) / parts, made = (n_ktiles + len - 1) / len;
     if (fwd_groups(nbh * n_qtiles * made, len, made, causal) != 1) return INFINITY;          // (several groups leave bf16)
     const float density = visible_share(n_qtiles, n_ktiles, causal), groups = lines * made;
