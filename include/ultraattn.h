@@ -200,8 +200,8 @@ int ua_bsa_bwd(const void *q, const void *k, const void *v, const void *dout,
  * j <= i + seqlen_k - seqlen_q; rows that see no key get o = 0, lse = -inf, zero gradients).
  * Rectangles with few tile lines (B * Nh * seqlen / 128 well below two workgroups per CU) run with
  * several groups of wavefronts per line, and where their walks are long they are cut into up to
- * UA_MAX_PARTS parts that run as workgroups of their own: the forward leaves partial (O, LSE) and
- * finishes with ua_merge's kernel, the backward leaves fp32 partial dQ (parts of the key range) and
+ * UA_MAX_PARTS parts that run as workgroups of their own: the forward leaves partial (O, LSE), O in
+ * bf16 or, for long causal rows, fp32, and merges them in a second launch, the backward leaves fp32 partial dQ (parts of the key range) and
  * dK, dV (parts of the query range) and sums them in one pass.  Of a large forward that is not
  * causal only the last query tiles are cut, those left over after the last full wave of workgroups;
  * their partial O is fp32.
