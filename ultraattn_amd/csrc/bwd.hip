@@ -3,7 +3,7 @@
 //
 //  dkdv_kernel : one workgroup per (key tile, head) walks the CSC column of query tiles.
 //                A wavefront owns 32 key rows; K and V fragments stay in registers, the Q and
-//                dO tiles stream through LDS.  Products (all 32x32x16 bf16 MFMA):
+//                dO tiles stream through LDS.  Products (bf16 MFMA, see Mma):
 //                  S [q,key]  = Q K^T          dP[q,key]  = dO V^T
 //                  dV^T[d,key] += dO^T P       dK^T[d,key] += Q^T dS
 //                In the accumulator layout a lane holds one key column, so S / dP blocks
@@ -76,63 +76,61 @@ __device__ __forceinline__ void touch_params() {
   asm volatile("" :: "s"(x[0]), "s"(x[1]), "s"(x[2]), "s"(x[3]), "s"(x[4]), "s"(x[5]), "s"(x[6]), "s"(x[7]), "s"(x[8]));
 }
 // 32 output rows of a wave: in the caller's strided bf16 tensor, or in part `part` of the fp32 partials.
+template <int kM>
 __device__ __forceinline__ void store_result(const __attribute__((address_space(4))) BwdSide* p, bf16* out, int64_t os_b, int64_t os_s,
                                              int64_t os_h, int n_heads, int part, int b, int64_t row0, int h, int64_t seq,
                                              const f32x16 (&acc)[4], float mul, uint32_t lds) {
   if (p->out_f32) {
     float* base = reinterpret_cast<float*>(out) + part * p->o_part;
-    store_rows_f32(base + (((int64_t)b * seq + row0) * n_heads + h) * kHeadDim, (int64_t)n_heads * kHeadDim, acc, mul, lds);
+    store_rows_f32<kM>(base + (((int64_t)b * seq + row0) * n_heads + h) * kHeadDim, (int64_t)n_heads * kHeadDim, acc, both(mul), lds);
   } else {
-    store_rows_bf16(out + b * os_b + row0 * os_s + h * os_h, os_s, acc, mul, lds);
+    store_rows_bf16<kM>(out + b * os_b + row0 * os_s + h * os_h, os_s, acc, both(mul), lds);
   }
 }
 
 // The same for one block of 32 columns.
+template <int kM>
 __device__ __forceinline__ void store_block(const __attribute__((address_space(4))) BwdSide* p, bf16* out, int64_t os_b, int64_t os_s,
                                             int64_t os_h, int n_heads, int part, int b, int64_t row0, int h, int64_t seq, int block,
                                             const f32x16& acc, float mul, uint32_t lds) {
   if (p->out_f32) {
     float* base = reinterpret_cast<float*>(out) + part * p->o_part;
-    store_block_f32(base + (((int64_t)b * seq + row0) * n_heads + h) * kHeadDim + 32 * block, (int64_t)n_heads * kHeadDim, acc, mul, lds);
+    store_block_f32<kM>(base + (((int64_t)b * seq + row0) * n_heads + h) * kHeadDim + 32 * block, (int64_t)n_heads * kHeadDim, acc, both(mul), lds);
   } else {
-    store_block_bf16(out + b * os_b + row0 * os_s + h * os_h + 32 * block, os_s, acc, mul, lds);
+    store_block_bf16<kM>(out + b * os_b + row0 * os_s + h * os_h + 32 * block, os_s, acc, both(mul), lds);
   }
 }
 
 // ---- dK/dV ------------------------------------------------------------------------------------
 // Four wavefronts, wave w owns key rows 32w..32w+31 and keeps their K and V rows as B operands; the
 // query side is streamed in half tiles of 64 rows (two blocks of 32) through two LDS stages.  Per block:
-//   S = Q K^T - lse/scale,  dP' = dO V^T - delta        16 MFMAs, Q and dO rows read 128 bits at a time
+//   S = Q K^T - lse/scale,  dP' = dO V^T - delta        16 row fragments, Q and dO read 128 bits at a time
 //   P = exp2(scale*log2e*S), dS = P * dP'               in the accumulators' lanes
-//   dV^T += dO^T P,  dK^T += Q^T dS                     16 MFMAs, Q and dO read through the transposing path
+//   dV^T += dO^T P,  dK^T += Q^T dS                     16 column fragments, Q and dO read through the transposing path
 // P and dS never leave the wave.  The accumulators of S and dP' start from the rows' statistics.
 //
-// Bound: matrix pipe at the clock the socket's power allows (71 % busy at 1.68 GHz).  192 of a wave's 256 registers
+// Bound: the socket's power (both sides 69 % matrix-pipe busy at 1.87 GHz, causal 32k).  192 of a wave's 256 registers
 // hold K, V, dK and dV; two independent workgroups share a CU, so that one's exp2 and barriers hide behind
 // the other's MFMAs.  Against one workgroup of eight waves in two roles (S/dV and dP/dK, P handed over
 // through LDS): strided 128k, 32 heads 37.8 -> 33.5 ms, causal 32k 15.8 -> 13.7 ms (1.25-1.3 PFLOP/s of the four
-// products).  Row fragments are fetched two MFMAs ahead (three: the same within 0.5 %); a P computed during dP's MFMAs spills
-// registers: 3-15 % slower.
+// products, both kernels with 32x32x16).
 //
-// LDS: four consecutive rows (1 KiB, one copy instruction of one wave) lie at a pitch of 1040 bytes and a
-// row's 16-byte chunks are XORed with 4 * (row % 4).  16 consecutive rows then hit 16 different slots
-// (128-bit reads) and 4 consecutive rows 4 different 64-byte groups (transposing reads), while the
-// chunk bits that the XOR leaves alone, the row blocks and the stages are all compile-time offsets: four
-// address registers serve the 128-bit reads of both operands and four the transposing ones.
+// LDS: the V-type layout.  The chunk bits that its XOR leaves alone, the row blocks and the stages are all
+// compile-time offsets: four address registers serve the 128-bit reads of both operands and four the transposing ones.
 #define UA_LDS __attribute__((address_space(3)))
-constexpr int kGroupPitch = 1040;                       // bytes between groups of 4 rows
-constexpr int kBlockPitch = 8 * kGroupPitch;            // 32 rows
 // A group's LDS: stage s holds the first operand's rows at 2s * kPitch and the second's behind them; then the statistics
 // -lse/scale and -delta of either stage and the waves' list entries.
 template <int kForm>
 struct Stages : Groups<kForm> {
-  static constexpr int kPitch = Groups<kForm>::kRows / 4 * kGroupPitch;
+  static constexpr int kM = mma_of(kForm);
+  static constexpr int kBlockPitch = 8 * Mma<kM>::kPitch;            // 32 rows
+  static constexpr int kPitch = Groups<kForm>::kRows / 4 * Mma<kM>::kPitch;
   static constexpr int kStatBytes = 2 * Groups<kForm>::kRows * 4;
   static constexpr int kStat = 4 * kPitch;
   static constexpr int kEntries = kStat + 2 * kStatBytes;
   static constexpr int kBytes = kEntries + (kForm == 1 ? 4 * Walk<false, false>::kBytes : 0);
 };
-static_assert(3 * Stages<1>::kPitch + kBlockPitch + 6 * kGroupPitch < 65536, "operand offsets fit the instructions' offset field");
+static_assert(3 * Stages<1>::kPitch + Stages<1>::kBlockPitch + 4 * Mma<16>::kPitch + 32 < 65536, "operand offsets fit the instructions' offset field");
 
 __device__ __forceinline__ void keep_in_register(uint32_t& x) { asm volatile("" : "+v"(x)); }
 __device__ __forceinline__ float in_scalar(float x) {            // a wave-uniform value in a scalar register
@@ -148,15 +146,18 @@ __device__ __forceinline__ bf16x8 lds_abs_tr_pair(uint32_t a_lo, uint32_t a_hi) 
 }
 // Per-lane absolute LDS addresses within the first operand's half tile of stage 0; the second operand, later
 // rows and stage 1 are compile-time offsets.
+// (The row reads of 32x32x16, whose chunks come in pairs 32 bytes apart that the XOR leaves alone, need four address registers too.)
+template <int kM>
 struct PairAddr {
-  uint32_t nat[4];      // 128-bit row reads: row lane%32, chunks 4*j + lane/32 (and + 2)
-  uint32_t tr[4];       // transposing reads for d-block j
+  uint32_t nat[4];      // 128-bit row reads
+  uint32_t tr[4];       // transposing reads
   __device__ __forceinline__ PairAddr(uint32_t lds_base, int lane) {
-    const int l32 = lane & 31, hi = lane >> 5, i16 = lane & 15, grp = (lane >> 4) & 1, r4 = i16 >> 2;
+    using M = Mma<kM>;
+    const int row = M::a_row(lane);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      nat[j] = lds_base + (l32 >> 2) * kGroupPitch + (l32 & 3) * kRowBytes + ((((j ^ (l32 & 3)) << 2) + hi) << 4);
-      tr[j] = lds_base + hi * kGroupPitch + r4 * kRowBytes + (((j ^ r4) << 2) + 2 * grp + ((i16 & 3) >> 1)) * 16 + (i16 & 1) * 8;
+      nat[j] = lds_base + (row >> 2) * M::kPitch + (row & 3) * kRowBytes + (slot_v(row, M::a_chunk(lane, kM == 32 ? 2 * j : j)) << 4);
+      tr[j] = lds_base + M::tr_offset(lane, j);
       keep_in_register(nat[j]);
       keep_in_register(tr[j]);
     }
@@ -166,12 +167,15 @@ struct PairAddr {
     for (int j = 0; j < 4; ++j) { nat[j] += bytes; tr[j] += bytes; }
   }
 };
-// Fragment reads at a compile-time offset: k-step ks of 32 rows, and 16 rows x d-block m transposed.
-template <int kOff>
-__device__ __forceinline__ bf16x8 pair_nat(const PairAddr& ad, int ks) { return lds_abs_b128(ad.nat[ks >> 1] + (kOff + 32 * (ks & 1))); }
-template <int kOff>
-__device__ __forceinline__ bf16x8 pair_tr(const PairAddr& ad, int step16, int m) {
-  return lds_abs_tr_pair(ad.tr[m] + (kOff + 4 * kGroupPitch * step16), ad.tr[m] + (kOff + 4 * kGroupPitch * step16 + 2 * kGroupPitch));
+// Fragment reads (i of 8) at a compile-time offset: of a block's 32 rows, and of those rows transposed.
+template <int kOff, int kM>
+__device__ __forceinline__ bf16x8 pair_nat(const PairAddr<kM>& ad, int i) {
+  return lds_abs_b128(ad.nat[i >> 1] + (kOff + (kM == 32 ? 32 * (i & 1) : Mma<kM>::a_offset(i, Mma<kM>::kPitch))));
+}
+template <int kOff, int kM>
+__device__ __forceinline__ bf16x8 pair_tr(const PairAddr<kM>& ad, int i) {
+  using M = Mma<kM>;
+  return lds_abs_tr_pair(ad.tr[M::tr_reg(i)] + (kOff + M::tr_first(i)), ad.tr[M::tr_reg(i)] + (kOff + M::tr_first(i) + M::kTrSecond));
 }
 
 // The walked pair of operands (Q and dO, or K and V): asynchronous copies of a group's rows into an LDS stage.
@@ -190,7 +194,7 @@ struct PairStream {
     const int row = 4 * wave + (lane >> 4), chunk = (lane & 15) ^ ((lane >> 4) << 2);
     xoff = (row * xs + chunk * 8) * 2;
     yoff = (row * ys + chunk * 8) * 2;
-    lds = __builtin_amdgcn_readfirstlane(lds_base + wave * kGroupPitch);
+    lds = __builtin_amdgcn_readfirstlane(lds_base + wave * Mma<S::kM>::kPitch);
   }
   // Without `more` the copies that follow read nothing and fill with zeros a stage that no step reads: no branch at each of them.
   __device__ __forceinline__ void tile(int t, bool more) {
@@ -198,10 +202,12 @@ struct PairStream {
     rx = make_rsrc_words(x + row0 * xs, more ? (uint32_t)((kTile - 1) * xs + kHeadDim) * 2 : 0);
     ry = make_rsrc_words(y + row0 * ys, more ? (uint32_t)((kTile - 1) * ys + kHeadDim) * 2 : 0);
   }
+  // (Opaque in every step: the sums of the copies' LDS addresses would occupy scalar registers all along, and vector lanes.)
+  __device__ __forceinline__ void next_step() { asm volatile("" : "+s"(lds)); }
   // copy n of kCopies into stage kStage, rows from 64 or 32 * part of the tile on
   template <int kStage>
   __device__ __forceinline__ void copy(int n, int part) const {
-    const int j = n >> 1, at = 2 * kStage * S::kPitch + S::kWaves * j * kGroupPitch, row = part * S::kRows + 4 * S::kWaves * j;
+    const int j = n >> 1, at = 2 * kStage * S::kPitch + S::kWaves * j * Mma<S::kM>::kPitch, row = part * S::kRows + 4 * S::kWaves * j;
     if (n & 1) dma16_abs(ry, lds + at + S::kPitch, yoff, row * ys * 2);
     else       dma16_abs(rx, lds + at, xoff, row * xs * 2);
   }
@@ -209,9 +215,89 @@ struct PairStream {
 
 // One block of 32 query rows for this wave's 32 keys.  kOff = LDS offset of the block's Q rows; dO lies kPitch
 // behind, -delta kStatBytes / 2 behind -lse/scale.  `copy(n)`, n = 0 .. kCopies - 1, is called between the first MFMAs.
+// With 16x16x32 the first 16 rows' P and dS are made before the second ones' products begin: 8 registers fewer are live, which hold
+// a third fragment ahead (all 32 rows at once, two ahead: causal 8192, 32 heads, 1462 us, so 1419; one head, causal 4096, 154 and 123).
+// Without the barrier between the two halves the compiler mixes them again and takes 2 % longer.
 template <int kOff, int kPitch, int kStatOff, int kStatBytes, int kCopies, class Copy>
-__device__ __forceinline__ void dkdv_block(const PairAddr& ad, uint32_t stat_base, const bf16x8 (&kf)[8], const bf16x8 (&vf)[8], f32x16 (&dk)[4],
+__device__ __forceinline__ void dkdv_block(const PairAddr<16>& ad, uint32_t stat_base, const bf16x8 (&kf)[8], const bf16x8 (&vf)[8], f32x16 (&dk)[4],
                                            f32x16 (&dv)[4], float scale_log2, bool mask, Copy copy) {
+  using M = Mma<16>;
+  f32x4 s[2][2], dp[2][2], lse[2], delta[2];                      // [qb][n], [qb]
+  uint32_t stat = stat_base + 16 * (fresh_lane() >> 4);           // this lane group's 4 consecutive row statistics
+  keep_in_register(stat);                // (the reads' offsets then are constants: a lone workgroup 2 % faster)
+  auto rd_stat = [&](int qb) {
+    lse[qb] = *reinterpret_cast<const UA_LDS f32x4*>(stat + (kStatOff + 64 * qb));
+    delta[qb] = *reinterpret_cast<const UA_LDS f32x4*>(stat + (kStatOff + kStatBytes / 2 + 64 * qb));
+  };
+  rd_stat(0);
+  __builtin_amdgcn_sched_barrier(0);       // the reads below, mixed with what came before them, spill registers
+  // 16 row fragments, Q and dO alternating, of the first and then of the second 16 rows, fetched kAhead reads ahead of their MFMAs
+  constexpr int kAhead = 3;
+  bf16x8 fr[16];
+  auto rd = [&](int i) {
+    const int part = 2 * (i >> 1 & 3) + (i >> 3);
+    return (i & 1) ? pair_nat<kOff + kPitch>(ad, part) : pair_nat<kOff>(ad, part);
+  };
+#pragma unroll
+  for (int i = 0; i < kAhead; ++i) fr[i] = rd(i);
+  __builtin_amdgcn_sched_group_barrier(0x100, kAhead, 0);
+  bf16x8 pb[2], dsb[2];
+  // transposed fragments i: dO for i even (dV), Q for i odd (dK); columns 16 * (i / 2)
+  auto rd_tr = [&](int i) { return (i & 1) ? pair_tr<kOff>(ad, i >> 1) : pair_tr<kOff + kPitch>(ad, i >> 1); };
+  constexpr int kTAhead = 2;
+  bf16x8 ft[16];
+#pragma unroll
+  for (int qb = 0; qb < 2; ++qb) {
+#pragma unroll
+    for (int i = 8 * qb; i < 8 * qb + 8; ++i) {
+      if (i + kAhead < 16) fr[i + kAhead] = rd(i + kAhead);
+      const int ks = i >> 1 & 3;
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        if (i & 1) dp[qb][n] = M::mfma(fr[i], vf[2 * ks + n], ks == 0 ? delta[qb] : dp[qb][n]);
+        else       s[qb][n] = M::mfma(fr[i], kf[2 * ks + n], ks == 0 ? lse[qb] : s[qb][n]);
+      }
+      M::interleave<1>();
+      if ((i + 1) * kCopies / 16 != i * kCopies / 16) copy(i * kCopies / 16);
+    }
+    // element j of block (qb, n): query row 16*qb + 4*(lane/16) + j, key column 16*n + lane%16
+    if (mask) {
+      const int lane = fresh_lane(), ahead = (lane & 15) - 4 * (lane >> 4);
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (ahead + 16 * n > 16 * qb + j) s[qb][n][j] = -INFINITY;
+    }
+    if (qb == 1) {
+#pragma unroll
+      for (int i = 0; i < kTAhead; ++i) ft[i] = rd_tr(i);
+    }
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float pv = fast_exp2(s[qb][n][j] * scale_log2);
+        pb[n][4 * qb + j] = (bf16)pv;
+        dsb[n][4 * qb + j] = (bf16)(pv * dp[qb][n][j]);
+      }
+    if (qb == 0) rd_stat(1);
+    if (qb == 0) __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    if (i + kTAhead < 16) ft[i + kTAhead] = rd_tr(i + kTAhead);
+    if (i & 1) M::second(dk, i >> 1, ft[i], dsb);
+    else       M::second(dv, i >> 1, ft[i], pb);
+    M::interleave<2>();
+  }
+}
+
+// The same with 32x32x16.
+template <int kOff, int kPitch, int kStatOff, int kStatBytes, int kCopies, class Copy>
+__device__ __forceinline__ void dkdv_block(const PairAddr<32>& ad, uint32_t stat_base, const bf16x8 (&kf)[8], const bf16x8 (&vf)[8], f32x16 (&dk)[4],
+                                           f32x16 (&dv)[4], float scale_log2, bool mask, Copy copy) {
+  using M = Mma<32>;
   f32x16 s, dp;
   uint32_t stat = stat_base + 16 * (fresh_lane() >> 5);           // this lane half's 4 consecutive row statistics
   keep_in_register(stat);                // (the reads' offsets then are constants: a lone workgroup 2 % faster)
@@ -235,17 +321,15 @@ __device__ __forceinline__ void dkdv_block(const PairAddr& ad, uint32_t stat_bas
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       if (i + kAhead < 16) fr[i + kAhead] = rd(i + kAhead);
-      if (i & 1) dp = mfma32(fr[i], vf[i >> 1], dp);
-      else       s = mfma32(fr[i], kf[i >> 1], s);
+      if (i & 1) dp = M::mfma(fr[i], vf[i >> 1], dp);
+      else       s = M::mfma(fr[i], kf[i >> 1], s);
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
       if ((i + 1) * kCopies / 16 != i * kCopies / 16) copy(i * kCopies / 16);
     }
   }
   // transposed fragments i: dO for i even (dV), Q for i odd (dK); d-block (i/2)%4, 16-row step i/8
-  auto rd_tr = [&](int i) {
-    return (i & 1) ? pair_tr<kOff>(ad, i >> 3, (i >> 1) & 3) : pair_tr<kOff + kPitch>(ad, i >> 3, (i >> 1) & 3);
-  };
+  auto rd_tr = [&](int i) { return (i & 1) ? pair_tr<kOff>(ad, i >> 1) : pair_tr<kOff + kPitch>(ad, i >> 1); };
   constexpr int kTAhead = 2;
   bf16x8 fr[16];
 #pragma unroll
@@ -266,8 +350,8 @@ __device__ __forceinline__ void dkdv_block(const PairAddr& ad, uint32_t stat_bas
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
     if (i + kTAhead < 16) fr[i + kTAhead] = rd_tr(i + kTAhead);
-    if (i & 1) dk[(i >> 1) & 3] = mfma32(fr[i], dsb[i >> 3], dk[(i >> 1) & 3]);
-    else       dv[(i >> 1) & 3] = mfma32(fr[i], pb[i >> 3], dv[(i >> 1) & 3]);
+    if (i & 1) M::second(dk, i >> 1, fr[i], dsb);
+    else       M::second(dv, i >> 1, fr[i], pb);
     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
     __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
   }
@@ -340,7 +424,7 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& given, uint32_t lds_b
     stat = S::kSteps == 2 ? load_stat(ent, part_of(1)) : load_stat(walk.at(min(e0 + 1, e1 - 1)), group);
   }
 
-  // K and V rows as B operands: lane holds key row 32*k_block + lane%32, d = 16*ks + 8*hi .. +7
+  // K and V rows as B operands
   // (through the stage that the first step fills)
   const int k_block = S::kWaves * sub + wave, krow0 = kt * kTile + k_block * 32;
   bf16x8 kf[8], vf[8];
@@ -349,8 +433,8 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& given, uint32_t lds_b
     load_rows(kraw, p.k + b * p.ks.b + (int64_t)krow0 * p.ks.s + h * p.ks.h, p.ks.s);
     load_rows(vraw, p.v + b * p.vs.b + (int64_t)krow0 * p.vs.s + h * p.vs.h, p.vs.s);
     const uint32_t turn = lds_base + 2 * S::kPitch + wave * kWaveRowsBytes;
-    rows_to_frags(kf, kraw, turn);
-    rows_to_frags(vf, vraw, turn);
+    rows_to_frags<S::kM>(kf, kraw, turn);
+    rows_to_frags<S::kM>(vf, vraw, turn);
   } else {
     const int64_t line0 = (int64_t)kt * kTile + sub * 32 * S::kWaves;
     const uint32_t k_lds = lds_block + 2 * S::kPitch, v_lds = k_lds + S::kBytes;           // stage 1 of groups 0 and 1
@@ -358,14 +442,14 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& given, uint32_t lds_b
     copy_shared_rows<32 * S::kWaves, S::kThreads>(p.v + b * p.vs.b + line0 * p.vs.s + h * p.vs.h, (int)p.vs.s, v_lds);
     wait_vmem_all();
     __syncthreads();
-    shared_rows_to_frags(kf, k_lds, wave);
-    shared_rows_to_frags(vf, v_lds, wave);
+    shared_rows_to_frags<S::kM>(kf, k_lds, wave);
+    shared_rows_to_frags<S::kM>(vf, v_lds, wave);
   }
   f32x16 dk[4], dv[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) { dk[i] = f32x16{0}; dv[i] = f32x16{0}; }
 
-  PairAddr ad(lds_base, lane);
+  PairAddr<S::kM> ad(lds_base, lane);
   if (e0 < e1) put_stat(0, st0);
   // The compiler does not see the copies that the walk has in flight.  Were the K and V rows still
   // outstanding for it there, it would wait for them by count inside the loop, i.e. for the copies: they are
@@ -388,6 +472,7 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& given, uint32_t lds_b
     }
     put_stat(kStage ^ 1, stat);
     stat = S::kSteps == 2 ? load_stat(ent_next, part_of(kStage)) : load_stat(walk.at(min(e + 2, e1 - 1)), group);
+    in.next_step();
     if (!kFirst) in.tile(walk.tile(ent_next), e + 1 < e1);
     const bool causal = (ent >> 30) != 0;
     // causal tile: query block nb sees none of the wave's keys when nb < k_block, some when nb == k_block
@@ -396,7 +481,7 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& given, uint32_t lds_b
     if (!causal) {
       auto block = [&](auto mb_tag) {
         constexpr int kMb = decltype(mb_tag)::value;
-        dkdv_block<kOff + kMb * kBlockPitch, S::kPitch, kStatOff + kMb * 128, S::kStatBytes, kCopies>(
+        dkdv_block<kOff + kMb * S::kBlockPitch, S::kPitch, kStatOff + kMb * 128, S::kStatBytes, kCopies>(
             ad, lds_base + S::kStat, kf, vf, dk, dv, scale_log2, false, [&](int n) { in.template copy<kStage ^ 1>(kMb * kCopies + n, part_next); });
       };
       block(std::integral_constant<int, 0>{});
@@ -411,10 +496,10 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& given, uint32_t lds_b
       for (int n = 0; n < in.kCopies; ++n) in.template copy<kStage ^ 1>(n, part_next);
 #pragma unroll 1
       for (int mb = max(k_block - nb, 0); mb < kBlocks; ++mb) {
-        ad.shift(mb * kBlockPitch);
+        ad.shift(mb * S::kBlockPitch);
         dkdv_block<kOff, S::kPitch, kStatOff, S::kStatBytes, 0>(ad, lds_base + S::kStat + mb * 128, kf, vf, dk, dv, scale_log2, nb + mb == k_block,
                                                                 [](int) {});
-        ad.shift(-mb * kBlockPitch);
+        ad.shift(-mb * S::kBlockPitch);
       }
     }
     if (!kFirst) ent = ent_next;
@@ -433,18 +518,18 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& given, uint32_t lds_b
     __syncthreads();
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb)
-      if (group) add_block(area(0), mb, dv[mb]); else add_block(area(1), mb, dk[mb]);
+      if (group) add_block<S::kM>(area(0), mb, dv[mb], both(1.f), both(1.f)); else add_block<S::kM>(area(1), mb, dk[mb], both(1.f), both(1.f));
   }
   f32x16 dk_sum, dv_sum;             // four groups: each finishes a block of 32 columns of both
   if constexpr (kForm == 4) {
-    constexpr float kOnes[4] = {1.f, 1.f, 1.f, 1.f};
+    const RowPair kOnes[4] = {both(1.f), both(1.f), both(1.f), both(1.f)};
     put_acc(area(group), dk, group);
     __syncthreads();
-    sum_blocks(dk_sum, dk, group, area, kOnes);
+    sum_blocks<S::kM>(dk_sum, dk, group, area, kOnes);
     __syncthreads();
     put_acc(area(group), dv, group);
     __syncthreads();
-    sum_blocks(dv_sum, dv, group, area, kOnes);
+    sum_blocks<S::kM>(dv_sum, dv, group, area, kOnes);
   }
   const ParamsLate pl = params_late();
   const int64_t seq_k = (int64_t)pl->n_ktiles * kTile;
@@ -452,28 +537,29 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& given, uint32_t lds_b
   if constexpr (kForm == 4) {
     // (this wave alone reads the block of its own area that it turns through)
     const uint32_t turn = area(group) + 4096 * group;
-    store_block(&pl->cols, pl->cols.out0, pl->cols.o0s.b, pl->cols.o0s.s, pl->cols.o0s.h, pl->n_heads, part, b, krow_out, h, seq_k, group, dk_sum, pl->scale, turn);
-    store_block(&pl->cols, pl->cols.out1, pl->cols.o1s.b, pl->cols.o1s.s, pl->cols.o1s.h, pl->n_heads, part, b, krow_out, h, seq_k, group, dv_sum, 1.f, turn);
+    store_block<S::kM>(&pl->cols, pl->cols.out0, pl->cols.o0s.b, pl->cols.o0s.s, pl->cols.o0s.h, pl->n_heads, part, b, krow_out, h, seq_k, group, dk_sum, pl->scale, turn);
+    store_block<S::kM>(&pl->cols, pl->cols.out1, pl->cols.o1s.b, pl->cols.o1s.s, pl->cols.o1s.h, pl->n_heads, part, b, krow_out, h, seq_k, group, dv_sum, 1.f, turn);
   } else {
     const uint32_t turn = kForm == 1 ? lds_base + wave * kWaveRowsBytes : area(group ^ 1);
     if (kForm == 1 || group == 0)
-      store_result(&pl->cols, pl->cols.out0, pl->cols.o0s.b, pl->cols.o0s.s, pl->cols.o0s.h, pl->n_heads, part, b, krow_out, h, seq_k, dk, pl->scale, turn);
+      store_result<S::kM>(&pl->cols, pl->cols.out0, pl->cols.o0s.b, pl->cols.o0s.s, pl->cols.o0s.h, pl->n_heads, part, b, krow_out, h, seq_k, dk, pl->scale, turn);
     if (kForm == 1 || group == 1)
-      store_result(&pl->cols, pl->cols.out1, pl->cols.o1s.b, pl->cols.o1s.s, pl->cols.o1s.h, pl->n_heads, part, b, krow_out, h, seq_k, dv, 1.f, turn);
+      store_result<S::kM>(&pl->cols, pl->cols.out1, pl->cols.o1s.b, pl->cols.o1s.s, pl->cols.o1s.h, pl->n_heads, part, b, krow_out, h, seq_k, dv, 1.f, turn);
   }
 }
 
 // ---- dQ -----------------------------------------------------------------------------------------
 // Four wavefronts, wave w owns query rows 32w..32w+31 and keeps their Q and dO rows as B operands; K and V are
-// streamed like dK/dV's operands.  Per block of 32 keys: S^T = K Q^T and dP'^T = V dO^T - delta (16 MFMAs),
-// dS^T in the lanes, dQ^T += K^T dS^T (8 MFMAs).  A lane holds one query column, so -delta is one value per
-// lane: it is kept in 16 registers that dP's first MFMA takes as its addend, which spares 16 moves per block.
-template <int kOff, int kPitch, int kCopies, class Copy, class Side>
-__device__ __forceinline__ void dq_block(const PairAddr& ad, const bf16x8 (&qf)[8], const bf16x8 (&dof)[8], const f32x16& neg_delta,
-                                         f32x16 (&dq)[4], float scale_log2, float lse2, bool mask, Copy copy, Side side) {
+// streamed like dK/dV's operands.  Per block of 32 keys: S^T = K Q^T and dP'^T = V dO^T - delta (16 row fragments),
+// dS^T in the lanes, dQ^T += K^T dS^T (8 column fragments).  A lane holds one query column, or one of each 16, so -delta is one
+// value for all of a column's accumulators: it is kept in registers that dP's first MFMAs take as their addend, which spares moves.
+template <int kM, int kOff, int kPitch, int kCopies, class Copy, class Side>
+__device__ __forceinline__ void dq_block(const PairAddr<kM>& ad, const bf16x8 (&qf)[8], const bf16x8 (&dof)[8], const typename Mma<kM>::Start& neg_delta,
+                                         f32x16 (&dq)[4], float scale_log2, const float (&lse2)[2], bool mask, Copy copy, Side side) {
+  using M = Mma<kM>;
   f32x16 s, dp;
   {
-    // 16 row fragments, K and V alternating, fetched kAhead reads ahead of their MFMA
+    // 16 row fragments, K and V alternating, fetched kAhead reads ahead of their MFMAs
     constexpr int kAhead = 4;
     bf16x8 fr[16];
     auto rd = [&](int i) { return (i & 1) ? pair_nat<kOff + kPitch>(ad, i >> 1) : pair_nat<kOff>(ad, i >> 1); };
@@ -483,10 +569,9 @@ __device__ __forceinline__ void dq_block(const PairAddr& ad, const bf16x8 (&qf)[
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       if (i + kAhead < 16) fr[i + kAhead] = rd(i + kAhead);
-      if (i & 1) dp = mfma32(fr[i], dof[i >> 1], i == 1 ? neg_delta : dp);
-      else       s = mfma32(fr[i], qf[i >> 1], i == 0 ? f32x16{0} : s);
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      if (i & 1) M::first(dp, i >> 1, fr[i], dof, neg_delta);
+      else       M::first(s, i >> 1, fr[i], qf, M::start({0.f, 0.f}));
+      M::template interleave<1>();
       if ((i + 1) * kCopies / 16 != i * kCopies / 16) copy(i * kCopies / 16);
     }
   }
@@ -494,27 +579,26 @@ __device__ __forceinline__ void dq_block(const PairAddr& ad, const bf16x8 (&qf)[
   constexpr int kTAhead = 3;
   bf16x8 tfr[8];
 #pragma unroll
-  for (int i = 0; i < kTAhead; ++i) tfr[i] = pair_tr<kOff>(ad, i >> 2, i & 3);
-  // element i: key 8*(i/4) + 4*hi + i%4 of the block, query column lane%32
+  for (int i = 0; i < kTAhead; ++i) tfr[i] = pair_tr<kOff>(ad, i);
+  // element i: key quad_row + i % 4 of the block, query column col
   if (mask) {
-    const int lane = fresh_lane(), q_b = lane & 31, hi4 = 4 * (lane >> 5);
+    const int lane = fresh_lane(), ahead = M::quad_row(lane, 0) - M::col(lane, 0);
 #pragma unroll
     for (int i = 0; i < 16; ++i)
-      if (8 * (i >> 2) + hi4 + (i & 3) > q_b) s[i] = -INFINITY;
+      if (ahead + M::quad_row(0, i >> 2) + (i & 3) > M::col(0, M::quad_n(i >> 2))) s[i] = -INFINITY;
   }
   side();
   bf16x8 dsb[2];
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
-    const float pv = fast_exp2(fmaf(s[i], scale_log2, -lse2));
-    dsb[i >> 3][i & 7] = (bf16)(pv * dp[i]);
+    const float pv = fast_exp2(fmaf(s[i], scale_log2, -lse2[M::quad_n(i >> 2)]));
+    dsb[M::slot_n(i)][M::slot_j(i)] = (bf16)(pv * dp[i]);
   }
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    if (i + kTAhead < 8) tfr[i + kTAhead] = pair_tr<kOff>(ad, (i + kTAhead) >> 2, (i + kTAhead) & 3);
-    dq[i & 3] = mfma32(tfr[i], dsb[i >> 2], dq[i & 3]);
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-    __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+    if (i + kTAhead < 8) tfr[i + kTAhead] = pair_tr<kOff>(ad, i + kTAhead);
+    M::second(dq, i, tfr[i], dsb);
+    M::template interleave<2>();
   }
 }
 
@@ -524,7 +608,7 @@ __device__ __forceinline__ void dq_walk(const BwdParams& given, uint32_t lds_blo
   static_assert(kDense || kForm == 1, "lists run with one group");
   if (kForm == 1 && kDense && p.rows_ahead) __builtin_amdgcn_s_setprio(1);
   using S = Stages<kForm>;
-  const int tid = threadIdx.x % (64 * S::kWaves), lane = tid & 63, l32 = lane & 31;
+  const int tid = threadIdx.x % (64 * S::kWaves), lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int group = S::kCount == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * S::kWaves));
   const uint32_t lds_base = lds_block + group * S::kBytes;
@@ -561,7 +645,7 @@ __device__ __forceinline__ void dq_walk(const BwdParams& given, uint32_t lds_blo
     for (int n = 0; n < in.kCopies; ++n) in.template copy<0>(n, part_of(0));
   }
 
-  const int q_block = S::kWaves * sub + wave, qrow0 = qt * kTile + q_block * 32, qrow = qrow0 + l32;
+  const int q_block = S::kWaves * sub + wave, qrow0 = qt * kTile + q_block * 32;
   bf16x8 qf[8], dof[8];
   u32x4 qraw[8], doraw[8];
   const uint32_t q_lds = lds_block + 2 * S::kPitch, do_lds = q_lds + S::kBytes;            // stage 1 of groups 0 and 1
@@ -573,28 +657,34 @@ __device__ __forceinline__ void dq_walk(const BwdParams& given, uint32_t lds_blo
     copy_shared_rows<32 * S::kWaves, S::kThreads>(p.q + b * p.qs.b + line0 * p.qs.s + h * p.qs.h, (int)p.qs.s, q_lds);
     copy_shared_rows<32 * S::kWaves, S::kThreads>(p.dout + b * p.ds.b + line0 * p.ds.s + h * p.ds.h, (int)p.ds.s, do_lds);
   }
-  const float lse_raw = p.lse[((int64_t)b * p.n_heads + h) * seq_q + qrow];
-  const float neg_delta = -p.delta[((int64_t)b * p.n_heads + h) * seq_q + qrow];
+  using M = Mma<S::kM>;
+  float lse_raw[2], neg_delta[2];          // of the lane's queries
+#pragma unroll
+  for (int n = 0; n < M::kCols; ++n) {
+    const int64_t row = ((int64_t)b * p.n_heads + h) * seq_q + qrow0 + M::col(lane, n);
+    lse_raw[n] = p.lse[row];
+    neg_delta[n] = -p.delta[row];
+  }
   if constexpr (kForm == 1) {
     const uint32_t turn = lds_base + 2 * S::kPitch + wave * kWaveRowsBytes;      // in the stage that the first step fills
-    rows_to_frags(qf, qraw, turn);
-    rows_to_frags(dof, doraw, turn);
+    rows_to_frags<S::kM>(qf, qraw, turn);
+    rows_to_frags<S::kM>(dof, doraw, turn);
   } else {
     wait_vmem_all();
     __syncthreads();
-    shared_rows_to_frags(qf, q_lds, wave);
-    shared_rows_to_frags(dof, do_lds, wave);
+    shared_rows_to_frags<S::kM>(qf, q_lds, wave);
+    shared_rows_to_frags<S::kM>(dof, do_lds, wave);
   }
-  const float lse2 = (lse_raw == -INFINITY) ? INFINITY : lse_raw * kLog2e;
-  f32x16 nd;
+  float lse2[2];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) nd[i] = neg_delta;
-  asm volatile("" : "+v"(nd));         // 16 registers, not one value moved into an accumulator again and again
+  for (int n = 0; n < M::kCols; ++n) lse2[n] = (lse_raw[n] == -INFINITY) ? INFINITY : lse_raw[n] * kLog2e;
+  typename M::Start nd = M::start(neg_delta);
+  M::keep(nd);         // registers, not one value moved into an accumulator again and again
 
   f32x16 dq[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) dq[i] = f32x16{0};
-  const PairAddr ad(lds_base, lane);
+  const PairAddr<S::kM> ad(lds_base, lane);
   // the rows arrive before the walk (see dkdv_kernel)
 #pragma unroll
   for (int ks = 0; ks < 8; ++ks) asm volatile("" : "+v"(qf[ks]), "+v"(dof[ks]));
@@ -610,6 +700,7 @@ __device__ __forceinline__ void dq_walk(const BwdParams& given, uint32_t lds_blo
     };
     // (of a list beside the first block, which one group always sees; a group of several may see none of its blocks)
     if (kDense) look_ahead();
+    in.next_step();
     if (!kFirst) in.tile(walk.tile(ent_next), e + 1 < e1);
     wait_vmem_all();
     __syncthreads();            // this stage has landed; everyone is done with the other one, which the copies now fill
@@ -620,7 +711,7 @@ __device__ __forceinline__ void dq_walk(const BwdParams& given, uint32_t lds_blo
     auto block = [&](auto mb_tag) {
       constexpr int kMb = decltype(mb_tag)::value;
       if (!causal || q_block >= nb + kMb)
-        dq_block<kOff + kMb * kBlockPitch, S::kPitch, kCopies>(ad, qf, dof, nd, dq, p.scale_log2, lse2, causal && q_block == nb + kMb,
+        dq_block<S::kM, kOff + kMb * S::kBlockPitch, S::kPitch, kCopies>(ad, qf, dof, nd, dq, p.scale_log2, lse2, causal && q_block == nb + kMb,
                                                                [&](int n) { in.template copy<kStage ^ 1>(kMb * kCopies + n, part_next); },
                                                                [&]() { if (!kDense && kFirst && kMb == 0) look_ahead(); });
     };
@@ -646,10 +737,10 @@ __device__ __forceinline__ void dq_walk(const BwdParams& given, uint32_t lds_blo
   if constexpr (kForm == 4) {
     put_acc(area(group), dq, group);
     __syncthreads();
-    constexpr float kOnes[4] = {1.f, 1.f, 1.f, 1.f};
+    const RowPair kOnes[4] = {both(1.f), both(1.f), both(1.f), both(1.f)};
     f32x16 sum;
-    sum_blocks(sum, dq, group, area, kOnes);
-    store_block(&pl->rows, pl->rows.out0, pl->rows.o0s.b, pl->rows.o0s.s, pl->rows.o0s.h, pl->n_heads, part, b, qrow_out, h, seq_out, group, sum,
+    sum_blocks<S::kM>(sum, dq, group, area, kOnes);
+    store_block<S::kM>(&pl->rows, pl->rows.out0, pl->rows.o0s.b, pl->rows.o0s.s, pl->rows.o0s.h, pl->n_heads, part, b, qrow_out, h, seq_out, group, sum,
                 pl->scale, area(group) + 4096 * group);
   } else {
     uint32_t turn = lds_base + wave * kWaveRowsBytes;                // stage 0: everyone left it before the last step
@@ -659,9 +750,9 @@ __device__ __forceinline__ void dq_walk(const BwdParams& given, uint32_t lds_blo
       __syncthreads();
       if (group) return;
 #pragma unroll
-      for (int mb = 0; mb < 4; ++mb) add_block(turn, mb, dq[mb]);
+      for (int mb = 0; mb < 4; ++mb) add_block<S::kM>(turn, mb, dq[mb], both(1.f), both(1.f));
     }
-    store_result(&pl->rows, pl->rows.out0, pl->rows.o0s.b, pl->rows.o0s.s, pl->rows.o0s.h, pl->n_heads, part, b, qrow_out, h, seq_out, dq, pl->scale,
+    store_result<S::kM>(&pl->rows, pl->rows.out0, pl->rows.o0s.b, pl->rows.o0s.s, pl->rows.o0s.h, pl->n_heads, part, b, qrow_out, h, seq_out, dq, pl->scale,
                  turn);
   }
 }
@@ -737,14 +828,14 @@ static void place(BwdParams& p, int lines) {
 }
 static unsigned row_blocks(const BwdParams& p) { return (unsigned)(p.batch * p.n_heads * p.n_qtiles * p.rows.n_parts); }
 // The form (see Groups) for n lines of 128 rows on both sides of a rectangle that is not causal together (parts counted):
-//  - four groups while half lines leave a CU one workgroup at most (8 heads of 1024: 34 us with one group, 24 with four).
+//  - four groups while half lines leave a CU one workgroup at most (8 heads of 1024: 34 us with one group, 24 with four; one tile 8.7 and 7.5).
 //  - half lines of two groups up to 256 lines: the columns' half lines, which take longer, share the CUs with the rows', and the two
 //    workgroups of a CU are in different phases of their steps (32 heads of 512 23.1 us with one group, in halves 19.8; 42 of 384 21.0 and
 //    18.9).  Beyond, whole lines of one group fill the device as well and copy half as much (44 heads of 384, 264 lines: 21.1, in halves
 //    23.2; 22 of 768 34.3 and 35.7).
 // A causal one's form is chosen with its cut, see bwd_plan.  Tile lists run with one group, as in the forward.
-static int bwd_form(int64_t n, int64_t both_walks) {
-  if (both_walks >= 3 && 2 * n <= kCus) return 4;
+static int bwd_form(int64_t n) {
+  if (2 * n <= kCus) return 4;
   return 2 * n > kCus && n <= kCus ? kHalves : 1;
 }
 static int launch_bwd(BwdParams& p, int form, hipStream_t st) {
@@ -857,7 +948,7 @@ static BwdPlan bwd_plan(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, in
   BwdWalk cols[9], rows[9];
   const int n_cols = sides(cols, max_cols, n_qtiles), n_rows = sides(rows, max_rows, n_ktiles);
   const int n_forms = causal && nbh * (n_ktiles + n_qtiles) <= 3 * kCus ? 3 : 1;
-  if (n_cols * n_rows * n_forms == 1) return {1, 1, causal ? 1 : bwd_form(nbh * ((int64_t)n_ktiles + n_qtiles), (int64_t)n_qtiles + n_ktiles)};
+  if (n_cols * n_rows * n_forms == 1) return {1, 1, causal ? 1 : bwd_form(nbh * ((int64_t)n_ktiles + n_qtiles))};
   const float wk = (float)nbh * n_ktiles, wq = (float)nbh * n_qtiles, tiles = visible_share(n_qtiles, n_ktiles, causal) * wk * n_qtiles;
   BwdPlan best = {1, 1, 1};
   float best_us = INFINITY;
@@ -867,7 +958,7 @@ static BwdPlan bwd_plan(int64_t nbh, int n_qtiles, int n_ktiles, bool causal, in
       const float mb = ((c.n > 1 ? 2.f * c.n * wk : 0.f) + (r.n > 1 ? r.n * wq : 0.f)) * (kTile * kHeadDim * 4 / 1e6f), full = fminf(mb / 8, 2.f);
       const float sum = mb > 0.f ? 1.96f + (c.n > 1 ? 0.7f : 0.f) + (c.n > 1 && r.n > 1 ? 0.58f : 0.f) + mb / 4.34f + 0.31f * full * full : 0.f;
       for (int f = 0; f < n_forms; ++f) {
-        const int form = causal ? kCausalRates[f].form : bwd_form(nbh * ((int64_t)n_ktiles * c.n + (int64_t)n_qtiles * r.n), (int64_t)c.len + r.len);
+        const int form = causal ? kCausalRates[f].form : bwd_form(nbh * ((int64_t)n_ktiles * c.n + (int64_t)n_qtiles * r.n));
         float us = causal ? bwd_causal_us(kCausalRates[f], (float)nbh, n_qtiles, n_ktiles, tiles, c, r)
                           : bwd_us(form, (float)nbh, n_qtiles, n_ktiles, c, r) * (mb > 0.f ? 1.035f : 1.f);
         us += sum;

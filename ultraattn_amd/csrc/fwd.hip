@@ -6,11 +6,10 @@
 // being consumed.  Each wavefront owns 32 query rows and computes the TRANSPOSED products
 //     S^T[key, q] = K Q^T      (A = K fragment from LDS, B = Q fragment held in registers)
 //     O^T[d,  q] += V^T P^T    (A = V^T fragment via transposing LDS reads, B = P^T)
-// with v_mfma_f32_32x32x16_bf16.  In the 32x32 accumulator layout a lane holds ONE query
-// column (lane % 32) and 16 rows, so the online-softmax statistics of a query row live in one
-// lane (mirrored in lane ^ 32): the row max needs a single cross-half exchange, the rescale of
-// O^T is lane local, and S^T's accumulator registers are, after exp2 and bf16 packing, exactly
-// the B operand of the second product.
+// In the accumulator layout (see Mma) a lane holds one query column, or one of each block of 16, so the online-softmax
+// statistics of a query row live in one lane and its mirrors: the row max needs an exchange over those alone, the rescale of
+// O^T is lane local, and S^T's accumulator registers are, after exp2 and bf16 packing, exactly the B operand of the second
+// product.
 #include <algorithm>
 #include <type_traits>
 #include "ua_common.h"
@@ -37,6 +36,14 @@ struct FwdParams {
   int64_t o_part, lse_part;
 };
 
+// The kernel's parameters read again from the kernel-argument segment.
+typedef const __attribute__((address_space(4))) FwdParams* ParamsLate;
+__device__ __forceinline__ ParamsLate params_late() {
+  ParamsLate p = (ParamsLate)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return p;
+}
+
 // P is computed against the row's current reference max without looking at the new scores'
 // max; only when a block's row sum shows that some score exceeded the reference by more than
 // ~2^kRaiseLog2 is the reference raised (and O, l rescaled, P recomputed).  O/l stay exact
@@ -46,105 +53,114 @@ constexpr float kRaiseSum = 16777216.f;     // 2^24
 struct SoftmaxState {
   float m_run = -INFINITY;   // reference max of the row (log2 domain, scaled)
   float m_use = 0.f;         // m_run, or 0 while the row has not seen a visible key
-  float l_run = 0.f;         // this half-wave's partial row sum
+  float l_run = 0.f;         // this lane's partial row sum
 };
 
 // kB blocks of 32 keys for this wave's 32 query rows.  With `mask` (wave-uniform) keys beyond
 // the query's own tile-local index are hidden; `key0` = tile-local index of the first key.
 // kCopies: `copy(n)`, n = 0 .. 7, is called between the MFMAs of S; `side()` beside the softmax.
-template <int kB, bool kCopies, class Copy, class Side>
+template <int kM, int kB, bool kCopies, class Copy, class Side>
 __device__ __forceinline__ void key_blocks(const unsigned char* sK, const unsigned char* sV, const bf16x8 (&qf)[8],
-                                          f32x16 (&oacc)[4], SoftmaxState& st, const TrLane& tr, float scale_log2,
-                                          int l32, int hi, int q_block, int key0, bool mask, bool first, Copy copy, Side side) {
+                                          f32x16 (&oacc)[4], SoftmaxState (&st)[2], const int (&nat)[Mma<kM>::kRowRegs], const int (&tr)[4], float scale_log2,
+                                          int q_block, int key0, bool mask, bool first, Copy copy, Side side) {
+  using M = Mma<kM>;
   // ---- S^T = K Q^T : kB blocks of 32 keys x 32 queries -----------------------------------
-  // The 8 * kB K fragments are fetched kAhead reads ahead of the MFMA that consumes them, so the
-  // LDS latency is covered by the preceding MFMAs instead of being paid before each one.
+  // The 8 * kB K fragments are fetched kAhead reads ahead of the MFMAs that consume them, so the
+  // LDS latency is covered by the preceding MFMAs instead of being paid before each pair.
   f32x16 s[kB];
-#pragma unroll
-  for (int mb = 0; mb < kB; ++mb) s[mb] = f32x16{0};
   {
-    constexpr int kAhead = 4;
+    constexpr int kAhead = kM == 16 ? 3 : 4;
+    constexpr int kParts = kM == 16 ? 2 : 1;                  // fragments of a block's rows, taken in turn with those of the other blocks
     bf16x8 kfr[8 * kB];
+    auto frag = [](int i) { return i / (kParts * kB) * kParts + i % kParts; };
+    auto block = [](int i) { return i / kParts % kB; };
+    auto rd = [&](int i) {
+      return lds_read_b128(sK, nat[M::a_reg(frag(i))] + M::a_offset(frag(i), 4 * kRowBytes) + 32 * kRowBytes * block(i));
+    };
 #pragma unroll
-    for (int i = 0; i < kAhead; ++i) kfr[i] = lds_read_b128(sK, lds_off_k(32 * (i % kB) + l32, 2 * (i / kB) + hi));
+    for (int i = 0; i < kAhead; ++i) kfr[i] = rd(i);
     __builtin_amdgcn_sched_group_barrier(0x100, kAhead, 0);   // kAhead LDS reads up front
 #pragma unroll
     for (int i = 0; i < 8 * kB; ++i) {
-      if (i + kAhead < 8 * kB) {
-        const int j = i + kAhead;
-        kfr[j] = lds_read_b128(sK, lds_off_k(32 * (j % kB) + l32, 2 * (j / kB) + hi));
-      }
-      s[i % kB] = mfma32(kfr[i], qf[i / kB], s[i % kB]);
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // then 1 MFMA, 1 LDS read, ...
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      if (i + kAhead < 8 * kB) kfr[i + kAhead] = rd(i + kAhead);
+      M::first(s[block(i)], frag(i), kfr[i], qf, M::start({0.f, 0.f}));
+      M::template interleave<1>();                              // then the fragment's MFMAs and 1 LDS read, ...
       if (kCopies && (i + 1) % kB == 0) copy(i / kB);
     }
   }
-  // element (mb, i) of this lane: key key0 + 32*mb + 8*(i/4) + 4*hi + i%4, query 32 * q_block + lane%32 of the tile
+  // element (mb, i) of this lane: key key0 + 32 * mb + quad_row + i % 4, query 32 * q_block + col of the tile
   if (mask) {
-    const int lane = fresh_lane(), q_local = 32 * q_block + (lane & 31), hi4 = 4 * (lane >> 5);
+    const int lane = fresh_lane(), ahead = key0 + M::quad_row(lane, 0) - 32 * q_block - M::col(lane, 0);
 #pragma unroll
     for (int mb = 0; mb < kB; ++mb)
 #pragma unroll
       for (int i = 0; i < 16; ++i)
-        if (key0 + 32 * mb + 8 * (i >> 2) + hi4 + (i & 3) > q_local) s[mb][i] = -INFINITY;
+        if (ahead + 32 * mb + M::quad_row(0, i >> 2) + (i & 3) > M::col(0, M::quad_n(i >> 2))) s[mb][i] = -INFINITY;
   }
   // the first V^T fragments are fetched now: their latency hides behind the softmax
   constexpr int kVAhead = 3;
   bf16x8 vfr[4];
+  auto rd_v = [&](int i) {               // fragment i % 8 of 32 keys
+    const int at = tr[M::tr_reg(i & 7)] + M::tr_first(i & 7) + 8 * M::kPitch * (i >> 3);
+    const bf16x4 lo = lds_read_tr16_b64(sV, at), hi = lds_read_tr16_b64(sV, at + M::kTrSecond);
+    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  };
 #pragma unroll
-  for (int i = 0; i < kVAhead; ++i) vfr[i] = lds_read_tr_frag<lds_off_v>(sV, tr, 16 * (i >> 2), i & 3);
+  for (int i = 0; i < kVAhead; ++i) vfr[i] = rd_v(i);
   side();
   // ---- online softmax (fp32, log2 domain) ---------------------------------------------------
-  float rs = 0.f;
-  bf16x8 pf[2 * kB];
+  float rs[2];
+  bf16x8 pf[kB][2];
+  auto exponentials = [&]() {
+    rs[0] = rs[1] = 0.f;
+#pragma unroll
+    for (int mb = 0; mb < kB; ++mb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int n = M::quad_n(i >> 2);
+        const float pv = fast_exp2(fmaf(s[mb][i], scale_log2, -st[n].m_use));
+        rs[n] += pv;
+        pf[mb][M::slot_n(i)][M::slot_j(i)] = (bf16)pv;
+      }
+  };
   bool raise = first;
   if (!first) {
-#pragma unroll
-    for (int mb = 0; mb < kB; ++mb)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const float pv = fast_exp2(fmaf(s[mb][i], scale_log2, -st.m_use));
-        rs += pv;
-        pf[mb * 2 + (i >> 3)][i & 7] = (bf16)pv;
-      }
-    raise = __builtin_amdgcn_ballot_w64(!(rs < kRaiseSum)) != 0;       // wave-uniform, rare
+    exponentials();
+    raise = __builtin_amdgcn_ballot_w64(!((M::kCols == 2 ? rs[0] + rs[1] : rs[0]) < kRaiseSum)) != 0;       // wave-uniform, rare
   }
   if (raise) {
-    float mx = -INFINITY;
 #pragma unroll
-    for (int i = 0; i < 16; ++i)
+    for (int n = 0; n < M::kCols; ++n) {
+      SoftmaxState& t = st[n];
+      float mx = -INFINITY;
 #pragma unroll
-      for (int mb = 0; mb < kB; ++mb) mx = fmaxf(mx, s[mb][i]);
-    mx = xhalf_max(mx) * scale_log2;
-    const float m_new = fmaxf(st.m_run, mx);
-    const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
-    const float alpha = (m_new == st.m_run) ? 1.f : fast_exp2(st.m_run - m_use);      // m_run = -inf -> 0
-    st.m_run = m_new;
-    st.m_use = m_use;
-    st.l_run *= alpha;
+      for (int i = 0; i < 16; ++i)
 #pragma unroll
-    for (int mbd = 0; mbd < 4; ++mbd)
+        for (int mb = 0; mb < kB; ++mb)
+          if (M::quad_n(i >> 2) == n) mx = fmaxf(mx, s[mb][i]);
+      mx = M::column_max(mx) * scale_log2;
+      const float m_new = fmaxf(t.m_run, mx);
+      const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
+      const float alpha = (m_new == t.m_run) ? 1.f : fast_exp2(t.m_run - m_use);      // m_run = -inf -> 0
+      t.m_run = m_new;
+      t.m_use = m_use;
+      t.l_run *= alpha;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) oacc[mbd][i] *= alpha;
-    rs = 0.f;
+      for (int mbd = 0; mbd < 4; ++mbd)
 #pragma unroll
-    for (int mb = 0; mb < kB; ++mb)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const float pv = fast_exp2(fmaf(s[mb][i], scale_log2, -m_use));
-        rs += pv;
-        pf[mb * 2 + (i >> 3)][i & 7] = (bf16)pv;
-      }
+        for (int i = 0; i < 16; ++i)
+          if (M::quad_n(i >> 2) == n) oacc[mbd][i] *= alpha;
+    }
+    exponentials();
   }
-  st.l_run += rs;
-  // ---- O^T += V^T P^T : 4 blocks of 32 d x 32 queries, 2 * kB steps of 16 keys -------------------
+#pragma unroll
+  for (int n = 0; n < M::kCols; ++n) st[n].l_run += rs[n];
+  // ---- O^T += V^T P^T : 128 d x 32 queries, kB steps of 32 keys --------------------------------
 #pragma unroll
   for (int i = 0; i < 8 * kB; ++i) {
-    if (i + kVAhead < 8 * kB) vfr[(i + kVAhead) & 3] = lds_read_tr_frag<lds_off_v>(sV, tr, 16 * ((i + kVAhead) >> 2), (i + kVAhead) & 3);
-    oacc[i & 3] = mfma32(vfr[i & 3], pf[i >> 2], oacc[i & 3]);
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // 1 MFMA
-    __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);   // 2 LDS reads (one fragment)
+    if (i + kVAhead < 8 * kB) vfr[(i + kVAhead) & 3] = rd_v(i + kVAhead);
+    M::second(oacc, i & 7, vfr[i & 3], pf[i >> 3]);
+    M::template interleave<2>();                              // MFMAs and 2 LDS reads of one fragment
   }
 }
 
@@ -152,16 +168,17 @@ __device__ __forceinline__ void key_blocks(const unsigned char* sK, const unsign
 // are combined through LDS.  A launch that gives a CU one workgroup of four waves at most runs it at
 // one wave per SIMD, where a half tile takes 1.2 us of which the matrix pipe is busy 0.4; with more groups the CU is
 // as full as with two workgroups, without partial results in memory.
-template <int kForm, bool kDense>
+template <int kForm, bool kDense, int kM>
 __global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void fwd_kernel(const FwdParams p) {
+  using M = Mma<kM>;
   constexpr int kWaves = Groups<kForm>::kWaves, kRows = Groups<kForm>::kRows, kLines = Groups<kForm>::kLines;
-  constexpr int kStageBytes = kRows * kRowBytes;
+  constexpr int kStageBytes = kRows * kRowBytes, kStageV = kRows / 4 * M::kPitch;
   // two pipeline stages per group, distinct arrays so that reads of one stage need not wait for the
   // copies in flight into the other
   __shared__ __attribute__((aligned(1024))) unsigned char sKA[kForm * kStageBytes];
-  __shared__ __attribute__((aligned(1024))) unsigned char sVA[kForm * kStageBytes];
+  __shared__ __attribute__((aligned(1024))) unsigned char sVA[kForm * kStageV];
   __shared__ __attribute__((aligned(1024))) unsigned char sKB[kForm * kStageBytes];
-  __shared__ __attribute__((aligned(1024))) unsigned char sVB[kForm * kStageBytes];
+  __shared__ __attribute__((aligned(1024))) unsigned char sVB[kForm * kStageV];
   // With four groups the query rows have room of their own: the first step's copies need not wait for everyone's reads of them
   // (with the step's barrier at its end: two causal tiles 6.4 -> 6.25 us, 8 heads of 1024 12.75 -> 12.5).
   constexpr bool kOwnQ = kForm == 4;
@@ -171,9 +188,8 @@ __global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void fwd_kernel(const F
   const int wave_in_block = __builtin_amdgcn_readfirstlane(tid >> 6);
   // (group a constant for one group: the stages' addresses then are constants too, ten additions fewer per tile)
   const int wave = kForm == 1 ? wave_in_block : wave_in_block % kWaves, group = kForm == 1 ? 0 : wave_in_block / kWaves;
-  unsigned char *const kA = sKA + group * kStageBytes, *const vA = sVA + group * kStageBytes;
-  unsigned char *const kB = sKB + group * kStageBytes, *const vB = sVB + group * kStageBytes;
-  const int l32 = lane & 31, hi = lane >> 5;
+  unsigned char *const kA = sKA + group * kStageBytes, *const vA = sVA + group * kStageV;
+  unsigned char *const kB = sKB + group * kStageBytes, *const vB = sVB + group * kStageV;
   int pos, bh;
   map_block(blockIdx.x, p.map, pos, bh);
   const int sub = pos & (kLines - 1);      // which half of the tile's rows
@@ -202,8 +218,8 @@ __global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void fwd_kernel(const F
   const bf16* vbase = p.v + b * p.vs.b + h * p.vs.h;
   const int k_stride = (int)p.ks.s, v_stride = (int)p.vs.s;
   int koff[4], voff[4];
-  dma_voffsets<lds_off_k, kWaves>(koff, k_stride, wave, lane);
-  dma_voffsets<lds_off_v, kWaves>(voff, v_stride, wave, lane);
+  dma_voffsets<slot_k, kWaves>(koff, k_stride, wave, lane);
+  dma_voffsets<slot_v, kWaves>(voff, v_stride, wave, lane);
   const int k_half = kRows * k_stride * 2, v_half = kRows * v_stride * 2;                 // bytes of one stage in memory
   const uint32_t k_extent = (uint32_t)((kTile - 1) * k_stride + kHeadDim) * 2;            // bytes of one tile
   const uint32_t v_extent = (uint32_t)((kTile - 1) * v_stride + kHeadDim) * 2;
@@ -216,14 +232,17 @@ __global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void fwd_kernel(const F
     k_rsrc = make_rsrc_words(kbase + (int64_t)t * kTile * k_stride, more ? k_extent : 0);
     v_rsrc = make_rsrc_words(vbase + (int64_t)t * kTile * v_stride, more ? v_extent : 0);
   };
+  // Where the wave's copies land in a stage; made opaque in every step, as the sums with the stages' addresses would occupy scalar
+  // registers all along (and 15 to 24 of those vector lanes).
+  int k_wave = wave * 1024, v_wave = wave * M::kPitch;
   auto copy_piece = [&](int n, unsigned char* k_stage, unsigned char* v_stage, int part) {
     const int j = n >> 1;                  // (the offsets of pieces 16 rows apart differ by that alone: one register each for K and V)
-    if (n & 1) dma16_abs(v_rsrc, lds_at(v_stage) + (4 * j + wave) * 1024, voff[0], part * v_half + j * 32 * v_stride);
-    else       dma16_abs(k_rsrc, lds_at(k_stage) + (4 * j + wave) * 1024, koff[0], part * k_half + j * 32 * k_stride);
+    if (n & 1) dma16_abs(v_rsrc, lds_at(v_stage) + 4 * M::kPitch * j + v_wave, voff[0], part * v_half + j * 32 * v_stride);
+    else       dma16_abs(k_rsrc, lds_at(k_stage) + 4096 * j + k_wave, koff[0], part * k_half + j * 32 * k_stride);
   };
   auto copy_stage = [&](int t, unsigned char* k_stage, unsigned char* v_stage, int part) {
-    dma_rows_buf<kWaves>(k_stage, make_rsrc(kbase + (int64_t)t * kTile * k_stride, k_extent), koff, part * k_half, wave);
-    dma_rows_buf<kWaves>(v_stage, make_rsrc(vbase + (int64_t)t * kTile * v_stride, v_extent), voff, part * v_half, wave);
+    dma_rows_buf<kWaves, 1024>(k_stage, make_rsrc(kbase + (int64_t)t * kTile * k_stride, k_extent), koff, part * k_half, wave);
+    dma_rows_buf<kWaves, M::kPitch>(v_stage, make_rsrc(vbase + (int64_t)t * kTile * v_stride, v_extent), voff, part * v_half, wave);
   };
 
   // A step is one half of a tile, in order; with more groups half or quarter `group` of a tile.
@@ -243,8 +262,7 @@ __global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void fwd_kernel(const F
     }
   }
 
-  // Q fragment (B operand of S^T): lane holds query row 32*q_block + lane%32,
-  // d = 16*ks + 8*(lane/32) .. +7 for ks = 0..7.
+  // Q fragments (B operands of S^T)
   // (through the stage that the first step fills)
   const int q_block = kWaves * sub + wave;
   const int qrow0 = qt * kTile + q_block * 32;
@@ -252,13 +270,13 @@ __global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void fwd_kernel(const F
   if constexpr (kForm == 1) {
     u32x4 raw[8];
     load_rows(raw, p.q + b * p.qs.b + (int64_t)qrow0 * p.qs.s + h * p.qs.h, p.qs.s);
-    rows_to_frags(qf, raw, (uint32_t)(uintptr_t)(lds_byte*)((wave < 2 ? kB : vB) + (wave & 1) * kWaveRowsBytes));
+    rows_to_frags<kM>(qf, raw, (uint32_t)(uintptr_t)(lds_byte*)((wave < 2 ? kB : vB) + (wave & 1) * kWaveRowsBytes));
   } else {
     const uint32_t q_lds = lds_at(kOwnQ ? sQ : sKB);
     copy_shared_rows<32 * kWaves>(p.q + b * p.qs.b + ((int64_t)qt * kTile + sub * 32 * kWaves) * p.qs.s + h * p.qs.h, (int)p.qs.s, q_lds);
     wait_vmem_all();
     __syncthreads();
-    shared_rows_to_frags(qf, q_lds, wave);
+    shared_rows_to_frags<kM>(qf, q_lds, wave);
     if (!kOwnQ) __syncthreads();
   }
 #pragma unroll
@@ -267,8 +285,12 @@ __global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void fwd_kernel(const F
   f32x16 oacc[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) oacc[i] = f32x16{0};
-  SoftmaxState st;
-  const TrLane tr(lane);
+  SoftmaxState st[2];                      // of the lane's queries
+  int nat[M::kRowRegs], tr[4];             // row reads of K, transposing reads of V
+#pragma unroll
+  for (int i = 0; i < M::kRowRegs; ++i) nat[i] = lds_off_k(M::a_row(lane), M::a_chunk(lane, i));
+#pragma unroll
+  for (int i = 0; i < 4; ++i) tr[i] = M::tr_offset(lane, i);
 
   bool started = false;
   auto step = [&](int e, auto stage_tag) {
@@ -286,7 +308,10 @@ __global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void fwd_kernel(const F
       wait_vmem_all();
       __syncthreads();
     };
-    if (kForm == 1) landed();
+    if (kForm == 1) {
+      asm volatile("" : "+s"(k_wave), "+s"(v_wave));
+      landed();
+    }
     unsigned char *const k_other = kStage ? kA : kB, *const v_other = kStage ? vA : vB;
     if (kForm > 1 && e + 1 < e1) copy_stage(walk.tile(ent_next), k_other, v_other, group);
     auto copy = [&](int n) { copy_piece(n, k_other, v_other, kStage ^ 1); };
@@ -294,7 +319,7 @@ __global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void fwd_kernel(const F
     const int half = kForm == 1 ? kStage : group;
     const bool causal = (ent >> 30) != 0;
     if (!causal || kBlocks * half <= q_block) {
-      key_blocks<kBlocks, kForm == 1>(kStage ? kB : kA, kStage ? vB : vA, qf, oacc, st, tr, p.scale_log2, l32, hi, q_block, kRows * half,
+      key_blocks<kM, kBlocks, kForm == 1>(kStage ? kB : kA, kStage ? vB : vA, qf, oacc, st, nat, tr, p.scale_log2, q_block, kRows * half,
                                         causal && q_block < kBlocks * half + kBlocks, kForm == 1 ? kStage == 0 && e == e0 : !started, copy,
                                         [&]() { if (kFirst) look_ahead(); });
       started = true;
@@ -320,60 +345,78 @@ __global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void fwd_kernel(const F
   }
 
   // ---- epilogue: normalise, write O (bf16) and LSE (natural log) -------------------------
-  float l_tot = xhalf_sum(st.l_run);
-  bf16* orow = p.o + b * p.os.b + (int64_t)qrow0 * p.os.s + h * p.os.h;
-  float* lrow = p.lse + ((int64_t)b * p.n_heads + h) * ((int64_t)p.n_qtiles * kTile) + qrow0;
-  int64_t o_stride = p.os.s;
+  float l_tot[2];
+#pragma unroll
+  for (int n = 0; n < M::kCols; ++n) l_tot[n] = M::column_sum(st[n].l_run);
+  auto inverse = [&]() {
+    RowPair r;
+#pragma unroll
+    for (int n = 0; n < M::kCols; ++n) r.x[n] = l_tot[n] > 0.f ? 1.f / l_tot[n] : 0.f;
+    return r;
+  };
+  // (what only the end needs is read from the kernel-argument segment now: it would occupy scalar registers during a long walk)
+  const FwdParams& pe = kForm == 1 ? *(const FwdParams*)params_late() : p;
+  bf16* orow = pe.o + b * pe.os.b + (int64_t)qrow0 * pe.os.s + h * pe.os.h;
+  float* lrow = pe.lse + ((int64_t)b * pe.n_heads + h) * ((int64_t)pe.n_qtiles * kTile) + qrow0;
+  int64_t o_stride = pe.os.s;
   int64_t part_at = 0;                     // element of the partial O
   if (part >= 0) {
-    const int64_t seq = (int64_t)(p.n_qtiles - p.n_whole) * kTile, row = qrow0 - (int64_t)p.n_whole * kTile;
-    part_at = part * p.o_part + ((b * seq + row) * p.n_heads + h) * kHeadDim;
-    orow = static_cast<bf16*>(p.part_o) + part_at;
-    lrow = p.part_lse + part * p.lse_part + ((int64_t)b * p.n_heads + h) * seq + row;
-    o_stride = (int64_t)p.n_heads * kHeadDim;
+    const int64_t seq = (int64_t)(pe.n_qtiles - pe.n_whole) * kTile, row = qrow0 - (int64_t)pe.n_whole * kTile;
+    part_at = part * pe.o_part + ((b * seq + row) * pe.n_heads + h) * kHeadDim;
+    orow = static_cast<bf16*>(pe.part_o) + part_at;
+    lrow = pe.part_lse + part * pe.lse_part + ((int64_t)b * pe.n_heads + h) * seq + row;
+    o_stride = (int64_t)pe.n_heads * kHeadDim;
   }
   if constexpr (kForm == 1) {
-    const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+    const RowPair inv = inverse();
     const uint32_t turn = lds_at((wave < 2 ? kA : vA) + (wave & 1) * kWaveRowsBytes);
-    if (part >= 0 && p.part_f32)    store_rows_f32(static_cast<float*>(p.part_o) + part_at, o_stride, oacc, inv, turn);
-    else                            store_rows_bf16(orow, o_stride, oacc, inv, turn);
+    if (part >= 0 && pe.part_f32)   store_rows_f32<kM>(static_cast<float*>(pe.part_o) + part_at, o_stride, oacc, inv, turn);
+    else                            store_rows_bf16<kM>(orow, o_stride, oacc, inv, turn);
   } else {
     // the groups exchange their rows' max, sum and O.  Area x of the stages' LDS belongs to group x % kForm of wave x / kForm.
-    __shared__ float stat[8][2][64];
+    __shared__ float stat[8][M::kCols][2][64];
     auto area = [&](int x) { return lds_at(x < 2 ? sKA : x < 4 ? sVA : x < 6 ? sKB : sVB) + (x & 1) * kAccBytes; };
     const int own = wave * kForm + group;
     constexpr bool kAll = kForm == 2;        // the first group finishes whole rows; with four groups each a block of 32 columns
-    stat[own][0][lane] = st.m_run;
-    stat[own][1][lane] = l_tot;
+#pragma unroll
+    for (int n = 0; n < M::kCols; ++n) {
+      stat[own][n][0][lane] = st[n].m_run;
+      stat[own][n][1][lane] = l_tot[n];
+    }
     if (!kAll || group == 1) put_acc(area(own), oacc, kAll ? -1 : group);
     __syncthreads();
     if (kAll && group == 1) return;
-    float m = -INFINITY, w[kForm];
+    RowPair w[kForm];
 #pragma unroll
-    for (int g = 0; g < kForm; ++g) m = fmaxf(m, stat[wave * kForm + g][0][lane]);
-    const float ms = m == -INFINITY ? 0.f : m;
-    l_tot = 0.f;
+    for (int n = 0; n < M::kCols; ++n) {
+      float m = -INFINITY;
 #pragma unroll
-    for (int g = 0; g < kForm; ++g) {
-      w[g] = fast_exp2(stat[wave * kForm + g][0][lane] - ms);
-      l_tot += stat[wave * kForm + g][1][lane] * w[g];
+      for (int g = 0; g < kForm; ++g) m = fmaxf(m, stat[wave * kForm + g][n][0][lane]);
+      const float ms = m == -INFINITY ? 0.f : m;
+      l_tot[n] = 0.f;
+#pragma unroll
+      for (int g = 0; g < kForm; ++g) {
+        w[g].x[n] = fast_exp2(stat[wave * kForm + g][n][0][lane] - ms);
+        l_tot[n] += stat[wave * kForm + g][n][1][lane] * w[g].x[n];
+      }
+      st[n].m_run = m;
     }
-    st.m_run = m;
-    const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+    const RowPair inv = inverse();
     if constexpr (kAll) {
 #pragma unroll
-      for (int mb = 0; mb < 4; ++mb) add_block(area(own + 1), mb, oacc[mb], w[0], w[1]);
-      store_rows_bf16(orow, o_stride, oacc, inv, area(own + 1));
+      for (int mb = 0; mb < 4; ++mb) add_block<kM>(area(own + 1), mb, oacc[mb], w[0], w[1]);
+      store_rows_bf16<kM>(orow, o_stride, oacc, inv, area(own + 1));
     } else {
       f32x16 o;
-      sum_blocks(o, oacc, group, [&](int g) { return area(wave * kForm + g); }, w);
-      store_block_bf16(orow + 32 * group, o_stride, o, inv, area(own) + 4096 * group);
+      sum_blocks<kM>(o, oacc, group, [&](int g) { return area(wave * kForm + g); }, w);
+      store_block_bf16<kM>(orow + 32 * group, o_stride, o, inv, area(own) + 4096 * group);
     }
   }
   const int out_lane = fresh_lane();
   if (out_lane < 32 && group == 0) {
-    const float lse = l_tot > 0.f ? (st.m_run + __builtin_amdgcn_logf(l_tot)) * kLn2 : -INFINITY;
-    lrow[out_lane] = lse;
+    const bool second = M::kCols == 2 && out_lane >= 16;
+    const float l = l_tot[second ? 1 : 0], m = st[second ? 1 : 0].m_run;
+    lrow[out_lane] = l > 0.f ? (m + __builtin_amdgcn_logf(l)) * kLn2 : -INFINITY;
   }
 }
 
@@ -408,7 +451,7 @@ static int fwd_common(FwdParams& p, const void* q, const void* k, const void* v,
 
 // Groups per workgroup for n lines of 128 rows (parts counted) of a dense rectangle:
 //  - four, on half lines, while those leave a CU one workgroup at most (8 heads of 1024: 17.2 us with two groups, 13.8
-//    with four; 2048: 29.9, 24.3).  A walk of one tile is not worth the handing over at its end (6.1 us, one group 5.7).
+//    with four; 2048: 29.9, 24.3; walks of one tile 5.7 and 5.5, causal 6.1 and 5.5).
 //  - two, on whole lines, up to one workgroup per CU and from three tiles on (32 heads of 1024: 25 us with one, 22 with two).
 //  - The rows of an uncut causal rectangle differ in length.  Run one after the other, longest first, they are
 //    balanced, which workgroups resident side by side from the start do not achieve: four groups up to 256 lines of 16
@@ -420,7 +463,7 @@ static int fwd_common(FwdParams& p, const void* q, const void* k, const void* v,
 // head, causal 4096: forward 35 us with four groups, 58 with one, backward 51 and 119; from 512 lines on little changes).
 static int fwd_groups(int64_t n, int64_t walk, int n_parts, bool dense_causal) {
   const bool uneven = dense_causal && n_parts == 1;
-  if (walk >= 2 && (2 * n <= kCus || (uneven && n <= kCus && walk >= 16))) return 4;
+  if (2 * n <= kCus || (uneven && n <= kCus && walk >= 16)) return 4;
   return walk >= 3 && n <= (uneven ? 2 * kCus : kCus) ? 2 : 1;
 }
 // `plain`: one group per workgroup.
@@ -429,19 +472,29 @@ static int fwd_launch(FwdParams& p, bool plain, hipStream_t st) {
   // (several groups copy Q through a buffer descriptor, whose offsets have 32 bits)
   const int form = plain || p.qs.s > (INT32_MAX >> 9) ? 1 : fwd_groups(n, p.part_len, p.n_parts, p.dense_causal);
   const int n_cut = p.n_qtiles - p.n_whole;
+  // Several groups a line: 32x32x16 for launches of less than 8 visible tiles a CU, whose few steps end before the larger instruction count
+  // of 16x16x32 is made up for (32 heads of 512 9.44 us, with 16x16x32 9.63; 16 of 1024 14.3, 14.5; causal 32 of 1024 18.75, 18.9), the other way
+  // from there on (32 heads of 1024 21.8 and 21.1; 8 of 4096 66.6, 63.1; causal 16 of 3072 47.9, 45.8).
+  const bool wide = visible_share(p.n_qtiles, p.n_ktiles, p.dense_causal) * p.batch * p.n_heads * p.n_qtiles * p.n_ktiles < 8.f * kCus;
   p.map = block_map(p.batch * p.n_heads, (p.n_whole + n_cut * p.n_parts) * (form == 4 ? 2 : 1));
   p.by_heads = make_div(p.n_heads);
   p.by_cut = make_div(n_cut ? n_cut : 1);
   switch (form) {
-    case 4: hipLaunchKernelGGL((fwd_kernel<4, true>), dim3(2 * n), dim3(512), 0, st, p); break;
-    case 2: hipLaunchKernelGGL((fwd_kernel<2, true>), dim3(n), dim3(512), 0, st, p); break;
+    case 4:
+      if (wide) hipLaunchKernelGGL((fwd_kernel<4, true, 32>), dim3(2 * n), dim3(512), 0, st, p);
+      else      hipLaunchKernelGGL((fwd_kernel<4, true, 16>), dim3(2 * n), dim3(512), 0, st, p);
+      break;
+    case 2:
+      if (wide) hipLaunchKernelGGL((fwd_kernel<2, true, 32>), dim3(n), dim3(512), 0, st, p);
+      else      hipLaunchKernelGGL((fwd_kernel<2, true, 16>), dim3(n), dim3(512), 0, st, p);
+      break;
     default:
       // Up to two workgroups per CU the whole launch is resident at once, and those after the first 256 join them in
       // launch order.  Lists come roughly by falling length, so the first ones are taken in reverse: long and
       // short lists then share a CU (strided 8k, 8 heads: the longest sum on a CU 40 -> 37 tiles, causal 96 -> 65).
       if (!p.dense && n > kCus && n <= 2 * kCus) p.n_first = kCus * p.n_qtiles / (int)n;
-      if (p.dense) hipLaunchKernelGGL((fwd_kernel<1, true>), dim3(n), dim3(256), 0, st, p);
-      else         hipLaunchKernelGGL((fwd_kernel<1, false>), dim3(n), dim3(256), 0, st, p);
+      if (p.dense) hipLaunchKernelGGL((fwd_kernel<1, true, 16>), dim3(n), dim3(256), 0, st, p);
+      else         hipLaunchKernelGGL((fwd_kernel<1, false, 16>), dim3(n), dim3(256), 0, st, p);
   }
   return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH;
 }

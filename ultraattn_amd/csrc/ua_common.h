@@ -28,9 +28,10 @@ struct Strides3 { int64_t b, s, h; };   // element strides of (batch, token, hea
 // K-type layout: chunk index XOR (row mod 16): 16 consecutive rows at one logical column
 // land in 16 different 16-byte slots, so 128-bit row-fragment reads are conflict free.
 __device__ __forceinline__ int lds_off_k(int r, int c) { return r * kRowBytes + ((c ^ (r & 15)) << 4); }
-// V-type layout: 64-byte group index XOR (row mod 4): the 4 consecutive rows that one
-// transposing 64-bit read gathers land in 4 different bank groups.
-__device__ __forceinline__ int lds_off_v(int r, int c) { return r * kRowBytes + ((c ^ ((r & 3) << 2)) << 4); }
+// V-type layout: fours of rows (1 KiB each, one copy of one wave) lie at a pitch of 1 KiB and a bit (Mma::kPitch), and the 64-byte
+// group index is XORed with row mod 4, so that 128-bit reads of rows and transposing reads are free of bank conflicts.
+__device__ __forceinline__ int slot_v(int r, int c) { return c ^ ((r & 3) << 2); }
+__device__ __forceinline__ int slot_k(int r, int c) { return c ^ (r & 15); }
 
 __device__ __forceinline__ bf16x8 lds_read_b128(const unsigned char* smem, int off) {
   return *reinterpret_cast<const bf16x8*>(smem + off);
@@ -42,42 +43,160 @@ __device__ __forceinline__ bf16x4 lds_read_tr16_b64(const unsigned char* smem, i
   return __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(smem + off));
 }
 
-__device__ __forceinline__ float xhalf_max(float x) {   // max over lane l and lane l^32
-  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float xhalf_sum(float x) {   // sum over lane l and lane l^32
-  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+template <int kLanes>                       // 16 or 32: with lane l ^ kLanes
+__device__ __forceinline__ void swap_lanes(float x, float& a, float& b) {
+  const uint32_t u = __float_as_uint(x);
+  const auto r = kLanes == 16 ? __builtin_amdgcn_permlane16_swap(u, u, false, false) : __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  a = __uint_as_float(r[0]);
+  b = __uint_as_float(r[1]);
 }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
-__device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-}
-
-// Per-lane constants of the transposing reads that build an A operand of X^T from a
-// row-major tile X[row][col] in LDS: the MFMA row index is the tile column
-// (32*mb + lane%32), the contraction index runs over tile rows.  For a 16-row step starting
-// at row0, lane half hi = lane/32 supplies contraction slots j = 0..7 = tile rows
-// row0 + 8*(j/4) + 4*hi + j%4, the same slots that a 32x32 accumulator block hands to the
-// next product when it is reused as the B operand.
-struct TrLane {
-  int row_in, chunk_in, sub;
-  __device__ __forceinline__ explicit TrLane(int lane) {
-    const int i16 = lane & 15, grp = (lane >> 4) & 1, hi = lane >> 5;
-    row_in = (i16 >> 2) + 4 * hi;
-    chunk_in = 2 * grp + ((i16 & 3) >> 1);
-    sub = (i16 & 1) * 8;
+// ---- the matrix instruction of a walk: v_mfma_f32_16x16x32_bf16 or v_mfma_f32_32x32x16_bf16 -----------------------
+// Both work on blocks of 32 x 32: acc[i] of a lane = row quad_row(i / 4) + i % 4, column col(quad_n(i / 4)).  The transposed products of the
+// walks turn a block's accumulators, packed to bf16, into the B operand of the next product without leaving the lane.
+//
+// On random operands, at the socket's power limit, a loop of 16x16x32 instructions that uses every A operand twice runs at 2.06
+// PFLOP/s, one of 32x32x16 at 1.75 (its accumulators take twice the register traffic a flop).  The long launches, which that
+// limit holds, gain 3 to 5 % in the forward (causal 32k, 32 heads 7.16 -> 6.85 ms, strided 128k 17.7 -> 17.1) and 7 to 8 % in the
+// backward (23.5 -> 21.7, 57.8 -> 53.6), at 1.81 and 1.87 instead of 1.60 GHz.  But there are twice as many instructions to
+// issue: beside a wave that issues them another one's fma, exp2 and add take 28 cycles instead of 22, and a step of a lone
+// workgroup takes 6 % more cycles.  Launches of several groups a line that end in 5 to 20 us never meet the limit; with 16x16x32 they
+// lose 1 to 5 % in the forward and up to 13 in the backward, so they run on 32x32x16 (see fwd_launch, mma_of).
+template <int kM> struct Mma;
+template <>
+struct Mma<16> {
+  static constexpr int kCols = 2, kRowRegs = 4;            // columns a lane holds; address registers of row reads
+  // Pitch of the V-type layout's fours.  A transposing read gathers 32 bytes of each row of two fours per half wave: the rows are in
+  // different 64-byte groups, the two fours in different halves of one.  A 128-bit read of 16 rows is served 16 lanes
+  // at a time, half of the rows from either of two adjacent lane groups, whose chunks differ by one: different slots, too.  (With the fours'
+  // starts 0, 32, 16 and 48 bytes into a 64-byte group the backward, 32 heads of 4096, met 68 million conflict cycles, so 0.8.)
+  static constexpr int kPitch = 1056;
+  static __device__ __forceinline__ int col(int lane, int n) { return 16 * n + (lane & 15); }
+  static __device__ __forceinline__ int quad_row(int lane, int q) { return 16 * (q >> 1) + 4 * (lane >> 4); }
+  static constexpr __device__ int quad_n(int q) { return q & 1; }
+  static __device__ __forceinline__ int quad_chunk(int lane, int q) { return 2 * (q >> 1) + (lane >> 5); }     // of 8 rows
+  static __device__ __forceinline__ int quad_half(int lane) { return lane >> 4 & 1; }
+  static __device__ __forceinline__ int quad_piece(int lane, int q) { return 4 * (q >> 1) + (lane >> 4); }       // of 4 rows
+  // B fragment i (of 8) of 32 rows of 128: row and 16-byte chunk
+  static __device__ __forceinline__ int frag_row(int lane, int i) { return 16 * (i & 1) + (lane & 15); }
+  static __device__ __forceinline__ int frag_chunk(int lane, int i) { return 4 * (i >> 1) + (lane >> 4); }
+  // First product, contracted over the 128: A fragment i (of 8) = 16 rows, a quarter of them.  (row and chunk of address register j; the
+  // fragments' register and what lies between them)
+  static __device__ __forceinline__ int a_row(int lane) { return lane & 15; }
+  static __device__ __forceinline__ int a_chunk(int lane, int j) { return 4 * j + (lane >> 4); }
+  static constexpr __device__ int a_reg(int i) { return i >> 1; }
+  static constexpr __device__ int a_offset(int i, int four_pitch) { return (i & 1) * 4 * four_pitch; }
+  // Second product, contracted over 32 rows: A fragment i = columns 16 * i .. + 15, all rows, read through the transposing path
+  // as two halves: lane group g supplies rows 4g .. 4g + 3 and 16 + 4g .., as two blocks of 16 accumulator rows do.
+  static __device__ __forceinline__ int tr_offset(int lane, int m) {
+    const int g = lane >> 4, r = (lane & 15) >> 2, c = lane & 3;
+    return kPitch * g + r * kRowBytes + (slot_v(r, 4 * m + (c >> 1)) << 4) + (c & 1) * 8;
+  }
+  static constexpr __device__ int tr_reg(int i) { return i >> 1; }
+  static constexpr __device__ int tr_first(int i) { return 32 * (i & 1); }
+  static constexpr int kTrSecond = 4 * kPitch;
+  static constexpr __device__ int slot_n(int i) { return i >> 2 & 1; }                    // where acc[i] goes in the next B operand
+  static constexpr __device__ int slot_j(int i) { return 4 * (i >> 3) + (i & 3); }
+  static __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
+  static __device__ __forceinline__ f32x4 quad(const f32x16& x, int q) { return f32x4{x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]}; }
+  static __device__ __forceinline__ void into(f32x16& x, int q, bf16x8 a, bf16x8 b, f32x4 c) {
+    c = mfma(a, b, c);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[4 * q + j] = c[j];
+  }
+  struct Start { f32x4 of[2]; };           // what a lane's columns start from
+  static __device__ __forceinline__ Start start(const float (&x)[2]) { return {{f32x4{x[0], x[0], x[0], x[0]}, f32x4{x[1], x[1], x[1], x[1]}}}; }
+  static __device__ __forceinline__ void keep(Start& s) { asm volatile("" : "+v"(s.of[0]), "+v"(s.of[1])); }
+  static __device__ __forceinline__ void first(f32x16& acc, int i, bf16x8 a, const bf16x8 (&f)[8], const Start& from) {
+#pragma unroll
+    for (int n = 0; n < 2; ++n) into(acc, 2 * (i & 1) + n, a, f[2 * (i >> 1) + n], i < 2 ? from.of[n] : quad(acc, 2 * (i & 1) + n));
+  }
+  static __device__ __forceinline__ void second(f32x16 (&acc)[4], int i, bf16x8 a, const bf16x8 (&f)[2]) {
+#pragma unroll
+    for (int n = 0; n < 2; ++n) into(acc[i >> 1], 2 * (i & 1) + n, a, f[n], quad(acc[i >> 1], 2 * (i & 1) + n));
+  }
+  static __device__ __forceinline__ float column_max(float x) {
+    float a, b;
+    swap_lanes<16>(x, a, b);
+    swap_lanes<32>(fmaxf(a, b), a, b);
+    return fmaxf(a, b);
+  }
+  static __device__ __forceinline__ float column_sum(float x) {
+    float a, b;
+    swap_lanes<16>(x, a, b);
+    swap_lanes<32>(a + b, a, b);
+    return a + b;
+  }
+  // The instructions' order: an LDS read after the first of a fragment's two MFMAs, or (`reads` = 2) after either.
+  template <int kReads>
+  static __device__ __forceinline__ void interleave() {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    if (kReads == 2) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
   }
 };
-template <int (*OFF)(int, int)>
-__device__ __forceinline__ bf16x8 lds_read_tr_frag(const unsigned char* smem, const TrLane& t, int row0, int mb) {
-  const bf16x4 lo = lds_read_tr16_b64(smem, OFF(row0 + t.row_in, 4 * mb + t.chunk_in) + t.sub);
-  const bf16x4 hi = lds_read_tr16_b64(smem, OFF(row0 + 8 + t.row_in, 4 * mb + t.chunk_in) + t.sub);
-  return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-}
+template <>
+struct Mma<32> {
+  static constexpr int kCols = 1, kRowRegs = 8;
+  static constexpr int kPitch = 1040;      // (the rows of two fours that a half wave gathers are whole 64-byte groups)
+  static __device__ __forceinline__ int col(int lane, int) { return lane & 31; }
+  static __device__ __forceinline__ int quad_row(int lane, int q) { return 8 * q + 4 * (lane >> 5); }
+  static constexpr __device__ int quad_n(int) { return 0; }
+  static __device__ __forceinline__ int quad_chunk(int, int q) { return q; }
+  static __device__ __forceinline__ int quad_half(int lane) { return lane >> 5; }
+  static __device__ __forceinline__ int quad_piece(int lane, int q) { return 2 * q + (lane >> 5); }
+  static __device__ __forceinline__ int frag_row(int lane, int) { return lane & 31; }
+  static __device__ __forceinline__ int frag_chunk(int lane, int i) { return 2 * i + (lane >> 5); }
+  // First product: A fragment i = 32 rows, an eighth of the 128.
+  static __device__ __forceinline__ int a_row(int lane) { return lane & 31; }
+  static __device__ __forceinline__ int a_chunk(int lane, int j) { return 2 * j + (lane >> 5); }
+  static constexpr __device__ int a_reg(int i) { return i; }
+  static constexpr __device__ int a_offset(int, int) { return 0; }
+  // Second product: A fragment i = columns 32 * (i % 4) .. + 31, 16 rows from 16 * (i / 4) on; lane half h supplies rows 4h .. 4h + 3 and 8 + 4h ..
+  static __device__ __forceinline__ int tr_offset(int lane, int m) {
+    const int i16 = lane & 15, r = i16 >> 2;
+    return kPitch * (lane >> 5) + r * kRowBytes + (slot_v(r, 4 * m + 2 * (lane >> 4 & 1) + ((i16 & 3) >> 1)) << 4) + (i16 & 1) * 8;
+  }
+  static constexpr __device__ int tr_reg(int i) { return i & 3; }
+  static constexpr __device__ int tr_first(int i) { return 4 * kPitch * (i >> 2); }
+  static constexpr int kTrSecond = 2 * kPitch;
+  static constexpr __device__ int slot_n(int i) { return i >> 3; }
+  static constexpr __device__ int slot_j(int i) { return i & 7; }
+  static __device__ __forceinline__ f32x16 mfma(bf16x8 a, bf16x8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
+  struct Start { f32x16 of; };
+  static __device__ __forceinline__ Start start(const float (&x)[2]) {
+    Start s;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s.of[i] = x[0];
+    return s;
+  }
+  static __device__ __forceinline__ void keep(Start& s) { asm volatile("" : "+v"(s.of)); }
+  static __device__ __forceinline__ void first(f32x16& acc, int i, bf16x8 a, const bf16x8 (&f)[8], const Start& from) {
+    acc = mfma(a, f[i], i == 0 ? from.of : acc);
+  }
+  static __device__ __forceinline__ void second(f32x16 (&acc)[4], int i, bf16x8 a, const bf16x8 (&f)[2]) { acc[i & 3] = mfma(a, f[i >> 2], acc[i & 3]); }
+  static __device__ __forceinline__ float column_max(float x) {
+    float a, b;
+    swap_lanes<32>(x, a, b);
+    return fmaxf(a, b);
+  }
+  static __device__ __forceinline__ float column_sum(float x) {
+    float a, b;
+    swap_lanes<32>(x, a, b);
+    return a + b;
+  }
+  template <int kReads>
+  static __device__ __forceinline__ void interleave() {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x100, kReads, 0);
+  }
+};
+// Of a form of the backward's walks (see Groups).  The several groups' kernels, whose groups' indices take registers too, spill with 16x16x32 or
+// read one fragment ahead: 8 heads of 2048 are 6 % faster all the same, of 1024 1 % and, causal, 3 % slower, 256 x 256 causal 13 %.
+constexpr int mma_of(int form) { return form == 1 ? 16 : 32; }
 
 // ---- row tiles of one wave: 32 rows of 256 bytes between memory and the operand / accumulator layouts ---------
 // In those layouts a lane owns 8 or 16 bytes of a row, and a load or store straight from them touches 32 rows per
@@ -104,13 +223,14 @@ __device__ __forceinline__ void load_rows(u32x4 (&raw)[8], const bf16* rows, int
 #pragma unroll
   for (int i = 0; i < 8; ++i) raw[i] = *reinterpret_cast<const u32x4*>(p + 4 * i * row_stride);
 }
-// B operands of 32 rows: fragment ks of a lane = row lane % 32, elements 16 * ks + 8 * (lane / 32) .. + 7.
+// B operands of 32 rows.
+template <int kM>
 __device__ __forceinline__ void rows_to_frags(bf16x8 (&f)[8], const u32x4 (&raw)[8], uint32_t lds) {
   const int lane = fresh_lane();
 #pragma unroll
   for (int i = 0; i < 8; ++i) lds_put(lds + row_slot(4 * i + (lane >> 4), lane & 15), raw[i]);
 #pragma unroll
-  for (int ks = 0; ks < 8; ++ks) f[ks] = lds_get<bf16x8>(lds + row_slot(lane & 31, 2 * ks + (lane >> 5)));
+  for (int i = 0; i < 8; ++i) f[i] = lds_get<bf16x8>(lds + row_slot(Mma<kM>::frag_row(lane, i), Mma<kM>::frag_chunk(lane, i)));
 }
 // buffer_load_dwordx4 ... lds with the LDS destination (wave-uniform) in M0; see dma16_buf.
 // M0 is declared clobbered; "memory" is left out on purpose so that LDS reads of the other
@@ -144,40 +264,47 @@ __device__ __forceinline__ void copy_shared_rows(const bf16* rows, int row_strid
     dma16_abs(rsrc, lds + (4 * sixteen + (w & 3)) * 1024, voff, sixteen * 32 * row_stride);
   }
 }
+template <int kM>
 __device__ __forceinline__ void shared_rows_to_frags(bf16x8 (&f)[8], uint32_t lds, int block) {
   const int lane = fresh_lane();
 #pragma unroll
-  for (int ks = 0; ks < 8; ++ks) f[ks] = lds_get<bf16x8>(lds + row_slot(32 * block + (lane & 31), 2 * ks + (lane >> 5)));
+  for (int i = 0; i < 8; ++i) f[i] = lds_get<bf16x8>(lds + row_slot(32 * block + Mma<kM>::frag_row(lane, i), Mma<kM>::frag_chunk(lane, i)));
 }
-// acc[mb][4g + j] holds column 32 * mb + 8 * g + 4 * (lane / 32) + j of row lane % 32; written times `mul` as bf16.
-__device__ __forceinline__ void store_rows_bf16(bf16* rows, int64_t row_stride, const f32x16 (&acc)[4], float mul, uint32_t lds) {
+// Accumulators of 32 rows x 128 columns: acc[m] is block m of 32 columns, transposed (a lane's columns of the block are rows here).  A
+// lane's factors of its rows:
+struct RowPair { float x[2]; };
+__device__ __forceinline__ RowPair both(float x) { return {{x, x}}; }
+// The rows times `mul` as bf16.
+template <int kM>
+__device__ __forceinline__ void store_rows_bf16(bf16* rows, int64_t row_stride, const f32x16 (&acc)[4], RowPair mul, uint32_t lds) {
+  using M = Mma<kM>;
   const int lane = fresh_lane();
 #pragma unroll
-  for (int mb = 0; mb < 4; ++mb)
+  for (int i = 0; i < 16; ++i) {
+    bf16x4 w;
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      bf16x4 w;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) w[j] = (bf16)(acc[mb][4 * g + j] * mul);
-      lds_put(lds + row_slot(lane & 31, 4 * mb + g) + 8 * (lane >> 5), w);
-    }
+    for (int j = 0; j < 4; ++j) w[j] = (bf16)(acc[i >> 2][4 * (i & 3) + j] * mul.x[M::quad_n(i & 3)]);
+    lds_put(lds + row_slot(M::col(lane, M::quad_n(i & 3)), 4 * (i >> 2) + M::quad_chunk(lane, i & 3)) + 8 * M::quad_half(lane), w);
+  }
   bf16* p = rows + (lane >> 4) * row_stride + (lane & 15) * 8;
 #pragma unroll
   for (int i = 0; i < 8; ++i)
     *reinterpret_cast<u32x4*>(p + 4 * i * row_stride) = lds_get<u32x4>(lds + row_slot(4 * i + (lane >> 4), lane & 15));
 }
 // The same as fp32, half a row at a time.
-__device__ __forceinline__ void store_rows_f32(float* rows, int64_t row_stride, const f32x16 (&acc)[4], float mul, uint32_t lds) {
+template <int kM>
+__device__ __forceinline__ void store_rows_f32(float* rows, int64_t row_stride, const f32x16 (&acc)[4], RowPair mul, uint32_t lds) {
+  using M = Mma<kM>;
   const int lane = fresh_lane();
 #pragma unroll
   for (int half = 0; half < 2; ++half) {
 #pragma unroll
-    for (int m = 0; m < 2; ++m)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x16& a = acc[2 * half + m];
-        lds_put(lds + row_slot(lane & 31, 8 * m + 2 * g + (lane >> 5)), f32x4{a[4 * g] * mul, a[4 * g + 1] * mul, a[4 * g + 2] * mul, a[4 * g + 3] * mul});
-      }
+    for (int i = 0; i < 8; ++i) {
+      const f32x16& a = acc[2 * half + (i >> 2)];
+      const int q = 4 * (i & 3);
+      const float f = mul.x[M::quad_n(i & 3)];
+      lds_put(lds + row_slot(M::col(lane, M::quad_n(i & 3)), 8 * (i >> 2) + M::quad_piece(lane, i & 3)), f32x4{a[q] * f, a[q + 1] * f, a[q + 2] * f, a[q + 3] * f});
+    }
     float* p = rows + (lane >> 4) * row_stride + 64 * half + (lane & 15) * 4;
 #pragma unroll
     for (int i = 0; i < 8; ++i)
@@ -185,16 +312,19 @@ __device__ __forceinline__ void store_rows_f32(float* rows, int64_t row_stride, 
   }
 }
 
-// One block of 32 columns of the same rows (a wave's share after a sum over groups): acc[4g + j] = column
-// 8 * g + 4 * (lane / 32) + j of row lane % 32, `rows` already at the block; through 2 or 4 KiB of LDS.
-__device__ __forceinline__ void store_block_bf16(bf16* rows, int64_t row_stride, const f32x16& acc, float mul, uint32_t lds) {
-  const int lane = fresh_lane(), r = lane & 31;
+// One block of 32 columns of the same rows (a wave's share after a sum over groups), `rows` already at the block; through 2
+// or 4 KiB of LDS.
+template <int kM>
+__device__ __forceinline__ void store_block_bf16(bf16* rows, int64_t row_stride, const f32x16& acc, RowPair mul, uint32_t lds) {
+  using M = Mma<kM>;
+  const int lane = fresh_lane();
 #pragma unroll
-  for (int g = 0; g < 4; ++g) {
+  for (int i = 0; i < 4; ++i) {
+    const int r = M::col(lane, M::quad_n(i));
     bf16x4 w;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) w[j] = (bf16)(acc[4 * g + j] * mul);
-    lds_put(lds + r * 64 + ((g ^ (r >> 2 & 3)) << 4) + 8 * (lane >> 5), w);
+    for (int j = 0; j < 4; ++j) w[j] = (bf16)(acc[4 * i + j] * mul.x[M::quad_n(i)]);
+    lds_put(lds + r * 64 + ((M::quad_chunk(lane, i) ^ (r >> 2 & 3)) << 4) + 8 * M::quad_half(lane), w);
   }
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
@@ -202,12 +332,16 @@ __device__ __forceinline__ void store_block_bf16(bf16* rows, int64_t row_stride,
     *reinterpret_cast<u32x4*>(rows + row * row_stride + 8 * c) = lds_get<u32x4>(lds + row * 64 + ((c ^ (row >> 2 & 3)) << 4));
   }
 }
-__device__ __forceinline__ void store_block_f32(float* rows, int64_t row_stride, const f32x16& acc, float mul, uint32_t lds) {
-  const int lane = fresh_lane(), r = lane & 31;
+template <int kM>
+__device__ __forceinline__ void store_block_f32(float* rows, int64_t row_stride, const f32x16& acc, RowPair mul, uint32_t lds) {
+  using M = Mma<kM>;
+  const int lane = fresh_lane();
 #pragma unroll
-  for (int g = 0; g < 4; ++g)
-    lds_put(lds + r * 128 + (((2 * g + (lane >> 5)) ^ (r >> 1 & 7)) << 4),
-            f32x4{acc[4 * g] * mul, acc[4 * g + 1] * mul, acc[4 * g + 2] * mul, acc[4 * g + 3] * mul});
+  for (int i = 0; i < 4; ++i) {
+    const int r = M::col(lane, M::quad_n(i));
+    const float f = mul.x[M::quad_n(i)];
+    lds_put(lds + r * 128 + ((M::quad_piece(lane, i) ^ (r >> 1 & 7)) << 4), f32x4{acc[4 * i] * f, acc[4 * i + 1] * f, acc[4 * i + 2] * f, acc[4 * i + 3] * f});
+  }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int row = 8 * i + (lane >> 3), c = lane & 7;
@@ -223,31 +357,32 @@ __device__ __forceinline__ void put_acc(uint32_t lds, const f32x16 (&acc)[4], in
   for (int mb = 0; mb < 4; ++mb) {
     if (mb == own) continue;
 #pragma unroll
-    for (int g = 0; g < 4; ++g) lds_put(lds + 4096 * mb + 1024 * g, f32x4{acc[mb][4 * g], acc[mb][4 * g + 1], acc[mb][4 * g + 2], acc[mb][4 * g + 3]});
+    for (int i = 0; i < 4; ++i) lds_put(lds + 4096 * mb + 1024 * i, f32x4{acc[mb][4 * i], acc[mb][4 * i + 1], acc[mb][4 * i + 2], acc[mb][4 * i + 3]});
   }
 }
-// acc = acc * wa + (block mb) * wb
-__device__ __forceinline__ void add_block(uint32_t lds, int mb, f32x16& acc, float wa = 1.f, float wb = 1.f) {
+// acc = acc * wa + (block mb in LDS) * wb
+template <int kM>
+__device__ __forceinline__ void add_block(uint32_t lds, int mb, f32x16& acc, RowPair wa, RowPair wb) {
   lds += 16 * fresh_lane() + 4096 * mb;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const f32x4 x = lds_get<f32x4>(lds + 1024 * i);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[4 * i + j] = acc[4 * i + j] * wa + x[j] * wb;
+    for (int j = 0; j < 4; ++j) acc[4 * i + j] = acc[4 * i + j] * wa.x[Mma<kM>::quad_n(i)] + x[j] * wb.x[Mma<kM>::quad_n(i)];
   }
 }
 // sum = the groups' blocks `own` in order, times w: this wave's from its accumulators, the other groups' from at(g).
 // (Its own block through LDS as well was a fourth of what the four groups' end moves there: 8 heads of 1024, forward
 // 12.85 -> 12.75 us, backward 19.8 -> 19.4; 32 of 512, forward 10.2 -> 9.9.)
-template <class At>
-__device__ __forceinline__ void sum_blocks(f32x16& sum, const f32x16 (&acc)[4], int own, At at, const float (&w)[4]) {
+template <int kM, class At>
+__device__ __forceinline__ void sum_blocks(f32x16& sum, const f32x16 (&acc)[4], int own, At at, const RowPair (&w)[4]) {
   sum = f32x16{0};
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
-    if (g != own) add_block(at(g), own, sum, 1.f, w[g]);
+    if (g != own) add_block<kM>(at(g), own, sum, both(1.f), w[g]);
     if (g == own) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) sum[i] += acc[g][i] * w[g];
+      for (int i = 0; i < 16; ++i) sum[i] += acc[g][i] * w[g].x[Mma<kM>::quad_n(i >> 2)];
     }
   }
 }
@@ -317,21 +452,21 @@ __device__ __forceinline__ void dma16_buf(__amdgpu_buffer_rsrc_t r, unsigned cha
 // Per-thread byte offsets for staging 16 * NW rows of 128 bf16 with NW waves: each thread issues 4
 // copies; copy i of wave w fills LDS rows 4*(NW*i + w) .. +3; lane l lands in
 // that group's row l/16, physical 16-byte slot l%16, so it must fetch the logical chunk that the
-// XOR layout `OFF` maps to that slot.
-template <int (*OFF)(int, int), int NW>
+// XOR layout `SLOT` maps to that slot.
+template <int (*SLOT)(int, int), int NW>
 __device__ __forceinline__ void dma_voffsets(int (&off)[4], int row_stride, int wave, int lane) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int r = 4 * (NW * i + wave) + (lane >> 4);
-    const int c = ((OFF(r, 0) - r * kRowBytes) >> 4) ^ (lane & 15);
-    off[i] = (r * row_stride + c * 8) * 2;
+    off[i] = (r * row_stride + SLOT(r, lane & 15) * 8) * 2;
   }
 }
-template <int NW>
+// The fours of rows at a pitch of kPitch bytes.
+template <int NW, int kPitch>
 __device__ __forceinline__ void dma_rows_buf(unsigned char* lds, __amdgpu_buffer_rsrc_t r, const int (&voff)[4],
                                                   int soff, int wave) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) dma16_buf(r, lds + (NW * i + wave) * 1024, voff[i], soff);
+  for (int i = 0; i < 4; ++i) dma16_buf(r, lds + (NW * i + wave) * kPitch, voff[i], soff);
 }
 
 // n / d for 0 <= n < 2^31 as one multiplication: mul = ceil(2^shift / d), shift = 31 + ceil(log2 d), is off by less than d, so that
