@@ -109,7 +109,7 @@ __device__ __forceinline__ void key_blocks(const unsigned char* sK, const unsign
   for (int i = 0; i < kVAhead; ++i) vfr[i] = rd_v(i);
   side();
   // ---- online softmax (fp32, log2 domain) ---------------------------------------------------
-  float rs[2];
+  float rs[2] = {0.f, 0.f};
   bf16x8 pf[kB][2];
   auto exponentials = [&]() {
     rs[0] = rs[1] = 0.f;
@@ -126,7 +126,7 @@ __device__ __forceinline__ void key_blocks(const unsigned char* sK, const unsign
   bool raise = first;
   if (!first) {
     exponentials();
-    raise = __builtin_amdgcn_ballot_w64(!((M::kCols == 2 ? rs[0] + rs[1] : rs[0]) < kRaiseSum)) != 0;       // wave-uniform, rare
+    raise = __builtin_amdgcn_ballot_w64(!(rs[0] < kRaiseSum) || (M::kCols == 2 && !(rs[1] < kRaiseSum))) != 0;       // wave-uniform, rare
   }
   if (raise) {
 #pragma unroll
@@ -139,7 +139,9 @@ __device__ __forceinline__ void key_blocks(const unsigned char* sK, const unsign
         for (int mb = 0; mb < kB; ++mb)
           if (M::quad_n(i >> 2) == n) mx = fmaxf(mx, s[mb][i]);
       mx = M::column_max(mx) * scale_log2;
-      const float m_new = fmaxf(t.m_run, mx);
+      // (only rows that need it: a row's result must not depend on the rows that share its wave)
+      const bool needed = first || M::column_max(rs[n] < kRaiseSum ? 0.f : 1.f) > 0.f;
+      const float m_new = needed ? fmaxf(t.m_run, mx) : t.m_run;
       const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
       const float alpha = (m_new == t.m_run) ? 1.f : fast_exp2(t.m_run - m_use);      // m_run = -inf -> 0
       t.m_run = m_new;
@@ -420,6 +422,179 @@ __global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void fwd_kernel(const F
   }
 }
 
+// Tile lists of few lines (see few_lines): the walk of fwd_kernel<1> with eight waves of 16 rows instead of four of 32, two on every
+// SIMD, one in its products while the other is in its softmax.  A row meets the same products and sums in the same order, so that
+// its result is the same bit for bit.
+// Bound: LDS.  Every K and V fragment is read for 16 rows instead of 32, 256 KiB a half tile at the 128 bytes a cycle that LDS
+// gives: 0.92 us a half tile, with four waves 0.99.  Where two workgroups share a CU it is slower.
+template <int kWaveRows>
+__global__ __launch_bounds__(512, 2) void fwd_short_kernel(const FwdParams p) {
+  using M = Mma<16>;
+  static_assert(kWaveRows == 16 && M::kCols * 16 == 32, "one of the two columns that a lane of fwd_kernel holds");
+  constexpr int kHalfRows = 64, kStageK = kHalfRows * kRowBytes, kStageV = kHalfRows / 4 * M::kPitch;
+  __shared__ __attribute__((aligned(1024))) unsigned char sKA[kStageK];
+  __shared__ __attribute__((aligned(1024))) unsigned char sVA[kStageV];
+  __shared__ __attribute__((aligned(1024))) unsigned char sKB[kStageK];
+  __shared__ __attribute__((aligned(1024))) unsigned char sVB[kStageV];
+  const int lane = threadIdx.x & 63, row = lane & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int pos, bh;
+  map_block(blockIdx.x, p.map, pos, bh);
+  const int b = quotient(bh, p.by_heads), h = bh - b * p.n_heads;
+  const int qt = min(max(sload(p.q_order, pos), 0), p.n_qtiles - 1);
+  const int e0 = min(max(sload(p.row_ptr, qt), 0), p.nnz), e1 = min(max(sload(p.row_ptr, qt + 1), e0), p.nnz);
+  const bf16* const kbase = p.k + b * p.ks.b + h * p.ks.h;
+  const bf16* const vbase = p.v + b * p.vs.b + h * p.vs.h;
+  const int k_stride = (int)p.ks.s, v_stride = (int)p.vs.s;
+  // A stage's four copies: fours of rows `wave` and 8 + `wave` of K and V.
+  const int four_row = 4 * wave + (lane >> 4);
+  const int koff = (four_row * k_stride + slot_k(four_row, row) * 8) * 2, voff = (four_row * v_stride + slot_v(four_row, row) * 8) * 2;
+  const uint32_t k_extent = (uint32_t)((kTile - 1) * k_stride + kHeadDim) * 2, v_extent = (uint32_t)((kTile - 1) * v_stride + kHeadDim) * 2;
+  auto lds_at = [](unsigned char* x) { return (uint32_t)(uintptr_t)(lds_byte*)x; };
+  u32x4 k_rsrc, v_rsrc;                    // without `more` the copies fill with zeros a stage that no step reads
+  auto tile = [&](int t, bool more) {
+    k_rsrc = make_rsrc_words(kbase + (int64_t)t * kTile * k_stride, more ? k_extent : 0);
+    v_rsrc = make_rsrc_words(vbase + (int64_t)t * kTile * v_stride, more ? v_extent : 0);
+  };
+  auto copy = [&](int n, unsigned char* k_stage, unsigned char* v_stage, int half) {
+    const int j = n >> 1, first = half * kHalfRows + 32 * j;
+    if (n & 1) dma16_abs(v_rsrc, lds_at(v_stage) + (8 * j + wave) * M::kPitch, voff, first * v_stride * 2);
+    else       dma16_abs(k_rsrc, lds_at(k_stage) + (8 * j + wave) * 1024, koff, first * k_stride * 2);
+  };
+  Walk<false, true> walk(e0, e1, -1);
+  int ent = 0, ent_next = 0;
+  if (e0 < e1) {
+    walk.fetch(e0, p.col_idx, p.flag, p.n_ktiles);
+    ent = walk.at(e0);
+    tile(walk.tile(ent), true);
+#pragma unroll
+    for (int n = 0; n < 4; ++n) copy(n, sKA, sVA, 0);
+  }
+  const int qrow0 = qt * kTile + kWaveRows * wave, q_block = wave >> 1;
+  const bf16* const qrow = p.q + b * p.qs.b + (int64_t)(qrow0 + row) * p.qs.s + h * p.qs.h;
+  bf16x8 qf[4];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) qf[ks] = *reinterpret_cast<const bf16x8*>(qrow + 8 * M::a_chunk(lane, ks));
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) asm volatile("" : "+v"(qf[ks]));      // read before the walk
+  f32x4 oacc[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) oacc[i] = f32x4{0};
+  float m_run = -INFINITY, m_use = 0.f, l_run = 0.f;
+  int nat[4], tr[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    nat[i] = lds_off_k(M::a_row(lane), M::a_chunk(lane, i));
+    tr[i] = M::tr_offset(lane, i);
+  }
+  auto step = [&](int e, auto stage_tag) {
+    constexpr int kStage = decltype(stage_tag)::value;
+    const unsigned char *const sK = kStage ? sKB : sKA, *const sV = kStage ? sVB : sVA;
+    unsigned char *const k_other = kStage ? sKA : sKB, *const v_other = kStage ? sVA : sVB;
+    if (kStage == 1) tile(walk.tile(ent_next), e + 1 < e1);
+    wait_vmem_all();
+    __syncthreads();
+    const bool causal = (ent >> 30) != 0, hidden = causal && 2 * kStage > q_block;
+    if (hidden) {
+#pragma unroll
+      for (int n = 0; n < 4; ++n) copy(n, k_other, v_other, kStage ^ 1);
+    } else {
+      f32x4 s[4];
+      constexpr int kAhead = 4;
+      bf16x8 kfr[16];
+      auto rd = [&](int i) { return lds_read_b128(sK, nat[i >> 2] + 16 * kRowBytes * (i & 3)); };
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) kfr[i] = rd(i);
+      __builtin_amdgcn_sched_group_barrier(0x100, kAhead, 0);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        if (i + kAhead < 16) kfr[i + kAhead] = rd(i + kAhead);
+        s[i & 3] = M::mfma(kfr[i], qf[i >> 2], i < 4 ? f32x4{0} : s[i & 3]);
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        if ((i & 3) == 3) copy(i >> 2, k_other, v_other, kStage ^ 1);
+      }
+      if (causal && q_block < 2 * kStage + 2) {
+        const int ahead = kHalfRows * kStage + 4 * (fresh_lane() >> 4) - kWaveRows * wave - (fresh_lane() & 15);
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          if (ahead + 16 * (i >> 2) + (i & 3) > 0) s[i >> 2][i & 3] = -INFINITY;
+      }
+      constexpr int kVAhead = 4;
+      bf16x8 vfr[16];
+      auto rd_v = [&](int i) {
+        const int at = tr[(i & 7) >> 1] + M::tr_first(i & 7) + 8 * M::kPitch * (i >> 3);
+        const bf16x4 lo = lds_read_tr16_b64(sV, at), hi = lds_read_tr16_b64(sV, at + M::kTrSecond);
+        return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+      };
+#pragma unroll
+      for (int i = 0; i < kVAhead; ++i) vfr[i] = rd_v(i);
+      if (kStage == 0) {                     // the next tile's entry
+        if (!walk.has(e + 1)) walk.fetch(e + 1, p.col_idx, p.flag, p.n_ktiles);
+        ent_next = walk.at(min(e + 1, e1 - 1));
+      }
+      const bool first = kStage == 0 && e == e0;
+      float rs = 0.f;
+      bf16x8 pf[2];
+      auto exponentials = [&]() {
+        rs = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const float pv = fast_exp2(fmaf(s[i >> 2][i & 3], p.scale_log2, -m_use));
+          rs += pv;
+          pf[i >> 3][i & 7] = (bf16)pv;
+        }
+      };
+      bool raise = first;
+      if (!first) {
+        exponentials();
+        raise = __builtin_amdgcn_ballot_w64(!(rs < kRaiseSum)) != 0;
+      }
+      if (raise) {                           // as in key_blocks
+        float mx = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i >> 2][i & 3]);
+        mx = M::column_max(mx) * p.scale_log2;
+        const bool needed = first || M::column_max(rs < kRaiseSum ? 0.f : 1.f) > 0.f;
+        const float m_new = needed ? fmaxf(m_run, mx) : m_run;
+        const float m_at = (m_new == -INFINITY) ? 0.f : m_new;
+        const float alpha = (m_new == m_run) ? 1.f : fast_exp2(m_run - m_at);
+        m_run = m_new;
+        m_use = m_at;
+        l_run *= alpha;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) oacc[i] *= alpha;
+        exponentials();
+      }
+      l_run += rs;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        if (i + kVAhead < 16) vfr[i + kVAhead] = rd_v(i + kVAhead);
+        oacc[i & 7] = M::mfma(vfr[i], pf[i >> 3], oacc[i & 7]);
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+      }
+    }
+    if (kStage == 1) ent = ent_next;
+  };
+  for (int e = e0; e < e1; ++e) {
+    step(e, std::integral_constant<int, 0>{});
+    step(e, std::integral_constant<int, 1>{});
+  }
+  wait_vmem_all();
+  const float l_tot = M::column_sum(l_run), inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+  bf16* const orow = p.o + b * p.os.b + (int64_t)(qrow0 + row) * p.os.s + h * p.os.h + 4 * (lane >> 4);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    bf16x4 w;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[j] = (bf16)(oacc[i][j] * inv);
+    *reinterpret_cast<bf16x4*>(orow + 16 * i) = w;
+  }
+  if (lane < 16)
+    p.lse[((int64_t)b * p.n_heads + h) * ((int64_t)p.n_qtiles * kTile) + qrow0 + lane] =
+        l_tot > 0.f ? (m_run + __builtin_amdgcn_logf(l_tot)) * kLn2 : -INFINITY;
+}
+
 }  // namespace ua
 
 namespace ua {
@@ -466,6 +641,12 @@ static int fwd_groups(int64_t n, int64_t walk, int n_parts, bool dense_causal) {
   if (2 * n <= kCus || (uneven && n <= kCus && walk >= 16)) return 4;
   return walk >= 3 && n <= (uneven ? 2 * kCus : kCus) ? 2 : 1;
 }
+// Tile lists of n lines that run with eight waves a workgroup: up to one line a CU (one head, causal 4096: 63.6 us with four waves, 59.0; 8 heads
+// of causal 4096 64.9, 61.0), up to a line on every other CU where nearly all lines are of full length (8 heads of 4096 in full 68.3,
+// 72.0, one head of 1024 19.2, 18.9).  Both give the same bits.
+static bool few_lines(const FwdParams& p, int64_t n) {
+  return n <= ((int64_t)4 * p.nnz <= (int64_t)3 * p.n_qtiles * p.n_ktiles ? kCus : kCus / 2);
+}
 // `plain`: one group per workgroup.
 static int fwd_launch(FwdParams& p, bool plain, hipStream_t st) {
   const unsigned n = (unsigned)(p.batch * p.n_heads * (p.n_whole + (p.n_qtiles - p.n_whole) * p.n_parts));
@@ -493,8 +674,9 @@ static int fwd_launch(FwdParams& p, bool plain, hipStream_t st) {
       // launch order.  Lists come roughly by falling length, so the first ones are taken in reverse: long and
       // short lists then share a CU (strided 8k, 8 heads: the longest sum on a CU 40 -> 37 tiles, causal 96 -> 65).
       if (!p.dense && n > kCus && n <= 2 * kCus) p.n_first = kCus * p.n_qtiles / (int)n;
-      if (p.dense) hipLaunchKernelGGL((fwd_kernel<1, true, 16>), dim3(n), dim3(256), 0, st, p);
-      else         hipLaunchKernelGGL((fwd_kernel<1, false, 16>), dim3(n), dim3(256), 0, st, p);
+      if (p.dense)             hipLaunchKernelGGL((fwd_kernel<1, true, 16>), dim3(n), dim3(256), 0, st, p);
+      else if (few_lines(p, n)) hipLaunchKernelGGL((fwd_short_kernel<16>), dim3(n), dim3(512), 0, st, p);
+      else                     hipLaunchKernelGGL((fwd_kernel<1, false, 16>), dim3(n), dim3(256), 0, st, p);
   }
   return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH;
 }
