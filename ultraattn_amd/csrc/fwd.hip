@@ -171,7 +171,7 @@ __device__ __forceinline__ void key_blocks(const unsigned char* sK, const unsign
 // one wave per SIMD, where a half tile takes 1.2 us of which the matrix pipe is busy 0.4; with more groups the CU is
 // as full as with two workgroups, without partial results in memory.
 template <int kForm, bool kDense, int kM>
-__global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void fwd_kernel(const FwdParams p) {
+__device__ __forceinline__ void fwd_lines(const FwdParams& p) {
   using M = Mma<kM>;
   constexpr int kWaves = Groups<kForm>::kWaves, kRows = Groups<kForm>::kRows, kLines = Groups<kForm>::kLines;
   constexpr int kStageBytes = kRows * kRowBytes, kStageV = kRows / 4 * M::kPitch;
@@ -422,6 +422,15 @@ __global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void fwd_kernel(const F
   }
 }
 
+// Lists run on 16x16x32 matrix instructions, dense rectangles on 32x32x16.  Either sums a product in another order, so that a few in a hundred
+// entries of O round to the other bf16: delta = rowsum(dO * O), which the flash-attention signatures return in fp32 beside dense gradients,
+// would move by 1.5e-4, for 2 to 4 % of a long forward.
+template <int kForm, bool kDense>
+__global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void fwd_kernel(const FwdParams p) { fwd_lines<kForm, kDense, kDense ? 32 : 16>(p); }
+// A dense rectangle whose results are to be those of its tile list.
+template <int kM>
+__global__ __launch_bounds__(Groups<1>::kThreads, 2) void fwd_plain_kernel(const FwdParams p) { fwd_lines<1, true, kM>(p); }
+
 // Tile lists of few lines (see few_lines): the walk of fwd_kernel<1> with eight waves of 16 rows instead of four of 32, two on every
 // SIMD, one in its products while the other is in its softmax.  A row meets the same products and sums in the same order, so that
 // its result is the same bit for bit.
@@ -647,36 +656,31 @@ static int fwd_groups(int64_t n, int64_t walk, int n_parts, bool dense_causal) {
 static bool few_lines(const FwdParams& p, int64_t n) {
   return n <= ((int64_t)4 * p.nnz <= (int64_t)3 * p.n_qtiles * p.n_ktiles ? kCus : kCus / 2);
 }
-// `plain`: one group per workgroup.
+// `plain`: one group per workgroup, and of a dense rectangle the bits of its tile list.
 static int fwd_launch(FwdParams& p, bool plain, hipStream_t st) {
   const unsigned n = (unsigned)(p.batch * p.n_heads * (p.n_whole + (p.n_qtiles - p.n_whole) * p.n_parts));
   // (several groups copy Q through a buffer descriptor, whose offsets have 32 bits)
   const int form = plain || p.qs.s > (INT32_MAX >> 9) ? 1 : fwd_groups(n, p.part_len, p.n_parts, p.dense_causal);
   const int n_cut = p.n_qtiles - p.n_whole;
-  // Several groups a line: 32x32x16 for launches of less than 8 visible tiles a CU, whose few steps end before the larger instruction count
-  // of 16x16x32 is made up for (32 heads of 512 9.44 us, with 16x16x32 9.63; 16 of 1024 14.3, 14.5; causal 32 of 1024 18.75, 18.9), the other way
-  // from there on (32 heads of 1024 21.8 and 21.1; 8 of 4096 66.6, 63.1; causal 16 of 3072 47.9, 45.8).
-  const bool wide = visible_share(p.n_qtiles, p.n_ktiles, p.dense_causal) * p.batch * p.n_heads * p.n_qtiles * p.n_ktiles < 8.f * kCus;
   p.map = block_map(p.batch * p.n_heads, (p.n_whole + n_cut * p.n_parts) * (form == 4 ? 2 : 1));
   p.by_heads = make_div(p.n_heads);
   p.by_cut = make_div(n_cut ? n_cut : 1);
   switch (form) {
     case 4:
-      if (wide) hipLaunchKernelGGL((fwd_kernel<4, true, 32>), dim3(2 * n), dim3(512), 0, st, p);
-      else      hipLaunchKernelGGL((fwd_kernel<4, true, 16>), dim3(2 * n), dim3(512), 0, st, p);
+      hipLaunchKernelGGL((fwd_kernel<4, true>), dim3(2 * n), dim3(512), 0, st, p);
       break;
     case 2:
-      if (wide) hipLaunchKernelGGL((fwd_kernel<2, true, 32>), dim3(n), dim3(512), 0, st, p);
-      else      hipLaunchKernelGGL((fwd_kernel<2, true, 16>), dim3(n), dim3(512), 0, st, p);
+      hipLaunchKernelGGL((fwd_kernel<2, true>), dim3(n), dim3(512), 0, st, p);
       break;
     default:
       // Up to two workgroups per CU the whole launch is resident at once, and those after the first 256 join them in
       // launch order.  Lists come roughly by falling length, so the first ones are taken in reverse: long and
       // short lists then share a CU (strided 8k, 8 heads: the longest sum on a CU 40 -> 37 tiles, causal 96 -> 65).
       if (!p.dense && n > kCus && n <= 2 * kCus) p.n_first = kCus * p.n_qtiles / (int)n;
-      if (p.dense)             hipLaunchKernelGGL((fwd_kernel<1, true, 16>), dim3(n), dim3(256), 0, st, p);
+      if (p.dense && plain)    hipLaunchKernelGGL((fwd_plain_kernel<16>), dim3(n), dim3(256), 0, st, p);
+      else if (p.dense)        hipLaunchKernelGGL((fwd_kernel<1, true>), dim3(n), dim3(256), 0, st, p);
       else if (few_lines(p, n)) hipLaunchKernelGGL((fwd_short_kernel<16>), dim3(n), dim3(512), 0, st, p);
-      else                     hipLaunchKernelGGL((fwd_kernel<1, false, 16>), dim3(n), dim3(256), 0, st, p);
+      else                     hipLaunchKernelGGL((fwd_kernel<1, false>), dim3(n), dim3(256), 0, st, p);
   }
   return hipGetLastError() == hipSuccess ? UA_OK : UA_ERR_LAUNCH;
 }

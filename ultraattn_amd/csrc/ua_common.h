@@ -59,11 +59,11 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 //
 // On random operands, at the socket's power limit, a loop of 16x16x32 instructions that uses every A operand twice runs at 2.06
 // PFLOP/s, one of 32x32x16 at 1.75 (its accumulators take twice the register traffic a flop).  The long launches, which that
-// limit holds, gain 3 to 5 % in the forward (causal 32k, 32 heads 7.16 -> 6.85 ms, strided 128k 17.7 -> 17.1) and 7 to 8 % in the
-// backward (23.5 -> 21.7, 57.8 -> 53.6), at 1.81 and 1.87 instead of 1.60 GHz.  But there are twice as many instructions to
+// limit holds, gain 3 to 5 % in the forward (strided 128k 17.7 -> 17.1 ms) and 7 to 8 % in the backward (causal 32k, 32 heads
+// 23.5 -> 21.7, strided 128k 57.8 -> 53.6), at 1.81 and 1.87 instead of 1.60 GHz.  But there are twice as many instructions to
 // issue: beside a wave that issues them another one's fma, exp2 and add take 28 cycles instead of 22, and a step of a lone
-// workgroup takes 6 % more cycles.  Launches of several groups a line that end in 5 to 20 us never meet the limit; with 16x16x32 they
-// lose 1 to 5 % in the forward and up to 13 in the backward, so they run on 32x32x16 (see fwd_launch, mma_of).
+// workgroup takes 6 % more cycles.  Backward launches of several groups a line that end in 5 to 20 us never meet the limit; with 16x16x32 they
+// lose up to 13 %, so they run on 32x32x16 (see mma_of).  So do dense forwards, for their bits (see fwd_kernel).
 template <int kM> struct Mma;
 template <>
 struct Mma<16> {
