@@ -582,10 +582,11 @@ __device__ __forceinline__ void dq_block(const PairAddr<kM>& ad, const bf16x8 (&
   for (int i = 0; i < kTAhead; ++i) tfr[i] = pair_tr<kOff>(ad, i);
   // element i: key quad_row + i % 4 of the block, query column col
   if (mask) {
-    const int lane = fresh_lane(), ahead = M::quad_row(lane, 0) - M::col(lane, 0);
+    // (compared with the column, not its difference with 0: of 16 nested conditions the compiler keeps each in scalar registers)
+    const int lane = fresh_lane(), row = M::quad_row(lane, 0), col = M::col(lane, 0);
 #pragma unroll
     for (int i = 0; i < 16; ++i)
-      if (ahead + M::quad_row(0, i >> 2) + (i & 3) > M::col(0, M::quad_n(i >> 2))) s[i] = -INFINITY;
+      if (row + M::quad_row(0, i >> 2) + (i & 3) - M::col(0, M::quad_n(i >> 2)) > col) s[i] = -INFINITY;
   }
   side();
   bf16x8 dsb[2];

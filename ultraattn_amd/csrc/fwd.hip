@@ -90,12 +90,13 @@ __device__ __forceinline__ void key_blocks(const unsigned char* sK, const unsign
   }
   // element (mb, i) of this lane: key key0 + 32 * mb + quad_row + i % 4, query 32 * q_block + col of the tile
   if (mask) {
-    const int lane = fresh_lane(), ahead = key0 + M::quad_row(lane, 0) - 32 * q_block - M::col(lane, 0);
+    // (compared with the column, not their difference with 0: of 32 nested conditions the compiler keeps each in scalar registers)
+    const int lane = fresh_lane(), key = key0 + M::quad_row(lane, 0), query = 32 * q_block + M::col(lane, 0);
 #pragma unroll
     for (int mb = 0; mb < kB; ++mb)
 #pragma unroll
       for (int i = 0; i < 16; ++i)
-        if (ahead + 32 * mb + M::quad_row(0, i >> 2) + (i & 3) > M::col(0, M::quad_n(i >> 2))) s[mb][i] = -INFINITY;
+        if (key + 32 * mb + M::quad_row(0, i >> 2) + (i & 3) - M::col(0, M::quad_n(i >> 2)) > query) s[mb][i] = -INFINITY;
   }
   // the first V^T fragments are fetched now: their latency hides behind the softmax
   constexpr int kVAhead = 3;
