@@ -262,12 +262,12 @@ __device__ __forceinline__ void dkdv_block(const PairAddr<16>& ad, uint32_t stat
     }
     // element j of block (qb, n): query row 16*qb + 4*(lane/16) + j, key column 16*n + lane%16
     if (mask) {
-      const int lane = fresh_lane(), ahead = (lane & 15) - 4 * (lane >> 4);
+      const int lane = fresh_lane(), key = lane & 15, row = 4 * (lane >> 4);          // (not one difference: see dq_block)
 #pragma unroll
       for (int n = 0; n < 2; ++n)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          if (ahead + 16 * n > 16 * qb + j) s[qb][n][j] = -INFINITY;
+          if (row + 16 * qb + j - 16 * n < key) s[qb][n][j] = -INFINITY;
     }
     if (qb == 1) {
 #pragma unroll

@@ -524,10 +524,10 @@ __global__ __launch_bounds__(512, 2) void fwd_short_kernel(const FwdParams p) {
         if ((i & 3) == 3) copy(i >> 2, k_other, v_other, kStage ^ 1);
       }
       if (causal && q_block < 2 * kStage + 2) {
-        const int ahead = kHalfRows * kStage + 4 * (fresh_lane() >> 4) - kWaveRows * wave - (fresh_lane() & 15);
+        const int key = kHalfRows * kStage + 4 * (fresh_lane() >> 4), query = kWaveRows * wave + (fresh_lane() & 15);
 #pragma unroll
         for (int i = 0; i < 16; ++i)
-          if (ahead + 16 * (i >> 2) + (i & 3) > 0) s[i >> 2][i & 3] = -INFINITY;
+          if (key + 16 * (i >> 2) + (i & 3) > query) s[i >> 2][i & 3] = -INFINITY;
       }
       constexpr int kVAhead = 4;
       bf16x8 vfr[16];
