@@ -644,8 +644,8 @@ static int fwd_common(FwdParams& p, const void* q, const void* k, const void* v,
 //    two).
 // Groups sum in another order, so that the last bits of a row depend on how many lines the launch has.  Tile lists, whose
 // launches are shards of the rows and heads of one mask, therefore run with one group whatever their size: a row's result is
-// the same bit for bit in every launch that holds its list.  Lists of up to 128 lines pay for that with half-empty CUs (one
-// head, causal 4096: forward 35 us with four groups, 58 with one, backward 51 and 119; from 512 lines on little changes).
+// the same bit for bit in every launch that holds its list.  Lists of up to 128 lines pay for that (one head, causal 4096: forward
+// 35 us with four groups, 59 with one, see few_lines, backward 51 and 119; from 512 lines on little changes).
 static int fwd_groups(int64_t n, int64_t walk, int n_parts, bool dense_causal) {
   const bool uneven = dense_causal && n_parts == 1;
   if (2 * n <= kCus || (uneven && n <= kCus && walk >= 16)) return 4;
