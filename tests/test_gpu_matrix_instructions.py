@@ -1,5 +1,5 @@
-"""Walks on 16x16x32 and on 32x32x16 matrix instructions: dense launches on both sides of the bound of visible tiles at which the
-forward's groups change from one to the other, and rows whose reference max is raised in the middle of a walk."""
+"""Walks on 16x16x32 and on 32x32x16 matrix instructions: dense launches of one, two and four groups a line, of few and of many tiles, and
+rows whose reference max is raised in the middle of a walk."""
 import numpy as np
 import pytest
 import torch
