@@ -636,7 +636,8 @@ static int fwd_common(FwdParams& p, const void* q, const void* k, const void* v,
 
 // Groups per workgroup for n lines of 128 rows (parts counted) of a dense rectangle:
 //  - four, on half lines, while those leave a CU one workgroup at most (8 heads of 1024: 17.2 us with two groups, 13.8
-//    with four; 2048: 29.9, 24.3; walks of one tile 5.7 and 5.5, causal 6.1 and 5.5).
+//    with four; 2048: 29.9, 24.3).  Walks of one tile keep one group: four would take 5.5 us instead of 5.7, but a row would have
+//    other bits in a launch of up to 128 lines than in a longer one, and delta = rowsum(dO * O) move by 2.6e-3 with them.
 //  - two, on whole lines, up to one workgroup per CU and from three tiles on (32 heads of 1024: 25 us with one, 22 with two).
 //  - The rows of an uncut causal rectangle differ in length.  Run one after the other, longest first, they are
 //    balanced, which workgroups resident side by side from the start do not achieve: four groups up to 256 lines of 16
@@ -648,7 +649,7 @@ static int fwd_common(FwdParams& p, const void* q, const void* k, const void* v,
 // 35 us with four groups, 59 with one, see few_lines, backward 51 and 119; from 512 lines on little changes).
 static int fwd_groups(int64_t n, int64_t walk, int n_parts, bool dense_causal) {
   const bool uneven = dense_causal && n_parts == 1;
-  if (2 * n <= kCus || (uneven && n <= kCus && walk >= 16)) return 4;
+  if (walk >= 2 && (2 * n <= kCus || (uneven && n <= kCus && walk >= 16))) return 4;
   return walk >= 3 && n <= (uneven ? 2 * kCus : kCus) ? 2 : 1;
 }
 // Tile lists of n lines that run with eight waves a workgroup: up to one line a CU (one head, causal 4096: 63.6 us with four waves, 59.0; 8 heads
