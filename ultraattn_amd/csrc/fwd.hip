@@ -140,8 +140,9 @@ __device__ __forceinline__ void key_blocks(const unsigned char* sK, const unsign
         for (int mb = 0; mb < kB; ++mb)
           if (M::quad_n(i >> 2) == n) mx = fmaxf(mx, s[mb][i]);
       mx = M::column_max(mx) * scale_log2;
-      // (only rows that need it: a row's result must not depend on the rows that share its wave)
-      const bool needed = first || M::column_max(rs[n] < kRaiseSum ? 0.f : 1.f) > 0.f;
+      // (Of lists only the rows that need it: a row's result must not depend on the rows that share its wave, of which there are 16 or 32.
+      // Dense forwards raise all 32 rows at once and keep the bits that they have always had.)
+      const bool needed = kM == 32 || first || M::column_max(rs[n] < kRaiseSum ? 0.f : 1.f) > 0.f;
       const float m_new = needed ? fmaxf(t.m_run, mx) : t.m_run;
       const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
       const float alpha = (m_new == t.m_run) ? 1.f : fast_exp2(t.m_run - m_use);      // m_run = -inf -> 0
