@@ -88,16 +88,15 @@ __device__ __forceinline__ void store_result(const __attribute__((address_space(
   }
 }
 
-// The same for one block of 32 columns.
-template <int kM>
+// The same for one block of 32 columns (several groups).
 __device__ __forceinline__ void store_block(const __attribute__((address_space(4))) BwdSide* p, bf16* out, int64_t os_b, int64_t os_s,
                                             int64_t os_h, int n_heads, int part, int b, int64_t row0, int h, int64_t seq, int block,
                                             const f32x16& acc, float mul, uint32_t lds) {
   if (p->out_f32) {
     float* base = reinterpret_cast<float*>(out) + part * p->o_part;
-    store_block_f32<kM>(base + (((int64_t)b * seq + row0) * n_heads + h) * kHeadDim + 32 * block, (int64_t)n_heads * kHeadDim, acc, both(mul), lds);
+    store_block_f32(base + (((int64_t)b * seq + row0) * n_heads + h) * kHeadDim + 32 * block, (int64_t)n_heads * kHeadDim, acc, mul, lds);
   } else {
-    store_block_bf16<kM>(out + b * os_b + row0 * os_s + h * os_h + 32 * block, os_s, acc, both(mul), lds);
+    store_block_bf16(out + b * os_b + row0 * os_s + h * os_h + 32 * block, os_s, acc, mul, lds);
   }
 }
 
@@ -123,6 +122,7 @@ __device__ __forceinline__ void store_block(const __attribute__((address_space(4
 template <int kForm>
 struct Stages : Groups<kForm> {
   static constexpr int kM = mma_of(kForm);
+  static_assert(kForm == 1 || kM == 32, "sums over groups (add_block, sum_blocks, store_block) take a lane to hold one row");
   static constexpr int kBlockPitch = 8 * Mma<kM>::kPitch;            // 32 rows
   static constexpr int kPitch = Groups<kForm>::kRows / 4 * Mma<kM>::kPitch;
   static constexpr int kStatBytes = 2 * Groups<kForm>::kRows * 4;
@@ -518,18 +518,18 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& given, uint32_t lds_b
     __syncthreads();
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb)
-      if (group) add_block<S::kM>(area(0), mb, dv[mb], both(1.f), both(1.f)); else add_block<S::kM>(area(1), mb, dk[mb], both(1.f), both(1.f));
+      if (group) add_block(area(0), mb, dv[mb]); else add_block(area(1), mb, dk[mb]);
   }
   f32x16 dk_sum, dv_sum;             // four groups: each finishes a block of 32 columns of both
   if constexpr (kForm == 4) {
-    const RowPair kOnes[4] = {both(1.f), both(1.f), both(1.f), both(1.f)};
+    constexpr float kOnes[4] = {1.f, 1.f, 1.f, 1.f};
     put_acc(area(group), dk, group);
     __syncthreads();
-    sum_blocks<S::kM>(dk_sum, dk, group, area, kOnes);
+    sum_blocks(dk_sum, dk, group, area, kOnes);
     __syncthreads();
     put_acc(area(group), dv, group);
     __syncthreads();
-    sum_blocks<S::kM>(dv_sum, dv, group, area, kOnes);
+    sum_blocks(dv_sum, dv, group, area, kOnes);
   }
   const ParamsLate pl = params_late();
   const int64_t seq_k = (int64_t)pl->n_ktiles * kTile;
@@ -537,8 +537,8 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& given, uint32_t lds_b
   if constexpr (kForm == 4) {
     // (this wave alone reads the block of its own area that it turns through)
     const uint32_t turn = area(group) + 4096 * group;
-    store_block<S::kM>(&pl->cols, pl->cols.out0, pl->cols.o0s.b, pl->cols.o0s.s, pl->cols.o0s.h, pl->n_heads, part, b, krow_out, h, seq_k, group, dk_sum, pl->scale, turn);
-    store_block<S::kM>(&pl->cols, pl->cols.out1, pl->cols.o1s.b, pl->cols.o1s.s, pl->cols.o1s.h, pl->n_heads, part, b, krow_out, h, seq_k, group, dv_sum, 1.f, turn);
+    store_block(&pl->cols, pl->cols.out0, pl->cols.o0s.b, pl->cols.o0s.s, pl->cols.o0s.h, pl->n_heads, part, b, krow_out, h, seq_k, group, dk_sum, pl->scale, turn);
+    store_block(&pl->cols, pl->cols.out1, pl->cols.o1s.b, pl->cols.o1s.s, pl->cols.o1s.h, pl->n_heads, part, b, krow_out, h, seq_k, group, dv_sum, 1.f, turn);
   } else {
     const uint32_t turn = kForm == 1 ? lds_base + wave * kWaveRowsBytes : area(group ^ 1);
     if (kForm == 1 || group == 0)
@@ -738,10 +738,10 @@ __device__ __forceinline__ void dq_walk(const BwdParams& given, uint32_t lds_blo
   if constexpr (kForm == 4) {
     put_acc(area(group), dq, group);
     __syncthreads();
-    const RowPair kOnes[4] = {both(1.f), both(1.f), both(1.f), both(1.f)};
+    constexpr float kOnes[4] = {1.f, 1.f, 1.f, 1.f};
     f32x16 sum;
-    sum_blocks<S::kM>(sum, dq, group, area, kOnes);
-    store_block<S::kM>(&pl->rows, pl->rows.out0, pl->rows.o0s.b, pl->rows.o0s.s, pl->rows.o0s.h, pl->n_heads, part, b, qrow_out, h, seq_out, group, sum,
+    sum_blocks(sum, dq, group, area, kOnes);
+    store_block(&pl->rows, pl->rows.out0, pl->rows.o0s.b, pl->rows.o0s.s, pl->rows.o0s.h, pl->n_heads, part, b, qrow_out, h, seq_out, group, sum,
                 pl->scale, area(group) + 4096 * group);
   } else {
     uint32_t turn = lds_base + wave * kWaveRowsBytes;                // stage 0: everyone left it before the last step
@@ -751,7 +751,7 @@ __device__ __forceinline__ void dq_walk(const BwdParams& given, uint32_t lds_blo
       __syncthreads();
       if (group) return;
 #pragma unroll
-      for (int mb = 0; mb < 4; ++mb) add_block<S::kM>(turn, mb, dq[mb], both(1.f), both(1.f));
+      for (int mb = 0; mb < 4; ++mb) add_block(turn, mb, dq[mb]);
     }
     store_result<S::kM>(&pl->rows, pl->rows.out0, pl->rows.o0s.b, pl->rows.o0s.s, pl->rows.o0s.h, pl->n_heads, part, b, qrow_out, h, seq_out, dq, pl->scale,
                  turn);

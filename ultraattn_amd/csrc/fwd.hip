@@ -175,6 +175,7 @@ __device__ __forceinline__ void key_blocks(const unsigned char* sK, const unsign
 template <int kForm, bool kDense, int kM>
 __device__ __forceinline__ void fwd_lines(const FwdParams& p) {
   using M = Mma<kM>;
+  static_assert(kForm == 1 || kM == 32, "the groups' exchange takes a lane to hold one row");
   constexpr int kWaves = Groups<kForm>::kWaves, kRows = Groups<kForm>::kRows, kLines = Groups<kForm>::kLines;
   constexpr int kStageBytes = kRows * kRowBytes, kStageV = kRows / 4 * M::kPitch;
   // two pipeline stages per group, distinct arrays so that reads of one stage need not wait for the
@@ -352,12 +353,6 @@ __device__ __forceinline__ void fwd_lines(const FwdParams& p) {
   float l_tot[2];
 #pragma unroll
   for (int n = 0; n < M::kCols; ++n) l_tot[n] = M::column_sum(st[n].l_run);
-  auto inverse = [&]() {
-    RowPair r;
-#pragma unroll
-    for (int n = 0; n < M::kCols; ++n) r.x[n] = l_tot[n] > 0.f ? 1.f / l_tot[n] : 0.f;
-    return r;
-  };
   // (what only the end needs is read from the kernel-argument segment now: it would occupy scalar registers during a long walk)
   const FwdParams& pe = kForm == 1 ? *(const FwdParams*)params_late() : p;
   bf16* orow = pe.o + b * pe.os.b + (int64_t)qrow0 * pe.os.s + h * pe.os.h;
@@ -372,48 +367,43 @@ __device__ __forceinline__ void fwd_lines(const FwdParams& p) {
     o_stride = (int64_t)pe.n_heads * kHeadDim;
   }
   if constexpr (kForm == 1) {
-    const RowPair inv = inverse();
+    RowPair inv;
+#pragma unroll
+    for (int n = 0; n < M::kCols; ++n) inv.x[n] = l_tot[n] > 0.f ? 1.f / l_tot[n] : 0.f;
     const uint32_t turn = lds_at((wave < 2 ? kA : vA) + (wave & 1) * kWaveRowsBytes);
     if (part >= 0 && pe.part_f32)   store_rows_f32<kM>(static_cast<float*>(pe.part_o) + part_at, o_stride, oacc, inv, turn);
     else                            store_rows_bf16<kM>(orow, o_stride, oacc, inv, turn);
   } else {
     // the groups exchange their rows' max, sum and O.  Area x of the stages' LDS belongs to group x % kForm of wave x / kForm.
-    __shared__ float stat[8][M::kCols][2][64];
+    __shared__ float stat[8][2][64];
     auto area = [&](int x) { return lds_at(x < 2 ? sKA : x < 4 ? sVA : x < 6 ? sKB : sVB) + (x & 1) * kAccBytes; };
     const int own = wave * kForm + group;
     constexpr bool kAll = kForm == 2;        // the first group finishes whole rows; with four groups each a block of 32 columns
-#pragma unroll
-    for (int n = 0; n < M::kCols; ++n) {
-      stat[own][n][0][lane] = st[n].m_run;
-      stat[own][n][1][lane] = l_tot[n];
-    }
+    stat[own][0][lane] = st[0].m_run;
+    stat[own][1][lane] = l_tot[0];
     if (!kAll || group == 1) put_acc(area(own), oacc, kAll ? -1 : group);
     __syncthreads();
     if (kAll && group == 1) return;
-    RowPair w[kForm];
+    float m = -INFINITY, w[kForm];
 #pragma unroll
-    for (int n = 0; n < M::kCols; ++n) {
-      float m = -INFINITY;
+    for (int g = 0; g < kForm; ++g) m = fmaxf(m, stat[wave * kForm + g][0][lane]);
+    const float ms = m == -INFINITY ? 0.f : m;
+    l_tot[0] = 0.f;
 #pragma unroll
-      for (int g = 0; g < kForm; ++g) m = fmaxf(m, stat[wave * kForm + g][n][0][lane]);
-      const float ms = m == -INFINITY ? 0.f : m;
-      l_tot[n] = 0.f;
-#pragma unroll
-      for (int g = 0; g < kForm; ++g) {
-        w[g].x[n] = fast_exp2(stat[wave * kForm + g][n][0][lane] - ms);
-        l_tot[n] += stat[wave * kForm + g][n][1][lane] * w[g].x[n];
-      }
-      st[n].m_run = m;
+    for (int g = 0; g < kForm; ++g) {
+      w[g] = fast_exp2(stat[wave * kForm + g][0][lane] - ms);
+      l_tot[0] += stat[wave * kForm + g][1][lane] * w[g];
     }
-    const RowPair inv = inverse();
+    st[0].m_run = m;
+    const float inv = l_tot[0] > 0.f ? 1.f / l_tot[0] : 0.f;
     if constexpr (kAll) {
 #pragma unroll
-      for (int mb = 0; mb < 4; ++mb) add_block<kM>(area(own + 1), mb, oacc[mb], w[0], w[1]);
-      store_rows_bf16<kM>(orow, o_stride, oacc, inv, area(own + 1));
+      for (int mb = 0; mb < 4; ++mb) add_block(area(own + 1), mb, oacc[mb], w[0], w[1]);
+      store_rows_bf16<kM>(orow, o_stride, oacc, both(inv), area(own + 1));
     } else {
       f32x16 o;
-      sum_blocks<kM>(o, oacc, group, [&](int g) { return area(wave * kForm + g); }, w);
-      store_block_bf16<kM>(orow + 32 * group, o_stride, o, inv, area(own) + 4096 * group);
+      sum_blocks(o, oacc, group, [&](int g) { return area(wave * kForm + g); }, w);
+      store_block_bf16(orow + 32 * group, o_stride, o, inv, area(own) + 4096 * group);
     }
   }
   const int out_lane = fresh_lane();

@@ -312,19 +312,17 @@ __device__ __forceinline__ void store_rows_f32(float* rows, int64_t row_stride, 
   }
 }
 
-// One block of 32 columns of the same rows (a wave's share after a sum over groups), `rows` already at the block; through 2
-// or 4 KiB of LDS.
-template <int kM>
-__device__ __forceinline__ void store_block_bf16(bf16* rows, int64_t row_stride, const f32x16& acc, RowPair mul, uint32_t lds) {
-  using M = Mma<kM>;
-  const int lane = fresh_lane();
+// What follows serves the walks of several groups a line, which run on 32x32x16: a lane holds one of the 32 rows.
+// One block of 32 columns of the same rows (a wave's share after a sum over groups): acc[4g + j] = column
+// 8 * g + 4 * (lane / 32) + j of row lane % 32, `rows` already at the block; through 2 or 4 KiB of LDS.
+__device__ __forceinline__ void store_block_bf16(bf16* rows, int64_t row_stride, const f32x16& acc, float mul, uint32_t lds) {
+  const int lane = fresh_lane(), r = lane & 31;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = M::col(lane, M::quad_n(i));
+  for (int g = 0; g < 4; ++g) {
     bf16x4 w;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) w[j] = (bf16)(acc[4 * i + j] * mul.x[M::quad_n(i)]);
-    lds_put(lds + r * 64 + ((M::quad_chunk(lane, i) ^ (r >> 2 & 3)) << 4) + 8 * M::quad_half(lane), w);
+    for (int j = 0; j < 4; ++j) w[j] = (bf16)(acc[4 * g + j] * mul);
+    lds_put(lds + r * 64 + ((g ^ (r >> 2 & 3)) << 4) + 8 * (lane >> 5), w);
   }
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
@@ -332,16 +330,12 @@ __device__ __forceinline__ void store_block_bf16(bf16* rows, int64_t row_stride,
     *reinterpret_cast<u32x4*>(rows + row * row_stride + 8 * c) = lds_get<u32x4>(lds + row * 64 + ((c ^ (row >> 2 & 3)) << 4));
   }
 }
-template <int kM>
-__device__ __forceinline__ void store_block_f32(float* rows, int64_t row_stride, const f32x16& acc, RowPair mul, uint32_t lds) {
-  using M = Mma<kM>;
-  const int lane = fresh_lane();
+__device__ __forceinline__ void store_block_f32(float* rows, int64_t row_stride, const f32x16& acc, float mul, uint32_t lds) {
+  const int lane = fresh_lane(), r = lane & 31;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = M::col(lane, M::quad_n(i));
-    const float f = mul.x[M::quad_n(i)];
-    lds_put(lds + r * 128 + ((M::quad_piece(lane, i) ^ (r >> 1 & 7)) << 4), f32x4{acc[4 * i] * f, acc[4 * i + 1] * f, acc[4 * i + 2] * f, acc[4 * i + 3] * f});
-  }
+  for (int g = 0; g < 4; ++g)
+    lds_put(lds + r * 128 + (((2 * g + (lane >> 5)) ^ (r >> 1 & 7)) << 4),
+            f32x4{acc[4 * g] * mul, acc[4 * g + 1] * mul, acc[4 * g + 2] * mul, acc[4 * g + 3] * mul});
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int row = 8 * i + (lane >> 3), c = lane & 7;
@@ -361,28 +355,27 @@ __device__ __forceinline__ void put_acc(uint32_t lds, const f32x16 (&acc)[4], in
   }
 }
 // acc = acc * wa + (block mb in LDS) * wb
-template <int kM>
-__device__ __forceinline__ void add_block(uint32_t lds, int mb, f32x16& acc, RowPair wa, RowPair wb) {
+__device__ __forceinline__ void add_block(uint32_t lds, int mb, f32x16& acc, float wa = 1.f, float wb = 1.f) {
   lds += 16 * fresh_lane() + 4096 * mb;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const f32x4 x = lds_get<f32x4>(lds + 1024 * i);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[4 * i + j] = acc[4 * i + j] * wa.x[Mma<kM>::quad_n(i)] + x[j] * wb.x[Mma<kM>::quad_n(i)];
+    for (int j = 0; j < 4; ++j) acc[4 * i + j] = acc[4 * i + j] * wa + x[j] * wb;
   }
 }
 // sum = the groups' blocks `own` in order, times w: this wave's from its accumulators, the other groups' from at(g).
 // (Its own block through LDS as well was a fourth of what the four groups' end moves there: 8 heads of 1024, forward
 // 12.85 -> 12.75 us, backward 19.8 -> 19.4; 32 of 512, forward 10.2 -> 9.9.)
-template <int kM, class At>
-__device__ __forceinline__ void sum_blocks(f32x16& sum, const f32x16 (&acc)[4], int own, At at, const RowPair (&w)[4]) {
+template <class At>
+__device__ __forceinline__ void sum_blocks(f32x16& sum, const f32x16 (&acc)[4], int own, At at, const float (&w)[4]) {
   sum = f32x16{0};
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
-    if (g != own) add_block<kM>(at(g), own, sum, both(1.f), w[g]);
+    if (g != own) add_block(at(g), own, sum, 1.f, w[g]);
     if (g == own) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) sum[i] += acc[g][i] * w[g].x[Mma<kM>::quad_n(i >> 2)];
+      for (int i = 0; i < 16; ++i) sum[i] += acc[g][i] * w[g];
     }
   }
 }
