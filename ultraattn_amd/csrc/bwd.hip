@@ -175,7 +175,7 @@ __device__ __forceinline__ bf16x8 pair_nat(const PairAddr<kM>& ad, int i) {
 template <int kOff, int kM>
 __device__ __forceinline__ bf16x8 pair_tr(const PairAddr<kM>& ad, int i) {
   using M = Mma<kM>;
-  return lds_abs_tr_pair(ad.tr[M::tr_reg(i)] + (kOff + M::tr_first(i)), ad.tr[M::tr_reg(i)] + (kOff + M::tr_first(i) + M::kTrSecond));
+  return lds_abs_tr_pair(ad.tr[M::tr_reg(i)] + (kOff + M::tr_first(i)), ad.tr[M::tr_reg(i)] + (kOff + M::tr_first(i) + M::tr_second()));
 }
 
 // The walked pair of operands (Q and dO, or K and V): asynchronous copies of a group's rows into an LDS stage.

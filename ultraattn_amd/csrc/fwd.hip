@@ -102,8 +102,8 @@ __device__ __forceinline__ void key_blocks(const unsigned char* sK, const unsign
   constexpr int kVAhead = 3;
   bf16x8 vfr[4];
   auto rd_v = [&](int i) {               // fragment i % 8 of 32 keys
-    const int at = tr[M::tr_reg(i & 7)] + M::tr_first(i & 7) + 8 * M::kPitch * (i >> 3);
-    const bf16x4 lo = lds_read_tr16_b64(sV, at), hi = lds_read_tr16_b64(sV, at + M::kTrSecond);
+    const int at = tr[M::tr_reg(i & 7)] + M::tr_first(i & 7, M::kPitchV) + 8 * M::kPitchV * (i >> 3);
+    const bf16x4 lo = lds_read_tr16_b64(sV, at), hi = lds_read_tr16_b64(sV, at + M::tr_second(M::kPitchV));
     return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
   };
 #pragma unroll
@@ -177,7 +177,7 @@ __device__ __forceinline__ void fwd_lines(const FwdParams& p) {
   using M = Mma<kM>;
   static_assert(kForm == 1 || kM == 32, "the groups' exchange takes a lane to hold one row");
   constexpr int kWaves = Groups<kForm>::kWaves, kRows = Groups<kForm>::kRows, kLines = Groups<kForm>::kLines;
-  constexpr int kStageBytes = kRows * kRowBytes, kStageV = kRows / 4 * M::kPitch;
+  constexpr int kStageBytes = kRows * kRowBytes, kStageV = kRows / 4 * M::kPitchV;
   // two pipeline stages per group, distinct arrays so that reads of one stage need not wait for the
   // copies in flight into the other
   __shared__ __attribute__((aligned(1024))) unsigned char sKA[kForm * kStageBytes];
@@ -239,15 +239,15 @@ __device__ __forceinline__ void fwd_lines(const FwdParams& p) {
   };
   // Where the wave's copies land in a stage; made opaque in every step, as the sums with the stages' addresses would occupy scalar
   // registers all along (and 15 to 24 of those vector lanes).
-  int k_wave = wave * 1024, v_wave = wave * M::kPitch;
+  int k_wave = wave * 1024, v_wave = wave * M::kPitchV;
   auto copy_piece = [&](int n, unsigned char* k_stage, unsigned char* v_stage, int part) {
     const int j = n >> 1;                  // (the offsets of pieces 16 rows apart differ by that alone: one register each for K and V)
-    if (n & 1) dma16_abs(v_rsrc, lds_at(v_stage) + 4 * M::kPitch * j + v_wave, voff[0], part * v_half + j * 32 * v_stride);
+    if (n & 1) dma16_abs(v_rsrc, lds_at(v_stage) + 4 * M::kPitchV * j + v_wave, voff[0], part * v_half + j * 32 * v_stride);
     else       dma16_abs(k_rsrc, lds_at(k_stage) + 4096 * j + k_wave, koff[0], part * k_half + j * 32 * k_stride);
   };
   auto copy_stage = [&](int t, unsigned char* k_stage, unsigned char* v_stage, int part) {
     dma_rows_buf<kWaves, 1024>(k_stage, make_rsrc(kbase + (int64_t)t * kTile * k_stride, k_extent), koff, part * k_half, wave);
-    dma_rows_buf<kWaves, M::kPitch>(v_stage, make_rsrc(vbase + (int64_t)t * kTile * v_stride, v_extent), voff, part * v_half, wave);
+    dma_rows_buf<kWaves, M::kPitchV>(v_stage, make_rsrc(vbase + (int64_t)t * kTile * v_stride, v_extent), voff, part * v_half, wave);
   };
 
   // A step is one half of a tile, in order; with more groups half or quarter `group` of a tile.
@@ -295,7 +295,7 @@ __device__ __forceinline__ void fwd_lines(const FwdParams& p) {
 #pragma unroll
   for (int i = 0; i < M::kRowRegs; ++i) nat[i] = lds_off_k(M::a_row(lane), M::a_chunk(lane, i));
 #pragma unroll
-  for (int i = 0; i < 4; ++i) tr[i] = M::tr_offset(lane, i);
+  for (int i = 0; i < 4; ++i) tr[i] = M::tr_offset(lane, i, M::kPitchV);
 
   bool started = false;
   auto step = [&](int e, auto stage_tag) {
@@ -432,7 +432,7 @@ template <int kWaveRows>
 __global__ __launch_bounds__(512, 2) void fwd_short_kernel(const FwdParams p) {
   using M = Mma<16>;
   static_assert(kWaveRows == 16 && M::kCols * 16 == 32, "one of the two columns that a lane of fwd_kernel holds");
-  constexpr int kHalfRows = 64, kStageK = kHalfRows * kRowBytes, kStageV = kHalfRows / 4 * M::kPitch;
+  constexpr int kHalfRows = 64, kStageK = kHalfRows * kRowBytes, kStageV = kHalfRows / 4 * M::kPitchV;
   __shared__ __attribute__((aligned(1024))) unsigned char sKA[kStageK];
   __shared__ __attribute__((aligned(1024))) unsigned char sVA[kStageV];
   __shared__ __attribute__((aligned(1024))) unsigned char sKB[kStageK];
@@ -458,7 +458,7 @@ __global__ __launch_bounds__(512, 2) void fwd_short_kernel(const FwdParams p) {
   };
   auto copy = [&](int n, unsigned char* k_stage, unsigned char* v_stage, int half) {
     const int j = n >> 1, first = half * kHalfRows + 32 * j;
-    if (n & 1) dma16_abs(v_rsrc, lds_at(v_stage) + (8 * j + wave) * M::kPitch, voff, first * v_stride * 2);
+    if (n & 1) dma16_abs(v_rsrc, lds_at(v_stage) + (8 * j + wave) * M::kPitchV, voff, first * v_stride * 2);
     else       dma16_abs(k_rsrc, lds_at(k_stage) + (8 * j + wave) * 1024, koff, first * k_stride * 2);
   };
   Walk<false, true> walk(e0, e1, -1);
@@ -485,7 +485,7 @@ __global__ __launch_bounds__(512, 2) void fwd_short_kernel(const FwdParams p) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     nat[i] = lds_off_k(M::a_row(lane), M::a_chunk(lane, i));
-    tr[i] = M::tr_offset(lane, i);
+    tr[i] = M::tr_offset(lane, i, M::kPitchV);
   }
   auto step = [&](int e, auto stage_tag) {
     constexpr int kStage = decltype(stage_tag)::value;
@@ -523,8 +523,8 @@ __global__ __launch_bounds__(512, 2) void fwd_short_kernel(const FwdParams p) {
       constexpr int kVAhead = 4;
       bf16x8 vfr[16];
       auto rd_v = [&](int i) {
-        const int at = tr[(i & 7) >> 1] + M::tr_first(i & 7) + 8 * M::kPitch * (i >> 3);
-        const bf16x4 lo = lds_read_tr16_b64(sV, at), hi = lds_read_tr16_b64(sV, at + M::kTrSecond);
+        const int at = tr[(i & 7) >> 1] + M::tr_first(i & 7, M::kPitchV) + 8 * M::kPitchV * (i >> 3);
+        const bf16x4 lo = lds_read_tr16_b64(sV, at), hi = lds_read_tr16_b64(sV, at + M::tr_second(M::kPitchV));
         return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
       };
 #pragma unroll

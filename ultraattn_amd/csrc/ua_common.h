@@ -72,7 +72,7 @@ struct Mma<16> {
   // different 64-byte groups, the two fours in different halves of one.  A 128-bit read of 16 rows is served 16 lanes
   // at a time, half of the rows from either of two adjacent lane groups, whose chunks differ by one: different slots, too.  (With the fours'
   // starts 0, 32, 16 and 48 bytes into a 64-byte group the backward, 32 heads of 4096, met 68 million conflict cycles, so 0.8.)
-  static constexpr int kPitch = 1056;
+  static constexpr int kPitch = 1056, kPitchV = kPitch;
   static __device__ __forceinline__ int col(int lane, int n) { return 16 * n + (lane & 15); }
   static __device__ __forceinline__ int quad_row(int lane, int q) { return 16 * (q >> 1) + 4 * (lane >> 4); }
   static constexpr __device__ int quad_n(int q) { return q & 1; }
@@ -90,13 +90,13 @@ struct Mma<16> {
   static constexpr __device__ int a_offset(int i, int four_pitch) { return (i & 1) * 4 * four_pitch; }
   // Second product, contracted over 32 rows: A fragment i = columns 16 * i .. + 15, all rows, read through the transposing path
   // as two halves: lane group g supplies rows 4g .. 4g + 3 and 16 + 4g .., as two blocks of 16 accumulator rows do.
-  static __device__ __forceinline__ int tr_offset(int lane, int m) {
+  static __device__ __forceinline__ int tr_offset(int lane, int m, int pitch = kPitch) {
     const int g = lane >> 4, r = (lane & 15) >> 2, c = lane & 3;
-    return kPitch * g + r * kRowBytes + (slot_v(r, 4 * m + (c >> 1)) << 4) + (c & 1) * 8;
+    return pitch * g + r * kRowBytes + (slot_v(r, 4 * m + (c >> 1)) << 4) + (c & 1) * 8;
   }
   static constexpr __device__ int tr_reg(int i) { return i >> 1; }
-  static constexpr __device__ int tr_first(int i) { return 32 * (i & 1); }
-  static constexpr int kTrSecond = 4 * kPitch;
+  static constexpr __device__ int tr_first(int i, int = kPitch) { return 32 * (i & 1); }
+  static constexpr __device__ int tr_second(int pitch = kPitch) { return 4 * pitch; }
   static constexpr __device__ int slot_n(int i) { return i >> 2 & 1; }                    // where acc[i] goes in the next B operand
   static constexpr __device__ int slot_j(int i) { return 4 * (i >> 3) + (i & 3); }
   static __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
@@ -141,7 +141,8 @@ struct Mma<16> {
 template <>
 struct Mma<32> {
   static constexpr int kCols = 1, kRowRegs = 8;
-  static constexpr int kPitch = 1040;      // (the rows of two fours that a half wave gathers are whole 64-byte groups)
+  // (The rows of two fours that a half wave gathers are whole 64-byte groups.)  V of the forward, of which no rows are read, lies at 1024.
+  static constexpr int kPitch = 1040, kPitchV = 1024;
   static __device__ __forceinline__ int col(int lane, int) { return lane & 31; }
   static __device__ __forceinline__ int quad_row(int lane, int q) { return 8 * q + 4 * (lane >> 5); }
   static constexpr __device__ int quad_n(int) { return 0; }
@@ -156,13 +157,13 @@ struct Mma<32> {
   static constexpr __device__ int a_reg(int i) { return i; }
   static constexpr __device__ int a_offset(int, int) { return 0; }
   // Second product: A fragment i = columns 32 * (i % 4) .. + 31, 16 rows from 16 * (i / 4) on; lane half h supplies rows 4h .. 4h + 3 and 8 + 4h ..
-  static __device__ __forceinline__ int tr_offset(int lane, int m) {
+  static __device__ __forceinline__ int tr_offset(int lane, int m, int pitch = kPitch) {
     const int i16 = lane & 15, r = i16 >> 2;
-    return kPitch * (lane >> 5) + r * kRowBytes + (slot_v(r, 4 * m + 2 * (lane >> 4 & 1) + ((i16 & 3) >> 1)) << 4) + (i16 & 1) * 8;
+    return pitch * (lane >> 5) + r * kRowBytes + (slot_v(r, 4 * m + 2 * (lane >> 4 & 1) + ((i16 & 3) >> 1)) << 4) + (i16 & 1) * 8;
   }
   static constexpr __device__ int tr_reg(int i) { return i & 3; }
-  static constexpr __device__ int tr_first(int i) { return 4 * kPitch * (i >> 2); }
-  static constexpr int kTrSecond = 2 * kPitch;
+  static constexpr __device__ int tr_first(int i, int pitch = kPitch) { return 4 * pitch * (i >> 2); }
+  static constexpr __device__ int tr_second(int pitch = kPitch) { return 2 * pitch; }
   static constexpr __device__ int slot_n(int i) { return i >> 3; }
   static constexpr __device__ int slot_j(int i) { return i & 7; }
   static __device__ __forceinline__ f32x16 mfma(bf16x8 a, bf16x8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
