@@ -204,6 +204,10 @@ struct PairStream {
   }
   // (Opaque in every step: the sums of the copies' LDS addresses would occupy scalar registers all along, and vector lanes.)
   __device__ __forceinline__ void next_step() { asm volatile("" : "+s"(lds)); }
+  // The same for the strides, from which the copies then form their rows' offsets anew: dQ's walk of half lines had ten scalars in vector
+  // lanes otherwise and with them a private segment of 20 bytes, which no instruction used but every launch paid for (32 heads of 512, forward and
+  // backward, 34.93 -> 34.82 us).
+  __device__ __forceinline__ void next_strides() { asm volatile("" : "+s"(xs), "+s"(ys)); }
   // copy n of kCopies into stage kStage, rows from 64 or 32 * part of the tile on
   template <int kStage>
   __device__ __forceinline__ void copy(int n, int part) const {
@@ -472,7 +476,7 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& given, uint32_t lds_b
     }
     put_stat(kStage ^ 1, stat);
     stat = S::kSteps == 2 ? load_stat(ent_next, part_of(kStage)) : load_stat(walk.at(min(e + 2, e1 - 1)), group);
-    in.next_step();
+    if (kForm != kHalves) in.next_step();
     if (!kFirst) in.tile(walk.tile(ent_next), e + 1 < e1);
     const bool causal = (ent >> 30) != 0;
     // causal tile: query block nb sees none of the wave's keys when nb < k_block, some when nb == k_block
@@ -702,6 +706,7 @@ __device__ __forceinline__ void dq_walk(const BwdParams& given, uint32_t lds_blo
     // (of a list beside the first block, which one group always sees; a group of several may see none of its blocks)
     if (kDense) look_ahead();
     in.next_step();
+    if (kForm == kHalves) in.next_strides();
     if (!kFirst) in.tile(walk.tile(ent_next), e + 1 < e1);
     wait_vmem_all();
     __syncthreads();            // this stage has landed; everyone is done with the other one, which the copies now fill
