@@ -34,3 +34,31 @@ def test_no_kernel_has_a_private_segment(assembly):
     """One of 20 bytes, which no instruction used, made a backward of half lines and the launch before it longer."""
     sizes = _metadata(assembly, "private_segment_fixed_size")
     assert len(sizes) >= 12 and not any(sizes.values()), sizes
+
+
+# One group of waves a workgroup: what launches of more than a few hundred lines run, and all tile lists.
+ONE_GROUP = ["fwd_kernelILi1ELb0EE", "fwd_kernelILi1ELb1EE", "fwd_plain_kernelILi16EE", "fwd_short_kernelILi16EE",
+             "bwd_kernelILi1ELb0EE", "bwd_kernelILi1ELb1EE", "11dkdv_kernelE", "9dq_kernelE"]
+SEVERAL = ["fwd_kernelILi2ELb1EE", "fwd_kernelILi4ELb1EE", "bwd_kernelILi3ELb1EE", "bwd_kernelILi4ELb1EE"]
+
+
+def test_one_group_keeps_its_registers(assembly):
+    """All kernels of one group by name: no scalars in vector lanes, no vector registers in memory."""
+    scalars, vectors = _metadata(assembly, "sgpr_spill_count"), _metadata(assembly, "vgpr_spill_count")
+    for name in scalars:
+        assert sum(n in name + "E" for n in ONE_GROUP + SEVERAL) == 1, name
+    for n in ONE_GROUP:
+        found = [name for name in scalars if n in name]
+        assert len(found) == 1 and scalars[found[0]] == vectors[found[0]] == 0, (n, found)
+    assert not any(vectors.values()), vectors
+
+
+# (two half tiles, two products: 64 of 32x32x16 or 128 of 16x16x32)
+@pytest.mark.parametrize("kernel,mfmas", [("fwd_kernelILi1ELb0EE", 128), ("fwd_kernelILi1ELb1EE", 64), ("fwd_plain_kernelILi16EE", 128)])
+def test_no_address_arithmetic_between_matrix_instructions_of_either_kind(assembly, kernel, mfmas):
+    body = re.search(rf"^_ZN2ua\d+{kernel}\w*:.*?^\.Lfunc_end", assembly["fwd.hip"], flags=re.M | re.S).group(0)
+    blocks = [re.findall(r"^[ \t]+((?:[vs]|ds|buffer)_\w+)[ \t]*(.*)$", b, flags=re.M) for b in re.split(r"^(?:\.LBB\w+:|; %bb\.\d+:).*$", body, flags=re.M)]
+    walk = [b for b in blocks if any("mfma" in op for op, _ in b)]
+    assert sum("mfma" in op for b in walk for op, _ in b) == mfmas
+    integer = [f"{op} {args}" for b in walk for op, args in b if re.match(r"v_\w*(?:_u32|_i32|_b32|_u64|_b64)", op)]
+    assert not integer, integer
