@@ -115,6 +115,7 @@ def probe_lib():
         lib.bench_probe_mfma.restype, lib.bench_probe_mfma.argtypes = ci, [vp, vp, ci, ci, vp]
         lib.bench_probe_mfma_rotating.restype, lib.bench_probe_mfma_rotating.argtypes = ci, [vp, vp, ci, ci, vp]
         lib.bench_probe_mfma16_rotating.restype, lib.bench_probe_mfma16_rotating.argtypes = ci, [vp, vp, ci, ci, vp]
+        lib.bench_probe_mfma_reuse.restype, lib.bench_probe_mfma_reuse.argtypes = ci, [vp, vp, ci, ci, ci, ci, ci, vp]
         lib.bench_atomic_rate.restype, lib.bench_atomic_rate.argtypes = ci, [vp, ctypes.c_int64, ci, ci, ci, vp]
         lib.bench_stream_mix.restype = ci
         lib.bench_stream_mix.argtypes = [ctypes.POINTER(vp), ci, vp, ctypes.c_int64, ci, ci, vp]
@@ -586,10 +587,19 @@ def run_power(name):
     return out
 
 
+# (rows of the instruction, times an A operand is used in a row, whether the B operands come in turn forwards and backwards)
+MFMA_REUSE = [(rows, reuse, turn) for rows in (16, 32) for reuse, turn in ((1, 0), (2, 0), (2, 1), (4, 0), (4, 1))]
+
+
+def mfma_reuse_key(rows, reuse, turn):
+    shape = "16x16x32" if rows == 16 else "32x32x16"
+    return f"random_{shape}_a_used_{reuse}_times" + ("_b_in_turn" if turn else "")
+
+
 def probe_mfma(peak):
     """Sustained register-only MFMA rates: constant and random operand bits; both dense bf16
     instructions (32x32x16 and 16x16x32) with operands that change on every instruction, at 1 and at
-    2 waves per SIMD.  `measured_ceiling_tflops` = the best of the random-data figures: what the
+    2 waves per SIMD, and with operands that the next instruction uses again.  `measured_ceiling_tflops` = the best of the random-data figures: what the
     matrix pipes of this device deliver to any bf16 kernel fed with ordinary data."""
     import torch
     lib = probe_lib()
@@ -609,21 +619,35 @@ def probe_mfma(peak):
              ("rotating_random_1_wave_per_simd_tflops", lib.bench_probe_mfma_rotating, rot, 256, 80000, f32),
              ("rotating_random_16x16x32_tflops", lib.bench_probe_mfma16_rotating, rot, 512, 40000, f16),
              ("rotating_random_16x16x32_1_wave_per_simd_tflops", lib.bench_probe_mfma16_rotating, rot, 256, 80000, f16)]
+    for rows, reuse, turn in MFMA_REUSE:
+        runs.append((mfma_reuse_key(rows, reuse, turn) + "_tflops",
+                     lambda t, o, n, i, s, a=(rows, reuse, turn): lib.bench_probe_mfma_reuse(t, o, n, i, *a, s),
+                     rot, 512, 64000 // reuse, reuse * (16384.0 if rows == 16 else 32768.0)))
     for key, fn, t, n_blocks, iters, flop in runs:
-        assert fn(t.data_ptr(), out.data_ptr(), n_blocks, 2000, st) == 0
-        torch.cuda.synchronize()
-        e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        # 0.3 s before the clock has settled at what the power limit allows, then 0.3 s timed
+        launch = lambda: fn(t.data_ptr(), out.data_ptr(), n_blocks, iters, st)
+        assert launch() == 0
+        n, e0, e1 = 40, torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        for _ in range(2):
+            e0.record()
+            assert not any([launch() for _ in range(n)])
+            e1.record()
+            torch.cuda.synchronize()
+            ms = e0.elapsed_time(e1) / n
+            n = max(1, int(300 / ms))
+        assert not any([launch() for _ in range(n)])
         e0.record()
-        assert fn(t.data_ptr(), out.data_ptr(), n_blocks, iters, st) == 0
+        assert not any([launch() for _ in range(n)])
         e1.record()
         torch.cuda.synchronize()
-        res[key] = n_blocks * 4 * iters * flop / e0.elapsed_time(e1) / 1e9
+        res[key] = n_blocks * 4 * iters * flop / (e0.elapsed_time(e1) / n) / 1e9
     res["frac_of_peak_random"] = res["random_operands_tflops"] / peak
     res["measured_ceiling_tflops"] = max(v for k, v in res.items() if "random" in k and k.endswith("_tflops"))
     res["measured_ceiling_frac_of_peak"] = res["measured_ceiling_tflops"] / peak
     res["note"] = ("register-only MFMA loops, 512 (2 waves per SIMD) or 256 (1 wave per SIMD) workgroups of 4 waves: one A/B "
                    "operand pair reused for ever (constant bits, random N(0,1) bits), and 8x8 random fragments cycled so that "
-                   "the operands change on every instruction, for v_mfma_f32_32x32x16_bf16 and v_mfma_f32_16x16x32_bf16; the "
+                   "the operands change on every instruction, for v_mfma_f32_32x32x16_bf16 and v_mfma_f32_16x16x32_bf16, or every A "
+                   "fragment used 2 or 4 times in a row, as the attention walks use theirs twice with 16x16x32; the "
                    "clock follows power, power follows operand bit activity, so the best random figure is the practical "
                    "ceiling of any bf16 MFMA kernel on this device")
     return res
@@ -675,6 +699,12 @@ def device_ceilings(peak):
                            ("rotating_random", lib.bench_probe_mfma_rotating, rot)):
             out["mfma"][key + "_power"] = sampler.measure(lambda: fn(t.data_ptr(), sink.data_ptr(), 512, 20000, st), 1.5,
                                                           torch.cuda.synchronize)
+        out["mfma"]["rotating_random_16x16x32_power"] = sampler.measure(
+            lambda: lib.bench_probe_mfma16_rotating(rot.data_ptr(), sink.data_ptr(), 512, 20000, st), 1.5, torch.cuda.synchronize)
+        for rows, reuse, turn in MFMA_REUSE:
+            out["mfma"][mfma_reuse_key(rows, reuse, turn) + "_power"] = sampler.measure(
+                lambda: lib.bench_probe_mfma_reuse(rot.data_ptr(), sink.data_ptr(), 512, 64000 // reuse, rows, reuse, turn, st), 1.5,
+                torch.cuda.synchronize)
     atom = {}
     n_blocks, iters = 2048, 2048
     for mib in (8, 1024):

@@ -10,6 +10,9 @@
 //                      instruction, for v_mfma_f32_32x32x16_bf16 and v_mfma_f32_16x16x32_bf16; with 256 or 512
 //                      workgroups of 4 waves (1 or 2 waves per SIMD) they give the device's ceiling rather than
 //                      one instruction's at one occupancy.
+//   bench_probe_mfma_reuse: every A operand used 1, 2 or 4 times in a row, as a product of 16 or 32 rows with several columns does, the B
+//                      operands each time in the same order or (`turn`) in turn forwards and backwards, so that every instruction
+//                      shares an operand with the one before it.
 //   bench_stream_mix   n_src streams read and one written with 16-byte accesses, the access
 //                      shape of the merge kernel: the device's rate for that read:write mix.
 //   bench_atomic_rate  device-wide rate of L2 atomics (fp32 add, u32 add, f64 add) and of plain dword
@@ -101,6 +104,38 @@ __global__ __launch_bounds__(256) void probe_mfma16_rot_kernel(const u32x4* in, 
   for (int i = 0; i < 8; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) s += c[i][j];
+  out[blockIdx.x * 256 + threadIdx.x] = s;
+}
+
+// Operands that are used again: A fragment u times kReuse B fragments, which every two A fragments have in common (1: both change every time).
+__device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ f32x16 mfma(bf16x8 a, bf16x8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
+template <class Acc, int kAccs, int kReuse, bool kTurn>
+__global__ __launch_bounds__(256) void probe_mfma_reuse_kernel(const u32x4* in, float* out, int iters) {
+  bf16x8 a[8], b[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const u32x4 ra = in[(2 * i) * 256 + threadIdx.x], rb = in[(2 * i + 1) * 256 + threadIdx.x];
+    __builtin_memcpy(&a[i], &ra, 16);
+    __builtin_memcpy(&b[i], &rb, 16);
+  }
+  Acc c[kAccs];
+#pragma unroll
+  for (int i = 0; i < kAccs; ++i) c[i] = Acc{0};
+  for (int it = 0; it < iters; it += 256 / kReuse) {
+#pragma unroll
+    for (int u = 0; u < 256 / kReuse; ++u)
+#pragma unroll
+      for (int n = 0; n < kReuse; ++n) {
+        const int at = kReuse == 1 ? 3 * u : kReuse * ((u & 7) >> 1) + (kTurn && (u & 1) ? kReuse - 1 - n : n);
+        c[(kReuse * u + n) % kAccs] = mfma(a[u & 7], b[at & 7], c[(kReuse * u + n) % kAccs]);
+      }
+  }
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < kAccs; ++i)
+#pragma unroll
+    for (int j = 0; j < (int)(sizeof(Acc) / 4); ++j) s += c[i][j];
   out[blockIdx.x * 256 + threadIdx.x] = s;
 }
 
@@ -243,6 +278,23 @@ extern "C" int bench_probe_mfma16_rotating(const void* operands, float* out, int
   if (n_blocks <= 0 || iters <= 0) return -2;
   if (reinterpret_cast<uintptr_t>(operands) & 15) return -4;
   hipLaunchKernelGGL(probe_mfma16_rot_kernel, dim3(n_blocks), dim3(256), 0, (hipStream_t)stream,
+                     (const u32x4*)operands, out, iters);
+  return hipGetLastError() == hipSuccess ? 0 : -6;
+}
+
+// Same operand layout; every thread issues reuse x iters (rounded up to a multiple of 256) instructions of rows x rows (16 or 32).
+extern "C" int bench_probe_mfma_reuse(const void* operands, float* out, int n_blocks, int iters, int rows, int reuse, int turn, void* stream) {
+  if (!operands || !out) return -1;
+  if (n_blocks <= 0 || iters <= 0 || (rows != 16 && rows != 32) || (reuse != 1 && reuse != 2 && reuse != 4)) return -2;
+  if (reinterpret_cast<uintptr_t>(operands) & 15) return -4;
+  void (*const kernels[2][3][2])(const u32x4*, float*, int) = {
+      {{probe_mfma_reuse_kernel<f32x4, 8, 1, false>, probe_mfma_reuse_kernel<f32x4, 8, 1, false>},
+       {probe_mfma_reuse_kernel<f32x4, 8, 2, false>, probe_mfma_reuse_kernel<f32x4, 8, 2, true>},
+       {probe_mfma_reuse_kernel<f32x4, 8, 4, false>, probe_mfma_reuse_kernel<f32x4, 8, 4, true>}},
+      {{probe_mfma_reuse_kernel<f32x16, 4, 1, false>, probe_mfma_reuse_kernel<f32x16, 4, 1, false>},
+       {probe_mfma_reuse_kernel<f32x16, 4, 2, false>, probe_mfma_reuse_kernel<f32x16, 4, 2, true>},
+       {probe_mfma_reuse_kernel<f32x16, 4, 4, false>, probe_mfma_reuse_kernel<f32x16, 4, 4, true>}}};
+  hipLaunchKernelGGL(kernels[rows == 32][reuse / 2][turn != 0], dim3(n_blocks), dim3(256), 0, (hipStream_t)stream,
                      (const u32x4*)operands, out, iters);
   return hipGetLastError() == hipSuccess ? 0 : -6;
 }

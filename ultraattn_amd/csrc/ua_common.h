@@ -57,8 +57,9 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 // Both work on blocks of 32 x 32: acc[i] of a lane = row quad_row(i / 4) + i % 4, column col(quad_n(i / 4)).  The transposed products of the
 // walks turn a block's accumulators, packed to bf16, into the B operand of the next product without leaving the lane.
 //
-// On random operands, at the socket's power limit, a loop of 16x16x32 instructions that uses every A operand twice runs at 2.06
-// PFLOP/s, one of 32x32x16 at 1.75 (its accumulators take twice the register traffic a flop).  The long launches, which that
+// Register-only loops on random operands, at the socket's power limit: 16x16x32 runs at 2.0 to 2.1 GHz, 32x32x16 at 1.76 to 1.79.  With operands
+// that change every time that is 1.90 and 1.79 PFLOP/s, with every A operand used twice in a row, as the walks do with 16x16x32,
+// 1.98 and 1.81 (a B operand that two instructions share gives nothing).  The long launches, which that
 // limit holds, gain 3 to 5 % in the forward (strided 128k 17.7 -> 17.1 ms) and 7 to 8 % in the backward (causal 32k, 32 heads
 // 23.5 -> 21.7, strided 128k 57.8 -> 53.6), at 1.81 and 1.87 instead of 1.60 GHz.  But there are twice as many instructions to
 // issue: beside a wave that issues them another one's fma, exp2 and add take 28 cycles instead of 22, and a step of a lone
