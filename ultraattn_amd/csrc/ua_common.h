@@ -72,7 +72,8 @@ struct Mma<16> {
   // Pitch of the V-type layout's fours.  A transposing read gathers 32 bytes of each row of two fours per half wave: the rows are in
   // different 64-byte groups, the two fours in different halves of one.  A 128-bit read of 16 rows is served 16 lanes
   // at a time, half of the rows from either of two adjacent lane groups, whose chunks differ by one: different slots, too.  (With the fours'
-  // starts 0, 32, 16 and 48 bytes into a 64-byte group the backward, 32 heads of 4096, met 68 million conflict cycles, so 0.8.)
+  // starts 0, 32, 16 and 48 bytes into a 64-byte group the backward, 32 heads of 4096, met 68 million conflict cycles.  Now there are none in
+  // the walks; what is left, 0.8 million, is 384 a workgroup where its rows turn through LDS at the walk's ends.)
   static constexpr int kPitch = 1056, kPitchV = kPitch;
   static __device__ __forceinline__ int col(int lane, int n) { return 16 * n + (lane & 15); }
   static __device__ __forceinline__ int quad_row(int lane, int q) { return 16 * (q >> 1) + 4 * (lane >> 4); }
