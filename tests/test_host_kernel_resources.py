@@ -62,3 +62,16 @@ def test_no_address_arithmetic_between_matrix_instructions_of_either_kind(assemb
     assert sum("mfma" in op for b in walk for op, _ in b) == mfmas
     integer = [f"{op} {args}" for b in walk for op, args in b if re.match(r"v_\w*(?:_u32|_i32|_b32|_u64|_b64)", op)]
     assert not integer, integer
+
+
+@pytest.mark.parametrize("kernel", ["bwd_kernelILi1ELb0EE", "bwd_kernelILi1ELb1EE", "dkdv_kernelE"])
+def test_diagonal_tiles_do_not_wait_for_every_read(assembly, kernel):
+    """The block of dK/dV's second products on diagonal tiles (32 MFMAs, 32 transposing reads): its waits leave the next fragment's reads in flight,
+    but for the last fragment's (and the first one's at most)."""
+    body = re.search(rf"^_ZN2ua\d+{kernel}\w*:.*?^\.Lfunc_end", assembly["bwd.hip"], flags=re.M | re.S).group(0)
+    found = 0
+    for b in re.split(r"^(?:\.LBB\w+:|; %bb\.\d+:).*$", body, flags=re.M):
+        if b.count("v_mfma") == 32 and b.count("ds_read_b64_tr_b16") == 32:
+            found += 1
+            assert len(re.findall(r"lgkmcnt\(0\)", b)) <= 2, kernel
+    assert found == 2                                       # either half of a tile
