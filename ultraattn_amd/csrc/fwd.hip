@@ -643,11 +643,17 @@ static int fwd_groups(int64_t n, int64_t walk, int n_parts, bool dense_causal) {
   if (walk >= 2 && (2 * n <= kCus || (uneven && n <= kCus && walk >= 16))) return 4;
   return walk >= 3 && n <= (uneven ? 2 * kCus : kCus) ? 2 : 1;
 }
-// Tile lists of n lines that run with eight waves a workgroup: up to one line a CU (one head, causal 4096: 63.6 us with four waves, 59.0; 8 heads
-// of causal 4096 64.9, 61.0), up to a line on every other CU where nearly all lines are of full length (8 heads of 4096 in full 68.3,
-// 72.0, one head of 1024 19.2, 18.9).  Both give the same bits.
+// Tile lists of n lines that run with eight waves a workgroup: up to one line a CU, and up to seven on eight CUs where nearly all lines are of
+// full length.  Both kernels give the same bits, so that the line is drawn by time alone: us, four waves and eight
+//     lines                      128            208            240            256            320
+//     causal, 16 tiles     35.0   32.8    36.1   33.8    36.4   34.1    35.8   33.7    36.5   34.4
+//     causal, 64 tiles    122.9  113.5                                 125.5  115.8   126.3  121.2
+//     strided, 16 tiles    14.7   14.2    16.5   16.0    17.3   17.0    15.5   14.9    19.4   23.6
+//     global+local, 16     35.2   33.2    36.2   34.7    37.0   36.3    36.2   36.0    39.2   51.8
+//     full, 16 tiles       35.2   33.6    36.9   35.5    37.4   37.5    36.6   37.6    52.0   68.1
+//     full, 64 tiles      125.5  115.0                                 128.6  134.2   189.3  244.7
 static bool few_lines(const FwdParams& p, int64_t n) {
-  return n <= ((int64_t)4 * p.nnz <= (int64_t)3 * p.n_qtiles * p.n_ktiles ? kCus : kCus / 2);
+  return n <= ((int64_t)4 * p.nnz <= (int64_t)3 * p.n_qtiles * p.n_ktiles ? kCus : kCus / 8 * 7);
 }
 // `plain`: one group per workgroup, and of a dense rectangle the bits of its tile list.
 static int fwd_launch(FwdParams& p, bool plain, hipStream_t st) {
