@@ -75,3 +75,9 @@ def test_diagonal_tiles_do_not_wait_for_every_read(assembly, kernel):
             found += 1
             assert len(re.findall(r"lgkmcnt\(0\)", b)) <= 2, kernel
     assert found == 2                                       # either half of a tile
+
+
+def test_rows_leave_the_forward_whole(assembly):
+    """No kernel of the forward writes O in pieces of 8 bytes, 32 bytes of a row at a time: rows pass through LDS (the statistics are single dwords)."""
+    stores = set(re.findall(r"^\s+(global_store_\w+)", assembly["fwd.hip"], flags=re.M))
+    assert "global_store_dwordx4" in stores and stores <= {"global_store_dwordx4", "global_store_dword"}, stores

@@ -432,7 +432,7 @@ template <int kWaveRows>
 __global__ __launch_bounds__(512, 2) void fwd_short_kernel(const FwdParams p) {
   using M = Mma<16>;
   static_assert(kWaveRows == 16 && M::kCols * 16 == 32, "one of the two columns that a lane of fwd_kernel holds");
-  constexpr int kHalfRows = 64, kStageK = kHalfRows * kRowBytes, kStageV = kHalfRows / 4 * M::kPitchV;
+  constexpr int kHalfRows = 64, kStageK = kHalfRows * kRowBytes, kStageV = kHalfRows / 4 * M::kPitchV, kTurnBytes = kWaveRows * kRowBytes;
   __shared__ __attribute__((aligned(1024))) unsigned char sKA[kStageK];
   __shared__ __attribute__((aligned(1024))) unsigned char sVA[kStageV];
   __shared__ __attribute__((aligned(1024))) unsigned char sKB[kStageK];
@@ -471,10 +471,18 @@ __global__ __launch_bounds__(512, 2) void fwd_short_kernel(const FwdParams p) {
     for (int n = 0; n < 4; ++n) copy(n, sKA, sVA, 0);
   }
   const int qrow0 = qt * kTile + kWaveRows * wave, q_block = wave >> 1;
-  const bf16* const qrow = p.q + b * p.qs.b + (int64_t)(qrow0 + row) * p.qs.s + h * p.qs.h;
+  // Q rows come in, and O goes out, through LDS, so that memory sees whole rows (1.3 us of a walk of one tile, 7.5 -> 6.2 us)
+  // (through the stage that the first step fills)
+  const bf16* const qrow = p.q + b * p.qs.b + (int64_t)(qrow0 + (lane >> 4)) * p.qs.s + h * p.qs.h + 8 * row;
+  const uint32_t q_turn = lds_at(wave < 4 ? sKB : sVB) + (wave & 3) * kTurnBytes;
+  u32x4 raw[4];
   bf16x8 qf[4];
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks) qf[ks] = *reinterpret_cast<const bf16x8*>(qrow + 8 * M::a_chunk(lane, ks));
+  for (int i = 0; i < 4; ++i) raw[i] = *reinterpret_cast<const u32x4*>(qrow + 4 * i * p.qs.s);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) lds_put(q_turn + row_slot(4 * i + (lane >> 4), row), raw[i]);
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) qf[ks] = lds_get<bf16x8>(q_turn + row_slot(row, M::a_chunk(lane, ks)));
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks) asm volatile("" : "+v"(qf[ks]));      // read before the walk
   f32x4 oacc[8];
@@ -581,16 +589,21 @@ __global__ __launch_bounds__(512, 2) void fwd_short_kernel(const FwdParams p) {
     step(e, std::integral_constant<int, 0>{});
     step(e, std::integral_constant<int, 1>{});
   }
-  wait_vmem_all();
+  wait_vmem_all();              // the last step's copies filled with zeros a stage that is used for the results now
+  __syncthreads();
   const float l_tot = M::column_sum(l_run), inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-  bf16* const orow = p.o + b * p.os.b + (int64_t)(qrow0 + row) * p.os.s + h * p.os.h + 4 * (lane >> 4);
+  const uint32_t turn = lds_at(wave < 4 ? sKA : sVA) + (wave & 3) * kTurnBytes;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     bf16x4 w;
 #pragma unroll
     for (int j = 0; j < 4; ++j) w[j] = (bf16)(oacc[i][j] * inv);
-    *reinterpret_cast<bf16x4*>(orow + 16 * i) = w;
+    lds_put(turn + row_slot(row, 2 * i + (lane >> 5)) + 8 * (lane >> 4 & 1), w);
   }
+  bf16* const orow = p.o + b * p.os.b + (int64_t)(qrow0 + (lane >> 4)) * p.os.s + h * p.os.h + 8 * row;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    *reinterpret_cast<u32x4*>(orow + 4 * i * p.os.s) = lds_get<u32x4>(turn + row_slot(4 * i + (lane >> 4), row));
   if (lane < 16)
     p.lse[((int64_t)b * p.n_heads + h) * ((int64_t)p.n_qtiles * kTile) + qrow0 + lane] =
         l_tot > 0.f ? (m_run + __builtin_amdgcn_logf(l_tot)) * kLn2 : -INFINITY;
@@ -637,7 +650,7 @@ static int fwd_common(FwdParams& p, const void* q, const void* k, const void* v,
 // Groups sum in another order, so that the last bits of a row depend on how many lines the launch has.  Tile lists, whose
 // launches are shards of the rows and heads of one mask, therefore run with one group whatever their size: a row's result is
 // the same bit for bit in every launch that holds its list.  Lists of up to 128 lines pay for that (one head, causal 4096: forward
-// 35 us with four groups, 59 with one, see few_lines, backward 51 and 119; from 512 lines on little changes).
+// 35 us with four groups, 58 with one, see few_lines, backward 51 and 119; from 512 lines on little changes).
 static int fwd_groups(int64_t n, int64_t walk, int n_parts, bool dense_causal) {
   const bool uneven = dense_causal && n_parts == 1;
   if (walk >= 2 && (2 * n <= kCus || (uneven && n <= kCus && walk >= 16))) return 4;
@@ -646,12 +659,12 @@ static int fwd_groups(int64_t n, int64_t walk, int n_parts, bool dense_causal) {
 // Tile lists of n lines that run with eight waves a workgroup: up to one line a CU, and up to seven on eight CUs where nearly all lines are of
 // full length.  Both kernels give the same bits, so that the line is drawn by time alone: us, four waves and eight
 //     lines                      128            208            240            256            320
-//     causal, 16 tiles     35.0   32.8    36.1   33.8    36.4   34.1    35.8   33.7    36.5   34.4
-//     causal, 64 tiles    122.9  113.5                                 125.5  115.8   126.3  121.2
-//     strided, 16 tiles    14.7   14.2    16.5   16.0    17.3   17.0    15.5   14.9    19.4   23.6
-//     global+local, 16     35.2   33.2    36.2   34.7    37.0   36.3    36.2   36.0    39.2   51.8
-//     full, 16 tiles       35.2   33.6    36.9   35.5    37.4   37.5    36.6   37.6    52.0   68.1
-//     full, 64 tiles      125.5  115.0                                 128.6  134.2   189.3  244.7
+//     causal, 16 tiles     34.9   31.9    36.2   33.1    36.4   33.5    35.8   32.8    36.4   34.1
+//     causal, 64 tiles    124.5  115.0                                 125.9  117.4   126.2  122.3
+//     strided, 16 tiles    14.4   12.8    16.6   15.4    17.3   16.1    15.6   14.1    19.9   22.5
+//     global+local, 16     35.1   32.1    36.7   34.1    37.2   35.9    36.1   34.9    39.5   49.8
+//     full, 16 tiles       35.3   32.4    36.9   35.0    38.2   37.2    36.9   36.5    51.5   66.3
+//     full, 64 tiles      125.1  115.2                                 130.4  137.1   187.2  245.8
 static bool few_lines(const FwdParams& p, int64_t n) {
   return n <= ((int64_t)4 * p.nnz <= (int64_t)3 * p.n_qtiles * p.n_ktiles ? kCus : kCus / 8 * 7);
 }
