@@ -81,3 +81,15 @@ def test_rows_leave_the_forward_whole(assembly):
     """No kernel of the forward writes O in pieces of 8 bytes, 32 bytes of a row at a time: rows pass through LDS (the statistics are single dwords)."""
     stores = set(re.findall(r"^\s+(global_store_\w+)", assembly["fwd.hip"], flags=re.M))
     assert "global_store_dwordx4" in stores and stores <= {"global_store_dwordx4", "global_store_dword"}, stores
+
+
+def test_short_lists_do_not_wait_for_every_read(assembly):
+    """The blocks of the second products (16 MFMAs, 32 transposing reads, of which the first are in the block before or in this one): the waits leave
+    reads in flight, but for the last fragment's."""
+    body = re.search(r"^_ZN2ua\d+fwd_short_kernel\w*:.*?^\.Lfunc_end", assembly["fwd.hip"], flags=re.M | re.S).group(0)
+    found = 0
+    for b in re.split(r"^(?:\.LBB\w+:|; %bb\.\d+:).*$", body, flags=re.M):
+        if b.count("v_mfma") == 16 and b.count("ds_read_b64_tr_b16") >= 16:
+            found += 1
+            assert len(re.findall(r"lgkmcnt\(0\)", b)) <= 2
+    assert found >= 2                                       # either half of a tile

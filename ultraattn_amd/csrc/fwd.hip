@@ -427,7 +427,7 @@ __global__ __launch_bounds__(Groups<1>::kThreads, 2) void fwd_plain_kernel(const
 // SIMD, one in its products while the other is in its softmax.  A row meets the same products and sums in the same order, so that
 // its result is the same bit for bit.
 // Bound: LDS.  Every K and V fragment is read for 16 rows instead of 32, 256 KiB a half tile at the 128 bytes a cycle that LDS
-// gives: 0.92 us a half tile, with four waves 0.99.  Where two workgroups share a CU it is slower.
+// gives: 0.86 us a half tile, with four waves 0.97.  Where two workgroups share a CU it is slower.
 template <int kWaveRows>
 __global__ __launch_bounds__(512, 2) void fwd_short_kernel(const FwdParams p) {
   using M = Mma<16>;
@@ -537,6 +537,9 @@ __global__ __launch_bounds__(512, 2) void fwd_short_kernel(const FwdParams p) {
       };
 #pragma unroll
       for (int i = 0; i < kVAhead; ++i) vfr[i] = rd_v(i);
+      // (Here, before the softmax: one by one between the MFMAs, where the compiler puts those of a tile's first half, every one is waited for.
+      // One head, causal 4096, 57.8 -> 55.3 us.)
+      __builtin_amdgcn_sched_barrier(0);
       if (kStage == 0) {                     // the next tile's entry
         if (!walk.has(e + 1)) walk.fetch(e + 1, p.col_idx, p.flag, p.n_ktiles);
         ent_next = walk.at(min(e + 1, e1 - 1));
@@ -650,7 +653,7 @@ static int fwd_common(FwdParams& p, const void* q, const void* k, const void* v,
 // Groups sum in another order, so that the last bits of a row depend on how many lines the launch has.  Tile lists, whose
 // launches are shards of the rows and heads of one mask, therefore run with one group whatever their size: a row's result is
 // the same bit for bit in every launch that holds its list.  Lists of up to 128 lines pay for that (one head, causal 4096: forward
-// 35 us with four groups, 58 with one, see few_lines, backward 51 and 119; from 512 lines on little changes).
+// 35 us with four groups, 55 with one, see few_lines, backward 51 and 119; from 512 lines on little changes).
 static int fwd_groups(int64_t n, int64_t walk, int n_parts, bool dense_causal) {
   const bool uneven = dense_causal && n_parts == 1;
   if (walk >= 2 && (2 * n <= kCus || (uneven && n <= kCus && walk >= 16))) return 4;
@@ -659,12 +662,12 @@ static int fwd_groups(int64_t n, int64_t walk, int n_parts, bool dense_causal) {
 // Tile lists of n lines that run with eight waves a workgroup: up to one line a CU, and up to seven on eight CUs where nearly all lines are of
 // full length.  Both kernels give the same bits, so that the line is drawn by time alone: us, four waves and eight
 //     lines                      128            208            240            256            320
-//     causal, 16 tiles     34.9   31.9    36.2   33.1    36.4   33.5    35.8   32.8    36.4   34.1
-//     causal, 64 tiles    124.5  115.0                                 125.9  117.4   126.2  122.3
-//     strided, 16 tiles    14.4   12.8    16.6   15.4    17.3   16.1    15.6   14.1    19.9   22.5
-//     global+local, 16     35.1   32.1    36.7   34.1    37.2   35.9    36.1   34.9    39.5   49.8
-//     full, 16 tiles       35.3   32.4    36.9   35.0    38.2   37.2    36.9   36.5    51.5   66.3
-//     full, 64 tiles      125.1  115.2                                 130.4  137.1   187.2  245.8
+//     causal, 16 tiles     35.2   30.8    36.3   32.1    36.4   33.2    35.9   32.2    36.8   34.4
+//     causal, 64 tiles    123.3  109.5                                 126.6  113.6   126.5  121.2
+//     strided, 16 tiles    14.5   12.3    16.7   15.2    17.3   16.2    15.6   14.3    20.0   22.7
+//     global+local, 16     35.5   32.6    36.6   34.1    37.2   36.8    36.4   35.2    40.2   49.9
+//     full, 16 tiles       35.1   33.0    37.2   35.6    37.6   37.4    37.1   37.0    52.3   66.2
+//     full, 64 tiles      125.2  112.7                                 133.3  141.4   190.8  242.7
 static bool few_lines(const FwdParams& p, int64_t n) {
   return n <= ((int64_t)4 * p.nnz <= (int64_t)3 * p.n_qtiles * p.n_ktiles ? kCus : kCus / 8 * 7);
 }
