@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-@pytest.mark.parametrize("blocks,heads", [(32, 7), (16, 14), (15, 15), (16, 15)])        # 224, 224, 225 and 240 lines
+@pytest.mark.parametrize("blocks,heads", [(32, 7), (25, 9), (17, 15), (16, 16), (4, 64), (3, 86)])      # 224, 225 and 255 long lines; 256, 256 and 258 of up to 16 tiles
 def test_same_bits_around_the_bound(blocks, heads):
     g = torch.Generator().manual_seed(heads)
     few = [torch.randn(1, blocks * 128, heads, 128, generator=g).to(torch.bfloat16).to(DEV) for _ in range(3)]

@@ -660,16 +660,18 @@ static int fwd_groups(int64_t n, int64_t walk, int n_parts, bool dense_causal) {
   return walk >= 3 && n <= (uneven ? 2 * kCus : kCus) ? 2 : 1;
 }
 // Tile lists of n lines that run with eight waves a workgroup: up to one line a CU, and up to seven on eight CUs where nearly all lines are of
-// full length.  Both kernels give the same bits, so that the line is drawn by time alone: us, four waves and eight
+// full length and longer than 16 tiles.  Both kernels give the same bits, so that the line is drawn by time alone: us, four waves and eight
 //     lines                      128            208            240            256            320
 //     causal, 16 tiles     35.2   30.8    36.3   32.1    36.4   33.2    35.9   32.2    36.8   34.4
 //     causal, 64 tiles    123.3  109.5                                 126.6  113.6   126.5  121.2
 //     strided, 16 tiles    14.5   12.3    16.7   15.2    17.3   16.2    15.6   14.3    20.0   22.7
 //     global+local, 16     35.5   32.6    36.6   34.1    37.2   36.8    36.4   35.2    40.2   49.9
+//     full, 4 tiles        12.2   10.7    14.0   12.8    14.9   14.4    13.8   12.7    18.7   22.0
 //     full, 16 tiles       35.1   33.0    37.2   35.6    37.6   37.4    37.1   37.0    52.3   66.2
 //     full, 64 tiles      125.2  112.7                                 133.3  141.4   190.8  242.7
 static bool few_lines(const FwdParams& p, int64_t n) {
-  return n <= ((int64_t)4 * p.nnz <= (int64_t)3 * p.n_qtiles * p.n_ktiles ? kCus : kCus / 8 * 7);
+  const bool uneven = (int64_t)4 * p.nnz <= (int64_t)3 * p.n_qtiles * p.n_ktiles, brief = p.nnz <= 16 * (int64_t)p.n_qtiles;
+  return n <= (uneven || brief ? kCus : kCus / 8 * 7);
 }
 // `plain`: one group per workgroup, and of a dense rectangle the bits of its tile list.
 static int fwd_launch(FwdParams& p, bool plain, hipStream_t st) {
