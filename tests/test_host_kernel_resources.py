@@ -93,3 +93,12 @@ def test_short_lists_do_not_wait_for_every_read(assembly):
             found += 1
             assert len(re.findall(r"lgkmcnt\(0\)", b)) <= 2
     assert found >= 2                                       # either half of a tile
+
+
+def test_accumulators_are_cleared_in_pairs(assembly):
+    """No block of a one-group kernel clears 64 or 128 accumulator registers one by one."""
+    for text in assembly.values():
+        for body in re.findall(r"^_ZN2ua\d+\w*kernel\w*:.*?^\.Lfunc_end", text, flags=re.M | re.S):
+            if any(n in body.split(":", 1)[0] + "E" for n in ONE_GROUP):
+                most = max(b.count("v_mov_b32") for b in re.split(r"^(?:\.LBB\w+:|; %bb\.\d+:).*$", body, flags=re.M))
+                assert most < 64, (body[:60], most)

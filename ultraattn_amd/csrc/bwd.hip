@@ -455,7 +455,7 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& given, uint32_t lds_b
   }
   f32x16 dk[4], dv[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) { dk[i] = f32x16{0}; dv[i] = f32x16{0}; }
+  for (int i = 0; i < 4; ++i) { Mma<S::kM>::clear(dk[i]); Mma<S::kM>::clear(dv[i]); }
 
   PairAddr<S::kM> ad(lds_base, lane);
   if (e0 < e1) put_stat(0, st0);
@@ -692,7 +692,7 @@ __device__ __forceinline__ void dq_walk(const BwdParams& given, uint32_t lds_blo
 
   f32x16 dq[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) dq[i] = f32x16{0};
+  for (int i = 0; i < 4; ++i) M::clear(dq[i]);
   const PairAddr<S::kM> ad(lds_base, lane);
   // the rows arrive before the walk (see dkdv_kernel)
 #pragma unroll

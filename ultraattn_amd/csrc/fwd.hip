@@ -289,7 +289,7 @@ __device__ __forceinline__ void fwd_lines(const FwdParams& p) {
 
   f32x16 oacc[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) oacc[i] = f32x16{0};
+  for (int i = 0; i < 4; ++i) M::clear(oacc[i]);
   SoftmaxState st[2];                      // of the lane's queries
   int nat[M::kRowRegs], tr[4];             // row reads of K, transposing reads of V
 #pragma unroll

@@ -11,6 +11,7 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 
 constexpr int kCus = 256;               // compute units of the device
@@ -108,6 +109,17 @@ struct Mma<16> {
 #pragma unroll
     for (int j = 0; j < 4; ++j) x[4 * q + j] = c[j];
   }
+  // Zeros, two registers an instruction: of accumulators that are used four by four the compiler clears one register after the other, 128 of dK
+  // and dV, and 0.35 us of every backward over lists (one tile 9.3 -> 8.9 us).
+  static __device__ __forceinline__ void clear(f32x16& x) {
+#pragma unroll
+    for (int i = 0; i < 16; i += 2) {
+      f32x2 zeros;
+      asm volatile("v_mov_b64 %0, 0" : "=v"(zeros));
+      x[i] = zeros[0];
+      x[i + 1] = zeros[1];
+    }
+  }
   struct Start { f32x4 of[2]; };           // what a lane's columns start from
   static __device__ __forceinline__ Start start(const float (&x)[2]) { return {{f32x4{x[0], x[0], x[0], x[0]}, f32x4{x[1], x[1], x[1], x[1]}}}; }
   static __device__ __forceinline__ void keep(Start& s) { asm volatile("" : "+v"(s.of[0]), "+v"(s.of[1])); }
@@ -169,6 +181,7 @@ struct Mma<32> {
   static constexpr __device__ int slot_n(int i) { return i >> 3; }
   static constexpr __device__ int slot_j(int i) { return i & 7; }
   static __device__ __forceinline__ f32x16 mfma(bf16x8 a, bf16x8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
+  static __device__ __forceinline__ void clear(f32x16& x) { x = f32x16{0}; }
   struct Start { f32x16 of; };
   static __device__ __forceinline__ Start start(const float (&x)[2]) {
     Start s;
