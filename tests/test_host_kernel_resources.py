@@ -102,3 +102,9 @@ def test_accumulators_are_cleared_in_pairs(assembly):
             if any(n in body.split(":", 1)[0] + "E" for n in ONE_GROUP):
                 most = max(b.count("v_mov_b32") for b in re.split(r"^(?:\.LBB\w+:|; %bb\.\d+:).*$", body, flags=re.M))
                 assert most < 64, (body[:60], most)
+
+
+def test_short_dense_walks_do_not_wait_for_parameters_at_their_end(assembly):
+    """The dense forward of one group has nearly all it needs at its end in scalar registers (of 19 loads of parameters eight came behind the products)."""
+    body = re.search(r"^_ZN2ua\d+fwd_kernelILi1ELb1EE\w*:.*?^\.Lfunc_end", assembly["fwd.hip"], flags=re.M | re.S).group(0)
+    assert len(re.findall(r"s_load_dword", body[body.rindex("v_mfma"):])) <= 2
