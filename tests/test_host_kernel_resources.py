@@ -108,3 +108,8 @@ def test_short_dense_walks_do_not_wait_for_parameters_at_their_end(assembly):
     """The dense forward of one group has nearly all it needs at its end in scalar registers (of 19 loads of parameters eight came behind the products)."""
     body = re.search(r"^_ZN2ua\d+fwd_kernelILi1ELb1EE\w*:.*?^\.Lfunc_end", assembly["fwd.hip"], flags=re.M | re.S).group(0)
     assert len(re.findall(r"s_load_dword", body[body.rindex("v_mfma"):])) <= 2
+
+
+def test_no_scalars_in_vector_lanes_in_any_form(assembly):
+    spilled = _metadata(assembly, "sgpr_spill_count")
+    assert not any(spilled.values()), spilled

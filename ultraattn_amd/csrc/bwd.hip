@@ -59,13 +59,15 @@ __device__ __forceinline__ ParamsLate params_late() {
   asm volatile("" : "+s"(p));
   return p;
 }
-// With one group what a walk needs is read behind the branch that leads to it: read before, the parameters of both sides at once ask for more
+// What a walk needs is read behind the branch that leads to it: read before, the parameters of both sides at once ask for more
 // scalar registers than there are, and up to 61 of them live in vector lanes (causal 32 heads of 2048, backward 131.9 -> 121.6 us with
-// the two kinds of walk in kernels of their own).  The short walks of more groups start 2 % earlier with all parameters in flight before the branch.
-template <int kForm>
-__device__ __forceinline__ const BwdParams& params_of_walk(const BwdParams& given) { return kForm == 1 ? *(const BwdParams*)params_late() : given; }
-// Brings all parameters into the scalar cache while the first ones are on their way, for a walk that reads them behind a branch (short
-// walks of one group: 171 heads of 128, causal, 15.5 -> 14.9 us, 92 of 128 x 256 15.0 -> 14.3, 32 of 1024 53.2 -> 52.5).
+// the two kinds of walk in kernels of their own).  Of several groups, whose short walks are often the columns', the columns' are in flight before the
+// branch.  With both sides' there half lines had ten scalars in vector lanes and a private segment of 20 bytes, which no instruction used but every
+// launch paid for (32 heads of 512 18.4 -> 17.7 us, 16 of 1024 30.4 -> 29.8; four groups, 8 heads of causal 1024 18.0 -> 17.7).
+template <int kForm, bool kRows>
+__device__ __forceinline__ const BwdParams& params_of_walk(const BwdParams& given) { return kForm == 1 || kRows ? *(const BwdParams*)params_late() : given; }
+// Brings all parameters into the scalar cache while the first ones are on their way, for walks that read them behind a branch (short
+// ones of one group: 171 heads of 128, causal, 15.5 -> 14.9 us, 92 of 128 x 256 15.0 -> 14.3, 32 of 1024 53.2 -> 52.5).
 __device__ __forceinline__ void touch_params() {
   constexpr int kLines = 9, kWords = sizeof(BwdParams) / 4;
   static_assert(16 * (kLines - 1) < kWords && kWords <= 16 * kLines, "one word of every 64 bytes");
@@ -202,12 +204,8 @@ struct PairStream {
     rx = make_rsrc_words(x + row0 * xs, more ? (uint32_t)((kTile - 1) * xs + kHeadDim) * 2 : 0);
     ry = make_rsrc_words(y + row0 * ys, more ? (uint32_t)((kTile - 1) * ys + kHeadDim) * 2 : 0);
   }
-  // (Opaque in every step: the sums of the copies' LDS addresses would occupy scalar registers all along, and vector lanes.)
-  __device__ __forceinline__ void next_step() { asm volatile("" : "+s"(lds)); }
-  // The same for the strides, from which the copies then form their rows' offsets anew: dQ's walk of half lines had ten scalars in vector
-  // lanes otherwise and with them a private segment of 20 bytes, which no instruction used but every launch paid for (32 heads of 512, forward and
-  // backward, 34.93 -> 34.82 us).
-  __device__ __forceinline__ void next_strides() { asm volatile("" : "+s"(xs), "+s"(ys)); }
+  // (Opaque in every step: the sums of the copies' LDS addresses would occupy scalar registers all along, and vector lanes.  Half lines have scalars enough.)
+  __device__ __forceinline__ void next_step() { if (kForm != kHalves) asm volatile("" : "+s"(lds)); }
   // copy n of kCopies into stage kStage, rows from 64 or 32 * part of the tile on
   template <int kStage>
   __device__ __forceinline__ void copy(int n, int part) const {
@@ -371,7 +369,7 @@ __device__ __forceinline__ void dkdv_block(const PairAddr<32>& ad, uint32_t stat
 // per half tile of dK/dV, 0.9 of them MFMAs); the other groups fill the CU without partial results in memory.
 template <int kForm, bool kDense>
 __device__ __forceinline__ void dkdv_walk(const BwdParams& given, uint32_t lds_block, int block) {
-  const BwdParams& p = params_of_walk<kForm>(given);
+  const BwdParams& p = params_of_walk<kForm, false>(given);
   using S = Stages<kForm>;
   const int tid = threadIdx.x % (64 * S::kWaves), lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -480,7 +478,7 @@ __device__ __forceinline__ void dkdv_walk(const BwdParams& given, uint32_t lds_b
     }
     put_stat(kStage ^ 1, stat);
     stat = S::kSteps == 2 ? load_stat(ent_next, part_of(kStage)) : load_stat(walk.at(min(e + 2, e1 - 1)), group);
-    if (kForm != kHalves) in.next_step();
+    in.next_step();
     if (!kFirst) in.tile(walk.tile(ent_next), e + 1 < e1);
     const bool causal = (ent >> 30) != 0;
     // causal tile: query block nb sees none of the wave's keys when nb < k_block, some when nb == k_block
@@ -613,7 +611,7 @@ __device__ __forceinline__ void dq_block(const PairAddr<kM>& ad, const bf16x8 (&
 
 template <int kForm, bool kDense>
 __device__ __forceinline__ void dq_walk(const BwdParams& given, uint32_t lds_block, int block) {
-  const BwdParams& p = params_of_walk<kForm>(given);
+  const BwdParams& p = params_of_walk<kForm, true>(given);
   static_assert(kDense || kForm == 1, "lists run with one group");
   if (kForm == 1 && kDense && p.rows_ahead) __builtin_amdgcn_s_setprio(1);
   using S = Stages<kForm>;
@@ -710,7 +708,6 @@ __device__ __forceinline__ void dq_walk(const BwdParams& given, uint32_t lds_blo
     // (of a list beside the first block, which one group always sees; a group of several may see none of its blocks)
     if (kDense) look_ahead();
     in.next_step();
-    if (kForm == kHalves) in.next_strides();
     if (!kFirst) in.tile(walk.tile(ent_next), e + 1 < e1);
     wait_vmem_all();
     __syncthreads();            // this stage has landed; everyone is done with the other one, which the copies now fill
@@ -781,7 +778,7 @@ template <int kForm, bool kDense>
 __global__ __launch_bounds__(Groups<kForm>::kThreads, 2) void bwd_kernel(const BwdParams p) {
   __shared__ __attribute__((aligned(1024))) unsigned char smem[Stages<kForm>::kCount * Stages<kForm>::kBytes];
   const uint32_t lds_base = (uint32_t)(uintptr_t)(UA_LDS unsigned char*)smem;
-  if (kForm == 1) touch_params();
+  touch_params();
   if ((int)blockIdx.x < p.n_col_blocks) dkdv_walk<kForm, kDense>(p, lds_base, blockIdx.x);
   else                                  dq_walk<kForm, kDense>(p, lds_base, blockIdx.x - p.n_col_blocks);
 }
